@@ -19,6 +19,8 @@ PROBES_SRC = CSRC / "probes" / "probes.hip"      # measurement probes for bench.
 PROBES_LIB = PKG / "libgguf_probes.so"
 TORCH_BINDING_SRC = CSRC / "torch_binding" / "gguf_torch_ops.cpp"   # torch.ops._C_gguf.* compiled (host code)
 TORCH_BINDING_LIB = PKG / "_C_gguf_native.so"
+CALLS_SRC = CSRC / "torch_binding" / "gguf_calls.cpp"               # the layer calls of dispatch.py compiled (a CPython module)
+CALLS_LIB = PKG / "_gguf_calls.so"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -36,25 +38,34 @@ def _compile(src: Path, obj: Path) -> None:
         raise RuntimeError(f"hipcc failed on {src.name}:\n{err}")
 
 
-def build_torch_binding() -> Path:
-    """The compiled torch operator library over the C ABI (csrc/torch_binding): host code only, built with the C++
-    compiler against the headers of the torch that is installed, linked against libgguf_hip.so beside it."""
+def _build_against_torch(src: Path, lib: Path, libs: tuple[str, ...]) -> Path:
+    """Host code over the C ABI, built with the C++ compiler against the headers of the torch that is installed and
+    linked against libgguf_hip.so beside it."""
+    import sysconfig
+
     import torch
     from torch.utils import cpp_extension
 
     cxx = os.environ.get("CXX", "g++")
-    tmp = TORCH_BINDING_LIB.with_suffix(".so.tmp")
+    tmp = lib.with_suffix(".so.tmp")
     torch_lib = Path(torch.__file__).resolve().parent / "lib"
     cmd = [cxx, "-std=c++17", "-O2", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           *[f"-I{d}" for d in cpp_extension.include_paths()], "-I/opt/rocm/include", f"-I{PKG.parent / 'include'}",
-           str(TORCH_BINDING_SRC), "-o", str(tmp), f"-L{torch_lib}", "-ltorch", "-ltorch_cpu", "-lc10", "-ltorch_hip", "-lc10_hip",
+           *[f"-I{d}" for d in cpp_extension.include_paths()], f"-I{sysconfig.get_paths()['include']}", "-I/opt/rocm/include",
+           f"-I{PKG.parent / 'include'}", str(src), "-o", str(tmp), f"-L{torch_lib}", *[f"-l{name}" for name in libs],
            f"-L{PKG}", "-lgguf_hip", "-Wl,-rpath,$ORIGIN"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
-        raise RuntimeError("the torch binding failed to build:\n" + res.stderr)
-    os.replace(tmp, TORCH_BINDING_LIB)
-    return TORCH_BINDING_LIB
+        raise RuntimeError(f"{src.name} failed to build:\n" + res.stderr)
+    os.replace(tmp, lib)
+    return lib
+
+
+def build_torch_binding() -> Path:
+    """The compiled torch operator library and the compiled layer calls (csrc/torch_binding)."""
+    torch_libs = ("torch", "torch_cpu", "c10", "torch_hip", "c10_hip")
+    _build_against_torch(CALLS_SRC, CALLS_LIB, ("torch_python", *torch_libs, "amdhip64"))
+    return _build_against_torch(TORCH_BINDING_SRC, TORCH_BINDING_LIB, torch_libs)
 
 
 def build(verbose: bool = True) -> Path:

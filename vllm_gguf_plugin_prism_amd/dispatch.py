@@ -64,11 +64,54 @@ def select_moe_path(weight_type: int, weight_type2: int, tokens: int) -> str:
 # ---------------------------------------------------------------------------------------- tensor level
 
 
+class _NoCalls:
+    """Stands in for the compiled layer calls where they have not been built: serves nothing."""
+
+    @staticmethod
+    def linear(*args):
+        return None
+
+    merged_linear = moe = embedding = linear
+
+
+_CALLS = None
+
+
+def _calls():
+    """``_gguf_calls`` (csrc/torch_binding/gguf_calls.cpp): a layer call checked, allocated and launched in one step from
+    the interpreter.  Its functions return None for what they do not serve (and raise nothing then): the Python below
+    does.  One sequence's decode step of a [3072,1024] Q8_0 matrix spends 11 us in that Python against 3.6 us in its kernel."""
+    global _CALLS
+    if _CALLS is None:
+        import os
+
+        from . import _lib
+
+        path = os.environ.get("GGUF_HIP_LIBRARY", str(_lib.LIB_PATH))
+        if path != str(_lib.LIB_PATH) or not os.path.exists(path):
+            return _NoCalls                  # (the module is linked against the library in this folder)
+        _lib.lib()                           # torch's HIP runtime and libgguf_hip.so first (see _lib.lib)
+        try:
+            from . import _gguf_calls as calls
+        except ImportError as exc:
+            if (_lib.LIB_PATH.parent / "_gguf_calls.so").exists():   # built against another torch
+                import warnings
+
+                warnings.warn(f"_gguf_calls.so does not load ({exc}); rebuild it with `python -m vllm_gguf_plugin_prism_amd.build`.  "
+                              "Layer calls go through Python.", RuntimeWarning)
+            calls = _NoCalls
+        _CALLS = calls
+    return _CALLS
+
+
 def fused_mul_mat_gguf(x, weight, weight_type: int, *, out=None, bias=None):
     """``x @ dequant(weight).T`` through the path the reference would pick (linear.py:35-58).
 
     ``weight`` may be a slice ``merged[start:end, :row_bytes]`` of a padded merged tensor, ``out`` a column slice of the
     merged result and ``bias`` the matching slice of the layer bias: the a8 kernels address all three in place."""
+    y = (_CALLS or _calls()).linear(x, weight, weight_type, out, bias)
+    if y is not None:
+        return y
     import torch
 
     from . import ops
@@ -108,8 +151,6 @@ def apply_linear(x, weight, weight_type: int, *, shard_ids=(), shard_offset_map=
     call, as in the reference.  Shards of different types are multiplied one by one, but where the reference copies
     every shard out of the padded tensor on every call and concatenates the results, each call here reads its rows in
     place and writes its columns of the merged result, bias included."""
-    import torch
-
     shard_ids = list(shard_ids)
     if not shard_ids:
         return fused_mul_mat_gguf(x, weight, weight_type, bias=bias)
@@ -117,6 +158,11 @@ def apply_linear(x, weight, weight_type: int, *, shard_ids=(), shard_offset_map=
     types = [int((shard_weight_types or {}).get(i, weight_type)) for i in shard_ids]
     if len(set(types)) == 1:
         return fused_mul_mat_gguf(x, weight, types[0], bias=bias)
+    y = (_CALLS or _calls()).merged_linear(x, weight, shard_ids, shard_offset_map, types, bias)
+    if y is not None:
+        return y
+    import torch
+
     widths = [shard_offset_map[i][1] - shard_offset_map[i][0] for i in shard_ids]
     out = torch.empty(x.shape[0], sum(widths), dtype=x.dtype, device=x.device)
     col = 0
@@ -175,6 +221,9 @@ def moe_align_block_size(topk_ids, block_size: int, num_experts: int):
 
 def fused_moe_gguf(x, w1, w2, topk_weights, topk_ids, weight_type: int, weight_type2: int, activation: str = "silu"):
     """Two-stage GGUF MoE layer (fused_moe.py:34-133): gate/up GEMM, gated activation, down GEMM, weighted sum."""
+    y = (_CALLS or _calls()).moe(x, w1, w2, topk_weights, topk_ids, weight_type, weight_type2, activation)
+    if y is not None:
+        return y
     import torch
 
     from . import ops
@@ -233,6 +282,9 @@ def fused_moe_gguf(x, w1, w2, topk_weights, topk_ids, weight_type: int, weight_t
 def apply_gguf_embedding(x, weight, weight_type: int, hidden_size: int, dtype=None):
     """Embedding lookup from a packed table (vocal_embeds.py:79-98); the reference gathers the packed rows with
     index_select and dequantizes the copy, here one kernel reads the rows in place."""
+    y = (_CALLS or _calls()).embedding(x, weight, weight_type, hidden_size, dtype)
+    if y is not None:
+        return y
     import torch
 
     from . import ops
