@@ -196,6 +196,7 @@ __device__ __forceinline__ T finish(float v, const T* bias, int64_t n) {
 
 // q8_1 quantisation of M rows into the workspace (q8_1.hip).  act: gated activation applied while loading (see
 // q8_1_device.h).  half_plane: if not null, also the dequantized rows in half precision, [M][q8_kp(K)].
+// permuted: the quants of a row in the order of the streaming tile kernel (q8_permuted).
 // From how many pairs on the per-pair MoE operator sorts its pairs by expert and reads a shared expert once per group
 // of them: two pairs per expert on average.  While all the experts together fit the last-level cache the per-pair
 // kernel, which has no sort and no second launch, reads shared experts from there and stays ahead a little longer
@@ -206,7 +207,7 @@ static inline bool moe_share_pays(int64_t pairs, int64_t num_experts, int64_t ex
   return cached ? 2 * pairs >= 5 * num_experts : pairs >= 2 * num_experts;
 }
 int quantize_q8_1(const void* x, int xdtype, void* ws, int64_t M, int64_t K, hipStream_t stream, int act = 0,
-                  void* half_plane = nullptr);
+                  void* half_plane = nullptr, bool permuted = false);
 
 // Opt a kernel in to more than 64 KB of dynamic LDS, once per device: `done` is the caller's bit set of the devices
 // already served (one static per kernel instantiation).  The attribute belongs to the device the kernel's code object

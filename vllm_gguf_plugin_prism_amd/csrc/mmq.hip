@@ -25,6 +25,7 @@
 // The same kernel runs the grouped MoE contraction (reference: csrc/gguf/moe.cuh:5-129):
 // token rows are gathered through sorted_token_ids, the weight base moves to the block's
 // expert, and results scatter to the rows the slots name.
+#include "tile_stream.h"
 #include "mmq_formats.h"
 #include "q8_1_device.h"
 
@@ -621,13 +622,14 @@ int moe_tiles16(const void* W, const void* ws, void* Y, int dtype, int type, int
 int moe_vec_tiles(const void* X, int xdtype, void* workspace, const void* W, const int32_t* topk_ids, void* Y, int type, int N,
                   int K, int top_k, int tokens, int act, int num_experts, hipStream_t s) {
   const int pairs = tokens * top_k;
-  int rc = quantize_q8_1(X, xdtype, workspace, tokens, K, s, act);
-  if (rc != GGUF_OK) return rc;
   // Blocks of 16 slots while an expert has 16 pairs or fewer on average (most of a 32-slot block would be padding),
   // blocks of 32 above.  The routing arrays of either fit the room moe_vec_tiles_workspace reports.
   const int blk = pairs <= 16 * num_experts && moe_tiles16_ok(type) ? 16 : 32;
   const int64_t sorted_cap = (int64_t)pairs + (int64_t)num_experts * (blk - 1);
   const int64_t block_cap = sorted_cap / blk + 1;
+  const bool stream = blk == 16 && ts_moe_takes(type, N, K, sorted_cap, tokens, top_k);
+  int rc = quantize_q8_1(X, xdtype, workspace, tokens, K, s, act, nullptr, stream);
+  if (rc != GGUF_OK) return rc;
   int32_t* sorted = (int32_t*)((char*)workspace + (int64_t)tokens * q8_row_bytes(K));  // rows are a multiple of 4 bytes long
   int32_t* experts = sorted + sorted_cap;
   int32_t* post = experts + block_cap;
@@ -635,6 +637,7 @@ int moe_vec_tiles(const void* X, int xdtype, void* workspace, const void* W, con
   if (rc != GGUF_OK) return rc;
   const int64_t stride = (int64_t)N * (K / block_elems(type)) * block_bytes(type);
   MoeArgs moe = {sorted, experts, post, stride, top_k, pairs, type == T_Q4_K || type == T_Q5_K ? 1 : 0};
+  if (stream) return ts_moe(W, workspace, Y, xdtype, type, N, K, (int)(sorted_cap / 16 * 16), moe, s);
   if (blk == 16) return moe_tiles16(W, workspace, Y, xdtype, type, N, K, (int)(sorted_cap / 16 * 16), moe, s);
   const int ns = (int)(sorted_cap / 32 * 32);   // blocks past the padded total see expert -1 and leave
   switch (type) {
@@ -684,7 +687,7 @@ int64_t moe_tiles_layer_workspace(int64_t tokens, int64_t top_k, int64_t H, int6
 }
 
 int moe_prepare(const void* X, int xdtype, void* q8x, int tokens, int K, const int32_t* topk_ids, int numel, int num_experts, int block,
-                int32_t* sorted_ids, int sorted_capacity, int32_t* expert_ids, int expert_capacity, int32_t* num_post_padded,
+                int32_t* sorted_ids, int sorted_capacity, int32_t* expert_ids, int expert_capacity, int32_t* num_post_padded, bool permuted,
                 hipStream_t s);   // moe_aux.hip
 int moe_weighted_sum_live(const void* Y, const float* topk_weights, const int32_t* topk_ids, int num_experts, void* out, int dtype,
                           int64_t tokens, int64_t top_k, int64_t N, hipStream_t s, const int32_t* slot_of_pair = nullptr);   // moe_aux.hip
@@ -698,6 +701,10 @@ int moe_tiles_layer(const void* X, int xdtype, void* workspace, const void* W13,
                     const float* topk_w, void* out, int H, int I, int N_out, int top_k, int tokens, int act, int num_experts, bool vec_sums,
                     int block, hipStream_t s) {
   const int pairs = tokens * top_k, elt = xdtype == GGUF_DTYPE_F32 ? 4 : 2;
+  // the streaming tile kernel runs on blocks of 16 slots (up to 128 pairs per expert, which the workspace of the caller's
+  // block size has room for)
+  const bool stream = ts_layer_takes(type13, type2, H, I, N_out, tokens, top_k, num_experts);
+  if (stream) block = 16;
   char* q8x = (char*)workspace;
   char* q8h = q8x + up16((int64_t)tokens * q8_row_bytes(H));
   char* y2 = q8h + up16((int64_t)pairs * q8_row_bytes(I));
@@ -706,9 +713,9 @@ int moe_tiles_layer(const void* X, int xdtype, void* workspace, const void* W13,
   int32_t* experts = sorted + sorted_cap;
   int32_t* post = experts + block_cap;
   // the rows of X quantized and the routing sorted in one launch (two where the sort's histogram rows outgrow 64 KB of LDS)
-  int rc = moe_prepare(X, xdtype, q8x, tokens, H, topk_ids, pairs, num_experts, block, sorted, (int)sorted_cap, experts, (int)block_cap, post, s);
+  int rc = moe_prepare(X, xdtype, q8x, tokens, H, topk_ids, pairs, num_experts, block, sorted, (int)sorted_cap, experts, (int)block_cap, post, stream, s);
   if (rc == GGUF_NOT_TAKEN) {
-    rc = quantize_q8_1(X, xdtype, q8x, tokens, H, s);
+    rc = quantize_q8_1(X, xdtype, q8x, tokens, H, s, 0, nullptr, stream);
     if (rc != GGUF_OK) return rc;
     rc = gguf_moe_align_block_size(topk_ids, pairs, num_experts, block, sorted, sorted_cap, experts, block_cap, post, (gguf_stream_t)s);
   }
@@ -717,6 +724,14 @@ int moe_tiles_layer(const void* X, int xdtype, void* workspace, const void* W13,
   // vec_sums: the offset term of Q4_K / Q5_K as the per-pair operator forms it; else as the grouped operator does
   const auto gemv_sums = [&](int type) { return vec_sums && (type == T_Q4_K || type == T_Q5_K) ? 1 : 0; };
   const MoeArgs m1 = {sorted, experts, post, (int64_t)2 * I * (H / block_elems(type13)) * block_bytes(type13), top_k, pairs, gemv_sums(type13)};
+  if (stream) {
+    rc = ts_moe(W13, q8x, nullptr, xdtype, type13, 2 * I, H, ns, m1, s, Gate16{q8h, q8_row_bytes(I), I, (int)q8_kp(I), act});
+    if (rc != GGUF_OK) return rc;
+    const MoeArgs m2 = {sorted, experts, post, (int64_t)N_out * (I / block_elems(type2)) * block_bytes(type2), 1, pairs, gemv_sums(type2)};
+    rc = ts_moe(W2, q8h, y2, xdtype, type2, N_out, I, ns, m2, s);
+    if (rc != GGUF_OK) return rc;
+    return moe_weighted_sum_live(y2, topk_w, vec_sums ? nullptr : topk_ids, num_experts, out, xdtype, tokens, top_k, N_out, s);
+  }
   rc = block == 16 ? moe_tiles16_gate(W13, q8x, q8h, xdtype, type13, I, H, ns, m1, act, s)
                    : moe_tiles32_gate(W13, q8x, q8h, xdtype, type13, I, H, ns, m1, act, s);
   if (rc != GGUF_OK) return rc == GGUF_NOT_TAKEN ? GGUF_ERR_TYPE : rc;
@@ -863,6 +878,17 @@ int gguf::mmq_linear_impl(const void* W, int64_t w_row_pitch_bytes, const void* 
   if (workspace_bytes < M * (q8_row_bytes(K) + (engine == GGUF_MMQ_HALF ? 2 * q8_half_pitch(K) : 0))) return GGUF_ERR_WORKSPACE;
   const int64_t partial_room = workspace_bytes - rows_bytes;
   const bool tiles_at_5 = M <= 16 && rows16_direct_pays(type, (int)M, N, K, true) && rows16_direct_takes(W, w_row_pitch_bytes, type, (int)M, (int)N, (int)K, partial_room > 0 ? partial_room : 0);
+  if (engine != GGUF_MMQ_HALF && ts_dense_takes(type, M, N, K, w_row_pitch_bytes)) {
+    int rc = quantize_q8_1(x, xdtype, q8_workspace, M, K, s, 0, nullptr, true);
+    if (rc != GGUF_OK) return rc;
+    TsCall c = {};
+    c.W = W; c.ws = q8_workspace; c.Y = Y; c.dtype = xdtype; c.M = (int)M; c.N = (int)N; c.K = (int)K;
+    c.rt = M <= 16 ? 1 : 2;
+    c.w_pitch = la.w_pitch; c.ldy = la.ldy; c.bias = la.bias;
+    c.row_blocks = 1;
+    c.live_blocks = 1;
+    return ts_any(type, c, s);
+  }
   if (engine == GGUF_MMQ_AUTO && M <= 8 && !tiles_at_5) {
     // a handful of rows: the streaming GEMV kernel with the tile kernels' offset sums reads W once at close to the
     // GEMV's rate and is exact in int8; it declines shapes it does not cover
@@ -954,11 +980,13 @@ extern "C" int gguf_moe_mmq_block(const void* X, int xdtype, void* q8_workspace,
   const int64_t ybytes = tokens * top_k * N * (xdtype == GGUF_DTYPE_F32 ? 4 : 2);
   if ((uintptr_t)Y & 15) return GGUF_ERR_SHAPE;
   hipLaunchKernelGGL(zero_rows_kernel, dim3((unsigned)((ybytes / 16 + 256) / 256)), dim3(256), 0, s, (uint4*)Y, ybytes);
-  const int rc = quantize_q8_1(X, xdtype, q8_workspace, tokens, K, s, act);
+  const bool streams = block == 16 && ts_moe_takes(type, N, K, num_sorted, tokens, top_k);
+  const int rc = quantize_q8_1(X, xdtype, q8_workspace, tokens, K, s, act, nullptr, streams);
   if (rc != GGUF_OK) return rc;
   MoeArgs moe = {sorted_token_ids, expert_ids, num_tokens_post_padded, expert_stride_bytes, (int)top_k, (int)(tokens * top_k), 0};
   const int ns = (int)(num_sorted / block * block);  // a trailing partial block is ignored, like the reference's integer division
   if (ns == 0) return launch_status();
+  if (streams) return ts_moe(W, q8_workspace, Y, xdtype, type, (int)N, (int)K, ns, moe, s);
   if (block == 16) return moe_tiles16(W, q8_workspace, Y, xdtype, type, (int)N, (int)K, ns, moe, s);
   return moe_tiles32(W, q8_workspace, Y, xdtype, type, (int)N, (int)K, ns, moe, s);
 }

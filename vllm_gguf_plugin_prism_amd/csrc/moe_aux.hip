@@ -154,7 +154,7 @@ __global__ __launch_bounds__(ALIGN_THREADS) void moe_prepare_kernel(const T* __r
                                                                     int numel, int num_experts, int block,
                                                                     int32_t* __restrict__ sorted_ids, int sorted_capacity,
                                                                     int32_t* __restrict__ expert_ids, int expert_capacity,
-                                                                    int32_t* __restrict__ num_post_padded) {
+                                                                    int32_t* __restrict__ num_post_padded, bool permuted) {
   extern __shared__ int lds[];
   if (blockIdx.x == 0) {
     moe_align_body(topk_ids, numel, num_experts, block, sorted_ids, sorted_capacity, expert_ids, expert_capacity, num_post_padded, lds);
@@ -164,7 +164,7 @@ __global__ __launch_bounds__(ALIGN_THREADS) void moe_prepare_kernel(const T* __r
   const int64_t g = (int64_t)(blockIdx.x - 1) * ALIGN_THREADS + threadIdx.x;
   const int64_t m = g / per_row;
   if (m >= tokens) return;                                      // (per_row is a multiple of 64: whole waves leave)
-  q8_1_quantize_thread<T>(x, ws, K, Kp, row_bytes, ACT_NONE, m, (int)(g % per_row), nullptr);
+  q8_1_quantize_thread<T>(x, ws, K, Kp, row_bytes, ACT_NONE, m, (int)(g % per_row), nullptr, permuted);
 }
 
 // out[t, n] = sum_k  T( float(Y[t, k, n]) * w[t, k] )   accumulated in fp32 in the order k = 0 .. top_k-1 and rounded
@@ -204,7 +204,7 @@ int moe_weighted_sum_live(const void* Y, const float* topk_weights, const int32_
 
 // quantize_q8_1(X) and gguf_moe_align_block_size(topk_ids) in one launch (sizes checked by the caller)
 int moe_prepare(const void* X, int xdtype, void* q8x, int tokens, int K, const int32_t* topk_ids, int numel, int num_experts, int block,
-                int32_t* sorted_ids, int sorted_capacity, int32_t* expert_ids, int expert_capacity, int32_t* num_post_padded,
+                int32_t* sorted_ids, int sorted_capacity, int32_t* expert_ids, int expert_capacity, int32_t* num_post_padded, bool permuted,
                 hipStream_t s) {
   const int Kp = (int)q8_kp(K);
   const size_t lds = (size_t)(1 + ALIGN_WAVES) * num_experts * sizeof(int);
@@ -213,7 +213,7 @@ int moe_prepare(const void* X, int xdtype, void* q8x, int tokens, int K, const i
   const unsigned grid = 1 + (unsigned)((threads + ALIGN_THREADS - 1) / ALIGN_THREADS);
   GGUF_DISPATCH_DTYPE(xdtype, hipLaunchKernelGGL(moe_prepare_kernel<scalar_t>, dim3(grid), dim3(ALIGN_THREADS), lds, s, (const scalar_t*)X,
                                                  (char*)q8x, K, Kp, q8_row_bytes(K), tokens, topk_ids, numel, num_experts, block, sorted_ids,
-                                                 sorted_capacity, expert_ids, expert_capacity, num_post_padded));
+                                                 sorted_capacity, expert_ids, expert_capacity, num_post_padded, permuted));
   return launch_status();
 }
 

@@ -16,10 +16,10 @@ namespace gguf {
 template <typename T>
 __global__ __launch_bounds__(256) void quantize_q8_1_kernel(const T* __restrict__ x, char* __restrict__ ws, int K,
                                                            int Kp, int64_t row_bytes, int act,
-                                                           _Float16* __restrict__ xh) {
+                                                           _Float16* __restrict__ xh, bool permuted) {
   const int t = blockIdx.x * 256 + threadIdx.x;  // one thread per 8 values of the padded row
   if (t * 8 >= Kp) return;
-  q8_1_quantize_thread<T>(x, ws, K, Kp, row_bytes, act, blockIdx.y, t, xh);
+  q8_1_quantize_thread<T>(x, ws, K, Kp, row_bytes, act, blockIdx.y, t, xh, permuted);
 }
 
 __global__ void q8_1_unpack_kernel(const char* __restrict__ ws, int8_t* __restrict__ q, float* __restrict__ ds, int Kp,
@@ -37,7 +37,7 @@ __global__ void q8_1_unpack_kernel(const char* __restrict__ ws, int8_t* __restri
   }
 }
 
-int quantize_q8_1(const void* x, int xdtype, void* ws, int64_t M, int64_t K, hipStream_t stream, int act, void* half_plane) {
+int quantize_q8_1(const void* x, int xdtype, void* ws, int64_t M, int64_t K, hipStream_t stream, int act, void* half_plane, bool permuted) {
   if (M == 0) return GGUF_OK;
   const int Kp = (int)q8_kp(K);
   const int64_t rb = q8_row_bytes(K);
@@ -46,7 +46,7 @@ int quantize_q8_1(const void* x, int xdtype, void* ws, int64_t M, int64_t K, hip
     const int rows = (int)((M - off) < 65535 ? (M - off) : 65535);
     GGUF_DISPATCH_DTYPE(xdtype, hipLaunchKernelGGL(quantize_q8_1_kernel<scalar_t>, dim3(gx, rows), dim3(256), 0, stream,
                                                    (const scalar_t*)x + off * K * (act == ACT_NONE ? 1 : 2), (char*)ws + off * rb, (int)K, Kp, rb, act,
-                                                   half_plane ? (_Float16*)half_plane + off * q8_half_pitch(K) : (_Float16*)nullptr));
+                                                   half_plane ? (_Float16*)half_plane + off * q8_half_pitch(K) : (_Float16*)nullptr, permuted));
   }
   return launch_status();
 }

@@ -166,13 +166,18 @@ __device__ __forceinline__ Q8Quad q8_1_quantize8(const float (&v)[8]) {
   return r;
 }
 
+// Where the eight quants of values e .. e + 7 (e a multiple of 8) lie in a row stored for the streaming tile kernel: of
+// every 64 values, k group g of the matrix instruction's operand (values 8 g .. 8 g + 7 of both blocks) is one 16-byte
+// piece.  The planes of block scales and sums are as in the plain layout.
+__host__ __device__ __forceinline__ int q8_permuted(int e) { return (e & ~63) + 2 * (e & 24) + ((e >> 2) & 8); }
+
 // One thread of the row quantizer: the eight values [8 t, 8 t + 8) of padded row m -> eight quants, and from the first
 // lane of each quad the block's d, s and d * sum(q) planes.  The four lanes of a quad must run together (the block's
 // amax and sum cross them).  act: rows of x are [gate | up] and the gated activation is quantized; xh: also the
 // dequantized row in half precision.
 template <typename T>
 __device__ __forceinline__ void q8_1_quantize_thread(const T* __restrict__ x, char* __restrict__ ws, int K, int Kp, int64_t row_bytes, int act,
-                                                     int64_t m, int t, _Float16* __restrict__ xh) {
+                                                     int64_t m, int t, _Float16* __restrict__ xh, bool permuted = false) {
   const int e0 = t * 8;
   float v[8];
   if (e0 < K) {
@@ -184,7 +189,7 @@ __device__ __forceinline__ void q8_1_quantize_thread(const T* __restrict__ x, ch
   }
   const Q8Quad r = q8_1_quantize8(v);
   char* row = ws + m * row_bytes;
-  *(uint2*)(row + e0) = r.q;
+  *(uint2*)(row + (permuted ? q8_permuted(e0) : e0)) = r.q;
   if (xh) {
     // the dequantized row in half precision for the half-MFMA GEMM: RN16(d * q), d being the half-rounded scale.
     // d * q is exact in fp32; magnitudes past the half range saturate (only reachable from bf16 / fp32 inputs).

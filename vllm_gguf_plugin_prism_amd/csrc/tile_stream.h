@@ -1,0 +1,32 @@
+// Calls of the streaming tile kernel (tile_stream_core.h), for the code that routes to it.
+#pragma once
+#include "mmq_formats.h"
+
+namespace gguf {
+
+// One call of the kernel, dense (moe.sorted_token_ids null) or per block of 16 RT slots.
+struct TsCall {
+  const void* W;
+  const void* ws;              // q8_1 rows with permuted quants
+  void* Y;
+  int dtype, M, N, K, rt;      // rt: 16-row tiles of X per workgroup
+  int64_t w_pitch, ldy;
+  const void* bias;
+  bool gemv_sums;              // offset term on d * sum(q) instead of the stored sums
+  MoeArgs moe;
+  int row_blocks;              // tiles of 16 rt rows (dense) or blocks of slots
+  double live_blocks;          // how many of them hold pairs, estimated (dense: all)
+  Gate16 gate;                 // rows != null: the gated epilogue
+};
+
+// tile_stream.hip: whether a call is taken -- a dense product of M rows, a layer with this many (token, expert) pairs, an
+// expert GEMM on blocks of 16 slots by itself
+bool ts_dense_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch);
+bool ts_layer_takes(int type13, int type2, int64_t H, int64_t I, int64_t N_out, int64_t tokens, int64_t top_k, int64_t num_experts);
+bool ts_moe_takes(int type, int64_t N, int64_t K, int64_t num_sorted, int64_t tokens, int64_t top_k);
+int ts_any(int type, const TsCall& c, hipStream_t s);   // GGUF_NOT_TAKEN for other types
+// the grouped contraction over blocks of 16 slots; gate.rows: with the gated epilogue (W is [experts][2 inner][K])
+int ts_moe(const void* W, const void* ws, void* Y, int dtype, int type, int N, int K, int num_sorted, const MoeArgs& moe, hipStream_t s,
+           const Gate16& gate = Gate16{});
+
+}  // namespace gguf

@@ -1,0 +1,570 @@
+// Products with a few rows of activations (5 to 32), dense and per expert of an MoE layer, that run near the rate
+// the packed weights stream in.
+//
+// What bounds such a product is the weight stream; what keeps a kernel from it is everything around it: decoded weights
+// staged in LDS for the whole workgroup cost a barrier per step of K and line the waves up; operands read straight from
+// the packed blocks need four matrix instructions per block with three quarters of the activations zeroed.  Here the
+// waves of a workgroup walk their own weights on their own:
+//   * A wave's unit of work is a panel: 16 weight rows x 256 values of K.  It fetches the panel's bytes as 16-byte
+//     pieces, lane after lane, straight into its own LDS ring (global_load_lds; D panels in flight), reads its lanes'
+//     fields from there, asks for another panel and multiplies: one v_mfma_i32_16x16x32_i8 per 32-value block and 16
+//     rows of X.  No register holds bytes in flight and no barrier stands between panels.
+//   * The activations of a chunk of K (up to 16 panels) lie in LDS for the eight waves, fetched the same way, a row's
+//     1 KB per request; a chunk is fetched while the one before is multiplied where LDS has room for two.  (Operands
+//     read from global memory instead cost the CU's memory pipeline 64 cycles per request -- 16 rows, 16 cache lines --
+//     450 of them per panel, where the panel's bytes arrive in 250.)  The quantizer stores a row such that a lane's
+//     operand of two blocks is one 16-byte read (q8_permuted).
+//   * The offset term of Q4_0, Q4_K, Q5_K -- minus min times block sum, a contraction over blocks -- is two fp32 matrix
+//     instructions per panel (v_mfma_f32_16x16x4_f32, fp32 inputs and sums) instead of a multiply-add per result and
+//     block, and each lane decodes two of the eight mins instead of all of them.
+//   * Block sums leave the matrix unit as floats (the accumulator starts at the bit pattern of 1.5 * 2^23), so the two
+//     block scales are two multiply-adds per result.  About 150 vector instructions per 4096 Q4_K weights at 16 rows.
+//   * Where the output has fewer column groups than the chip has waves, KS waves share a group and deal K panel by
+//     panel; their partial tiles are added through LDS in the order of K (SPLIT).  Else a wave finishes its columns alone.
+// Measured (us per call with the quantizer's launch, before -> now; 5.15 TB/s is what a large copy reaches): [28672,8192]
+// Q4_K, 16 rows 45.7 -> 37.6 (3.5 TB/s with the quantizer's 3.5 us inside), 32 rows 73.7 -> 54.0; [6144,4096] Q8_0, 16 rows 18.8 -> 13.4;
+// [12288,1024] Q6_K, 16 rows 21.5 -> 11.7.  MoE layers: Q4_0, 64 experts, top-8, 64 tokens 112 -> 86; Q4_K with Q6_K, 128
+// experts, 300 tokens 262 -> 175.  What is left is the beginning of a workgroup (first chunk of activations, first
+// panels: 4 to 6 us) and the vector instructions around the multiplications.
+// Arithmetic as in the other integer kernels (mmq.cuh:2-104, vecdotq.cuh: exact int32 block sums, scales in fp32).
+#pragma once
+#include "mmq_i_core.h"
+#include "q8_1_device.h"
+#include "tile_stream.h"
+#include "tile_stream_formats.h"
+
+namespace gguf {
+
+constexpr int TS_NW = 8;       // waves per workgroup
+
+struct TsArgs {
+  int M, N, K, Kp;             // M: rows of X (dense)
+  uint32_t w_pitch, ws_row_bytes;
+  int np, ks_log2, ppr;        // panels per row; waves that share a column group; 16-byte pieces of LDS for a weight row's panel
+  int pc_log2, nbuf;           // panels per chunk of activations in LDS, chunks in LDS
+  int passes;                  // column groups a wave walks one after the other (more than one: all of K is one chunk)
+  uint32_t ppr_inv, rb_inv, topk_inv;   // 2^32 / (ppr, row blocks, top_k) rounded up: the kernel starts without a division
+  int plane, dtype;            // block sums for the offset term: 1 = stored sums, 2 = d * sum(q); GGUF_DTYPE_* of Y
+  int64_t ldy;
+  const void* bias;
+};
+
+typedef uint32_t u32x4_s __attribute__((ext_vector_type(4)));
+
+template <int N> __device__ __forceinline__ void ts_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+// wave-uniform 16-byte-per-lane fetch into LDS: lane l's bytes land at m0 + 16 l
+__device__ __forceinline__ void ts_fetch(uint32_t at, const void* base, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(at), "s"(base), "s"(lds) : "memory");
+}
+// the same for the lanes in `mask` only (all lanes are active before and after)
+__device__ __forceinline__ void ts_fetch_some(uint32_t at, const void* base, uint32_t lds, uint64_t mask) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(at), "s"(base), "s"(lds), "s"(mask) : "memory");
+}
+template <int ROR>
+__device__ __forceinline__ float ts_ror(float v) {   // rotation inside a row of 16 lanes
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 + ROR, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float ts_rounded(float v, int dtype) {   // to the result's type and back
+  return dtype == GGUF_DTYPE_F32 ? v : dtype == GGUF_DTYPE_F16 ? (float)(_Float16)v : bf16_to_f32(f32_to_bf16(v));
+}
+__device__ __forceinline__ void ts_store(void* Y, int64_t at, float v, const void* bias, int n, int dtype) {
+  if (dtype == GGUF_DTYPE_F16) ((_Float16*)Y)[at] = finish<_Float16>(v, (const _Float16*)bias, n);
+  else if (dtype == GGUF_DTYPE_BF16) ((bf16_t*)Y)[at] = finish<bf16_t>(v, (const bf16_t*)bias, n);
+  else ((float*)Y)[at] = finish<float>(v, (const float*)bias, n);
+}
+
+// Where the scales of block b of a chunk begin, in floats: XR per block, and a gap of sixteen behind every four blocks so
+// that threads that place four blocks each, one behind the other, meet different banks.  (Sums over whole fours of blocks.)
+template <int XR> __host__ __device__ __forceinline__ constexpr int ts_scale_at(int b) { return b * XR + (b >> 2) * 16; }
+
+// GATE: the first expert GEMM of a layer with its seam (Gate16): of four neighbouring column groups two are 32 features of
+// the gate half and two the same features of the up half; the sums meet in LDS and the workgroup finishes the q8_1
+// blocks of h from them.
+template <class F, int RT, bool GATE, bool SPLIT, int D>
+__global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_stream_kernel(const uint8_t* __restrict__ W, const char* __restrict__ ws,
+                                                                                  void* __restrict__ Y, TsArgs a, MoeArgs moe, Gate16 gate,
+                                                                                  int row_blocks, int total) {
+  static_assert(!GATE || (RT == 1 && !SPLIT), "a gated product takes its column groups whole, for 16 slots");
+  static_assert(D >= 2 && D <= 4, "one wait per number of panels requested behind the one at hand");
+  constexpr int NW = TS_NW, XR = 16 * RT, XR_LOG2 = RT == 1 ? 4 : 5;
+  constexpr int PPR_MIN = (F::PB + 15) / 16, PPR_MAX = (F::PB + 29) / 16;     // pieces of an aligned / of any panel row
+  constexpr int NI = (16 * (PPR_MAX | 1) + 63) / 64, FULL = 16 * PPR_MIN / 64;      // fetch instructions; those with all lanes on
+  extern __shared__ __align__(16) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4;
+
+  // ---- which rows, columns and panels
+  int wg = blockIdx.x;
+  const int total8 = total & ~7;                            // each of the 8 XCDs gets a contiguous run of workgroups
+  if (wg < total8) wg = (wg & 7) * (total8 >> 3) + (wg >> 3);
+  // (the blocks of one expert are neighbours: they share its weights)
+  const int col_wg = row_blocks == 1 ? wg : (int)__umulhi((uint32_t)wg, a.rb_inv), block = wg - col_wg * row_blocks;
+  const bool is_moe = moe.sorted_token_ids != nullptr;
+  if (is_moe) {
+    const int live = moe.num_tokens_post_padded[0], e = moe.expert_ids[block];
+    if (block * XR >= live || e < 0 || e > 255) return;     // (experts above 255: the reference's guard, moe.cuh:33)
+    W += (int64_t)e * moe.expert_stride;
+  }
+  const int KS = SPLIT ? 1 << a.ks_log2 : 1, CS = SPLIT ? NW >> a.ks_log2 : NW;
+  const int ks = SPLIT ? wave >> (3 - a.ks_log2) : 0, cs = SPLIT ? wave & (CS - 1) : wave;
+  const int passes = SPLIT ? 1 : a.passes;
+  const int groups = GATE ? gate.inner / 8 : (a.N + 15) / 16;   // (inner is a multiple of 32)
+  const int group0 = (col_wg * CS + cs) * passes;           // the first of this wave's column groups
+
+  // ---- LDS: [chunk buffers: quants [XR][pitch], scales and sums [blocks][XR]][fetch rings]; partial tiles over the chunks
+  const int PC = 1 << a.pc_log2, pitch = 256 * PC + 16;
+  const int xq_bytes = XR * pitch, xs_bytes = ts_scale_at<XR>(8 * PC) * 4 * (F::OFF ? 2 : 1), buf_bytes = xq_bytes + xs_bytes;
+  const int slot_bytes = 256 * a.ppr;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+  const int ring_off = a.nbuf * buf_bytes + wave * (D * slot_bytes);
+
+  // ---- fetching weights: piece number -> (row of the panel, 16-byte piece of it)
+  const uint32_t wmis = (uint32_t)((uintptr_t)W & 15);
+  const uint8_t* const wbase = W - wmis;
+  const uint32_t row_bytes = (uint32_t)(F::KQ ? a.np * F::PB : (a.K >> 5) * (F::PB / 8));
+  const int rows_all = GATE ? 2 * gate.inner : a.N;
+  const uint32_t last16 = ((uint32_t)(rows_all - 1) * a.w_pitch + wmis + row_bytes - 1) & ~15u;   // the last granule that holds bytes of W
+  uint32_t prow[NI], pc16[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int p = min(64 * i + lane, 16 * a.ppr - 1);
+    const uint32_t r = __umulhi((uint32_t)p, a.ppr_inv);
+    prow[i] = r * a.w_pitch;
+    pc16[i] = (uint32_t)min(p - (int)r * a.ppr, PPR_MAX - 1) * 16;   // (the piece that only spaces rows: the last again)
+  }
+  // byte offset of the first row of a column group, and of the last row a group may touch
+  const auto group_at = [&](int pass, uint32_t& last) -> uint32_t {
+    const int grp = group0 + pass;
+    if constexpr (GATE) {   // groups 4 u, 4 u + 1: features 32 u .. of the gate half; 4 u + 2, 4 u + 3: of the up half
+      const int half = (grp >> 1) & 1;
+      last = (uint32_t)((half + 1) * gate.inner - 1) * a.w_pitch;
+      return (uint32_t)(half * gate.inner + 32 * (grp >> 2) + 16 * (grp & 1)) * a.w_pitch;
+    } else {
+      last = (uint32_t)(a.N - 1) * a.w_pitch;
+      return (uint32_t)(16 * grp) * a.w_pitch;
+    }
+  };
+  const auto request = [&](int pass, int p, int slot) {
+    uint32_t last;
+    const uint32_t at = group_at(pass, last), off = (uint32_t)(p * F::PB) + wmis;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const uint32_t row = min(at + prow[i], last);
+      const uint32_t v = min(((row + off) & ~15u) + pc16[i], last16);
+      const uint32_t to = lds0 + ring_off + slot * slot_bytes + 1024 * i;
+      if (i < FULL) {
+        ts_fetch(v, wbase, to);
+      } else {   // (lanes past the panel's last piece stay out: their bytes would land in the next slot)
+        const int on = 16 * a.ppr - 64 * i;
+        ts_fetch_some(v, wbase, to, on >= 64 ? ~0ull : on <= 0 ? 0ull : (1ull << on) - 1);
+      }
+    }
+  };
+  // this wave's tasks, the panels of its column groups, and the next one to request
+  const int my_passes = max(0, min(passes, groups - group0));
+  const int np_mine = a.np > ks ? (a.np - ks + KS - 1) >> (SPLIT ? a.ks_log2 : 0) : 0;
+  const int tasks = np_mine * my_passes;
+  int rq_p = ks, rq_pass = 0, requested = 0;
+  const auto request_next = [&](int slot) {
+    if (requested >= tasks) return;
+    request(rq_pass, rq_p, slot);
+    ++requested;
+    rq_p += KS;
+    if (rq_p >= a.np) {
+      rq_p = ks;
+      ++rq_pass;
+    }
+  };
+
+  // ---- fetching activations.  Lane l knows where row l % XR of the tile begins; quants go to LDS directly, one row's
+  // 1 KB per request, scales and sums through registers (four blocks of a row per thread) so that LDS holds them block-major.
+  uint32_t row_at;
+  int pair_at = 0;                                          // MoE: the pair behind slot lane % XR
+  const int nb = a.Kp >> 5, nkb = a.K >> 5;
+  const auto fetch_quants = [&](int ch, int buf) {
+    const int parts_log2 = a.pc_log2 - 2;                   // KB of a row per chunk
+    for (int q = wave; q < XR << parts_log2; q += NW) {
+      const int row = q >> parts_log2, part = q & ((1 << parts_log2) - 1);
+      const uint32_t base = __builtin_amdgcn_readlane(row_at, row);
+      // (past the padded row's end: its last piece again)
+      const uint32_t at = min((uint32_t)(256 * PC * ch + 1024 * part + 16 * lane), (uint32_t)a.Kp - 16);
+      ts_fetch(base + at, ws, lds0 + buf * buf_bytes + row * pitch + 1024 * part);
+    }
+  };
+  constexpr int NS = 2;                                     // (row, four blocks, plane) items per thread, at most
+  u32x4_s sreg[NS];
+  const int items = (XR * 2 * PC) * (F::OFF ? 2 : 1);       // items, rows fastest
+  const auto scales_at = [&](int ch, int i) -> uint32_t {
+    const int it = tid + 64 * NW * i, row = it & (XR - 1), q = (it >> XR_LOG2) & (2 * PC - 1), plane = it >> (XR_LOG2 + 1 + a.pc_log2);
+    return __shfl(row_at, row) + a.Kp + (plane ? 4 * a.plane * nb : 0) + min(16 * (uint32_t)(2 * PC * ch + q), 4 * (uint32_t)nb - 16);
+  };
+  const auto place_scales = [&](int ch, int buf) {
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      const int it = tid + 64 * NW * i, row = it & (XR - 1), q = (it >> XR_LOG2) & (2 * PC - 1), plane = it >> (XR_LOG2 + 1 + a.pc_log2);
+      float* const to = (float*)(smem + buf * buf_bytes + xq_bytes) + plane * ts_scale_at<XR>(8 * PC) + row;
+      if (it < items)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t bits = sreg[i][e];   // (a bit cast applied to the vector element itself reads element 0)
+          to[ts_scale_at<XR>(4 * q) + e * XR] = 8 * PC * ch + 4 * q + e < nkb ? __uint_as_float(bits) : 0.0f;
+        }
+    }
+  };
+  // The first chunk's, counted by hand: between these two the registers belong to the loads (straight-line code).
+  const auto fetch_first_scales = [&]() {
+#pragma unroll
+    for (int i = 0; i < NS; ++i) asm volatile("global_load_dwordx4 %0, %1, %2" : "=&v"(sreg[i]) : "v"(scales_at(0, i)), "s"(ws) : "memory");
+  };
+  const auto first_scales_landed = [&]() {
+#pragma unroll
+    for (int i = 0; i < NS; ++i) asm volatile("" : "+v"(sreg[i]));
+  };
+
+  if (is_moe) {
+    // (the weights do not wait for the routing)
+    int id;
+    asm volatile("global_load_dword %0, %1, %2" : "=&v"(id) : "v"(4 * (uint32_t)(block * XR + (lane & (XR - 1)))), "s"(moe.sorted_token_ids) : "memory");
+#pragma unroll
+    for (int d = 0; d < D; ++d) request_next(d);
+    if (requested == D) ts_wait<D * NI>();
+    else ts_wait<0>();
+    asm volatile("" : "+v"(id));
+    pair_at = id;
+    row_at = (id < moe.num_pairs ? (moe.top_k == 1 ? (uint32_t)id : __umulhi((uint32_t)id, a.topk_inv)) : 0u) * a.ws_row_bytes;   // row 0 stands in for padding
+    fetch_first_scales();
+    fetch_quants(0, 0);
+    ts_wait<0>();
+  } else {
+    row_at = (uint32_t)min(block * XR + (lane & (XR - 1)), a.M - 1) * a.ws_row_bytes;
+    fetch_first_scales();
+    fetch_quants(0, 0);
+#pragma unroll
+    for (int d = 0; d < D; ++d) request_next(d);
+    if (requested == D) ts_wait<D * NI>();
+    else ts_wait<0>();
+  }
+  first_scales_landed();
+  place_scales(0, 0);
+  __syncthreads();
+
+  const v4i seed = {kSeedBits, kSeedBits, kSeedBits, kSeedBits};
+  const uint32_t half0 = g < 2 ? ~0u : 0u;                  // lanes that hold the first 16 values of a block
+  const auto store = [&](int m, int n, float v) {           // result row m of this workgroup's tile, feature n (all lanes together)
+    const int row = is_moe ? __shfl(pair_at, m) : block * XR + m;
+    if (n < a.N && row < (is_moe ? moe.num_pairs : a.M)) ts_store(Y, (int64_t)row * a.ldy + n, v, a.bias, n, a.dtype);
+  };
+  const int chunks = (a.np + PC - 1) >> a.pc_log2;
+  int t = 0, slot = 0;                                      // tasks done, ring slot of the next
+  f32x4 acc[RT], kept[4];                                   // kept (gated): the last four column groups' sums
+  for (int pass = 0; pass < passes; ++pass) {
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) acc[rt] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+  const int pass_end = min(tasks, (pass + 1) * np_mine);
+  int p = ks;
+  for (int ch = 0; ch < chunks; ++ch) {
+    const bool more = ch + 1 < chunks;
+    const int buf = a.nbuf == 2 ? ch & 1 : 0;
+    if constexpr (SPLIT) {
+      if (more) {
+        // (these loads are the compiler's to wait for, which will wait for every panel in flight along with them)
+#pragma unroll
+        for (int i = 0; i < NS; ++i) sreg[i] = *(const u32x4_s*)(ws + scales_at(ch + 1, i));
+        if (a.nbuf == 2) fetch_quants(ch + 1, buf ^ 1);
+      }
+    }
+    const char* const xq = smem + buf * buf_bytes;
+    const float* const xd = (const float*)(xq + xq_bytes);
+    for (; t < pass_end && p < (ch + 1) << a.pc_log2; p += KS) {
+      const int pl = p - (ch << a.pc_log2);                 // panel of the chunk
+      u32x4_s xa[RT][4];
+      float so[RT][2];
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) xa[rt][i] = *(const u32x4_s*)(xq + (16 * rt + c) * pitch + 256 * pl + 64 * i + 16 * g);
+        if constexpr (F::OFF) {
+          const float* const sums = xd + ts_scale_at<XR>(8 * PC) + ts_scale_at<XR>(8 * pl) + g * XR + 16 * rt + c;
+          so[rt][0] = sums[0];
+          so[rt][1] = sums[ts_scale_at<XR>(4)];
+        }
+      }
+      const int left = nkb - 8 * p;                         // blocks of the panel inside the row
+      // Loads return in order: the panel has landed once no more are outstanding than the panels behind it asked for.
+      const int ahead = requested - t - 1;
+      if (D > 3 && ahead >= 3) ts_wait<3 * NI>();
+      else if (D > 2 && ahead >= 2) ts_wait<2 * NI>();
+      else if (ahead >= 1) ts_wait<NI>();
+      else ts_wait<0>();
+      uint32_t last;
+      const uint32_t w_at = min(group_at(pass, last) + c * a.w_pitch, last) + (uint32_t)(p * F::PB) + wmis;
+      F w;
+      w.read(smem + ring_off + slot * slot_bytes + c * (16 * a.ppr), F::PB % 16 == 0 && a.ppr == F::PB / 16 ? 0u : w_at & 15, g);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot may be filled again
+      request_next(slot);
+      ++t;
+      slot = slot + 1 == D ? 0 : slot + 1;
+
+      float dw[8 * (32 / F::G)];
+      w.ready();
+      w.scales(dw);
+      // (opaque to the compiler, which would keep both masked copies of all operands over the column groups and spill)
+      uint32_t first = half0;
+      asm volatile("" : "+v"(first));
+      if (!F::KQ && left < 8) {
+#pragma unroll
+        for (int b = 0; b < 8; ++b) dw[b] = b < left ? dw[b] : 0.0f;   // (bytes behind the row's end need not be a number)
+      }
+      float m0 = 0.0f, m1 = 0.0f;
+      if constexpr (F::OFF) {
+        w.mins(g, m0, m1);
+        if (!F::KQ && left < 8) { m0 = g < left ? m0 : 0.0f; m1 = 4 + g < left ? m1 : 0.0f; }
+      }
+      // (the offsets of four blocks, then their products: the partial sums stay small, and so does what they round off)
+      f32x4 part[RT];
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+        part[rt] = F::OFF ? __builtin_amdgcn_mfma_f32_16x16x4f32(so[rt][0], -m0, (f32x4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0) : acc[rt];
+#pragma unroll
+      for (int b = 0; b < 8; ++b) {
+        if (F::OFF && b == 4) {
+#pragma unroll
+          for (int rt = 0; rt < RT; ++rt) part[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(so[rt][1], -m1, part[rt], 0, 0, 0);
+        }
+        const uint2 q = w.codes(b, g);
+        const long bv = (long)(((uint64_t)q.y << 32) | q.x);
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+          const f32x4 d8 = *(const f32x4*)(xd + ts_scale_at<XR>(8 * pl) + ts_scale_at<XR>(b) + 16 * rt + 4 * g);
+          const uint32_t alo = xa[rt][b >> 1][2 * (b & 1)], ahi = xa[rt][b >> 1][2 * (b & 1) + 1];
+          if constexpr (F::G == 32) {
+            const float nsd = -kSeed * dw[b];
+            const v4i s = __builtin_amdgcn_mfma_i32_16x16x32_i8((long)(((uint64_t)ahi << 32) | alo), bv, seed, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) part[rt][r] = __builtin_fmaf(seeded_times(s[r], dw[b], nsd), d8[r], part[rt][r]);
+          } else {
+            // a scale per 16 values: the activations of either half of the block, the other half's lanes zeroed
+            const long a0 = (long)(((uint64_t)(ahi & first) << 32) | (alo & first));
+            const long a1 = (long)(((uint64_t)(ahi & ~first) << 32) | (alo & ~first));
+            const float n0 = -kSeed * dw[2 * b], n1 = -kSeed * dw[2 * b + 1];
+            const v4i s0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a0, bv, seed, 0, 0, 0);
+            const v4i s1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a1, bv, seed, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              part[rt][r] = __builtin_fmaf(seeded_times(s0[r], dw[2 * b], n0), d8[r], part[rt][r]);
+              part[rt][r] = __builtin_fmaf(seeded_times(s1[r], dw[2 * b + 1], n1), d8[r], part[rt][r]);
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) acc[rt] = F::OFF ? acc[rt] + part[rt] : part[rt];
+    }
+    // ---- the next chunk of activations
+    if constexpr (SPLIT) {
+      if (more) {
+        if (a.nbuf == 1) {
+          __syncthreads();                                  // every wave is done with this one
+          fetch_quants(ch + 1, 0);
+        }
+        ts_wait<0>();
+        place_scales(ch + 1, a.nbuf == 2 ? buf ^ 1 : 0);
+        __syncthreads();
+      }
+    }
+  }
+  if constexpr (GATE) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) kept[i] = kept[i + 1];
+    kept[3] = acc[0];
+  } else if constexpr (!SPLIT) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) store(16 * rt + 4 * g + r, 16 * (group0 + pass) + c, acc[rt][r]);
+  }
+  }
+
+  if constexpr (GATE) {
+    // One (unit of 32 features, result register r) per wave and turn: a lane has slot 4 g + r of features 16 i + c, i = 0, 1:
+    // sums rounded as the operator stores them, activated, and quantized as q8_1_quantize8 does -- amax and the sum over
+    // the 32 features by the same butterfly (16 apart in the lane, then 8, 4, 2, 1 as rotations inside the row of 16 lanes,
+    // whose partners agree at each step).
+    // (the sums go over the activations, so that two workgroups still fit a CU's LDS)
+    __syncthreads();
+    float* const sums = (float*)smem;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (i >= 4 - passes) *(f32x4*)(sums + ((wave * passes + i - (4 - passes)) * 64 + lane) * 4) = kept[i];
+    __syncthreads();
+    for (int it = wave; it < 2 * passes * 4; it += NW) {
+      const int u = it >> 2, r = it & 3, unit = 2 * passes * col_wg + u;
+      if (32 * unit >= gate.inner) break;
+      const int pair = __shfl(pair_at, 4 * g + r);
+      float h[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const float gv = ts_rounded(sums[((4 * u + i) * 64 + lane) * 4 + r], a.dtype);
+        const float uv = ts_rounded(sums[((4 * u + 2 + i) * 64 + lane) * 4 + r], a.dtype);
+        h[i] = a.dtype == GGUF_DTYPE_F32 ? gate1<float>(gv, uv, gate.act) : a.dtype == GGUF_DTYPE_F16 ? gate1<_Float16>(gv, uv, gate.act) : gate1<bf16_t>(gv, uv, gate.act);
+      }
+      float amax = fmaxf(fabsf(h[0]), fabsf(h[1])), sum = h[0] + h[1];
+      amax = fmaxf(amax, ts_ror<8>(amax));
+      sum += ts_ror<8>(sum);
+      amax = fmaxf(amax, ts_ror<4>(amax));
+      sum += ts_ror<4>(sum);
+      amax = fmaxf(amax, ts_ror<2>(amax));
+      sum += ts_ror<2>(sum);
+      amax = fmaxf(amax, ts_ror<1>(amax));
+      sum += ts_ror<1>(sum);
+      const float d = amax / 127.0f, dd = amax == 0.0f ? 1.0f : d;
+      int q[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) q[i] = (int)roundf(h[i] / dd);
+      int isum = q[0] + q[1];
+      isum += dpp_mov_i<0x128>(isum);
+      isum += dpp_mov_i<0x124>(isum);
+      isum += dpp_mov_i<0x122>(isum);
+      isum += dpp_mov_i<0x121>(isum);
+      if (pair < moe.num_pairs) {
+        char* const row = gate.rows + (int64_t)pair * gate.row_bytes;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) row[q8_permuted(32 * unit + 16 * i + (c & 8)) + (c & 7)] = (char)q[i];
+        if (c == 0) {
+          float* fd = (float*)(row + gate.kp);
+          const int nbh = gate.kp >> 5;
+          const float dh = (float)(_Float16)d;
+          fd[unit] = dh;
+          fd[nbh + unit] = (float)(_Float16)sum;
+          fd[2 * nbh + unit] = dh * (float)isum;
+        }
+      }
+    }
+    return;
+  }
+  if constexpr (SPLIT) {
+    // ---- the KS partial tiles of every column group, added in the order of K
+    float* const red = (float*)smem;                        // [NW][RT][64] of four floats, over the activations
+    __syncthreads();
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) *(f32x4*)(red + ((wave * RT + rt) * 64 + lane) * 4) = acc[rt];
+    __syncthreads();
+    constexpr int per_cs = RT * 64;
+    for (int i = tid; i < CS * per_cs; i += 64 * NW) {
+      const int s = i / per_cs, rest = i - s * per_cs;      // column slice; (rt, lane) of its tiles
+      f32x4 v = *(const f32x4*)(red + (s * per_cs + rest) * 4);
+      for (int z = 1; z < KS; ++z) v += *(const f32x4*)(red + ((z * CS + s) * per_cs + rest) * 4);
+      const int l = rest & 63, rt = rest >> 6;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) store(16 * rt + 4 * (l >> 4) + r, 16 * (col_wg * CS + s) + (l & 15), v[r]);
+    }
+  }
+}
+
+static inline size_t ts_chunk_bytes(int rt, bool off, int pc) {
+  return (size_t)16 * rt * (256 * pc + 16) + (size_t)(8 * pc * 16 * rt + 2 * pc * 16) * 4 * (off ? 2 : 1);
+}
+
+template <class F, int RT, bool GATE, bool SPLIT, int D>
+static int ts_launch_d(const TsCall& c, int ks, const TsArgs& a, size_t lds, hipStream_t stream) {
+  auto kern = tile_stream_kernel<F, RT, GATE, SPLIT, D>;
+  if (lds > 64 * 1024) {
+    static std::atomic<uint64_t> done{0};
+    allow_large_lds(kern, 160 * 1024, done);
+  }
+  const int cols = GATE ? c.gate.inner / 8 : (c.N + 15) / 16, per_wg = TS_NW / ks * a.passes;
+  const int64_t total = (int64_t)((cols + per_wg - 1) / per_wg) * c.row_blocks;
+  // the quotients by reciprocal are exact while dividend times divisor stays below 2^32
+  if (total * c.row_blocks > 0xFFFFFFFFll || (int64_t)c.moe.num_pairs * (c.moe.top_k > 0 ? c.moe.top_k : 1) > 0xFFFFFFFFll) return GGUF_ERR_SHAPE;
+  hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(64 * TS_NW), lds, stream, (const uint8_t*)c.W, (const char*)c.ws, c.Y, a, c.moe, c.gate,
+                     c.row_blocks, (int)total);
+  return launch_status();
+}
+
+// Column groups a wave walks one after the other, given the rounds of workgroups on the chip with one each.  A second
+// group saves a beginning (4 to 6 us, as long as about six panels) but makes the last round longer: it pays from four
+// rounds on (64 experts of Q4_0, 300 tokens: 168 -> 159 us the layer; 128 experts, 64 tokens, three rounds: 106 -> 113),
+// and earlier where a group has only a few panels.
+static inline int ts_passes(int np, double rounds) {
+  int passes = rounds >= 4.0 ? 2 : 1;
+  while (passes < 4 && np * passes < 6 && rounds >= 1.5 * passes) passes *= 2;
+  return passes;
+}
+
+template <class F, int RT, bool GATE, bool SPLIT>
+static int ts_launch(const TsCall& c, int ks, hipStream_t stream) {
+  const int np = (c.K + 255) / 256, qk = F::KQ ? 256 : 32, bs = F::KQ ? F::PB : F::PB / 8;
+  const int64_t pitch = c.w_pitch ? c.w_pitch : (int64_t)(c.K / qk) * bs;
+  // pieces per row and panel: one more where a panel may begin inside one
+  const bool aligned = F::PB % 16 == 0 && pitch % 16 == 0 && (uintptr_t)c.W % 16 == 0 && (!c.moe.sorted_token_ids || c.moe.expert_stride % 16 == 0);
+  // (an odd number, so that the same field of 16 rows lies in different banks: [23376,1856] of Q4_0, 16 rows of X 23.2 -> 19.2 us)
+  const int ppr = (aligned ? F::PB / 16 : (F::PB + 29) / 16) | 1, top_k = c.moe.top_k > 0 ? c.moe.top_k : 1;
+  const auto bytes = [&](int pc, int nbuf, int d) { return nbuf * ts_chunk_bytes(RT, F::OFF, pc) + (size_t)TS_NW * d * 256 * ppr + 16; };
+  const size_t room = 160 * 1024;
+  int pc_log2 = 2, nbuf = 1;
+  while (pc_log2 < 4 && (1 << pc_log2) < np) ++pc_log2;
+  if (!SPLIT) {
+    if ((1 << pc_log2) < np || bytes(1 << pc_log2, 1, 2) > room) return GGUF_NOT_TAKEN;   // all of K in LDS
+  } else if (np > 8 || bytes(1 << pc_log2, 1, 2) > room) {
+    // two chunks, the second fetched while the first is multiplied, where that gives every wave of a split a panel
+    pc_log2 = 3;
+    while (pc_log2 > 2 && bytes(1 << pc_log2, 2, 2) > room) --pc_log2;
+    nbuf = 2;
+    if ((1 << pc_log2) < ks || bytes(1 << pc_log2, 2, 2) > room) {
+      nbuf = 1;
+      pc_log2 = 4;
+      while (pc_log2 > 2 && bytes(1 << pc_log2, 1, 2) > room) --pc_log2;
+    }
+  }
+  if ((1 << pc_log2) * 2 * 16 * RT * (F::OFF ? 2 : 1) > 2 * 64 * TS_NW) return GGUF_NOT_TAKEN;   // (two items of scales per thread)
+  // (two workgroups per CU overlap their beginnings and ends, and have as many panels in flight between them)
+  int d = RT == 1 && bytes(1 << pc_log2, nbuf, 2) <= room / 2 ? 2 : 4;
+  while (d > 2 && bytes(1 << pc_log2, nbuf, d) > room) --d;
+  size_t lds = bytes(1 << pc_log2, nbuf, d);                // (16 more: the cut of a last field may touch the word behind its row)
+  if (SPLIT && lds < (size_t)TS_NW * RT * 1024) lds = (size_t)TS_NW * RT * 1024;
+  if (lds > room) return GGUF_NOT_TAKEN;
+  const int cols = GATE ? c.gate.inner / 8 : (c.N + 15) / 16;
+  const int passes = SPLIT ? 1 : ts_passes(np, c.live_blocks * cols / TS_NW / (lds <= room / 2 ? 512.0 : 256.0));
+  const TsArgs a = {c.M, c.N, c.K, (int)q8_kp(c.K), (uint32_t)pitch, (uint32_t)q8_row_bytes(c.K), np, 31 - __builtin_clz(ks), ppr, pc_log2, nbuf, passes,
+                    (uint32_t)((0x100000000ull + ppr - 1) / ppr), (uint32_t)((0x100000000ull + c.row_blocks - 1) / c.row_blocks),
+                    (uint32_t)((0x100000000ull + top_k - 1) / top_k), c.gemv_sums ? 2 : 1, c.dtype, c.ldy ? c.ldy : (int64_t)c.N, c.bias};
+  switch (d) {
+    case 4: return ts_launch_d<F, RT, GATE, SPLIT, 4>(c, ks, a, lds, stream);
+    case 3: return ts_launch_d<F, RT, GATE, SPLIT, 3>(c, ks, a, lds, stream);
+    default: return ts_launch_d<F, RT, GATE, SPLIT, 2>(c, ks, a, lds, stream);
+  }
+}
+
+// KS waves share a column group where the output has fewer groups than the chip has waves: rounds of workgroups x (the
+// panels of a wave + a beginning and an end worth about five).
+static inline int ts_ks(int np, double groups) {
+  int best = 1;
+  double best_cost = 1e30;
+  for (int ks = 1; ks <= TS_NW; ks <<= 1) {
+    const double wgs = ceil(groups * ks / TS_NW), cost = ((np + ks - 1) / ks + 5.0) * ceil(wgs / 256.0);
+    if (cost < 0.97 * best_cost) { best_cost = cost; best = ks; }
+  }
+  return best;
+}
+
+template <class F, int RT>
+static int ts_run_rt(const TsCall& c, hipStream_t stream) {
+  const int np = (c.K + 255) / 256;
+  if (c.gate.rows) {
+    if constexpr (RT == 1) return ts_launch<F, 1, true, false>(c, 1, stream);
+    return GGUF_NOT_TAKEN;
+  }
+  const int ks = ts_ks(np, c.live_blocks * ((c.N + 15) / 16));
+  if (ks == 1 && np <= 16) {
+    const int rc = ts_launch<F, RT, false, false>(c, 1, stream);
+    if (rc != GGUF_NOT_TAKEN) return rc;
+  }
+  return ts_launch<F, RT, false, true>(c, ks, stream);
+}
+
+template <class F>
+static int ts_run(const TsCall& c, hipStream_t stream) {
+  return c.rt == 1 ? ts_run_rt<F, 1>(c, stream) : c.rt == 2 ? ts_run_rt<F, 2>(c, stream) : GGUF_NOT_TAKEN;
+}
+
+}  // namespace gguf
