@@ -1,0 +1,46 @@
+"""The prefill GEMM on the half-precision matrix unit (csrc/mmq_f_core.h) at the edges of its tiles and of the runs of
+super-blocks its workgroups share, and on the largest whole numbers its operands and sums have to hold, against the CPU
+oracle."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import gguf_oracle as o
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(w, x, qtype, n, pad=0, bias=None):
+    from vllm_gguf_plugin_prism_amd import ops
+    wd = torch.zeros(n, w.shape[1] + pad, dtype=torch.uint8, device="cuda")[:, :w.shape[1]]
+    wd.copy_(torch.from_numpy(w))
+    b = torch.from_numpy(bias).cuda() if bias is not None else None
+    y = ops.ggml_mul_mat_a8(wd, torch.from_numpy(x).cuda(), qtype, n, bias=b).cpu().numpy()
+    want = o.mul_mat_a8(w, x, qtype, n, "mmq") + (bias if bias is not None else 0.0)
+    assert o.rel_l2(y, want) <= 1e-5
+
+
+# one super-block; one row over a tile in either direction with tiles cut into runs, a padded pitch; runs that begin and
+# end inside tiles; more tiles than CUs (whole rounds and a shared rest)
+@pytest.mark.parametrize("qtype", [o.Q4_K, o.Q5_K, o.Q6_K])
+@pytest.mark.parametrize("m,n,k,pad", [(448, 2048, 256, 0), (513, 2049, 1024, 2), (460, 2176, 2816, 0), (600, 11000, 512, 6)])
+def test_tile_edges(qtype, m, n, k, pad):
+    rng = np.random.default_rng(m + k)
+    _check(o.make_weights(rng, qtype, n, k), rng.standard_normal((m, k)).astype(np.float32) + 0.3, qtype, n, pad,
+           rng.standard_normal(n).astype(np.float32))
+
+
+@pytest.mark.parametrize("qtype", [o.Q4_K, o.Q5_K, o.Q6_K])
+def test_largest_sums_are_exact(qtype):
+    rng = np.random.default_rng(qtype)
+    n, k, m = 2048, 512, 448
+    w = o.make_weights(rng, qtype, n, k).reshape(n, k // 256, -1)
+    if qtype == o.Q6_K:
+        w[:, :, :192], w[:, :, 192:208] = 0, 0x80          # codes -32, scales -128
+        w[1::2, :, :208] = 0xFF                            # codes 31, scales -1
+        w[1::4, :, 192:208] = 0x7F                         # codes 31, scales 127
+    else:
+        w[:, :, 4:] = 0xFF                                 # scales and mins 63, codes 15 or 31
+    x = np.where(rng.random((m, 1)) < 0.5, 1.0, -1.0).astype(np.float32) * (1.0 + np.arange(m, dtype=np.float32)[:, None] % 7) * np.ones((1, k), np.float32)
+    x[:, ::5] *= 0.97
+    _check(w.reshape(n, -1), x, qtype, n)

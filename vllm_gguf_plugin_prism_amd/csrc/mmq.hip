@@ -25,6 +25,7 @@
 // The same kernel runs the grouped MoE contraction (reference: csrc/gguf/moe.cuh:5-129):
 // token rows are gathered through sorted_token_ids, the weight base moves to the block's
 // expert, and results scatter to the rows the slots name.
+#include "mmq_f.h"
 #include "tile_stream.h"
 #include "mmq_formats.h"
 #include "q8_1_device.h"
@@ -822,7 +823,12 @@ extern "C" int64_t gguf_mmq_workspace_bytes_engine(int64_t M, int64_t N, int64_t
   if (engine == GGUF_MMQ_HALF) return mmq_rows_bytes(M, K, true) + gguf::mmq_half_partial_bytes((int)M, (int)N, (int)K);
   const int64_t pi = gguf::mmq_int_partial_bytes((int)M, (int)N, (int)K);
   const int64_t p16 = M <= gguf::MMQ_ROWS16_MAX ? gguf::mmq_rows16_partial_bytes((int)M, (int)N, (int)K) : 0;
-  return mmq_rows_bytes(M, K, false) + (pi > p16 ? pi : p16);
+  int64_t behind = pi > p16 ? pi : p16;
+  if (M > gguf::MMQ_ROWS16_MAX && K % 256 == 0) {   // (the type is not known here: room for the engine of the super-block formats, too)
+    const int64_t pf = gguf::mmqf_rows_bytes(M, K) + gguf::mmqf_plan((int)M, (int)N, (int)K, INT64_MAX).partial_bytes();
+    if (pf > behind) behind = pf;
+  }
+  return mmq_rows_bytes(M, K, false) + behind;
 }
 
 // room for either engine
@@ -905,6 +911,14 @@ int gguf::mmq_linear_impl(const void* W, int64_t w_row_pitch_bytes, const void* 
     const int rc = quantize_q8_1(x, xdtype, q8_workspace, M, K, s, 0, half_plane);
     if (rc != GGUF_OK) return rc;
     return mmq_half(W, q8_workspace, Y, xdtype, type, (int)M, (int)N, (int)K, partial, partial_bytes, s, la);
+  }
+  const int64_t half_rows = mmqf_rows_bytes(M, K);
+  if (partial_bytes >= half_rows && ((uintptr_t)partial & 15) == 0 && mmqf_takes(type, M, N, K, w_row_pitch_bytes)) {
+    const MmqfRows rows = mmqf_rows(partial, M, K);
+    int rc = quantize_whole(x, xdtype, rows, M, K, s);
+    if (rc != GGUF_OK) return rc;
+    const MmqfCall c = {W, rows, Y, xdtype, (int)M, (int)N, (int)K, (float*)((char*)partial + half_rows), partial_bytes - half_rows, la};
+    return mmqf(type, c, s);
   }
   int rc = quantize_q8_1(x, xdtype, q8_workspace, M, K, s);
   if (rc != GGUF_OK) return rc;

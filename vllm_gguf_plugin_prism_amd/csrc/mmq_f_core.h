@@ -1,0 +1,524 @@
+// Prefill GEMM on the super-block formats: integer arithmetic on the half-precision matrix unit.
+//
+//   Y[m, n] = sum_sb  d[n, sb] * ( sum_b  d8[m, b] * S[m, n, b] )  ( - dmin[n, sb] * sum_b  mn[n, b] * s8[m, b] )
+//   S[m, n, b] = sum over the 32 values of block b of  q8[m, k] * (sc[n, group of k] * q[n, k])         (exact)
+//
+// What bounds the contraction is the vector work per matrix result: a q8_1 block is 32 values deep and every result of a
+// block has to be scaled before the next one is added.  With the weight's own scale in that factor (mmq_i_core.h: int8
+// operands, d8 * d * sc per block) that is two or three multiply-adds per result and block, four where a weight scale
+// covers 16 values: 41 to 90 ns per 32 x 32 x 32 block and SIMD at full rate, of which the matrix unit needs 14.  Here the
+// integer scale sc goes into the weight operand.  sc * q is a whole number of at most 11 bits (Q4_K 63 * 15, Q5_K
+// 63 * 31), which half precision holds exactly; so are the quants of X; and the block's sum stays below 2^24, so the fp32
+// accumulator of v_mfma_f32_32x32x16_f16 holds it exactly, too, and hands it over as a float.  One multiply-add per result
+// and block is left (by d8, which is one register: a lane holds one row of X), and one per result and super-block for d:
+// 34 ns per 32 x 32 x 32 block.  Q6_K's products have 13 bits: two operands, q * (sc & ~15) and q * (sc & 15), 56 ns.
+// The offset term is a contraction over the eight blocks of a super-block of exact halves (the mins are 6-bit whole
+// numbers, the stored sums are halves): one more matrix instruction per super-block.
+//
+// Work split: workgroup tiles of 256 rows of X by 128 weight rows, eight waves of 64 x 64 (four accumulators of 32 x 32,
+// each twice: the super-block's sum and the total).  K in steps of 64: the rows of X (whole numbers in half precision,
+// written by the quantizer) go straight to LDS (global_load_lds, 16-byte pieces, the piece number xored with the row's so
+// that the operand reads meet all banks), the packed weights of the next step through registers, decoded once per
+// workgroup.  Two buffers, one barrier per step.  Whole rounds of tiles have a workgroup per tile; the super-blocks of the
+// tiles behind them are dealt in equal runs to all CUs (192 tiles on 256 CUs: 343 -> 288 us).
+//
+// Measured against the int8 engine, us per call with the quantizer: [4096,14336] Q4_K, 1531 rows 404 -> 288, 512 rows
+// 148 -> 107; [18944,3584] 512 rows 179 -> 139; Q6_K [4096,14336] 1531 rows 462 -> 389, [18944,3584] 512 rows 177 -> 176.
+// What bounds it now is power: on random operands the clock falls to about 2.0 GHz, at which the matrix instructions,
+// the multiply-adds and the operand reads of a step take about 0.45 us each; a step takes 1.2 us.  Tried and slower: four
+// waves per workgroup and two workgroups per CU (decoding twice), the two waves of a SIMD decoding at different times,
+// the fetches of X in front of the operand reads or spread over the step.
+#pragma once
+#include "mmq_formats.h"
+#include "mmq_f.h"
+
+namespace gguf {
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4_m __attribute__((ext_vector_type(4)));
+typedef float f32x2_m __attribute__((ext_vector_type(2)));
+
+// Two whole numbers below 1024 out of the low bytes (or nibbles) of the halves of v as 1024 + x each.
+__device__ __forceinline__ f16x2 magic2(uint32_t v) { return __builtin_bit_cast(f16x2, v | 0x64006400u); }
+__device__ __forceinline__ uint32_t bits2(f16x2 v) { return __builtin_bit_cast(uint32_t, v); }
+__device__ __forceinline__ f16x2 twice(_Float16 v) { return (f16x2){v, v}; }
+
+// Packed formats.  A step is quarter j of a super-block: blocks 2 j and 2 j + 1.  A thread decodes part p of a row's step:
+// values 8 p .. 8 p + 7 of both blocks, each as eight halves in the order of the rows of X (of four neighbours 0, 2, 1, 3).
+//   Head     what it takes from the super-block's header, loaded once per super-block; Scales: the same, unpacked
+//   PLANES   operands per weight;  OFF: the format has mins
+struct FQ4_K {
+  static constexpr int BS = 144, PLANES = 1;
+  static constexpr bool OFF = true;
+  struct Head { uint4 h; };
+  struct Scales { uint32_t s[2]; };
+  struct Raw { uint2 q; };
+  static __device__ __forceinline__ Head head(const uint8_t* sb) { return {ld<uint4>(sb)}; }
+  static __device__ __forceinline__ Raw fetch(const uint8_t* sb, int j, int p) { return {ld<uint2>(sb + 16 + 32 * j + 8 * p)}; }
+  static __device__ __forceinline__ Scales scales(const Head& hd) {
+    return {{hd.h.y & 0x3F3F3F3Fu, (hd.h.w & 0x0F0F0F0Fu) | ((hd.h.y >> 2) & 0x30303030u)}};
+  }
+  static __device__ __forceinline__ float d(const Head& hd) { return (float)__builtin_bit_cast(_Float16, (uint16_t)(hd.h.x & 0xFFFF)); }
+  static __device__ __forceinline__ float dmin(const Head& hd) { return (float)__builtin_bit_cast(_Float16, (uint16_t)(hd.h.x >> 16)); }
+  static __device__ __forceinline__ uint4 mins(const Head& hd) {   // eight halves
+    const uint32_t m[2] = {hd.h.z & 0x3F3F3F3Fu, ((hd.h.w >> 4) & 0x0F0F0F0Fu) | ((hd.h.z >> 2) & 0x30303030u)};
+    const f16x2 k = twice((_Float16)1024.0f);
+    uint32_t o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      o[i] = bits2(magic2(__builtin_amdgcn_perm(0u, m[i >> 1], i & 1 ? 0x0c030c02u : 0x0c010c00u)) - k);
+    return make_uint4(o[0], o[1], o[2], o[3]);
+  }
+  // the scales of blocks 2 j and 2 j + 1
+  template <int J> static __device__ __forceinline__ void pair(const Scales& sc, f16x2& s0, f16x2& s1) {
+    const uint32_t w = sc.s[J >> 1];
+    const f16x2 k = twice((_Float16)1024.0f);
+    s0 = magic2(__builtin_amdgcn_perm(0u, w, J & 1 ? 0x0c020c02u : 0x0c000c00u)) - k;
+    s1 = magic2(__builtin_amdgcn_perm(0u, w, J & 1 ? 0x0c030c03u : 0x0c010c01u)) - k;
+  }
+  template <int J> static __device__ __forceinline__ void decode(const Raw& r, const Scales& sc, int, uint4 (&lo)[1], uint4 (&hi)[1]) {
+    f16x2 s0, s1;
+    pair<J>(sc, s0, s1);
+    const f16x2 k = twice((_Float16)-1024.0f), n0 = s0 * k, n1 = s1 * k;   // (exact: six bits times a power of two)
+    uint32_t l[4], h[4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t a = i ? r.q.y : r.q.x, b = a >> 4;
+      l[2 * i] = bits2(__builtin_elementwise_fma(magic2(a & 0x000F000Fu), s0, n0));
+      l[2 * i + 1] = bits2(__builtin_elementwise_fma(magic2((a >> 8) & 0x000F000Fu), s0, n0));
+      h[2 * i] = bits2(__builtin_elementwise_fma(magic2(b & 0x000F000Fu), s1, n1));
+      h[2 * i + 1] = bits2(__builtin_elementwise_fma(magic2((b >> 8) & 0x000F000Fu), s1, n1));
+    }
+    lo[0] = make_uint4(l[0], l[1], l[2], l[3]);
+    hi[0] = make_uint4(h[0], h[1], h[2], h[3]);
+  }
+};
+
+struct FQ5_K : FQ4_K {   // Q4_K with a fifth bit, bit b of qh[k] for block b
+  static constexpr int BS = 176;
+  struct Raw { uint2 q, h; };
+  static __device__ __forceinline__ Raw fetch(const uint8_t* sb, int j, int p) {
+    return {ld<uint2>(sb + 48 + 32 * j + 8 * p), ld<uint2>(sb + 16 + 8 * p)};
+  }
+  template <int J> static __device__ __forceinline__ void decode(const Raw& r, const Scales& sc, int, uint4 (&lo)[1], uint4 (&hi)[1]) {
+    f16x2 s0, s1;
+    pair<J>(sc, s0, s1);
+    const f16x2 k = twice((_Float16)-1024.0f), n0 = s0 * k, n1 = s1 * k;
+    uint32_t l[4], h[4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t a = i ? r.q.y : r.q.x, t = i ? r.h.y : r.h.x;
+      const uint32_t a0 = (a & 0x0F0F0F0Fu) | (J < 2 ? (t << (4 - 2 * J)) & 0x10101010u : (t >> (2 * J - 4)) & 0x10101010u);
+      const uint32_t a1 = ((a >> 4) & 0x0F0F0F0Fu) | (J < 2 ? (t << (3 - 2 * J)) & 0x10101010u : (t >> (2 * J - 3)) & 0x10101010u);
+      l[2 * i] = bits2(__builtin_elementwise_fma(magic2(a0 & 0x00FF00FFu), s0, n0));
+      l[2 * i + 1] = bits2(__builtin_elementwise_fma(magic2((a0 >> 8) & 0x00FF00FFu), s0, n0));
+      h[2 * i] = bits2(__builtin_elementwise_fma(magic2(a1 & 0x00FF00FFu), s1, n1));
+      h[2 * i + 1] = bits2(__builtin_elementwise_fma(magic2((a1 >> 8) & 0x00FF00FFu), s1, n1));
+    }
+    lo[0] = make_uint4(l[0], l[1], l[2], l[3]);
+    hi[0] = make_uint4(h[0], h[1], h[2], h[3]);
+  }
+};
+
+struct FQ6_K {
+  static constexpr int BS = 210, PLANES = 2;
+  static constexpr bool OFF = false;
+  struct Head { uint32_t d; };
+  struct Scales {};
+  struct Raw { uint2 l0, l1, h; uint32_t s; };   // s: the scales of the step's four groups
+  static __device__ __forceinline__ Head head(const uint8_t* sb) { return {ld<uint16_t>(sb + 208)}; }
+  static __device__ __forceinline__ Raw fetch(const uint8_t* sb, int j, int p) {
+    const uint8_t* l = sb + 64 * (j >> 1) + 8 * p;
+    return {ld<uint2>(l), ld<uint2>(l + 32), ld<uint2>(sb + 128 + 32 * (j >> 1) + 8 * p), ld<uint32_t>(sb + 192 + 4 * j)};
+  }
+  static __device__ __forceinline__ Scales scales(const Head&) { return {}; }
+  static __device__ __forceinline__ float d(const Head& hd) { return (float)__builtin_bit_cast(_Float16, (uint16_t)hd.d); }
+  static __device__ __forceinline__ float dmin(const Head&) { return 0.0f; }
+  static __device__ __forceinline__ uint4 mins(const Head&) { return make_uint4(0, 0, 0, 0); }
+  // four 6-bit codes -> (code - 32) * (sc & ~15) and (code - 32) * (sc & 15), whole numbers of 10 bits (times 16) and 9 bits
+  static __device__ __forceinline__ void planes(uint32_t v, f16x2 sh, f16x2 sl, uint32_t& h0, uint32_t& h1, uint32_t& l0, uint32_t& l1) {
+    const f16x2 k = twice((_Float16)1056.0f);
+    const f16x2 a = magic2(v & 0x00FF00FFu) - k, b = magic2((v >> 8) & 0x00FF00FFu) - k;
+    h0 = bits2(a * sh);
+    h1 = bits2(b * sh);
+    l0 = bits2(a * sl);
+    l1 = bits2(b * sl);
+  }
+  template <int J> static __device__ __forceinline__ void decode(const Raw& r, const Scales&, int p, uint4 (&lo)[2], uint4 (&hi)[2]) {
+    // scales of the values of this part: group p / 2 of blocks 2 j and 2 j + 1
+    const uint32_t w = r.s;
+    const int c0 = (int)(int8_t)((w >> (8 * (p >> 1))) & 0xFF), c1 = (int)(int8_t)((w >> (16 + 8 * (p >> 1))) & 0xFF);
+    const f16x2 sh0 = twice((_Float16)(float)(c0 & ~15)), sl0 = twice((_Float16)(float)(c0 & 15));
+    const f16x2 sh1 = twice((_Float16)(float)(c1 & ~15)), sl1 = twice((_Float16)(float)(c1 & 15));
+    uint32_t a[2][4], b[2][4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t q0 = i ? r.l0.y : r.l0.x, q1 = i ? r.l1.y : r.l1.x, t = i ? r.h.y : r.h.x;
+      const uint32_t v0 = J & 1 ? ((q0 >> 4) & 0x0F0F0F0Fu) | (t & 0x30303030u) : (q0 & 0x0F0F0F0Fu) | ((t << 4) & 0x30303030u);
+      const uint32_t v1 = J & 1 ? ((q1 >> 4) & 0x0F0F0F0Fu) | ((t >> 2) & 0x30303030u) : (q1 & 0x0F0F0F0Fu) | ((t << 2) & 0x30303030u);
+      planes(v0, sh0, sl0, a[0][2 * i], a[0][2 * i + 1], a[1][2 * i], a[1][2 * i + 1]);
+      planes(v1, sh1, sl1, b[0][2 * i], b[0][2 * i + 1], b[1][2 * i], b[1][2 * i + 1]);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      lo[i] = make_uint4(a[i][0], a[i][1], a[i][2], a[i][3]);
+      hi[i] = make_uint4(b[i][0], b[i][1], b[i][2], b[i][3]);
+    }
+  }
+};
+
+struct MmqfArgs {
+  int M, N, nsb;               // rows of X, weight rows, super-blocks per row
+  int tiles_m, whole, shared, workers, per;   // tiles of one workgroup each; tiles shared by `workers`, `per` super-blocks each
+  int64_t w_pitch, ldy;
+  uint32_t x_pitch, rows;      // bytes between the rows of X; rows of the planes
+};
+
+// The sixteen values are computed at this point.
+__device__ __forceinline__ void pin16(float (&v)[16]) {
+  asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
+  asm volatile("" : "+v"(v[8]), "+v"(v[9]), "+v"(v[10]), "+v"(v[11]), "+v"(v[12]), "+v"(v[13]), "+v"(v[14]), "+v"(v[15]));
+}
+
+template <class F, int M_T, int N_T>
+__host__ __device__ constexpr int mmqf_buffer_bytes() { return 128 * (M_T + F::PLANES * N_T); }
+// d8 [8][M_T], of two super-blocks; then of the one at hand, for its end: sums [M_T] of eight halves, d [N_T] and, with
+// offsets, -dmin [N_T] and mins [N_T] of eight halves
+template <class F, int M_T, int N_T>
+__host__ __device__ constexpr size_t mmqf_lds() { return 2 * (size_t)(mmqf_buffer_bytes<F, M_T, N_T>() + 32 * M_T) + 16 * M_T + (F::OFF ? 24 : 4) * N_T; }
+
+// v, opaque to the compiler: what is formed from it is formed where it stands, not kept in registers over the loop
+__device__ __forceinline__ int afresh(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+template <int J> struct StepIndex { static constexpr int value = J; };
+
+template <class F, int WM, int WN, int TM, int TN, typename T>
+__global__ __launch_bounds__(64 * WM * WN, 2) void mmqf_kernel(const uint8_t* __restrict__ W, const char* __restrict__ X,
+                                                               const char* __restrict__ XD, const char* __restrict__ XS,
+                                                               T* __restrict__ Y, float* __restrict__ partial,
+                                                               const T* __restrict__ bias, MmqfArgs a) {
+  constexpr int NT = 64 * WM * WN, NWV = WM * WN, M_T = 32 * WM * TM, N_T = 32 * WN * TN;
+  constexpr int BUF = mmqf_buffer_bytes<F, M_T, N_T>(), PLANE_AT = 2 * BUF + 64 * M_T;
+  constexpr int PARTS = 4 * N_T / NT;                       // parts of a row's step that a thread decodes
+  constexpr int XI = M_T / 8 / NWV;                         // fetches of 8 rows of X per wave and step
+  static_assert(4 * N_T % NT == 0 && M_T % 64 == 0 && M_T % (8 * NWV) == 0, "tile and workgroup sizes must divide evenly");
+  extern __shared__ __align__(16) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN, lrow = lane & 31, lhalf = lane >> 5;
+
+  // ---- which work (as in mmqi_kernel: whole tiles in runs per XCD), then an equal run of super-blocks of the shared tiles
+  int wg = blockIdx.x;
+  const int whole8 = a.whole & ~7;
+  if (wg < whole8) wg = (wg & 7) * (whole8 >> 3) + (wg >> 3);
+  int sw = wg - a.whole;
+  const int shared8 = a.workers & ~7;
+  if (sw >= 0 && sw < shared8 && (a.whole & 7) == 0) sw = (sw & 7) * (shared8 >> 3) + (sw >> 3);
+  int unit = sw < 0 ? wg * a.nsb : a.whole * a.nsb + sw * a.per;
+  const int unit_end = sw < 0 ? unit + a.nsb : min((a.whole + a.shared) * a.nsb, unit + a.per);
+  for (int segment = 0; unit < unit_end; ++segment) {
+  const int tile = unit / a.nsb, sb0 = unit - tile * a.nsb, sb1 = min(a.nsb, sb0 + unit_end - unit);
+  unit += sb1 - sb0;
+  const int m_base = (tile % a.tiles_m) * M_T, n_base = (tile / a.tiles_m) * N_T;
+
+  // ---- staging plans
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+  // (a fetch puts its lanes' 16 bytes one behind the other: the lane of slot l % 8 of a row asks for the piece that belongs there)
+  const uint32_t x_at = (uint32_t)(8 * wave + (lane >> 3)) * a.x_pitch + 16 * ((lane & 7) ^ ((4 * wave + (lane >> 4)) & 7));
+  const auto fetch_lds = [&](uint32_t at, const char* base, uint32_t to) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(at), "s"(base), "s"(to) : "memory");
+  };
+  const char* const x_tile = X + (int64_t)m_base * a.x_pitch;
+  const auto fetch_x = [&](int g, int buf) {                // step g of the row (64 values, 128 bytes)
+#pragma unroll
+    for (int i = 0; i < XI; ++i)
+      fetch_lds(x_at, x_tile + (128u * (uint32_t)g + (uint32_t)(8 * NWV * i) * a.x_pitch), lds0 + buf * BUF + 1024 * (wave + NWV * i));
+  };
+  // the planes of a super-block of the rows of X: d8 is 8 rows of M_T floats, the sums M_T rows of 16 bytes
+  const auto fetch_d8 = [&](int sb, int pb) {
+#pragma unroll
+    for (int q = wave; q < M_T / 32; q += NWV)              // (1 KB each; 256 q is the float of the plane, of block 256 q / M_T)
+      fetch_lds(M_T >= 256 ? 16 * lane : 4 * (4 * lane / M_T * a.rows + 4 * lane % M_T), XD + 4 * ((int64_t)(8 * sb + 256 * q / M_T) * a.rows + m_base + 256 * q % M_T), lds0 + 2 * BUF + 32 * M_T * pb + 1024 * q);
+  };
+  const auto fetch_sums = [&](int sb) {
+#pragma unroll
+    for (int q = wave; q < M_T / 64; q += NWV)
+      fetch_lds(16 * lane, XS + 16 * ((int64_t)sb * a.rows + m_base + 64 * q), lds0 + PLANE_AT + 1024 * q);
+  };
+  // weights: a thread has PARTS parts of one row's step
+  const int w_n = tid * PARTS >> 2, part0 = tid * PARTS & 3;
+  const uint32_t w_row = (uint32_t)min(n_base + w_n, a.N - 1) * (uint32_t)a.w_pitch;   // (the matrix is below 4 GB: mmqf_takes)
+  typename F::Head hd;
+  typename F::Scales sc;
+  typename F::Raw raw[PARTS];
+  const auto fetch_raw = [&](int g) {
+#pragma unroll
+    for (int i = 0; i < PARTS; ++i) raw[i] = F::fetch(W + (w_row + (uint32_t)(g >> 2) * F::BS), g & 3, part0 + i);
+  };
+  const auto fetch_head = [&](int sb) { hd = F::head(W + (w_row + (uint32_t)sb * F::BS)); };
+  const auto stash_head = [&]() {
+    const int id = afresh(tid), n = id * PARTS >> 2;
+    char* const p = smem + PLANE_AT;
+    if ((id * PARTS & 3) == 0) {
+      *(float*)(p + 16 * M_T + 4 * n) = F::d(hd);
+      if (F::OFF) {
+        *(float*)(p + 16 * M_T + 4 * N_T + 4 * n) = -F::dmin(hd);
+        *(uint4*)(p + 16 * M_T + 8 * N_T + 16 * n) = F::mins(hd);
+      }
+    }
+  };
+  const auto stash = [&](auto step, int buf) {
+    constexpr int J = decltype(step)::value;
+    const int id = afresh(tid), n = id * PARTS >> 2, p0 = id * PARTS & 3;
+    char* const row = smem + (buf * BUF + 128 * (M_T + n));
+    const int s = (n >> 1) & 7;
+#pragma unroll
+    for (int i = 0; i < PARTS; ++i) {
+      uint4 lo[F::PLANES], hi[F::PLANES];
+      F::template decode<J>(raw[i], sc, p0 + i, lo, hi);
+#pragma unroll
+      for (int pl = 0; pl < F::PLANES; ++pl) {
+        *(uint4*)(row + 128 * N_T * pl + 16 * ((p0 + i) ^ s)) = lo[pl];
+        *(uint4*)(row + 128 * N_T * pl + 16 * ((4 + p0 + i) ^ s)) = hi[pl];
+      }
+    }
+  };
+
+  float acc[TN][TM][16], part_acc[TN][TM][16];
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int k = 0; k < TM; ++k)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][k][r] = 0.0f;
+  f32x16 zero;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) zero[r] = 0.0f;
+
+  // ---- one step of K: eight (block, tile pair) units, the matrix instructions of the next unit in front of the scaling
+  const int swz = (lrow >> 1) & 7;                          // (tile bases are multiples of 16 rows)
+  const int op0 = 128 * lrow + 16 * (lhalf ^ swz), x_op = 128 * 32 * TM * wm, w_op = 128 * (M_T + 32 * TN * wn);
+  struct Operands { f16x8 x[TM][2], w[TN][F::PLANES][2]; };
+  const auto load_x = [&](int base, int buf, int b, int k, Operands& o) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) o.x[k][h] = *(const f16x8*)(smem + (buf * BUF + (base ^ (16 * (4 * b + 2 * h)))) + x_op + 4096 * k);
+  };
+  const auto load_w = [&](int base, int buf, int b, int i, Operands& o) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const char* const at = smem + (buf * BUF + (base ^ (16 * (4 * b + 2 * h)))) + w_op;
+#pragma unroll
+      for (int pl = 0; pl < F::PLANES; ++pl) o.w[i][pl][h] = *(const f16x8*)(at + 128 * N_T * pl + 4096 * i);
+    }
+  };
+  // A unit is a block and a pair of tiles, U units per block.  The matrix instructions of unit u + 1 stand between the
+  // multiply-adds of unit u (each waits for the one before it), and an operand's successor is read as soon as the last
+  // instruction that takes it has started.
+  constexpr int U = TM * TN, P = 2 * F::PLANES;
+  const auto load_first = [&](int buf, Operands& o) {
+    const int base = afresh(op0);
+#pragma unroll
+    for (int i = 0; i < TN; ++i) load_w(base, buf, 0, i, o);
+#pragma unroll
+    for (int k = 0; k < TM; ++k) load_x(base, buf, 0, k, o);
+  };
+  const auto contract = [&](auto step, int buf, int pb, Operands& o) {
+    constexpr int J = decltype(step)::value;
+    const float* const xd = (const float*)(smem + 2 * BUF + 32 * M_T * pb) + 2 * J * M_T + 32 * TM * wm + lrow;
+    const int base = afresh(op0);
+    f32x16 s[2];
+    float d8[2][TM];
+#pragma unroll
+    for (int k = 0; k < TM; ++k) {
+      d8[0][k] = xd[32 * k];
+      d8[1][k] = xd[M_T + 32 * k];
+    }
+    const auto mfma = [&](int u, int piece, f32x16& v) {
+      const int i = u / TM, k = u % TM, pl = piece >> 1, h = piece & 1;
+      v = __builtin_amdgcn_mfma_f32_32x32x16_f16(o.w[i][pl][h], o.x[k][h], piece == 0 ? zero : v, 0, 0, 0);
+    };
+#pragma unroll
+    for (int piece = 0; piece < P; ++piece) mfma(0, piece, s[0]);
+#pragma unroll
+    for (int v = 0; v < 2 * U; ++v) {
+      const int b = v / U, u = v % U, i = u / TM, k = u % TM;
+#pragma unroll
+      for (int piece = 0; piece < P; ++piece) {
+        if (v + 1 < 2 * U) mfma((v + 1) % U, piece, s[(v + 1) & 1]);
+        if (piece == P - 1 && v < U) {   // (unit v + 1 of the first block has its operands)
+          const int un = v + 1, in = un / TM, kn = un % TM;
+          if (un < U && kn == TM - 1 && in < TN) load_w(base, buf, 1, in, o);
+          if (un < U && in == TN - 1) load_x(base, buf, 1, kn, o);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 16 / P * piece; r < 16 / P * (piece + 1); ++r)
+          part_acc[i][k][r] = J == 0 && b == 0 ? s[v & 1][r] * d8[b][k] : __builtin_fmaf(s[v & 1][r], d8[b][k], part_acc[i][k][r]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // (here and not later: the compiler would keep the products and scale them all at the end of the super-block)
+      pin16(part_acc[i][k]);
+    }
+  };
+  // the end of a super-block
+  const auto fold = [&]() {
+    const char* const xs = smem + PLANE_AT;
+    const char* const p = xs + 16 * M_T;
+    const int ln = afresh(lane), row = ln & 31, half = ln >> 5;
+    uint4 sv[TM];
+    if constexpr (F::OFF)
+#pragma unroll
+      for (int k = 0; k < TM; ++k) sv[k] = *(const uint4*)(xs + 16 * (32 * (TM * wm + k) + row));
+#pragma unroll
+    for (int i = 0; i < TN; ++i) {
+      const int n = 32 * (TN * wn + i);
+      __builtin_amdgcn_sched_barrier(0);
+      f32x16 off[F::OFF ? TM : 1];
+      f32x4_m d[4], dm[4];
+      if constexpr (F::OFF) {
+        // (a contraction over eight: the upper half of the lanes holds values 8 .. 15, zeros)
+        uint4 mv = *(const uint4*)(p + 8 * N_T + 16 * (n + row));
+        if (half) mv = make_uint4(0, 0, 0, 0);
+#pragma unroll
+        for (int k = 0; k < TM; ++k) {
+          const uint4 v = half ? make_uint4(0, 0, 0, 0) : sv[k];
+          off[k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, mv), __builtin_bit_cast(f16x8, v), zero, 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        d[q] = *(const f32x4_m*)(p + 4 * (n + 8 * q + 4 * half));
+        if (F::OFF) dm[q] = *(const f32x4_m*)(p + 4 * N_T + 4 * (n + 8 * q + 4 * half));
+      }
+#pragma unroll
+      for (int k = 0; k < TM; ++k) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          acc[i][k][r] = __builtin_fmaf(part_acc[i][k][r], d[r >> 2][r & 3], acc[i][k][r]);
+          if constexpr (F::OFF) acc[i][k][r] = __builtin_fmaf(off[k][r], dm[r >> 2][r & 3], acc[i][k][r]);
+        }
+        pin16(acc[i][k]);
+      }
+    }
+  };
+
+  const int g1 = 4 * sb1;
+  if (sb0 < sb1) {
+    fetch_head(sb0);
+    fetch_raw(4 * sb0);
+    fetch_d8(sb0, 0);
+    fetch_x(4 * sb0, 0);
+    sc = F::scales(hd);
+    stash(StepIndex<0>(), 0);
+    fetch_raw(4 * sb0 + 1);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    // In step g: the registers (step g + 1, loaded during g - 1) are decoded into the other buffer, the rows of X of
+    // g + 1 are asked for, the packed weights of g + 2, and step g is contracted.
+    for (int sb = sb0; sb < sb1; ++sb) {
+      const int pb = (sb - sb0) & 1;
+      const bool more = sb + 1 < sb1;
+      const auto turn = [&](auto step) {
+        constexpr int J = decltype(step)::value;
+        const int g = 4 * sb + J;
+        Operands o;
+        load_first(J & 1, o);                               // (they arrive under the decoding)
+        __builtin_amdgcn_sched_barrier(0);
+        if (J == 1) stash_head();                           // (the end of the super-block before has been)
+        if (J < 3 || more) {
+          if (J == 3) sc = F::scales(hd);
+          stash(StepIndex<(J + 1) & 3>(), (J + 1) & 1);
+          fetch_x(g + 1, (J + 1) & 1);
+          if (g + 2 < g1) fetch_raw(g + 2);
+        }
+        if (J == 1 && F::OFF) fetch_sums(sb);
+        if (J == 2 && more) {
+          fetch_d8(sb + 1, pb ^ 1);
+          fetch_head(sb + 1);
+        }
+        contract(step, J & 1, pb, o);
+        if (J == 3) fold();
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+      };
+      turn(StepIndex<0>());
+      turn(StepIndex<1>());
+      turn(StepIndex<2>());
+      turn(StepIndex<3>());
+    }
+  }
+
+  // ---- store: lane = one row of X, 16 features per tile in runs of four
+  float* const mine = sb1 - sb0 < a.nsb ? partial + (int64_t)(2 * sw + segment) * (M_T * N_T) : nullptr;
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int k = 0; k < TM; ++k)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        if (mine) {   // in the order of the registers: [wave][tile][run][lane] of four
+          *(f32x4_m*)(mine + (((wave * TN * TM + i * TM + k) * 4 + q) * 64 + lane) * 4) = (f32x4_m){acc[i][k][4 * q], acc[i][k][4 * q + 1], acc[i][k][4 * q + 2], acc[i][k][4 * q + 3]};
+        } else {
+          const int m = m_base + 32 * (TM * wm + k) + lrow, n = n_base + 32 * (TN * wn + i) + 8 * q + 4 * lhalf;
+          if (m < a.M)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (n + e < a.N) Y[(int64_t)m * a.ldy + n + e] = finish<T>(acc[i][k][4 * q + e], bias, n + e);
+        }
+      }
+  }
+}
+
+// Y tile = T(sum of its partial tiles) in the order of K; a workgroup per wave's share of a tile, a thread per run of four
+template <int WM, int WN, int TM, int TN, typename T>
+__global__ __launch_bounds__(256) void mmqf_reduce_kernel(const float* __restrict__ partial, T* __restrict__ Y, const T* __restrict__ bias, MmqfArgs a) {
+  constexpr int M_T = 32 * WM * TM, N_T = 32 * WN * TN;
+  const int t = blockIdx.x, tile = a.whole + t, sub = blockIdx.y, q = threadIdx.x >> 6, lane = threadIdx.x & 63;   // sub: (wave, tile of the wave)
+  const int wave = sub / (TN * TM), i = sub / TM % TN, k = sub % TM, wm = wave / WN, wn = wave % WN;
+  // the workers whose runs of super-blocks meet this tile; a worker's second partial tile is the tile it entered last
+  const int first = t * a.nsb / a.per, last = ((t + 1) * a.nsb - 1) / a.per;
+  if (first == last && t * a.nsb == first * a.per && a.per == a.nsb) return;   // (stored whole)
+  f32x4_m v = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int w = first; w <= last; ++w) v += *(const f32x4_m*)(partial + (int64_t)(2 * w + t - w * a.per / a.nsb) * (M_T * N_T) + ((sub * 4 + q) * 64 + lane) * 4);
+  const int m = (tile % a.tiles_m) * M_T + 32 * (TM * wm + k) + (lane & 31), n = (tile / a.tiles_m) * N_T + 32 * (TN * wn + i) + 8 * q + 4 * (lane >> 5);
+  if (m >= a.M) return;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (n + e < a.N) Y[(int64_t)m * a.ldy + n + e] = finish<T>(v[e], bias, n + e);
+}
+
+template <class F, int WM, int WN, int TM, int TN, typename T>
+static int mmqf_launch(const MmqfCall& c, const MmqfPlan& p, hipStream_t stream) {
+  constexpr int M_T = 32 * WM * TM, N_T = 32 * WN * TN;
+  constexpr size_t lds = mmqf_lds<F, M_T, N_T>();
+  static_assert(lds <= 160 * 1024, "tile does not fit in LDS");
+  auto kern = mmqf_kernel<F, WM, WN, TM, TN, T>;
+  static std::atomic<uint64_t> done{0};
+  allow_large_lds(kern, lds, done);
+  const MmqfArgs a = {c.M, c.N, c.K / 256, (c.M + M_T - 1) / M_T, p.whole, p.shared, p.workers, p.per,
+                      c.la.w_pitch ? c.la.w_pitch : (int64_t)(c.K / 256) * F::BS, c.la.ldy ? c.la.ldy : (int64_t)c.N, (uint32_t)(2 * c.x.pitch), (uint32_t)c.x.rows};
+  hipLaunchKernelGGL(kern, dim3(p.whole + p.workers), dim3(64 * WM * WN), lds, stream, (const uint8_t*)c.W, (const char*)c.x.x,
+                     (const char*)c.x.d, (const char*)c.x.s, (T*)c.Y, c.partial, (const T*)c.la.bias, a);
+  if (p.shared > 0)
+    hipLaunchKernelGGL((mmqf_reduce_kernel<WM, WN, TM, TN, T>), dim3(p.shared, WM * WN * TM * TN), dim3(256), 0, stream, c.partial, (T*)c.Y,
+                       (const T*)c.la.bias, a);
+  return launch_status();
+}
+
+template <class F, typename T>
+static int mmqf_typed(const MmqfCall& c, hipStream_t stream) {
+  const MmqfPlan p = mmqf_plan(c.M, c.N, c.K, c.partial_bytes);
+  return mmqf_launch<F, 4, 2, 2, 2, T>(c, p, stream);
+}
+
+template <class F>
+static int mmqf_fmt(const MmqfCall& c, hipStream_t stream) {
+  GGUF_DISPATCH_DTYPE(c.dtype, return (mmqf_typed<F, scalar_t>(c, stream)));
+  return GGUF_ERR_DTYPE;
+}
+
+}  // namespace gguf

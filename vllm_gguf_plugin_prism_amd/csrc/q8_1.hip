@@ -9,6 +9,7 @@
 // lane^2 / lane^1 are the butterfly partners for masks 16 / 8 (DPP quad
 // permutes) and masks 4, 2, 1 are in-register.  The fp32 addition tree is
 // therefore the same tree the reference evaluates.
+#include "mmq_f.h"
 #include "q8_1_device.h"
 
 namespace gguf {
@@ -20,6 +21,37 @@ __global__ __launch_bounds__(256) void quantize_q8_1_kernel(const T* __restrict_
   const int t = blockIdx.x * 256 + threadIdx.x;  // one thread per 8 values of the padded row
   if (t * 8 >= Kp) return;
   q8_1_quantize_thread<T>(x, ws, K, Kp, row_bytes, act, blockIdx.y, t, xh, permuted);
+}
+
+// The activations of mmq_f_core.h (MmqfRows): the quants as whole numbers in half precision, of four neighbours in the
+// order 0, 2, 1, 3, the block scales [block][row], the block sums as halves [super-block][row][8].
+template <typename T>
+__global__ __launch_bounds__(256) void quantize_whole_kernel(const T* __restrict__ x, MmqfRows r, int K, int64_t m0) {
+  const int t = blockIdx.x * 256 + threadIdx.x;  // one thread per 8 values
+  if (t * 8 >= K) return;                        // (K is a multiple of 256: quads stay together)
+  const int64_t m = m0 + blockIdx.y;
+  float v[8];
+  load8<T>(x + m * (int64_t)K + 8 * t, v);
+  const Q8Quad q = q8_1_quantize8(v);
+  union { _Float16 h[8]; uint4 v; } o;
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    o.h[(i & 4) | ((i & 1) << 1) | ((i >> 1) & 1)] = (_Float16)(float)(int8_t)((i < 4 ? q.q.x >> (8 * i) : q.q.y >> (8 * (i - 4))) & 0xFF);
+  *(uint4*)(r.x + m * r.pitch + 8 * t) = o.v;
+  if ((t & 3) == 0) {
+    const int b = t >> 2;
+    r.d[(int64_t)b * r.rows + m] = q.d;
+    r.s[((int64_t)(b >> 3) * r.rows + m) * 8 + (b & 7)] = (_Float16)q.s;
+  }
+}
+
+int quantize_whole(const void* x, int xdtype, const MmqfRows& r, int64_t M, int64_t K, hipStream_t stream) {
+  const int gx = (int)((K / 8 + 255) / 256);
+  for (int64_t off = 0; off < M; off += 65535) {
+    const int rows = (int)((M - off) < 65535 ? (M - off) : 65535);
+    GGUF_DISPATCH_DTYPE(xdtype, hipLaunchKernelGGL(quantize_whole_kernel<scalar_t>, dim3(gx, rows), dim3(256), 0, stream, (const scalar_t*)x, r, (int)K, off));
+  }
+  return launch_status();
 }
 
 __global__ void q8_1_unpack_kernel(const char* __restrict__ ws, int8_t* __restrict__ q, float* __restrict__ ds, int Kp,
