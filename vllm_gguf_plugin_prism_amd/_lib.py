@@ -82,6 +82,14 @@ _SIGNATURES = {
 }
 EXPORTS = tuple(_SIGNATURES)
 
+# entry points behind the layer calls only (csrc/dense_api.h), not part of the public header
+_LAYER_SIGNATURES = {
+    "gguf_dense_linear_takes": (_c.c_int, [_c.c_int, _c.c_int, _c.c_int64, _c.c_int64, _c.c_int64]),
+    "gguf_dense_linear_workspace_bytes": (_c.c_int64, [_c.c_int64, _c.c_int64, _c.c_int64]),
+    "gguf_dense_linear": (_c.c_int, [_c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_int, _c.c_void_p, _c.c_void_p, _c.c_int64,
+                                     _c.c_void_p, _c.c_int, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_void_p]),
+}
+
 
 class _Bound:
     """The library's entry points as attributes."""
@@ -116,7 +124,7 @@ def lib() -> "_Bound":
 
         handle = ctypes.CDLL(path)
         bound = _Bound()
-        for name, (res, args) in _SIGNATURES.items():
+        for name, (res, args) in (*_SIGNATURES.items(), *_LAYER_SIGNATURES.items()):
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args

@@ -11,6 +11,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/EmptyTensor.h>
+#include <ATen/ops/matmul.h>
 #include <ATen/hip/impl/HIPCachingAllocatorMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -19,12 +20,13 @@
 #include <algorithm>
 #include <vector>
 
+#include "../dense_api.h"
 #include "gguf_hip.h"
 
 namespace {
 
 // ---- what dispatch.py decides (select_mul_mat_path, mmvq_safe, select_moe_path), restated; tests compare the two
-enum Path { PATH_OTHER = 0, PATH_MMVQ = 1, PATH_MMQ = 2 };
+enum Path { PATH_OTHER = 0, PATH_MMVQ = 1, PATH_MMQ = 2, PATH_DENSE = 3 };
 
 bool is_matrix_type(int t) { return t == 2 || t == 3 || (t >= 6 && t <= 8) || (t >= 10 && t <= 14); }
 bool is_imatrix_type(int t) { return (t >= 16 && t <= 23) || t == 29; }
@@ -34,7 +36,7 @@ Path mul_mat_path(int type, int64_t batch, int64_t rows) {
   if (batch <= 0 || !(im || is_matrix_type(type))) return PATH_OTHER;
   const int64_t safe = im ? (rows > 5120 ? 8 : 16) : (rows > 5120 ? 2 : 6);
   if (batch <= safe) return PATH_MMVQ;
-  return im ? PATH_OTHER : PATH_MMQ;
+  return im ? PATH_DENSE : PATH_MMQ;
 }
 
 constexpr int64_t kMoeVecMaxTokens = 64, kMoeGroupedMaxExperts = 256;
@@ -108,6 +110,11 @@ struct Shard {
 // launches one shard on the current GPU; the workspace lives until the launches are queued
 int run_shard(const Shard& s, const at::Tensor& x, int xcode, gguf_stream_t stream) {
   const int64_t m = x.size(0), k = x.size(1);
+  if (s.path == PATH_DENSE) {
+    const int64_t bytes = gguf_dense_linear_workspace_bytes(s.rows, k, m);
+    const c10::DataPtr ws = scratch(bytes);
+    return gguf_dense_linear(s.w, s.pitch, x.const_data_ptr(), xcode, ws.get(), s.y, s.ldy, s.bias, s.type, s.rows, k, m, bytes, stream);
+  }
   const int64_t bytes = s.path == PATH_MMQ ? gguf_mmq_workspace_bytes_engine(m, s.rows, k, GGUF_MMQ_AUTO) : m * gguf_q8_1_row_bytes(k);
   const c10::DataPtr ws = scratch(bytes);
   if (s.path == PATH_MMVQ)
@@ -119,9 +126,24 @@ int run_shard(const Shard& s, const at::Tensor& x, int xcode, gguf_stream_t stre
 // activations the kernels take as they lie
 bool rows_ok(const at::Tensor& x) { return x.dim() == 2 && x.size(0) > 0 && x.size(1) > 0 && x.is_contiguous() && dtype_code(x.scalar_type()) >= 0; }
 bool packed_ok(const at::Tensor& w) { return w.dim() == 2 && w.scalar_type() == at::kByte && (w.size(1) <= 1 || w.stride(1) == 1); }
+// whether a call on this path is served here
+bool path_ok(Path p, int type, const at::Tensor& x, const at::Tensor& w, int64_t rows) {
+  if (p == PATH_DENSE)
+    return gguf_dense_linear_takes(type, dtype_code(x.scalar_type()), rows, x.size(1), x.size(0)) && ((uintptr_t)x.const_data_ptr() & 15) == 0 &&
+           ((uintptr_t)w.const_data_ptr() & 1) == 0 && (w.stride(0) & 1) == 0;
+  return p != PATH_OTHER;
+}
 int64_t row_bytes(int type, int64_t k) {   // 0 where K is not whole blocks of the type
   const int qk = gguf_block_elems(type);
   return qk == 0 || k % qk ? 0 : k / qk * gguf_block_bytes(type);
+}
+
+// a dense copy of the weights and a library product, the reference's two steps (quantization/linear.py:50-58)
+at::Tensor dense_copy_product(const at::Tensor& x, const at::Tensor& w, int type, gguf_stream_t stream) {
+  const NoGil nogil;
+  const at::Tensor dense = new_tensor({w.size(0), x.size(1)}, x.scalar_type());
+  if (gguf_dequantize(w.const_data_ptr(), type, dense.mutable_data_ptr(), dtype_code(x.scalar_type()), dense.numel(), stream) != GGUF_OK) return {};
+  return at::matmul(x, dense.t());
 }
 
 // linear(x, weight, weight_type, out, bias) -> Tensor | None
@@ -133,7 +155,13 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!w || !as_int(a[2], &type) || !rows_ok(*x) || !packed_ok(*w)) Py_RETURN_NONE;
   const int64_t m = x->size(0), k = x->size(1), rows = w->size(0), rb = row_bytes((int)type, k);
   const Path path = mul_mat_path((int)type, m, rows);
-  if (path == PATH_OTHER || rb == 0 || w->size(1) < rb || rows == 0) Py_RETURN_NONE;
+  if (rb == 0 || w->size(1) < rb || rows == 0) Py_RETURN_NONE;
+  if (!path_ok(path, (int)type, *x, *w, rows)) {
+    if (path != PATH_DENSE || w->size(1) != rb || !w->is_contiguous() || a[3] != Py_None || a[4] != Py_None) Py_RETURN_NONE;
+    at::Tensor y = dense_copy_product(*x, *w, (int)type, stream_of(dev));
+    if (!y.defined()) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(y));
+  }
   const at::Tensor *out = nullptr, *bias = nullptr;
   if (a[3] != Py_None) {
     out = plain(a[3], dev);
@@ -155,7 +183,7 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
                   bias ? bias->const_data_ptr() : nullptr};
     rc = run_shard(s, *x, dtype_code(x->scalar_type()), stream_of(dev));
   }
-  if (rc != GGUF_OK) return fail(rc, path == PATH_MMVQ ? "ggml_mul_mat_vec_a8" : "ggml_mul_mat_a8");
+  if (rc != GGUF_OK) return fail(rc, path == PATH_MMVQ ? "ggml_mul_mat_vec_a8" : path == PATH_MMQ ? "ggml_mul_mat_a8" : "dense_linear");
   if (out) return Py_NewRef(a[3]);
   return THPVariable_Wrap(std::move(y));
 }
@@ -186,7 +214,7 @@ PyObject* merged_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
       Py_RETURN_NONE;
     const int64_t rows = p.end - p.start, rb = row_bytes((int)p.type, k);
     p.path = mul_mat_path((int)p.type, m, rows);
-    if (p.path == PATH_OTHER || rows <= 0 || p.start < 0 || p.end > w->size(0) || rb == 0 || p.rb < rb || p.rb > w->size(1)) Py_RETURN_NONE;
+    if (rows <= 0 || !path_ok(p.path, (int)p.type, *x, *w, rows) || p.start < 0 || p.end > w->size(0) || rb == 0 || p.rb < rb || p.rb > w->size(1)) Py_RETURN_NONE;
     width += rows;
     if (!parts.empty() && parts.back().end == p.start && parts.back().type == p.type && parts.back().path == p.path)
       parts.back().end = p.end;
@@ -300,7 +328,7 @@ PyObject* path_name(PyObject*, PyObject* const* a, Py_ssize_t n) {
   int64_t v[3];
   if (n != 3 || !as_int(a[0], v) || !as_int(a[1], v + 1) || !as_int(a[2], v + 2)) return PyErr_Format(PyExc_TypeError, "mul_mat_path takes 3 integers"), nullptr;
   const Path p = mul_mat_path((int)v[0], v[1], v[2]);
-  if (p == PATH_OTHER) Py_RETURN_NONE;
+  if (p != PATH_MMVQ && p != PATH_MMQ) Py_RETURN_NONE;
   return PyUnicode_FromString(p == PATH_MMVQ ? "mmvq" : "mmq");
 }
 

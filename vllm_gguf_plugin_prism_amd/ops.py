@@ -207,6 +207,25 @@ def ggml_dequant_gemm(W: torch.Tensor, X: torch.Tensor, quant_type: int, row: in
     return out
 
 
+def dense_linear(W: torch.Tensor, X: torch.Tensor, quant_type: int, row: int, *, out: torch.Tensor | None = None,
+                 bias: torch.Tensor | None = None) -> torch.Tensor | None:
+    """``X @ dequant(W)^T`` of a codebook format with the weights rounded to X's dtype (csrc/dense_core.h), or ``None`` for
+    a call that kernel does not serve.  ``out`` / ``bias`` / sliced ``W``: as for :func:`ggml_mul_mat_vec_a8`."""
+    vecs, col = X.shape
+    if (X.dtype not in (torch.float16, torch.bfloat16) or not X.is_contiguous() or X.data_ptr() % 16
+            or W.data_ptr() % 2 or W.stride(0) % 2
+            or not _lib.lib().gguf_dense_linear_takes(int(quant_type), _code(X.dtype), row, col, vecs)):
+        return None
+    out, w_pitch, ldy = _shard_args(W, X, quant_type, row, out, bias)
+    with _on_device_of(X):
+        nbytes = _lib.lib().gguf_dense_linear_workspace_bytes(row, col, vecs)
+        ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=X.device)
+        rc = _lib.lib().gguf_dense_linear(W.data_ptr(), w_pitch, X.data_ptr(), _code(X.dtype), ws.data_ptr(), out.data_ptr(), ldy,
+                                          bias.data_ptr() if bias is not None else None, int(quant_type), row, col, vecs, nbytes, _stream(X))
+    _lib.check(rc, "dense_linear")
+    return out
+
+
 MOE_GROUPED_MAX_EXPERTS = 256
 
 
