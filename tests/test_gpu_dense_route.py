@@ -1,0 +1,44 @@
+"""What reaches the codebook formats' GEMM (csrc/dense_core.h) and what does not: ``fused_mul_mat_gguf`` takes every call that
+a dense copy of the weights and ``x @ dense.T`` (then ``add_`` of the bias, ``copy_`` to the result) takes, with their
+result, and refuses what they refuse, whether or not the number of rows is one that the GEMM serves."""
+import numpy as np
+import pytest
+import torch
+
+from vllm_gguf_plugin_prism_amd import dispatch as D
+from vllm_gguf_plugin_prism_amd import ops, synth
+
+pytestmark = pytest.mark.gpu
+QT, N, K, M = D.IQ4_XS, 512, 512, 40         # (40 rows: the GEMM serves the plain call)
+
+
+def _weights(pad=0):
+    packed = torch.from_numpy(synth.make_weights(np.random.default_rng(1), QT, N, K)).cuda()
+    w = torch.zeros(N, packed.shape[1] + pad, dtype=torch.uint8, device="cuda")
+    w[:, :packed.shape[1]] = packed
+    return w, packed
+
+
+def _x(*shape, dtype=torch.float16, seed=2):
+    return torch.from_numpy(np.random.default_rng(seed).standard_normal(shape).astype(np.float32)).to(dtype).cuda()
+
+
+def _dense(packed, dtype=torch.float16):
+    return ops.ggml_dequantize(packed, QT, N, K, dtype)
+
+
+def _close(got, want, rel=1e-3):              # two roundings to 16 bits and a sum in another order
+    assert got.shape == want.shape and got.dtype == want.dtype
+    assert ((got.double() - want.double()).norm() / want.double().norm()).item() <= rel
+
+
+def test_the_plain_call_is_served():
+    w, _ = _weights()
+    assert ops.dense_linear(w, _x(M, K), QT, N) is not None
+
+
+@pytest.mark.parametrize("shape", [(M, 3, K), (M, 1, K)])
+def test_activations_of_three_dimensions(shape):
+    w, packed = _weights()
+    x = _x(*shape)
+    _close(D.fused_mul_mat_gguf(x, w, QT), x @ _dense(packed).T)

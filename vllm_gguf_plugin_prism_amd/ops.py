@@ -211,6 +211,8 @@ def dense_linear(W: torch.Tensor, X: torch.Tensor, quant_type: int, row: int, *,
                  bias: torch.Tensor | None = None) -> torch.Tensor | None:
     """``X @ dequant(W)^T`` of a codebook format with the weights rounded to X's dtype (csrc/dense_core.h), or ``None`` for
     a call that kernel does not serve.  ``out`` / ``bias`` / sliced ``W``: as for :func:`ggml_mul_mat_vec_a8`."""
+    if X.dim() != 2:                         # (the product of a dense copy takes any number of leading dimensions)
+        return None
     vecs, col = X.shape
     if (X.dtype not in (torch.float16, torch.bfloat16) or not X.is_contiguous() or X.data_ptr() % 16
             or W.data_ptr() % 2 or W.stride(0) % 2
