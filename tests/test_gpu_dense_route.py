@@ -42,3 +42,34 @@ def test_activations_of_three_dimensions(shape):
     w, packed = _weights()
     x = _x(*shape)
     _close(D.fused_mul_mat_gguf(x, w, QT), x @ _dense(packed).T)
+
+
+@pytest.mark.parametrize("bias", ["fp32", "one", "row"])
+def test_a_bias_that_add_takes(bias):
+    w, packed = _weights()
+    x = _x(M, K)
+    b = {"fp32": _x(N, dtype=torch.float32), "one": _x(1), "row": _x(1, N)}[bias]
+    _close(D.fused_mul_mat_gguf(x, w, QT, bias=b), (x @ _dense(packed).T).add_(b))
+
+
+def test_a_result_that_copy_takes():
+    w, packed = _weights()
+    x = _x(M, K)
+    want = x @ _dense(packed).T
+    for out in (torch.empty(M, N, device="cuda"), torch.empty(N, M, dtype=x.dtype, device="cuda").T, torch.empty(2, M, N, dtype=x.dtype, device="cuda")):
+        got = D.fused_mul_mat_gguf(x, w, QT, out=out)
+        assert got is out
+        _close(got, want.to(out.dtype).expand(out.shape))
+
+
+def test_a_result_over_the_activations():      # (N == K)
+    w, packed = _weights()
+    same = _x(M, K)
+    want = same @ _dense(packed).T
+    _close(D.fused_mul_mat_gguf(same, w, QT, out=same), want)
+
+
+def test_a_result_whose_rows_overlap_is_refused():
+    w, _ = _weights()
+    with pytest.raises(RuntimeError):
+        D.fused_mul_mat_gguf(_x(M, K), w, QT, out=torch.empty(1, N, dtype=torch.float16, device="cuda").expand(M, N))

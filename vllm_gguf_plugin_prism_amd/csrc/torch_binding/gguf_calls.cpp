@@ -168,10 +168,13 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!out || out->dim() != 2 || out->size(0) != m || out->size(1) != rows || out->scalar_type() != x->scalar_type() ||
         (rows > 1 && out->stride(1) != 1))
       Py_RETURN_NONE;
+    // (`out.copy_(y)`, which the dense path's store stands in for, refuses rows that overlap and takes memory shared with x)
+    if (path == PATH_DENSE && ((m > 1 && out->stride(0) < rows) || out->is_alias_of(*x) || out->is_alias_of(*w))) Py_RETURN_NONE;
   }
   if (a[4] != Py_None) {
     bias = plain(a[4], dev);
     if (!bias || bias->dim() != 1 || bias->size(0) != rows || bias->scalar_type() != x->scalar_type() || !bias->is_contiguous()) Py_RETURN_NONE;
+    if (path == PATH_DENSE && out && out->is_alias_of(*bias)) Py_RETURN_NONE;
   }
   at::Tensor y;
   int rc;

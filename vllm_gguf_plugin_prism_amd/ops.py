@@ -207,6 +207,22 @@ def ggml_dequant_gemm(W: torch.Tensor, X: torch.Tensor, quant_type: int, row: in
     return out
 
 
+def _dense_result_fits(X: torch.Tensor, row: int, out: torch.Tensor | None, bias: torch.Tensor | None, *inputs: torch.Tensor) -> bool:
+    """Whether the result and the bias of a dense product lie as its kernel takes them.  ``y.add_(bias)`` and
+    ``out.copy_(y)``, which it stands in for, take more: other types, strides and broadcast shapes, and a result that
+    shares memory with what it is formed from."""
+    if bias is not None and (bias.shape != (row,) or bias.dtype != X.dtype or bias.device != X.device or not bias.is_contiguous()):
+        return False
+    if out is None:
+        return True
+    if out.shape != (X.shape[0], row) or out.dtype != X.dtype or out.device != X.device:
+        return False
+    if (row > 1 and out.stride(1) != 1) or (X.shape[0] > 1 and out.stride(0) < row):
+        return False
+    held = out.untyped_storage().data_ptr()
+    return all(t is None or t.untyped_storage().data_ptr() != held for t in (X, bias, *inputs))
+
+
 def dense_linear(W: torch.Tensor, X: torch.Tensor, quant_type: int, row: int, *, out: torch.Tensor | None = None,
                  bias: torch.Tensor | None = None) -> torch.Tensor | None:
     """``X @ dequant(W)^T`` of a codebook format with the weights rounded to X's dtype (csrc/dense_core.h), or ``None`` for
@@ -216,7 +232,8 @@ def dense_linear(W: torch.Tensor, X: torch.Tensor, quant_type: int, row: int, *,
     vecs, col = X.shape
     if (X.dtype not in (torch.float16, torch.bfloat16) or not X.is_contiguous() or X.data_ptr() % 16
             or W.data_ptr() % 2 or W.stride(0) % 2
-            or not _lib.lib().gguf_dense_linear_takes(int(quant_type), _code(X.dtype), row, col, vecs)):
+            or not _lib.lib().gguf_dense_linear_takes(int(quant_type), _code(X.dtype), row, col, vecs)
+            or not _dense_result_fits(X, row, out, bias, W)):
         return None
     out, w_pitch, ldy = _shard_args(W, X, quant_type, row, out, bias)
     with _on_device_of(X):
