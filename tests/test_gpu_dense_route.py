@@ -73,3 +73,27 @@ def test_a_result_whose_rows_overlap_is_refused():
     w, _ = _weights()
     with pytest.raises(RuntimeError):
         D.fused_mul_mat_gguf(_x(M, K), w, QT, out=torch.empty(1, N, dtype=torch.float16, device="cuda").expand(M, N))
+
+
+def test_weights_of_another_width_are_refused():
+    block = ops.quant_sizes(QT)[1]
+    wide, _ = _weights(pad=block)
+    for dtype in (torch.float16, torch.float32):   # (the GEMM takes no 32-bit activations)
+        with pytest.raises(RuntimeError):
+            D.fused_mul_mat_gguf(_x(M, K, dtype=dtype), wide, QT)
+    at, x = {"gate": (0, N, wide.shape[1]), "up": (0, N, wide.shape[1])}, _x(M, K)
+    with pytest.raises(RuntimeError):
+        D.apply_linear(x, wide, QT, shard_ids=("gate", "up"), shard_offset_map=at, shard_weight_types={"gate": QT, "up": D.IQ2_S})
+
+
+def test_bytes_behind_the_last_block_are_no_weights():
+    padded, packed = _weights(pad=6)
+    for dtype in (torch.float16, torch.float32):
+        x = _x(M, K, dtype=dtype)
+        _close(D.fused_mul_mat_gguf(x, padded, QT), x @ _dense(packed, dtype).T)
+
+
+def test_packed_weights_of_another_integer_type():
+    w, packed = _weights()
+    x = _x(M, K)
+    _close(D.fused_mul_mat_gguf(x, w.view(torch.int8), QT), x @ _dense(packed).T)

@@ -156,8 +156,9 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t m = x->size(0), k = x->size(1), rows = w->size(0), rb = row_bytes((int)type, k);
   const Path path = mul_mat_path((int)type, m, rows);
   if (rb == 0 || w->size(1) < rb || rows == 0) Py_RETURN_NONE;
+  if (path == PATH_DENSE && w->size(1) != rb) Py_RETURN_NONE;   // (wider weights do not fit x in the product of a dense copy)
   if (!path_ok(path, (int)type, *x, *w, rows)) {
-    if (path != PATH_DENSE || w->size(1) != rb || !w->is_contiguous() || a[3] != Py_None || a[4] != Py_None) Py_RETURN_NONE;
+    if (path != PATH_DENSE || !w->is_contiguous() || a[3] != Py_None || a[4] != Py_None) Py_RETURN_NONE;
     at::Tensor y = dense_copy_product(*x, *w, (int)type, stream_of(dev));
     if (!y.defined()) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(y));
@@ -217,7 +218,9 @@ PyObject* merged_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
       Py_RETURN_NONE;
     const int64_t rows = p.end - p.start, rb = row_bytes((int)p.type, k);
     p.path = mul_mat_path((int)p.type, m, rows);
-    if (rows <= 0 || !path_ok(p.path, (int)p.type, *x, *w, rows) || p.start < 0 || p.end > w->size(0) || rb == 0 || p.rb < rb || p.rb > w->size(1)) Py_RETURN_NONE;
+    if (rows <= 0 || !path_ok(p.path, (int)p.type, *x, *w, rows) || p.start < 0 || p.end > w->size(0) || rb == 0 || p.rb < rb || p.rb > w->size(1) ||
+        (p.path == PATH_DENSE && p.rb != rb))
+      Py_RETURN_NONE;
     width += rows;
     if (!parts.empty() && parts.back().end == p.start && parts.back().type == p.type && parts.back().path == p.path)
       parts.back().end = p.end;

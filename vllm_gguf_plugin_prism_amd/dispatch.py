@@ -133,8 +133,9 @@ def fused_mul_mat_gguf(x, weight, weight_type: int, *, out=None, bias=None):
         if y is not None:
             return y
         block_size, type_size = ops.quant_sizes(weight_type)
-        packed = weight if weight.is_contiguous() else weight.contiguous()
-        dense = ops.ggml_dequantize(packed, weight_type, rows, packed.shape[1] // type_size * block_size, x.dtype)
+        blocks = weight.shape[1] // type_size            # (bytes behind the last whole block are no weights)
+        packed = weight[:, :blocks * type_size].contiguous()
+        dense = ops.ggml_dequantize(packed, weight_type, rows, blocks * block_size, x.dtype)
         y = x @ dense.T
     if bias is not None:
         y.add_(bias)

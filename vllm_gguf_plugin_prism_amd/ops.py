@@ -207,6 +207,13 @@ def ggml_dequant_gemm(W: torch.Tensor, X: torch.Tensor, quant_type: int, row: in
     return out
 
 
+def _whole_rows(W: torch.Tensor, quant_type: int, row: int, col: int) -> bool:
+    """Whether ``W`` holds ``row`` rows of ``col`` weights and nothing else: the product of a dense copy refuses weights of
+    another width than the activations'."""
+    qk, bs = quant_sizes(quant_type)
+    return W.shape[0] == row and col % qk == 0 and W.shape[1] == col // qk * bs
+
+
 def _dense_result_fits(X: torch.Tensor, row: int, out: torch.Tensor | None, bias: torch.Tensor | None, *inputs: torch.Tensor) -> bool:
     """Whether the result and the bias of a dense product lie as its kernel takes them.  ``y.add_(bias)`` and
     ``out.copy_(y)``, which it stands in for, take more: other types, strides and broadcast shapes, and a result that
@@ -231,7 +238,8 @@ def dense_linear(W: torch.Tensor, X: torch.Tensor, quant_type: int, row: int, *,
         return None
     vecs, col = X.shape
     if (X.dtype not in (torch.float16, torch.bfloat16) or not X.is_contiguous() or X.data_ptr() % 16
-            or W.data_ptr() % 2 or W.stride(0) % 2
+            or W.dim() != 2 or W.dtype != torch.uint8 or (W.shape[1] > 1 and W.stride(1) != 1) or W.data_ptr() % 2 or W.stride(0) % 2
+            or not _whole_rows(W, quant_type, row, col) or W.device != X.device
             or not _lib.lib().gguf_dense_linear_takes(int(quant_type), _code(X.dtype), row, col, vecs)
             or not _dense_result_fits(X, row, out, bias, W)):
         return None
