@@ -11,9 +11,11 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/EmptyTensor.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/ops/matmul.h>
 #include <ATen/hip/impl/HIPCachingAllocatorMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/core/GradMode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <hip/hip_runtime_api.h>
 
@@ -52,9 +54,22 @@ const at::Tensor* plain(PyObject* o, int dev) {
   const at::Tensor& t = THPVariable_Unpack(o);
   if (!t.defined() || !t.is_cuda() || t.get_device() != dev || t.layout() != at::kStrided) return nullptr;
   if (t.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::Functionalize, c10::DispatchKey::Negative,
-                                               c10::DispatchKey::Conjugate, c10::DispatchKey::FuncTorchBatched})))
+                                               c10::DispatchKey::Conjugate, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper})))
     return nullptr;
   return &t;
+}
+
+// Whether torch would do more in the dense path's `x @ dense.T` (then `add_` of the bias, `copy_` to the result) than
+// multiply: record it for a gradient, carry a tangent along, hand it to a tensor subclass, cast its operands.  A kernel
+// on raw pointers cannot stand in for that; dispatch.py then takes the two steps.
+bool product_is_watched(PyObject* const* objects, std::initializer_list<const at::Tensor*> tensors) {
+  for (const at::Tensor* t : tensors) {
+    PyObject* const o = *objects++;
+    if (!t) continue;
+    if (!THPVariable_CheckExact(o) || (at::GradMode::is_enabled() && t->requires_grad()) || t->_fw_grad(0).defined()) return true;
+  }
+  const at::Tensor& x = **tensors.begin();
+  return at::autocast::is_autocast_enabled(at::kCUDA) && at::autocast::get_autocast_dtype(at::kCUDA) != x.scalar_type();
 }
 
 // the current GPU, or -1 where a dispatch mode (tracing, fake tensors) watches torch's calls
@@ -158,7 +173,7 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (rb == 0 || w->size(1) < rb || rows == 0) Py_RETURN_NONE;
   if (path == PATH_DENSE && w->size(1) != rb) Py_RETURN_NONE;   // (wider weights do not fit x in the product of a dense copy)
   if (!path_ok(path, (int)type, *x, *w, rows)) {
-    if (path != PATH_DENSE || !w->is_contiguous() || a[3] != Py_None || a[4] != Py_None) Py_RETURN_NONE;
+    if (path != PATH_DENSE || !w->is_contiguous() || a[3] != Py_None || a[4] != Py_None || !THPVariable_CheckExact(a[0])) Py_RETURN_NONE;
     at::Tensor y = dense_copy_product(*x, *w, (int)type, stream_of(dev));
     if (!y.defined()) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(y));
@@ -177,6 +192,10 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!bias || bias->dim() != 1 || bias->size(0) != rows || bias->scalar_type() != x->scalar_type() || !bias->is_contiguous()) Py_RETURN_NONE;
     if (path == PATH_DENSE && out && out->is_alias_of(*bias)) Py_RETURN_NONE;
   }
+  if (path == PATH_DENSE) {
+    PyObject* const objects[] = {a[0], a[3], a[4]};
+    if (product_is_watched(objects, {x, out, bias})) Py_RETURN_NONE;
+  }
   at::Tensor y;
   int rc;
   {
@@ -188,7 +207,10 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     rc = run_shard(s, *x, dtype_code(x->scalar_type()), stream_of(dev));
   }
   if (rc != GGUF_OK) return fail(rc, path == PATH_MMVQ ? "ggml_mul_mat_vec_a8" : path == PATH_MMQ ? "ggml_mul_mat_a8" : "dense_linear");
-  if (out) return Py_NewRef(a[3]);
+  if (out) {
+    if (path == PATH_DENSE && !out->is_inference()) out->unsafeGetTensorImpl()->bump_version();   // (as copy_ does)
+    return Py_NewRef(a[3]);
+  }
   return THPVariable_Wrap(std::move(y));
 }
 
@@ -231,6 +253,10 @@ PyObject* merged_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (a[5] != Py_None) {
     bias = plain(a[5], dev);
     if (!bias || bias->dim() != 1 || bias->size(0) != width || bias->scalar_type() != x->scalar_type() || !bias->is_contiguous()) Py_RETURN_NONE;
+  }
+  if (std::any_of(parts.begin(), parts.end(), [](const Part& p) { return p.path == PATH_DENSE; })) {
+    PyObject* const objects[] = {a[0], a[5]};
+    if (product_is_watched(objects, {x, bias})) Py_RETURN_NONE;
   }
   at::Tensor y;
   int rc = GGUF_OK;

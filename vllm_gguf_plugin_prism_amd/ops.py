@@ -230,11 +230,27 @@ def _dense_result_fits(X: torch.Tensor, row: int, out: torch.Tensor | None, bias
     return all(t is None or t.untyped_storage().data_ptr() != held for t in (X, bias, *inputs))
 
 
+def _product_is_watched(X: torch.Tensor, *others: torch.Tensor | None) -> bool:
+    """Whether torch would do more in ``X @ dense.T`` (then ``add_`` of a bias, ``copy_`` to a result) than multiply: record
+    it for a gradient, carry a tangent along, map it over a batch, show it to a dispatch mode or a tensor subclass, cast
+    its operands.  No kernel launched on raw pointers can stand in for such a product."""
+    if torch._C._len_torch_dispatch_stack() or torch.autograd.forward_ad._current_level >= 0:
+        return True
+    if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != X.dtype:
+        return True
+    graph = torch.is_grad_enabled()
+    for t in (X, *others):
+        if t is not None and (type(t) not in (torch.Tensor, torch.nn.Parameter) or torch._C._functorch.is_functorch_wrapped_tensor(t)
+                              or t.layout != torch.strided or t.is_neg() or (graph and t.requires_grad)):
+            return True
+    return False
+
+
 def dense_linear(W: torch.Tensor, X: torch.Tensor, quant_type: int, row: int, *, out: torch.Tensor | None = None,
                  bias: torch.Tensor | None = None) -> torch.Tensor | None:
     """``X @ dequant(W)^T`` of a codebook format with the weights rounded to X's dtype (csrc/dense_core.h), or ``None`` for
     a call that kernel does not serve.  ``out`` / ``bias`` / sliced ``W``: as for :func:`ggml_mul_mat_vec_a8`."""
-    if X.dim() != 2:                         # (the product of a dense copy takes any number of leading dimensions)
+    if X.dim() != 2 or _product_is_watched(X, out, bias):   # (the product of a dense copy takes any number of leading dimensions)
         return None
     vecs, col = X.shape
     if (X.dtype not in (torch.float16, torch.bfloat16) or not X.is_contiguous() or X.data_ptr() % 16
@@ -250,6 +266,8 @@ def dense_linear(W: torch.Tensor, X: torch.Tensor, quant_type: int, row: int, *,
         rc = _lib.lib().gguf_dense_linear(W.data_ptr(), w_pitch, X.data_ptr(), _code(X.dtype), ws.data_ptr(), out.data_ptr(), ldy,
                                           bias.data_ptr() if bias is not None else None, int(quant_type), row, col, vecs, nbytes, _stream(X))
     _lib.check(rc, "dense_linear")
+    if not out.is_inference():
+        torch.autograd.graph.increment_version(out)   # (as copy_ does: a graph that saved the old values is told)
     return out
 
 
