@@ -83,22 +83,26 @@ int gguf_dequantize_rows(const void* W, int type, const int64_t* row_ids, int64_
 int gguf_mmvq(const void* W, const void* x, int xdtype, void* q8_workspace, void* Y, int type, int64_t N, int64_t K,
               int64_t M, gguf_stream_t stream);
 
-/* Same contraction, prefill path on int8 MFMA.
+/* Same contraction, prefill path on the matrix unit.
  * Replaces ggml_mul_mat_a8 (gguf_kernel.cu:220-290, mmq.cuh:2-610). */
 int gguf_mmq(const void* W, const void* x, int xdtype, void* q8_workspace, void* Y, int type, int64_t N, int64_t K,
              int64_t M, gguf_stream_t stream);
 
 /* gguf_mmq with the arithmetic engine chosen by the caller.  The reference has one engine (dp4a, mmq.cuh:2-104);
- * this library has two:
+ * this library has two arithmetics, the first of them on two units:
  *   GGUF_MMQ_INT8  int8 MFMA on the block codes, block scales applied in fp32: the reference's arithmetic, differing
- *                  only in the order of the fp32 additions.  This is what gguf_mmq runs.
+ *                  only in the order of the fp32 additions.
  *   GGUF_MMQ_HALF  half-precision MFMA on operands that carry their scales (activation d8*q and weight d*q, each
  *                  rounded to half): about 1.8 times faster, relative deviation about 2e-4 in the l2 norm, below
  *                  the rounding of a half or bfloat16 result -- but not the reference's arithmetic, so only for
  *                  callers that ask.  Not for fp32 results; not for Q4_1 / Q5_1.
  *   GGUF_MMQ_AUTO  INT8; with M <= 8 the streaming GEMV kernel instead, switched to this operator's offset sums
  *                  (Q4_K, Q5_K, Q5_0 are the formats where the reference's GEMV and its tile GEMM form them
- *                  differently), which is exact in int8 and reads W once at the GEMV's rate.
+ *                  differently), which is exact in int8 and reads W once at the GEMV's rate; and for Q4_K, Q5_K and
+ *                  Q6_K at some hundred rows, where that is faster and workspace_bytes has room for the rows in
+ *                  half precision (gguf_mmq_workspace_bytes has), the same exact whole-number products on
+ *                  half-precision MFMA: quants and scale-times-code operands are whole numbers that half precision
+ *                  holds, their sums are whole numbers that fp32 holds.  This is what gguf_mmq runs.
  * workspace_bytes is the size of q8_workspace; 0 stands for the minimum, M * gguf_q8_1_row_bytes(K).  Given
  * gguf_mmq_workspace_bytes(M, N, K) bytes, either engine splits K over several workgroups per output tile where the
  * output tiles alone would leave much of the chip idle (few tokens, a narrow N with a long K, a sparse last round of
@@ -108,8 +112,8 @@ int gguf_mmq(const void* W, const void* x, int xdtype, void* q8_workspace, void*
 #define GGUF_MMQ_INT8 1
 #define GGUF_MMQ_HALF 2
 int64_t gguf_mmq_workspace_bytes(int64_t M, int64_t N, int64_t K);   /* room for either engine */
-/* The same for one engine (GGUF_MMQ_AUTO counts as GGUF_MMQ_INT8): only the half engine pays for the half-precision
- * copy of the rows (64 bytes per 32 values on top of the 44).  GGUF_MMQ_HALF needs at least its row region,
+/* The same for one engine (GGUF_MMQ_AUTO counts as GGUF_MMQ_INT8, and with this much room runs as it): only the half
+ * engine pays for the half-precision copy of the rows (64 bytes per 32 values on top of the 44).  GGUF_MMQ_HALF needs at least its row region,
  * M * (gguf_q8_1_row_bytes(K) + 2 * (roundup(K, 512) + 128)) bytes, and returns GGUF_ERR_WORKSPACE below that; for it
  * workspace_bytes = 0 is not accepted. */
 int64_t gguf_mmq_workspace_bytes_engine(int64_t M, int64_t N, int64_t K, int engine);

@@ -44,3 +44,16 @@ def test_largest_sums_are_exact(qtype):
     x = np.where(rng.random((m, 1)) < 0.5, 1.0, -1.0).astype(np.float32) * (1.0 + np.arange(m, dtype=np.float32)[:, None] % 7) * np.ones((1, k), np.float32)
     x[:, ::5] *= 0.97
     _check(w.reshape(n, -1), x, qtype, n)
+
+
+# the int8 engine is there for who asks for it: the results differ in the order of the sums only
+@pytest.mark.parametrize("qtype", [o.Q4_K, o.Q5_K, o.Q6_K])
+def test_the_int8_engine_can_be_asked_for(qtype):
+    from vllm_gguf_plugin_prism_amd import ops
+    rng = np.random.default_rng(qtype)
+    n, k, m = 2048, 1024, 460
+    w, x = o.make_weights(rng, qtype, n, k), rng.standard_normal((m, k)).astype(np.float32)
+    wd, xd, want = torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda(), o.mul_mat_a8(w, x, qtype, n, "mmq")
+    auto, int8 = (ops.ggml_mul_mat_a8(wd, xd, qtype, n, engine=e).cpu().numpy() for e in ("auto", "int8"))
+    assert o.rel_l2(auto, want) <= 1e-5 and o.rel_l2(int8, want) <= 1e-5
+    assert not np.array_equal(auto, int8), "one engine for both"

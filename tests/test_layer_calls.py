@@ -72,3 +72,20 @@ def test_results_are_those_of_the_python_path(m, dt, monkeypatch):
     table = packed(D.Q6_K, 64, k)
     rows = torch.from_numpy(rng.integers(0, 64, size=(m, 2))).cuda()
     _both(monkeypatch, lambda: D.apply_gguf_embedding(rows, table, D.Q6_K, k, dt))
+
+
+def test_workspace_is_that_of_the_engine_that_runs():
+    from vllm_gguf_plugin_prism_amd import _lib, ops
+    L = _lib.lib()
+
+    def layer(qt, n, k, m):
+        qk, size = ops.quant_sizes(qt)
+        return L.gguf_mmq_layer_workspace_bytes(qt, n, k, m, k // qk * size)
+
+    n, k, m = 4096, 14336, 2048
+    int8 = L.gguf_mmq_workspace_bytes_engine(m, n, k, ops.MMQ_ENGINES["int8"])
+    for qt in (D.Q8_0, D.Q4_0, D.Q3_K):                       # formats whose products stay on the int8 unit
+        assert layer(qt, n, k, m) == int8
+    assert layer(D.Q4_K, n, k, 64) == L.gguf_mmq_workspace_bytes_engine(64, n, k, ops.MMQ_ENGINES["int8"])
+    # one form of the rows (halves, block scales, block sums) and at most two partial tiles per CU, not the int8 rows too
+    assert m * 2 * k <= layer(D.Q4_K, n, k, m) <= m * (2 * (k + 640) + k // 8 + k // 16) + 256 * 2 * 256 * 128 * 4

@@ -25,6 +25,7 @@
 // The same kernel runs the grouped MoE contraction (reference: csrc/gguf/moe.cuh:5-129):
 // token rows are gathered through sorted_token_ids, the weight base moves to the block's
 // expert, and results scatter to the rows the slots name.
+#include "dense_api.h"
 #include "mmq_f.h"
 #include "tile_stream.h"
 #include "mmq_formats.h"
@@ -823,12 +824,14 @@ extern "C" int64_t gguf_mmq_workspace_bytes_engine(int64_t M, int64_t N, int64_t
   if (engine == GGUF_MMQ_HALF) return mmq_rows_bytes(M, K, true) + gguf::mmq_half_partial_bytes((int)M, (int)N, (int)K);
   const int64_t pi = gguf::mmq_int_partial_bytes((int)M, (int)N, (int)K);
   const int64_t p16 = M <= gguf::MMQ_ROWS16_MAX ? gguf::mmq_rows16_partial_bytes((int)M, (int)N, (int)K) : 0;
-  int64_t behind = pi > p16 ? pi : p16;
-  if (M > gguf::MMQ_ROWS16_MAX && K % 256 == 0) {   // (the type is not known here: room for the engine of the super-block formats, too)
-    const int64_t pf = gguf::mmqf_rows_bytes(M, K) + gguf::mmqf_plan((int)M, (int)N, (int)K, INT64_MAX).partial_bytes();
-    if (pf > behind) behind = pf;
-  }
-  return mmq_rows_bytes(M, K, false) + behind;
+  return mmq_rows_bytes(M, K, false) + (pi > p16 ? pi : p16);
+}
+
+extern "C" int64_t gguf_mmq_layer_workspace_bytes(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes) {
+  if (M <= 0 || N <= 0 || K <= 0 || M > 0x7FFFFFF0LL || N > 0x7FFFFFF0LL || K > 0x7FFFFFF0LL) return 0;
+  if (gguf::mmqf_takes(type, M, N, K, w_row_pitch_bytes))
+    return gguf::mmqf_rows_bytes(M, K) + gguf::mmqf_plan((int)M, (int)N, (int)K, INT64_MAX).partial_bytes();
+  return gguf_mmq_workspace_bytes_engine(M, N, K, GGUF_MMQ_INT8);
 }
 
 // room for either engine
@@ -903,6 +906,17 @@ int gguf::mmq_linear_impl(const void* W, int64_t w_row_pitch_bytes, const void* 
     const int rc = mmvq_any(type, W, x, q8_workspace, Y, xdtype, N, K, M, s, lt);
     if (rc != GGUF_NOT_TAKEN) return rc;
   }
+  if (engine == GGUF_MMQ_AUTO && mmqf_takes(type, M, N, K, w_row_pitch_bytes) && ((uintptr_t)q8_workspace & 15) == 0) {
+    // the same whole-number products on the half-precision matrix unit, where there is room for its form of the rows
+    const int64_t half_rows = mmqf_rows_bytes(M, K);
+    if (workspace_bytes >= half_rows) {
+      const MmqfRows rows = mmqf_rows(q8_workspace, M, K);
+      int rc = quantize_whole(x, xdtype, rows, M, K, s);
+      if (rc != GGUF_OK) return rc;
+      const MmqfCall c = {W, rows, Y, xdtype, (int)M, (int)N, (int)K, (float*)((char*)q8_workspace + half_rows), workspace_bytes - half_rows, la};
+      return mmqf(type, c, s);
+    }
+  }
   if (engine == GGUF_MMQ_AUTO) engine = GGUF_MMQ_INT8;   // the reference's arithmetic; the half engine is for callers that ask
   float* partial = (float*)((char*)q8_workspace + rows_bytes);
   const int64_t partial_bytes = workspace_bytes > rows_bytes ? workspace_bytes - rows_bytes : 0;
@@ -911,14 +925,6 @@ int gguf::mmq_linear_impl(const void* W, int64_t w_row_pitch_bytes, const void* 
     const int rc = quantize_q8_1(x, xdtype, q8_workspace, M, K, s, 0, half_plane);
     if (rc != GGUF_OK) return rc;
     return mmq_half(W, q8_workspace, Y, xdtype, type, (int)M, (int)N, (int)K, partial, partial_bytes, s, la);
-  }
-  const int64_t half_rows = mmqf_rows_bytes(M, K);
-  if (partial_bytes >= half_rows && ((uintptr_t)partial & 15) == 0 && mmqf_takes(type, M, N, K, w_row_pitch_bytes)) {
-    const MmqfRows rows = mmqf_rows(partial, M, K);
-    int rc = quantize_whole(x, xdtype, rows, M, K, s);
-    if (rc != GGUF_OK) return rc;
-    const MmqfCall c = {W, rows, Y, xdtype, (int)M, (int)N, (int)K, (float*)((char*)partial + half_rows), partial_bytes - half_rows, la};
-    return mmqf(type, c, s);
   }
   int rc = quantize_q8_1(x, xdtype, q8_workspace, M, K, s);
   if (rc != GGUF_OK) return rc;

@@ -130,7 +130,7 @@ int run_shard(const Shard& s, const at::Tensor& x, int xcode, gguf_stream_t stre
     const c10::DataPtr ws = scratch(bytes);
     return gguf_dense_linear(s.w, s.pitch, x.const_data_ptr(), xcode, ws.get(), s.y, s.ldy, s.bias, s.type, s.rows, k, m, bytes, stream);
   }
-  const int64_t bytes = s.path == PATH_MMQ ? gguf_mmq_workspace_bytes_engine(m, s.rows, k, GGUF_MMQ_AUTO) : m * gguf_q8_1_row_bytes(k);
+  const int64_t bytes = s.path == PATH_MMQ ? gguf_mmq_layer_workspace_bytes(s.type, s.rows, k, m, s.pitch) : m * gguf_q8_1_row_bytes(k);
   const c10::DataPtr ws = scratch(bytes);
   if (s.path == PATH_MMVQ)
     return gguf_mmvq_linear(s.w, s.pitch, x.const_data_ptr(), xcode, ws.get(), s.y, s.ldy, s.bias, s.type, s.rows, k, m, stream);

@@ -12,6 +12,7 @@
 #include <algorithm>
 #include <optional>
 
+#include "../dense_api.h"
 #include "gguf_hip.h"
 
 namespace {
@@ -68,7 +69,8 @@ at::Tensor ggml_mul_mat_a8(const at::Tensor& W, const at::Tensor& X, int64_t typ
   const c10::hip::HIPGuardMasqueradingAsCUDA guard(X.device());
   const int64_t vecs = X.size(0), col = X.size(1);
   at::Tensor out = at::empty({vecs, row}, X.options());
-  const int64_t bytes = std::max<int64_t>(gguf_mmq_workspace_bytes_engine(vecs, row, col, GGUF_MMQ_AUTO), 16);
+  const int qk = gguf_block_elems((int)type);   // (0: a type that the call refuses)
+  const int64_t bytes = std::max<int64_t>(gguf_mmq_layer_workspace_bytes((int)type, row, col, vecs, qk ? col / qk * gguf_block_bytes((int)type) : 0), 16);
   at::Tensor ws = workspace(X, bytes);
   check(gguf_mmq_engine(W.data_ptr(), X.data_ptr(), dtype_code(X.scalar_type()), ws.data_ptr(), out.data_ptr(), (int)type, row, col, vecs,
                         GGUF_MMQ_AUTO, bytes, stream_of(X)),

@@ -172,14 +172,17 @@ def ggml_mul_mat_a8(W: torch.Tensor, X: torch.Tensor, quant_type: int, row: int,
     """Prefill GEMM ``q8_1(X) @ W^T`` on MFMA (reference: gguf_kernel.cu:220-290).
 
     ``engine``: ``"int8"`` keeps the reference's integer arithmetic (exact int8 dot products per block on int8 MFMA,
-    block scales in fp32) and is what ``"auto"`` means; ``"half"`` is opt-in and multiplies the dequantized operands
-    on half-precision MFMA (faster, about 2e-4 relative deviation from the integer result, half and bfloat16 results
-    only).  ``out`` / ``bias`` / sliced ``W``: as for :func:`ggml_mul_mat_vec_a8`."""
+    block scales in fp32).  ``"auto"`` keeps it, too, on the unit that is faster: Q4_K, Q5_K and Q6_K products of some
+    hundred rows run as exact whole numbers on half-precision MFMA (csrc/mmq_f_core.h).  ``"half"`` is opt-in and
+    multiplies the dequantized, rounded operands on half-precision MFMA (about 2e-4 relative deviation from the integer
+    result, half and bfloat16 results only).  ``out`` / ``bias`` / sliced ``W``: as for :func:`ggml_mul_mat_vec_a8`."""
     out, w_pitch, ldy = _shard_args(W, X, quant_type, row, out, bias)
     vecs, col = X.shape
     with _on_device_of(X):
-        # (only the half engine pays for the half-precision copy of the rows)
-        nbytes = max(_lib.lib().gguf_mmq_workspace_bytes_engine(vecs, row, col, MMQ_ENGINES[engine]), 16)
+        if engine == "auto":
+            nbytes = max(_lib.lib().gguf_mmq_layer_workspace_bytes(int(quant_type), row, col, vecs, w_pitch), 16)
+        else:
+            nbytes = max(_lib.lib().gguf_mmq_workspace_bytes_engine(vecs, row, col, MMQ_ENGINES[engine]), 16)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=X.device)
         rc = _lib.lib().gguf_mmq_linear(W.data_ptr(), w_pitch, X.data_ptr(), _code(X.dtype), ws.data_ptr(), out.data_ptr(), ldy,
                                         bias.data_ptr() if bias is not None else None, int(quant_type), row, col, vecs,
