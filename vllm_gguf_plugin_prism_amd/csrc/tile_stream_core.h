@@ -99,7 +99,7 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
   if (wg < total8) wg = (wg & 7) * (total8 >> 3) + (wg >> 3);
   // (the blocks of one expert are neighbours: they share its weights)
   const int col_wg = row_blocks == 1 ? wg : (int)__umulhi((uint32_t)wg, a.rb_inv), block = wg - col_wg * row_blocks;
-  const bool is_moe = moe.sorted_token_ids != nullptr;
+  const bool is_moe = RT == 1 && moe.sorted_token_ids != nullptr;   // (blocks of 16 slots only)
   if (is_moe) {
     const int live = moe.num_tokens_post_padded[0], e = moe.expert_ids[block];
     if (block * XR >= live || e < 0 || e > 255) return;     // (experts above 255: the reference's guard, moe.cuh:33)
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
   };
 
   // ---- fetching activations.  Lane l knows where row l % XR of the tile begins; quants go to LDS directly, one row's
-  // 1 KB per request, scales and sums through registers (four blocks of a row per thread) so that LDS holds them block-major.
+  // 1 KB per request, scales and sums (four blocks of a row per thread) take a detour so that LDS holds them block-major.
   uint32_t row_at;
   int pair_at = 0;                                          // MoE: the pair behind slot lane % XR
   const int nb = a.Kp >> 5, nkb = a.K >> 5;
@@ -211,25 +211,45 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
         }
     }
   };
-  // The first chunk's, counted by hand: between these two the registers belong to the loads (straight-line code).
+  // The first chunk's are asked for before the weights and must not wait for those, so the compiler cannot be the one that
+  // waits, and a register of its own is nothing that a load in flight may own.  They land in LDS, the 64 items of a wave
+  // one behind the other where the 64 items' transposed copy begins, and are spread out from there: the items of a wave
+  // are all rows of neighbouring blocks, so nobody else has anything in that place, and a wave's reads come before its writes.
+  const auto first_scales_lds = [&](int i) -> uint32_t {
+    const int it = 64 * (wave + NW * i), q = (it >> XR_LOG2) & (2 * PC - 1), plane = it >> (XR_LOG2 + 1 + a.pc_log2);
+    return (uint32_t)(xq_bytes + 4 * (plane * ts_scale_at<XR>(8 * PC) + ts_scale_at<XR>(4 * q)));
+  };
   const auto fetch_first_scales = [&]() {
 #pragma unroll
-    for (int i = 0; i < NS; ++i) asm volatile("global_load_dwordx4 %0, %1, %2" : "=&v"(sreg[i]) : "v"(scales_at(0, i)), "s"(ws) : "memory");
+    for (int i = 0; i < NS; ++i)
+      if (64 * (wave + NW * i) < items) ts_fetch(scales_at(0, i), ws, lds0 + first_scales_lds(i));
   };
-  const auto first_scales_landed = [&]() {
+  const auto place_first_scales = [&]() {
+    f32x4 v[NS];
 #pragma unroll
-    for (int i = 0; i < NS; ++i) asm volatile("" : "+v"(sreg[i]));
+    for (int i = 0; i < NS; ++i)
+      if (64 * (wave + NW * i) < items) v[i] = *(const f32x4*)(smem + first_scales_lds(i) + 16 * lane);
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      const int it = tid + 64 * NW * i, row = it & (XR - 1), q = (it >> XR_LOG2) & (2 * PC - 1), plane = it >> (XR_LOG2 + 1 + a.pc_log2);
+      float* const to = (float*)(smem + xq_bytes) + plane * ts_scale_at<XR>(8 * PC) + row;
+      if (64 * (wave + NW * i) < items)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) to[ts_scale_at<XR>(4 * q) + e * XR] = 4 * q + e < nkb ? v[i][e] : 0.0f;
+    }
   };
 
   if (is_moe) {
-    // (the weights do not wait for the routing)
-    int id;
-    asm volatile("global_load_dword %0, %1, %2" : "=&v"(id) : "v"(4 * (uint32_t)(block * XR + (lane & (XR - 1)))), "s"(moe.sorted_token_ids) : "memory");
+    // The weights do not wait for the routing: the pairs behind a block's slots come as scalar loads, which have a counter
+    // of their own, and are waited for behind the first requests of weights without waiting for the weights.
+    int slot_ids[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) slot_ids[r] = moe.sorted_token_ids[block * 16 + r];
 #pragma unroll
     for (int d = 0; d < D; ++d) request_next(d);
-    if (requested == D) ts_wait<D * NI>();
-    else ts_wait<0>();
-    asm volatile("" : "+v"(id));
+    int id = slot_ids[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) id = c == r ? slot_ids[r] : id;
     pair_at = id;
     row_at = (id < moe.num_pairs ? (moe.top_k == 1 ? (uint32_t)id : __umulhi((uint32_t)id, a.topk_inv)) : 0u) * a.ws_row_bytes;   // row 0 stands in for padding
     fetch_first_scales();
@@ -244,8 +264,7 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
     if (requested == D) ts_wait<D * NI>();
     else ts_wait<0>();
   }
-  first_scales_landed();
-  place_scales(0, 0);
+  place_first_scales();
   __syncthreads();
 
   const v4i seed = {kSeedBits, kSeedBits, kSeedBits, kSeedBits};
@@ -550,6 +569,7 @@ static inline int ts_ks(int np, double groups) {
 template <class F, int RT>
 static int ts_run_rt(const TsCall& c, hipStream_t stream) {
   const int np = (c.K + 255) / 256;
+  if (RT != 1 && c.moe.sorted_token_ids) return GGUF_NOT_TAKEN;
   if (c.gate.rows) {
     if constexpr (RT == 1) return ts_launch<F, 1, true, false>(c, 1, stream);
     return GGUF_NOT_TAKEN;
