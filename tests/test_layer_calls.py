@@ -1,5 +1,6 @@
 """The compiled layer calls (csrc/torch_binding/gguf_calls.cpp): the path they pick is dispatch.py's, what they do not
-serve falls back to Python, and their results are those of the Python path bit for bit."""
+serve falls back to Python, and their results are those of the Python path bit for bit, merged shards' to the order of a
+32-bit sum."""
 import numpy as np
 import pytest
 import torch
@@ -89,3 +90,53 @@ def test_workspace_is_that_of_the_engine_that_runs():
     assert layer(D.Q4_K, n, k, 64) == L.gguf_mmq_workspace_bytes_engine(64, n, k, ops.MMQ_ENGINES["int8"])
     # one form of the rows (halves, block scales, block sums) and at most two partial tiles per CU, not the int8 rows too
     assert m * 2 * k <= layer(D.Q4_K, n, k, m) <= m * (2 * (k + 640) + k // 8 + k // 16) + 256 * 2 * 256 * 128 * 4
+
+
+def _merged(rng, parts, k):
+    """The merged tensor of shards q, k, v with these (type, rows), the map of the shards and their types."""
+    packed = [torch.from_numpy(synth.make_weights(rng, qt, n, k)).cuda() for qt, n in parts]
+    w = torch.zeros(sum(n for _, n in parts), max(p.shape[1] for p in packed), dtype=torch.uint8, device="cuda")
+    at, row = {}, 0
+    for i, p in zip("qkv", packed):
+        w[row:row + p.shape[0], :p.shape[1]] = p
+        at[i] = (row, row + p.shape[0], p.shape[1])
+        row += p.shape[0]
+    return w, at, {i: qt for i, (qt, _) in zip("qkv", parts)}
+
+
+# q and k are one matrix to the compiled call and two to Python: every path, at sizes where the two split K differently
+@pytest.mark.gpu
+@pytest.mark.parametrize("qt,dt,m,rows,k", [
+    (D.Q4_K, torch.float32, 1, (2048, 512), 4096), (D.Q8_0, torch.float32, 6, (4096, 1024), 2048), (D.Q4_K, torch.float32, 12, (4096, 1024), 4096),
+    (D.Q4_0, torch.float32, 40, (1024, 256), 4096), (D.Q6_K, torch.float32, 100, (3072, 1024), 2048), (D.Q4_K, torch.float32, 460, (4096, 1024), 2048),
+    (D.IQ4_XS, torch.bfloat16, 40, (1024, 512), 4096), (D.IQ4_XS, torch.float16, 300, (2560, 640), 2560)])
+def test_merged_shards_differ_by_the_order_of_a_sum(qt, dt, m, rows, k, monkeypatch):
+    rng = np.random.default_rng(m)
+    w, at, types = _merged(rng, [(qt, rows[0]), (qt, rows[1]), (D.Q5_K, 256)], k)
+    x = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).to(dt).cuda()
+    ids = ("q", "k", "v")
+    assert D._calls().merged_linear(x, w, list(ids), at, [types[i] for i in ids], None) is not None, "not served"
+    got = D.apply_linear(x, w, qt, shard_ids=ids, shard_offset_map=at, shard_weight_types=types)
+    with monkeypatch.context() as p:
+        p.setattr(D, "_CALLS", D._NoCalls)
+        want = D.apply_linear(x, w, qt, shard_ids=ids, shard_offset_map=at, shard_weight_types=types)
+    # 32-bit sums of K products in another order; in 16 bits the two may round to neighbours
+    rel = {torch.float32: 1e-6, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dt]
+    assert ((got.double() - want.double()).norm() / want.double().norm()).item() <= rel
+    assert torch.equal(got[:, sum(rows):], want[:, sum(rows):])
+
+
+# the codebook GEMM serves both shards but not the matrix that they are together: it is asked about what would run
+@pytest.mark.gpu
+def test_merged_shards_are_asked_about_as_one_matrix():
+    from vllm_gguf_plugin_prism_amd import _lib, ops
+    rng, m, n, k = np.random.default_rng(0), 1108, 1024, 2048
+    takes = lambda rows: _lib.lib().gguf_dense_linear_takes(D.IQ4_XS, ops._code(torch.float16), rows, k, m)  # noqa: E731
+    assert takes(n) and not takes(2 * n)
+    w, at, types = _merged(rng, [(D.IQ4_XS, n), (D.IQ4_XS, n), (D.IQ4_NL, n)], k)
+    x = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).to(torch.float16).cuda()
+    ids = ["q", "k", "v"]
+    assert D._calls().merged_linear(x, w, ids, at, [types[i] for i in ids], None) is None
+    got = D.apply_linear(x, w, D.IQ4_XS, shard_ids=ids, shard_offset_map=at, shard_weight_types=types)
+    want = [D.fused_mul_mat_gguf(x, w[a:b, :r].contiguous(), types[i]) for i, (a, b, r) in at.items()]
+    assert torch.equal(got, torch.cat(want, 1))

@@ -5,8 +5,9 @@
 //
 // Every function returns None for a call it does not serve (another device than the current one, tensors that are not
 // plain dense ones, a malformed shape, an unquantized type, ...) before anything is allocated or launched; dispatch.py
-// then takes its Python path, which raises what there is to raise.  The results are the same either way: same entry
-// points of the C ABI with the same arguments.
+// then takes its Python path, which raises what there is to raise.  Both make the same calls of the C ABI with the same
+// arguments, and so have the same results bit for bit, but for merged shards (merged_linear), whose sums may be split in
+// another order.
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -218,7 +219,9 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // whose types differ, in the order of shard_ids; shard_offset_map[id] = (first row, row behind the last, bytes of a row)
 // and types lists their ggml types.  Neighbouring shards of one type whose rows lie next to each other and which take
 // the same path are one matrix with more rows and so one call: q and k of a mixed recipe, [4096 + 1024, 4096] Q4_K,
-// 9.1 -> 5.6 us of kernel time.
+// 9.1 -> 5.6 us of kernel time.  The path is that of the shards, each by its own rows, as in the reference's policy; within
+// it, how many workgroups share a sum over K depends on the rows of the whole matrix, so a result may differ from the
+// single shard's by the order of a 32-bit sum.
 PyObject* merged_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 6) return PyErr_Format(PyExc_TypeError, "merged_linear takes 6 arguments"), nullptr;
   const int dev = current_gpu();
@@ -240,7 +243,7 @@ PyObject* merged_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
       Py_RETURN_NONE;
     const int64_t rows = p.end - p.start, rb = row_bytes((int)p.type, k);
     p.path = mul_mat_path((int)p.type, m, rows);
-    if (rows <= 0 || !path_ok(p.path, (int)p.type, *x, *w, rows) || p.start < 0 || p.end > w->size(0) || rb == 0 || p.rb < rb || p.rb > w->size(1) ||
+    if (rows <= 0 || p.start < 0 || p.end > w->size(0) || rb == 0 || p.rb < rb || p.rb > w->size(1) ||
         (p.path == PATH_DENSE && p.rb != rb))
       Py_RETURN_NONE;
     width += rows;
@@ -249,6 +252,8 @@ PyObject* merged_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     else
       parts.push_back(p);
   }
+  for (const Part& p : parts)
+    if (!path_ok(p.path, (int)p.type, *x, *w, p.end - p.start)) Py_RETURN_NONE;
   const at::Tensor* bias = nullptr;
   if (a[5] != Py_None) {
     bias = plain(a[5], dev);
