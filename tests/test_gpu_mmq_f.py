@@ -51,9 +51,44 @@ def test_largest_sums_are_exact(qtype):
 def test_the_int8_engine_can_be_asked_for(qtype):
     from vllm_gguf_plugin_prism_amd import ops
     rng = np.random.default_rng(qtype)
-    n, k, m = 2048, 1024, 460
+    n, k, m = 2176, 3584, 460
+    assert _taken(qtype, m, n, k)
     w, x = o.make_weights(rng, qtype, n, k), rng.standard_normal((m, k)).astype(np.float32)
     wd, xd, want = torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda(), o.mul_mat_a8(w, x, qtype, n, "mmq")
     auto, int8 = (ops.ggml_mul_mat_a8(wd, xd, qtype, n, engine=e).cpu().numpy() for e in ("auto", "int8"))
     assert o.rel_l2(auto, want) <= 1e-5 and o.rel_l2(int8, want) <= 1e-5
     assert not np.array_equal(auto, int8), "one engine for both"
+
+
+def _taken(qtype, m, n, k, pad=0):
+    from vllm_gguf_plugin_prism_amd import _lib, ops
+    qk, size = ops.quant_sizes(qtype)
+    return _lib.lib().gguf_mmq_layer_route(qtype, n, k, m, k // qk * size + pad) == 2
+
+
+# sizes that the cost rule sends here for all three formats: part of a tile of rows, its tiles cut into runs; one row and one
+# column over a tile; runs that begin and end inside tiles; a whole round and a shared rest, narrower than the rows
+@pytest.mark.parametrize("qtype", [o.Q4_K, o.Q5_K, o.Q6_K])
+@pytest.mark.parametrize("m,n,k,pad", [(200, 640, 768, 0), (257, 257, 768, 2), (460, 2176, 3584, 0), (255, 33000, 1280, 6)])
+def test_tile_edges_where_it_is_taken(qtype, m, n, k, pad):
+    assert _taken(qtype, m, n, k, pad)
+    rng = np.random.default_rng(m + k)
+    _check(o.make_weights(rng, qtype, n, k), rng.standard_normal((m, k)).astype(np.float32) + 0.3, qtype, n, pad,
+           rng.standard_normal(n).astype(np.float32))
+
+
+@pytest.mark.parametrize("qtype", [o.Q4_K, o.Q5_K, o.Q6_K])
+def test_largest_sums_are_exact_where_it_is_taken(qtype):
+    rng = np.random.default_rng(qtype)
+    n, k, m = 640, 768, 200
+    assert _taken(qtype, m, n, k)
+    w = o.make_weights(rng, qtype, n, k).reshape(n, k // 256, -1)
+    if qtype == o.Q6_K:
+        w[:, :, :192], w[:, :, 192:208] = 0, 0x80          # codes -32, scales -128
+        w[1::2, :, :208] = 0xFF                            # codes 31, scales -1
+        w[1::4, :, 192:208] = 0x7F                         # codes 31, scales 127
+    else:
+        w[:, :, 4:] = 0xFF                                 # scales and mins 63, codes 15 or 31
+    x = np.where(rng.random((m, 1)) < 0.5, 1.0, -1.0).astype(np.float32) * (1.0 + np.arange(m, dtype=np.float32)[:, None] % 7) * np.ones((1, k), np.float32)
+    x[:, ::5] *= 0.97
+    _check(w.reshape(n, -1), x, qtype, n)

@@ -140,3 +140,13 @@ def test_merged_shards_are_asked_about_as_one_matrix():
     got = D.apply_linear(x, w, D.IQ4_XS, shard_ids=ids, shard_offset_map=at, shard_weight_types=types)
     want = [D.fused_mul_mat_gguf(x, w[a:b, :r].contiguous(), types[i]) for i, (a, b, r) in at.items()]
     assert torch.equal(got, torch.cat(want, 1))
+
+
+# measured, us, half-precision unit / int8 unit: where either is the faster one by a third or more
+@pytest.mark.parametrize("qt,m,n,k,half", [
+    (D.Q4_K, 288, 2560, 1024, 0), (D.Q4_K, 384, 18944, 1024, 0), (D.Q5_K, 1536, 1024, 1024, 0), (D.Q6_K, 512, 8192, 2560, 0),      # 42 / 21, 85 / 53, 45 / 28, 94 / 70
+    (D.Q4_K, 160, 11008, 14336, 1), (D.Q5_K, 192, 11008, 11008, 1), (D.Q4_K, 256, 28672, 14336, 1), (D.Q4_K, 512, 4096, 14336, 1)])  # 147 / 264, 135 / 225, 335 / 547, 107 / 148
+def test_products_run_on_the_faster_unit(qt, m, n, k, half):
+    from vllm_gguf_plugin_prism_amd import _lib, ops
+    qk, size = ops.quant_sizes(qt)
+    assert _lib.lib().gguf_mmq_layer_route(qt, n, k, m, k // qk * size) == (2 if half else 0)

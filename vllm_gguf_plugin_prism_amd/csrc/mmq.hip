@@ -834,6 +834,11 @@ extern "C" int64_t gguf_mmq_layer_workspace_bytes(int type, int64_t N, int64_t K
   return gguf_mmq_workspace_bytes_engine(M, N, K, GGUF_MMQ_INT8);
 }
 
+extern "C" int gguf_mmq_layer_route(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes) {
+  if (M <= 0 || N <= 0 || K <= 0 || M > 0x7FFFFFF0LL || N > 0x7FFFFFF0LL || K > 0x7FFFFFF0LL) return 0;
+  return gguf::ts_dense_takes(type, M, N, K, w_row_pitch_bytes) ? 1 : gguf::mmqf_takes(type, M, N, K, w_row_pitch_bytes) ? 2 : 0;
+}
+
 // room for either engine
 extern "C" int64_t gguf_mmq_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   const int64_t a = gguf_mmq_workspace_bytes_engine(M, N, K, GGUF_MMQ_INT8), b = gguf_mmq_workspace_bytes_engine(M, N, K, GGUF_MMQ_HALF);

@@ -37,6 +37,8 @@ struct MmqfPlan {
 };
 MmqfPlan mmqf_plan(int M, int N, int K, int64_t partial_bytes_available);
 
+double mmq_int_us(int type, int M, int N, int K);   // mmq_i.hip
+
 bool mmqf_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch);
 int mmqf(int type, const MmqfCall& c, hipStream_t stream);
 

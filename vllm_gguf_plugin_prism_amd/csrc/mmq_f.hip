@@ -3,18 +3,28 @@
 
 namespace gguf {
 
+// About how long a product takes, us, quantizer included (as mmq_int_us, fitted to the same calls and right to about 8 %): a
+// super-block of a tile, the beginning and the store of a round of tiles, the partial tiles' way through memory and how
+// many of them are added one after the other, the rows of X, the result.
+static double mmqf_us(int type, int M, int N, int K) {
+  const MmqfPlan p = mmqf_plan(M, N, K, INT64_MAX);
+  const int nsb = K / 256, rounds = (p.whole + 255) / 256;
+  const double sb = type == T_Q4_K ? 5.85 : type == T_Q5_K ? 6.2 : 8.0;
+  double us = 6.5 + rounds * (nsb * sb + 8.6) + 1e-6 * M * (0.9 * K + 1.2 * N);
+  if (p.shared > 0) us += p.per * sb + (type == T_Q6_K ? 3.8 : 2.2) + 0.036 * (p.workers + p.shared) + 0.23 * nsb / p.per;
+  return us;
+}
+
 bool mmqf_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch) {
   if (type != T_Q4_K && type != T_Q5_K && type != T_Q6_K) return false;
   // (offsets inside the matrix and inside the rows of X are 32-bit)
   if (N * w_pitch > 0xFFFF0000ll || mmqf_rows_bytes(M, K) > 0xFFFF0000ll) return false;
   if ((M / 256 + 1) * (N / 128 + 1) * (K / 256) > 0x7FFFFFFFll) return false;   // (super-blocks of all tiles are counted in an int)
-  // Where it is faster than the int8 engine (us, this / int8).  Below 193 rows most of a tile would be padding; up to 320 the
-  // single row of tiles wants an output that is neither narrow nor much wider than the chip ([18944,3584] Q4_K, 256 rows
-  // 105 / 101, [1024,4096] 23.9 / 23.2, [4096,14336] 64 / 85, [14336,4096] 69 / 88).  Q6_K has two operands to multiply:
-  // from 448 rows on, and not on narrow outputs ([14336,4096] 384 rows 145 / 127, 512 rows 147 / 158; [1024,4096] 1024 rows
-  // 40 / 38).
-  if (type == T_Q6_K) return M >= 448 && N >= 2048;
-  return M >= 320 || (M > 192 && N >= 2048 && N <= 16384);
+  // Where it is the faster one by the two estimates.  Its tiles of 256 rows want rows, and a long K to be worth a beginning;
+  // us, this / int8: [2560,1024] Q4_K 288 rows 42 / 21, [18944,1024] 384 rows 85 / 53, [8192,2560] Q6_K 512 rows 94 / 70;
+  // [4096,14336] Q4_K 512 rows 107 / 148, [11008,14336] 160 rows 147 / 264, [28672,14336] 256 rows 335 / 547.  Over 5100 calls of
+  // random sizes the estimates lose 0.7 % against always taking the faster engine.
+  return M >= 128 && M <= 0x7FFFFFF0ll && mmqf_us(type, (int)M, (int)N, (int)K) < 0.97 * mmq_int_us(type, (int)M, (int)N, (int)K);
 }
 
 // (a pitch that is not a multiple of 4096 bytes: see q8_half_pitch)

@@ -25,7 +25,8 @@
 // Measured against the int8 engine, us per call with the quantizer: [4096,14336] Q4_K, 1531 rows 404 -> 288, 512 rows
 // 148 -> 107; [18944,3584] 512 rows 179 -> 139; Q6_K [4096,14336] 1531 rows 462 -> 389, [18944,3584] 512 rows 177 -> 176.
 // What bounds it now is power: on random operands the clock falls to about 2.0 GHz, at which the matrix instructions,
-// the multiply-adds and the operand reads of a step take about 0.45 us each; a step takes 1.2 us.  Tried and slower: four
+// the multiply-adds and the operand reads of a step take about 0.45 us each; a step takes 1.2 us, a super-block, which is
+// four steps and its end, 5.9 (Q6_K 8.0).  Tried and slower: four
 // waves per workgroup and two workgroups per CU (decoding twice), the two waves of a SIMD decoding at different times,
 // the fetches of X in front of the operand reads or spread over the step.
 #pragma once
