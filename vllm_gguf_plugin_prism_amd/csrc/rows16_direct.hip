@@ -420,6 +420,18 @@ static Direct16Plan direct16_plan(int M, int N, int K, int64_t partial_bytes_ava
   }
   return p;
 }
+// About how long a product of K-quants takes, quantizer included, us (see ts_us, tile_stream.hip): rounds of workgroups, the
+// column tiles of each, a second launch where K is split, the weights' and (two tiles of rows) the activations' way.
+double rows16_direct_us(int type, int M, int N, int K) {
+  struct Cost { double base, round, tile, split, weights, k; };
+  static const Cost cost[2][3] = {{{5.4, 0.6, 1.88, 2.9, 0.098, 0}, {5.6, 0, 2.46, 2.8, 0.123, 0}, {6.4, -0.6, 5.0, 3.4, 0.141, 0}},
+                                  {{3.3, 3.0, 2.92, 1.8, 0.039, 0.24}, {3.4, 3.0, 3.25, 1.9, 0.053, 0.20}, {3.3, 5.2, 4.28, 2.4, 0.023, 0.19}}};
+  const Cost& c = cost[M > 16][type - T_Q4_K];
+  const Direct16Plan p = direct16_plan(M, N, K, INT64_MAX);
+  const int slots = p.rt == 2 ? 256 : 512, rounds = (p.tiles * p.gsplits + slots - 1) / slots;
+  return c.base + rounds * (c.round + c.tile * p.np) + (p.gsplits > 1 ? c.split : 0) + 1e-6 * c.weights * N * K + 1e-3 * c.k * K;
+}
+
 int64_t rows16_direct_partial_bytes(int M, int N, int K) { return K % 256 || M > 32 ? 0 : direct16_plan(M, N, K, INT64_MAX).partial_bytes(); }
 
 // bytes of 256 values

@@ -4,6 +4,20 @@
 
 namespace gguf {
 
+constexpr int TS_NW = 8;       // waves per workgroup
+
+// KS waves share a column group where the output has fewer groups than the chip has waves: rounds of workgroups x (the
+// panels of a wave + a beginning and an end worth about five).
+static inline int ts_ks(int np, double groups) {
+  int best = 1;
+  double best_cost = 1e30;
+  for (int ks = 1; ks <= TS_NW; ks <<= 1) {
+    const double wgs = ceil(groups * ks / TS_NW), cost = ((np + ks - 1) / ks + 5.0) * ceil(wgs / 256.0);
+    if (cost < 0.97 * best_cost) { best_cost = cost; best = ks; }
+  }
+  return best;
+}
+
 // One call of the kernel, dense (moe.sorted_token_ids null) or per block of 16 RT slots.
 struct TsCall {
   const void* W;

@@ -21,40 +21,52 @@ static bool ts_size_ok(int64_t rows_w, int64_t w_pitch, int64_t rows_x, int64_t 
   return rows_w * w_pitch <= 0xFFFF0000ll && rows_x * q8_row_bytes(K) <= 0xFFFF0000ll;
 }
 
-// Where the kernel is the faster one, from sweeps of N 512 .. 28672, K 1024 .. 14336 and 5 .. 32 rows of X.  (us with the
-// quantizer's launch, this kernel / the other; the others are the GEMV up to 8 rows, the 16-row kernels above.)
+// About how long a product of K-quants takes on this kernel, quantizer included, us: rounds of workgroups on the chip, each
+// a beginning and its waves' panels, the weights' and the activations' way.  The same for the kernels that run otherwise:
+// the one that reads the packed blocks (rows16_direct_us), and up to eight rows and 8M weights the GEMV, whose time is the
+// rows of X that every workgroup quantizes and the columns.  Fitted to 4900 calls of 256 .. 28672 columns, K 512 ..
+// 18944 and 5 .. 32 rows of X; on 2250 others of random sizes right to 4 .. 5 % here, 4 % (two tiles of rows) and 8 .. 11 %
+// (one) there, so that they lose 0.3 to 0.5 % against always taking the faster kernel.
+struct TsCost { double base, round, panel, weights, k; };
+static double ts_us(int type, int M, int N, int K) {
+  static const TsCost cost[2][3] = {{{-0.4, 6.76, 0.50, 0.056, 0.50}, {-0.2, 6.70, 0.65, 0.062, 0.48}, {1.0, 5.58, 1.11, 0.071, 0.44}},      // Q4_K, Q5_K, Q6_K
+                                    {{-4.1, 10.4, 0.99, 0.057, 0.73}, {-3.3, 9.7, 1.13, 0.061, 0.71}, {-4.1, 10.4, 1.80, 0.075, 0.68}}};   // two tiles of rows
+  const TsCost& c = cost[M > 16][type - T_Q4_K];
+  const int np = (K + 255) / 256, groups = (N + 15) / 16, ks = ts_ks(np, groups);
+  const double rounds = ceil(ceil((double)groups * ks / TS_NW) / 256.0);
+  return c.base + rounds * (c.round + c.panel * ((np + ks - 1) / ks)) + 1e-6 * c.weights * N * K + 1e-3 * c.k * K;
+}
+double rows16_direct_us(int type, int M, int N, int K);   // rows16_direct.hip
+static double ts_others_us(int type, int M, int N, int K) {
+  const bool small = (int64_t)N * K < (8 << 20);
+  // (Q6_K's GEMV takes four rows: below 8M weights, too, it is the kernel of the packed blocks, but another line fits)
+  if (type == T_Q6_K && M <= 16 && small) return 8.8 + 1e-3 * (0.70 * N + 0.48 * K);
+  // (the GEMV's eight rows have no room in LDS from K = 16384 on)
+  if (type == T_Q6_K || M > 8 || !small || K >= 16384) return rows16_direct_us(type, M, N, K);
+  return (type == T_Q4_K ? 4.2 : 4.7) + 1e-3 * ((type == T_Q4_K ? 0.26 : 0.41) * N + 0.15 * (M + 0.5) * K) + 0.11e-6 * N * K;
+}
+
+// Where the kernel is the faster one.
 bool ts_dense_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch) {
   if (M < 5 || M > 32 || !ts_type_ok(type) || !ts_size_ok(N, w_pitch, M, K)) return false;
-  const int64_t weights = N * K;
-  // Few columns and a long K leave most CUs without a workgroup (K is shared by the waves of one, not by several).
-  if (N <= 2048 && K > (M <= 16 && (type == T_Q4_0 || type == T_Q8_0) ? 8192 : 4096)) return false;
-  if (type == T_Q4_0 || type == T_Q8_0) {
-    // The GEMV's waves hold all rows' sums: from seven rows on it falls behind where K is long ([4096,8192] Q4_0, 8 rows:
-    // 14.7 / 17.5; [4096,4096] 11.0 / 10.3).
-    // (rows that do not begin on 16 bytes are cut out of two reads each: [19504,6016] Q8_0, 8 rows: 38.6 / 33.6,
-    // [12240,18112] Q4_0, 16 rows: 59 / 50; [6544,18144] Q8_0 40.5 / 49.9)
-    const bool aligned = w_pitch % 16 == 0;
-    if (type == T_Q4_0 && !aligned && K >= 6000) return false;
-    if (M <= 8) return M >= 7 && K >= (aligned ? 5120 : 12000);
-    // Above: all, but for the sizes at which the other kernel's column tiles are one even round of the chip
-    // ([4096,4096] Q4_0, 16 rows: 11.3 / 10.4; [2048,4096] 10.8 / 12.3; [5120,4096] 12.6 / 14.2; [14336,4096] 18.0 / 21.8;
-    // Q8_0 11.3 / 11.9, 10.2 / 14.1, 12.7 / 18.4, 18.5 / 25.4).
-    return !(type == T_Q4_0 && M <= 16 && N <= 4096 && weights > 9000000 && weights < 20000000);
-  }
-  // K-quants: the kernel that reads the packed blocks reaches the same rate in the middle of the range and starts in 3 us less.
-  // Short rows ([6144,2048] Q4_K 9.0 / 10.4, [12288,1024] 8.7 / 12.5, Q6_K 11.8 / 13.8, 11.7 / 21.5; Q4_K [4096,2560] 9.8 / 8.4)
-  if (K <= 2048) return M >= 9 || type == T_Q6_K || N >= 6144;
-  // Narrow outputs ([2048,4096] Q4_K 9.8 / 11.0, Q6_K 12.1 / 13.3; [2048,3072] 9.4 / 8.2)
-  if (N <= 2048) return K > (type == T_Q6_K ? 3072 : 3584);
-  // Q6_K, whose other kernel reads nine fields per block: all but the middle ([4096,4096] 11.9 / 10.8, [6144,4096] 14.6 / 14.4,
-  // [14336,4096] 21.5 / 22.7 and at 32 rows 28.2 / 27.5, [19536,4096], which is 60 % of a round, 30.8 / 29.7; [8192,2560] 12.6 / 14.3, [28672,4096] 31.6 / 38.0, [12288,5120]
-  // 24.5 / 34.6, [4096,14336] 23.8 / 27.2 and at 32 rows 32.8 / 46.8)
-  if (type == T_Q6_K) return K >= 5120 || (N >= 24000 || (N >= 8192 && (K <= 3072 || (M <= 16 && N <= 16384))));
-  if (N > 4096 && N < 6144) return false;                   // (a round of workgroups and a quarter: [5120,12288] Q4_K 21.7 / 21.0)
-  // Two tiles of rows ([4096,8192] Q4_K, 32 rows: 18.3 / 20.6; [4096,14336] 26.9 / 35.2)
-  if (M > 16 && N >= 4096 && K >= 8192) return true;
-  // Large ones ([8192,8192] Q4_K 18.4 / 20.7, [28672,4096] 21.5 / 24.5, [28672,8192] 37.0 / 44.6; [16384,4096] 17.1 / 16.0)
-  return weights >= 110000000 || (weights >= 58000000 && K >= 8192);
+  // [11008,4096] Q4_K 24 rows, this / the other kernel: 19.9 / 39.1, [5120,4096] 14.7 / 25.6, [28672,1024] 5 rows 10.3 / 19.9; but
+  // [8192,3584] 12 rows 13.1 / 11.2, [1024,14336] 17.0 / 11.7, [4096,1024] 5 rows 7.6 / 5.7.
+  if (type >= T_Q4_K && type <= T_Q6_K) return ts_us(type, (int)M, (int)N, (int)K) < ts_others_us(type, (int)M, (int)N, (int)K);
+  // Q4_0, Q8_0, from the same sweeps (us, this / the other kernel: the GEMV up to 8 rows, the 16-row kernels above).
+  // Few columns and a long K leave most CUs without a workgroup, as K is shared by the waves of one and not by several
+  // ([512,14336] Q4_0 24 rows 26.1 / 17.7, [1024,14336] 12 rows 18.5 / 17.9; [2048,8192] 24 rows 18.1 / 19.2, Q8_0 16.9 / 22.1).
+  if (M <= 16 ? N <= 2048 && K > 8192 : K > 4096 && K > (type == T_Q8_0 ? 8 : 4) * N) return false;
+  // The GEMV's waves hold all rows' sums: from seven rows on it falls behind where K is long ([4096,8192] Q4_0, 8 rows:
+  // 15.2 / 18.5; [4096,4096] 10.9 / 10.7; Q8_0 16.4 / 17.7, 11.6 / 10.8).
+  // (rows that do not begin on 16 bytes are cut out of two reads each: [19504,6016] Q8_0, 8 rows: 38.6 / 33.6,
+  // [12240,18112] Q4_0, 16 rows: 59 / 50; [6544,18144] Q8_0 40.5 / 49.9)
+  const bool aligned = w_pitch % 16 == 0;
+  if (type == T_Q4_0 && !aligned && K >= 6000) return false;
+  if (M <= 8) return M >= 7 && K >= (aligned ? 5120 : 12000);
+  // Above: all, but for what the kernel that reads the packed Q4_0 blocks has done in one launch and a single round, K not
+  // split and the columns no more than the CUs hold: [4096,4096] 16 rows 11.1 / 10.3, [2048,3072] 10.1 / 9.0; where it is two
+  // launches, [2560,4096] 10.7 / 16.0, or two rounds, [5120,4096] 12.9 / 14.7, or the rows short, [4096,2048] 8.7 / 10.0, it falls behind.
+  return !(type == T_Q4_0 && M <= 16 && K > 2048 && K <= 4096 && K % 256 == 0 && N <= 4096 && (K < 4096 || N > 3056));
 }
 
 bool ts_moe_takes(int type, int64_t N, int64_t K, int64_t num_sorted, int64_t tokens, int64_t top_k) {

@@ -35,8 +35,6 @@
 
 namespace gguf {
 
-constexpr int TS_NW = 8;       // waves per workgroup
-
 struct TsArgs {
   int M, N, K, Kp;             // M: rows of X (dense)
   uint32_t w_pitch, ws_row_bytes;
@@ -552,18 +550,6 @@ static int ts_launch(const TsCall& c, int ks, hipStream_t stream) {
     case 3: return ts_launch_d<F, RT, GATE, SPLIT, 3>(c, ks, a, lds, stream);
     default: return ts_launch_d<F, RT, GATE, SPLIT, 2>(c, ks, a, lds, stream);
   }
-}
-
-// KS waves share a column group where the output has fewer groups than the chip has waves: rounds of workgroups x (the
-// panels of a wave + a beginning and an end worth about five).
-static inline int ts_ks(int np, double groups) {
-  int best = 1;
-  double best_cost = 1e30;
-  for (int ks = 1; ks <= TS_NW; ks <<= 1) {
-    const double wgs = ceil(groups * ks / TS_NW), cost = ((np + ks - 1) / ks + 5.0) * ceil(wgs / 256.0);
-    if (cost < 0.97 * best_cost) { best_cost = cost; best = ks; }
-  }
-  return best;
 }
 
 template <class F, int RT>
