@@ -9,18 +9,18 @@ static bool dense_type_ok(int type) { return block_elems(type) && type >= T_IQ2_
 // A plan for tiles of `mt` rows of X and about how many us it takes.  The tiles of the last, partly filled round are shared
 // by all workgroups where that is shorter than a round of its own: a run, the reduction's launch, and the partial tiles'
 // way through memory.
-static DensePlan dense_plan_for(int mt, int M, int N, int K, double* cost) {
+static TilePlan dense_plan_for(int mt, int M, int N, int K, double* cost) {
   const int units = (K + 255) / 256, slots = mt == 256 ? 256 : 512;
   // us per unit of a tile, measured where the chip is full (two workgroups per CU below 256 rows) and where a CU has one
   const double full = mt == 64 ? 4.6 : mt == 128 ? 6.4 : 5.5, alone = mt == 64 ? 3.3 : mt == 128 ? 3.8 : 5.5;
   const int64_t t = (int64_t)((M + mt - 1) / mt) * ((N + 127) / 128);
   const int rest = (int)(t % slots);
   const double whole = (double)(t / slots) * units * full;
-  const DensePlan plain = {mt, (int)t, 0, 0, 1};
+  const TilePlan plain = {mt, (int)t, 0, 0, 1};
   *cost = whole + (rest == 0 ? 0.0 : units * (rest <= 256 ? alone : 0.85 * full));
   if (rest == 0) return plain;
   const int per = (int)(((int64_t)rest * units + slots - 1) / slots), workers = (rest * units + per - 1) / per;
-  const DensePlan shared = {mt, (int)(t - rest), rest, workers, per};
+  const TilePlan shared = {mt, (int)(t - rest), rest, workers, per};
   const double c = whole + per * (workers <= 256 ? alone : full) + 3.0 + 0.012 * mt / 64 * (workers + rest);
   if (c >= *cost) return plain;
   *cost = c;
@@ -28,12 +28,12 @@ static DensePlan dense_plan_for(int mt, int M, int N, int K, double* cost) {
 }
 
 // Rows of X per tile: what M rows are had for in the least time (`least`, us).
-static DensePlan dense_plan(int M, int N, int K, double& least) {
-  DensePlan best = {};
+static TilePlan dense_plan(int M, int N, int K, double& least) {
+  TilePlan best = {};
   least = 1e300;
   for (int mt = 64; mt <= 256; mt *= 2) {
     double c;
-    const DensePlan p = dense_plan_for(mt, M, N, K, &c);
+    const TilePlan p = dense_plan_for(mt, M, N, K, &c);
     if (c < least) {
       least = c;
       best = p;
@@ -42,7 +42,7 @@ static DensePlan dense_plan(int M, int N, int K, double& least) {
   return best;
 }
 
-static int dense_any(int type, const DenseCall& c, const DensePlan& p, hipStream_t s) {
+static int dense_any(int type, const DenseCall& c, const TilePlan& p, hipStream_t s) {
   switch (type) {
     case T_IQ2_XXS: return dense_iq2_xxs(c, p, s);
     case T_IQ2_XS: return dense_iq2_xs(c, p, s);
@@ -91,7 +91,7 @@ extern "C" int gguf_dense_linear(const void* W, int64_t w_row_pitch_bytes, const
   if (N == 0 || M == 0) return GGUF_OK;
   if (2 * M * K > 0xFFFF0000LL || (M / 64 + 1) * (N / 128 + 1) * (K / 256 + 1) > 0x7FFFFFFFLL) return GGUF_ERR_SHAPE;
   double us;
-  const DensePlan p = dense_plan((int)M, (int)N, (int)K, us);
+  const TilePlan p = dense_plan((int)M, (int)N, (int)K, us);
   if (!W || !x || !Y || (p.shared && !workspace)) return GGUF_ERR_NULL;
   if (((uintptr_t)W & 1) || (w_row_pitch_bytes & 1) || ((uintptr_t)x & 15)) return GGUF_ERR_SHAPE;
   if (p.shared && (workspace_bytes < p.partial_bytes() || ((uintptr_t)workspace & 15))) return GGUF_ERR_WORKSPACE;

@@ -25,10 +25,9 @@
 namespace gguf {
 
 struct DenseArgs {
-  int M, N, K, units;                         // units: blocks of 256 values per row, the last one may be part of one
-  int tiles_m, whole, shared, workers, per;
-  int64_t w_pitch, ldy;
-  int quads;                                  // rows of Y take stores of four values
+  TileRuns r;                                 // (the last unit of a row may be part of one)
+  int K;
+  int64_t w_pitch;
 };
 
 template <typename T> struct DenseType;
@@ -44,7 +43,6 @@ template <> struct DenseType<bf16_t> {
 };
 
 typedef float dense_f16v __attribute__((ext_vector_type(16)));
-typedef float dense_f4v __attribute__((ext_vector_type(4)));
 typedef float dense_f2v __attribute__((ext_vector_type(2)));
 
 template <int J> struct DenseStep { static constexpr int value = J; };
@@ -52,23 +50,6 @@ template <int J> struct DenseStep { static constexpr int value = J; };
 template <int M_T> __host__ __device__ constexpr int dense_buffer_bytes() { return 128 * (M_T + 128); }
 template <class F, int M_T> __host__ __device__ constexpr size_t dense_lds() {
   return 2 * (size_t)dense_buffer_bytes<M_T>() + F::TABLE * sizeof(typename F::Entry);
-}
-
-// four neighbouring results of a row
-template <typename T>
-__device__ __forceinline__ void dense_store(dense_f4v v, int m, int n, T* Y, const T* bias, const DenseArgs& a) {
-  if (m >= a.M) return;
-  T* const y = Y + (int64_t)m * a.ldy + n;
-  if (a.quads && n + 3 < a.N) {
-    alignas(8) T o[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = finish<T>(v[e], bias, n + e);
-    *(uint2*)y = *(const uint2*)o;
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (n + e < a.N) y[e] = finish<T>(v[e], bias, n + e);
-  }
 }
 
 template <class F, int WM, int WN, int TM, int TN, int OCC, typename T>
@@ -84,20 +65,14 @@ __global__ __launch_bounds__(64 * WM * WN, 2 * OCC) void dense_kernel(const uint
   for (int i = tid; i < F::TABLE; i += 512) table[i] = F::entry(i);
   if (F::TABLE) __syncthreads();
 
-  // ---- which work: whole tiles in runs per XCD, then equal runs of units of the shared tiles
-  int wg = blockIdx.x;
-  const int whole8 = a.whole & ~7;
-  if (wg < whole8) wg = (wg & 7) * (whole8 >> 3) + (wg >> 3);
-  int sw = wg - a.whole;
-  const int shared8 = a.workers & ~7;
-  if (sw >= 0 && sw < shared8 && (a.whole & 7) == 0) sw = (sw & 7) * (shared8 >> 3) + (sw >> 3);
-  int unit = sw < 0 ? wg * a.units : a.whole * a.units + sw * a.per;
-  const int unit_end = sw < 0 ? unit + a.units : min((a.whole + a.shared) * a.units, unit + a.per);
+  const TileWork work = tile_work(a.r);
+  const int unit_end = work.end;
+  int unit = work.first;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
   for (int segment = 0; unit < unit_end; ++segment) {
-    const int tile = unit / a.units, u0 = unit - tile * a.units, u1 = min(a.units, u0 + unit_end - unit);
+    const int tile = unit / a.r.units, u0 = unit - tile * a.r.units, u1 = min(a.r.units, u0 + unit_end - unit);
     unit += u1 - u0;
-    const int m_base = (tile % a.tiles_m) * M_T, n_base = (tile / a.tiles_m) * N_T;
+    const int m_base = (tile % a.r.tiles_m) * M_T, n_base = (tile / a.r.tiles_m) * N_T;
     const int g0 = 4 * u0, g1 = min(4 * u1, (a.K + 63) >> 6), g_half = a.K & 63 ? a.K >> 6 : -1;   // g_half: a step of 32 values
 
     // ---- rows of X: a fetch puts its lanes' 16 bytes one behind the other, so the lane of slot l % 8 of a row asks for
@@ -105,7 +80,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2 * OCC) void dense_kernel(const uint
     const int x_piece = (lane & 7) ^ ((4 * wave + (lane >> 4)) & 7);
     uint32_t x_at[XI];
 #pragma unroll
-    for (int i = 0; i < XI; ++i) x_at[i] = (uint32_t)min(m_base + 8 * (wave + 8 * i) + (lane >> 3), a.M - 1) * (uint32_t)(2 * a.K) + 16 * x_piece;
+    for (int i = 0; i < XI; ++i) x_at[i] = (uint32_t)min(m_base + 8 * (wave + 8 * i) + (lane >> 3), a.r.M - 1) * (uint32_t)(2 * a.K) + 16 * x_piece;
     const auto fetch_x = [&](int g, int buf) {
 #pragma unroll
       for (int i = 0; i < XI; ++i) {
@@ -115,7 +90,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2 * OCC) void dense_kernel(const uint
     };
     // ---- weights: sixteen values, part w_p of row w_n's step
     const int w_n = tid >> 2, w_p = tid & 3, h = w_p & 1, w_swz = (w_n >> 1) & 7;
-    const uint8_t* const w_row = W + (int64_t)min(n_base + w_n, a.N - 1) * a.w_pitch;
+    const uint8_t* const w_row = W + (int64_t)min(n_base + w_n, a.r.N - 1) * a.w_pitch;
     const auto fetch_raw = [&](int g) {
       const int ib = 2 * g + (g == g_half ? 0 : w_p >> 1);   // sub-block of 32 of the row
       if constexpr (F::QK == 256) return F::fetch(w_row + (uint32_t)(g >> 2) * F::BS, ib & 7, h);
@@ -210,52 +185,26 @@ __global__ __launch_bounds__(64 * WM * WN, 2 * OCC) void dense_kernel(const uint
     }
 
     // ---- store: lane = one row of X, 16 features per tile in runs of four
-    float* const mine = u1 - u0 < a.units ? partial + (int64_t)(2 * sw + segment) * (M_T * N_T) : nullptr;
+    float* const mine = u1 - u0 < a.r.units ? partial + (int64_t)(2 * work.worker + segment) * (M_T * N_T) : nullptr;
 #pragma unroll
     for (int i = 0; i < TN; ++i)
 #pragma unroll
       for (int k = 0; k < TM; ++k)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const dense_f4v v = {acc[i][k][4 * q], acc[i][k][4 * q + 1], acc[i][k][4 * q + 2], acc[i][k][4 * q + 3]};
+          const tile_f4v v = {acc[i][k][4 * q], acc[i][k][4 * q + 1], acc[i][k][4 * q + 2], acc[i][k][4 * q + 3]};
           if (mine) {   // in the order of the registers: [wave][tile][run][lane] of four
-            *(dense_f4v*)(mine + (((wave * TN * TM + i * TM + k) * 4 + q) * 64 + lane) * 4) = v;
+            *(tile_f4v*)(mine + (((wave * TN * TM + i * TM + k) * 4 + q) * 64 + lane) * 4) = v;
           } else {
             const int m = m_base + 32 * (TM * wm + k) + lrow, n = n_base + 32 * (TN * wn + i) + 8 * q + 4 * lhalf;
-            dense_store(v, m, n, Y, bias, a);
+            tile_store(v, m, n, Y, bias, a.r);
           }
         }
   }
 }
 
-// Y tile = T(sum of its partial tiles) in the order of K; a workgroup per wave's share of a tile, a thread per run of four
-template <int WM, int WN, int TM, int TN, typename T>
-__global__ __launch_bounds__(256) void dense_reduce_kernel(const float* __restrict__ partial, T* __restrict__ Y, const T* __restrict__ bias, DenseArgs a) {
-  constexpr int M_T = 32 * WM * TM, N_T = 32 * WN * TN;
-  const int t = blockIdx.x, tile = a.whole + t, sub = blockIdx.y, q = threadIdx.x >> 6, lane = threadIdx.x & 63;   // sub: (wave, tile of the wave)
-  const int wave = sub / (TN * TM), i = sub / TM % TN, k = sub % TM, wm = wave / WN, wn = wave % WN;
-  const int m = (tile % a.tiles_m) * M_T + 32 * (TM * wm + k) + (lane & 31), n = (tile / a.tiles_m) * N_T + 32 * (TN * wn + i) + 8 * q + 4 * (lane >> 5);
-  // the workers whose runs of units meet this tile; a worker's second partial tile is the tile it entered last
-  const int first = t * a.units / a.per, last = ((t + 1) * a.units - 1) / a.per;
-  if ((first == last && t * a.units == first * a.per && a.per == a.units) || m >= a.M) return;   // (stored whole, or padding)
-  // (eight partial tiles asked for at a time: one after the other, sixteen of them take longer than the product did)
-  dense_f4v v = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int w0 = first; w0 <= last; w0 += 8) {
-    dense_f4v p[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int w = min(w0 + i, last);
-      p[i] = *(const dense_f4v*)(partial + (int64_t)(2 * w + t - w * a.per / a.units) * (M_T * N_T) + ((sub * 4 + q) * 64 + lane) * 4);
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (w0 + i <= last) v += p[i];
-  }
-  dense_store(v, m, n, Y, bias, a);
-}
-
 template <class F, int WM, int WN, int TM, int TN, int OCC, typename T>
-static int dense_launch(const DenseCall& c, const DensePlan& p, hipStream_t stream) {
+static int dense_launch(const DenseCall& c, const TilePlan& p, hipStream_t stream) {
   constexpr int M_T = 32 * WM * TM;
   constexpr size_t lds = dense_lds<F, M_T>();
   static_assert(OCC * lds <= 160 * 1024, "tile does not fit in LDS");
@@ -263,18 +212,17 @@ static int dense_launch(const DenseCall& c, const DensePlan& p, hipStream_t stre
   static std::atomic<uint64_t> done{0};
   allow_large_lds(kern, lds, done);
   const int64_t ldy = c.la.ldy ? c.la.ldy : (int64_t)c.N;
-  const DenseArgs a = {c.M, c.N, c.K, (c.K + 255) / 256, (c.M + M_T - 1) / M_T, p.whole, p.shared, p.workers, p.per,
-                       c.la.w_pitch ? c.la.w_pitch : (int64_t)(c.K / F::QK) * F::BS, ldy, ldy % 4 == 0 && ((uintptr_t)c.Y & 7) == 0};
+  const DenseArgs a = {tile_runs<T>(p, c.M, c.N, (c.K + 255) / 256, c.Y, ldy), c.K, c.la.w_pitch ? c.la.w_pitch : (int64_t)(c.K / F::QK) * F::BS};
   hipLaunchKernelGGL(kern, dim3(p.whole + p.workers), dim3(512), lds, stream, (const uint8_t*)c.W, (const char*)c.X, (T*)c.Y, c.partial,
                      (const T*)c.la.bias, a);
   if (p.shared > 0)
-    hipLaunchKernelGGL((dense_reduce_kernel<WM, WN, TM, TN, T>), dim3(p.shared, 8 * TM * TN), dim3(256), 0, stream, c.partial, (T*)c.Y,
-                       (const T*)c.la.bias, a);
+    hipLaunchKernelGGL((tile_reduce_kernel<WM, WN, TM, TN, T>), dim3(p.shared, 8 * TM * TN), dim3(256), 0, stream, c.partial, (T*)c.Y,
+                       (const T*)c.la.bias, a.r);
   return launch_status();
 }
 
 template <class F, typename T>
-static int dense_typed(const DenseCall& c, const DensePlan& p, hipStream_t s) {
+static int dense_typed(const DenseCall& c, const TilePlan& p, hipStream_t s) {
   switch (p.mt) {
     case 64: return dense_launch<F, 2, 4, 1, 1, 2, T>(c, p, s);
     case 128: return dense_launch<F, 4, 2, 1, 2, 2, T>(c, p, s);
@@ -283,7 +231,7 @@ static int dense_typed(const DenseCall& c, const DensePlan& p, hipStream_t s) {
 }
 
 template <class F>
-static int dense_fmt(const DenseCall& c, const DensePlan& p, hipStream_t s) {
+static int dense_fmt(const DenseCall& c, const TilePlan& p, hipStream_t s) {
   return c.dtype == GGUF_DTYPE_F16 ? dense_typed<F, _Float16>(c, p, s) : dense_typed<F, bf16_t>(c, p, s);
 }
 

@@ -1,6 +1,6 @@
 // The prefill GEMM of the super-block formats on the half-precision matrix unit (mmq_f_core.h), for the code that routes to it.
 #pragma once
-#include "gguf_common.h"
+#include "tile_runs.h"
 
 namespace gguf {
 
@@ -27,15 +27,7 @@ struct MmqfCall {
   LinearArgs la;
 };
 
-// How the tiles of one launch are handed out: `whole` tiles get a workgroup each; the super-blocks of the `shared` tiles
-// behind them, one tile after the other, are dealt to `workers` workgroups in runs of `per` (at most a tile's), which
-// leave fp32 partial tiles, two each at most.
-struct MmqfPlan {
-  int mt, nt;                  // rows of X and weight rows of a tile
-  int whole, shared, workers, per;
-  int64_t partial_bytes() const { return (int64_t)workers * 2 * mt * nt * 4; }
-};
-MmqfPlan mmqf_plan(int M, int N, int K, int64_t partial_bytes_available);
+TilePlan mmqf_plan(int M, int N, int K, int64_t partial_bytes_available);
 
 double mmq_int_us(int type, int M, int N, int K);   // mmq_i.hip
 

@@ -7,7 +7,7 @@ namespace gguf {
 // super-block of a tile, the beginning and the store of a round of tiles, the partial tiles' way through memory and how
 // many of them are added one after the other, the rows of X, the result.
 static double mmqf_us(int type, int M, int N, int K) {
-  const MmqfPlan p = mmqf_plan(M, N, K, INT64_MAX);
+  const TilePlan p = mmqf_plan(M, N, K, INT64_MAX);
   const int nsb = K / 256, rounds = (p.whole + 255) / 256;
   const double sb = type == T_Q4_K ? 5.85 : type == T_Q5_K ? 6.2 : 8.0;
   double us = 6.5 + rounds * (nsb * sb + 8.6) + 1e-6 * M * (0.9 * K + 1.2 * N);
@@ -42,14 +42,14 @@ int64_t mmqf_rows_bytes(int64_t M, int64_t K) {
 // 256 x 128 tiles, one workgroup per CU.  The tiles of the last, partly filled round are shared by all workgroups where
 // that is shorter than a round of its own: a run, its second beginning, and the partial tiles' way through memory (a
 // super-block of a tile takes about 6 us, writing and adding a partial tile 0.06).
-MmqfPlan mmqf_plan(int M, int N, int K, int64_t avail) {
+TilePlan mmqf_plan(int M, int N, int K, int64_t avail) {
   const int slots = 256, nsb = K / 256;
   const int64_t t = (int64_t)((M + 255) / 256) * ((N + 127) / 128);
   const int rest = (int)(t % slots);
-  const MmqfPlan plain = {256, 128, (int)t, 0, 0, 1};
+  const TilePlan plain = {256, (int)t, 0, 0, 1};
   if (rest == 0) return plain;
   const int per = (rest * nsb + slots - 1) / slots, workers = (rest * nsb + per - 1) / per;
-  const MmqfPlan p = {256, 128, (int)(t - rest), rest, workers, per};
+  const TilePlan p = {256, (int)(t - rest), rest, workers, per};
   return per + 2.0 + 0.011 * (workers + rest) < nsb + 1.0 && p.partial_bytes() <= avail ? p : plain;
 }
 

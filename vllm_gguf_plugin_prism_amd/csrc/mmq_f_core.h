@@ -38,7 +38,6 @@ namespace gguf {
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x4_m __attribute__((ext_vector_type(4)));
 typedef float f32x2_m __attribute__((ext_vector_type(2)));
 
 // Two whole numbers below 1024 out of the low bytes (or nibbles) of the halves of v as 1024 + x each.
@@ -171,9 +170,8 @@ struct FQ6_K {
 };
 
 struct MmqfArgs {
-  int M, N, nsb;               // rows of X, weight rows, super-blocks per row
-  int tiles_m, whole, shared, workers, per;   // tiles of one workgroup each; tiles shared by `workers`, `per` super-blocks each
-  int64_t w_pitch, ldy;
+  TileRuns r;                  // (units are super-blocks)
+  int64_t w_pitch;
   uint32_t x_pitch, rows;      // bytes between the rows of X; rows of the planes
 };
 
@@ -183,12 +181,15 @@ __device__ __forceinline__ void pin16(float (&v)[16]) {
   asm volatile("" : "+v"(v[8]), "+v"(v[9]), "+v"(v[10]), "+v"(v[11]), "+v"(v[12]), "+v"(v[13]), "+v"(v[14]), "+v"(v[15]));
 }
 
-template <class F, int M_T, int N_T>
-__host__ __device__ constexpr int mmqf_buffer_bytes() { return 128 * (M_T + F::PLANES * N_T); }
+// eight waves of TM x TN tiles of 32 x 32
+constexpr int MMQF_WM = 4, MMQF_WN = 2, MMQF_TM = 2, MMQF_TN = 2, MMQF_MT = 32 * MMQF_WM * MMQF_TM, MMQF_NT = 32 * MMQF_WN * MMQF_TN;
+
+template <class F>
+__host__ __device__ constexpr int mmqf_buffer_bytes() { return 128 * (MMQF_MT + F::PLANES * MMQF_NT); }
 // d8 [8][M_T], of two super-blocks; then of the one at hand, for its end: sums [M_T] of eight halves, d [N_T] and, with
 // offsets, -dmin [N_T] and mins [N_T] of eight halves
-template <class F, int M_T, int N_T>
-__host__ __device__ constexpr size_t mmqf_lds() { return 2 * (size_t)(mmqf_buffer_bytes<F, M_T, N_T>() + 32 * M_T) + 16 * M_T + (F::OFF ? 24 : 4) * N_T; }
+template <class F>
+__host__ __device__ constexpr size_t mmqf_lds() { return 2 * (size_t)(mmqf_buffer_bytes<F>() + 32 * MMQF_MT) + 16 * MMQF_MT + (F::OFF ? 24 : 4) * MMQF_NT; }
 
 // v, opaque to the compiler: what is formed from it is formed where it stands, not kept in registers over the loop
 __device__ __forceinline__ int afresh(int v) {
@@ -198,33 +199,26 @@ __device__ __forceinline__ int afresh(int v) {
 
 template <int J> struct StepIndex { static constexpr int value = J; };
 
-template <class F, int WM, int WN, int TM, int TN, typename T>
-__global__ __launch_bounds__(64 * WM * WN, 2) void mmqf_kernel(const uint8_t* __restrict__ W, const char* __restrict__ X,
+template <class F, typename T>
+__global__ __launch_bounds__(64 * MMQF_WM * MMQF_WN, 2) void mmqf_kernel(const uint8_t* __restrict__ W, const char* __restrict__ X,
                                                                const char* __restrict__ XD, const char* __restrict__ XS,
                                                                T* __restrict__ Y, float* __restrict__ partial,
                                                                const T* __restrict__ bias, MmqfArgs a) {
-  constexpr int NT = 64 * WM * WN, NWV = WM * WN, M_T = 32 * WM * TM, N_T = 32 * WN * TN;
-  constexpr int BUF = mmqf_buffer_bytes<F, M_T, N_T>(), PLANE_AT = 2 * BUF + 64 * M_T;
-  constexpr int PARTS = 4 * N_T / NT;                       // parts of a row's step that a thread decodes
+  constexpr int WN = MMQF_WN, TM = MMQF_TM, TN = MMQF_TN, NWV = MMQF_WM * WN, M_T = MMQF_MT, N_T = MMQF_NT;
+  constexpr int BUF = mmqf_buffer_bytes<F>(), PLANE_AT = 2 * BUF + 64 * M_T;
   constexpr int XI = M_T / 8 / NWV;                         // fetches of 8 rows of X per wave and step
-  static_assert(4 * N_T % NT == 0 && M_T % 64 == 0 && M_T % (8 * NWV) == 0, "tile and workgroup sizes must divide evenly");
+  static_assert(4 * N_T == 64 * NWV && M_T == 256, "a thread per part of a row's step; a fetch per row of block scales");
   extern __shared__ __align__(16) char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN, lrow = lane & 31, lhalf = lane >> 5;
 
-  // ---- which work (as in mmqi_kernel: whole tiles in runs per XCD), then an equal run of super-blocks of the shared tiles
-  int wg = blockIdx.x;
-  const int whole8 = a.whole & ~7;
-  if (wg < whole8) wg = (wg & 7) * (whole8 >> 3) + (wg >> 3);
-  int sw = wg - a.whole;
-  const int shared8 = a.workers & ~7;
-  if (sw >= 0 && sw < shared8 && (a.whole & 7) == 0) sw = (sw & 7) * (shared8 >> 3) + (sw >> 3);
-  int unit = sw < 0 ? wg * a.nsb : a.whole * a.nsb + sw * a.per;
-  const int unit_end = sw < 0 ? unit + a.nsb : min((a.whole + a.shared) * a.nsb, unit + a.per);
+  const TileWork work = tile_work(a.r);
+  const int unit_end = work.end;
+  int unit = work.first;
   for (int segment = 0; unit < unit_end; ++segment) {
-  const int tile = unit / a.nsb, sb0 = unit - tile * a.nsb, sb1 = min(a.nsb, sb0 + unit_end - unit);
+  const int tile = unit / a.r.units, sb0 = unit - tile * a.r.units, sb1 = min(a.r.units, sb0 + unit_end - unit);
   unit += sb1 - sb0;
-  const int m_base = (tile % a.tiles_m) * M_T, n_base = (tile / a.tiles_m) * N_T;
+  const int m_base = (tile % a.r.tiles_m) * M_T, n_base = (tile / a.r.tiles_m) * N_T;
 
   // ---- staging plans
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
@@ -242,29 +236,26 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void mmqf_kernel(const uint8_t* __
   // the planes of a super-block of the rows of X: d8 is 8 rows of M_T floats, the sums M_T rows of 16 bytes
   const auto fetch_d8 = [&](int sb, int pb) {
 #pragma unroll
-    for (int q = wave; q < M_T / 32; q += NWV)              // (1 KB each; 256 q is the float of the plane, of block 256 q / M_T)
-      fetch_lds(M_T >= 256 ? 16 * lane : 4 * (4 * lane / M_T * a.rows + 4 * lane % M_T), XD + 4 * ((int64_t)(8 * sb + 256 * q / M_T) * a.rows + m_base + 256 * q % M_T), lds0 + 2 * BUF + 32 * M_T * pb + 1024 * q);
+    for (int q = wave; q < 8; q += NWV)                     // (1 KB each, a block's)
+      fetch_lds(16 * lane, XD + 4 * ((int64_t)(8 * sb + q) * a.rows + m_base), lds0 + 2 * BUF + 32 * M_T * pb + 1024 * q);
   };
   const auto fetch_sums = [&](int sb) {
 #pragma unroll
     for (int q = wave; q < M_T / 64; q += NWV)
       fetch_lds(16 * lane, XS + 16 * ((int64_t)sb * a.rows + m_base + 64 * q), lds0 + PLANE_AT + 1024 * q);
   };
-  // weights: a thread has PARTS parts of one row's step
-  const int w_n = tid * PARTS >> 2, part0 = tid * PARTS & 3;
-  const uint32_t w_row = (uint32_t)min(n_base + w_n, a.N - 1) * (uint32_t)a.w_pitch;   // (the matrix is below 4 GB: mmqf_takes)
+  // weights: a thread has one part of a row's step
+  const int w_n = tid >> 2, part = tid & 3;
+  const uint32_t w_row = (uint32_t)min(n_base + w_n, a.r.N - 1) * (uint32_t)a.w_pitch;   // (the matrix is below 4 GB: mmqf_takes)
   typename F::Head hd;
   typename F::Scales sc;
-  typename F::Raw raw[PARTS];
-  const auto fetch_raw = [&](int g) {
-#pragma unroll
-    for (int i = 0; i < PARTS; ++i) raw[i] = F::fetch(W + (w_row + (uint32_t)(g >> 2) * F::BS), g & 3, part0 + i);
-  };
+  typename F::Raw raw;
+  const auto fetch_raw = [&](int g) { raw = F::fetch(W + (w_row + (uint32_t)(g >> 2) * F::BS), g & 3, part); };
   const auto fetch_head = [&](int sb) { hd = F::head(W + (w_row + (uint32_t)sb * F::BS)); };
   const auto stash_head = [&]() {
-    const int id = afresh(tid), n = id * PARTS >> 2;
+    const int id = afresh(tid), n = id >> 2;
     char* const p = smem + PLANE_AT;
-    if ((id * PARTS & 3) == 0) {
+    if ((id & 3) == 0) {
       *(float*)(p + 16 * M_T + 4 * n) = F::d(hd);
       if (F::OFF) {
         *(float*)(p + 16 * M_T + 4 * N_T + 4 * n) = -F::dmin(hd);
@@ -274,18 +265,15 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void mmqf_kernel(const uint8_t* __
   };
   const auto stash = [&](auto step, int buf) {
     constexpr int J = decltype(step)::value;
-    const int id = afresh(tid), n = id * PARTS >> 2, p0 = id * PARTS & 3;
+    const int id = afresh(tid), n = id >> 2, p = id & 3;
     char* const row = smem + (buf * BUF + 128 * (M_T + n));
     const int s = (n >> 1) & 7;
+    uint4 lo[F::PLANES], hi[F::PLANES];
+    F::template decode<J>(raw, sc, p, lo, hi);
 #pragma unroll
-    for (int i = 0; i < PARTS; ++i) {
-      uint4 lo[F::PLANES], hi[F::PLANES];
-      F::template decode<J>(raw[i], sc, p0 + i, lo, hi);
-#pragma unroll
-      for (int pl = 0; pl < F::PLANES; ++pl) {
-        *(uint4*)(row + 128 * N_T * pl + 16 * ((p0 + i) ^ s)) = lo[pl];
-        *(uint4*)(row + 128 * N_T * pl + 16 * ((4 + p0 + i) ^ s)) = hi[pl];
-      }
+    for (int pl = 0; pl < F::PLANES; ++pl) {
+      *(uint4*)(row + 128 * N_T * pl + 16 * (p ^ s)) = lo[pl];
+      *(uint4*)(row + 128 * N_T * pl + 16 * ((4 + p) ^ s)) = hi[pl];
     }
   };
 
@@ -379,7 +367,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void mmqf_kernel(const uint8_t* __
       const int n = 32 * (TN * wn + i);
       __builtin_amdgcn_sched_barrier(0);
       f32x16 off[F::OFF ? TM : 1];
-      f32x4_m d[4], dm[4];
+      tile_f4v d[4], dm[4];
       if constexpr (F::OFF) {
         // (a contraction over eight: the upper half of the lanes holds values 8 .. 15, zeros)
         uint4 mv = *(const uint4*)(p + 8 * N_T + 16 * (n + row));
@@ -392,8 +380,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void mmqf_kernel(const uint8_t* __
       }
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        d[q] = *(const f32x4_m*)(p + 4 * (n + 8 * q + 4 * half));
-        if (F::OFF) dm[q] = *(const f32x4_m*)(p + 4 * N_T + 4 * (n + 8 * q + 4 * half));
+        d[q] = *(const tile_f4v*)(p + 4 * (n + 8 * q + 4 * half));
+        if (F::OFF) dm[q] = *(const tile_f4v*)(p + 4 * N_T + 4 * (n + 8 * q + 4 * half));
       }
 #pragma unroll
       for (int k = 0; k < TM; ++k) {
@@ -454,66 +442,39 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void mmqf_kernel(const uint8_t* __
   }
 
   // ---- store: lane = one row of X, 16 features per tile in runs of four
-  float* const mine = sb1 - sb0 < a.nsb ? partial + (int64_t)(2 * sw + segment) * (M_T * N_T) : nullptr;
+  float* const mine = sb1 - sb0 < a.r.units ? partial + (int64_t)(2 * work.worker + segment) * (M_T * N_T) : nullptr;
 #pragma unroll
   for (int i = 0; i < TN; ++i)
 #pragma unroll
     for (int k = 0; k < TM; ++k)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
+        const tile_f4v v = {acc[i][k][4 * q], acc[i][k][4 * q + 1], acc[i][k][4 * q + 2], acc[i][k][4 * q + 3]};
         if (mine) {   // in the order of the registers: [wave][tile][run][lane] of four
-          *(f32x4_m*)(mine + (((wave * TN * TM + i * TM + k) * 4 + q) * 64 + lane) * 4) = (f32x4_m){acc[i][k][4 * q], acc[i][k][4 * q + 1], acc[i][k][4 * q + 2], acc[i][k][4 * q + 3]};
+          *(tile_f4v*)(mine + (((wave * TN * TM + i * TM + k) * 4 + q) * 64 + lane) * 4) = v;
         } else {
-          const int m = m_base + 32 * (TM * wm + k) + lrow, n = n_base + 32 * (TN * wn + i) + 8 * q + 4 * lhalf;
-          if (m < a.M)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (n + e < a.N) Y[(int64_t)m * a.ldy + n + e] = finish<T>(acc[i][k][4 * q + e], bias, n + e);
+          tile_store(v, m_base + 32 * (TM * wm + k) + lrow, n_base + 32 * (TN * wn + i) + 8 * q + 4 * lhalf, Y, bias, a.r);
         }
       }
   }
 }
 
-// Y tile = T(sum of its partial tiles) in the order of K; a workgroup per wave's share of a tile, a thread per run of four
-template <int WM, int WN, int TM, int TN, typename T>
-__global__ __launch_bounds__(256) void mmqf_reduce_kernel(const float* __restrict__ partial, T* __restrict__ Y, const T* __restrict__ bias, MmqfArgs a) {
-  constexpr int M_T = 32 * WM * TM, N_T = 32 * WN * TN;
-  const int t = blockIdx.x, tile = a.whole + t, sub = blockIdx.y, q = threadIdx.x >> 6, lane = threadIdx.x & 63;   // sub: (wave, tile of the wave)
-  const int wave = sub / (TN * TM), i = sub / TM % TN, k = sub % TM, wm = wave / WN, wn = wave % WN;
-  // the workers whose runs of super-blocks meet this tile; a worker's second partial tile is the tile it entered last
-  const int first = t * a.nsb / a.per, last = ((t + 1) * a.nsb - 1) / a.per;
-  if (first == last && t * a.nsb == first * a.per && a.per == a.nsb) return;   // (stored whole)
-  f32x4_m v = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int w = first; w <= last; ++w) v += *(const f32x4_m*)(partial + (int64_t)(2 * w + t - w * a.per / a.nsb) * (M_T * N_T) + ((sub * 4 + q) * 64 + lane) * 4);
-  const int m = (tile % a.tiles_m) * M_T + 32 * (TM * wm + k) + (lane & 31), n = (tile / a.tiles_m) * N_T + 32 * (TN * wn + i) + 8 * q + 4 * (lane >> 5);
-  if (m >= a.M) return;
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-    if (n + e < a.N) Y[(int64_t)m * a.ldy + n + e] = finish<T>(v[e], bias, n + e);
-}
-
-template <class F, int WM, int WN, int TM, int TN, typename T>
-static int mmqf_launch(const MmqfCall& c, const MmqfPlan& p, hipStream_t stream) {
-  constexpr int M_T = 32 * WM * TM, N_T = 32 * WN * TN;
-  constexpr size_t lds = mmqf_lds<F, M_T, N_T>();
-  static_assert(lds <= 160 * 1024, "tile does not fit in LDS");
-  auto kern = mmqf_kernel<F, WM, WN, TM, TN, T>;
-  static std::atomic<uint64_t> done{0};
-  allow_large_lds(kern, lds, done);
-  const MmqfArgs a = {c.M, c.N, c.K / 256, (c.M + M_T - 1) / M_T, p.whole, p.shared, p.workers, p.per,
-                      c.la.w_pitch ? c.la.w_pitch : (int64_t)(c.K / 256) * F::BS, c.la.ldy ? c.la.ldy : (int64_t)c.N, (uint32_t)(2 * c.x.pitch), (uint32_t)c.x.rows};
-  hipLaunchKernelGGL(kern, dim3(p.whole + p.workers), dim3(64 * WM * WN), lds, stream, (const uint8_t*)c.W, (const char*)c.x.x,
-                     (const char*)c.x.d, (const char*)c.x.s, (T*)c.Y, c.partial, (const T*)c.la.bias, a);
-  if (p.shared > 0)
-    hipLaunchKernelGGL((mmqf_reduce_kernel<WM, WN, TM, TN, T>), dim3(p.shared, WM * WN * TM * TN), dim3(256), 0, stream, c.partial, (T*)c.Y,
-                       (const T*)c.la.bias, a);
-  return launch_status();
-}
-
 template <class F, typename T>
 static int mmqf_typed(const MmqfCall& c, hipStream_t stream) {
-  const MmqfPlan p = mmqf_plan(c.M, c.N, c.K, c.partial_bytes);
-  return mmqf_launch<F, 4, 2, 2, 2, T>(c, p, stream);
+  const TilePlan p = mmqf_plan(c.M, c.N, c.K, c.partial_bytes);
+  constexpr size_t lds = mmqf_lds<F>();
+  static_assert(lds <= 160 * 1024, "tile does not fit in LDS");
+  auto kern = mmqf_kernel<F, T>;
+  static std::atomic<uint64_t> done{0};
+  allow_large_lds(kern, lds, done);
+  const MmqfArgs a = {tile_runs<T>(p, c.M, c.N, c.K / 256, c.Y, c.la.ldy ? c.la.ldy : (int64_t)c.N),
+                      c.la.w_pitch ? c.la.w_pitch : (int64_t)(c.K / 256) * F::BS, (uint32_t)(2 * c.x.pitch), (uint32_t)c.x.rows};
+  hipLaunchKernelGGL(kern, dim3(p.whole + p.workers), dim3(64 * MMQF_WM * MMQF_WN), lds, stream, (const uint8_t*)c.W, (const char*)c.x.x,
+                     (const char*)c.x.d, (const char*)c.x.s, (T*)c.Y, c.partial, (const T*)c.la.bias, a);
+  if (p.shared > 0)
+    hipLaunchKernelGGL((tile_reduce_kernel<MMQF_WM, MMQF_WN, MMQF_TM, MMQF_TN, T>), dim3(p.shared, MMQF_WM * MMQF_WN * MMQF_TM * MMQF_TN), dim3(256),
+                       0, stream, c.partial, (T*)c.Y, (const T*)c.la.bias, a.r);
+  return launch_status();
 }
 
 template <class F>
