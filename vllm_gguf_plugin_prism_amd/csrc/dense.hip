@@ -87,7 +87,7 @@ extern "C" int gguf_dense_linear(const void* W, int64_t w_row_pitch_bytes, const
   if (!dense_type_ok(type)) return GGUF_ERR_TYPE;
   if (xdtype != GGUF_DTYPE_F16 && xdtype != GGUF_DTYPE_BF16) return GGUF_ERR_DTYPE;
   const int qk = block_elems(type);
-  if (N < 0 || M < 0 || K <= 0 || K % qk || w_row_pitch_bytes < K / qk * block_bytes(type) || y_row_pitch < N) return GGUF_ERR_SHAPE;
+  if (N < 0 || M < 0 || K <= 0 || N > 0x7FFFFFF0LL || M > 0x7FFFFFF0LL || K > 0x7FFFFFF0LL || K % qk || w_row_pitch_bytes < K / qk * block_bytes(type) || y_row_pitch < N) return GGUF_ERR_SHAPE;
   if (N == 0 || M == 0) return GGUF_OK;
   if (2 * M * K > 0xFFFF0000LL || (M / 64 + 1) * (N / 128 + 1) * (K / 256 + 1) > 0x7FFFFFFFLL) return GGUF_ERR_SHAPE;
   double us;
