@@ -12,10 +12,11 @@ Infinity Cache, with every input resident in HBM before the clock starts.
 
 Beside it:
   roofline      the GEMV kernel against the 8 TB/s HBM peak, timed per launch with HIP events over at least 100 launches
-  mmq           the second half of the metric: Q6_K prefill GEMM at M=512 in TOPS against the
-                5.03 POPS dense int8 MFMA peak, on the operator's default engine: exact int8 dot products on
-                v_mfma_i32_32x32x32_i8 with fp32 block scales, the reference's arithmetic.  The opt-in engine that
-                multiplies dequantized operands on half-precision MFMA is timed beside it as ``half_engine``
+  mmq           the second half of the metric: Q6_K prefill GEMM at M=512, [18944,3584] and [3584,18944], in TOPS against
+                the 5.03 POPS dense int8 MFMA peak, on ``engine="int8"``: exact int8 dot products on int8 MFMA with fp32
+                block scales, the reference's arithmetic.  Beside it ``default_engine``, which picks per shape between
+                that and exact whole-number products on half-precision MFMA, with the unit that ran and its peak, and
+                ``half_engine``, the opt-in that multiplies dequantized, rounded operands on half-precision MFMA
   other_configs the remaining BASELINE configurations (1: Q8_0 small, 2: batch sweep, 4: codebook formats, 5: MoE layer)
   cpu_baseline  the reference's CPU path (block dequantize + fp32 matmul) restated in numpy/torch,
                 timed on one host core on a bounded sample of the same workload
@@ -37,7 +38,7 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0          # MI355X HBM3E
 INT8_PEAK_TOPS = 5033.0        # dense int8 MFMA, double-K shapes v_mfma_i32_32x32x32_i8 / 16x16x64_i8 (256 CU x 8192 op/clk x 2.4 GHz)
 INT8_LEGACY_PEAK_TOPS = 2516.0 # the legacy-K shapes (v_mfma_i32_32x32x16_i8, 16x16x32_i8) run at half of it
-# the matrix instruction the integer engine issues per format: formats whose weight scale changes every 16 values
+# the matrix instruction the int8 engine issues per format: formats whose weight scale changes every 16 values
 # multiply 16 values at a time
 MMQ_INSTRUCTION = {14: "v_mfma_i32_32x32x16_i8", 11: "v_mfma_i32_32x32x16_i8"}
 F16_PEAK_TFLOPS = 2516.0       # dense half-precision MFMA
@@ -167,7 +168,9 @@ def _other_configs(rng, dev, w_14336x4096):
         res[f"config4_{name}_gemv_bs1"] = {"us": ms * 1e3, "GBps": gemv_bytes(qt, n, k, 1) / (ms * 1e-3) / 1e9}
         x = xs(256, k)
         ms = _timed_ms(lambda i: dispatch.fused_mul_mat_gguf(x, base, qt), 10)
-        res[f"config4_{name}_m256_dequant_then_gemm"] = {"us": ms * 1e3, "TFLOPS": 2.0 * 256 * n * k / (ms * 1e-3) / 1e12}
+        # (the key stems from the reference's two steps; one kernel now decodes the weights while it multiplies)
+        res[f"config4_{name}_m256_dequant_then_gemm"] = {"us": ms * 1e3, "TFLOPS": 2.0 * 256 * n * k / (ms * 1e-3) / 1e12,
+                                                         "runs": "codebook GEMM: weights rounded to the activations' dtype, half-precision MFMA"}
         ms = _timed_ms(lambda i: ops.ggml_mul_mat_a8(base, x, qt, n), 10)
         res[f"config4_{name}_m256_a8_gemm"] = {"us": ms * 1e3, "TOPS": 2.0 * 256 * n * k / (ms * 1e-3) / 1e12}
         del cp, base
@@ -188,7 +191,7 @@ def _other_configs(rng, dev, w_14336x4096):
                                          "distinct_expert_GBps": distinct * expert_bytes / (ms * 1e-3) / 1e9}
     # every entry against the roofline its operator is bound by: HBM for dequantize / GEMV / per-pair MoE (algorithmic
     # bytes; for the MoE layer each distinct expert once), int8 MFMA for the a8 tile GEMMs, half-precision MFMA for the
-    # library GEMM of the dequantize-then-GEMM route
+    # codebook formats' GEMM on unquantized activations
     for v in res.values():
         if "GBps" in v:
             v["roofline"] = {"bound": "hbm", "peak_GBps": HBM_PEAK_GBS, "frac": v["GBps"] / HBM_PEAK_GBS}
@@ -420,7 +423,9 @@ def main() -> int:
 
     # ---------------------------------------------------------------- config 3: Q6_K MMQ at M=512
     if not args.no_mmq:
-        tables = {"auto": {}, "half": {}}
+        from vllm_gguf_plugin_prism_amd import _lib
+
+        tables = {"int8": {}, "auto": {}, "half": {}}
         for n, k in CFG3_SHAPES:
             w = np.concatenate([synth.make_weights(rng, Q6_K, min(2048, n - r), k) for r in range(0, n, 2048)], axis=0)
             wd = torch.from_numpy(w).to(dev)
@@ -428,10 +433,14 @@ def main() -> int:
                 x = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).to(torch.float16).to(dev)
                 for engine, table in tables.items():
                     call = lambda i, engine=engine: ops.ggml_mul_mat_a8(wd, x, Q6_K, n, engine=engine)  # noqa: E731
+                    if not args.profile:
+                        _timed_ms(call, 20)   # (untimed: whichever engine came first paid 7 % for the clocks coming up)
                     ms = _timed_ms(call, 20, eager=args.profile)
                     tops = 2.0 * m * n * k / (ms * 1e-3) / 1e12
-                    table[f"{n}x{k}@M{m}"] = {"ms": ms, "TOPS": tops, "frac_int8_peak": tops / INT8_PEAK_TOPS,
-                                              "frac_int8_legacy_k_peak": tops / INT8_LEGACY_PEAK_TOPS}
+                    on_half = engine == "half" or (engine == "auto" and _lib.lib().gguf_mmq_layer_route(Q6_K, n, k, m, k // 256 * 210) == 2)
+                    table[f"{n}x{k}@M{m}"] = {"ms": ms, "TOPS": tops, "unit": "half-precision MFMA" if on_half else "int8 MFMA",
+                                              **({"frac_f16_peak": tops / F16_PEAK_TFLOPS} if on_half else
+                                                 {"frac_int8_peak": tops / INT8_PEAK_TOPS, "frac_int8_legacy_k_peak": tops / INT8_LEGACY_PEAK_TOPS})}
             del wd
         ops_total = sum(2.0 * 512 * n * k for n, k in CFG3_SHAPES)
 
@@ -439,10 +448,10 @@ def main() -> int:
             t_total = sum(v["ms"] for key, v in table.items() if key.endswith("@M512")) * 1e-3
             return ops_total / t_total / 1e12
 
-        tops512, half512 = at_m512(tables["auto"]), at_m512(tables["half"])
+        tops512, auto512, half512 = at_m512(tables["int8"]), at_m512(tables["auto"]), at_m512(tables["half"])
         out["mmq"] = {
             "metric": "Q6_K MMQ int8 TOPS @M=512", "value": tops512, "unit": "TOPS",
-            "engine": "gguf_mmq's default: exact int8 dot products per block on int8 MFMA, fp32 block scales",
+            "engine": "engine='int8': exact int8 dot products per block on int8 MFMA, fp32 block scales",
             "matrix_instruction": MMQ_INSTRUCTION.get(Q6_K, "v_mfma_i32_32x32x32_i8")
                                   + " (Q6_K's weight scale changes every 16 values: the legacy-K shape, whose own peak is half the chip's)",
             "dtype": "int8 products, int32 sums per block, fp32 accumulation",
@@ -453,7 +462,10 @@ def main() -> int:
                                           "frac_of_legacy_k_peak": tops512 / INT8_LEGACY_PEAK_TOPS,
                                           "used_for_frac": "double_k_int8_peak_TOPS (the chip's dense int8 peak)"},
                          "traffic": {f"{n}x{k}": _traffic(f"mmqi_q6_k_{n}x{k}_m512") for n, k in CFG3_SHAPES}},
-            "per_shape": tables["auto"],
+            "per_shape": tables["int8"],
+            "default_engine": {"value": auto512, "unit": "TOPS", "per_shape": tables["auto"],
+                               "note": "engine='auto', what gguf_mmq and the dispatch run: the same exact whole-number products, per shape "
+                                       "on int8 MFMA or, where its cost estimate is lower, on v_mfma_f32_32x32x16_f16"},
             "half_engine": {"value": half512, "unit": "TOPS", "frac_of_f16_mfma_peak": half512 / F16_PEAK_TFLOPS,
                             "per_shape": tables["half"],
                             "note": "engine='half', opt-in: dequantized operands on v_mfma_f32_32x32x16_f16; not the "

@@ -24,9 +24,10 @@
 //
 // Measured against the int8 engine, us per call with the quantizer: [4096,14336] Q4_K, 1531 rows 404 -> 288, 512 rows
 // 148 -> 107; [18944,3584] 512 rows 179 -> 139; Q6_K [4096,14336] 1531 rows 462 -> 389, [18944,3584] 512 rows 177 -> 176.
-// What bounds it now is power: on random operands the clock falls to about 2.0 GHz, at which the matrix instructions,
-// the multiply-adds and the operand reads of a step take about 0.45 us each; a step takes 1.2 us, a super-block, which is
-// four steps and its end, 5.9 (Q6_K 8.0).  Tried and slower: four
+// What bounds it now is vector issue beside the matrix unit, at a clock that falls to about 2.0 GHz under this load: by
+// counters ([4096,14336] Q4_K, 1531 rows) the vector ALU issues in 64 % of the SIMD cycles and the matrix unit is busy in
+// 32 %, Q6_K 52 % and 45 %.  The matrix instructions, the multiply-adds and the operand reads of a step take about 0.45 us
+// each; a step takes 1.2 us, a super-block, which is four steps and its end, 5.9 (Q6_K 8.0).  Tried and slower: four
 // waves per workgroup and two workgroups per CU (decoding twice), the two waves of a SIMD decoding at different times,
 // the fetches of X in front of the operand reads or spread over the step.
 #pragma once
