@@ -67,6 +67,36 @@ def test_replays_match_eager(case):
         assert torch.equal(out, eager), case
 
 
+# the layer calls (compiled, allocating per call) on the streaming tiles, with tiles whose K is shared on the whole-number
+# GEMM and on the codebook GEMM, and through merged shards
+@pytest.mark.parametrize("qtype,m,n,k", [(o.Q4_K, 12, 2080, 4096), (o.Q4_K, 200, 640, 768), (o.IQ4_XS, 70, 640, 1280)])
+def test_layer_calls_replay_as_eager(qtype, m, n, k):
+    from vllm_gguf_plugin_prism_amd import _lib, dispatch
+    rng = np.random.default_rng(m)
+    wn = o.make_weights(rng, qtype, n, k)
+    route = _lib.lib().gguf_mmq_layer_route(qtype, n, k, m, wn.shape[1])
+    assert route == {12: 1, 200: 2, 70: 0}[m] and (m != 70 or _lib.lib().gguf_dense_linear_workspace_bytes(n, k, m) > 0)
+    w, bias = _dev(wn), torch.randn(n, dtype=torch.float16, device="cuda")
+    xs = [torch.randn(m, k, dtype=torch.float16, device="cuda") for _ in range(3)]
+    x = xs[0].clone()
+    at, types = {"gate": (0, 320, wn.shape[1]), "up": (320, 640, wn.shape[1])}, {"gate": qtype, "up": qtype}
+
+    def fn():
+        return dispatch.fused_mul_mat_gguf(x, w, qtype, bias=bias), dispatch._calls().merged_linear(x, w, ["gate", "up"], at, [types["gate"], types["up"]], None)
+
+    assert fn()[1] is not None
+    graph, out = _capture(fn)
+    for xi in xs:
+        x.copy_(xi)
+        eager = [v.clone() for v in fn()]
+        torch.cuda.synchronize()
+        for v in out:
+            v.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out[0], eager[0]) and torch.equal(out[1], eager[1])
+
+
 @pytest.mark.parametrize("case", ["split_k", "few_rows"])
 def test_entry_point_without_workspace_replays_match_eager(case):
     """gguf_mmq_static is meant for callers under graph capture: gguf_mmq_static_capacity() is called once beforehand

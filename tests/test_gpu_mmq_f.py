@@ -1,6 +1,6 @@
 """The prefill GEMM on the half-precision matrix unit (csrc/mmq_f_core.h) at the edges of its tiles and of the runs of
 super-blocks its workgroups share, and on the largest whole numbers its operands and sums have to hold, against the CPU
-oracle."""
+oracle; and the int8 engine on the same sizes, asked for by name."""
 import numpy as np
 import pytest
 import torch
@@ -21,7 +21,8 @@ def _check(w, x, qtype, n, pad=0, bias=None):
 
 
 # one super-block; one row over a tile in either direction with tiles cut into runs, a padded pitch; runs that begin and
-# end inside tiles; more tiles than CUs (whole rounds and a shared rest)
+# end inside tiles; more tiles than CUs (whole rounds and a shared rest).  (The cost rule leaves most of these to the int8
+# engine; the sizes further down are sent here.)
 @pytest.mark.parametrize("qtype", [o.Q4_K, o.Q5_K, o.Q6_K])
 @pytest.mark.parametrize("m,n,k,pad", [(448, 2048, 256, 0), (513, 2049, 1024, 2), (460, 2176, 2816, 0), (600, 11000, 512, 6)])
 def test_tile_edges(qtype, m, n, k, pad):
