@@ -168,3 +168,9 @@ def test_products_of_a_few_rows_run_on_the_faster_kernel(qt, m, n, k, stream):
     from vllm_gguf_plugin_prism_amd import _lib, ops
     qk, size = ops.quant_sizes(qt)
     assert _lib.lib().gguf_mmq_layer_route(qt, n, k, m, k // qk * size) == stream
+
+
+def test_codebook_gemm_declines_types_it_does_not_know():
+    from vllm_gguf_plugin_prism_amd import ops
+    w, x = torch.zeros(8, 136, dtype=torch.uint8), torch.zeros(40, 256, dtype=torch.float16)
+    assert ops.dense_linear(w, x, D.Q4_K, 8) is None and ops.dense_linear(w, x, 99, 8) is None

@@ -258,10 +258,10 @@ def dense_linear(W: torch.Tensor, X: torch.Tensor, quant_type: int, row: int, *,
     vecs, col = X.shape
     if (X.dtype not in (torch.float16, torch.bfloat16) or not X.is_contiguous() or X.data_ptr() % 16
             or W.dim() != 2 or W.dtype != torch.uint8 or (W.shape[1] > 1 and W.stride(1) != 1) or W.data_ptr() % 2 or W.stride(0) % 2
-            or not _whole_rows(W, quant_type, row, col) or W.device != X.device
-            or not _lib.lib().gguf_dense_linear_takes(int(quant_type), _code(X.dtype), row, col, vecs)
-            or not _dense_result_fits(X, row, out, bias, W)):
+            or W.device != X.device or not _lib.lib().gguf_dense_linear_takes(int(quant_type), _code(X.dtype), row, col, vecs)
+            or not _whole_rows(W, quant_type, row, col) or not _dense_result_fits(X, row, out, bias, W)):
         return None
+    given = out
     out, w_pitch, ldy = _shard_args(W, X, quant_type, row, out, bias)
     with _on_device_of(X):
         nbytes = _lib.lib().gguf_dense_linear_workspace_bytes(row, col, vecs)
@@ -269,7 +269,7 @@ def dense_linear(W: torch.Tensor, X: torch.Tensor, quant_type: int, row: int, *,
         rc = _lib.lib().gguf_dense_linear(W.data_ptr(), w_pitch, X.data_ptr(), _code(X.dtype), ws.data_ptr(), out.data_ptr(), ldy,
                                           bias.data_ptr() if bias is not None else None, int(quant_type), row, col, vecs, nbytes, _stream(X))
     _lib.check(rc, "dense_linear")
-    if not out.is_inference():
+    if given is not None and not out.is_inference():
         torch.autograd.graph.increment_version(out)   # (as copy_ does: a graph that saved the old values is told)
     return out
 
