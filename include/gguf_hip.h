@@ -99,9 +99,9 @@ int gguf_mmq(const void* W, const void* x, int xdtype, void* q8_workspace, void*
  *   GGUF_MMQ_AUTO  INT8; with M <= 8 the streaming GEMV kernel instead, switched to this operator's offset sums
  *                  (Q4_K, Q5_K, Q5_0 are the formats where the reference's GEMV and its tile GEMM form them
  *                  differently), which is exact in int8 and reads W once at the GEMV's rate; and for Q4_K, Q5_K and
- *                  Q6_K at some hundred rows, where that is faster and workspace_bytes has room for the rows in
- *                  half precision (gguf_mmq_workspace_bytes has), the same exact whole-number products on
- *                  half-precision MFMA: quants and scale-times-code operands are whole numbers that half precision
+ *                  Q6_K at some hundred rows, where that is faster with the room that workspace_bytes leaves for the
+ *                  rows in half precision (gguf_mmq_workspace_bytes has it) and partial tiles, the same exact
+ *                  whole-number products on half-precision MFMA: quants and scale-times-code operands are whole numbers that half precision
  *                  holds, their sums are whole numbers that fp32 holds.  This is what gguf_mmq runs.
  * workspace_bytes is the size of q8_workspace; 0 stands for the minimum, M * gguf_q8_1_row_bytes(K).  Given
  * gguf_mmq_workspace_bytes(M, N, K) bytes, either engine splits K over several workgroups per output tile where the

@@ -71,10 +71,10 @@ def test_replays_match_eager(case):
 # GEMM and on the codebook GEMM, and through merged shards
 @pytest.mark.parametrize("qtype,m,n,k", [(o.Q4_K, 12, 2080, 4096), (o.Q4_K, 200, 640, 768), (o.IQ4_XS, 70, 640, 1280)])
 def test_layer_calls_replay_as_eager(qtype, m, n, k):
-    from vllm_gguf_plugin_prism_amd import _lib, dispatch
+    from vllm_gguf_plugin_prism_amd import _lib, dispatch, ops
     rng = np.random.default_rng(m)
     wn = o.make_weights(rng, qtype, n, k)
-    route = _lib.lib().gguf_mmq_layer_route(qtype, n, k, m, wn.shape[1])
+    route = ops._mmq_route(qtype, n, k, m, wn.shape[1])
     assert route == {12: 1, 200: 2, 70: 0}[m] and (m != 70 or _lib.lib().gguf_dense_linear_workspace_bytes(n, k, m) > 0)
     w, bias = _dev(wn), torch.randn(n, dtype=torch.float16, device="cuda")
     xs = [torch.randn(m, k, dtype=torch.float16, device="cuda") for _ in range(3)]

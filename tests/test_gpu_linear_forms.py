@@ -9,7 +9,7 @@ from oracle import gguf_oracle as o
 from vllm_gguf_plugin_prism_amd import dispatch as D
 
 pytestmark = pytest.mark.gpu
-SIZES = {1: (12, 2080, 4096), 2: (200, 640, 768)}         # route of gguf_mmq_layer_route -> rows, N, K
+SIZES = {1: (12, 2080, 4096), 2: (200, 640, 768)}         # route -> rows, N, K
 
 
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32])
@@ -17,13 +17,13 @@ SIZES = {1: (12, 2080, 4096), 2: (200, 640, 768)}         # route of gguf_mmq_la
 @pytest.mark.parametrize("qtype", [o.Q4_K, o.Q5_K, o.Q6_K])
 @pytest.mark.parametrize("route", [1, 2])
 def test_forms(route, qtype, offset, pad, column, spare, dt):
-    from vllm_gguf_plugin_prism_amd import _lib
+    from vllm_gguf_plugin_prism_amd import ops
     m, n, k = SIZES[route]
     rng = np.random.default_rng(route + qtype)
     packed = o.make_weights(rng, qtype, n, k)
     rb = packed.shape[1]
     pitch = rb + pad
-    assert _lib.lib().gguf_mmq_layer_route(qtype, n, k, m, pitch) == route
+    assert ops._mmq_route(qtype, n, k, m, pitch) == route
     raw = torch.zeros(offset + n * pitch, dtype=torch.uint8, device="cuda")
     w = raw[offset:].view(n, pitch)[:, :rb]
     w.copy_(torch.from_numpy(packed))

@@ -62,9 +62,9 @@ def test_the_int8_engine_can_be_asked_for(qtype):
 
 
 def _taken(qtype, m, n, k, pad=0):
-    from vllm_gguf_plugin_prism_amd import _lib, ops
+    from vllm_gguf_plugin_prism_amd import ops
     qk, size = ops.quant_sizes(qtype)
-    return _lib.lib().gguf_mmq_layer_route(qtype, n, k, m, k // qk * size + pad) == 2
+    return ops._mmq_route(qtype, n, k, m, k // qk * size + pad) == 2
 
 
 # sizes that the cost rule sends here for all three formats: part of a tile of rows, its tiles cut into runs; one row and one

@@ -60,10 +60,10 @@ def test_moe_layer_edges(qtype, tokens, e, hid, inner):
 @pytest.mark.parametrize("qtype,m,n,k", [(q, *s) for q in DEEP for s in ((5, 5200, 4352), (24, 5205, 4096), (8, 12300, 2304), (16, 28688, 512))] + [
     (o.Q4_0, 12, 2560, 4096), (o.Q8_0, 24, 2048, 8192)])
 def test_dense_where_it_is_taken(qtype, m, n, k):
-    from vllm_gguf_plugin_prism_amd import _lib, ops
+    from vllm_gguf_plugin_prism_amd import ops
     rng = np.random.default_rng(n + m)
     w = o.make_weights(rng, qtype, n, k)
-    assert _lib.lib().gguf_mmq_layer_route(qtype, n, k, m, w.shape[1]) == 1
+    assert ops._mmq_route(qtype, n, k, m, w.shape[1]) == 1
     x = rng.standard_normal((m, k)).astype(np.float32)
     y = ops.ggml_mul_mat_a8(torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda(), qtype, n)
     assert o.rel_l2(y.cpu().numpy(), o.mul_mat_a8(w, x, qtype, n, "mmq")) <= 1e-5

@@ -153,9 +153,20 @@ def test_codebook_gemm_refuses_sizes_beyond_its_integers():
     (D.Q4_K, 288, 2560, 1024, 0), (D.Q4_K, 384, 18944, 1024, 0), (D.Q5_K, 1536, 1024, 1024, 0), (D.Q6_K, 512, 8192, 2560, 0),      # 42 / 21, 85 / 53, 45 / 28, 94 / 70
     (D.Q4_K, 160, 11008, 14336, 1), (D.Q5_K, 192, 11008, 11008, 1), (D.Q4_K, 256, 28672, 14336, 1), (D.Q4_K, 512, 4096, 14336, 1)])  # 147 / 264, 135 / 225, 335 / 547, 107 / 148
 def test_products_run_on_the_faster_unit(qt, m, n, k, half):
-    from vllm_gguf_plugin_prism_amd import _lib, ops
+    from vllm_gguf_plugin_prism_amd import ops
     qk, size = ops.quant_sizes(qt)
-    assert _lib.lib().gguf_mmq_layer_route(qt, n, k, m, k // qk * size) == (2 if half else 0)
+    assert ops._mmq_route(qt, n, k, m, k // qk * size) == (2 if half else 0)
+
+
+# with less room the K of few tiles is not shared by the chip: sixteen workgroups with 56 super-blocks each are no faster
+# unit, and neither is the one whose rows have no room
+def test_the_unit_is_chosen_for_the_workspace_that_is_there():
+    from vllm_gguf_plugin_prism_amd import _lib, ops
+    L, n, k, m, pitch = _lib.lib(), 2048, 14336, 256, 14336 // 256 * 144
+    full = L.gguf_mmq_layer_workspace_bytes(D.Q4_K, n, k, m, pitch)
+    assert ops._mmq_route(D.Q4_K, n, k, m, pitch) == 2
+    assert ops._mmq_route(D.Q4_K, n, k, m, pitch, full // 2) == 0
+    assert ops._mmq_route(D.Q4_K, n, k, m, pitch, m * L.gguf_q8_1_row_bytes(k)) == 0
 
 
 # measured, us, streaming tile kernel / the kernel that runs otherwise: where either is the faster one by a tenth or more
@@ -165,9 +176,9 @@ def test_products_run_on_the_faster_unit(qt, m, n, k, half):
     (D.Q4_K, 5, 4096, 1024, 0), (D.Q4_K, 12, 8192, 3584, 0), (D.Q5_K, 24, 512, 14336, 0), (D.Q6_K, 12, 1024, 14336, 0),    # 7.6 / 5.7, 13 / 11, 25 / 15, 22 / 14
     (D.Q4_0, 24, 512, 14336, 0), (D.Q4_0, 12, 4096, 3072, 0)])                                                             # 26 / 18, 11 / 9
 def test_products_of_a_few_rows_run_on_the_faster_kernel(qt, m, n, k, stream):
-    from vllm_gguf_plugin_prism_amd import _lib, ops
+    from vllm_gguf_plugin_prism_amd import ops
     qk, size = ops.quant_sizes(qt)
-    assert _lib.lib().gguf_mmq_layer_route(qt, n, k, m, k // qk * size) == stream
+    assert ops._mmq_route(qt, n, k, m, k // qk * size) == stream
 
 
 def test_codebook_gemm_declines_types_it_does_not_know():

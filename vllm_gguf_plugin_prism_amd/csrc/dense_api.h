@@ -9,7 +9,7 @@
  *
  * gguf_mmq_layer_workspace_bytes: the workspace with which gguf_mmq_linear on GGUF_MMQ_AUTO runs at full speed for weights
  * of this type, at a 16-byte boundary.  (gguf_mmq_workspace_bytes_engine does not know the type.)  gguf_mmq_layer_route: the
- * kernel that such a call runs, for the tests of a kernel: 1 the streaming tile kernel, 2 the half-precision unit's, 0 another. */
+ * kernel that a call with a workspace of this size runs: 1 the streaming tile kernel, 2 the half-precision unit's, 0 another. */
 #pragma once
 #include <stdint.h>
 #ifdef __cplusplus
@@ -20,7 +20,7 @@ int64_t gguf_dense_linear_workspace_bytes(int64_t N, int64_t K, int64_t M);
 int gguf_dense_linear(const void* W, int64_t w_row_pitch_bytes, const void* x, int xdtype, void* workspace, void* Y, int64_t y_row_pitch,
                       const void* bias, int type, int64_t N, int64_t K, int64_t M, int64_t workspace_bytes, void* stream);
 int64_t gguf_mmq_layer_workspace_bytes(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes);
-int gguf_mmq_layer_route(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes);
+int gguf_mmq_layer_route(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes);
 #ifdef __cplusplus
 }
 #endif

@@ -829,14 +829,15 @@ extern "C" int64_t gguf_mmq_workspace_bytes_engine(int64_t M, int64_t N, int64_t
 
 extern "C" int64_t gguf_mmq_layer_workspace_bytes(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes) {
   if (M <= 0 || N <= 0 || K <= 0 || M > 0x7FFFFFF0LL || N > 0x7FFFFFF0LL || K > 0x7FFFFFF0LL) return 0;
-  if (gguf::mmqf_takes(type, M, N, K, w_row_pitch_bytes))
+  if (gguf::mmqf_takes(type, M, N, K, w_row_pitch_bytes, INT64_MAX, 0))
     return gguf::mmqf_rows_bytes(M, K) + gguf::mmqf_plan((int)M, (int)N, (int)K, INT64_MAX).partial_bytes();
   return gguf_mmq_workspace_bytes_engine(M, N, K, GGUF_MMQ_INT8);
 }
 
-extern "C" int gguf_mmq_layer_route(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes) {
+extern "C" int gguf_mmq_layer_route(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes) {
   if (M <= 0 || N <= 0 || K <= 0 || M > 0x7FFFFFF0LL || N > 0x7FFFFFF0LL || K > 0x7FFFFFF0LL) return 0;
-  return gguf::ts_dense_takes(type, M, N, K, w_row_pitch_bytes) ? 1 : gguf::mmqf_takes(type, M, N, K, w_row_pitch_bytes) ? 2 : 0;
+  if (gguf::ts_dense_takes(type, M, N, K, w_row_pitch_bytes)) return 1;
+  return gguf::mmqf_takes(type, M, N, K, w_row_pitch_bytes, workspace_bytes, mmq_rows_bytes(M, K, false)) ? 2 : 0;
 }
 
 // room for either engine
@@ -911,16 +912,14 @@ int gguf::mmq_linear_impl(const void* W, int64_t w_row_pitch_bytes, const void* 
     const int rc = mmvq_any(type, W, x, q8_workspace, Y, xdtype, N, K, M, s, lt);
     if (rc != GGUF_NOT_TAKEN) return rc;
   }
-  if (engine == GGUF_MMQ_AUTO && mmqf_takes(type, M, N, K, w_row_pitch_bytes) && ((uintptr_t)q8_workspace & 15) == 0) {
-    // the same whole-number products on the half-precision matrix unit, where there is room for its form of the rows
+  if (engine == GGUF_MMQ_AUTO && ((uintptr_t)q8_workspace & 15) == 0 && mmqf_takes(type, M, N, K, w_row_pitch_bytes, workspace_bytes, rows_bytes)) {
+    // the same whole-number products on the half-precision matrix unit
     const int64_t half_rows = mmqf_rows_bytes(M, K);
-    if (workspace_bytes >= half_rows) {
-      const MmqfRows rows = mmqf_rows(q8_workspace, M, K);
-      int rc = quantize_whole(x, xdtype, rows, M, K, s);
-      if (rc != GGUF_OK) return rc;
-      const MmqfCall c = {W, rows, Y, xdtype, (int)M, (int)N, (int)K, (float*)((char*)q8_workspace + half_rows), workspace_bytes - half_rows, la};
-      return mmqf(type, c, s);
-    }
+    const MmqfRows rows = mmqf_rows(q8_workspace, M, K);
+    int rc = quantize_whole(x, xdtype, rows, M, K, s);
+    if (rc != GGUF_OK) return rc;
+    const MmqfCall c = {W, rows, Y, xdtype, (int)M, (int)N, (int)K, (float*)((char*)q8_workspace + half_rows), workspace_bytes - half_rows, la};
+    return mmqf(type, c, s);
   }
   if (engine == GGUF_MMQ_AUTO) engine = GGUF_MMQ_INT8;   // the reference's arithmetic; the half engine is for callers that ask
   float* partial = (float*)((char*)q8_workspace + rows_bytes);

@@ -29,9 +29,11 @@ struct MmqfCall {
 
 TilePlan mmqf_plan(int M, int N, int K, int64_t partial_bytes_available);
 
-double mmq_int_us(int type, int M, int N, int K);   // mmq_i.hip
+double mmq_int_us(int type, int M, int N, int K, int64_t partial_bytes_available);   // mmq_i.hip
 
-bool mmqf_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch);
+// Whether a product with a workspace of this size is taken: it has room for the rows here, and is the faster one with what is
+// left for partial tiles here and behind the int8 rows (int8_rows_bytes) there.
+bool mmqf_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, int64_t workspace_bytes, int64_t int8_rows_bytes);
 int mmqf(int type, const MmqfCall& c, hipStream_t stream);
 
 }  // namespace gguf

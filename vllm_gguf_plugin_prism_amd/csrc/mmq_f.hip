@@ -6,8 +6,8 @@ namespace gguf {
 // About how long a product takes, us, quantizer included (as mmq_int_us, fitted to the same calls and right to about 8 %): a
 // super-block of a tile, the beginning and the store of a round of tiles, the partial tiles' way through memory and how
 // many of them are added one after the other, the rows of X, the result.
-static double mmqf_us(int type, int M, int N, int K) {
-  const TilePlan p = mmqf_plan(M, N, K, INT64_MAX);
+static double mmqf_us(int type, int M, int N, int K, int64_t avail) {
+  const TilePlan p = mmqf_plan(M, N, K, avail);
   const int nsb = K / 256, rounds = (p.whole + 255) / 256;
   const double sb = type == T_Q4_K ? 5.85 : type == T_Q5_K ? 6.2 : 8.0;
   double us = 6.5 + rounds * (nsb * sb + 8.6) + 1e-6 * M * (0.9 * K + 1.2 * N);
@@ -15,16 +15,18 @@ static double mmqf_us(int type, int M, int N, int K) {
   return us;
 }
 
-bool mmqf_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch) {
-  if (type != T_Q4_K && type != T_Q5_K && type != T_Q6_K) return false;
+bool mmqf_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, int64_t workspace_bytes, int64_t int8_rows_bytes) {
+  if ((type != T_Q4_K && type != T_Q5_K && type != T_Q6_K) || M < 128 || M > 0x7FFFFFF0ll) return false;
   // (offsets inside the matrix and inside the rows of X are 32-bit)
-  if (N * w_pitch > 0xFFFF0000ll || mmqf_rows_bytes(M, K) > 0xFFFF0000ll) return false;
+  const int64_t rows = mmqf_rows_bytes(M, K);
+  if (N * w_pitch > 0xFFFF0000ll || rows > 0xFFFF0000ll || workspace_bytes < rows) return false;
   if ((M / 256 + 1) * (N / 128 + 1) * (K / 256) > 0x7FFFFFFFll) return false;   // (super-blocks of all tiles are counted in an int)
   // Where it is the faster one by the two estimates.  Its tiles of 256 rows want rows, and a long K to be worth a beginning;
   // us, this / int8: [2560,1024] Q4_K 288 rows 42 / 21, [18944,1024] 384 rows 85 / 53, [8192,2560] Q6_K 512 rows 94 / 70;
   // [4096,14336] Q4_K 512 rows 107 / 148, [11008,14336] 160 rows 147 / 264, [28672,14336] 256 rows 335 / 547.  Over 5100 calls of
   // random sizes the estimates lose 0.7 % against always taking the faster engine.
-  return M >= 128 && M <= 0x7FFFFFF0ll && mmqf_us(type, (int)M, (int)N, (int)K) < 0.97 * mmq_int_us(type, (int)M, (int)N, (int)K);
+  return mmqf_us(type, (int)M, (int)N, (int)K, workspace_bytes - rows) <
+         0.97 * mmq_int_us(type, (int)M, (int)N, (int)K, workspace_bytes > int8_rows_bytes ? workspace_bytes - int8_rows_bytes : 0);
 }
 
 // (a pitch that is not a multiple of 4096 bytes: see q8_half_pitch)

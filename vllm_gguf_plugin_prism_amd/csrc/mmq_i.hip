@@ -66,9 +66,9 @@ MmqiPlan mmq_int_plan(int M, int N, int K, int64_t avail, bool wide_ok) {
 // (mmqf_takes).  us: the plan's steps at what one takes, the partial tiles' way through memory, the quantizer and the
 // result.  Fitted to 5600 calls, 13 x 10 sizes of N and K from 512 x 1024 to 28672 x 14336, 128 to 2048 rows; on 5100 others of
 // random sizes right to about 7 % (root of the mean square).
-double mmq_int_us(int type, int M, int N, int K) {
+double mmq_int_us(int type, int M, int N, int K, int64_t avail) {
   const bool wide = type != T_Q5_K;
-  const MmqiPlan p = mmq_int_plan(M, N, K, INT64_MAX, wide);
+  const MmqiPlan p = mmq_int_plan(M, N, K, avail, wide);
   const int slots = p.cfg == 2 || p.cfg == 3 ? 256 : 512;
   const double cost = plan_cost(p, slots, p.cfg == 3 ? 0.6 : p.cfg == 2 ? 1.8 : 1.0, K), step = type == T_Q4_K ? 2.06 : type == T_Q5_K ? 2.12 : 2.22;
   return 4.5 + step * cost + 1e-6 * (0.031 / 0.032768 * p.shared * (p.splits + 1) * p.mt() * p.nt() + 1.1 * M * K + 0.6 * M * N + 0.16 * N * K);

@@ -233,6 +233,15 @@ def _dense_result_fits(X: torch.Tensor, row: int, out: torch.Tensor | None, bias
     return all(t is None or t.untyped_storage().data_ptr() != held for t in (X, bias, *inputs))
 
 
+def _mmq_route(quant_type: int, row: int, col: int, vecs: int, w_pitch: int, workspace_bytes: int | None = None) -> int:
+    """The kernel that :func:`ggml_mul_mat_a8` runs on its own workspace or one of this size: 1 the streaming tile kernel,
+    2 the half-precision unit's whole-number GEMM, 0 another."""
+    L = _lib.lib()
+    if workspace_bytes is None:
+        workspace_bytes = L.gguf_mmq_layer_workspace_bytes(int(quant_type), row, col, vecs, w_pitch)
+    return L.gguf_mmq_layer_route(int(quant_type), row, col, vecs, w_pitch, workspace_bytes)
+
+
 def _product_is_watched(X: torch.Tensor, *others: torch.Tensor | None) -> bool:
     """Whether torch would do more in ``X @ dense.T`` (then ``add_`` of a bias, ``copy_`` to a result) than multiply: record
     it for a gradient, carry a tangent along, map it over a batch, show it to a dispatch mode or a tensor subclass, cast
