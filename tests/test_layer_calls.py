@@ -172,7 +172,7 @@ def test_the_unit_is_chosen_for_the_workspace_that_is_there():
 # measured, us, streaming tile kernel / the kernel that runs otherwise: where either is the faster one by a tenth or more
 @pytest.mark.parametrize("qt,m,n,k,stream", [
     (D.Q4_K, 24, 11008, 4096, 1), (D.Q5_K, 32, 5120, 4096, 1), (D.Q6_K, 8, 2560, 4096, 1), (D.Q4_0, 12, 2560, 4096, 1),    # 20 / 39, 15 / 28, 11 / 17, 11 / 16
-    (D.Q8_0, 24, 2048, 5120, 1), (D.Q4_K, 5, 28672, 1024, 1),                                                              # 14 / 18, 10 / 20
+    (D.Q8_0, 24, 2048, 5120, 1), (D.Q4_K, 5, 28672, 1024, 1), (D.Q4_0, 17, 2304, 11264, 1),                                # 14 / 18, 10 / 20, 23 / 26
     (D.Q4_K, 5, 4096, 1024, 0), (D.Q4_K, 12, 8192, 3584, 0), (D.Q5_K, 24, 512, 14336, 0), (D.Q6_K, 12, 1024, 14336, 0),    # 7.6 / 5.7, 13 / 11, 25 / 15, 22 / 14
     (D.Q4_0, 24, 512, 14336, 0), (D.Q4_0, 12, 4096, 3072, 0)])                                                             # 26 / 18, 11 / 9
 def test_products_of_a_few_rows_run_on_the_faster_kernel(qt, m, n, k, stream):

@@ -54,8 +54,9 @@ bool ts_dense_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch) 
   if (type >= T_Q4_K && type <= T_Q6_K) return ts_us(type, (int)M, (int)N, (int)K) < ts_others_us(type, (int)M, (int)N, (int)K);
   // Q4_0, Q8_0, from the same sweeps (us, this / the other kernel: the GEMV up to 8 rows, the 16-row kernels above).
   // Few columns and a long K leave most CUs without a workgroup, as K is shared by the waves of one and not by several
-  // ([512,14336] Q4_0 24 rows 26.1 / 17.7, [1024,14336] 12 rows 18.5 / 17.9; [2048,8192] 24 rows 18.1 / 19.2, Q8_0 16.9 / 22.1).
-  if (M <= 16 ? N <= 2048 && K > 8192 : K > 4096 && K > (type == T_Q8_0 ? 8 : 4) * N) return false;
+  // ([512,14336] Q4_0 24 rows 26.1 / 17.7, [1024,14336] 12 rows 18.5 / 17.9; [2048,8192] 24 rows 18.1 / 19.2, Q8_0 16.9 / 22.1;
+  // [2304,11264] Q4_0 17 rows 23.0 / 25.8).
+  if (N <= 2048 && (M <= 16 ? K > 8192 : K > 4096 && K > (type == T_Q8_0 ? 8 : 4) * N)) return false;
   // The GEMV's waves hold all rows' sums: from seven rows on it falls behind where K is long ([4096,8192] Q4_0, 8 rows:
   // 15.2 / 18.5; [4096,4096] 10.9 / 10.7; Q8_0 16.4 / 17.7, 11.6 / 10.8).
   // (rows that do not begin on 16 bytes are cut out of two reads each: [19504,6016] Q8_0, 8 rows: 38.6 / 33.6,
