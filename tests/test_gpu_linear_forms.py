@@ -9,7 +9,7 @@ from oracle import gguf_oracle as o
 from vllm_gguf_plugin_prism_amd import dispatch as D
 
 pytestmark = pytest.mark.gpu
-SIZES = {1: (12, 2080, 4096), 2: (200, 640, 768)}         # route -> rows, N, K
+SIZES = {1: (12, 2080, 4096), 2: (200, 512, 768)}         # route -> rows, N, K
 
 
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32])

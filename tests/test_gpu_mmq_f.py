@@ -70,7 +70,7 @@ def _taken(qtype, m, n, k, pad=0):
 # sizes that the cost rule sends here for all three formats: part of a tile of rows, its tiles cut into runs; one row and one
 # column over a tile; runs that begin and end inside tiles; a whole round and a shared rest, narrower than the rows
 @pytest.mark.parametrize("qtype", [o.Q4_K, o.Q5_K, o.Q6_K])
-@pytest.mark.parametrize("m,n,k,pad", [(200, 640, 768, 0), (257, 257, 768, 2), (460, 2176, 3584, 0), (255, 33000, 1280, 6)])
+@pytest.mark.parametrize("m,n,k,pad", [(200, 512, 768, 0), (257, 129, 768, 2), (460, 2176, 3584, 0), (255, 33000, 1280, 6)])
 def test_tile_edges_where_it_is_taken(qtype, m, n, k, pad):
     assert _taken(qtype, m, n, k, pad)
     rng = np.random.default_rng(m + k)
@@ -81,7 +81,7 @@ def test_tile_edges_where_it_is_taken(qtype, m, n, k, pad):
 @pytest.mark.parametrize("qtype", [o.Q4_K, o.Q5_K, o.Q6_K])
 def test_largest_sums_are_exact_where_it_is_taken(qtype):
     rng = np.random.default_rng(qtype)
-    n, k, m = 640, 768, 200
+    n, k, m = 512, 768, 200
     assert _taken(qtype, m, n, k)
     w = o.make_weights(rng, qtype, n, k).reshape(n, k // 256, -1)
     if qtype == o.Q6_K:

@@ -25,8 +25,10 @@ bool mmqf_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, int6
   // us, this / int8: [2560,1024] Q4_K 288 rows 42 / 21, [18944,1024] 384 rows 85 / 53, [8192,2560] Q6_K 512 rows 94 / 70;
   // [4096,14336] Q4_K 512 rows 107 / 148, [11008,14336] 160 rows 147 / 264, [28672,14336] 256 rows 335 / 547.  Over 5100 calls of
   // random sizes the estimates lose 0.7 % against always taking the faster engine.
-  return mmqf_us(type, (int)M, (int)N, (int)K, workspace_bytes - rows) <
-         0.97 * mmq_int_us(type, (int)M, (int)N, (int)K, workspace_bytes > int8_rows_bytes ? workspace_bytes - int8_rows_bytes : 0);
+  // (A start of 1.5 us for the int8 engine: where the two are close, on products of 20 to 30 us, this one is the likelier to be
+  // slower than its estimate.)
+  return mmqf_us(type, (int)M, (int)N, (int)K, workspace_bytes - rows) + 1.5 <
+         mmq_int_us(type, (int)M, (int)N, (int)K, workspace_bytes > int8_rows_bytes ? workspace_bytes - int8_rows_bytes : 0);
 }
 
 // (a pitch that is not a multiple of 4096 bytes: see q8_half_pitch)

@@ -71,7 +71,8 @@ double mmq_int_us(int type, int M, int N, int K, int64_t avail) {
   const MmqiPlan p = mmq_int_plan(M, N, K, avail, wide);
   const int slots = p.cfg == 2 || p.cfg == 3 ? 256 : 512;
   const double cost = plan_cost(p, slots, p.cfg == 3 ? 0.6 : p.cfg == 2 ? 1.8 : 1.0, K), step = type == T_Q4_K ? 2.06 : type == T_Q5_K ? 2.12 : 2.22;
-  return 4.5 + step * cost + 1e-6 * (0.031 / 0.032768 * p.shared * (p.splits + 1) * p.mt() * p.nt() + 1.1 * M * K + 0.6 * M * N + 0.16 * N * K);
+  const double us = 4.5 + step * cost + 1e-6 * (0.031 / 0.032768 * p.shared * (p.splits + 1) * p.mt() * p.nt() + 1.1 * M * K + 0.6 * M * N + 0.16 * N * K);
+  return us * (1.0 + 0.05 * us / (us + 400.0));   // (the clock falls under a long product)
 }
 
 // (the workspace is sized without knowing the format: room for whichever shape a format may take)
