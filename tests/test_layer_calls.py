@@ -1,6 +1,5 @@
 """The compiled layer calls (csrc/torch_binding/gguf_calls.cpp): the path they pick is dispatch.py's, what they do not
-serve falls back to Python, and their results are those of the Python path bit for bit, merged shards' to the order of a
-32-bit sum."""
+serve falls back to Python, and their results are those of the Python path bit for bit."""
 import numpy as np
 import pytest
 import torch
@@ -104,26 +103,38 @@ def _merged(rng, parts, k):
     return w, at, {i: qt for i, (qt, _) in zip("qkv", parts)}
 
 
-# q and k are one matrix to the compiled call and two to Python: every path, at sizes where the two split K differently
+# q and k are one matrix: every path, at sizes where that splits K differently than each shard by itself
 @pytest.mark.gpu
 @pytest.mark.parametrize("qt,dt,m,rows,k", [
     (D.Q4_K, torch.float32, 1, (2048, 512), 4096), (D.Q8_0, torch.float32, 6, (4096, 1024), 2048), (D.Q4_K, torch.float32, 12, (4096, 1024), 4096),
     (D.Q4_0, torch.float32, 40, (1024, 256), 4096), (D.Q6_K, torch.float32, 100, (3072, 1024), 2048), (D.Q4_K, torch.float32, 460, (4096, 1024), 2048),
     (D.IQ4_XS, torch.bfloat16, 40, (1024, 512), 4096), (D.IQ4_XS, torch.float16, 300, (2560, 640), 2560)])
-def test_merged_shards_differ_by_the_order_of_a_sum(qt, dt, m, rows, k, monkeypatch):
+def test_merged_shards(qt, dt, m, rows, k, monkeypatch):
     rng = np.random.default_rng(m)
     w, at, types = _merged(rng, [(qt, rows[0]), (qt, rows[1]), (D.Q5_K, 256)], k)
     x = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).to(dt).cuda()
     ids = ("q", "k", "v")
     assert D._calls().merged_linear(x, w, list(ids), at, [types[i] for i in ids], None) is not None, "not served"
+    bias = torch.from_numpy(rng.standard_normal(w.shape[0]).astype(np.float32)).to(dt).cuda()
+    _both(monkeypatch, lambda: D.apply_linear(x, w, qt, shard_ids=ids, shard_offset_map=at, shard_weight_types=types, bias=bias))
     got = D.apply_linear(x, w, qt, shard_ids=ids, shard_offset_map=at, shard_weight_types=types)
-    with monkeypatch.context() as p:
-        p.setattr(D, "_CALLS", D._NoCalls)
-        want = D.apply_linear(x, w, qt, shard_ids=ids, shard_offset_map=at, shard_weight_types=types)
-    # 32-bit sums of K products in another order; in 16 bits the two may round to neighbours
+    want = torch.cat([D.fused_mul_mat_gguf(x, w[a:b, :r].contiguous(), types[i]) for i, (a, b, r) in at.items()], 1)
+    # against shard by shard: 32-bit sums of K products in another order; in 16 bits the two may round to neighbours
     rel = {torch.float32: 1e-6, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dt]
     assert ((got.double() - want.double()).norm() / want.double().norm()).item() <= rel
     assert torch.equal(got[:, sum(rows):], want[:, sum(rows):])
+
+
+# past 32 rows a run keeps to the unit of its largest shard: K = 1024 with 300 rows is for the half-precision unit at 512
+# columns and for the int8 unit at 640
+def test_runs_of_shards_keep_to_the_unit_of_the_largest():
+    types = {"q": D.Q4_K, "k": D.Q4_K, "v": D.Q6_K}
+    for m, k, rows, merged in ((300, 1024, (512, 128), False), (300, 1024, (512, 512), False), (40, 1024, (512, 128), True), (512, 4096, (4096, 1024), True),
+                               (12, 1024, (512, 128), True), (1, 1024, (512, 128), True)):
+        rb = k // 256 * 210
+        w, x = torch.zeros(sum(rows) + 130, rb, dtype=torch.uint8), torch.zeros(m, k)
+        shards = [(0, rows[0], k // 256 * 144, D.Q4_K), (rows[0], sum(rows), k // 256 * 144, D.Q4_K), (sum(rows), sum(rows) + 130, rb, D.Q6_K)]
+        assert [len(run) for _, run in D._shard_runs(x, w, shards)] == ([2, 1] if merged else [1, 1, 1]), (m, k, rows)
 
 
 # the codebook GEMM serves both shards but not the matrix that they are together: it is asked about what would run

@@ -6,8 +6,7 @@
 // Every function returns None for a call it does not serve (another device than the current one, tensors that are not
 // plain dense ones, a malformed shape, an unquantized type, ...) before anything is allocated or launched; dispatch.py
 // then takes its Python path, which raises what there is to raise.  Both make the same calls of the C ABI with the same
-// arguments, and so have the same results bit for bit, but for merged shards (merged_linear), whose sums may be split in
-// another order.
+// arguments, and so have the same results bit for bit.
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -219,9 +218,10 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // whose types differ, in the order of shard_ids; shard_offset_map[id] = (first row, row behind the last, bytes of a row)
 // and types lists their ggml types.  Neighbouring shards of one type whose rows lie next to each other and which take
 // the same path are one matrix with more rows and so one call: q and k of a mixed recipe, [4096 + 1024, 4096] Q4_K,
-// 9.1 -> 5.6 us of kernel time.  The path is that of the shards, each by its own rows, as in the reference's policy; within
-// it, how many workgroups share a sum over K depends on the rows of the whole matrix, so a result may differ from the
-// single shard's by the order of a 32-bit sum.
+// 9.1 -> 5.6 us of kernel time.  The path is that of the shards, each by its own rows, as in the reference's policy, and past
+// 32 rows of X, where launches no longer count, a run keeps to the matrix unit that its largest shard takes by itself;
+// within that, how many workgroups share a sum over K depends on the rows of the whole matrix, so a result may differ from
+// the single shard's by the order of a 32-bit sum.  (dispatch.py, _shard_runs, does the same.)
 PyObject* merged_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 6) return PyErr_Format(PyExc_TypeError, "merged_linear takes 6 arguments"), nullptr;
   const int dev = current_gpu();
@@ -231,7 +231,12 @@ PyObject* merged_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (count == 0 || PyList_GET_SIZE(a[4]) != count) Py_RETURN_NONE;
   const int64_t m = x->size(0), k = x->size(1);
   const size_t esz = x->element_size();
-  struct Part { int64_t start, end, type, rb; Path path; };
+  struct Part { int64_t start, end, type, rb, largest; Path path; };
+  const auto half_unit = [&](const Part& p, int64_t rows) {
+    if (m <= 32) return false;
+    const int64_t pitch = w->size(0) > 1 ? w->stride(0) : p.rb;
+    return gguf_mmq_layer_route((int)p.type, rows, k, m, pitch, gguf_mmq_layer_workspace_bytes((int)p.type, rows, k, m, pitch)) == 2;
+  };
   std::vector<Part> parts;
   int64_t width = 0;
   for (Py_ssize_t i = 0; i < count; ++i) {
@@ -247,10 +252,18 @@ PyObject* merged_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
         (p.path == PATH_DENSE && p.rb != rb))
       Py_RETURN_NONE;
     width += rows;
-    if (!parts.empty() && parts.back().end == p.start && parts.back().type == p.type && parts.back().path == p.path)
-      parts.back().end = p.end;
-    else
-      parts.push_back(p);
+    p.largest = rows;
+    if (!parts.empty()) {
+      Part& last = parts.back();
+      const int64_t largest = std::max(last.largest, rows);
+      if (last.end == p.start && last.type == p.type && last.rb == p.rb && last.path == p.path &&
+          (p.path != PATH_MMQ || half_unit(p, largest) == half_unit(p, p.end - last.start))) {
+        last.end = p.end;
+        last.largest = largest;
+        continue;
+      }
+    }
+    parts.push_back(p);
   }
   for (const Part& p : parts)
     if (!path_ok(p.path, (int)p.type, *x, *w, p.end - p.start)) Py_RETURN_NONE;

@@ -151,9 +151,10 @@ def apply_linear(x, weight, weight_type: int, *, shard_ids=(), shard_offset_map=
     ``weight`` is the layer's packed tensor.  For a merged layer (q/k/v, gate/up) ``shard_ids`` lists the shards in
     output order, ``shard_offset_map[id] = (start_row, end_row, row_bytes)`` locates each one in the padded tensor and
     ``shard_weight_types[id]`` gives its ggml type (default ``weight_type``).  Shards of one type are multiplied in one
-    call, as in the reference.  Shards of different types are multiplied one by one, but where the reference copies
-    every shard out of the padded tensor on every call and concatenates the results, each call here reads its rows in
-    place and writes its columns of the merged result, bias included."""
+    call, as in the reference.  Where types differ, the reference copies every shard out of the padded tensor on every
+    call, multiplies it and concatenates the results; here every call reads its rows in place and writes its columns of
+    the merged result, bias included, and neighbouring shards of one type are one matrix and one call (:func:`_shard_runs`),
+    whose 32-bit sums may be added in another order than shard by shard."""
     shard_ids = list(shard_ids)
     if not shard_ids:
         return fused_mul_mat_gguf(x, weight, weight_type, bias=bias)
@@ -166,15 +167,54 @@ def apply_linear(x, weight, weight_type: int, *, shard_ids=(), shard_offset_map=
         return y
     import torch
 
-    widths = [shard_offset_map[i][1] - shard_offset_map[i][0] for i in shard_ids]
-    out = torch.empty(x.shape[0], sum(widths), dtype=x.dtype, device=x.device)
+    from . import ops
+
+    shards = [(*shard_offset_map[i], t) for i, t in zip(shard_ids, types)]
+    out = torch.empty(x.shape[0], sum(end - start for start, end, _, _ in shards), dtype=x.dtype, device=x.device)
     col = 0
-    for i, t, w in zip(shard_ids, types, widths):
-        start, end, row_bytes = shard_offset_map[i]
-        fused_mul_mat_gguf(x, weight[start:end, :row_bytes], t, out=out[:, col:col + w],
-                           bias=None if bias is None else bias[col:col + w])
-        col += w
+
+    def columns(t, n):
+        return None if t is None else t[..., col:col + n]
+
+    for path, run in _shard_runs(x, weight, shards):
+        start, end, row_bytes, t = run[0][0], run[-1][1], *run[0][2:]
+        rows, w = end - start, weight[start:end, :row_bytes]
+        if path == "mmvq" and len(run) > 1:
+            ops.ggml_mul_mat_vec_a8(w, x, t, rows, out=columns(out, rows), bias=columns(bias, rows))
+        elif path == "mmq" and len(run) > 1:
+            ops.ggml_mul_mat_a8(w, x, t, rows, out=columns(out, rows), bias=columns(bias, rows))
+        elif len(run) == 1 or ops.dense_linear(w, x, t, rows, out=columns(out, rows), bias=columns(bias, rows)) is None:
+            for start, end, row_bytes, t in run:
+                fused_mul_mat_gguf(x, weight[start:end, :row_bytes], t, out=columns(out, end - start), bias=columns(bias, end - start))
+                col += end - start
+            continue
+        col += rows
     return out
+
+
+def _shard_runs(x, weight, shards):
+    """Which shards ``(first row, row behind the last, bytes of a row, type)`` of a merged layer are one matrix: neighbours
+    of one type and path whose rows touch, as ``(path, shards)``.  The path is that of every shard by its own rows, and
+    past the few rows of X that are bound by launches and weights (32) the run keeps to the matrix unit that its largest
+    shard takes by itself.  gguf_calls.cpp does the same."""
+    from . import ops
+
+    def unit(t, rows):
+        return int(x.shape[0]) > 32 and x.dim() == 2 and ops._mmq_route(t, rows, x.shape[1], x.shape[0], weight.stride(0)) == 2
+
+    runs = []
+    for shard in shards:
+        start, end, row_bytes, t = shard
+        path = select_mul_mat_path(int(t), x.shape[0], end - start)
+        if runs and path in ("mmvq", "mmq", "dequant") and runs[-1][0] == path:
+            last = runs[-1][1]
+            if last[-1][1:] == (start, row_bytes, t):
+                largest = max(b - a for a, b, _, _ in (*last, shard))
+                if path != "mmq" or unit(t, largest) == unit(t, end - last[0][0]):
+                    last.append(shard)
+                    continue
+        runs.append((path, [shard]))
+    return runs
 
 
 def _activation(name: str, inp):
