@@ -9,7 +9,9 @@
  *
  * gguf_mmq_layer_workspace_bytes: the workspace with which gguf_mmq_linear on GGUF_MMQ_AUTO runs at full speed for weights
  * of this type, at a 16-byte boundary.  (gguf_mmq_workspace_bytes_engine does not know the type.)  gguf_mmq_layer_route: the
- * kernel that a call with a workspace of this size runs: 1 the streaming tile kernel, 2 the half-precision unit's, 0 another. */
+ * kernel that a call with a workspace of this size runs where it is not on the wide tiles: 1 the streaming tile kernel, 2 the
+ * half-precision unit's, 0 another.  gguf_mmq_layer_unit: the same, 3 where it is.  gguf_moe_mmq_layer_wide: whether
+ * gguf_moe_mmq_layer with the workspace it asks for, at addresses divisible by 16, runs on them. */
 #pragma once
 #include <stdint.h>
 #ifdef __cplusplus
@@ -20,6 +22,8 @@ int64_t gguf_dense_linear_workspace_bytes(int64_t N, int64_t K, int64_t M);
 int gguf_dense_linear(const void* W, int64_t w_row_pitch_bytes, const void* x, int xdtype, void* workspace, void* Y, int64_t y_row_pitch,
                       const void* bias, int type, int64_t N, int64_t K, int64_t M, int64_t workspace_bytes, void* stream);
 int64_t gguf_mmq_layer_workspace_bytes(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes);
+int gguf_moe_mmq_layer_wide(int type13, int type2, int64_t H, int64_t I, int64_t N_out, int64_t top_k, int64_t tokens, int64_t num_experts);
+int gguf_mmq_layer_unit(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes);
 int gguf_mmq_layer_route(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes);
 #ifdef __cplusplus
 }

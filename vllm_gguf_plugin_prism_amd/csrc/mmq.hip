@@ -28,6 +28,7 @@
 #include "dense_api.h"
 #include "mmq_f.h"
 #include "tile_stream.h"
+#include "tile_wide.h"
 #include "mmq_formats.h"
 #include "q8_1_device.h"
 
@@ -689,10 +690,12 @@ int64_t moe_tiles_layer_workspace(int64_t tokens, int64_t top_k, int64_t H, int6
 }
 
 int moe_prepare(const void* X, int xdtype, void* q8x, int tokens, int K, const int32_t* topk_ids, int numel, int num_experts, int block,
-                int32_t* sorted_ids, int sorted_capacity, int32_t* expert_ids, int expert_capacity, int32_t* num_post_padded, bool permuted,
+                int32_t* sorted_ids, int sorted_capacity, int32_t* expert_ids, int expert_capacity, int32_t* num_post_padded, int layout,
                 hipStream_t s);   // moe_aux.hip
 int moe_weighted_sum_live(const void* Y, const float* topk_weights, const int32_t* topk_ids, int num_experts, void* out, int dtype,
                           int64_t tokens, int64_t top_k, int64_t N, hipStream_t s, const int32_t* slot_of_pair = nullptr);   // moe_aux.hip
+int moe_weighted_sum_parts(const void* Y, int parts, const float* topk_weights, const int32_t* topk_ids, int num_experts, void* out, int dtype, int64_t tokens,
+                           int64_t top_k, int64_t N, hipStream_t s);   // moe_aux.hip
 int moe_prepare_sorted(const void* X, int xdtype, void* q8x_sorted, int K, const int32_t* topk_ids, int numel, int top_k, int num_experts,
                        int block, int32_t* sorted_ids, int sorted_capacity, int32_t* expert_ids, int expert_capacity,
                        int32_t* num_post_padded, int32_t* slot_of_pair, hipStream_t s);   // moe_aux.hip
@@ -744,6 +747,65 @@ int moe_tiles_layer(const void* X, int xdtype, void* workspace, const void* W13,
   // the grouped operator leaves the rows of pairs whose expert id names no expert at zero (the sort drops them): the
   // sum takes them as zero instead of reading rows of y2 that nobody wrote
   return moe_weighted_sum_live(y2, topk_w, vec_sums ? nullptr : topk_ids, num_experts, out, xdtype, tokens, top_k, N_out, s);
+}
+
+// ---- A MoE layer whose experts see more than a few pairs each, on the wide tile kernel (blocks of 32 or 64 slots): the same four
+// launches with the grouped operator's arithmetic, the rows of X and h as records.
+// [records of X][records of h][second GEMM's result, pairs x N_out][sorted ids, expert ids, padded total]
+// into how many parts the second GEMM cuts K: fp32 sums that the weighted sum adds
+static int wide_layer_parts(int64_t tokens, int64_t top_k, int64_t I, int64_t N_out, int64_t num_experts, int rt) {
+  if (N_out % 8 != 0 || tokens > 65535) return 1;
+  const int64_t pairs = tokens * top_k, cap = pairs + num_experts * (32 * rt - 1);
+  return wide_ksplit(moe_blocks_estimate((int)cap, (int)pairs, 32 * rt) * ((N_out + 127) / 128), (int)I);
+}
+
+int64_t wide_layer_workspace(int64_t tokens, int64_t top_k, int64_t H, int64_t I, int64_t N_out, int64_t num_experts, int elt, int rt) {
+  const int64_t pairs = tokens * top_k, cap = pairs + num_experts * (32 * rt - 1);
+  const int parts = wide_layer_parts(tokens, top_k, I, N_out, num_experts, rt);
+  return up16(wide_rows_bytes(tokens, H)) + up16(wide_rows_bytes(pairs, I)) + up16(pairs * N_out * (parts > 1 ? 4 * parts : elt)) + (cap + cap / (32 * rt) + 2) * 4;
+}
+
+int wide_layer(const void* X, int xdtype, void* workspace, const void* W13, int type13, const void* W2, int type2, const int32_t* topk_ids,
+               const float* topk_w, void* out, int H, int I, int N_out, int top_k, int tokens, int act, int num_experts, int rt, hipStream_t s) {
+  const int pairs = tokens * top_k, elt = xdtype == GGUF_DTYPE_F32 ? 4 : 2, block = 32 * rt;
+  const int64_t cap = (int64_t)pairs + (int64_t)num_experts * (block - 1), block_cap = cap / block + 1;
+  char* const x = (char*)workspace;
+  char* const h = x + up16(wide_rows_bytes(tokens, H));
+  char* const y2 = h + up16(wide_rows_bytes(pairs, I));
+  const int parts = (uintptr_t)out % 16 == 0 ? wide_layer_parts(tokens, top_k, I, N_out, num_experts, rt) : 1;
+  int32_t* const sorted = (int32_t*)(y2 + up16((int64_t)pairs * N_out * (parts > 1 ? 4 * parts : elt)));
+  int32_t* const experts = sorted + cap;
+  int32_t* const post = experts + block_cap;
+  int rc = moe_prepare(X, xdtype, x, tokens, H, topk_ids, pairs, num_experts, block, sorted, (int)cap, experts, (int)block_cap, post, 2, s);
+  if (rc != GGUF_OK) return rc;
+  WideCall c = {};
+  c.dtype = xdtype;
+  c.rt = rt;
+  c.ksplit = 1;
+  c.row_blocks = (int)(cap / block);
+  c.W = W13;
+  c.x = x;
+  c.x_rows = tokens;
+  c.N = 2 * I;
+  c.K = H;
+  c.moe = MoeArgs{sorted, experts, post, (int64_t)2 * I * (H / block_elems(type13)) * block_bytes(type13), top_k, pairs, 0};
+  c.gate = Gate16{h, 0, I, 0, act};
+  rc = wide_any(type13, c, s);
+  if (rc != GGUF_OK) return rc;
+  c.W = W2;
+  c.x = h;
+  c.x_rows = pairs;
+  c.Y = y2;
+  c.N = N_out;
+  c.K = I;
+  c.moe = MoeArgs{sorted, experts, post, (int64_t)N_out * (I / block_elems(type2)) * block_bytes(type2), 1, pairs, 0};
+  c.gate = Gate16{};
+  c.ksplit = parts;
+  c.partial = (float*)y2;
+  rc = wide_any(type2, c, s);
+  if (rc != GGUF_OK) return rc;
+  if (parts > 1) return moe_weighted_sum_parts(y2, parts, topk_w, topk_ids, num_experts, out, xdtype, tokens, top_k, N_out, s);
+  return moe_weighted_sum_live(y2, topk_w, topk_ids, num_experts, out, xdtype, tokens, top_k, N_out, s);
 }
 
 // ---- A MoE layer whose experts see many pairs each, on the pipelined integer engine: the routing is sorted into blocks of
@@ -829,15 +891,21 @@ extern "C" int64_t gguf_mmq_workspace_bytes_engine(int64_t M, int64_t N, int64_t
 
 extern "C" int64_t gguf_mmq_layer_workspace_bytes(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes) {
   if (M <= 0 || N <= 0 || K <= 0 || M > 0x7FFFFFF0LL || N > 0x7FFFFFF0LL || K > 0x7FFFFFF0LL) return 0;
-  if (gguf::mmqf_takes(type, M, N, K, w_row_pitch_bytes, INT64_MAX, 0))
-    return gguf::mmqf_rows_bytes(M, K) + gguf::mmqf_plan((int)M, (int)N, (int)K, INT64_MAX).partial_bytes();
-  return gguf_mmq_workspace_bytes_engine(M, N, K, GGUF_MMQ_INT8);
+  const int64_t others = gguf::mmqf_takes(type, M, N, K, w_row_pitch_bytes, INT64_MAX, 0)
+                             ? gguf::mmqf_rows_bytes(M, K) + gguf::mmqf_plan((int)M, (int)N, (int)K, INT64_MAX).partial_bytes()
+                             : gguf_mmq_workspace_bytes_engine(M, N, K, GGUF_MMQ_INT8);
+  return gguf::wide_dense_room(type, M, N, K, w_row_pitch_bytes, others);
 }
 
 extern "C" int gguf_mmq_layer_route(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes) {
   if (M <= 0 || N <= 0 || K <= 0 || M > 0x7FFFFFF0LL || N > 0x7FFFFFF0LL || K > 0x7FFFFFF0LL) return 0;
   if (gguf::ts_dense_takes(type, M, N, K, w_row_pitch_bytes)) return 1;
   return gguf::mmqf_takes(type, M, N, K, w_row_pitch_bytes, workspace_bytes, mmq_rows_bytes(M, K, false)) ? 2 : 0;
+}
+
+extern "C" int gguf_mmq_layer_unit(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes) {
+  const int route = gguf_mmq_layer_route(type, N, K, M, w_row_pitch_bytes, workspace_bytes);
+  return route != 1 && M > 0 && N > 0 && K > 0 && gguf::wide_dense_plan(type, M, N, K, w_row_pitch_bytes, workspace_bytes).rt ? 3 : route;
 }
 
 // room for either engine
@@ -911,6 +979,10 @@ int gguf::mmq_linear_impl(const void* W, int64_t w_row_pitch_bytes, const void* 
     lt.tile_sums = true;
     const int rc = mmvq_any(type, W, x, q8_workspace, Y, xdtype, N, K, M, s, lt);
     if (rc != GGUF_NOT_TAKEN) return rc;
+  }
+  if (engine == GGUF_MMQ_AUTO && ((uintptr_t)q8_workspace & 15) == 0) {
+    const WidePlan p = wide_dense_plan(type, M, N, K, w_row_pitch_bytes, workspace_bytes);
+    if (p.rt) return wide_dense(type, W, x, xdtype, q8_workspace, Y, (int)M, (int)N, (int)K, p, la, s);
   }
   if (engine == GGUF_MMQ_AUTO && ((uintptr_t)q8_workspace & 15) == 0 && mmqf_takes(type, M, N, K, w_row_pitch_bytes, workspace_bytes, rows_bytes)) {
     // the same whole-number products on the half-precision matrix unit

@@ -29,6 +29,7 @@ struct MmqfCall {
 
 TilePlan mmqf_plan(int M, int N, int K, int64_t partial_bytes_available);
 
+double mmqf_us(int type, int M, int N, int K, int64_t partial_bytes_available);
 double mmq_int_us(int type, int M, int N, int K, int64_t partial_bytes_available);   // mmq_i.hip
 
 // Whether a product with a workspace of this size is taken: it has room for the rows here, and is the faster one with what is

@@ -6,7 +6,7 @@ namespace gguf {
 // About how long a product takes, us, quantizer included (as mmq_int_us, fitted to the same calls and right to about 8 %): a
 // super-block of a tile, the beginning and the store of a round of tiles, the partial tiles' way through memory and how
 // many of them are added one after the other, the rows of X, the result.
-static double mmqf_us(int type, int M, int N, int K, int64_t avail) {
+double mmqf_us(int type, int M, int N, int K, int64_t avail) {
   const TilePlan p = mmqf_plan(M, N, K, avail);
   const int nsb = K / 256, rounds = (p.whole + 255) / 256;
   const double sb = type == T_Q4_K ? 5.85 : type == T_Q5_K ? 6.2 : 8.0;

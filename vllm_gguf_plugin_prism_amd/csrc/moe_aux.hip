@@ -154,17 +154,18 @@ __global__ __launch_bounds__(ALIGN_THREADS) void moe_prepare_kernel(const T* __r
                                                                     int numel, int num_experts, int block,
                                                                     int32_t* __restrict__ sorted_ids, int sorted_capacity,
                                                                     int32_t* __restrict__ expert_ids, int expert_capacity,
-                                                                    int32_t* __restrict__ num_post_padded, bool permuted) {
+                                                                    int32_t* __restrict__ num_post_padded, int layout) {
   extern __shared__ int lds[];
   if (blockIdx.x == 0) {
     moe_align_body(topk_ids, numel, num_experts, block, sorted_ids, sorted_capacity, expert_ids, expert_capacity, num_post_padded, lds);
     return;
   }
-  const int per_row = Kp / 8;                                   // threads a row takes
+  const int per_row = (layout == 2 ? K : Kp) / 8;               // threads a row takes
   const int64_t g = (int64_t)(blockIdx.x - 1) * ALIGN_THREADS + threadIdx.x;
   const int64_t m = g / per_row;
-  if (m >= tokens) return;                                      // (per_row is a multiple of 64: whole waves leave)
-  q8_1_quantize_thread<T>(x, ws, K, Kp, row_bytes, ACT_NONE, m, (int)(g % per_row), nullptr, permuted);
+  if (m >= tokens) return;                                      // (per_row is a multiple of 32: whole quads leave)
+  if (layout == 2) wide_quantize_thread<T>(x, ws, K, tokens, m, (int)(g % per_row));
+  else q8_1_quantize_thread<T>(x, ws, K, Kp, row_bytes, ACT_NONE, m, (int)(g % per_row), nullptr, layout == 1);
 }
 
 // out[t, n] = sum_k  T( float(Y[t, k, n]) * w[t, k] )   accumulated in fp32 in the order k = 0 .. top_k-1 and rounded
@@ -189,8 +190,74 @@ __global__ __launch_bounds__(256) void moe_weighted_sum_kernel(const T* __restri
   }
 }
 
+// The same from rows that are sums of fp32 parts, [parts][tokens * top_k][N] (rounded to T after they are added, as the GEMM would
+// have stored them); PARTS 0: from rows of T.  Four or eight values a thread; what the call costs at some hundred tokens is
+// the way to the rows and back, so all of a token's rows are asked for at once.
+template <typename T, int PARTS, int V>
+__global__ __launch_bounds__(256) void moe_weighted_sum_wide_kernel(const void* __restrict__ Y, int parts, int64_t stride, const float* __restrict__ w, T* __restrict__ out,
+                                                                    int top_k, int64_t N, const int32_t* __restrict__ ids, int num_experts) {
+  const int64_t t = blockIdx.y;
+  const int64_t n = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V;
+  if (n >= N) return;
+  struct alignas(sizeof(T) * V) Row { T v[V]; };
+  float acc[V];
+#pragma unroll
+  for (int e = 0; e < V; ++e) acc[e] = 0.0f;
+#pragma unroll 4
+  for (int k = 0; k < top_k; ++k) {
+    const int64_t row = t * top_k + k;
+    const bool live = !ids || (unsigned)ids[row] < (unsigned)num_experts;
+    const float wk = w[row];
+    float v[V];
+    if constexpr (PARTS) {
+      const float* p = (const float*)Y + row * N + n;
+#pragma unroll
+      for (int e = 0; e < V; ++e) v[e] = p[e];
+      for (int z = 1; z < parts; ++z)
+#pragma unroll
+        for (int e = 0; e < V; ++e) v[e] += p[z * stride + e];
+#pragma unroll
+      for (int e = 0; e < V; ++e) v[e] = to_f32<T>(from_f32<T>(v[e]));
+    } else {
+      const Row r = *(const Row*)((const T*)Y + row * N + n);
+#pragma unroll
+      for (int e = 0; e < V; ++e) v[e] = to_f32<T>(r.v[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < V; ++e) acc[e] += to_f32<T>(from_f32<T>((live ? v[e] : 0.0f) * wk));
+  }
+  Row o;
+#pragma unroll
+  for (int e = 0; e < V; ++e) o.v[e] = from_f32<T>(acc[e]);
+  *(Row*)(out + t * N + n) = o;
+}
+
+// rows of parts (parts > 1, fp32) or of T; false: not for these sizes and addresses
+template <typename T>
+static bool moe_weighted_sum_wide(const void* Y, int parts, int64_t stride, const float* w, void* out, int64_t tokens, int64_t top_k, int64_t N, const int32_t* ids,
+                                  int num_experts, hipStream_t s) {
+  constexpr int V = 16 / sizeof(T);
+  if (N % V != 0 || tokens > 65535 || (uintptr_t)Y % 16 != 0 || (uintptr_t)out % 16 != 0) return false;
+  const dim3 grid((unsigned)((N / V + 255) / 256), (unsigned)tokens);
+  if (parts > 1) hipLaunchKernelGGL((moe_weighted_sum_wide_kernel<T, 1, V>), grid, dim3(256), 0, s, Y, parts, stride, w, (T*)out, (int)top_k, N, ids, num_experts);
+  else hipLaunchKernelGGL((moe_weighted_sum_wide_kernel<T, 0, V>), grid, dim3(256), 0, s, Y, 1, (int64_t)0, w, (T*)out, (int)top_k, N, ids, num_experts);
+  return true;
+}
+
+int moe_weighted_sum_parts(const void* Y, int parts, const float* topk_weights, const int32_t* topk_ids, int num_experts, void* out, int dtype, int64_t tokens,
+                           int64_t top_k, int64_t N, hipStream_t s) {
+  bool done = false;
+  GGUF_DISPATCH_DTYPE(dtype, done = moe_weighted_sum_wide<scalar_t>(Y, parts, tokens * top_k * N, topk_weights, out, tokens, top_k, N, topk_ids, num_experts, s));
+  return done ? launch_status() : GGUF_NOT_TAKEN;
+}
+
 int moe_weighted_sum_live(const void* Y, const float* topk_weights, const int32_t* topk_ids, int num_experts, void* out, int dtype,
                           int64_t tokens, int64_t top_k, int64_t N, hipStream_t s, const int32_t* slot_of_pair) {
+  if (!slot_of_pair) {
+    bool done = false;
+    GGUF_DISPATCH_DTYPE(dtype, done = moe_weighted_sum_wide<scalar_t>(Y, 1, 0, topk_weights, out, tokens, top_k, N, topk_ids, num_experts, s));
+    if (done) return launch_status();
+  }
   const unsigned gx = (unsigned)((N + 255) / 256 < 64 ? (N + 255) / 256 : 64);
   for (int64_t t0 = 0; t0 < tokens; t0 += 65535) {
     const unsigned gy = (unsigned)(tokens - t0 < 65535 ? tokens - t0 : 65535);
@@ -202,18 +269,19 @@ int moe_weighted_sum_live(const void* Y, const float* topk_weights, const int32_
   return launch_status();
 }
 
-// quantize_q8_1(X) and gguf_moe_align_block_size(topk_ids) in one launch (sizes checked by the caller)
+// quantize_q8_1(X) and gguf_moe_align_block_size(topk_ids) in one launch (sizes checked by the caller).  layout of the rows: 0 plain,
+// 1 permuted (q8_permuted), 2 records (quantize_wide)
 int moe_prepare(const void* X, int xdtype, void* q8x, int tokens, int K, const int32_t* topk_ids, int numel, int num_experts, int block,
-                int32_t* sorted_ids, int sorted_capacity, int32_t* expert_ids, int expert_capacity, int32_t* num_post_padded, bool permuted,
+                int32_t* sorted_ids, int sorted_capacity, int32_t* expert_ids, int expert_capacity, int32_t* num_post_padded, int layout,
                 hipStream_t s) {
   const int Kp = (int)q8_kp(K);
   const size_t lds = (size_t)(1 + ALIGN_WAVES) * num_experts * sizeof(int);
   if (lds > 65536) return GGUF_NOT_TAKEN;
-  const int64_t threads = (int64_t)tokens * (Kp / 8);
+  const int64_t threads = (int64_t)tokens * ((layout == 2 ? K : Kp) / 8);
   const unsigned grid = 1 + (unsigned)((threads + ALIGN_THREADS - 1) / ALIGN_THREADS);
   GGUF_DISPATCH_DTYPE(xdtype, hipLaunchKernelGGL(moe_prepare_kernel<scalar_t>, dim3(grid), dim3(ALIGN_THREADS), lds, s, (const scalar_t*)X,
                                                  (char*)q8x, K, Kp, q8_row_bytes(K), tokens, topk_ids, numel, num_experts, block, sorted_ids,
-                                                 sorted_capacity, expert_ids, expert_capacity, num_post_padded, permuted));
+                                                 sorted_capacity, expert_ids, expert_capacity, num_post_padded, layout));
   return launch_status();
 }
 

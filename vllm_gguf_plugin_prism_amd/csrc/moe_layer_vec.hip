@@ -20,6 +20,8 @@
 //
 // Where experts are shared by a few pairs each (the per-pair operator's tile route on blocks of 16 slots) the same entry
 // point runs the layer in four launches on the tile kernels instead (mmq.hip, moe_tiles_layer).
+#include "dense_api.h"
+#include "tile_wide.h"
 #include "mmvq_core.h"
 
 namespace gguf {
@@ -520,8 +522,16 @@ extern "C" int64_t gguf_moe_mmq_layer_workspace_bytes(int type13, int type2, int
   using namespace gguf;
   const int route = gguf_moe_mmq_layer_takes(type13, type2, H, I, N_out, top_k, tokens, num_experts);
   const int elt = xdtype == GGUF_DTYPE_F32 ? 4 : 2;
-  if (route == 3) return moe_sorted_layer_workspace(tokens, top_k, H, I, N_out, num_experts, elt, (int)MOE_SORTED_BLOCK);
-  return route ? moe_tiles_layer_workspace(tokens, top_k, H, I, N_out, num_experts, elt, route == 1 ? 16 : 32) : 0;
+  if (!route) return 0;
+  const int64_t most = route == 3 ? moe_sorted_layer_workspace(tokens, top_k, H, I, N_out, num_experts, elt, (int)MOE_SORTED_BLOCK)
+                                  : moe_tiles_layer_workspace(tokens, top_k, H, I, N_out, num_experts, elt, route == 1 ? 16 : 32);
+  const int rt = wide_layer_takes(type13, type2, H, I, N_out, tokens, top_k, num_experts);
+  return rt ? std::max(most, wide_layer_workspace(tokens, top_k, H, I, N_out, num_experts, elt, rt)) : most;
+}
+
+extern "C" int gguf_moe_mmq_layer_wide(int type13, int type2, int64_t H, int64_t I, int64_t N_out, int64_t top_k, int64_t tokens, int64_t num_experts) {
+  return gguf_moe_mmq_layer_takes(type13, type2, H, I, N_out, top_k, tokens, num_experts) &&
+         gguf::wide_layer_takes(type13, type2, H, I, N_out, tokens, top_k, num_experts) ? 1 : 0;
 }
 
 extern "C" int gguf_moe_mmq_layer(const void* X, int xdtype, const void* W13, int type13, const void* W2, int type2, const int32_t* topk_ids,
@@ -536,6 +546,12 @@ extern "C" int gguf_moe_mmq_layer(const void* X, int xdtype, const void* W13, in
   if (!route) return GGUF_ERR_SHAPE;
   if (!X || !W13 || !W2 || !topk_ids || !topk_weights || !workspace || !out) return GGUF_ERR_NULL;
   if (((uintptr_t)W13 | (uintptr_t)W2) & 1) return GGUF_ERR_SHAPE;   // packed blocks sit at even addresses
+  // the wide tile kernel, where the workspace has room for its records
+  const int rt = wide_layer_takes(type13, type2, H, I, N_out, tokens, top_k, num_experts);
+  if (rt && wide_aligned(type13, W13) && wide_aligned(type2, W2) &&
+      workspace_bytes >= wide_layer_workspace(tokens, top_k, H, I, N_out, num_experts, xdtype == GGUF_DTYPE_F32 ? 4 : 2, rt))
+    return wide_layer(X, xdtype, workspace, W13, type13, W2, type2, topk_ids, topk_weights, out, (int)H, (int)I, (int)N_out, (int)top_k, (int)tokens, act,
+                      (int)num_experts, rt, (hipStream_t)stream);
   if (route == 3) {
     const int sorted_block = (int)MOE_SORTED_BLOCK;
     if (workspace_bytes < moe_sorted_layer_workspace(tokens, top_k, H, I, N_out, num_experts, xdtype == GGUF_DTYPE_F32 ? 4 : 2, sorted_block))

@@ -211,5 +211,25 @@ __device__ __forceinline__ void q8_1_quantize_thread(const T* __restrict__ x, ch
   }
 }
 
+// The activations of the wide tile kernel (tile_wide.h): the eight values [8 t, 8 t + 8) of row m of `rows` -> eight quants as
+// halves, of four neighbours in the order 0, 2, 1, 3, in the record of their 128 values; the block's scale and sum from the
+// first lane of each quad.
+constexpr int WIDE_REC = 272, WIDE_D_AT = 256, WIDE_S_AT = 264;
+template <typename T>
+__device__ __forceinline__ void wide_quantize_thread(const T* __restrict__ x, char* __restrict__ records, int K, int64_t rows, int64_t m, int t) {
+  float v[8];
+  load8<T>(x + m * (int64_t)K + 8 * t, v);
+  const Q8Quad q = q8_1_quantize8(v);
+  union { _Float16 h[8]; uint4 v; } o;
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    o.h[(i & 4) | ((i & 1) << 1) | ((i >> 1) & 1)] = (_Float16)(float)(int8_t)((i < 4 ? q.q.x >> (8 * i) : q.q.y >> (8 * (i - 4))) & 0xFF);
+  char* const rec = records + ((int64_t)(t >> 4) * rows + m) * WIDE_REC;
+  *(uint4*)(rec + 16 * (t & 15)) = o.v;
+  if ((t & 3) == 0) {
+    *(_Float16*)(rec + WIDE_D_AT + 2 * ((t >> 2) & 3)) = (_Float16)q.d;
+    *(_Float16*)(rec + WIDE_S_AT + 2 * ((t >> 2) & 3)) = (_Float16)q.s;
+  }
+}
 
 }  // namespace gguf

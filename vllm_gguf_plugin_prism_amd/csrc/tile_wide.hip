@@ -1,0 +1,177 @@
+// Which calls the wide tile kernel (tile_wide_core.h) takes, by ggml type.
+#include "tile_wide.h"
+#include "mmq_f.h"
+
+namespace gguf {
+
+int wide_q4_0(const WideCall& c, hipStream_t s);
+int wide_q8_0(const WideCall& c, hipStream_t s);
+int wide_q4_k(const WideCall& c, hipStream_t s);
+int wide_q5_k(const WideCall& c, hipStream_t s);
+int wide_q6_k(const WideCall& c, hipStream_t s);
+
+static bool wide_type_ok(int type) {
+  switch (type) {
+    case T_Q4_0: case T_Q8_0: case T_Q4_K: case T_Q5_K: case T_Q6_K: return true;
+    default: return false;
+  }
+}
+
+// (blocks of 144, 176, 18, 34 bytes: 256 values are whole 16-byte pieces, and rows of whole super-blocks begin where W does)
+bool wide_aligned(int type, const void* W) { return type == T_Q6_K || (uintptr_t)W % 16 == 0; }
+
+// offsets inside a matrix and inside the records of a row of super-blocks are 32-bit
+static bool wide_size_ok(int type, int64_t N, int64_t K, int64_t x_rows) {
+  return K % 256 == 0 && N * (K / block_elems(type) * block_bytes(type)) <= 0xFFFF0000ll && x_rows * WIDE_REC <= 0xFFFF0000ll;
+}
+
+int wide_layer_takes(int type13, int type2, int64_t H, int64_t I, int64_t N_out, int64_t tokens, int64_t top_k, int64_t num_experts) {
+  const int64_t pairs = tokens * top_k;
+  if (!wide_type_ok(type13) || !wide_type_ok(type2) || num_experts > 256 || !wide_size_ok(type13, 2 * I, H, tokens) || !wide_size_ok(type2, N_out, I, pairs)) return 0;
+  if (pairs * top_k > 0xFFFFFFFFll) return 0;               // (the kernel's quotient by reciprocal)
+  // Measured against the kernels that run otherwise on 600 layers of random sizes, more than 64 tokens each: 0.80 of their time, from
+  // 30 pairs per expert on 0.71.  `wgs` is the first GEMM's workgroups (64 features of h for 32 slots each, estimated): below 150
+  // most CUs have one or none, and its beginning and end lie beside nothing (layers of 25 to 40 us, 1.1 to 1.5 times as long).
+  // While an expert's pairs fill little more than one block of 16 slots, the streaming tiles pad less and have as much
+  // decoding: there Q5_K and Q6_K take 0.83, the others as long on average, Q4_0 and Q4_K 0.87 on long rows, Q8_0 0.91 on
+  // many workgroups.  (Tiles of 64 rows: 1.05 to 1.4 times as long below 64 pairs per expert, up to 1.07 times as fast above.)
+  const int64_t cap = pairs + num_experts * 31;
+  const double wgs = moe_blocks_estimate((int)cap, (int)pairs, 32) * (double)((I + 63) / 64);
+  if (wgs < 150.0) return 0;
+  if (pairs < 18 * num_experts && type13 != T_Q5_K && type13 != T_Q6_K && (type13 == T_Q8_0 ? wgs < 700.0 : H < 2304)) return 0;
+  return 1;
+}
+
+// A workgroup walks its panels one after the other, about 1.7 us each beside two others on the CU, which holds three: where the
+// tiles are fewer than that, the panels of a tile are dealt to several, three panels each at least.
+int wide_ksplit(double tiles, int K) {
+  const int np = K / 256;
+  int ks = 1;
+  while (ks < 8 && tiles * ks < 500.0 && np >= 3 * 2 * ks) ks *= 2;
+  return ks;
+}
+
+// Y = the sum of the parts of K in their order, rounded, plus the bias
+template <typename T, int V>
+__global__ __launch_bounds__(256) void wide_sum_kernel(const float* __restrict__ parts, int ksplit, int64_t stride, T* __restrict__ Y, int N, int64_t ldy,
+                                                       const T* __restrict__ bias) {
+  const int n = (blockIdx.x * 256 + threadIdx.x) * V;
+  if (n >= N) return;
+  const float* const p = parts + (int64_t)blockIdx.y * N + n;
+  struct alignas(4 * V) Row { float v[V]; } v = *(const Row*)p;
+#pragma unroll 4
+  for (int z = 1; z < ksplit; ++z) {
+    const Row r = *(const Row*)(p + z * stride);
+#pragma unroll
+    for (int e = 0; e < V; ++e) v.v[e] += r.v[e];
+  }
+  T* const y = Y + (int64_t)blockIdx.y * ldy + n;
+#pragma unroll
+  for (int e = 0; e < V; ++e) y[e] = finish<T>(v.v[e], bias, n + e);
+}
+
+int wide_any(int type, const WideCall& c, hipStream_t s) {
+  switch (type) {
+    case T_Q4_0: return wide_q4_0(c, s);
+    case T_Q8_0: return wide_q8_0(c, s);
+    case T_Q4_K: return wide_q4_k(c, s);
+    case T_Q5_K: return wide_q5_k(c, s);
+    case T_Q6_K: return wide_q6_k(c, s);
+  }
+  return GGUF_NOT_TAKEN;
+}
+
+static int64_t wide_records(int64_t M, int64_t K) { return (wide_rows_bytes(M, K) + 255) / 256 * 256; }
+
+int64_t wide_dense_workspace(int64_t M, int64_t N, int64_t K, const WidePlan& p) {
+  return wide_records(M, K) + (p.ksplit > 1 ? 4 * p.ksplit * M * N : 0);
+}
+
+// About how long a product takes, us, quantizer and the sum of the parts included: rounds of workgroups on the chip with their
+// panels, which take longer the more workgroups share a CU; the weights, the rows of X, the parts of K.  Fitted to 4000 calls of
+// random sizes (33 .. 700 rows, 512 .. 28672 columns, K 512 .. 18944, both heights of tiles, K cut into 1 .. 16); right to
+// 6 .. 8 %, so that the plan chosen by it takes 1.5 .. 3 % longer than the best.
+struct WideCost { double base, panel, weights, x, part, alone; };
+static double wide_us(int type, int M, int N, int K, const WidePlan& p) {
+  static const WideCost cost[4][2] = {{{7.8, 3.15, 0.028, 1.34, 1.36, 0.45}, {8.6, 3.87, 0.0, 1.29, 1.33, 0.63}},     // Q4_0
+                                      {{7.2, 2.85, 0.009, 1.72, 1.44, 0.40}, {8.3, 3.08, 0.0, 1.73, 1.23, 0.54}},     // Q4_K
+                                      {{7.4, 3.20, 0.014, 1.82, 1.38, 0.40}, {8.4, 3.27, 0.0, 1.50, 1.46, 0.57}},     // Q5_K
+                                      {{7.3, 4.77, 0.019, 1.50, 1.43, 0.40}, {8.5, 4.80, 0.0, 1.71, 1.18, 0.54}}};    // Q6_K
+  const WideCost& c = cost[type == T_Q4_0 ? 0 : type - T_Q4_K + 1][p.rt - 1];
+  const double r = (double)((M + 32 * p.rt - 1) / (32 * p.rt)) * (double)((N + 127) / 128) * p.ksplit / (p.rt == 1 ? 768.0 : 512.0);
+  const int np = K / 256, per = (np + p.ksplit - 1) / p.ksplit;
+  double us = c.base + c.panel * per * (c.alone + (1.0 - c.alone) * (r < 1.0 ? r : 1.0)) * 0.5 * (ceil(r) + (r > 1.0 ? r : 1.0)) + 1e-6 * (c.weights * N * K + c.x * M * K);
+  if (p.ksplit > 1) us += 2.0 + 1e-6 * c.part * p.ksplit * M * N;
+  return us;
+}
+
+static WidePlan wide_best(int type, int M, int N, int K, int64_t workspace_bytes, double& us) {
+  static const int parts[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 16};
+  WidePlan best = {0, 1};
+  us = 1e30;
+  for (int rt = 1; rt <= 2; ++rt)
+    for (int ks : parts) {
+      const WidePlan p = {rt, ks};
+      if ((ks > 1 && 3 * ks > K / 256) || wide_dense_workspace(M, N, K, p) > workspace_bytes) continue;
+      const double t = wide_us(type, M, N, K, p);
+      if (t < us) { us = t; best = p; }
+    }
+  return best;
+}
+
+static bool wide_dense_ok(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch) {
+  return (type == T_Q4_0 || (type >= T_Q4_K && type <= T_Q6_K)) && M >= 33 && M <= 2048 && K % 256 == 0 && N * w_pitch <= 0xFFFF0000ll && wide_size_ok(type, N, K, M);
+}
+
+// How long the unit takes that runs otherwise (mmq_int_us is fitted to the K-quants: Q4_0 takes 0.86 of what it says of a
+// type it does not know).
+static double wide_others_us(int type, int M, int N, int K, int64_t workspace_bytes) {
+  const int64_t int8_rows = (M * q8_row_bytes(K) + 255) / 256 * 256;
+  double us = mmq_int_us(type, M, N, K, workspace_bytes > int8_rows ? workspace_bytes - int8_rows : 0) * (type == T_Q4_0 ? 0.86 : 1.0);
+  if (type != T_Q4_0 && M >= 128 && workspace_bytes >= mmqf_rows_bytes(M, K)) us = std::min(us, mmqf_us(type, M, N, K, workspace_bytes - mmqf_rows_bytes(M, K)) + 1.5);
+  return us;
+}
+
+// Where it is the faster one by these estimates: [7968,2560] Q4_K 308 rows, others / this: 57 / 41 us, [11008,4096] 64 rows 29 / 19; but
+// [14784,4352] Q6_K 398 rows 156 / 188.  (Q8_0, whose operands need no scale on the int8 unit, is never more than a few per
+// cent faster here, and up to 45 % slower.)
+WidePlan wide_dense_plan(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, int64_t workspace_bytes) {
+  if (!wide_dense_ok(type, M, N, K, w_pitch)) return {0, 1};
+  double us;
+  const WidePlan p = wide_best(type, (int)M, (int)N, (int)K, workspace_bytes, us);
+  return p.rt && us < 0.98 * wide_others_us(type, (int)M, (int)N, (int)K, workspace_bytes) ? p : WidePlan{0, 1};
+}
+
+// The workspace that takes the call, given the size that the others would want: theirs where that costs less than a tenth.
+int64_t wide_dense_room(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, int64_t others_bytes) {
+  if (!wide_dense_ok(type, M, N, K, w_pitch)) return others_bytes;
+  double us, us_there;
+  const WidePlan p = wide_best(type, (int)M, (int)N, (int)K, INT64_MAX, us);
+  wide_best(type, (int)M, (int)N, (int)K, others_bytes, us_there);
+  if (us_there < 1.10 * us || us >= 0.98 * wide_others_us(type, (int)M, (int)N, (int)K, others_bytes)) return others_bytes;
+  return std::max(others_bytes, wide_dense_workspace(M, N, K, p));
+}
+
+int wide_dense(int type, const void* W, const void* x, int dtype, void* workspace, void* Y, int M, int N, int K, const WidePlan& p, const LinearArgs& la, hipStream_t s) {
+  int rc = quantize_wide(x, dtype, workspace, M, K, s);
+  if (rc != GGUF_OK) return rc;
+  WideCall c = {};
+  c.W = W; c.x = workspace; c.x_rows = M; c.Y = Y; c.dtype = dtype; c.M = M; c.N = N; c.K = K;
+  c.w_pitch = la.w_pitch; c.ldy = la.ldy; c.bias = la.bias;
+  c.row_blocks = (M + 32 * p.rt - 1) / (32 * p.rt);
+  c.rt = p.rt; c.ksplit = p.ksplit;
+  c.partial = (float*)((char*)workspace + wide_records(M, K));
+  rc = wide_any(type, c, s);
+  if (rc != GGUF_OK || p.ksplit == 1) return rc;
+  const int64_t ldy = la.ldy ? la.ldy : N;
+  const int V = N % 4 == 0 ? 4 : 1;
+  const dim3 grid((unsigned)((N / V + 255) / 256), (unsigned)M);
+  if (V == 4) {
+    GGUF_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((wide_sum_kernel<scalar_t, 4>), grid, dim3(256), 0, s, c.partial, p.ksplit, (int64_t)M * N, (scalar_t*)Y, N, ldy, (const scalar_t*)la.bias));
+  } else {
+    GGUF_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((wide_sum_kernel<scalar_t, 1>), grid, dim3(256), 0, s, c.partial, p.ksplit, (int64_t)M * N, (scalar_t*)Y, N, ldy, (const scalar_t*)la.bias));
+  }
+  return launch_status();
+}
+
+}  // namespace gguf

@@ -1,0 +1,226 @@
+// Packed formats as the wide tile kernel (tile_wide_core.h) reads them: one *panel* is 256 values of K of one weight row, PB
+// contiguous bytes that a wave has fetched into LDS.  A lane is (row = lane % 32, half = lane / 32) of v_mfma_f32_32x32x16_f16
+// and supplies, of every block of 32 values, the sixteen k = 16 half .. 16 half + 15 of its row: two operands of eight
+// halves, whole numbers, of four neighbours in the order 0, 2, 1, 3.
+//   KQ       super-blocks: the integer scale of a block (or of 16 values) is in the operand, d and -dmin on the sum of the
+//            super-block; else the block's scale is on every block's sum
+//   CUT      panels may begin anywhere, `at` bytes into a 16-byte piece (even); else all of them begin on one
+//   PLANES   operands per weight;  OFF: an offset term, factor() * sum over the blocks of offsets() * block sum
+//   read()   takes the lane's bytes into registers (so that the LDS slot can be filled again); scale_to() leaves scales for
+//            the lanes that hold the results: [32] d, [32] -dmin, or [8][32] block scales
+#pragma once
+#include "tile_stream_formats.h"
+
+namespace gguf {
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+// Bytes 0 and 2 (or 1 and 3) of v, two whole numbers, as the halves 1024 + x: the bytes below 0x64.
+template <int ODD> __device__ __forceinline__ f16x2 wide_bytes(uint32_t v) {
+  return __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, v, ODD ? 0x04030401u : 0x04020400u));
+}
+// The same for the bits of `mask` in the low byte of each half.  (The mask lies in a register, so that the two operations are one
+// instruction, which takes a single scalar operand.)
+__device__ __forceinline__ uint32_t in_vgpr(uint32_t v) {
+  uint32_t r;
+  asm("v_mov_b32 %0, %1" : "=v"(r) : "s"(v));
+  return r;
+}
+__device__ __forceinline__ f16x2 wide_bits(uint32_t v, uint32_t mask) { return __builtin_bit_cast(f16x2, (v & mask) | 0x64006400u); }
+__device__ __forceinline__ f16x2 both(float v) { return (f16x2){(_Float16)v, (_Float16)v}; }
+__device__ __forceinline__ f16x8 wide_operand(f16x2 a, f16x2 b, f16x2 c, f16x2 d) {
+  return __builtin_bit_cast(f16x8, make_uint4(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, c),
+                                              __builtin_bit_cast(uint32_t, d)));
+}
+__device__ __forceinline__ uint32_t word(const uint4& v, int i) { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
+
+template <bool C>
+struct WQ4_KT {
+  static constexpr int PB = 144, PLANES = 1;
+  static constexpr bool CUT = C, KQ = true, OFF = true;
+  uint4 h, q[4];
+  uint32_t s[2];
+  static __device__ __forceinline__ uint4 piece(const char* p, uint32_t at) { return C ? lds_cut16(p, at) : *(const uint4*)(p + at); }
+  __device__ __forceinline__ void read(const char* p, uint32_t at, int half) {
+    h = piece(p, at);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q[i] = piece(p, at + 16 + 32 * i + 16 * half);
+  }
+  __device__ __forceinline__ void scale_to(float* to, int row, int) {
+    to[row] = half_bits(h.x & 0xFFFF);
+    to[32 + row] = -half_bits(h.x >> 16);
+    s[0] = h.y & 0x3F3F3F3Fu;
+    s[1] = (h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u);
+  }
+  __device__ __forceinline__ uint4 offsets() const {   // the mins, eight halves
+    const uint32_t m[2] = {h.z & 0x3F3F3F3Fu, ((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u)};
+    uint32_t o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      o[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, m[i >> 1], i & 1 ? 0x04030402u : 0x04010400u)) - both(1024.0f));
+    return make_uint4(o[0], o[1], o[2], o[3]);
+  }
+  __device__ __forceinline__ f16x2 scale(int b) const {   // 1024 + the block's scale, twice
+    const uint32_t at = b & 3;
+    return __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, s[b >> 2], 0x04000400u | at << 16 | at));
+  }
+  // (high nibbles stay where they are, sixteen times as large, and the scale is a sixteenth: all exact)
+  __device__ __forceinline__ void operand(int b, int, f16x8 (&o)[1][2]) const {
+    const bool high = b & 1;
+    const f16x2 sc = high ? __builtin_elementwise_fma(scale(b), both(0.0625f), both(-64.0f)) : scale(b) - both(1024.0f);
+    const f16x2 n = sc * both(-1024.0f);
+    const uint32_t mask = in_vgpr(high ? 0x00F000F0u : 0x000F000Fu);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t x = word(q[b >> 1], 2 * i), y = word(q[b >> 1], 2 * i + 1);
+      o[0][i] = wide_operand(__builtin_elementwise_fma(wide_bits(x, mask), sc, n), __builtin_elementwise_fma(wide_bits(x >> 8, mask), sc, n),
+                             __builtin_elementwise_fma(wide_bits(y, mask), sc, n), __builtin_elementwise_fma(wide_bits(y >> 8, mask), sc, n));
+    }
+  }
+};
+
+template <bool C>
+struct WQ5_KT : WQ4_KT<C> {   // Q4_K with a fifth bit, bit b of qh[k] for block b
+  static constexpr int PB = 176;
+  using WQ4_KT<C>::h;
+  using WQ4_KT<C>::q;
+  using WQ4_KT<C>::piece;
+  uint4 qh;
+  __device__ __forceinline__ void read(const char* p, uint32_t at, int half) {
+    h = piece(p, at);
+    qh = piece(p, at + 16 + 16 * half);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q[i] = piece(p, at + 48 + 32 * i + 16 * half);
+  }
+  __device__ __forceinline__ void operand(int b, int, f16x8 (&o)[1][2]) const {
+    const f16x2 sc = this->scale(b) - both(1024.0f), n = sc * both(-1024.0f);
+    const auto codes = [&](int i) {
+      const uint32_t a = word(q[b >> 1], i), t = word(qh, i);
+      return ((b & 1 ? a >> 4 : a) & 0x0F0F0F0Fu) | ((b <= 4 ? t << (4 - b) : t >> (b - 4)) & 0x10101010u);
+    };
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t x = codes(2 * i), y = codes(2 * i + 1);
+      o[0][i] = wide_operand(__builtin_elementwise_fma(wide_bytes<0>(x), sc, n), __builtin_elementwise_fma(wide_bytes<1>(x), sc, n),
+                             __builtin_elementwise_fma(wide_bytes<0>(y), sc, n), __builtin_elementwise_fma(wide_bytes<1>(y), sc, n));
+    }
+  }
+};
+
+// Block b = 4 n + t: low nibbles (t < 2) or high ones of ql[64 n + 32 (t % 2) ..], bits 2 t of qh[32 n ..]; a scale per 16
+// values, so one for a lane and block.  (code - 32) * scale has 13 bits: two operands, on scale & ~15 and scale & 15.
+struct WQ6_K {
+  static constexpr int PB = 210, PLANES = 2;
+  static constexpr bool CUT = true, KQ = true, OFF = false;
+  uint4 l[4], hi[2], sc;
+  uint32_t d;
+  __device__ __forceinline__ void read(const char* p, uint32_t at, int half) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) l[i] = lds_cut16(p, at + 32 * i + 16 * half);
+#pragma unroll
+    for (int n = 0; n < 2; ++n) hi[n] = lds_cut16(p, at + 128 + 32 * n + 16 * half);
+    sc = lds_cut16(p, at + 192);
+    d = lds_h(p, at + 208);
+  }
+  __device__ __forceinline__ void scale_to(float* to, int row, int half) {
+    to[row] = half_bits(d);
+    const int up = 8 * half;                                // the lane's scales are the even bytes
+    sc = make_uint4(sc.x >> up, sc.y >> up, sc.z >> up, sc.w >> up);
+  }
+  __device__ __forceinline__ uint4 offsets() const { return make_uint4(0, 0, 0, 0); }
+  __device__ __forceinline__ void operand(int b, int, f16x8 (&o)[2][2]) const {
+    const int n = b >> 2, t = b & 3;
+    // 1024 + the scale's byte, twice; its upper half as 128 more than it is
+    const uint32_t c = __builtin_bit_cast(uint32_t, __builtin_amdgcn_perm(0x64646464u, word(sc, b >> 1), b & 1 ? 0x04020402u : 0x04000400u));
+    const f16x2 sl = __builtin_bit_cast(f16x2, c & 0x640F640Fu) - both(1024.0f);
+    const f16x2 sh = __builtin_bit_cast(f16x2, (c ^ 0x00800080u) & 0x64F064F0u) - both(1152.0f);
+    const auto codes = [&](int i) {
+      const uint32_t a = word(l[2 * n + (t & 1)], i), u = word(hi[n], i);
+      return ((t < 2 ? a : a >> 4) & 0x0F0F0F0Fu) | ((t == 0 ? u << 4 : t == 1 ? u << 2 : t == 2 ? u : u >> 2) & 0x30303030u);
+    };
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t x = codes(2 * i), y = codes(2 * i + 1);
+      const f16x2 k = both(1056.0f), x0 = wide_bytes<0>(x) - k, x1 = wide_bytes<1>(x) - k, y0 = wide_bytes<0>(y) - k, y1 = wide_bytes<1>(y) - k;
+      o[0][i] = wide_operand(x0 * sh, x1 * sh, y0 * sh, y1 * sh);
+      o[1][i] = wide_operand(x0 * sl, x1 * sl, y0 * sl, y1 * sl);
+    }
+  }
+};
+
+// Eight blocks of BB bytes, an fp16 scale in front of each.
+template <int BB, bool C>
+struct W32 {
+  static constexpr int PB = 8 * BB, PLANES = 1;
+  static constexpr bool CUT = C, KQ = false;
+  uint4 q[8];
+  uint32_t d[4];                                            // the eight scales, two in a word
+  // sixteen bytes from 2 + lane_at of every block (lane_at a multiple of 16; the blocks' bytes begin 2, 4, 6, 0, ... behind an
+  // 8-byte word)
+  __device__ __forceinline__ void read_blocks(const char* p, uint32_t at, uint32_t lane_at) {
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+      if (C) {
+        q[b] = lds_cut16(p, at + BB * b + 2 + lane_at);
+        continue;
+      }
+      const int first = BB * b + 2, cut = first % 8;
+      const uint2* const w = (const uint2*)(p + (first - cut) + lane_at);
+      const uint2 a = w[0], c = w[1];
+      if (cut == 0) {
+        q[b] = make_uint4(a.x, a.y, c.x, c.y);
+      } else {
+        const uint2 e = w[2];
+        const uint32_t x0 = cut >= 4 ? a.y : a.x, x1 = cut >= 4 ? c.x : a.y, x2 = cut >= 4 ? c.y : c.x, x3 = cut >= 4 ? e.x : c.y, x4 = cut >= 4 ? e.y : e.x;
+        q[b] = cut == 4 ? make_uint4(x0, x1, x2, x3)
+                        : make_uint4(__builtin_amdgcn_alignbit(x1, x0, 16), __builtin_amdgcn_alignbit(x2, x1, 16), __builtin_amdgcn_alignbit(x3, x2, 16),
+                                     __builtin_amdgcn_alignbit(x4, x3, 16));
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d[i] = lds_h(p, (C ? at : 0u) + BB * 2 * i) | lds_h(p, (C ? at : 0u) + BB * (2 * i + 1)) << 16;
+  }
+  __device__ __forceinline__ void scale_to(float* to, int row, int half) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) to[32 * (4 * half + i) + row] = half_bits(((half ? d[2 + (i >> 1)] : d[i >> 1]) >> (16 * (i & 1))) & 0xFFFF);
+  }
+};
+
+// values 0..15 of a block are the low nibbles of its 16 bytes, 16..31 the high ones; d (q - 8), the 8 on the block sum
+template <bool C>
+struct WQ4_0T : W32<18, C> {
+  static constexpr bool OFF = true;
+  static constexpr float FACTOR = -8.0f;
+  using W32<18, C>::d;
+  using W32<18, C>::q;
+  __device__ __forceinline__ void read(const char* p, uint32_t at, int) { this->read_blocks(p, at, 0); }
+  __device__ __forceinline__ uint4 offsets() const { return make_uint4(d[0], d[1], d[2], d[3]); }
+  __device__ __forceinline__ void operand(int b, int half, f16x8 (&o)[1][2]) const {
+    const uint32_t mask = half ? 0x00F000F0u : 0x000F000Fu;
+    const f16x2 sc = both(half ? 0.0625f : 1.0f), n = both(half ? -64.0f : -1024.0f);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t x = word(q[b], 2 * i), y = word(q[b], 2 * i + 1);
+      o[0][i] = wide_operand(__builtin_elementwise_fma(wide_bits(x, mask), sc, n), __builtin_elementwise_fma(wide_bits(x >> 8, mask), sc, n),
+                             __builtin_elementwise_fma(wide_bits(y, mask), sc, n), __builtin_elementwise_fma(wide_bits(y >> 8, mask), sc, n));
+    }
+  }
+};
+
+struct WQ8_0 : W32<34, false> {
+  static constexpr bool OFF = false;
+  static constexpr float FACTOR = 0.0f;
+  __device__ __forceinline__ void read(const char* p, uint32_t at, int half) { read_blocks(p, at, 16 * half); }
+  __device__ __forceinline__ uint4 offsets() const { return make_uint4(0, 0, 0, 0); }
+  __device__ __forceinline__ void operand(int b, int, f16x8 (&o)[1][2]) const {
+    const f16x2 k = both(1152.0f);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t x = word(q[b], 2 * i) ^ 0x80808080u, y = word(q[b], 2 * i + 1) ^ 0x80808080u;
+      o[0][i] = wide_operand(wide_bytes<0>(x) - k, wide_bytes<1>(x) - k, wide_bytes<0>(y) - k, wide_bytes<1>(y) - k);
+    }
+  }
+};
+
+}  // namespace gguf

@@ -232,10 +232,10 @@ PyObject* merged_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t m = x->size(0), k = x->size(1);
   const size_t esz = x->element_size();
   struct Part { int64_t start, end, type, rb, largest; Path path; };
-  const auto half_unit = [&](const Part& p, int64_t rows) {
-    if (m <= 32) return false;
+  const auto unit = [&](const Part& p, int64_t rows) {
+    if (m <= 32) return 0;
     const int64_t pitch = w->size(0) > 1 ? w->stride(0) : p.rb;
-    return gguf_mmq_layer_route((int)p.type, rows, k, m, pitch, gguf_mmq_layer_workspace_bytes((int)p.type, rows, k, m, pitch)) == 2;
+    return gguf_mmq_layer_unit((int)p.type, rows, k, m, pitch, gguf_mmq_layer_workspace_bytes((int)p.type, rows, k, m, pitch));
   };
   std::vector<Part> parts;
   int64_t width = 0;
@@ -257,7 +257,7 @@ PyObject* merged_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
       Part& last = parts.back();
       const int64_t largest = std::max(last.largest, rows);
       if (last.end == p.start && last.type == p.type && last.rb == p.rb && last.path == p.path &&
-          (p.path != PATH_MMQ || half_unit(p, largest) == half_unit(p, p.end - last.start))) {
+          (p.path != PATH_MMQ || unit(p, largest) == unit(p, p.end - last.start))) {
         last.end = p.end;
         last.largest = largest;
         continue;

@@ -200,7 +200,7 @@ def _shard_runs(x, weight, shards):
     from . import ops
 
     def unit(t, rows):
-        return int(x.shape[0]) > 32 and x.dim() == 2 and ops._mmq_route(t, rows, x.shape[1], x.shape[0], weight.stride(0)) == 2
+        return x.dim() == 2 and int(x.shape[0]) > 32 and ops._mmq_unit(t, rows, x.shape[1], x.shape[0], weight.stride(0))
 
     runs = []
     for shard in shards:

@@ -234,12 +234,19 @@ def _dense_result_fits(X: torch.Tensor, row: int, out: torch.Tensor | None, bias
 
 
 def _mmq_route(quant_type: int, row: int, col: int, vecs: int, w_pitch: int, workspace_bytes: int | None = None) -> int:
-    """The kernel that :func:`ggml_mul_mat_a8` runs on its own workspace or one of this size: 1 the streaming tile kernel,
-    2 the half-precision unit's whole-number GEMM, 0 another."""
+    """The kernel that :func:`ggml_mul_mat_a8` runs on its own workspace or one of this size where it is not on the wide
+    tiles: 1 the streaming tile kernel, 2 the half-precision unit's whole-number GEMM, 0 another."""
     L = _lib.lib()
     if workspace_bytes is None:
         workspace_bytes = L.gguf_mmq_layer_workspace_bytes(int(quant_type), row, col, vecs, w_pitch)
     return L.gguf_mmq_layer_route(int(quant_type), row, col, vecs, w_pitch, workspace_bytes)
+
+
+def _mmq_unit(quant_type: int, row: int, col: int, vecs: int, w_pitch: int) -> int:
+    """:func:`_mmq_route`, 3 where the call runs on the wide tiles."""
+    L = _lib.lib()
+    workspace_bytes = L.gguf_mmq_layer_workspace_bytes(int(quant_type), row, col, vecs, w_pitch)
+    return L.gguf_mmq_layer_unit(int(quant_type), row, col, vecs, w_pitch, workspace_bytes)
 
 
 def _product_is_watched(X: torch.Tensor, *others: torch.Tensor | None) -> bool:
