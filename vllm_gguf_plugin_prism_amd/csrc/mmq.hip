@@ -905,7 +905,7 @@ extern "C" int gguf_mmq_layer_route(int type, int64_t N, int64_t K, int64_t M, i
 
 extern "C" int gguf_mmq_layer_unit(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes) {
   const int route = gguf_mmq_layer_route(type, N, K, M, w_row_pitch_bytes, workspace_bytes);
-  return route != 1 && M > 0 && N > 0 && K > 0 && gguf::wide_dense_plan(type, M, N, K, w_row_pitch_bytes, workspace_bytes).rt ? 3 : route;
+  return route != 1 && M > 0 && N > 0 && K > 0 && gguf::wide_dense_plan(type, M, N, K, w_row_pitch_bytes, workspace_bytes).rt ? route + 4 : route;
 }
 
 // room for either engine

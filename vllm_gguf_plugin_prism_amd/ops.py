@@ -243,7 +243,7 @@ def _mmq_route(quant_type: int, row: int, col: int, vecs: int, w_pitch: int, wor
 
 
 def _mmq_unit(quant_type: int, row: int, col: int, vecs: int, w_pitch: int) -> int:
-    """:func:`_mmq_route`, 3 where the call runs on the wide tiles."""
+    """:func:`_mmq_route`, 4 more where the call runs on the wide tiles."""
     L = _lib.lib()
     workspace_bytes = L.gguf_mmq_layer_workspace_bytes(int(quant_type), row, col, vecs, w_pitch)
     return L.gguf_mmq_layer_unit(int(quant_type), row, col, vecs, w_pitch, workspace_bytes)
