@@ -8,16 +8,36 @@ from oracle import gguf_oracle as o
 
 pytestmark = pytest.mark.gpu
 
-DENSE = (o.Q4_0, o.Q4_K, o.Q5_K, o.Q6_K)
+DENSE = (o.Q4_0, o.Q4_K, o.Q5_K, o.Q6_K, o.Q2_K, o.Q3_K, o.Q4_1, o.Q5_1)
+ONES = (o.Q4_1, o.Q5_1)
 
 
 # one row over a tile of 32 and of 64; a last column tile of one, four, some columns; one panel, K in one part and in
 # several, a part that is longer than another; more tiles than a round of workgroups; rows of W a pitch apart that moves
-# them through the positions inside 16 bytes
+# them through the positions inside 16 bytes (whole 16 bytes where only those are taken)
 @pytest.mark.parametrize("qtype", DENSE)
 @pytest.mark.parametrize("m,n,k,pad", [(33, 4097, 256, 0), (64, 2052, 1536, 2), (33, 640, 2560, 0), (97, 1300, 768, 0), (160, 1030, 2304, 6),
                                        (300, 2500, 512, 0), (64, 256, 8192, 0), (97, 25604, 256, 0)])
 def test_dense_edges(qtype, m, n, k, pad):
+    check_dense(qtype, m, n, k, 8 * pad if qtype in ONES else pad)
+
+
+# the last panel has one block, four, seven; K in one part and in several; more rows than other types are taken with
+@pytest.mark.parametrize("qtype,m,n,k", [(o.Q4_1, 33, 640, 2176), (o.Q4_1, 97, 1300, 896), (o.Q5_1, 64, 2052, 1600), (o.Q5_1, 200, 256, 2496),
+                                         (o.Q4_1, 40, 300, 384), (o.Q2_K, 2100, 130, 256), (o.Q5_1, 2100, 130, 320)])
+def test_last_panels(qtype, m, n, k):
+    check_dense(qtype, m, n, k, 0)
+
+
+# a workspace for half of the rows: two passes (the oracle on rows of both, of the second's last tile)
+def test_two_passes():
+    from vllm_gguf_plugin_prism_amd import _lib
+    m, n, k = 2041, 2052, 3072
+    assert _lib.lib().gguf_mmq_layer_workspace_bytes(o.Q2_K, n, k, m, k // 256 * 84) < k // 128 * m * 272
+    check_dense(o.Q2_K, m, n, k, 0, np.r_[:3, 1020:1030, m - 30:m])
+
+
+def check_dense(qtype, m, n, k, pad, rows=np.s_[:]):
     from vllm_gguf_plugin_prism_amd import ops
     rng = np.random.default_rng(n + m)
     w = o.make_weights(rng, qtype, n, k)
@@ -27,7 +47,7 @@ def test_dense_edges(qtype, m, n, k, pad):
     x = rng.standard_normal((m, k)).astype(np.float32) + 0.3
     bias = rng.standard_normal(n).astype(np.float32)
     y = ops.ggml_mul_mat_a8(wd, torch.from_numpy(x).cuda(), qtype, n, bias=torch.from_numpy(bias).cuda())
-    assert o.rel_l2(y.cpu().numpy(), o.mul_mat_a8(w, x, qtype, n, "mmq") + bias) <= 1e-5
+    assert o.rel_l2(y.cpu().numpy()[rows], o.mul_mat_a8(w, x[rows], qtype, n, "mmq") + bias) <= 1e-5
 
 
 # the largest operands and sums, and scales that are subnormal halves (an offset that is rounded away would be all of it)
@@ -41,6 +61,12 @@ def test_largest_sums_and_smallest_scales(qtype):
     if qtype == o.Q6_K:
         w[:, :, :192], w[:, :, 192:208] = 0, 0x80          # codes -32, scales -128
         w[::2, :, 208:210] = np.frombuffer(np.float16(3e-6).tobytes(), np.uint8)
+    elif qtype in (o.Q2_K, o.Q3_K):
+        at = size - (4 if qtype == o.Q2_K else 2)          # (scales 31 for Q3_K, codes -4 where its third bits are clear)
+        w[:, :, :at] = 0xFF
+        if qtype == o.Q3_K:
+            w[1::3, :, :96] = 0
+        w[::2, :, at : at + 2] = np.frombuffer(np.float16(3e-6).tobytes(), np.uint8)
     else:
         w[:, :, 4 if qtype != o.Q4_0 else 2:] = 0xFF
         w[::2, :, :2] = np.frombuffer(np.float16(3e-6).tobytes(), np.uint8)

@@ -980,7 +980,7 @@ int gguf::mmq_linear_impl(const void* W, int64_t w_row_pitch_bytes, const void* 
     const int rc = mmvq_any(type, W, x, q8_workspace, Y, xdtype, N, K, M, s, lt);
     if (rc != GGUF_NOT_TAKEN) return rc;
   }
-  if (engine == GGUF_MMQ_AUTO && ((uintptr_t)q8_workspace & 15) == 0) {
+  if (engine == GGUF_MMQ_AUTO && ((uintptr_t)q8_workspace & 15) == 0 && wide_dense_aligned(type, W)) {
     const WidePlan p = wide_dense_plan(type, M, N, K, w_row_pitch_bytes, workspace_bytes);
     if (p.rt) return wide_dense(type, W, x, xdtype, q8_workspace, Y, (int)M, (int)N, (int)K, p, la, s);
   }

@@ -57,11 +57,11 @@ int quantize_whole(const void* x, int xdtype, const MmqfRows& r, int64_t M, int6
 template <typename T>
 __global__ __launch_bounds__(256) void quantize_wide_kernel(const T* __restrict__ x, char* __restrict__ records, int K, int64_t rows, int64_t m0) {
   const int t = blockIdx.x * 256 + threadIdx.x;
-  if (t * 8 < K) wide_quantize_thread<T>(x, records, K, rows, m0 + blockIdx.y, t);   // (K is a multiple of 256: quads stay together)
+  if (t * 8 < (K + 255) / 256 * 256) wide_quantize_thread<T>(x, records, K, rows, m0 + blockIdx.y, t);   // (whole records: quads stay together)
 }
 
 int quantize_wide(const void* x, int xdtype, void* records, int64_t M, int64_t K, hipStream_t stream) {
-  const int gx = (int)((K / 8 + 255) / 256);
+  const int gx = (int)(((K + 255) / 256 * 32 + 255) / 256);
   for (int64_t off = 0; off < M; off += 65535) {
     const int rows = (int)((M - off) < 65535 ? (M - off) : 65535);
     GGUF_DISPATCH_DTYPE(xdtype, hipLaunchKernelGGL(quantize_wide_kernel<scalar_t>, dim3(gx, rows), dim3(256), 0, stream, (const scalar_t*)x, (char*)records, (int)K, M, off));

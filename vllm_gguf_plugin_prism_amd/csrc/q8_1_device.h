@@ -217,8 +217,8 @@ __device__ __forceinline__ void q8_1_quantize_thread(const T* __restrict__ x, ch
 constexpr int WIDE_REC = 272, WIDE_D_AT = 256, WIDE_S_AT = 264;
 template <typename T>
 __device__ __forceinline__ void wide_quantize_thread(const T* __restrict__ x, char* __restrict__ records, int K, int64_t rows, int64_t m, int t) {
-  float v[8];
-  load8<T>(x + m * (int64_t)K + 8 * t, v);
+  float v[8] = {};
+  if (8 * t < K) load8<T>(x + m * (int64_t)K + 8 * t, v);   // (behind K: zeros)
   const Q8Quad q = q8_1_quantize8(v);
   union { _Float16 h[8]; uint4 v; } o;
 #pragma unroll

@@ -35,7 +35,7 @@ typedef float wide_f4 __attribute__((ext_vector_type(4)));
 constexpr int WIDE_NW = 4, WIDE_N = 32 * WIDE_NW;
 
 struct WideArgs {
-  int M, N, np;                // rows of X (dense); weight rows; panels per row
+  int M, N, np, nkb;           // rows of X (dense); weight rows; panels and blocks per row (the last panel may have fewer than eight)
   int col_wgs;                 // workgroups side by side
   uint32_t w_pitch, x_plane;   // bytes between weight rows; between the records of neighbouring panels of a row of X
   uint32_t topk_inv;           // 2^32 / top_k rounded up
@@ -93,7 +93,7 @@ __device__ __forceinline__ void wide_pin(float (&v)[16]) {   // the sixteen valu
 // LDS: two buffers of records | a panel per wave | a wave's scales for the lanes that hold results | the slots' pairs
 template <class F> constexpr int wide_ppr() { return ((F::CUT ? F::PB + 29 : F::PB) / 16) | 1; }   // 16-byte pieces of a panel row (odd: banks)
 template <int R> constexpr int wide_xbuf() { return (32 * R * (WIDE_REC / 16) + 63) / 64 * 1024; }
-template <class F> constexpr int wide_scale_bytes() { return F::KQ ? (F::OFF ? 256 : 128) : 1024; }
+template <class F> constexpr int wide_scale_bytes() { return F::KIND == SUPER ? (F::OFF ? 256 : 128) : 1024; }
 template <class F, int R> constexpr size_t wide_lds() {
   return 2 * wide_xbuf<R>() + (size_t)WIDE_NW * (512 * wide_ppr<F>() + wide_scale_bytes<F>() + 256) + 16;
 }
@@ -152,7 +152,8 @@ __global__ __launch_bounds__(64 * WIDE_NW, R == 1 ? 3 : 2) void tile_wide_kernel
   const auto row_of = [&](int r) { return GATE ? (r < 16 ? min(n0 + r, gate.inner - 1) : gate.inner + min(n0 + r - 16, gate.inner - 1)) : min(n0 + r, a.N - 1); };
   const uint32_t wmis = F::CUT ? (uint32_t)((uintptr_t)W & 15) : 0u;
   const uint8_t* const wbase = W - wmis;
-  const uint32_t last16 = ((uint32_t)(rows_all - 1) * a.w_pitch + wmis + (uint32_t)(a.np * F::PB) - 1) & ~15u;   // the last granule that holds bytes of W
+  const uint32_t row_bytes = F::KIND == SUPER ? (uint32_t)(a.np * F::PB) : (uint32_t)(a.nkb * (F::PB / 8));
+  const uint32_t last16 = ((uint32_t)(rows_all - 1) * a.w_pitch + wmis + row_bytes - 1) & ~15u;   // the last granule that holds bytes of W
   uint32_t w_at[NI], w_piece[NI];
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
@@ -207,6 +208,7 @@ __global__ __launch_bounds__(64 * WIDE_NW, R == 1 ? 3 : 2) void tile_wide_kernel
   for (int p = p0; p < p1; ++p) {
     F w;
     uint2 sums[R][2];
+    f32x16 off[R];
 #pragma unroll
     for (int hh = 0; hh < 2; ++hh) {
       // This chunk's records have landed, and with hh = 0 the panel; what was asked for behind them are the next panel's weights.
@@ -221,12 +223,14 @@ __global__ __launch_bounds__(64 * WIDE_NW, R == 1 ? 3 : 2) void tile_wide_kernel
         const char* const panel = smem + RING_AT + wave * SLOT + lrow * (16 * PPR);
         const uint32_t at = F::CUT ? ((uint32_t)row_of(lrow) * a.w_pitch + wmis + (uint32_t)(p * F::PB)) & 15 : 0u;
         w.read(panel, at, half);
+        if (F::KIND != SUPER && a.nkb < 8 * (p + 1)) w.limit(a.nkb - 8 * p);
         w.scale_to((float*)scales, lrow, half);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the panel's place may be filled again
         if (p + 1 < p1) request(p + 1);
       }
       const char* const xrow = smem + hh * XB + lrow * WIDE_REC;
       float d8[R][4];
+      uint2 dh[R], sh[R];                                   // the same as halves, and the sums
       f16x8 xo[2][2], wo[F::PLANES][2];
 #pragma unroll
       for (int k = 0; k < R; ++k) {
@@ -235,7 +239,8 @@ __global__ __launch_bounds__(64 * WIDE_NW, R == 1 ? 3 : 2) void tile_wide_kernel
         d8[k][1] = half_bits(v.x >> 16);
         d8[k][2] = half_bits(v.y & 0xFFFF);
         d8[k][3] = half_bits(v.y >> 16);
-        sums[k][hh] = make_uint2(v.z, v.w);
+        sums[k][hh] = sh[k] = make_uint2(v.z, v.w);
+        dh[k] = make_uint2(v.x, v.y);
         // (as floats from here on: the compiler would have every multiply-add convert its scale, in a form that takes twice as long)
         asm volatile("" : "+v"(d8[k][0]), "+v"(d8[k][1]), "+v"(d8[k][2]), "+v"(d8[k][3]));
       }
@@ -258,53 +263,81 @@ __global__ __launch_bounds__(64 * WIDE_NW, R == 1 ? 3 : 2) void tile_wide_kernel
       for (int u = 0; u < U; ++u) {
         const int b = 4 * hh + u / R, k = u % R;
         __builtin_amdgcn_sched_barrier(0);
+        f16x8 xm, xn;                                       // the operands of unit u, whose place is taken now
+        if constexpr (F::MIN16) { xm = xo[u & 1][0]; xn = xo[u & 1][1]; }
         if (u + 2 < U) load_x(u + 2, xo[u & 1]);
         if (u + 1 < U && (u + 1) % R == 0) w.operand(4 * hh + (u + 1) / R, half, wo);
         wide_f4 dw[4];
-        if constexpr (!F::KQ)
+        uint2 wd[4], wm[4];
+        f16x2 xd, xs;
+        if constexpr (F::KIND == BLOCK)
 #pragma unroll
           for (int q = 0; q < 4; ++q) dw[q] = *(const wide_f4*)(scales + 4 * (32 * b + 8 * q + 4 * half));
+        if constexpr (F::KIND == HALVES) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            wd[q] = *(const uint2*)(scales + 2 * (32 * b + 8 * q + 4 * half));
+            wm[q] = *(const uint2*)(scales + 512 + 2 * (32 * b + 8 * q + 4 * half));
+          }
+          const uint32_t twice = u / R & 1 ? 0x03020302u : 0x01000100u;
+          xd = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0u, u / R < 2 ? dh[k].x : dh[k].y, twice));
+          xs = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0u, u / R < 2 ? sh[k].x : sh[k].y, twice));
+        }
+        if constexpr (F::MIN16) {
+          // d8 times the sum of the lane's sixteen quants (whole numbers up to 2032, exact as halves), a contraction over the
+          // block's two groups in fp32
+          f16x8 v = xm + xn;
+          const f16x2 t = (f16x2){v[0], v[1]} + (f16x2){v[2], v[3]}, z = (f16x2){v[4], v[5]} + (f16x2){v[6], v[7]}, y = t + z;
+          off[k] = __builtin_amdgcn_mfma_f32_32x32x2f32(w.min16(b), d8[k][b & 3] * (float)(y[0] + y[1]), b == 0 ? zero : off[k], 0, 0, 0);
+        }
 #pragma unroll
         for (int piece = 0; piece < P; ++piece) {
           if (u + 1 < U) mfma(u + 1, piece);
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
           for (int r = 16 / P * piece; r < 16 / P * (piece + 1); ++r) {
-            if constexpr (F::KQ) part[k][r] = b == 0 ? s[u & 1][r] * d8[k][b & 3] : __builtin_fmaf(s[u & 1][r], d8[k][b & 3], part[k][r]);
-            else acc[k][r] = __builtin_fmaf(s[u & 1][r] * dw[r >> 2][r & 3], d8[k][b & 3], acc[k][r]);
+            if constexpr (F::KIND == SUPER) {
+              part[k][r] = b == 0 ? s[u & 1][r] * d8[k][b & 3] : __builtin_fmaf(s[u & 1][r], d8[k][b & 3], part[k][r]);
+            } else if constexpr (F::KIND == BLOCK) {
+              acc[k][r] = __builtin_fmaf(s[u & 1][r] * dw[r >> 2][r & 3], d8[k][b & 3], acc[k][r]);
+            } else {
+              const uint32_t dp = r & 2 ? wd[r >> 2].y : wd[r >> 2].x, mp = r & 2 ? wm[r >> 2].y : wm[r >> 2].x;
+              const f16x2 dd = __builtin_bit_cast(f16x2, dp) * xd, ms = __builtin_bit_cast(f16x2, mp) * xs;
+              acc[k][r] += __builtin_fmaf(s[u & 1][r], (float)dd[r & 1], (float)ms[r & 1]);
+            }
           }
           __builtin_amdgcn_sched_barrier(0);
         }
-        if constexpr (F::KQ) wide_pin(part[k]);
+        if constexpr (F::KIND == SUPER) wide_pin(part[k]);
         else wide_pin(acc[k]);
       }
     }
     // ---- the end of the panel: the offsets (a contraction over eight: the upper half of the lanes holds values 8 .. 15, zeros),
     // the super-block's scales
     uint4 mv = make_uint4(0, 0, 0, 0);
-    if (F::OFF && half == 0) mv = w.offsets();
+    if (F::OFF && !F::MIN16 && half == 0) mv = w.offsets();
+    if constexpr (F::KIND == SUPER || F::OFF)
 #pragma unroll
     for (int k = 0; k < R; ++k) {
-      f32x16 off;
-      if constexpr (F::OFF) {
+      if constexpr (F::OFF && !F::MIN16) {
         const uint4 sv = half ? make_uint4(0, 0, 0, 0) : make_uint4(sums[k][0].x, sums[k][0].y, sums[k][1].x, sums[k][1].y);
-        off = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, mv), __builtin_bit_cast(f16x8, sv), zero, 0, 0, 0);
+        off[k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, mv), __builtin_bit_cast(f16x8, sv), zero, 0, 0, 0);
       }
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         wide_f4 d, dm;
-        if constexpr (F::KQ) {
+        if constexpr (F::KIND == SUPER) {
           d = *(const wide_f4*)(scales + 4 * (8 * q + 4 * half));
           if constexpr (F::OFF) dm = *(const wide_f4*)(scales + 128 + 4 * (8 * q + 4 * half));
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           float& v = acc[k][4 * q + e];
-          if constexpr (F::KQ) {
+          if constexpr (F::KIND == SUPER) {
             v = __builtin_fmaf(part[k][4 * q + e], d[e], v);
-            if constexpr (F::OFF) v = __builtin_fmaf(off[4 * q + e], dm[e], v);
+            if constexpr (F::OFF) v = __builtin_fmaf(off[k][4 * q + e], dm[e], v);
           } else if constexpr (F::OFF) {
-            v = __builtin_fmaf(off[4 * q + e], F::FACTOR, v);
+            v = __builtin_fmaf(off[k][4 * q + e], F::FACTOR, v);
           }
         }
       }
@@ -383,7 +416,7 @@ __global__ __launch_bounds__(64 * WIDE_NW, R == 1 ? 3 : 2) void tile_wide_kernel
 template <class F, int R, bool GATE>
 static int wide_launch(const WideCall& c, hipStream_t stream) {
   constexpr size_t lds = wide_lds<F, R>();
-  const int qk = F::KQ ? 256 : 32, bs = F::KQ ? F::PB : F::PB / 8;
+  const int qk = F::KIND == SUPER ? 256 : 32, bs = F::KIND == SUPER ? F::PB : F::PB / 8;
   const int64_t pitch = c.w_pitch ? c.w_pitch : (int64_t)(c.K / qk) * bs;
   if (!F::CUT && (pitch % 16 != 0 || (uintptr_t)c.W % 16 != 0 || (c.moe.sorted_token_ids && c.moe.expert_stride % 16 != 0))) return GGUF_NOT_TAKEN;
   auto kern = tile_wide_kernel<F, R, GATE>;
@@ -394,7 +427,7 @@ static int wide_launch(const WideCall& c, hipStream_t stream) {
   const int dtype = split ? GGUF_DTYPE_F32 : c.dtype, elt = dtype == GGUF_DTYPE_F32 ? 4 : 2;
   const int64_t ldy = split || !c.ldy ? (int64_t)c.N : c.ldy, rows_y = c.moe.sorted_token_ids ? c.moe.num_pairs : c.M;
   void* const y = split ? (void*)c.partial : c.Y;
-  const WideArgs a = {c.M, c.N, c.K / 256, cols, (uint32_t)pitch, (uint32_t)(c.x_rows * WIDE_REC), (uint32_t)((0x100000000ull + top_k - 1) / top_k),
+  const WideArgs a = {c.M, c.N, (c.K + 255) / 256, c.K / 32, cols, (uint32_t)pitch, (uint32_t)(c.x_rows * WIDE_REC), (uint32_t)((0x100000000ull + top_k - 1) / top_k),
                       dtype, ldy % 4 == 0 && (uintptr_t)y % (4 * elt) == 0, ldy, split ? nullptr : c.bias, split ? c.ksplit : 1, rows_y * ldy};
   hipLaunchKernelGGL(kern, dim3((unsigned)((int64_t)c.row_blocks * cols), (unsigned)a.ksplit), dim3(64 * WIDE_NW), lds, stream, (const uint8_t*)c.W, (const char*)c.x,
                      y, a, c.moe, c.gate);
@@ -402,16 +435,20 @@ static int wide_launch(const WideCall& c, hipStream_t stream) {
 }
 
 template <class F>
-static int wide_run(const WideCall& c, hipStream_t s) {
-  if (c.K % 256 != 0) return GGUF_NOT_TAKEN;
-  if (c.gate.rows) return c.rt == 1 ? wide_launch<F, 1, true>(c, s) : GGUF_NOT_TAKEN;
+static int wide_dense_run(const WideCall& c, hipStream_t s) {
+  if (c.gate.rows || c.moe.sorted_token_ids || c.K % (F::KIND == SUPER ? 256 : 32) != 0) return GGUF_NOT_TAKEN;
   return c.rt == 1 ? wide_launch<F, 1, false>(c, s) : wide_launch<F, 2, false>(c, s);
+}
+template <class F>
+static int wide_run(const WideCall& c, hipStream_t s) {
+  if (!c.moe.sorted_token_ids) return wide_dense_run<F>(c, s);
+  if (c.K % 256 != 0 || c.rt != 1) return GGUF_NOT_TAKEN;   // (blocks of 32 slots only)
+  return c.gate.rows ? wide_launch<F, 1, true>(c, s) : wide_launch<F, 1, false>(c, s);
 }
 // a dense product whose rows do not begin on 16 bytes (a shard of a merged tensor as wide as its widest one): A the panels that do
 template <class A, class F>
 static int wide_run_either(const WideCall& c, hipStream_t s) {
-  if (c.moe.sorted_token_ids || ((uintptr_t)c.W % 16 == 0 && c.w_pitch % 16 == 0)) return wide_run<A>(c, s);
-  return c.rt == 1 ? wide_launch<F, 1, false>(c, s) : wide_launch<F, 2, false>(c, s);
+  return c.moe.sorted_token_ids || ((uintptr_t)c.W % 16 == 0 && c.w_pitch % 16 == 0) ? wide_run<A>(c, s) : wide_dense_run<F>(c, s);
 }
 
 }  // namespace gguf

@@ -2,12 +2,16 @@
 // contiguous bytes that a wave has fetched into LDS.  A lane is (row = lane % 32, half = lane / 32) of v_mfma_f32_32x32x16_f16
 // and supplies, of every block of 32 values, the sixteen k = 16 half .. 16 half + 15 of its row: two operands of eight
 // halves, whole numbers, of four neighbours in the order 0, 2, 1, 3.
-//   KQ       super-blocks: the integer scale of a block (or of 16 values) is in the operand, d and -dmin on the sum of the
-//            super-block; else the block's scale is on every block's sum
+//   KIND     SUPER: super-blocks, the integer scale of a block (or of 16 values) is in the operand, d and -dmin on the sum of the
+//            super-block; BLOCK: the block's scale is on every block's sum; HALVES: on every block's sum half(d * d8), and
+//            half(m * s8) added, the products rounded to half precision as the reference's __hmul2 leaves them
+//            (vecdotq.cuh:71-93, 179-198)
 //   CUT      panels may begin anywhere, `at` bytes into a 16-byte piece (even); else all of them begin on one
-//   PLANES   operands per weight;  OFF: an offset term, factor() * sum over the blocks of offsets() * block sum
+//   PLANES   operands per weight;  OFF: an offset term, FACTOR (or -dmin) * sum over the blocks of offsets() * block sum;
+//   MIN16    the offset is a min per 16 values, min16(), times d8 * the sum of those quants
 //   read()   takes the lane's bytes into registers (so that the LDS slot can be filled again); scale_to() leaves scales for
-//            the lanes that hold the results: [32] d, [32] -dmin, or [8][32] block scales
+//            the lanes that hold the results: [32] d, [32] -dmin; [8][32] block scales; [8][32] d, [8][32] m as halves
+//   limit()  the panel has only so many blocks; what lies behind them need not be a number (formats of 32-value blocks)
 #pragma once
 #include "tile_stream_formats.h"
 
@@ -35,10 +39,13 @@ __device__ __forceinline__ f16x8 wide_operand(f16x2 a, f16x2 b, f16x2 c, f16x2 d
 }
 __device__ __forceinline__ uint32_t word(const uint4& v, int i) { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
 
+enum WideKind { SUPER, BLOCK, HALVES };
+
 template <bool C>
 struct WQ4_KT {
-  static constexpr int PB = 144, PLANES = 1;
-  static constexpr bool CUT = C, KQ = true, OFF = true;
+  static constexpr int PB = 144, PLANES = 1, KIND = SUPER;
+  static constexpr bool CUT = C, OFF = true, MIN16 = false;
+  __device__ __forceinline__ void limit(int) {}
   uint4 h, q[4];
   uint32_t s[2];
   static __device__ __forceinline__ uint4 piece(const char* p, uint32_t at) { return C ? lds_cut16(p, at) : *(const uint4*)(p + at); }
@@ -111,8 +118,9 @@ struct WQ5_KT : WQ4_KT<C> {   // Q4_K with a fifth bit, bit b of qh[k] for block
 // Block b = 4 n + t: low nibbles (t < 2) or high ones of ql[64 n + 32 (t % 2) ..], bits 2 t of qh[32 n ..]; a scale per 16
 // values, so one for a lane and block.  (code - 32) * scale has 13 bits: two operands, on scale & ~15 and scale & 15.
 struct WQ6_K {
-  static constexpr int PB = 210, PLANES = 2;
-  static constexpr bool CUT = true, KQ = true, OFF = false;
+  static constexpr int PB = 210, PLANES = 2, KIND = SUPER;
+  static constexpr bool CUT = true, OFF = false, MIN16 = false;
+  __device__ __forceinline__ void limit(int) {}
   uint4 l[4], hi[2], sc;
   uint32_t d;
   __device__ __forceinline__ void read(const char* p, uint32_t at, int half) {
@@ -149,11 +157,87 @@ struct WQ6_K {
   }
 };
 
+// Codes of 3 bits less 4 times a signed 6-bit scale per 16 values: one operand.  Block b = 4 n + t: bits 2 t of qs[32 n ..], the
+// third bit, of the other sign, bit b of hmask[k]; scale 2 b + half: four bits of the first eight bytes, two of the last four.
+struct WQ3_K {
+  static constexpr int PB = 110, PLANES = 1, KIND = SUPER;
+  static constexpr bool CUT = true, OFF = false, MIN16 = false;
+  uint4 q[2], hm, sc;
+  uint32_t d;
+  __device__ __forceinline__ void limit(int) {}
+  __device__ __forceinline__ void read(const char* p, uint32_t at, int half) {
+    hm = lds_cut16(p, at + 16 * half);
+#pragma unroll
+    for (int n = 0; n < 2; ++n) q[n] = lds_cut16(p, at + 32 + 32 * n + 16 * half);
+    const uint2 lo = lds_cut8(p, at + 96), hi = lds_cut8(p, at + 102);   // (bytes 96 .. 103, 102 .. 109)
+    sc = make_uint4(lo.x, lo.y, __builtin_amdgcn_alignbit(hi.y, hi.x, 16), 0);
+    d = hi.y >> 16;
+  }
+  __device__ __forceinline__ void scale_to(float* to, int row, int half) {
+    to[row] = half_bits(d);
+    const int up = 8 * half;                                // the lane's scales are the even bytes
+    sc = make_uint4(sc.x >> up, sc.y >> up, sc.z >> up, 0);
+  }
+  __device__ __forceinline__ uint4 offsets() const { return make_uint4(0, 0, 0, 0); }
+  __device__ __forceinline__ void operand(int b, int, f16x8 (&o)[1][2]) const {
+    const int n = b >> 2, t = b & 3;
+    const uint32_t lo = ((t < 2 ? sc.x : sc.y) >> (16 * (t & 1) + 4 * n)) & 15u, hi = (sc.z >> (16 * (t & 1) + 4 * n + 2 * (t >> 1))) & 3u;
+    const f16x2 s = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, lo | hi << 4, 0x04000400u)) - both(1056.0f), k = both(1028.0f);
+    const auto codes = [&](int i) {
+      const uint32_t a = word(q[n], i) >> (2 * t), m = word(hm, i);
+      return (a & 0x03030303u) | ((b <= 2 ? m << (2 - b) : m >> (b - 2)) & 0x04040404u);
+    };
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t x = codes(2 * i), y = codes(2 * i + 1);
+      o[0][i] = wide_operand((wide_bytes<0>(x) - k) * s, (wide_bytes<1>(x) - k) * s, (wide_bytes<0>(y) - k) * s, (wide_bytes<1>(y) - k) * s);
+    }
+  }
+};
+
+// Codes of 2 bits, a 4-bit scale and a 4-bit min per 16 values.  Block b = 4 n + t: bits 2 t of qs[32 n ..].
+struct WQ2_K {
+  static constexpr int PB = 84, PLANES = 1, KIND = SUPER;
+  static constexpr bool CUT = true, OFF = true, MIN16 = true;
+  uint4 q[2], sc;
+  uint32_t dm;
+  __device__ __forceinline__ void limit(int) {}
+  __device__ __forceinline__ void read(const char* p, uint32_t at, int half) {
+    sc = lds_cut16(p, at);
+#pragma unroll
+    for (int n = 0; n < 2; ++n) q[n] = lds_cut16(p, at + 16 + 32 * n + 16 * half);
+    dm = lds_h(p, at + 80) | lds_h(p, at + 82) << 16;
+  }
+  __device__ __forceinline__ void scale_to(float* to, int row, int half) {
+    to[row] = half_bits(dm & 0xFFFF);
+    to[32 + row] = -half_bits(dm >> 16);
+    const int up = 8 * half;                                // the lane's scales are the even bytes
+    sc = make_uint4(sc.x >> up, sc.y >> up, sc.z >> up, sc.w >> up);
+  }
+  __device__ __forceinline__ uint4 offsets() const { return make_uint4(0, 0, 0, 0); }
+  __device__ __forceinline__ float min16(int b) const { return (float)((word(sc, b >> 1) >> (16 * (b & 1) + 4)) & 15u); }
+  __device__ __forceinline__ void operand(int b, int, f16x8 (&o)[1][2]) const {
+    const int n = b >> 2, t = b & 3;
+    const uint32_t c = (word(sc, b >> 1) >> (16 * (b & 1))) & 15u;
+    const f16x2 s = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, c, 0x04000400u)) - both(1024.0f), z = s * both(-1024.0f);   // (exact)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t x = (word(q[n], 2 * i) >> (2 * t)) & 0x03030303u, y = (word(q[n], 2 * i + 1) >> (2 * t)) & 0x03030303u;
+      o[0][i] = wide_operand(__builtin_elementwise_fma(wide_bytes<0>(x), s, z), __builtin_elementwise_fma(wide_bytes<1>(x), s, z),
+                             __builtin_elementwise_fma(wide_bytes<0>(y), s, z), __builtin_elementwise_fma(wide_bytes<1>(y), s, z));
+    }
+  }
+};
+
 // Eight blocks of BB bytes, an fp16 scale in front of each.
 template <int BB, bool C>
 struct W32 {
-  static constexpr int PB = 8 * BB, PLANES = 1;
-  static constexpr bool CUT = C, KQ = false;
+  static constexpr int PB = 8 * BB, PLANES = 1, KIND = BLOCK;
+  static constexpr bool CUT = C, MIN16 = false;
+  __device__ __forceinline__ void limit(int left) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d[i] = 2 * i + 1 < left ? d[i] : 2 * i < left ? d[i] & 0xFFFFu : 0u;
+  }
   uint4 q[8];
   uint32_t d[4];                                            // the eight scales, two in a word
   // sixteen bytes from 2 + lane_at of every block (lane_at a multiple of 16; the blocks' bytes begin 2, 4, 6, 0, ... behind an
@@ -204,6 +288,64 @@ struct WQ4_0T : W32<18, C> {
       const uint32_t x = word(q[b], 2 * i), y = word(q[b], 2 * i + 1);
       o[0][i] = wide_operand(__builtin_elementwise_fma(wide_bits(x, mask), sc, n), __builtin_elementwise_fma(wide_bits(x >> 8, mask), sc, n),
                              __builtin_elementwise_fma(wide_bits(y, mask), sc, n), __builtin_elementwise_fma(wide_bits(y >> 8, mask), sc, n));
+    }
+  }
+};
+
+// a block's fifth bits, of the lane's values 4 i .. 4 i + 3, as 16 in four bytes (bits: those of its sixteen values)
+__device__ __forceinline__ uint32_t fifth_bits(uint32_t bits, int i) { return __umul24((i ? bits >> (4 * i - 4) : bits << 4) & 0xF0u, 0x204081u) & 0x10101010u; }
+
+// Q4_1, Q5_1: d q + m
+template <bool FIFTH>
+struct WQ45_1 {
+  static constexpr int BB = FIFTH ? 24 : 20, PB = 8 * BB, PLANES = 1, KIND = HALVES;
+  static constexpr bool CUT = false, OFF = false, MIN16 = false;
+  uint4 q[8];
+  uint32_t dm[8], qh[FIFTH ? 4 : 1];
+  __device__ __forceinline__ void limit(int left) {
+#pragma unroll
+    for (int b = 0; b < 8; ++b) dm[b] = b < left ? dm[b] : 0u;
+  }
+  __device__ __forceinline__ void read(const char* p, uint32_t, int half) {
+    constexpr int N = BB / 4;
+    uint32_t v[8 * N];
+#pragma unroll
+    for (int i = 0; i < 2 * N; ++i) {
+      const uint4 x = ((const uint4*)p)[i];
+      v[4 * i] = x.x; v[4 * i + 1] = x.y; v[4 * i + 2] = x.z; v[4 * i + 3] = x.w;
+    }
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+      const int i = N * b;
+      dm[b] = v[i];
+      q[b] = make_uint4(v[i + N - 4], v[i + N - 3], v[i + N - 2], v[i + N - 1]);
+      if constexpr (FIFTH) {
+        const uint32_t five = (v[i + 1] >> (16 * half)) & 0xFFFFu;
+        qh[b >> 1] = b & 1 ? qh[b >> 1] | five << 16 : five;
+      }
+    }
+  }
+  __device__ __forceinline__ void scale_to(float* to, int row, int half) {
+    uint16_t* const h = (uint16_t*)to;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t v = half ? dm[4 + i] : dm[i];
+      h[32 * (4 * half + i) + row] = (uint16_t)(v & 0xFFFF);
+      h[256 + 32 * (4 * half + i) + row] = (uint16_t)(v >> 16);
+    }
+  }
+  __device__ __forceinline__ uint4 offsets() const { return make_uint4(0, 0, 0, 0); }
+  __device__ __forceinline__ void operand(int b, int half, f16x8 (&o)[1][2]) const {
+    const f16x2 k = both(1024.0f);
+    const auto codes = [&](int i) {
+      const uint32_t v = (word(q[b], i) >> (4 * half)) & 0x0F0F0F0Fu;
+      if constexpr (FIFTH) return v | fifth_bits(qh[b >> 1] >> (16 * (b & 1)), i);
+      else return v;
+    };
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t x = codes(2 * i), y = codes(2 * i + 1);
+      o[0][i] = wide_operand(wide_bytes<0>(x) - k, wide_bytes<1>(x) - k, wide_bytes<0>(y) - k, wide_bytes<1>(y) - k);
     }
   }
 };
