@@ -1,0 +1,64 @@
+"""Products of 5 to 32 rows on the streaming tile kernel (csrc/tile_stream_core.h) of the formats without a grouped layer on it,
+and the GEMV operator's rows there, at the edges of its tiles against the CPU oracle."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import gguf_oracle as o
+
+pytestmark = pytest.mark.gpu
+
+TILES = (o.Q2_K, o.Q3_K, o.Q4_1, o.Q5_0, o.Q5_1)
+GEMV = (o.Q4_0, o.Q8_0, o.Q4_K, o.Q5_K, o.Q6_K, *TILES, o.IQ4_NL, o.IQ4_XS)
+
+
+# one tile of rows, full and in part, two, several (the GEMV operator takes any number), more than a launch's; a last column group of one, four, all columns; K in one panel and in several, one of
+# them in part (formats of 32-value blocks); K over the waves of a workgroup; rows a pitch apart that moves them inside 16 bytes
+def check(op, path, qtype, m, n, k, pad):
+    rng = np.random.default_rng(n + m)
+    block, _ = o.QUANT_SIZES[qtype]
+    k = k // block * block
+    w = o.make_weights(rng, qtype, n, k)
+    wd = torch.zeros(n, w.shape[1] + pad, dtype=torch.uint8, device="cuda")[:, :w.shape[1]]
+    wd.copy_(torch.from_numpy(w))
+    x = rng.standard_normal((m, k)).astype(np.float32) + 0.3
+    bias = rng.standard_normal(n).astype(np.float32)
+    y = op(wd, torch.from_numpy(x).cuda(), qtype, n, bias=torch.from_numpy(bias).cuda())
+    assert o.rel_l2(y.cpu().numpy(), o.mul_mat_a8(w, x, qtype, n, path) + bias) <= 1e-5
+
+
+SIZES = [(5, 4097, 256, 0), (9, 2052, 1568, 2), (16, 640, 2848, 0), (17, 1300, 768, 6), (31, 1040, 4384, 0), (32, 260, 9216, 0)]
+
+
+@pytest.mark.parametrize("qtype", TILES)
+@pytest.mark.parametrize("m,n,k,pad", SIZES)
+def test_tiles(qtype, m, n, k, pad):
+    from vllm_gguf_plugin_prism_amd import ops
+    check(ops.ggml_mul_mat_a8, "mmq", qtype, m, n, k, pad)
+
+
+@pytest.mark.parametrize("qtype", GEMV)
+@pytest.mark.parametrize("m,n,k,pad", [*SIZES, (6, 4100, 9216, 0), (70, 1040, 2304, 0), (515, 130, 768, 0)])
+def test_gemv_operator(qtype, m, n, k, pad):
+    from vllm_gguf_plugin_prism_amd import ops
+    check(ops.ggml_mul_mat_vec_a8, "mmvq", qtype, m, n, k, pad)
+
+
+# the largest codes and scales of either sign, so that no block sum leaves the range in which it is exact
+@pytest.mark.parametrize("qtype", TILES)
+def test_largest_sums(qtype):
+    from vllm_gguf_plugin_prism_amd import ops
+    rng = np.random.default_rng(qtype)
+    n, k, m = 384, 512, 12
+    block, size = o.QUANT_SIZES[qtype]
+    w = o.make_weights(rng, qtype, n, k).reshape(n, k // block, size)
+    first, last = {o.Q2_K: (0, 80), o.Q3_K: (0, 108), o.Q4_1: (4, 20), o.Q5_0: (2, 22), o.Q5_1: (4, 24)}[qtype]
+    w[:, :, first:last] = 0xFF
+    w[1::2, :, first:last] = 0
+    w = w.reshape(n, -1)
+    x = rng.choice([-1.0, 1.0], size=(m, k)).astype(np.float32) * 3.0
+    x[: m // 2] = np.abs(x[: m // 2])
+    y = ops.ggml_mul_mat_a8(torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda(), qtype, n).cpu().numpy()
+    want = o.mul_mat_a8(w, x, qtype, n, "mmq")
+    for part in (np.s_[::2], np.s_[1::2]):
+        assert np.linalg.norm(y[:, part] - want[:, part]) <= 1e-5 * np.linalg.norm(want[:, part])

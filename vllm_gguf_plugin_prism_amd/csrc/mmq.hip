@@ -962,15 +962,7 @@ int gguf::mmq_linear_impl(const void* W, int64_t w_row_pitch_bytes, const void* 
   const int64_t partial_room = workspace_bytes - rows_bytes;
   const bool tiles_at_5 = M <= 16 && rows16_direct_pays(type, (int)M, N, K, true) && rows16_direct_takes(W, w_row_pitch_bytes, type, (int)M, (int)N, (int)K, partial_room > 0 ? partial_room : 0);
   if (engine != GGUF_MMQ_HALF && ts_dense_takes(type, M, N, K, w_row_pitch_bytes)) {
-    int rc = quantize_q8_1(x, xdtype, q8_workspace, M, K, s, 0, nullptr, true);
-    if (rc != GGUF_OK) return rc;
-    TsCall c = {};
-    c.W = W; c.ws = q8_workspace; c.Y = Y; c.dtype = xdtype; c.M = (int)M; c.N = (int)N; c.K = (int)K;
-    c.rt = M <= 16 ? 1 : 2;
-    c.w_pitch = la.w_pitch; c.ldy = la.ldy; c.bias = la.bias;
-    c.row_blocks = 1;
-    c.live_blocks = 1;
-    return ts_any(type, c, s);
+    return ts_dense(type, W, x, xdtype, q8_workspace, Y, M, (int)N, (int)K, false, la, s);
   }
   if (engine == GGUF_MMQ_AUTO && M <= 8 && !tiles_at_5) {
     // a handful of rows: the streaming GEMV kernel with the tile kernels' offset sums reads W once at close to the

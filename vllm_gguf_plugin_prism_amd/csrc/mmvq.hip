@@ -1,6 +1,7 @@
 // C entry points of the decode-path GEMV and of the per-pair MoE GEMV.  The kernels live in mmvq_core.h and are
 // instantiated per group of formats in the mmvq_<group>.hip files; this file validates and routes by ggml type.
 #include "gguf_common.h"
+#include "tile_stream.h"
 
 namespace gguf {
 
@@ -38,35 +39,13 @@ int moe_vec_group_iq_c(int type, const void* W, const void* x, void* Y, int dtyp
 
 namespace gguf {
 // one GEMV call after validation; with la.tile_sums the result is GGUF_NOT_TAKEN where the streaming kernel does not apply
-// rows16_direct.hip: 16-row MFMA tiles read straight from the packed blocks (Q4_K, Q5_K, Q6_K)
-bool rows16_direct_takes(const void* W, int64_t w_pitch, int type, int M, int N, int K, int64_t partial_bytes);
-bool rows16_direct_pays(int type, int M, int64_t N, int64_t K, bool against_gemv);
-int rows16_direct(const void* W, const void* ws, void* Y, int dtype, int type, int M, int N, int K, float* partial, int64_t partial_bytes,
-                  hipStream_t s, const LinearArgs& la, bool gemv_sums);
-
 int mmvq_any(int type, const void* W, const void* x, void* q8_workspace, void* Y, int xdtype, int64_t N, int64_t K, int64_t M,
              hipStream_t s, const LinearArgs& la) {
-  // Five rows or more (nine for Q4_0 / Q8_0) of a matrix of at least 8M weights: the tile kernel's time does not grow
-  // with the rows (up to 16 or 32 per launch), the streaming kernel's does (Q4_K [14336,4096] at 8 / 16 rows 22 / 42 us
-  // against 17 us, Q6_K 36 / 71 against 27 us, Q4_0 at 16 rows 36 against 22 us).  The operator's workspace holds the quantized rows and nothing else, so K up to 4096 (beyond that
-  // the tile kernel wants room for partial tiles).  The arithmetic stays the GEMV's (offset term on d8 * sum(q8)).
-  if (!la.tile_sums && N <= 0x7FFFFFF0LL && K <= 0x7FFFFFF0LL && rows16_direct_pays(type, (int)(M < 16 ? M : 16), N, K, true) &&
-      rows16_direct_takes(W, la.w_pitch, type, 16, (int)N, (int)K, 0)) {
-    int rc = quantize_q8_1(x, xdtype, q8_workspace, M, K, s);
-    if (rc != GGUF_OK) return rc;
-    const int64_t ldy = la.ldy ? la.ldy : N, esz = xdtype == GGUF_DTYPE_F32 ? 4 : 2;
-    const int step = rows16_direct_takes(W, la.w_pitch, type, 32, (int)N, (int)K, 0) ? 32 : 16;   // (the K-quants take 32 rows per launch)
-    for (int64_t m0 = 0; m0 < M; m0 += step) {
-      const int rows = (int)(M - m0 < step ? M - m0 : step);
-      rc = rows16_direct(W, (const char*)q8_workspace + m0 * q8_row_bytes(K), (char*)Y + m0 * ldy * esz, xdtype, type, rows, (int)N, (int)K,
-                         nullptr, 0, s, la, true);
-      // takes() was asked for a full chunk above; a chunk the tile kernel then declines is a planning error, never a
-      // result the caller should see as the internal "not taken" code with part of Y written
-      if (rc == GGUF_NOT_TAKEN) return GGUF_ERR_LAUNCH;
-      if (rc != GGUF_OK) return rc;
-    }
-    return GGUF_OK;
-  }
+  // Five rows or more: tiles of rows, whose time does not grow with the rows in a tile, in the GEMV's arithmetic (the rule
+  // and both sides' times: ts_dense_takes).  The operator's workspace, the quantized rows, is what they want.
+  const int64_t pitch = la.w_pitch ? la.w_pitch : K / block_elems(type) * block_bytes(type);
+  if (!la.tile_sums && ((uintptr_t)q8_workspace & 15) == 0 && ts_dense_takes(type, M, N, K, pitch, true))
+    return ts_dense(type, W, x, xdtype, q8_workspace, Y, M, (int)N, (int)K, true, la, s);
   switch (type) {
     case T_Q4_0: return mmvq_group_std_a(type, W, x, q8_workspace, Y, xdtype, N, K, M, s, la);
     case T_Q4_1: return mmvq_group_std_a(type, W, x, q8_workspace, Y, xdtype, N, K, M, s, la);

@@ -418,14 +418,14 @@ static int dense16_fmt(const void* W, const void* ws, void* Y, int dtype, int M,
 }
 
 int rows16_direct(const void* W, const void* ws, void* Y, int dtype, int type, int M, int N, int K, float* partial, int64_t partial_bytes,
-                  hipStream_t s, const LinearArgs& la, bool gemv_sums);   // rows16_direct.hip
+                  hipStream_t s, const LinearArgs& la);   // rows16_direct.hip
 bool rows16_direct_pays(int type, int M, int64_t N, int64_t K, bool against_gemv);
 
 // q8_1(X) . W^T for a few rows of X (the quantized rows are in the workspace); GGUF_NOT_TAKEN for other formats.
 int mmq_rows16(const void* W, const void* ws, void* Y, int dtype, int type, int M, int N, int K, float* partial, int64_t partial_bytes,
                hipStream_t s, const LinearArgs& la) {
   if (rows16_direct_pays(type, M, N, K, false)) {   // straight from the packed blocks (the K-quants up to 32 rows, Q4_0 / Q8_0 up to 16)
-    const int rc = rows16_direct(W, ws, Y, dtype, type, M, N, K, partial, partial_bytes, s, la, false);
+    const int rc = rows16_direct(W, ws, Y, dtype, type, M, N, K, partial, partial_bytes, s, la);
     if (rc != GGUF_NOT_TAKEN) return rc;
   }
   // the 16-deep formats pay two MFMAs and four vector instructions per result and block on the staged tiles as in the

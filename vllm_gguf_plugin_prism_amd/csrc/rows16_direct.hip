@@ -57,11 +57,10 @@ struct Direct16Args {
 
 enum { DIRECT_Q4_K = 0, DIRECT_Q5_K = 1, DIRECT_Q6_K = 2, DIRECT_Q4_0 = 3, DIRECT_Q8_0 = 4 };
 
-// NP: 16-column tiles a wave takes in turn (the workgroup owns 16 NP columns).  GSUM (Q4_K, Q5_K): the offset term
-// multiplies d8 * sum(q8), the GEMV operator's arithmetic (vecdotq.cuh:328-351), instead of the stored block sum.
+// NP: 16-column tiles a wave takes in turn (the workgroup owns 16 NP columns).
 // RT: 16-row tiles of X (1 or 2).  With two, every weight operand meets both tiles' activations; the 32 rows of a
 // 4096-value stretch fill LDS, so one workgroup runs per CU, with twice the registers.
-template <typename T, int KSPL, int NP, int FMT, bool GSUM, int RT>
+template <typename T, int KSPL, int NP, int FMT, int RT>
 __global__ __launch_bounds__(64 * KSPL, RT == 2 ? 2 : 4) void rows16_direct_kernel(const uint8_t* __restrict__ W, const char* __restrict__ ws,
                                                                       T* __restrict__ Y, const T* __restrict__ bias, Direct16Args a) {
   constexpr bool Q5 = FMT == DIRECT_Q5_K, Q6 = FMT == DIRECT_Q6_K, Q40 = FMT == DIRECT_Q4_0, Q80 = FMT == DIRECT_Q8_0;
@@ -151,7 +150,7 @@ __global__ __launch_bounds__(64 * KSPL, RT == 2 ? 2 : 4) void rows16_direct_kern
     for (int i = 0; i < SI; ++i) {
       const int kb = min(at + TPR * i, spr - 1);
       dreg[rt][i] = asc[kb];
-      sreg[rt][i] = asc[(GSUM ? 2 : 1) * (a.Kp / 32) + kb];   // the stored sum s8, or du = d8 * sum(q8)
+      sreg[rt][i] = asc[a.Kp / 32 + kb];                        // the stored sum
     }
   }
   Blk cur, nxt;
@@ -167,16 +166,7 @@ __global__ __launch_bounds__(64 * KSPL, RT == 2 ? 2 : 4) void rows16_direct_kern
 #pragma unroll
   for (int i = 0; i < SI; ++i) {
     // d8 and s8 are half-precision values widened to fp32 by the quantizer: the narrowing is exact.  du is not one, but
-    // du / d8 = sum(q8) is an integer of at most 13 bits (|sum| <= 32 * 127 = 4064), exact as a quotient; a half holds
-    // integers exactly only up to 2048, so the sum travels as a 16-bit integer in the place of the second half and is
-    // widened again where d8 multiplies it together with the block sum.
-    // (the hardware reciprocal's last-bit error rounds away: the quotient lies within 4065 * 2^-22 of an integer)
-    h2_d pair = {(_Float16)dreg[rt][i], (_Float16)sreg[rt][i]};
-    if constexpr (GSUM) {
-      const int qsum = dreg[rt][i] != 0.0f ? (int)__builtin_rintf(sreg[rt][i] * __builtin_amdgcn_rcpf(dreg[rt][i])) : 0;
-      const uint32_t bits = (uint32_t)__builtin_bit_cast(uint16_t, pair[0]) | ((uint32_t)qsum << 16);
-      pair = __builtin_bit_cast(h2_d, bits);
-    }
+    const h2_d pair = {(_Float16)dreg[rt][i], (_Float16)sreg[rt][i]};
     xsc[min(at + TPR * i, spr - 1) * XR + 16 * rt + am] = pair;
   }
   if constexpr (XROWS > XR)
@@ -336,14 +326,8 @@ __global__ __launch_bounds__(64 * KSPL, RT == 2 ? 2 : 4) void rows16_direct_kern
 #pragma unroll
               for (int r = 0; r < 4; ++r) {
                 const h2_d hh = __builtin_bit_cast(h2_d, scw[r]);
-                if constexpr (GSUM) {   // d8 * (S * dw - m * sum(q8)): the offset joins the block sum before d8 is applied
-                  const float qsum = (float)((int)scw[r] >> 16);   // the 16-bit integer staged in place of the second half
-                  const float u = __builtin_fmaf(qsum, nm, seeded_times(S[r], w, nsw));
-                  acc[rt][q][r] = __builtin_fmaf(u, (float)hh[0], acc[rt][q][r]);
-                } else {
-                  acc[rt][q][r] = __builtin_fmaf(seeded_times(S[r], w, nsw), (float)hh[0], acc[rt][q][r]);
-                  acc[rt][q][r] = __builtin_fmaf((float)hh[1], nm, acc[rt][q][r]);
-                }
+                acc[rt][q][r] = __builtin_fmaf(seeded_times(S[r], w, nsw), (float)hh[0], acc[rt][q][r]);
+                acc[rt][q][r] = __builtin_fmaf((float)hh[1], nm, acc[rt][q][r]);
               }
             }
           }
@@ -439,14 +423,14 @@ static inline int direct_block_bytes(int type) {
   return type == T_Q6_K ? 210 : type == T_Q5_K ? 176 : type == T_Q4_0 ? 8 * 18 : type == T_Q8_0 ? 8 * 34 : 144;
 }
 
-template <typename T, int NP, int FMT, bool GSUM, int RT = 1>
+template <typename T, int NP, int FMT, int RT = 1>
 static int rows16_direct_launch(const void* W, const void* ws, void* Y, int M, int N, int K, float* partial, const Direct16Plan& p,
                                 hipStream_t stream, const LinearArgs& la) {
   constexpr int KSPL = kDirectKspl, N_T = 16 * NP, XROWS = FMT == DIRECT_Q4_K || FMT == DIRECT_Q5_K ? 16 * RT : 16 * RT + 1;
   constexpr int BS = FMT == DIRECT_Q6_K ? 210 : FMT == DIRECT_Q5_K ? 176 : FMT == DIRECT_Q4_0 ? 8 * 18 : FMT == DIRECT_Q8_0 ? 8 * 34 : 144;
   const size_t act = (size_t)XROWS * (p.per_wg * 256 + 16) + (size_t)p.per_wg * 8 * 16 * RT * 4, red = (size_t)KSPL * 16 * RT * N_T * 4;
   const size_t lds = act > red ? act : red;
-  auto kern = rows16_direct_kernel<T, KSPL, NP, FMT, GSUM, RT>;
+  auto kern = rows16_direct_kernel<T, KSPL, NP, FMT, RT>;
   if (lds > 65536) {
     static std::atomic<uint64_t> done{0};
     allow_large_lds(kern, RT * 80 * 1024, done);
@@ -463,27 +447,16 @@ static int rows16_direct_launch(const void* W, const void* ws, void* Y, int M, i
 
 template <typename T, int FMT>
 static int rows16_direct_typed(const void* W, const void* ws, void* Y, int M, int N, int K, float* partial, const Direct16Plan& p,
-                               hipStream_t stream, const LinearArgs& la, bool gemv_sums) {
-  if constexpr (FMT == DIRECT_Q4_K || FMT == DIRECT_Q5_K) {   // (the two operators agree on the other formats)
-    if (gemv_sums) {
-      if (p.rt == 2) {   // 17 .. 32 rows
-        if (p.np == 4) return rows16_direct_launch<T, 4, FMT, true, 2>(W, ws, Y, M, N, K, partial, p, stream, la);
-        if (p.np == 2) return rows16_direct_launch<T, 2, FMT, true, 2>(W, ws, Y, M, N, K, partial, p, stream, la);
-        return rows16_direct_launch<T, 1, FMT, true, 2>(W, ws, Y, M, N, K, partial, p, stream, la);
-      }
-      if (p.np == 2) return rows16_direct_launch<T, 2, FMT, true>(W, ws, Y, M, N, K, partial, p, stream, la);
-      return rows16_direct_launch<T, 1, FMT, true>(W, ws, Y, M, N, K, partial, p, stream, la);
-    }
-  }
+                               hipStream_t stream, const LinearArgs& la) {
   if constexpr (FMT == DIRECT_Q4_K || FMT == DIRECT_Q5_K || FMT == DIRECT_Q6_K) {
     if (p.rt == 2) {   // 17 .. 32 rows
-      if (p.np == 4) return rows16_direct_launch<T, 4, FMT, false, 2>(W, ws, Y, M, N, K, partial, p, stream, la);
-      if (p.np == 2) return rows16_direct_launch<T, 2, FMT, false, 2>(W, ws, Y, M, N, K, partial, p, stream, la);
-      return rows16_direct_launch<T, 1, FMT, false, 2>(W, ws, Y, M, N, K, partial, p, stream, la);
+      if (p.np == 4) return rows16_direct_launch<T, 4, FMT, 2>(W, ws, Y, M, N, K, partial, p, stream, la);
+      if (p.np == 2) return rows16_direct_launch<T, 2, FMT, 2>(W, ws, Y, M, N, K, partial, p, stream, la);
+      return rows16_direct_launch<T, 1, FMT, 2>(W, ws, Y, M, N, K, partial, p, stream, la);
     }
   }
-  if (p.np == 2) return rows16_direct_launch<T, 2, FMT, false>(W, ws, Y, M, N, K, partial, p, stream, la);
-  return rows16_direct_launch<T, 1, FMT, false>(W, ws, Y, M, N, K, partial, p, stream, la);
+  if (p.np == 2) return rows16_direct_launch<T, 2, FMT>(W, ws, Y, M, N, K, partial, p, stream, la);
+  return rows16_direct_launch<T, 1, FMT>(W, ws, Y, M, N, K, partial, p, stream, la);
 }
 
 // Whether rows16_direct() would run this call.
@@ -513,28 +486,27 @@ bool rows16_direct_pays(int type, int M, int64_t N, int64_t K, bool against_gemv
 
 // Q4_K, Q5_K (W and its row pitch 16-byte aligned), Q6_K with at most 32 rows of X, Q4_0 or Q8_0 with at most 16;
 // GGUF_NOT_TAKEN otherwise.
-// gemv_sums: the GEMV operator's offset term (see GSUM) instead of the tile operator's.
 int rows16_direct(const void* W, const void* ws, void* Y, int dtype, int type, int M, int N, int K, float* partial, int64_t partial_bytes,
-                  hipStream_t s, const LinearArgs& la, bool gemv_sums) {
+                  hipStream_t s, const LinearArgs& la) {
   if (!rows16_direct_takes(W, la.w_pitch, type, M, N, K, partial_bytes)) return GGUF_NOT_TAKEN;
   const Direct16Plan p = direct16_plan(M, N, K, partial_bytes);
   if (type == T_Q6_K) {
-    GGUF_DISPATCH_DTYPE(dtype, return (rows16_direct_typed<scalar_t, DIRECT_Q6_K>(W, ws, Y, M, N, K, partial, p, s, la, gemv_sums)));
+    GGUF_DISPATCH_DTYPE(dtype, return (rows16_direct_typed<scalar_t, DIRECT_Q6_K>(W, ws, Y, M, N, K, partial, p, s, la)));
     return GGUF_ERR_DTYPE;
   }
   if (type == T_Q4_0) {
-    GGUF_DISPATCH_DTYPE(dtype, return (rows16_direct_typed<scalar_t, DIRECT_Q4_0>(W, ws, Y, M, N, K, partial, p, s, la, gemv_sums)));
+    GGUF_DISPATCH_DTYPE(dtype, return (rows16_direct_typed<scalar_t, DIRECT_Q4_0>(W, ws, Y, M, N, K, partial, p, s, la)));
     return GGUF_ERR_DTYPE;
   }
   if (type == T_Q8_0) {
-    GGUF_DISPATCH_DTYPE(dtype, return (rows16_direct_typed<scalar_t, DIRECT_Q8_0>(W, ws, Y, M, N, K, partial, p, s, la, gemv_sums)));
+    GGUF_DISPATCH_DTYPE(dtype, return (rows16_direct_typed<scalar_t, DIRECT_Q8_0>(W, ws, Y, M, N, K, partial, p, s, la)));
     return GGUF_ERR_DTYPE;
   }
   if (type == T_Q5_K) {
-    GGUF_DISPATCH_DTYPE(dtype, return (rows16_direct_typed<scalar_t, DIRECT_Q5_K>(W, ws, Y, M, N, K, partial, p, s, la, gemv_sums)));
+    GGUF_DISPATCH_DTYPE(dtype, return (rows16_direct_typed<scalar_t, DIRECT_Q5_K>(W, ws, Y, M, N, K, partial, p, s, la)));
     return GGUF_ERR_DTYPE;
   }
-  GGUF_DISPATCH_DTYPE(dtype, return (rows16_direct_typed<scalar_t, DIRECT_Q4_K>(W, ws, Y, M, N, K, partial, p, s, la, gemv_sums)));
+  GGUF_DISPATCH_DTYPE(dtype, return (rows16_direct_typed<scalar_t, DIRECT_Q4_K>(W, ws, Y, M, N, K, partial, p, s, la)));
   return GGUF_ERR_DTYPE;
 }
 

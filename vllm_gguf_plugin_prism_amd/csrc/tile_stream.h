@@ -27,6 +27,7 @@ struct TsCall {
   int64_t w_pitch, ldy;
   const void* bias;
   bool gemv_sums;              // offset term on d * sum(q) instead of the stored sums
+  bool gemv;                   // the GEMV operator's arithmetic (Q5_0: see TQ5_0)
   MoeArgs moe;
   int row_blocks;              // tiles of 16 rt rows (dense) or blocks of slots
   double live_blocks;          // how many of them hold pairs, estimated (dense: all)
@@ -35,7 +36,8 @@ struct TsCall {
 
 // tile_stream.hip: whether a call is taken -- a dense product of M rows, a layer with this many (token, expert) pairs, an
 // expert GEMM on blocks of 16 slots by itself
-bool ts_dense_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch);
+bool ts_dense_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, bool gemv = false);   // gemv: in place of the GEMV
+int ts_dense(int type, const void* W, const void* x, int dtype, void* workspace, void* Y, int64_t M, int N, int K, bool gemv, const LinearArgs& la, hipStream_t s);
 bool ts_layer_takes(int type13, int type2, int64_t H, int64_t I, int64_t N_out, int64_t tokens, int64_t top_k, int64_t num_experts);
 bool ts_moe_takes(int type, int64_t N, int64_t K, int64_t num_sorted, int64_t tokens, int64_t top_k);
 int ts_any(int type, const TsCall& c, hipStream_t s);   // GGUF_NOT_TAKEN for other types

@@ -8,6 +8,13 @@ int ts_q8_0(const TsCall& c, hipStream_t s);
 int ts_q4_k(const TsCall& c, hipStream_t s);
 int ts_q5_k(const TsCall& c, hipStream_t s);
 int ts_q6_k(const TsCall& c, hipStream_t s);
+int ts_q2_k(const TsCall& c, hipStream_t s);
+int ts_q3_k(const TsCall& c, hipStream_t s);
+int ts_q4_1(const TsCall& c, hipStream_t s);
+int ts_q5_0(const TsCall& c, hipStream_t s);
+int ts_q5_1(const TsCall& c, hipStream_t s);
+int ts_iq4_nl(const TsCall& c, hipStream_t s);
+int ts_iq4_xs(const TsCall& c, hipStream_t s);
 
 static bool ts_type_ok(int type) {
   switch (type) {
@@ -46,9 +53,46 @@ static double ts_others_us(int type, int M, int N, int K) {
   return (type == T_Q4_K ? 4.2 : 4.7) + 1e-3 * ((type == T_Q4_K ? 0.26 : 0.41) * N + 0.15 * (M + 0.5) * K) + 0.11e-6 * N * K;
 }
 
+// Five to eight rows of the types whose GEMV is the other kernel: its time hardly depends on the type (13 % off over 2300 calls of
+// 512 .. 28672 columns and K 512 .. 18944), this kernel's is as above, with `cut` per panel where rows do not begin on 16 bytes and
+// fields are cut out of two reads (right to 3 .. 5 %).
+static bool ts_passes_gemv(int type, int M, int N, int K, bool aligned) {
+  struct Cost { int type; double base, round, panel, weights, k, cut; };
+  static const Cost costs[] = {{T_Q4_0, -1.5, 8.2, 1.01, 0.009, 0.32, 0.085}, {T_Q4_1, 0.3, 6.4, 1.12, 0.022, 0.38, 0.072}, {T_Q5_0, -2.1, 8.9, 1.18, 0.014, 0.36, 0.076},
+                               {T_Q5_1, 0.4, 6.4, 1.48, 0.028, 0.34, 0.075}, {T_Q8_0, -2.2, 9.0, 0.71, 0.051, 0.29, 0.078}, {T_IQ4_NL, 0.6, 6.1, 1.09, 0.026, 0.32, 0.071},
+                               {T_IQ4_XS, -2.0, 8.5, 1.05, 0.015, 0.37, 0.0}};
+  for (const Cost& c : costs) {
+    if (c.type != type) continue;
+    const int np = (K + 255) / 256, groups = (N + 15) / 16, ks = ts_ks(np, groups);
+    const double rounds = ceil(ceil((double)groups * ks / TS_NW) / 256.0);
+    const double us = c.base + rounds * (c.round + c.panel * ((np + ks - 1) / ks)) + 1e-6 * c.weights * N * K + 1e-3 * c.k * K + (aligned ? 0.0 : c.cut * np);
+    return us < 0.93 * (4.1 + 1e-3 * (0.18 * N + (0.2 * M - 0.08) * K) + 1e-6 * (0.072 + 0.015 * M) * N * K);
+  }
+  return false;
+}
+
 // Where the kernel is the faster one.
-bool ts_dense_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch) {
-  if (M < 5 || M > 32 || !ts_type_ok(type) || !ts_size_ok(N, w_pitch, M, K)) return false;
+bool ts_dense_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, bool gemv) {
+  if (M < 5 || (M > 32 && !gemv) || N > 0x7FFFFFF0ll || K > 0x7FFFFFF0ll || M > 0x7FFFFFF0ll || !ts_size_ok(N, w_pitch, M < 512 ? M : 512, K)) return false;
+  const bool aligned = w_pitch % 16 == 0;
+  switch (type) {
+    // Against the staged 16-row kernels, or the GEMV: 1.2 to 1.7 times as fast at 5 rows, from 9 on Q2_K 1.9 to 2.4 times, Q3_K 1.3 to
+    // 1.6 ([4096,4096], 12 rows: Q2_K 26.3 / 10.6 us, Q3_K 15.8 / 10.9).
+    case T_Q2_K: case T_Q3_K: return true;
+    // 1.6 to 2.1 times from 9 rows on ([14336,4096] Q4_1 12 rows 41.1 / 18.3)
+    case T_Q4_1: case T_Q5_1: return M >= 9 || ts_passes_gemv(type, (int)M, (int)N, (int)K, aligned);
+    // (the staged kernel's decoding is the least here: 1.2 times, but 0.85 at 64M weights and more whose rows begin anywhere, and where
+    // a long K on few columns leaves most CUs without a workgroup: [736,6560] 20 rows 15.8 / 19.1)
+    case T_Q5_0: return M >= 9 ? (aligned || N * K < (64 << 20)) && (N > 1280 || K <= 5120) : ts_passes_gemv(type, (int)M, (int)N, (int)K, aligned);
+    // (more rows than the GEMV's are not multiplied in whole numbers) 1.6 times from 9 rows on, [4096,14336] IQ4_XS 16 rows 69.6 / 24
+    case T_IQ4_NL: case T_IQ4_XS: return gemv && (M >= 9 || ts_passes_gemv(type, (int)M, (int)N, (int)K, aligned));
+  }
+  if (!ts_type_ok(type)) return false;
+  // The GEMV operator: its time grows with the rows ([4096,14336] 6 rows, GEMV / this: Q4_K 32.7 / 19.0, Q6_K 41.2 / 23.2).  Q4_K and Q5_K,
+  // whose GEMV decodes little, stay there on small matrices ([2048,2048] 5 rows 6.5 / 7.9).
+  if (gemv && M >= 9) return true;
+  if (gemv && type >= T_Q4_K && type <= T_Q6_K) return type == T_Q6_K || N * K >= (8 << 20);
+  if (gemv || (M <= 6 && type <= T_Q8_0)) return ts_passes_gemv(type, (int)M, (int)N, (int)K, aligned);
   // [11008,4096] Q4_K 24 rows, this / the other kernel: 19.9 / 39.1, [5120,4096] 14.7 / 25.6, [28672,1024] 5 rows 10.3 / 19.9; but
   // [8192,3584] 12 rows 13.1 / 11.2, [1024,14336] 17.0 / 11.7, [4096,1024] 5 rows 7.6 / 5.7.
   if (type >= T_Q4_K && type <= T_Q6_K) return ts_us(type, (int)M, (int)N, (int)K) < ts_others_us(type, (int)M, (int)N, (int)K);
@@ -61,7 +105,6 @@ bool ts_dense_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch) 
   // 15.2 / 18.5; [4096,4096] 10.9 / 10.7; Q8_0 16.4 / 17.7, 11.6 / 10.8).
   // (rows that do not begin on 16 bytes are cut out of two reads each: [19504,6016] Q8_0, 8 rows: 38.6 / 33.6,
   // [12240,18112] Q4_0, 16 rows: 59 / 50; [6544,18144] Q8_0 40.5 / 49.9)
-  const bool aligned = w_pitch % 16 == 0;
   if (type == T_Q4_0 && !aligned && K >= 6000) return false;
   if (M <= 8) return M >= 7 && K >= (aligned ? 5120 : 12000);
   // Above: all, but for what the kernel that reads the packed Q4_0 blocks has done in one launch and a single round, K not
@@ -103,8 +146,37 @@ int ts_any(int type, const TsCall& c, hipStream_t s) {
     case T_Q4_K: return ts_q4_k(c, s);
     case T_Q5_K: return ts_q5_k(c, s);
     case T_Q6_K: return ts_q6_k(c, s);
+    case T_Q2_K: return ts_q2_k(c, s);
+    case T_Q3_K: return ts_q3_k(c, s);
+    case T_Q4_1: return ts_q4_1(c, s);
+    case T_Q5_0: return ts_q5_0(c, s);
+    case T_Q5_1: return ts_q5_1(c, s);
+    case T_IQ4_NL: return ts_iq4_nl(c, s);
+    case T_IQ4_XS: return ts_iq4_xs(c, s);
   }
   return GGUF_NOT_TAKEN;
+}
+
+int ts_dense(int type, const void* W, const void* x, int dtype, void* workspace, void* Y, int64_t M, int N, int K, bool gemv, const LinearArgs& la, hipStream_t s) {
+  int rc = quantize_q8_1(x, dtype, workspace, M, K, s, 0, nullptr, true);
+  if (rc != GGUF_OK) return rc;
+  TsCall c = {};
+  c.W = W; c.dtype = dtype; c.N = N; c.K = K;
+  c.rt = M <= 16 ? 1 : 2;
+  c.w_pitch = la.w_pitch; c.ldy = la.ldy; c.bias = la.bias;
+  c.gemv = gemv;
+  c.gemv_sums = gemv && (type == T_Q4_K || type == T_Q5_K);   // (the others' offset is on the stored sums there too)
+  constexpr int64_t STEP = 512;                             // rows per launch, 16 tiles: the kernel's quotients by reciprocal stay exact
+  for (int64_t m = 0; m < M; m += STEP) {
+    c.ws = (const char*)workspace + m * q8_row_bytes(K);
+    c.Y = (char*)Y + m * (la.ldy ? la.ldy : N) * (dtype == GGUF_DTYPE_F32 ? 4 : 2);
+    c.M = (int)(M - m < STEP ? M - m : STEP);
+    c.row_blocks = (c.M + 16 * c.rt - 1) / (16 * c.rt);
+    c.live_blocks = c.row_blocks;
+    rc = ts_any(type, c, s);
+    if (rc != GGUF_OK) return rc == GGUF_NOT_TAKEN ? GGUF_ERR_LAUNCH : rc;   // (part of Y may be written: nobody else takes over)
+  }
+  return GGUF_OK;
 }
 
 int ts_moe(const void* W, const void* ws, void* Y, int dtype, int type, int N, int K, int num_sorted, const MoeArgs& moe, hipStream_t s,

@@ -78,6 +78,8 @@ template <int XR> __host__ __device__ __forceinline__ constexpr int ts_scale_at(
 // GATE: the first expert GEMM of a layer with its seam (Gate16): of four neighbouring column groups two are 32 features of
 // the gate half and two the same features of the up half; the sums meet in LDS and the workgroup finishes the q8_1
 // blocks of h from them.
+template <class F> constexpr bool ts_sums() { return F::OFF == 1 || F::HALVES; }   // the activations' block sums are wanted
+
 template <class F, int RT, bool GATE, bool SPLIT, int D>
 __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_stream_kernel(const uint8_t* __restrict__ W, const char* __restrict__ ws,
                                                                                   void* __restrict__ Y, TsArgs a, MoeArgs moe, Gate16 gate,
@@ -85,6 +87,7 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
   static_assert(!GATE || (RT == 1 && !SPLIT), "a gated product takes its column groups whole, for 16 slots");
   static_assert(D >= 2 && D <= 4, "one wait per number of panels requested behind the one at hand");
   constexpr int NW = TS_NW, XR = 16 * RT, XR_LOG2 = RT == 1 ? 4 : 5;
+  constexpr bool SUMS = ts_sums<F>(), OFFSET = F::OFF == 1;
   constexpr int PPR_MIN = (F::PB + 15) / 16, PPR_MAX = (F::PB + 29) / 16;     // pieces of an aligned / of any panel row
   constexpr int NI = (16 * (PPR_MAX | 1) + 63) / 64, FULL = 16 * PPR_MIN / 64;      // fetch instructions; those with all lanes on
   extern __shared__ __align__(16) char smem[];
@@ -111,7 +114,7 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
 
   // ---- LDS: [chunk buffers: quants [XR][pitch], scales and sums [blocks][XR]][fetch rings]; partial tiles over the chunks
   const int PC = 1 << a.pc_log2, pitch = 256 * PC + 16;
-  const int xq_bytes = XR * pitch, xs_bytes = ts_scale_at<XR>(8 * PC) * 4 * (F::OFF ? 2 : 1), buf_bytes = xq_bytes + xs_bytes;
+  const int xq_bytes = XR * pitch, xs_bytes = ts_scale_at<XR>(8 * PC) * 4 * (SUMS ? 2 : 1), buf_bytes = xq_bytes + xs_bytes;
   const int slot_bytes = 256 * a.ppr;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
   const int ring_off = a.nbuf * buf_bytes + wave * (D * slot_bytes);
@@ -191,7 +194,7 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
   };
   constexpr int NS = 2;                                     // (row, four blocks, plane) items per thread, at most
   u32x4_s sreg[NS];
-  const int items = (XR * 2 * PC) * (F::OFF ? 2 : 1);       // items, rows fastest
+  const int items = (XR * 2 * PC) * (SUMS ? 2 : 1);       // items, rows fastest
   const auto scales_at = [&](int ch, int i) -> uint32_t {
     const int it = tid + 64 * NW * i, row = it & (XR - 1), q = (it >> XR_LOG2) & (2 * PC - 1), plane = it >> (XR_LOG2 + 1 + a.pc_log2);
     return __shfl(row_at, row) + a.Kp + (plane ? 4 * a.plane * nb : 0) + min(16 * (uint32_t)(2 * PC * ch + q), 4 * (uint32_t)nb - 16);
@@ -300,7 +303,7 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
       for (int rt = 0; rt < RT; ++rt) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) xa[rt][i] = *(const u32x4_s*)(xq + (16 * rt + c) * pitch + 256 * pl + 64 * i + 16 * g);
-        if constexpr (F::OFF) {
+        if constexpr (OFFSET) {
           const float* const sums = xd + ts_scale_at<XR>(8 * PC) + ts_scale_at<XR>(8 * pl) + g * XR + 16 * rt + c;
           so[rt][0] = sums[0];
           so[rt][1] = sums[ts_scale_at<XR>(4)];
@@ -324,16 +327,21 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
 
       float dw[8 * (32 / F::G)];
       w.ready();
-      w.scales(dw);
+      uint32_t dm[8];
+      if constexpr (F::HALVES) w.words(dm);
+      else w.scales(dw);
       // (opaque to the compiler, which would keep both masked copies of all operands over the column groups and spill)
       uint32_t first = half0;
       asm volatile("" : "+v"(first));
       if (!F::KQ && left < 8) {
 #pragma unroll
-        for (int b = 0; b < 8; ++b) dw[b] = b < left ? dw[b] : 0.0f;   // (bytes behind the row's end need not be a number)
+        for (int b = 0; b < 8; ++b) {                       // (bytes behind the row's end need not be a number)
+          if constexpr (F::HALVES) dm[b] = b < left ? dm[b] : 0u;
+          else dw[b] = b < left ? dw[b] : 0.0f;
+        }
       }
       float m0 = 0.0f, m1 = 0.0f;
-      if constexpr (F::OFF) {
+      if constexpr (OFFSET) {
         w.mins(g, m0, m1);
         if (!F::KQ && left < 8) { m0 = g < left ? m0 : 0.0f; m1 = 4 + g < left ? m1 : 0.0f; }
       }
@@ -341,10 +349,10 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
       f32x4 part[RT];
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
-        part[rt] = F::OFF ? __builtin_amdgcn_mfma_f32_16x16x4f32(so[rt][0], -m0, (f32x4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0) : acc[rt];
+        part[rt] = OFFSET ? __builtin_amdgcn_mfma_f32_16x16x4f32(so[rt][0], -m0, (f32x4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0) : acc[rt];
 #pragma unroll
       for (int b = 0; b < 8; ++b) {
-        if (F::OFF && b == 4) {
+        if (OFFSET && b == 4) {
 #pragma unroll
           for (int rt = 0; rt < RT; ++rt) part[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(so[rt][1], -m1, part[rt], 0, 0, 0);
         }
@@ -354,11 +362,29 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
         for (int rt = 0; rt < RT; ++rt) {
           const f32x4 d8 = *(const f32x4*)(xd + ts_scale_at<XR>(8 * pl) + ts_scale_at<XR>(b) + 16 * rt + 4 * g);
           const uint32_t alo = xa[rt][b >> 1][2 * (b & 1)], ahi = xa[rt][b >> 1][2 * (b & 1) + 1];
-          if constexpr (F::G == 32) {
+          if constexpr (F::HALVES) {
+            typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+            const f32x4 s8 = *(const f32x4*)(xd + ts_scale_at<XR>(8 * PC) + ts_scale_at<XR>(8 * pl) + ts_scale_at<XR>(b) + 16 * rt + 4 * g);
+            const h2 v = __builtin_bit_cast(h2, dm[b]), dv = {v[0], v[0]}, mv = {v[1], v[1]};
+            const v4i s = __builtin_amdgcn_mfma_i32_16x16x32_i8((long)(((uint64_t)ahi << 32) | alo), bv, seed, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; r += 2) {                // (d8 and s8 are halves in fp32)
+              const h2 dd = (h2){(_Float16)d8[r], (_Float16)d8[r + 1]} * dv, ms = (h2){(_Float16)s8[r], (_Float16)s8[r + 1]} * mv;
+#pragma unroll
+              for (int e = 0; e < 2; ++e) part[rt][r + e] += __builtin_fmaf(seeded_times(s[r + e], 1.0f, -kSeed), (float)dd[e], (float)ms[e]);
+            }
+          } else if constexpr (F::G == 32) {
             const float nsd = -kSeed * dw[b];
             const v4i s = __builtin_amdgcn_mfma_i32_16x16x32_i8((long)(((uint64_t)ahi << 32) | alo), bv, seed, 0, 0, 0);
 #pragma unroll
             for (int r = 0; r < 4; ++r) part[rt][r] = __builtin_fmaf(seeded_times(s[r], dw[b], nsd), d8[r], part[rt][r]);
+            if constexpr (F::OFF == 2) {
+              const uint2 mq = w.min_codes(b);
+              const float dmin = w.dmin();
+              const v4i sm = __builtin_amdgcn_mfma_i32_16x16x32_i8((long)(((uint64_t)ahi << 32) | alo), (long)(((uint64_t)mq.y << 32) | mq.x), seed, 0, 0, 0);
+#pragma unroll
+              for (int r = 0; r < 4; ++r) part[rt][r] = __builtin_fmaf(seeded_times(sm[r], -dmin, kSeed * dmin), d8[r], part[rt][r]);
+            }
           } else {
             // a scale per 16 values: the activations of either half of the block, the other half's lanes zeroed
             const long a0 = (long)(((uint64_t)(ahi & first) << 32) | (alo & first));
@@ -375,7 +401,7 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
         }
       }
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt) acc[rt] = F::OFF ? acc[rt] + part[rt] : part[rt];
+      for (int rt = 0; rt < RT; ++rt) acc[rt] = OFFSET ? acc[rt] + part[rt] : part[rt];
     }
     // ---- the next chunk of activations
     if constexpr (SPLIT) {
@@ -516,7 +542,7 @@ static int ts_launch(const TsCall& c, int ks, hipStream_t stream) {
   const bool aligned = F::PB % 16 == 0 && pitch % 16 == 0 && (uintptr_t)c.W % 16 == 0 && (!c.moe.sorted_token_ids || c.moe.expert_stride % 16 == 0);
   // (an odd number, so that the same field of 16 rows lies in different banks: [23376,1856] of Q4_0, 16 rows of X 23.2 -> 19.2 us)
   const int ppr = (aligned ? F::PB / 16 : (F::PB + 29) / 16) | 1, top_k = c.moe.top_k > 0 ? c.moe.top_k : 1;
-  const auto bytes = [&](int pc, int nbuf, int d) { return nbuf * ts_chunk_bytes(RT, F::OFF, pc) + (size_t)TS_NW * d * 256 * ppr + 16; };
+  const auto bytes = [&](int pc, int nbuf, int d) { return nbuf * ts_chunk_bytes(RT, ts_sums<F>(), pc) + (size_t)TS_NW * d * 256 * ppr + 16; };
   const size_t room = 160 * 1024;
   int pc_log2 = 2, nbuf = 1;
   while (pc_log2 < 4 && (1 << pc_log2) < np) ++pc_log2;
@@ -533,7 +559,7 @@ static int ts_launch(const TsCall& c, int ks, hipStream_t stream) {
       while (pc_log2 > 2 && bytes(1 << pc_log2, 1, 2) > room) --pc_log2;
     }
   }
-  if ((1 << pc_log2) * 2 * 16 * RT * (F::OFF ? 2 : 1) > 2 * 64 * TS_NW) return GGUF_NOT_TAKEN;   // (two items of scales per thread)
+  if ((1 << pc_log2) * 2 * 16 * RT * (ts_sums<F>() ? 2 : 1) > 2 * 64 * TS_NW) return GGUF_NOT_TAKEN;   // (two items of scales per thread)
   // (two workgroups per CU overlap their beginnings and ends, and have as many panels in flight between them)
   int d = RT == 1 && bytes(1 << pc_log2, nbuf, 2) <= room / 2 ? 2 : 4;
   while (d > 2 && bytes(1 << pc_log2, nbuf, d) > room) --d;
@@ -555,11 +581,6 @@ static int ts_launch(const TsCall& c, int ks, hipStream_t stream) {
 template <class F, int RT>
 static int ts_run_rt(const TsCall& c, hipStream_t stream) {
   const int np = (c.K + 255) / 256;
-  if (RT != 1 && c.moe.sorted_token_ids) return GGUF_NOT_TAKEN;
-  if (c.gate.rows) {
-    if constexpr (RT == 1) return ts_launch<F, 1, true, false>(c, 1, stream);
-    return GGUF_NOT_TAKEN;
-  }
   const int ks = ts_ks(np, c.live_blocks * ((c.N + 15) / 16));
   if (ks == 1 && np <= 16) {
     const int rc = ts_launch<F, RT, false, false>(c, 1, stream);
@@ -569,8 +590,16 @@ static int ts_run_rt(const TsCall& c, hipStream_t stream) {
 }
 
 template <class F>
-static int ts_run(const TsCall& c, hipStream_t stream) {
+static int ts_dense_run(const TsCall& c, hipStream_t stream) {
+  if (c.moe.sorted_token_ids || c.gate.rows) return GGUF_NOT_TAKEN;
   return c.rt == 1 ? ts_run_rt<F, 1>(c, stream) : c.rt == 2 ? ts_run_rt<F, 2>(c, stream) : GGUF_NOT_TAKEN;
+}
+
+template <class F>
+static int ts_run(const TsCall& c, hipStream_t stream) {
+  if (!c.moe.sorted_token_ids) return ts_dense_run<F>(c, stream);
+  if (c.rt != 1) return GGUF_NOT_TAKEN;
+  return c.gate.rows ? ts_launch<F, 1, true, false>(c, 1, stream) : ts_run_rt<F, 1>(c, stream);
 }
 
 }  // namespace gguf
