@@ -735,7 +735,7 @@ int moe_tiles_layer(const void* X, int xdtype, void* workspace, const void* W13,
     const MoeArgs m2 = {sorted, experts, post, (int64_t)N_out * (I / block_elems(type2)) * block_bytes(type2), 1, pairs, gemv_sums(type2)};
     rc = ts_moe(W2, q8h, y2, xdtype, type2, N_out, I, ns, m2, s);
     if (rc != GGUF_OK) return rc;
-    return moe_weighted_sum_live(y2, topk_w, vec_sums ? nullptr : topk_ids, num_experts, out, xdtype, tokens, top_k, N_out, s);
+    return moe_weighted_sum_live(y2, topk_w, topk_ids, num_experts, out, xdtype, tokens, top_k, N_out, s);
   }
   rc = block == 16 ? moe_tiles16_gate(W13, q8x, q8h, xdtype, type13, I, H, ns, m1, act, s)
                    : moe_tiles32_gate(W13, q8x, q8h, xdtype, type13, I, H, ns, m1, act, s);
@@ -744,9 +744,9 @@ int moe_tiles_layer(const void* X, int xdtype, void* workspace, const void* W13,
   const MoeArgs m2 = {sorted, experts, post, (int64_t)N_out * (I / block_elems(type2)) * block_bytes(type2), 1, pairs, gemv_sums(type2)};
   rc = block == 16 ? moe_tiles16(W2, q8h, y2, xdtype, type2, N_out, I, ns, m2, s) : moe_tiles32(W2, q8h, y2, xdtype, type2, N_out, I, ns, m2, s);
   if (rc != GGUF_OK) return rc == GGUF_NOT_TAKEN ? GGUF_ERR_TYPE : rc;
-  // the grouped operator leaves the rows of pairs whose expert id names no expert at zero (the sort drops them): the
-  // sum takes them as zero instead of reading rows of y2 that nobody wrote
-  return moe_weighted_sum_live(y2, topk_w, vec_sums ? nullptr : topk_ids, num_experts, out, xdtype, tokens, top_k, N_out, s);
+  // a pair whose expert id names no expert adds nothing (the sort drops it): the sum takes its row as zero instead of reading
+  // one of y2 that nobody wrote
+  return moe_weighted_sum_live(y2, topk_w, topk_ids, num_experts, out, xdtype, tokens, top_k, N_out, s);
 }
 
 // ---- A MoE layer whose experts see more than a few pairs each, on the wide tile kernel (blocks of 32 or 64 slots): the same four

@@ -21,6 +21,7 @@
 // Where experts are shared by a few pairs each (the per-pair operator's tile route on blocks of 16 slots) the same entry
 // point runs the layer in four launches on the tile kernels instead (mmq.hip, moe_tiles_layer).
 #include "dense_api.h"
+#include "tile_stream.h"
 #include "tile_wide.h"
 #include "mmvq_core.h"
 
@@ -284,13 +285,16 @@ static MoeUpPlan moe_up_plan(int H, int I, int pairs) {
   p.rows = row_split(H);
   if (!p.rows.ok || I <= 0 || I % 32 != 0 || pairs <= 0 || pairs > 65535) return p;
   if ((int64_t)(H / F::QK) * F::BS > (int64_t)UINT32_MAX) return p;
-  const int64_t cus = num_cus();
-  int64_t best = INT64_MAX;
-  for (int R = 32; R <= I && R <= 4096; R += 32) {
-    const int bands = (I + R - 1) / R;
-    const int64_t rounds = ((int64_t)bands * pairs + cus - 1) / cus;
-    const int64_t cost = rounds * ((2 * R + p.rows.slots - 1) / p.rows.slots + 16);
-    if (cost < best) { best = cost; p.R = R; p.bands = bands; }
+  // (A layer asks for its plans three times, twice for whether it is served: every width and 64-bit quotients took 3 us a time, 9 of
+  //  the 12 us that a call of one token took the host.  Of the widths with as many bands the narrowest is the cheapest.)
+  const uint32_t cus = (uint32_t)num_cus(), groups = (uint32_t)I / 32;
+  uint64_t best = UINT64_MAX;
+  for (uint32_t g = 1; g <= groups && g <= 128;) {          // R / 32
+    const uint32_t bands = (groups + g - 1) / g, wgs = bands * (uint32_t)pairs;   // (below 2^31: I is, pairs 65535 at most, so is bands)
+    const uint64_t cost = (uint64_t)((wgs + cus - 1) / cus) * ((64 * g + p.rows.slots - 1) / (uint32_t)p.rows.slots + 16);
+    if (cost < best) { best = cost; p.R = (int)(32 * g); p.bands = (int)bands; }
+    if (wgs <= cus || bands == 1) break;                    // (one round: wider bands only take longer)
+    g = (groups + bands - 2) / (bands - 1);                 // the narrowest with fewer bands
   }
   const int G = (p.rows.half ? 2 : 4) * p.rows.S;
   p.lds = (size_t)H + (size_t)(H / 32) * 4 * (F::AUX != AUX_NONE ? 2 : 1) + F::TABLE_BYTES + (size_t)2 * p.R * G * 4 + (size_t)p.R * 4;
@@ -313,16 +317,22 @@ static MoeSumPlan moe_sum_plan(int N, int K, int top_k, int tokens) {
   p.slots = p.rows.slots / top_k;
   if (p.slots < 1) return p;
   if ((int64_t)(K / F::QK) * F::BS > (int64_t)UINT32_MAX) return p;
-  const int64_t cus = num_cus();
-  const int max_bands = (int)std::max<int64_t>(64, (cus + tokens - 1) / tokens);
-  int64_t best = INT64_MAX;
+  const uint32_t cus = (uint32_t)num_cus(), n = (uint32_t)N, slots = (uint32_t)p.slots;
+  const uint32_t max_bands = std::max<uint32_t>(64, (cus + tokens - 1) / tokens);
+  uint64_t best = UINT64_MAX;
   p.rows_per_wg = N;
-  for (int b = 1; b <= max_bands; ++b) {
-    const int rows = (N + b - 1) / b;
-    if (rows < p.slots && b > 1) break;
-    const int64_t wgs = (int64_t)((N + rows - 1) / rows) * tokens, rounds = (wgs + cus - 1) / cus;
-    const int64_t cost = rounds * ((rows + p.slots - 1) / p.slots + 16);
-    if (cost < best) { best = cost; p.rows_per_wg = rows; }
+  // (as many bands as make one round have the fewest turns of those that do: it begins at the fewest bands with as many)
+  const uint32_t one = std::max<uint32_t>(1, cus / tokens), first = ((n + one - 1) / one + slots - 1) / slots * slots;
+  uint32_t b = (n + first - 1) / first;
+  if (b > 1 && (n + b - 1) / b < slots) b = (n + 2 * slots - 1) / (2 * slots);   // (bands of fewer rows than a turn takes are none)
+  while (b <= max_bands) {
+    const uint32_t rows = (n + b - 1) / b;
+    if (rows < slots && b > 1) break;
+    const uint32_t wgs = (n + rows - 1) / rows * (uint32_t)tokens, turns = (rows + slots - 1) / slots;   // (at most 256 bands of 65535 tokens)
+    const uint64_t cost = (uint64_t)((wgs + cus - 1) / cus) * (turns + 16);
+    if (cost < best) { best = cost; p.rows_per_wg = (int)rows; }
+    if (turns == 1) break;
+    b = std::max(b + 1, (n + (turns - 1) * slots - 1) / ((turns - 1) * slots));   // the fewest bands with fewer turns
   }
   p.grid = (N + p.rows_per_wg - 1) / p.rows_per_wg;
   p.lds = ((F::TABLE_BYTES + 15) & ~(size_t)15) + (size_t)top_k * p.rows_per_wg * (p.rows.half ? 2 : 4) * p.rows.S * 4;
@@ -402,7 +412,10 @@ static int moe_layer_takes(int type13, int type2, int H, int I, int N_out, int t
   const int64_t pairs = (int64_t)tokens * top_k;
   const bool shared13 = num_experts > 0 && moe_share_pays(pairs, num_experts, (int64_t)2 * I * (H / qk13) * block_bytes(type13));
   const bool shared2 = num_experts > 0 && moe_share_pays(pairs, num_experts, (int64_t)N_out * (I / qk2) * block_bytes(type2));
-  if (shared13 || shared2) {
+  // Both say it by pairs per expert alone.  Where the streaming tiles are estimated, the estimates overrule them by more than 12 %
+  // (2000 layers of 0.5 .. 4 pairs per expert: 2.8 % faster on average, 183 by more than 5 %, 10 slower by more than that).
+  const double gain = 2 * pairs >= num_experts && pairs <= 4 * num_experts ? ts_layer_gain(type13, type2, H, I, N_out, tokens, top_k, num_experts) : 0.0;
+  if (gain > 0.0 ? gain > (shared13 || shared2 ? 0.89 : 1.12) : shared13 || shared2) {
     // (where only one of the two says so -- the thresholds differ by half a pair per expert between experts that fit the
     //  last-level cache together and experts that do not -- the other is near its own break-even: both go to the tiles)
     const int block = moe_tiles_layer_block(type13, type2, pairs, num_experts, I, true);

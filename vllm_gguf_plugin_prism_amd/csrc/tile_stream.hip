@@ -139,6 +139,26 @@ bool ts_layer_takes(int type13, int type2, int64_t H, int64_t I, int64_t N_out, 
   return pairs <= most * num_experts;
 }
 
+// How many times as long a layer with a few pairs per expert takes on the kernels that take pair by pair, by two estimates; 0 where
+// it does not run here.  Pair by pair costs every pair's products with its expert's weights, and the weights of the
+// experts that are hit once from memory; the tiles cost the experts' weights and decoding once, and rounds of workgroups.
+// us, M weights, MB; fitted to 2000 layers of 8 .. 128 experts with 0.5 .. 4 pairs each and right to 13 and 12 %.  [gate|up] 128 x 1536 x 2048, Q4_K and Q6_K down, 24
+// tokens of 8 pairs 109 us pair by pair, 79 here; 32 x 2048 x 1536 Q8_0 12 tokens of 4 pairs 36, 41.
+double ts_layer_gain(int type13, int type2, int64_t H, int64_t I, int64_t N_out, int64_t tokens, int64_t top_k, int64_t num_experts) {
+  if (num_experts <= 0 || num_experts > 256 || !ts_type_ok(type13) || !ts_type_ok(type2) || !ts_layer_takes(type13, type2, H, I, N_out, tokens, top_k, num_experts)) return 0.0;
+  struct Cost { int type; double pair, tile; };
+  static const Cost costs[] = {{T_Q4_0, 0.0685, 0.050}, {T_Q8_0, 0.0992, 0.042}, {T_Q4_K, 0.0768, 0.024}, {T_Q5_K, 0.105, 0.062}, {T_Q6_K, 0.136, 0.117}};
+  const auto of = [&](int type) { int i = 0; while (costs[i].type != type) ++i; return costs[i]; };
+  const Cost c13 = of(type13), c2 = of(type2);
+  const double pairs = (double)(tokens * top_k), live = num_experts * (1.0 - exp(-pairs / num_experts)), w13 = 2e-6 * I * H, w2 = 1e-6 * N_out * I;
+  const double mb = live * (w13 / block_elems(type13) * block_bytes(type13) + w2 / block_elems(type2) * block_bytes(type2));
+  const double by_pair = 9.2 + pairs * (w13 * c13.pair + w2 * c2.pair) + 0.035 * mb;
+  const double rounds13 = live * (I / 64.0) / 512.0, rounds2 = live * (N_out / 128.0) / 512.0;
+  const double by_tile = 15.7 + live * (w13 * c13.tile + w2 * c2.tile) + 0.136 * mb + 0.65 * (rounds13 > 1.0 ? rounds13 : 1.0) * H / 256.0 +
+                         0.236 * (rounds2 > 1.0 ? rounds2 : 1.0) * I / 256.0;
+  return by_pair / by_tile;
+}
+
 int ts_any(int type, const TsCall& c, hipStream_t s) {
   switch (type) {
     case T_Q4_0: return ts_q4_0(c, s);
