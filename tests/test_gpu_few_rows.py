@@ -1,5 +1,5 @@
-"""Products of 5 to 32 rows on the streaming tile kernel (csrc/tile_stream_core.h) of the formats without a grouped layer on it,
-and the GEMV operator's rows there, at the edges of its tiles against the CPU oracle."""
+"""Products on the streaming tile kernel (csrc/tile_stream_core.h): 5 to 32 rows of the formats without a grouped layer on it, the
+GEMV operator's rows and more rows of small matrices, at the edges of its tiles against the CPU oracle."""
 import numpy as np
 import pytest
 import torch
@@ -42,6 +42,16 @@ def test_tiles(qtype, m, n, k, pad):
 def test_gemv_operator(qtype, m, n, k, pad):
     from vllm_gguf_plugin_prism_amd import ops
     check(ops.ggml_mul_mat_vec_a8, "mmvq", qtype, m, n, k, pad)
+
+
+# small matrices with more rows: tiles of 32 rows side by side, the last one in part
+@pytest.mark.parametrize("qtype", (o.Q4_0, o.Q8_0, o.Q4_K, o.Q5_K, o.Q6_K, *TILES))
+@pytest.mark.parametrize("m,n,k,pad", [(33, 1041, 256, 2), (97, 700, 1568, 0), (160, 260, 3072, 6), (512, 130, 768, 0)])
+def test_more_rows(qtype, m, n, k, pad):
+    from vllm_gguf_plugin_prism_amd import ops
+    block, size = o.QUANT_SIZES[qtype]
+    assert ops._mmq_unit(qtype, n, k // block * block, m, k // block * size + pad) & 8
+    check(ops.ggml_mul_mat_a8, "mmq", qtype, m, n, k, pad)
 
 
 # the largest codes and scales of either sign, so that no block sum leaves the range in which it is exact

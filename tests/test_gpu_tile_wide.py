@@ -16,15 +16,15 @@ ONES = (o.Q4_1, o.Q5_1)
 # several, a part that is longer than another; more tiles than a round of workgroups; rows of W a pitch apart that moves
 # them through the positions inside 16 bytes (whole 16 bytes where only those are taken)
 @pytest.mark.parametrize("qtype", DENSE)
-@pytest.mark.parametrize("m,n,k,pad", [(33, 4097, 256, 0), (64, 2052, 1536, 2), (33, 640, 2560, 0), (97, 1300, 768, 0), (160, 1030, 2304, 6),
-                                       (300, 2500, 512, 0), (64, 256, 8192, 0), (97, 25604, 256, 0)])
+@pytest.mark.parametrize("m,n,k,pad", [(513, 1025, 256, 0), (577, 1300, 768, 2), (33, 4101, 4096, 0), (513, 2052, 512, 6), (577, 256, 8192, 0),
+                                       (40, 8196, 2048, 0), (97, 25604, 256, 0)])
 def test_dense_edges(qtype, m, n, k, pad):
     check_dense(qtype, m, n, k, 8 * pad if qtype in ONES else pad)
 
 
 # the last panel has one block, four, seven; K in one part and in several; more rows than other types are taken with
-@pytest.mark.parametrize("qtype,m,n,k", [(o.Q4_1, 33, 640, 2176), (o.Q4_1, 97, 1300, 896), (o.Q5_1, 64, 2052, 1600), (o.Q5_1, 200, 256, 2496),
-                                         (o.Q4_1, 40, 300, 384), (o.Q2_K, 2100, 130, 256), (o.Q5_1, 2100, 130, 320)])
+@pytest.mark.parametrize("qtype,m,n,k", [(o.Q4_1, 545, 640, 2176), (o.Q4_1, 577, 1300, 896), (o.Q5_1, 513, 2052, 1600), (o.Q5_1, 577, 256, 2496),
+                                         (o.Q4_1, 521, 300, 384), (o.Q2_K, 2100, 130, 256), (o.Q5_1, 2100, 130, 320)])
 def test_last_panels(qtype, m, n, k):
     check_dense(qtype, m, n, k, 0)
 
@@ -37,13 +37,21 @@ def test_two_passes():
     check_dense(o.Q2_K, m, n, k, 0, np.r_[:3, 1020:1030, m - 30:m])
 
 
-def check_dense(qtype, m, n, k, pad, rows=np.s_[:]):
+# the half-precision unit where it is still the fastest: a row and a column over a tile, tiles cut into runs; whole rounds and a
+# shared rest (the oracle on rows of several tiles)
+@pytest.mark.parametrize("qtype", (o.Q4_K, o.Q5_K, o.Q6_K))
+@pytest.mark.parametrize("m,n,k,pad", [(511, 2177, 8192, 2), (700, 2176, 5120, 0)])
+def test_half_precision_unit_behind_them(qtype, m, n, k, pad):
+    check_dense(qtype, m, n, k, pad, np.r_[:3, 250:260, m - 30:m], 2)
+
+
+def check_dense(qtype, m, n, k, pad, rows=np.s_[:], unit=None):
     from vllm_gguf_plugin_prism_amd import ops
     rng = np.random.default_rng(n + m)
     w = o.make_weights(rng, qtype, n, k)
     wd = torch.zeros(n, w.shape[1] + pad, dtype=torch.uint8, device="cuda")[:, :w.shape[1]]
     wd.copy_(torch.from_numpy(w))
-    assert ops._mmq_unit(qtype, n, k, m, wd.stride(0)) >= 4
+    assert ops._mmq_unit(qtype, n, k, m, wd.stride(0)) & 4 if unit is None else ops._mmq_unit(qtype, n, k, m, wd.stride(0)) == unit
     x = rng.standard_normal((m, k)).astype(np.float32) + 0.3
     bias = rng.standard_normal(n).astype(np.float32)
     y = ops.ggml_mul_mat_a8(wd, torch.from_numpy(x).cuda(), qtype, n, bias=torch.from_numpy(bias).cuda())
@@ -55,7 +63,7 @@ def check_dense(qtype, m, n, k, pad, rows=np.s_[:]):
 def test_largest_sums_and_smallest_scales(qtype):
     from vllm_gguf_plugin_prism_amd import ops
     rng = np.random.default_rng(qtype)
-    n, k, m = 384, 512, 40
+    n, k, m = 384, 512, 520
     block, size = o.QUANT_SIZES[qtype]
     w = o.make_weights(rng, qtype, n, k).reshape(n, k // block, size)
     if qtype == o.Q6_K:

@@ -9,8 +9,9 @@
  *
  * gguf_mmq_layer_workspace_bytes: the workspace with which gguf_mmq_linear on GGUF_MMQ_AUTO runs at full speed for weights
  * of this type, at a 16-byte boundary.  (gguf_mmq_workspace_bytes_engine does not know the type.)  gguf_mmq_layer_route: the
- * kernel that a call with a workspace of this size runs where it is not on the wide tiles: 1 the streaming tile kernel, 2 the
- * half-precision unit's, 0 another.  gguf_mmq_layer_unit: the same, 4 more where it is.  gguf_moe_mmq_layer_wide: whether
+ * kernel that a call with a workspace of this size runs where it is neither on the wide tiles nor, with more than 32 rows, on the
+ * streaming ones: 1 the streaming tile kernel, 2 the half-precision unit's, 0 another.  gguf_mmq_layer_unit: the same, 4 more where
+ * it is on the wide tiles, 8 more on the streaming ones.  gguf_moe_mmq_layer_wide: whether
  * gguf_moe_mmq_layer with the workspace it asks for, at addresses divisible by 16, runs on them. */
 #pragma once
 #include <stdint.h>

@@ -899,13 +899,15 @@ extern "C" int64_t gguf_mmq_layer_workspace_bytes(int type, int64_t N, int64_t K
 
 extern "C" int gguf_mmq_layer_route(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes) {
   if (M <= 0 || N <= 0 || K <= 0 || M > 0x7FFFFFF0LL || N > 0x7FFFFFF0LL || K > 0x7FFFFFF0LL) return 0;
-  if (gguf::ts_dense_takes(type, M, N, K, w_row_pitch_bytes)) return 1;
+  if (M <= 32 && gguf::ts_dense_takes(type, M, N, K, w_row_pitch_bytes)) return 1;
   return gguf::mmqf_takes(type, M, N, K, w_row_pitch_bytes, workspace_bytes, mmq_rows_bytes(M, K, false)) ? 2 : 0;
 }
 
 extern "C" int gguf_mmq_layer_unit(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes) {
   const int route = gguf_mmq_layer_route(type, N, K, M, w_row_pitch_bytes, workspace_bytes);
-  return route != 1 && M > 0 && N > 0 && K > 0 && gguf::wide_dense_plan(type, M, N, K, w_row_pitch_bytes, workspace_bytes).rt ? route + 4 : route;
+  if (route == 1 || M <= 0 || N <= 0 || K <= 0) return route;
+  if (M > 32 && gguf::ts_dense_takes(type, M, N, K, w_row_pitch_bytes)) return route + 8;
+  return gguf::wide_dense_plan(type, M, N, K, w_row_pitch_bytes, workspace_bytes).rt ? route + 4 : route;
 }
 
 // room for either engine
@@ -961,7 +963,7 @@ int gguf::mmq_linear_impl(const void* W, int64_t w_row_pitch_bytes, const void* 
   if (workspace_bytes < M * (q8_row_bytes(K) + (engine == GGUF_MMQ_HALF ? 2 * q8_half_pitch(K) : 0))) return GGUF_ERR_WORKSPACE;
   const int64_t partial_room = workspace_bytes - rows_bytes;
   const bool tiles_at_5 = M <= 16 && rows16_direct_pays(type, (int)M, N, K, true) && rows16_direct_takes(W, w_row_pitch_bytes, type, (int)M, (int)N, (int)K, partial_room > 0 ? partial_room : 0);
-  if (engine != GGUF_MMQ_HALF && ts_dense_takes(type, M, N, K, w_row_pitch_bytes)) {
+  if (engine != GGUF_MMQ_HALF && (M <= 32 || engine == GGUF_MMQ_AUTO) && ts_dense_takes(type, M, N, K, w_row_pitch_bytes)) {
     return ts_dense(type, W, x, xdtype, q8_workspace, Y, M, (int)N, (int)K, false, la, s);
   }
   if (engine == GGUF_MMQ_AUTO && M <= 8 && !tiles_at_5) {

@@ -71,9 +71,26 @@ static bool ts_passes_gemv(int type, int M, int N, int K, bool aligned) {
   return false;
 }
 
+// More than 32 rows: every 32 of them read the weights again, which is nothing while the matrix is small and the tiles are few; the
+// kernels behind it share a sum over K between workgroups there, two launches more than this one.  How many M products of
+// rows (in whole tiles of 32) and weights, from 3000 calls of 33 .. 500 rows and up to 20M weights: below these 1.2 to 1.4 times as fast
+// on average (three in a hundred slower by more than 3 %), over all of them 1.08 (Q3_K) to 1.18 (Q8_0, Q5_0).
+static double ts_most_work(int type) {
+  switch (type) {
+    case T_Q8_0: return 28;
+    case T_Q4_0: return 24;
+    case T_Q4_K: case T_Q5_K: case T_Q6_K: case T_Q5_0: return 20;   // (Q5_0 at 32: [4880,640] 259 rows 15.5 / 21.3)
+    case T_Q4_1: return 16;
+    case T_Q5_1: return 14;
+    case T_Q2_K: case T_Q3_K: return 12;
+  }
+  return 0;
+}
+
 // Where the kernel is the faster one.
 bool ts_dense_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, bool gemv) {
-  if (M < 5 || (M > 32 && !gemv) || N > 0x7FFFFFF0ll || K > 0x7FFFFFF0ll || M > 0x7FFFFFF0ll || !ts_size_ok(N, w_pitch, M < 512 ? M : 512, K)) return false;
+  if (M < 5 || (M > 512 && !gemv) || N > 0x7FFFFFF0ll || K > 0x7FFFFFF0ll || M > 0x7FFFFFF0ll || !ts_size_ok(N, w_pitch, M < 512 ? M : 512, K)) return false;
+  if (M > 32 && !gemv) return 1e-6 * ((M + 31) / 32) * N * K < ts_most_work(type);
   const bool aligned = w_pitch % 16 == 0;
   switch (type) {
     // Against the staged 16-row kernels, or the GEMV: 1.2 to 1.7 times as fast at 5 rows, from 9 on Q2_K 1.9 to 2.4 times, Q3_K 1.3 to
