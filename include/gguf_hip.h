@@ -102,7 +102,8 @@ int gguf_mmq(const void* W, const void* x, int xdtype, void* q8_workspace, void*
  *                  Q6_K at some hundred rows, where that is faster with the room that workspace_bytes leaves for the
  *                  rows in half precision (gguf_mmq_workspace_bytes has it) and partial tiles, the same exact
  *                  whole-number products on half-precision MFMA: quants and scale-times-code operands are whole numbers that half precision
- *                  holds, their sums are whole numbers that fp32 holds.  This is what gguf_mmq runs.
+ *                  holds, their sums are whole numbers that fp32 holds (tiles of 32 or 64 rows, by the same estimates, also for
+ *                  Q4_0, Q4_1, Q5_1, Q2_K, Q3_K).  This is what gguf_mmq runs.
  * workspace_bytes is the size of q8_workspace; 0 stands for the minimum, M * gguf_q8_1_row_bytes(K).  Given
  * gguf_mmq_workspace_bytes(M, N, K) bytes, either engine splits K over several workgroups per output tile where the
  * output tiles alone would leave much of the chip idle (few tokens, a narrow N with a long K, a sparse last round of

@@ -1,4 +1,4 @@
-// Products with a few rows of activations (5 to 32), dense and per expert of an MoE layer, that run near the rate
+// Products with a few rows of activations (5 to 32; up to 512 of a small matrix), dense and per expert of an MoE layer, that run near the rate
 // the packed weights stream in.
 //
 // What bounds such a product is the weight stream; what keeps a kernel from it is everything around it: decoded weights
