@@ -963,9 +963,9 @@ int gguf::mmq_linear_impl(const void* W, int64_t w_row_pitch_bytes, const void* 
   if (workspace_bytes < M * (q8_row_bytes(K) + (engine == GGUF_MMQ_HALF ? 2 * q8_half_pitch(K) : 0))) return GGUF_ERR_WORKSPACE;
   const int64_t partial_room = workspace_bytes - rows_bytes;
   const bool tiles_at_5 = M <= 16 && rows16_direct_pays(type, (int)M, N, K, true) && rows16_direct_takes(W, w_row_pitch_bytes, type, (int)M, (int)N, (int)K, partial_room > 0 ? partial_room : 0);
-  if (engine != GGUF_MMQ_HALF && (M <= 32 || engine == GGUF_MMQ_AUTO) && ts_dense_takes(type, M, N, K, w_row_pitch_bytes)) {
+  // (it fetches the quantized rows in pieces of 16 bytes)
+  if (engine != GGUF_MMQ_HALF && (M <= 32 || engine == GGUF_MMQ_AUTO) && ((uintptr_t)q8_workspace & 15) == 0 && ts_dense_takes(type, M, N, K, w_row_pitch_bytes))
     return ts_dense(type, W, x, xdtype, q8_workspace, Y, M, (int)N, (int)K, false, la, s);
-  }
   if (engine == GGUF_MMQ_AUTO && M <= 8 && !tiles_at_5) {
     // a handful of rows: the streaming GEMV kernel with the tile kernels' offset sums reads W once at close to the
     // GEMV's rate and is exact in int8; it declines shapes it does not cover
