@@ -9,7 +9,7 @@ from oracle import gguf_oracle as o
 pytestmark = pytest.mark.gpu
 
 TILES = (o.Q2_K, o.Q3_K, o.Q4_1, o.Q5_0, o.Q5_1)
-GEMV = (o.Q4_0, o.Q8_0, o.Q4_K, o.Q5_K, o.Q6_K, *TILES, o.IQ4_NL, o.IQ4_XS)
+GEMV = (o.Q4_0, o.Q8_0, o.Q4_K, o.Q5_K, o.Q6_K, *TILES, o.IQ4_NL, o.IQ4_XS, o.IQ2_XXS, o.IQ2_XS, o.IQ2_S, o.IQ3_XXS, o.IQ3_S)
 
 
 # one tile of rows, full and in part, two, several (the GEMV operator takes any number), more than a launch's; a last column group of one, four, all columns; K in one panel and in several, one of

@@ -15,6 +15,11 @@ int ts_q5_0(const TsCall& c, hipStream_t s);
 int ts_q5_1(const TsCall& c, hipStream_t s);
 int ts_iq4_nl(const TsCall& c, hipStream_t s);
 int ts_iq4_xs(const TsCall& c, hipStream_t s);
+int ts_iq2_xxs(const TsCall& c, hipStream_t s);
+int ts_iq2_xs(const TsCall& c, hipStream_t s);
+int ts_iq2_s(const TsCall& c, hipStream_t s);
+int ts_iq3_xxs(const TsCall& c, hipStream_t s);
+int ts_iq3_s(const TsCall& c, hipStream_t s);
 
 static bool ts_type_ok(int type) {
   switch (type) {
@@ -102,6 +107,10 @@ bool ts_dense_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, 
     // a long K on few columns leaves most CUs without a workgroup: [736,6560] 20 rows 15.8 / 19.1)
     case T_Q5_0: return M >= 9 ? (aligned || N * K < (64 << 20)) && (N > 1280 || K <= 5120) : ts_passes_gemv(type, (int)M, (int)N, (int)K, aligned);
     // (more rows than the GEMV's are not multiplied in whole numbers) 1.6 times from 9 rows on, [4096,14336] IQ4_XS 16 rows 69.6 / 24
+    // (and 1.5 to 2.1 times with the grids' two or three lookups per eight weights, [4096,14336] IQ2_XXS 16 rows 68.8 / 21.1; fewer rows:
+    // 1.2 to 1.4 times where rows are long, 1.2 at 7 and 8 rows of 8M to 64M weights, where larger ones lose up to 18 %)
+    case T_IQ2_XXS: case T_IQ2_XS: case T_IQ2_S: case T_IQ3_XXS: case T_IQ3_S:
+      return gemv && (M >= 9 || (K >= 2 * N && N * K >= (16 << 20)) || (M >= 7 && N * K >= (8 << 20) && N * K < (64 << 20)));
     case T_IQ4_NL: case T_IQ4_XS: return gemv && (M >= 9 || ts_passes_gemv(type, (int)M, (int)N, (int)K, aligned));
   }
   if (!ts_type_ok(type)) return false;
@@ -190,6 +199,11 @@ int ts_any(int type, const TsCall& c, hipStream_t s) {
     case T_Q5_1: return ts_q5_1(c, s);
     case T_IQ4_NL: return ts_iq4_nl(c, s);
     case T_IQ4_XS: return ts_iq4_xs(c, s);
+    case T_IQ2_XXS: return ts_iq2_xxs(c, s);
+    case T_IQ2_XS: return ts_iq2_xs(c, s);
+    case T_IQ2_S: return ts_iq2_s(c, s);
+    case T_IQ3_XXS: return ts_iq3_xxs(c, s);
+    case T_IQ3_S: return ts_iq3_s(c, s);
   }
   return GGUF_NOT_TAKEN;
 }

@@ -32,6 +32,7 @@
 #include "q8_1_device.h"
 #include "tile_stream.h"
 #include "tile_stream_formats.h"
+#include <type_traits>
 
 namespace gguf {
 
@@ -78,6 +79,9 @@ template <int XR> __host__ __device__ __forceinline__ constexpr int ts_scale_at(
 // GATE: the first expert GEMM of a layer with its seam (Gate16): of four neighbouring column groups two are 32 features of
 // the gate half and two the same features of the up half; the sums meet in LDS and the workgroup finishes the q8_1
 // blocks of h from them.
+// bytes of LDS that a format's tables take (F::TABLE, filled by F::tables, read through the member tab), 0 for most
+template <class F, class = void> struct TsTable { static constexpr int value = 0; };
+template <class F> struct TsTable<F, std::void_t<decltype(F::TABLE)>> { static constexpr int value = (F::TABLE + 15) / 16 * 16; };
 template <class F> constexpr bool ts_sums() { return F::OFF == 1 || F::HALVES; }   // the activations' block sums are wanted
 
 template <class F, int RT, bool GATE, bool SPLIT, int D>
@@ -120,6 +124,7 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
   const int ring_off = a.nbuf * buf_bytes + wave * (D * slot_bytes);
 
   // ---- fetching weights: piece number -> (row of the panel, 16-byte piece of it)
+  const int table_off = a.nbuf * buf_bytes + NW * (D * slot_bytes) + 16;   // (a last field's cut may touch the word behind the rings)
   const uint32_t wmis = (uint32_t)((uintptr_t)W & 15);
   const uint8_t* const wbase = W - wmis;
   const uint32_t row_bytes = (uint32_t)(F::KQ ? a.np * F::PB : (a.K >> 5) * (F::PB / 8));
@@ -266,6 +271,7 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
     else ts_wait<0>();
   }
   place_first_scales();
+  if constexpr (TsTable<F>::value) F::tables(smem + table_off);
   __syncthreads();
 
   const v4i seed = {kSeedBits, kSeedBits, kSeedBits, kSeedBits};
@@ -319,6 +325,7 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
       uint32_t last;
       const uint32_t w_at = min(group_at(pass, last) + c * a.w_pitch, last) + (uint32_t)(p * F::PB) + wmis;
       F w;
+      if constexpr (TsTable<F>::value) w.tab = smem + table_off;
       w.read(smem + ring_off + slot * slot_bytes + c * (16 * a.ppr), F::PB % 16 == 0 && a.ppr == F::PB / 16 ? 0u : w_at & 15, g);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot may be filled again
       request_next(slot);
@@ -542,7 +549,7 @@ static int ts_launch(const TsCall& c, int ks, hipStream_t stream) {
   const bool aligned = F::PB % 16 == 0 && pitch % 16 == 0 && (uintptr_t)c.W % 16 == 0 && (!c.moe.sorted_token_ids || c.moe.expert_stride % 16 == 0);
   // (an odd number, so that the same field of 16 rows lies in different banks: [23376,1856] of Q4_0, 16 rows of X 23.2 -> 19.2 us)
   const int ppr = (aligned ? F::PB / 16 : (F::PB + 29) / 16) | 1, top_k = c.moe.top_k > 0 ? c.moe.top_k : 1;
-  const auto bytes = [&](int pc, int nbuf, int d) { return nbuf * ts_chunk_bytes(RT, ts_sums<F>(), pc) + (size_t)TS_NW * d * 256 * ppr + 16; };
+  const auto bytes = [&](int pc, int nbuf, int d) { return nbuf * ts_chunk_bytes(RT, ts_sums<F>(), pc) + (size_t)TS_NW * d * 256 * ppr + 16 + TsTable<F>::value; };
   const size_t room = 160 * 1024;
   int pc_log2 = 2, nbuf = 1;
   while (pc_log2 < 4 && (1 << pc_log2) < np) ++pc_log2;
