@@ -27,9 +27,15 @@
 // What bounds it now is vector issue beside the matrix unit, at a clock that falls to about 2.0 GHz under this load: by
 // counters ([4096,14336] Q4_K, 1531 rows) the vector ALU issues in 64 % of the SIMD cycles and the matrix unit is busy in
 // 32 %, Q6_K 52 % and 45 %.  The matrix instructions, the multiply-adds and the operand reads of a step take about 0.45 us
-// each; a step takes 1.2 us, a super-block, which is four steps and its end, 5.9 (Q6_K 8.0).  Tried and slower: four
-// waves per workgroup and two workgroups per CU (decoding twice), the two waves of a SIMD decoding at different times,
-// the fetches of X in front of the operand reads or spread over the step.
+// each; a step takes 1.2 us, a super-block, which is four steps and its end, 5.9 (Q6_K 8.0).  So what is left out counts, not
+// what is hidden: with decoding in 30 instead of 50 vector instructions per wave and step (masks and the 1024s as one
+// instruction, high nibbles left where they are), LDS addresses whose constants lie in the instructions (40 additions fewer per
+// super-block) and the contraction in front of the other wave's decoding the same product takes 299 -> 287 us, Q6_K 170 -> 168.  The
+// contraction alone, matrix instructions and multiply-adds in registers, takes a SIMD 50 to 56 ns per 32 x 32 x 32 block at any
+// interleaving (one wave or two, bursts of one to four blocks, 16 x 16 x 32 tiles): the clock falls as they get denser.
+// Tried and slower: four waves per workgroup and two workgroups per CU (decoding twice), the two waves of a SIMD decoding at
+// different times, the fetches of X in front of the operand reads or spread over the step; the barrier in the middle of a step
+// and the next step's operands behind it, so that no step begins with waiting (same bits, 299 -> 316 us, Q6_K 170 -> 190).
 #pragma once
 #include "mmq_formats.h"
 #include "mmq_f.h"
@@ -41,8 +47,21 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x2_m __attribute__((ext_vector_type(2)));
 
-// Two whole numbers below 1024 out of the low bytes (or nibbles) of the halves of v as 1024 + x each.
-__device__ __forceinline__ f16x2 magic2(uint32_t v) { return __builtin_bit_cast(f16x2, v | 0x64006400u); }
+// Whole numbers x below 1024 as the halves 1024 + x: the bits `mask` of both halves of v (`magic`, 0x64006400, in a vector register,
+// makes the two operations one instruction, which takes a single scalar operand); bytes 0 and 2, or 1 and 3, of v; the same
+// byte of v twice.
+__device__ __forceinline__ uint32_t in_register(uint32_t v) {
+  uint32_t r;
+  asm("v_mov_b32 %0, %1" : "=v"(r) : "s"(v));
+  return r;
+}
+__device__ __forceinline__ f16x2 magic_bits(uint32_t v, uint32_t mask, uint32_t magic) { return __builtin_bit_cast(f16x2, (v & mask) | magic); }
+template <int ODD> __device__ __forceinline__ f16x2 magic_bytes(uint32_t v) {
+  return __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, v, ODD ? 0x04030401u : 0x04020400u));
+}
+template <int AT> __device__ __forceinline__ f16x2 magic_twice(uint32_t v) {
+  return __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, v, 0x04000400u | AT << 16 | AT));
+}
 __device__ __forceinline__ uint32_t bits2(f16x2 v) { return __builtin_bit_cast(uint32_t, v); }
 __device__ __forceinline__ f16x2 twice(_Float16 v) { return (f16x2){v, v}; }
 
@@ -69,28 +88,25 @@ struct FQ4_K {
     uint32_t o[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      o[i] = bits2(magic2(__builtin_amdgcn_perm(0u, m[i >> 1], i & 1 ? 0x0c030c02u : 0x0c010c00u)) - k);
+      o[i] = bits2(__builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, m[i >> 1], i & 1 ? 0x04030402u : 0x04010400u)) - k);
     return make_uint4(o[0], o[1], o[2], o[3]);
   }
-  // the scales of blocks 2 j and 2 j + 1
-  template <int J> static __device__ __forceinline__ void pair(const Scales& sc, f16x2& s0, f16x2& s1) {
-    const uint32_t w = sc.s[J >> 1];
-    const f16x2 k = twice((_Float16)1024.0f);
-    s0 = magic2(__builtin_amdgcn_perm(0u, w, J & 1 ? 0x0c020c02u : 0x0c000c00u)) - k;
-    s1 = magic2(__builtin_amdgcn_perm(0u, w, J & 1 ? 0x0c030c03u : 0x0c010c01u)) - k;
-  }
+  // 1024 + the scale of block 2 J + B, twice
+  template <int J, int B> static __device__ __forceinline__ f16x2 scale(const Scales& sc) { return magic_twice<2 * (J & 1) + B>(sc.s[J >> 1]); }
+  // (high nibbles stay where they are, sixteen times as large, and their scale is a sixteenth: all exact)
   template <int J> static __device__ __forceinline__ void decode(const Raw& r, const Scales& sc, int, uint4 (&lo)[1], uint4 (&hi)[1]) {
-    f16x2 s0, s1;
-    pair<J>(sc, s0, s1);
+    const uint32_t magic = in_register(0x64006400u);
+    const f16x2 s0 = scale<J, 0>(sc) - twice((_Float16)1024.0f);
+    const f16x2 s1 = __builtin_elementwise_fma(scale<J, 1>(sc), twice((_Float16)0.0625f), twice((_Float16)-64.0f));
     const f16x2 k = twice((_Float16)-1024.0f), n0 = s0 * k, n1 = s1 * k;   // (exact: six bits times a power of two)
     uint32_t l[4], h[4];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const uint32_t a = i ? r.q.y : r.q.x, b = a >> 4;
-      l[2 * i] = bits2(__builtin_elementwise_fma(magic2(a & 0x000F000Fu), s0, n0));
-      l[2 * i + 1] = bits2(__builtin_elementwise_fma(magic2((a >> 8) & 0x000F000Fu), s0, n0));
-      h[2 * i] = bits2(__builtin_elementwise_fma(magic2(b & 0x000F000Fu), s1, n1));
-      h[2 * i + 1] = bits2(__builtin_elementwise_fma(magic2((b >> 8) & 0x000F000Fu), s1, n1));
+      const uint32_t a = i ? r.q.y : r.q.x, b = a >> 8;
+      l[2 * i] = bits2(__builtin_elementwise_fma(magic_bits(a, 0x000F000Fu, magic), s0, n0));
+      l[2 * i + 1] = bits2(__builtin_elementwise_fma(magic_bits(b, 0x000F000Fu, magic), s0, n0));
+      h[2 * i] = bits2(__builtin_elementwise_fma(magic_bits(a, 0x00F000F0u, magic), s1, n1));
+      h[2 * i + 1] = bits2(__builtin_elementwise_fma(magic_bits(b, 0x00F000F0u, magic), s1, n1));
     }
     lo[0] = make_uint4(l[0], l[1], l[2], l[3]);
     hi[0] = make_uint4(h[0], h[1], h[2], h[3]);
@@ -104,19 +120,17 @@ struct FQ5_K : FQ4_K {   // Q4_K with a fifth bit, bit b of qh[k] for block b
     return {ld<uint2>(sb + 48 + 32 * j + 8 * p), ld<uint2>(sb + 16 + 8 * p)};
   }
   template <int J> static __device__ __forceinline__ void decode(const Raw& r, const Scales& sc, int, uint4 (&lo)[1], uint4 (&hi)[1]) {
-    f16x2 s0, s1;
-    pair<J>(sc, s0, s1);
-    const f16x2 k = twice((_Float16)-1024.0f), n0 = s0 * k, n1 = s1 * k;
+    const f16x2 k = twice((_Float16)-1024.0f), s0 = scale<J, 0>(sc) + k, s1 = scale<J, 1>(sc) + k, n0 = s0 * k, n1 = s1 * k;
     uint32_t l[4], h[4];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const uint32_t a = i ? r.q.y : r.q.x, t = i ? r.h.y : r.h.x;
       const uint32_t a0 = (a & 0x0F0F0F0Fu) | (J < 2 ? (t << (4 - 2 * J)) & 0x10101010u : (t >> (2 * J - 4)) & 0x10101010u);
       const uint32_t a1 = ((a >> 4) & 0x0F0F0F0Fu) | (J < 2 ? (t << (3 - 2 * J)) & 0x10101010u : (t >> (2 * J - 3)) & 0x10101010u);
-      l[2 * i] = bits2(__builtin_elementwise_fma(magic2(a0 & 0x00FF00FFu), s0, n0));
-      l[2 * i + 1] = bits2(__builtin_elementwise_fma(magic2((a0 >> 8) & 0x00FF00FFu), s0, n0));
-      h[2 * i] = bits2(__builtin_elementwise_fma(magic2(a1 & 0x00FF00FFu), s1, n1));
-      h[2 * i + 1] = bits2(__builtin_elementwise_fma(magic2((a1 >> 8) & 0x00FF00FFu), s1, n1));
+      l[2 * i] = bits2(__builtin_elementwise_fma(magic_bytes<0>(a0), s0, n0));
+      l[2 * i + 1] = bits2(__builtin_elementwise_fma(magic_bytes<1>(a0), s0, n0));
+      h[2 * i] = bits2(__builtin_elementwise_fma(magic_bytes<0>(a1), s1, n1));
+      h[2 * i + 1] = bits2(__builtin_elementwise_fma(magic_bytes<1>(a1), s1, n1));
     }
     lo[0] = make_uint4(l[0], l[1], l[2], l[3]);
     hi[0] = make_uint4(h[0], h[1], h[2], h[3]);
@@ -141,7 +155,7 @@ struct FQ6_K {
   // four 6-bit codes -> (code - 32) * (sc & ~15) and (code - 32) * (sc & 15), whole numbers of 10 bits (times 16) and 9 bits
   static __device__ __forceinline__ void planes(uint32_t v, f16x2 sh, f16x2 sl, uint32_t& h0, uint32_t& h1, uint32_t& l0, uint32_t& l1) {
     const f16x2 k = twice((_Float16)1056.0f);
-    const f16x2 a = magic2(v & 0x00FF00FFu) - k, b = magic2((v >> 8) & 0x00FF00FFu) - k;
+    const f16x2 a = magic_bytes<0>(v) - k, b = magic_bytes<1>(v) - k;
     h0 = bits2(a * sh);
     h1 = bits2(b * sh);
     l0 = bits2(a * sl);
@@ -149,10 +163,12 @@ struct FQ6_K {
   }
   template <int J> static __device__ __forceinline__ void decode(const Raw& r, const Scales&, int p, uint4 (&lo)[2], uint4 (&hi)[2]) {
     // scales of the values of this part: group p / 2 of blocks 2 j and 2 j + 1
-    const uint32_t w = r.s;
-    const int c0 = (int)(int8_t)((w >> (8 * (p >> 1))) & 0xFF), c1 = (int)(int8_t)((w >> (16 + 8 * (p >> 1))) & 0xFF);
-    const f16x2 sh0 = twice((_Float16)(float)(c0 & ~15)), sl0 = twice((_Float16)(float)(c0 & 15));
-    const f16x2 sh1 = twice((_Float16)(float)(c1 & ~15)), sl1 = twice((_Float16)(float)(c1 & 15));
+    const uint32_t w = r.s >> (8 * (p >> 1));
+    // scale & 15 and, its sign bit flipped and taken off again, scale & ~15
+    const uint32_t c0 = bits2(magic_twice<0>(w)), c1 = bits2(magic_twice<2>(w));
+    const f16x2 k = twice((_Float16)1024.0f), kh = twice((_Float16)1152.0f);
+    const f16x2 sl0 = __builtin_bit_cast(f16x2, c0 & 0x640F640Fu) - k, sh0 = __builtin_bit_cast(f16x2, (c0 ^ 0x00800080u) & 0x64F064F0u) - kh;
+    const f16x2 sl1 = __builtin_bit_cast(f16x2, c1 & 0x640F640Fu) - k, sh1 = __builtin_bit_cast(f16x2, (c1 ^ 0x00800080u) & 0x64F064F0u) - kh;
     uint32_t a[2][4], b[2][4];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -197,6 +213,13 @@ __device__ __forceinline__ int afresh(int v) {
   asm volatile("" : "+v"(v));
   return v;
 }
+
+// LDS by byte numbers: what is constant in one goes into the instruction (from a pointer, a zero is added first).
+template <typename V> using lds_ptr = __attribute__((address_space(3))) V*;
+template <typename V> __device__ __forceinline__ V lds_get(uint32_t at) { return *(lds_ptr<const V>)(uintptr_t)at; }
+template <typename V> __device__ __forceinline__ void lds_put(uint32_t at, V v) { *(lds_ptr<V>)(uintptr_t)at = v; }
+typedef uint32_t u32x4_m __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ u32x4_m as_vector(const uint4& v) { return (u32x4_m){v.x, v.y, v.z, v.w}; }
 
 template <int J> struct StepIndex { static constexpr int value = J; };
 
@@ -247,6 +270,9 @@ __global__ __launch_bounds__(64 * MMQF_WM * MMQF_WN, 2) void mmqf_kernel(const u
   };
   // weights: a thread has one part of a row's step
   const int w_n = tid >> 2, part = tid & 3;
+  // (its two places in a buffer are pieces p and 4 + p, xored like the operands' pieces)
+  const auto w_place = [&](int id) { return lds0 + 128 * (M_T + (id >> 2)) + 16 * ((id & 3) ^ ((id >> 3) & 7)); };
+  const uint32_t w_to = w_place(tid);                       // (two planes leave no register for it)
   const uint32_t w_row = (uint32_t)min(n_base + w_n, a.r.N - 1) * (uint32_t)a.w_pitch;   // (the matrix is below 4 GB: mmqf_takes)
   typename F::Head hd;
   typename F::Scales sc;
@@ -255,26 +281,24 @@ __global__ __launch_bounds__(64 * MMQF_WM * MMQF_WN, 2) void mmqf_kernel(const u
   const auto fetch_head = [&](int sb) { hd = F::head(W + (w_row + (uint32_t)sb * F::BS)); };
   const auto stash_head = [&]() {
     const int id = afresh(tid), n = id >> 2;
-    char* const p = smem + PLANE_AT;
     if ((id & 3) == 0) {
-      *(float*)(p + 16 * M_T + 4 * n) = F::d(hd);
+      const uint32_t at = lds0 + PLANE_AT + 16 * M_T + 4 * n;
+      lds_put<float>(at, F::d(hd));
       if (F::OFF) {
-        *(float*)(p + 16 * M_T + 4 * N_T + 4 * n) = -F::dmin(hd);
-        *(uint4*)(p + 16 * M_T + 8 * N_T + 16 * n) = F::mins(hd);
+        lds_put<float>(at + 4 * N_T, -F::dmin(hd));
+        lds_put<u32x4_m>(at + 8 * N_T + 12 * n, as_vector(F::mins(hd)));
       }
     }
   };
   const auto stash = [&](auto step, int buf) {
     constexpr int J = decltype(step)::value;
-    const int id = afresh(tid), n = id >> 2, p = id & 3;
-    char* const row = smem + (buf * BUF + 128 * (M_T + n));
-    const int s = (n >> 1) & 7;
+    const uint32_t to = F::PLANES == 1 ? (uint32_t)afresh((int)w_to) : w_place(afresh(tid));
     uint4 lo[F::PLANES], hi[F::PLANES];
-    F::template decode<J>(raw, sc, p, lo, hi);
+    F::template decode<J>(raw, sc, afresh(tid) & 3, lo, hi);
 #pragma unroll
     for (int pl = 0; pl < F::PLANES; ++pl) {
-      *(uint4*)(row + 128 * N_T * pl + 16 * (p ^ s)) = lo[pl];
-      *(uint4*)(row + 128 * N_T * pl + 16 * ((4 + p) ^ s)) = hi[pl];
+      lds_put(to + (buf * BUF + 128 * N_T * pl), as_vector(lo[pl]));
+      lds_put((to ^ 64) + (buf * BUF + 128 * N_T * pl), as_vector(hi[pl]));
     }
   };
 
@@ -291,41 +315,39 @@ __global__ __launch_bounds__(64 * MMQF_WM * MMQF_WN, 2) void mmqf_kernel(const u
 
   // ---- one step of K: eight (block, tile pair) units, the matrix instructions of the next unit in front of the scaling
   const int swz = (lrow >> 1) & 7;                          // (tile bases are multiples of 16 rows)
-  const int op0 = 128 * lrow + 16 * (lhalf ^ swz), x_op = 128 * 32 * TM * wm, w_op = 128 * (M_T + 32 * TN * wn);
+  // (the operands of block b, half h are 64 b + 32 h away, by xor: rows are 128 bytes)
+  const uint32_t op0 = 128 * lrow + 16 * (lhalf ^ swz), x_op = lds0 + 128 * 32 * TM * wm, w_op = lds0 + 128 * (M_T + 32 * TN * wn);
   struct Operands { f16x8 x[TM][2], w[TN][F::PLANES][2]; };
-  const auto load_x = [&](int base, int buf, int b, int k, Operands& o) {
+  const auto load_x = [&](uint32_t at, int b, int k, Operands& o) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) o.x[k][h] = *(const f16x8*)(smem + (buf * BUF + (base ^ (16 * (4 * b + 2 * h)))) + x_op + 4096 * k);
+    for (int h = 0; h < 2; ++h) o.x[k][h] = lds_get<f16x8>((at ^ (64 * b + 32 * h)) + 4096 * k);
   };
-  const auto load_w = [&](int base, int buf, int b, int i, Operands& o) {
+  const auto load_w = [&](uint32_t at, int b, int i, Operands& o) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const char* const at = smem + (buf * BUF + (base ^ (16 * (4 * b + 2 * h)))) + w_op;
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int pl = 0; pl < F::PLANES; ++pl) o.w[i][pl][h] = *(const f16x8*)(at + 128 * N_T * pl + 4096 * i);
-    }
+      for (int pl = 0; pl < F::PLANES; ++pl) o.w[i][pl][h] = lds_get<f16x8>((at ^ (64 * b + 32 * h)) + (128 * N_T * pl + 4096 * i));
   };
   // A unit is a block and a pair of tiles, U units per block.  The matrix instructions of unit u + 1 stand between the
   // multiply-adds of unit u (each waits for the one before it), and an operand's successor is read as soon as the last
   // instruction that takes it has started.
   constexpr int U = TM * TN, P = 2 * F::PLANES;
   const auto load_first = [&](int buf, Operands& o) {
-    const int base = afresh(op0);
+    const uint32_t xat = x_op + buf * BUF + afresh(op0), wat = w_op + buf * BUF + afresh(op0);
 #pragma unroll
-    for (int i = 0; i < TN; ++i) load_w(base, buf, 0, i, o);
+    for (int i = 0; i < TN; ++i) load_w(wat, 0, i, o);
 #pragma unroll
-    for (int k = 0; k < TM; ++k) load_x(base, buf, 0, k, o);
+    for (int k = 0; k < TM; ++k) load_x(xat, 0, k, o);
   };
   const auto contract = [&](auto step, int buf, int pb, Operands& o) {
     constexpr int J = decltype(step)::value;
-    const float* const xd = (const float*)(smem + 2 * BUF + 32 * M_T * pb) + 2 * J * M_T + 32 * TM * wm + lrow;
-    const int base = afresh(op0);
+    const uint32_t xd = lds0 + 2 * BUF + 32 * M_T * pb + 128 * TM * wm + 4 * (afresh(lane) & 31), xat = x_op + buf * BUF + afresh(op0), wat = w_op + buf * BUF + afresh(op0);
     f32x16 s[2];
     float d8[2][TM];
 #pragma unroll
     for (int k = 0; k < TM; ++k) {
-      d8[0][k] = xd[32 * k];
-      d8[1][k] = xd[M_T + 32 * k];
+      d8[0][k] = lds_get<float>(xd + (8 * J * M_T + 128 * k));
+      d8[1][k] = lds_get<float>(xd + (8 * J * M_T + 4 * M_T + 128 * k));
     }
     const auto mfma = [&](int u, int piece, f32x16& v) {
       const int i = u / TM, k = u % TM, pl = piece >> 1, h = piece & 1;
@@ -341,8 +363,8 @@ __global__ __launch_bounds__(64 * MMQF_WM * MMQF_WN, 2) void mmqf_kernel(const u
         if (v + 1 < 2 * U) mfma((v + 1) % U, piece, s[(v + 1) & 1]);
         if (piece == P - 1 && v < U) {   // (unit v + 1 of the first block has its operands)
           const int un = v + 1, in = un / TM, kn = un % TM;
-          if (un < U && kn == TM - 1 && in < TN) load_w(base, buf, 1, in, o);
-          if (un < U && in == TN - 1) load_x(base, buf, 1, kn, o);
+          if (un < U && kn == TM - 1 && in < TN) load_w(wat, 1, in, o);
+          if (un < U && in == TN - 1) load_x(xat, 1, kn, o);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -356,33 +378,31 @@ __global__ __launch_bounds__(64 * MMQF_WM * MMQF_WN, 2) void mmqf_kernel(const u
   };
   // the end of a super-block
   const auto fold = [&]() {
-    const char* const xs = smem + PLANE_AT;
-    const char* const p = xs + 16 * M_T;
     const int ln = afresh(lane), row = ln & 31, half = ln >> 5;
-    uint4 sv[TM];
+    const uint32_t at = lds0 + PLANE_AT + 16 * M_T + 4 * (32 * TN * wn + 4 * half);    // d of the lane's first result
+    u32x4_m sv[TM];
     if constexpr (F::OFF)
 #pragma unroll
-      for (int k = 0; k < TM; ++k) sv[k] = *(const uint4*)(xs + 16 * (32 * (TM * wm + k) + row));
+      for (int k = 0; k < TM; ++k) {
+        // (a contraction over eight: the upper half of the lanes holds values 8 .. 15, zeros beside mins, which are finite)
+        sv[k] = lds_get<u32x4_m>(lds0 + PLANE_AT + 16 * (32 * (TM * wm) + row) + 512 * k);
+        if (half) sv[k] = (u32x4_m){0, 0, 0, 0};
+      }
 #pragma unroll
     for (int i = 0; i < TN; ++i) {
-      const int n = 32 * (TN * wn + i);
       __builtin_amdgcn_sched_barrier(0);
       f32x16 off[F::OFF ? TM : 1];
       tile_f4v d[4], dm[4];
       if constexpr (F::OFF) {
-        // (a contraction over eight: the upper half of the lanes holds values 8 .. 15, zeros)
-        uint4 mv = *(const uint4*)(p + 8 * N_T + 16 * (n + row));
-        if (half) mv = make_uint4(0, 0, 0, 0);
+        const u32x4_m mv = lds_get<u32x4_m>(lds0 + PLANE_AT + 16 * M_T + 8 * N_T + 16 * (32 * TN * wn + row) + 512 * i);
 #pragma unroll
-        for (int k = 0; k < TM; ++k) {
-          const uint4 v = half ? make_uint4(0, 0, 0, 0) : sv[k];
-          off[k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, mv), __builtin_bit_cast(f16x8, v), zero, 0, 0, 0);
-        }
+        for (int k = 0; k < TM; ++k)
+          off[k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, mv), __builtin_bit_cast(f16x8, sv[k]), zero, 0, 0, 0);
       }
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        d[q] = *(const tile_f4v*)(p + 4 * (n + 8 * q + 4 * half));
-        if (F::OFF) dm[q] = *(const tile_f4v*)(p + 4 * N_T + 4 * (n + 8 * q + 4 * half));
+        d[q] = lds_get<tile_f4v>(at + (128 * i + 32 * q));
+        if (F::OFF) dm[q] = lds_get<tile_f4v>(at + (4 * N_T + 128 * i + 32 * q));
       }
 #pragma unroll
       for (int k = 0; k < TM; ++k) {
@@ -430,7 +450,9 @@ __global__ __launch_bounds__(64 * MMQF_WM * MMQF_WN, 2) void mmqf_kernel(const u
           fetch_d8(sb + 1, pb ^ 1);
           fetch_head(sb + 1);
         }
+        __builtin_amdgcn_s_setprio(1);                      // (over the other wave's decoding)
         contract(step, J & 1, pb, o);
+        __builtin_amdgcn_s_setprio(0);
         if (J == 3) fold();
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
