@@ -28,6 +28,7 @@ struct TsCall {
   const void* bias;
   bool gemv_sums;              // offset term on d * sum(q) instead of the stored sums
   bool gemv;                   // the GEMV operator's arithmetic (Q5_0: see TQ5_0)
+  bool dealt;                  // dense, up to 32 rows: a column group's panels dealt to the waves of a workgroup
   MoeArgs moe;
   int row_blocks;              // tiles of 16 rt rows (dense) or blocks of slots
   double live_blocks;          // how many of them hold pairs, estimated (dense: all)

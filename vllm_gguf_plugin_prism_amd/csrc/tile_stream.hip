@@ -28,6 +28,20 @@ static bool ts_type_ok(int type) {
   }
 }
 
+// the tile operator's types that there are streaming tiles for, and the GEMV operator's
+static bool ts_tile_type_ok(int type) {
+  switch (type) {
+    case T_Q2_K: case T_Q3_K: case T_Q4_1: case T_Q5_0: case T_Q5_1: return true;
+    default: return ts_type_ok(type);
+  }
+}
+static bool ts_gemv_type_ok(int type) {
+  switch (type) {
+    case T_IQ2_XXS: case T_IQ2_XS: case T_IQ2_S: case T_IQ3_XXS: case T_IQ3_S: case T_IQ4_NL: case T_IQ4_XS: return true;
+    default: return ts_tile_type_ok(type);
+  }
+}
+
 // offsets inside a matrix and inside the quantized rows are 32-bit
 static bool ts_size_ok(int64_t rows_w, int64_t w_pitch, int64_t rows_x, int64_t K) {
   return rows_w * w_pitch <= 0xFFFF0000ll && rows_x * q8_row_bytes(K) <= 0xFFFF0000ll;
@@ -92,9 +106,34 @@ static double ts_most_work(int type) {
   return 0;
 }
 
+// Where the panels of a column group are dealt to the waves of a workgroup (tile_dealt_kernel) instead.  Against whatever ran before (the
+// streaming tiles, the kernel of the packed blocks, the staged 16-row tiles, the GEMV), over 7900 random products of 5 .. 32 rows, N 256 ..
+// 28672, K 512 .. 18944, both operators: where these lines take it 1.28 times as fast on average, over all 1.21 (Q2_K 1.30, Q3_K 1.27, Q4_1 1.22,
+// Q4_K, Q6_K, Q8_0, Q4_0 1.20, Q5_K, Q5_0 1.16, IQ4_XS 1.25, IQ2 and IQ3 1.16 to 1.19), 0.9 % short of always taking the faster; one in sixty is
+// slower by more than 3 %, the worst by 20 %.  us, before / dealt: [4096,4096] 12 rows Q4_K 11.0 / 8.4, Q6_K 12.5 / 10.0, [4096,14336] 12 rows Q6_K
+// 25.4 / 18.9, [2048,2048] Q4_K 8.5 / 6.7.
+static bool ts_dealt_takes(int type, int64_t M, int64_t N, int64_t K) {
+  if (M < 5 || M > 32) return false;
+  const int64_t groups = (N + 15) / 16, np = (K + 255) / 256;
+  // (a long K on few columns is cut between workgroups by the kernel of the packed blocks: [832,15872] Q6_K 11 rows 13.9 / 17.0)
+  if ((type == T_Q4_K || type == T_Q5_K || type == T_Q6_K) && groups <= 56 && K > 13000) return false;
+  // two tiles of rows leave room for one workgroup per CU: one round, or rows long enough to be worth a beginning
+  if (M > 16) return groups <= 256 || (K >= 4096 && groups <= 768);
+  const bool blocks32 = type == T_Q4_0 || type == T_Q4_1 || type == T_Q5_0 || type == T_Q5_1 || type == T_Q8_0 || type == T_IQ4_NL;
+  // Every group reads the activations again: past 1536 of them the waves with columns of their own are ahead ([28672,4096] Q4_K, 16 rows
+  // 21.5 / 24.5) unless K is too long for their LDS; and two panels per row are work for two waves of eight.
+  if (!blocks32) return (groups <= 1536 && groups <= 256 * np) || K >= 12000;
+  // (these decode more per panel, or keep two values per block and row: the beginning weighs less there)
+  if (M >= 9) return groups <= 512 || K >= 4096;
+  // the GEMV, one launch, is ahead on short rows, with Q5_0 and Q8_0 on small matrices ([480,2336] Q8_0 5 rows 5.4 / 6.9)
+  if (type == T_Q4_1 || type == T_Q5_1) return K >= 2048 && (groups <= 512 || K >= 8192);
+  return K >= 2048 && (N * K > 3000000 || (type != T_Q5_0 && type != T_Q8_0));
+}
+
 // Where the kernel is the faster one.
 bool ts_dense_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, bool gemv) {
   if (M < 5 || (M > 512 && !gemv) || N > 0x7FFFFFF0ll || K > 0x7FFFFFF0ll || M > 0x7FFFFFF0ll || !ts_size_ok(N, w_pitch, M < 512 ? M : 512, K)) return false;
+  if ((gemv ? ts_gemv_type_ok(type) : ts_tile_type_ok(type)) && ts_dealt_takes(type, M, N, K)) return true;
   if (M > 32 && !gemv) return 1e-6 * ((M + 31) / 32) * N * K < ts_most_work(type);
   const bool aligned = w_pitch % 16 == 0;
   switch (type) {
@@ -237,6 +276,7 @@ int ts_dense(int type, const void* W, const void* x, int dtype, void* workspace,
   c.rt = M <= 16 ? 1 : 2;
   c.w_pitch = la.w_pitch; c.ldy = la.ldy; c.bias = la.bias;
   c.gemv = gemv;
+  c.dealt = ts_dealt_takes(type, M, N, K);
   c.gemv_sums = gemv && (type == T_Q4_K || type == T_Q5_K);   // (the others' offset is on the stored sums there too)
   constexpr int64_t STEP = 512;                             // rows per launch, 16 tiles: the kernel's quotients by reciprocal stay exact
   for (int64_t m = 0; m < M; m += STEP) {

@@ -49,6 +49,7 @@ struct TsArgs {
 };
 
 typedef uint32_t u32x4_s __attribute__((ext_vector_type(4)));
+typedef _Float16 ts_h2 __attribute__((ext_vector_type(2)));
 
 template <int N> __device__ __forceinline__ void ts_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 // wave-uniform 16-byte-per-lane fetch into LDS: lane l's bytes land at m0 + 16 l
@@ -83,6 +84,92 @@ template <int XR> __host__ __device__ __forceinline__ constexpr int ts_scale_at(
 template <class F, class = void> struct TsTable { static constexpr int value = 0; };
 template <class F> struct TsTable<F, std::void_t<decltype(F::TABLE)>> { static constexpr int value = (F::TABLE + 15) / 16 * 16; };
 template <class F> constexpr bool ts_sums() { return F::OFF == 1 || F::HALVES; }   // the activations' block sums are wanted
+
+// A panel's products: acc += what the lane's column of it has with the rows of X.  xa: the lane's quants of the eight blocks; so: block
+// sums g and 4 + g of row c; left: blocks of the panel inside the row; half0: all bits in the lanes that hold the first 16
+// values of a block; d8_of, s8_of: block scales and sums of the lane's four result rows.
+template <class F, int RT, class D8, class S8>
+__device__ __forceinline__ void ts_multiply(F& w, const u32x4_s (&xa)[RT][4], const float (&so)[RT][2], int left, int g, uint32_t half0, D8 d8_of, S8 s8_of,
+                                            f32x4 (&acc)[RT]) {
+  constexpr bool OFFSET = F::OFF == 1;
+  const v4i seed = {kSeedBits, kSeedBits, kSeedBits, kSeedBits};
+  float dw[8 * (32 / F::G)];
+  w.ready();
+  uint32_t dm[8];
+  if constexpr (F::HALVES) w.words(dm);
+  else w.scales(dw);
+  // (opaque to the compiler, which would keep both masked copies of all operands over the column groups and spill)
+  uint32_t first = half0;
+  asm volatile("" : "+v"(first));
+  if (!F::KQ && left < 8) {
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {                       // (bytes behind the row's end need not be a number)
+      if constexpr (F::HALVES) dm[b] = b < left ? dm[b] : 0u;
+      else dw[b] = b < left ? dw[b] : 0.0f;
+    }
+  }
+  float m0 = 0.0f, m1 = 0.0f;
+  if constexpr (OFFSET) {
+    w.mins(g, m0, m1);
+    if (!F::KQ && left < 8) { m0 = g < left ? m0 : 0.0f; m1 = 4 + g < left ? m1 : 0.0f; }
+  }
+  // (the offsets of four blocks, then their products: the partial sums stay small, and so does what they round off)
+  f32x4 part[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+    part[rt] = OFFSET ? __builtin_amdgcn_mfma_f32_16x16x4f32(so[rt][0], -m0, (f32x4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0) : acc[rt];
+#pragma unroll
+  for (int b = 0; b < 8; ++b) {
+    if (OFFSET && b == 4) {
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) part[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(so[rt][1], -m1, part[rt], 0, 0, 0);
+    }
+    const uint2 q = w.codes(b, g);
+    const long bv = (long)(((uint64_t)q.y << 32) | q.x);
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      const f32x4 d8 = d8_of(rt, b);
+      const uint32_t alo = xa[rt][b >> 1][2 * (b & 1)], ahi = xa[rt][b >> 1][2 * (b & 1) + 1];
+      if constexpr (F::HALVES) {
+        const f32x4 s8 = s8_of(rt, b);
+        const ts_h2 v = __builtin_bit_cast(ts_h2, dm[b]), dv = {v[0], v[0]}, mv = {v[1], v[1]};
+        const v4i s = __builtin_amdgcn_mfma_i32_16x16x32_i8((long)(((uint64_t)ahi << 32) | alo), bv, seed, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; r += 2) {                // (d8 and s8 are halves in fp32)
+          const ts_h2 dd = (ts_h2){(_Float16)d8[r], (_Float16)d8[r + 1]} * dv, ms = (ts_h2){(_Float16)s8[r], (_Float16)s8[r + 1]} * mv;
+#pragma unroll
+          for (int e = 0; e < 2; ++e) part[rt][r + e] += __builtin_fmaf(seeded_times(s[r + e], 1.0f, -kSeed), (float)dd[e], (float)ms[e]);
+        }
+      } else if constexpr (F::G == 32) {
+        const float nsd = -kSeed * dw[b];
+        const v4i s = __builtin_amdgcn_mfma_i32_16x16x32_i8((long)(((uint64_t)ahi << 32) | alo), bv, seed, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) part[rt][r] = __builtin_fmaf(seeded_times(s[r], dw[b], nsd), d8[r], part[rt][r]);
+        if constexpr (F::OFF == 2) {
+          const uint2 mq = w.min_codes(b);
+          const float dmin = w.dmin();
+          const v4i sm = __builtin_amdgcn_mfma_i32_16x16x32_i8((long)(((uint64_t)ahi << 32) | alo), (long)(((uint64_t)mq.y << 32) | mq.x), seed, 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) part[rt][r] = __builtin_fmaf(seeded_times(sm[r], -dmin, kSeed * dmin), d8[r], part[rt][r]);
+        }
+      } else {
+        // a scale per 16 values: the activations of either half of the block, the other half's lanes zeroed
+        const long a0 = (long)(((uint64_t)(ahi & first) << 32) | (alo & first));
+        const long a1 = (long)(((uint64_t)(ahi & ~first) << 32) | (alo & ~first));
+        const float n0 = -kSeed * dw[2 * b], n1 = -kSeed * dw[2 * b + 1];
+        const v4i s0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a0, bv, seed, 0, 0, 0);
+        const v4i s1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a1, bv, seed, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          part[rt][r] = __builtin_fmaf(seeded_times(s0[r], dw[2 * b], n0), d8[r], part[rt][r]);
+          part[rt][r] = __builtin_fmaf(seeded_times(s1[r], dw[2 * b + 1], n1), d8[r], part[rt][r]);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) acc[rt] = OFFSET ? acc[rt] + part[rt] : part[rt];
+}
 
 template <class F, int RT, bool GATE, bool SPLIT, int D>
 __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_stream_kernel(const uint8_t* __restrict__ W, const char* __restrict__ ws,
@@ -274,7 +361,6 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
   if constexpr (TsTable<F>::value) F::tables(smem + table_off);
   __syncthreads();
 
-  const v4i seed = {kSeedBits, kSeedBits, kSeedBits, kSeedBits};
   const uint32_t half0 = g < 2 ? ~0u : 0u;                  // lanes that hold the first 16 values of a block
   const auto store = [&](int m, int n, float v) {           // result row m of this workgroup's tile, feature n (all lanes together)
     const int row = is_moe ? __shfl(pair_at, m) : block * XR + m;
@@ -332,83 +418,8 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
       ++t;
       slot = slot + 1 == D ? 0 : slot + 1;
 
-      float dw[8 * (32 / F::G)];
-      w.ready();
-      uint32_t dm[8];
-      if constexpr (F::HALVES) w.words(dm);
-      else w.scales(dw);
-      // (opaque to the compiler, which would keep both masked copies of all operands over the column groups and spill)
-      uint32_t first = half0;
-      asm volatile("" : "+v"(first));
-      if (!F::KQ && left < 8) {
-#pragma unroll
-        for (int b = 0; b < 8; ++b) {                       // (bytes behind the row's end need not be a number)
-          if constexpr (F::HALVES) dm[b] = b < left ? dm[b] : 0u;
-          else dw[b] = b < left ? dw[b] : 0.0f;
-        }
-      }
-      float m0 = 0.0f, m1 = 0.0f;
-      if constexpr (OFFSET) {
-        w.mins(g, m0, m1);
-        if (!F::KQ && left < 8) { m0 = g < left ? m0 : 0.0f; m1 = 4 + g < left ? m1 : 0.0f; }
-      }
-      // (the offsets of four blocks, then their products: the partial sums stay small, and so does what they round off)
-      f32x4 part[RT];
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
-        part[rt] = OFFSET ? __builtin_amdgcn_mfma_f32_16x16x4f32(so[rt][0], -m0, (f32x4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0) : acc[rt];
-#pragma unroll
-      for (int b = 0; b < 8; ++b) {
-        if (OFFSET && b == 4) {
-#pragma unroll
-          for (int rt = 0; rt < RT; ++rt) part[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(so[rt][1], -m1, part[rt], 0, 0, 0);
-        }
-        const uint2 q = w.codes(b, g);
-        const long bv = (long)(((uint64_t)q.y << 32) | q.x);
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-          const f32x4 d8 = *(const f32x4*)(xd + ts_scale_at<XR>(8 * pl) + ts_scale_at<XR>(b) + 16 * rt + 4 * g);
-          const uint32_t alo = xa[rt][b >> 1][2 * (b & 1)], ahi = xa[rt][b >> 1][2 * (b & 1) + 1];
-          if constexpr (F::HALVES) {
-            typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-            const f32x4 s8 = *(const f32x4*)(xd + ts_scale_at<XR>(8 * PC) + ts_scale_at<XR>(8 * pl) + ts_scale_at<XR>(b) + 16 * rt + 4 * g);
-            const h2 v = __builtin_bit_cast(h2, dm[b]), dv = {v[0], v[0]}, mv = {v[1], v[1]};
-            const v4i s = __builtin_amdgcn_mfma_i32_16x16x32_i8((long)(((uint64_t)ahi << 32) | alo), bv, seed, 0, 0, 0);
-#pragma unroll
-            for (int r = 0; r < 4; r += 2) {                // (d8 and s8 are halves in fp32)
-              const h2 dd = (h2){(_Float16)d8[r], (_Float16)d8[r + 1]} * dv, ms = (h2){(_Float16)s8[r], (_Float16)s8[r + 1]} * mv;
-#pragma unroll
-              for (int e = 0; e < 2; ++e) part[rt][r + e] += __builtin_fmaf(seeded_times(s[r + e], 1.0f, -kSeed), (float)dd[e], (float)ms[e]);
-            }
-          } else if constexpr (F::G == 32) {
-            const float nsd = -kSeed * dw[b];
-            const v4i s = __builtin_amdgcn_mfma_i32_16x16x32_i8((long)(((uint64_t)ahi << 32) | alo), bv, seed, 0, 0, 0);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) part[rt][r] = __builtin_fmaf(seeded_times(s[r], dw[b], nsd), d8[r], part[rt][r]);
-            if constexpr (F::OFF == 2) {
-              const uint2 mq = w.min_codes(b);
-              const float dmin = w.dmin();
-              const v4i sm = __builtin_amdgcn_mfma_i32_16x16x32_i8((long)(((uint64_t)ahi << 32) | alo), (long)(((uint64_t)mq.y << 32) | mq.x), seed, 0, 0, 0);
-#pragma unroll
-              for (int r = 0; r < 4; ++r) part[rt][r] = __builtin_fmaf(seeded_times(sm[r], -dmin, kSeed * dmin), d8[r], part[rt][r]);
-            }
-          } else {
-            // a scale per 16 values: the activations of either half of the block, the other half's lanes zeroed
-            const long a0 = (long)(((uint64_t)(ahi & first) << 32) | (alo & first));
-            const long a1 = (long)(((uint64_t)(ahi & ~first) << 32) | (alo & ~first));
-            const float n0 = -kSeed * dw[2 * b], n1 = -kSeed * dw[2 * b + 1];
-            const v4i s0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a0, bv, seed, 0, 0, 0);
-            const v4i s1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a1, bv, seed, 0, 0, 0);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              part[rt][r] = __builtin_fmaf(seeded_times(s0[r], dw[2 * b], n0), d8[r], part[rt][r]);
-              part[rt][r] = __builtin_fmaf(seeded_times(s1[r], dw[2 * b + 1], n1), d8[r], part[rt][r]);
-            }
-          }
-        }
-      }
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) acc[rt] = OFFSET ? acc[rt] + part[rt] : part[rt];
+      ts_multiply<F, RT>(w, xa, so, left, g, half0, [&](int rt, int b) { return *(const f32x4*)(xd + ts_scale_at<XR>(8 * pl) + ts_scale_at<XR>(b) + 16 * rt + 4 * g); },
+                         [&](int rt, int b) { return *(const f32x4*)(xd + ts_scale_at<XR>(8 * PC) + ts_scale_at<XR>(8 * pl) + ts_scale_at<XR>(b) + 16 * rt + 4 * g); }, acc);
     }
     // ---- the next chunk of activations
     if constexpr (SPLIT) {
@@ -511,6 +522,157 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
   }
 }
 
+// A column group per workgroup, its panels of K dealt to the eight waves: where the output has too few column groups for a wave
+// each.  No two waves of a workgroup multiply the same activations then, so a wave fetches those of its panel beside the
+// panel's weights, into a place of its own, and meets the others only for the sum: no chunk of activations that the workgroup
+// waits for, loads, and waits for again (2.5 us each, seven of them at K = 14336).  A wave has one panel under way, asked for as soon
+// as the one before is in registers, and sixteen waves share a CU: two panels a wave on eight waves were slower by a fifth, as
+// were one workgroup of sixteen waves (a tenth) and of four.
+// In LDS: the panel's bytes, block scales and sums of its sixteen rows of X (32 bytes each, 512 the plane), their quants, 256 bytes
+// a row.  An operand is 16 bytes of each of sixteen rows, all in the same banks: piece j of row r lies in place j ^ r, which the
+// fetch sees to (a lane asks for the piece that belongs where its bytes land).  Rows past X are fetched up to a multiple of four
+// only: what lies in LDS behind them stands in rows of the result that are not stored.
+// What bounds it is the weight stream, and beside it the activations' way to every workgroup (2.3 us of [4096,14336]'s 15) and the
+// vector instructions of a panel (Q6_K 350: 5 us).  Without the quantizer's launch, us, streaming tiles / this, 12 rows: Q6_K [4096,14336]
+// 22.1 / 15.1, [4096,4096] 9.6 / 7.1, [1024,4096] 8.5 / 5.9; Q4_K [4096,14336] 16.9 / 11.7, [11008,4096] 13.4 / 10.7, [2048,2048] 5.8 / 4.0; 24
+// rows Q6_K [4096,14336] 29.5 / 25.0, [4096,4096] 11.5 / 8.9.  Tried and slower: workgroups that stay and walk several column groups, the
+// next one's first panel under way over the sum (0.86 to 1.06 times the speed: the addresses cost more than the beginning).
+template <class F, int RT> __host__ __device__ constexpr int ts_dealt_place(int ppr, int xn) { return 256 * ppr + 1024 * RT + 1024 * xn; }
+// (two workgroups of one tile of rows share a CU where its registers suffice)
+template <class F, int RT> constexpr int ts_dealt_waves() { return RT == 1 && !F::HALVES && (F::KQ || F::OFF != 1) ? 4 : 2; }
+template <class F, int RT>
+__global__ __launch_bounds__(64 * TS_NW, (ts_dealt_waves<F, RT>())) void tile_dealt_kernel(const uint8_t* __restrict__ W, const char* __restrict__ ws, void* __restrict__ Y, TsArgs a) {
+  constexpr int NW = TS_NW;
+  constexpr bool SUMS = ts_sums<F>(), OFFSET = F::OFF == 1;
+  constexpr int PPR_MIN = (F::PB + 15) / 16, PPR_MAX = (F::PB + 29) / 16;
+  constexpr int NI = (16 * (PPR_MAX | 1) + 63) / 64, FULL = 16 * PPR_MIN / 64;
+  extern __shared__ __align__(16) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  int wg = blockIdx.x;
+  const int total8 = gridDim.x & ~7u;                       // each of the 8 XCDs gets a contiguous run of workgroups
+  if (wg < total8) wg = (wg & 7) * (total8 >> 3) + (wg >> 3);
+  const int xn = (a.M + 3) >> 2;                            // fetches of quants per panel, four rows each
+  const int w_bytes = 256 * a.ppr, place = ts_dealt_place<F, RT>(a.ppr, xn);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+  const int mine = wave * place, table_off = NW * place + 16;   // (a last field's cut may touch the word behind its row)
+
+  const uint32_t wmis = (uint32_t)((uintptr_t)W & 15);
+  const uint8_t* const wbase = W - wmis;
+  const uint32_t row_bytes = (uint32_t)(F::KQ ? a.np * F::PB : (a.K >> 5) * (F::PB / 8));
+  const uint32_t last16 = ((uint32_t)(a.N - 1) * a.w_pitch + wmis + row_bytes - 1) & ~15u;   // the last granule that holds bytes of W
+  uint32_t w_row[NI], pc16[NI];                             // where the piece's row begins; the piece
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int p = min(64 * i + lane, 16 * a.ppr - 1);
+    const uint32_t r = __umulhi((uint32_t)p, a.ppr_inv);
+    w_row[i] = (uint32_t)min(16 * wg + (int)r, a.N - 1) * a.w_pitch + wmis;
+    pc16[i] = (uint32_t)min(p - (int)r * a.ppr, PPR_MAX - 1) * 16;   // (the piece that only spaces rows: the last again)
+  }
+  uint32_t x_at[4 * RT], s_at[RT];
+#pragma unroll
+  for (int i = 0; i < 4 * RT; ++i) {
+    const int row = 4 * i + g;
+    x_at[i] = (uint32_t)min(row, a.M - 1) * a.ws_row_bytes + 16 * (uint32_t)(c ^ (row & 15));
+  }
+  // (a lane: half of a row's eight scales, in the upper half of the lanes of its sums)
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+    s_at[rt] = (uint32_t)min(16 * rt + ((lane & 31) >> 1), a.M - 1) * a.ws_row_bytes + (uint32_t)a.Kp + 16 * (lane & 1) + (SUMS && lane >= 32 ? 4 * a.plane * (a.Kp >> 5) : 0);
+  const auto request = [&](int p) {
+    const uint32_t to = lds0 + mine, off = (uint32_t)(p * F::PB);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const uint32_t v = min(((w_row[i] + off) & ~15u) + pc16[i], last16);
+      if (i < FULL) {
+        ts_fetch(v, wbase, to + 1024 * i);
+      } else {   // (lanes past the panel's last piece stay out: their bytes would land behind it)
+        const int on = 16 * a.ppr - 64 * i;
+        ts_fetch_some(v, wbase, to + 1024 * i, on >= 64 ? ~0ull : on <= 0 ? 0ull : (1ull << on) - 1);
+      }
+    }
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) ts_fetch(s_at[rt] + 32 * (uint32_t)p, ws, to + w_bytes + 1024 * rt);
+#pragma unroll
+    for (int i = 0; i < 4 * RT; ++i)
+      if (i < xn) ts_fetch(x_at[i] + 256 * (uint32_t)p, ws, to + w_bytes + 1024 * RT + 1024 * i);
+  };
+  if (wave < a.np) request(wave);
+  if constexpr (TsTable<F>::value) {
+    F::tables(smem + table_off);
+    __syncthreads();
+  }
+
+  const uint32_t half0 = g < 2 ? ~0u : 0u;                  // lanes that hold the first 16 values of a block
+  const int nkb = a.K >> 5;
+  f32x4 acc[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) acc[rt] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+  const char* const at = smem + mine;
+  const char* const scales = at + w_bytes;
+  const uint32_t w_lane = (uint32_t)min(16 * wg + c, a.N - 1) * a.w_pitch + wmis;
+  for (int p = wave; p < a.np; p += NW) {
+    const int left = nkb - 8 * p;                           // blocks of the panel inside the row
+    ts_wait<0>();
+    F w;
+    if constexpr (TsTable<F>::value) w.tab = smem + table_off;
+    w.read(at + c * (16 * a.ppr), F::PB % 16 == 0 && a.ppr == F::PB / 16 ? 0u : (w_lane + (uint32_t)(p * F::PB)) & 15, g);
+    u32x4_s xa[RT][4];
+    float so[RT][2];
+    // of rows 4 g + r, blocks 0 .. 7: the block scales, or, with HALVES, (scale, sum) as the halves that they are (behind a row's last
+    // block lie the quantizer's zeros)
+    float d8[RT][4][8];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) xa[rt][i] = *(const u32x4_s*)(scales + 1024 * RT + 4096 * rt + 256 * c + 16 * ((4 * i + g) ^ c));
+      if constexpr (OFFSET) {
+        so[rt][0] = *(const float*)(scales + 1024 * rt + 512 + 32 * c + 4 * g);
+        so[rt][1] = *(const float*)(scales + 1024 * rt + 512 + 32 * c + 16 + 4 * g);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const f32x4 v = *(const f32x4*)(scales + 1024 * rt + 32 * (4 * g + r) + 16 * h);
+          f32x4 z = v;
+          if constexpr (F::HALVES) z = *(const f32x4*)(scales + 1024 * rt + 512 + 32 * (4 * g + r) + 16 * h);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if constexpr (F::HALVES) d8[rt][r][4 * h + e] = __builtin_bit_cast(float, (ts_h2){(_Float16)v[e], (_Float16)z[e]});
+            else d8[rt][r][4 * h + e] = v[e];
+          }
+        }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // the place may be filled again
+    if (p + NW < a.np) request(p + NW);
+    const auto of = [&](int rt, int b, int half) {
+      f32x4 o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if constexpr (F::HALVES) o[r] = (float)__builtin_bit_cast(ts_h2, d8[rt][r][b])[half];
+        else o[r] = d8[rt][r][b];
+      }
+      return o;
+    };
+    ts_multiply<F, RT>(w, xa, so, left, g, half0, [&](int rt, int b) { return of(rt, b, 0); }, [&](int rt, int b) { return of(rt, b, 1); }, acc);
+  }
+
+  // ---- the eight partial tiles, added in the order of the waves
+  __syncthreads();
+  float* const red = (float*)smem;                          // [NW][RT][64] of four floats, over the panels
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) *(f32x4*)(red + ((wave * RT + rt) * 64 + lane) * 4) = acc[rt];
+  __syncthreads();
+  if (tid < 256 * RT) {
+    const int n = tid & 15, m = tid >> 4, l = 16 * ((m >> 2) & 3) + n, rt = m >> 4;   // result row m, feature n of the group
+    float v = red[(rt * 64 + l) * 4 + (m & 3)];
+#pragma unroll
+    for (int z = 1; z < NW; ++z) v += red[((z * RT + rt) * 64 + l) * 4 + (m & 3)];
+    if (m < a.M && 16 * wg + n < a.N) ts_store(Y, (int64_t)m * a.ldy + 16 * wg + n, v, a.bias, 16 * wg + n, a.dtype);
+  }
+}
+
 static inline size_t ts_chunk_bytes(int rt, bool off, int pc) {
   return (size_t)16 * rt * (256 * pc + 16) + (size_t)(8 * pc * 16 * rt + 2 * pc * 16) * 4 * (off ? 2 : 1);
 }
@@ -586,8 +748,31 @@ static int ts_launch(const TsCall& c, int ks, hipStream_t stream) {
 }
 
 template <class F, int RT>
+static int ts_dealt_launch(const TsCall& c, hipStream_t stream) {
+  if (c.M > 16 * RT || c.row_blocks != 1) return GGUF_NOT_TAKEN;
+  const int np = (c.K + 255) / 256, qk = F::KQ ? 256 : 32, bs = F::KQ ? F::PB : F::PB / 8;
+  const int64_t pitch = c.w_pitch ? c.w_pitch : (int64_t)(c.K / qk) * bs;
+  const bool aligned = F::PB % 16 == 0 && pitch % 16 == 0 && (uintptr_t)c.W % 16 == 0;
+  const int ppr = (aligned ? F::PB / 16 : (F::PB + 29) / 16) | 1;   // (odd: banks)
+  size_t lds = (size_t)TS_NW * ts_dealt_place<F, RT>(ppr, (c.M + 3) / 4) + 16 + TsTable<F>::value;
+  if (lds < (size_t)TS_NW * RT * 1024) lds = (size_t)TS_NW * RT * 1024;
+  if (lds > 160 * 1024) return GGUF_NOT_TAKEN;
+  auto kern = tile_dealt_kernel<F, RT>;
+  static std::atomic<uint64_t> done{0};
+  if (lds > 64 * 1024) allow_large_lds(kern, 160 * 1024, done);
+  const TsArgs a = {c.M, c.N, c.K, (int)q8_kp(c.K), (uint32_t)pitch, (uint32_t)q8_row_bytes(c.K), np, 3, ppr, 0, 0, 1, (uint32_t)((0x100000000ull + ppr - 1) / ppr), 0, 0,
+                    c.gemv_sums ? 2 : 1, c.dtype, c.ldy ? c.ldy : (int64_t)c.N, c.bias};
+  hipLaunchKernelGGL(kern, dim3((unsigned)((c.N + 15) / 16)), dim3(64 * TS_NW), lds, stream, (const uint8_t*)c.W, (const char*)c.ws, c.Y, a);
+  return launch_status();
+}
+
+template <class F, int RT>
 static int ts_run_rt(const TsCall& c, hipStream_t stream) {
   const int np = (c.K + 255) / 256;
+  if (c.dealt) {
+    const int rc = ts_dealt_launch<F, RT>(c, stream);
+    if (rc != GGUF_NOT_TAKEN) return rc;
+  }
   const int ks = ts_ks(np, c.live_blocks * ((c.N + 15) / 16));
   if (ks == 1 && np <= 16) {
     const int rc = ts_launch<F, RT, false, false>(c, 1, stream);
