@@ -67,3 +67,11 @@ def test_dense_where_it_is_taken(qtype, m, n, k):
     x = rng.standard_normal((m, k)).astype(np.float32)
     y = ops.ggml_mul_mat_a8(torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda(), qtype, n)
     assert o.rel_l2(y.cpu().numpy(), o.mul_mat_a8(w, x, qtype, n, "mmq")) <= 1e-5
+
+
+# layers whose last round of workgroups is cut finer: behind a full round in both products, an odd number of panels dealt to two waves,
+# more blocks than expected, inner sizes that end inside a workgroup's features; all of a product in one round
+@pytest.mark.parametrize("qtype,tokens,e,hid,inner", [(o.Q4_0, 60, 40, 736, 1056), (o.Q8_0, 90, 44, 544, 2080), (o.Q4_K, 60, 40, 2304, 1024), (o.Q6_K, 40, 36, 1280, 1280),
+                                                      (o.Q5_K, 12, 6, 768, 512)])
+def test_moe_layer_last_round(qtype, tokens, e, hid, inner):
+    test_moe_layer_edges(qtype, tokens, e, hid, inner)
