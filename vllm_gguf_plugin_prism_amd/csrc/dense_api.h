@@ -10,7 +10,7 @@
  * gguf_mmq_layer_workspace_bytes: the workspace with which gguf_mmq_linear on GGUF_MMQ_AUTO runs at full speed for weights
  * of this type, at a 16-byte boundary.  (gguf_mmq_workspace_bytes_engine does not know the type.)  gguf_mmq_layer_route: the
  * kernel that such a call with a workspace of this size runs: 1 the streaming tile kernel, 4 the wide tiles, 2 the
- * half-precision unit's, 0 another.  gguf_mmq_layer_unit: the same, with 2 added to 1 (past 32 rows) and 4 where the
+ * half-precision unit's, 0 another; up to 32 rows the one that stands behind tile_dealt_kernel, whose lines are its own.  gguf_mmq_layer_unit: the same, with 2 added to 1 (past 32 rows) and 4 where the
  * half-precision unit would run a call that these decline.  gguf_moe_mmq_layer_wide: whether
  * gguf_moe_mmq_layer with the workspace it asks for, at addresses divisible by 16, runs on the wide tiles. */
 #pragma once

@@ -899,7 +899,7 @@ extern "C" int64_t gguf_mmq_layer_workspace_bytes(int type, int64_t N, int64_t K
 
 extern "C" int gguf_mmq_layer_route(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes) {
   if (M <= 0 || N <= 0 || K <= 0 || M > 0x7FFFFFF0LL || N > 0x7FFFFFF0LL || K > 0x7FFFFFF0LL) return 0;
-  if (gguf::ts_dense_takes(type, M, N, K, w_row_pitch_bytes)) return 1;
+  if (gguf::ts_stream_takes(type, M, N, K, w_row_pitch_bytes)) return 1;
   if (gguf::wide_dense_plan(type, M, N, K, w_row_pitch_bytes, workspace_bytes).rt) return 4;
   return gguf::mmqf_takes(type, M, N, K, w_row_pitch_bytes, workspace_bytes, mmq_rows_bytes(M, K, false)) ? 2 : 0;
 }

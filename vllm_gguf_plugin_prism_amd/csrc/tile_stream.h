@@ -37,6 +37,7 @@ struct TsCall {
 
 // tile_stream.hip: whether a call is taken -- a dense product of M rows, a layer with this many (token, expert) pairs, an
 // expert GEMM on blocks of 16 slots by itself; how much faster than pair by pair a layer is (0: not taken)
+bool ts_stream_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, bool gemv = false);   // without those that deal panels
 bool ts_dense_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, bool gemv = false);   // gemv: in place of the GEMV
 int ts_dense(int type, const void* W, const void* x, int dtype, void* workspace, void* Y, int64_t M, int N, int K, bool gemv, const LinearArgs& la, hipStream_t s);
 bool ts_layer_takes(int type13, int type2, int64_t H, int64_t I, int64_t N_out, int64_t tokens, int64_t top_k, int64_t num_experts);

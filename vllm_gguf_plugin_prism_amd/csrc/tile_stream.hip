@@ -113,7 +113,7 @@ static double ts_most_work(int type) {
 // slower by more than 3 %, the worst by 20 %.  us, before / dealt: [4096,4096] 12 rows Q4_K 11.0 / 8.4, Q6_K 12.5 / 10.0, [4096,14336] 12 rows Q6_K
 // 25.4 / 18.9, [2048,2048] Q4_K 8.5 / 6.7.
 static bool ts_dealt_takes(int type, int64_t M, int64_t N, int64_t K) {
-  if (M < 5 || M > 32) return false;
+  if (M < 5 || M > 32 || N > 0x7FFFFF0ll || K > 0x7FFFFF0ll) return false;
   const int64_t groups = (N + 15) / 16, np = (K + 255) / 256;
   // (a long K on few columns is cut between workgroups by the kernel of the packed blocks: [832,15872] Q6_K 11 rows 13.9 / 17.0)
   if ((type == T_Q4_K || type == T_Q5_K || type == T_Q6_K) && groups <= 56 && K > 13000) return false;
@@ -130,10 +130,9 @@ static bool ts_dealt_takes(int type, int64_t M, int64_t N, int64_t K) {
   return K >= 2048 && (N * K > 3000000 || (type != T_Q5_0 && type != T_Q8_0));
 }
 
-// Where the kernel is the faster one.
-bool ts_dense_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, bool gemv) {
+// Where tile_stream_kernel is the faster one of those that do not deal panels.
+bool ts_stream_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, bool gemv) {
   if (M < 5 || (M > 512 && !gemv) || N > 0x7FFFFFF0ll || K > 0x7FFFFFF0ll || M > 0x7FFFFFF0ll || !ts_size_ok(N, w_pitch, M < 512 ? M : 512, K)) return false;
-  if ((gemv ? ts_gemv_type_ok(type) : ts_tile_type_ok(type)) && ts_dealt_takes(type, M, N, K)) return true;
   if (M > 32 && !gemv) return 1e-6 * ((M + 31) / 32) * N * K < ts_most_work(type);
   const bool aligned = w_pitch % 16 == 0;
   switch (type) {
@@ -176,6 +175,12 @@ bool ts_dense_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, 
   // split and the columns no more than the CUs hold: [4096,4096] 16 rows 11.1 / 10.3, [2048,3072] 10.1 / 9.0; where it is two
   // launches, [2560,4096] 10.7 / 16.0, or two rounds, [5120,4096] 12.9 / 14.7, or the rows short, [4096,2048] 8.7 / 10.0, it falls behind.
   return !(type == T_Q4_0 && M <= 16 && K > 2048 && K <= 4096 && K % 256 == 0 && N <= 4096 && (K < 4096 || N > 3056));
+}
+
+// Dense products on either kernel.
+bool ts_dense_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, bool gemv) {
+  return ((gemv ? ts_gemv_type_ok(type) : ts_tile_type_ok(type)) && ts_dealt_takes(type, M, N, K) && ts_size_ok(N, w_pitch, M, K)) ||
+         ts_stream_takes(type, M, N, K, w_pitch, gemv);
 }
 
 bool ts_moe_takes(int type, int64_t N, int64_t K, int64_t num_sorted, int64_t tokens, int64_t top_k) {
