@@ -90,6 +90,10 @@ _LAYER_SIGNATURES = {
     "gguf_mmq_layer_unit": (_c.c_int, [_c.c_int, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64]),
     "gguf_moe_mmq_layer_wide": (_c.c_int, [_c.c_int, _c.c_int, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64]),
     "gguf_mmq_layer_route": (_c.c_int, [_c.c_int, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64]),
+    "gguf_linear_two_takes": (_c.c_int, [_c.c_int, _c.c_int64, _c.c_int64, _c.c_int, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int]),
+    "gguf_linear_two": (_c.c_int, [_c.c_void_p, _c.c_int64, _c.c_int, _c.c_int64, _c.c_void_p, _c.c_void_p,
+                                   _c.c_void_p, _c.c_int64, _c.c_int, _c.c_int64, _c.c_void_p, _c.c_void_p,
+                                   _c.c_void_p, _c.c_int, _c.c_void_p, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int, _c.c_void_p]),
     "gguf_dense_linear": (_c.c_int, [_c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_int, _c.c_void_p, _c.c_void_p, _c.c_int64,
                                      _c.c_void_p, _c.c_int, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_void_p]),
 }

@@ -10,9 +10,14 @@
  * gguf_mmq_layer_workspace_bytes: the workspace with which gguf_mmq_linear on GGUF_MMQ_AUTO runs at full speed for weights
  * of this type, at a 16-byte boundary.  (gguf_mmq_workspace_bytes_engine does not know the type.)  gguf_mmq_layer_route: the
  * kernel that such a call with a workspace of this size runs: 1 the streaming tile kernel, 4 the wide tiles, 2 the
- * half-precision unit's, 0 another; up to 32 rows the one that stands behind tile_dealt_kernel, whose lines are its own.  gguf_mmq_layer_unit: the same, with 2 added to 1 (past 32 rows) and 4 where the
- * half-precision unit would run a call that these decline.  gguf_moe_mmq_layer_wide: whether
- * gguf_moe_mmq_layer with the workspace it asks for, at addresses divisible by 16, runs on the wide tiles. */
+ * half-precision unit's, 0 another; up to 32 rows the one that stands behind tile_dealt_kernel, whose lines are its own.
+ * gguf_mmq_layer_unit: the same, with 2 added to 1 (past 32 rows) and 4 where the half-precision unit would run a call that these decline.  gguf_moe_mmq_layer_wide: whether
+ * gguf_moe_mmq_layer with the workspace it asks for, at addresses divisible by 16, runs on the wide tiles.
+ *
+ * gguf_linear_two: two products of the same x, up to 32 rows, as two calls of gguf_mmvq_linear (gemv) or gguf_mmq_linear would run them
+ * (the same results bit for bit), x quantized once and, for most pairs of types that recipes mix, in one launch behind that: shards of a merged
+ * layer, columns of one result of this row pitch.  The workspace, M * gguf_q8_1_row_bytes(K), begins on 16 bytes.
+ * gguf_linear_two_takes: 1 for a pair that it serves. */
 #pragma once
 #include <stdint.h>
 #ifdef __cplusplus
@@ -25,6 +30,9 @@ int gguf_dense_linear(const void* W, int64_t w_row_pitch_bytes, const void* x, i
 int64_t gguf_mmq_layer_workspace_bytes(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes);
 int gguf_moe_mmq_layer_wide(int type13, int type2, int64_t H, int64_t I, int64_t N_out, int64_t top_k, int64_t tokens, int64_t num_experts);
 int gguf_mmq_layer_unit(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes);
+int gguf_linear_two_takes(int type, int64_t N, int64_t w_row_pitch_bytes, int type2, int64_t N2, int64_t w_row_pitch_bytes2, int64_t K, int64_t M, int gemv);
+int gguf_linear_two(const void* W, int64_t w_row_pitch_bytes, int type, int64_t N, void* Y, const void* bias, const void* W2, int64_t w_row_pitch_bytes2, int type2,
+                    int64_t N2, void* Y2, const void* bias2, const void* x, int xdtype, void* q8_workspace, int64_t y_row_pitch, int64_t K, int64_t M, int gemv, void* stream);
 int gguf_mmq_layer_route(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes);
 #ifdef __cplusplus
 }

@@ -558,7 +558,7 @@ template <class F, int RT> __host__ __device__ constexpr int ts_dealt_place(int 
 // (two workgroups of one tile of rows share a CU where its registers suffice)
 template <class F, int RT> constexpr int ts_dealt_waves() { return RT == 1 && !F::HALVES && (F::KQ || F::OFF != 1) ? 4 : 2; }
 template <class F, int RT>
-__global__ __launch_bounds__(64 * TS_NW, (ts_dealt_waves<F, RT>())) void tile_dealt_kernel(const uint8_t* __restrict__ W, const char* __restrict__ ws, void* __restrict__ Y, TsArgs a) {
+__device__ __forceinline__ void tile_dealt_body(const uint8_t* __restrict__ W, const char* __restrict__ ws, void* __restrict__ Y, const TsArgs& a, int wg, int groups) {
   constexpr int NW = TS_NW;
   constexpr bool SUMS = ts_sums<F>(), OFFSET = F::OFF == 1;
   constexpr int PPR_MIN = (F::PB + 15) / 16, PPR_MAX = (F::PB + 29) / 16;
@@ -566,8 +566,7 @@ __global__ __launch_bounds__(64 * TS_NW, (ts_dealt_waves<F, RT>())) void tile_de
   extern __shared__ __align__(16) char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
-  int wg = blockIdx.x;
-  const int total8 = gridDim.x & ~7u;                       // each of the 8 XCDs gets a contiguous run of workgroups
+  const int total8 = groups & ~7;                           // each of the 8 XCDs gets a contiguous run of workgroups
   if (wg < total8) wg = (wg & 7) * (total8 >> 3) + (wg >> 3);
   const int xn = (a.M + 3) >> 2;                            // fetches of quants per panel, four rows each
   const int w_bytes = 256 * a.ppr, place = ts_dealt_place<F, RT>(a.ppr, xn);
@@ -690,6 +689,20 @@ __global__ __launch_bounds__(64 * TS_NW, (ts_dealt_waves<F, RT>())) void tile_de
   }
 }
 
+template <class F, int RT>
+__global__ __launch_bounds__(64 * TS_NW, (ts_dealt_waves<F, RT>())) void tile_dealt_kernel(const uint8_t* __restrict__ W, const char* __restrict__ ws, void* __restrict__ Y, TsArgs a) {
+  tile_dealt_body<F, RT>(W, ws, Y, a, blockIdx.x, gridDim.x);
+}
+
+// The same for two matrices with the same rows of X, those of a merged layer whose recipe gives one of its tensors more bits: the
+// workgroups of the second, often too few for the chip by themselves, run beside the first's, and a launch less.
+template <class F, class G, int RT>
+__global__ __launch_bounds__(64 * TS_NW, (ts_dealt_waves<F, RT>() < ts_dealt_waves<G, RT>() ? ts_dealt_waves<F, RT>() : ts_dealt_waves<G, RT>())) void tile_dealt_pair_kernel(
+    const uint8_t* __restrict__ W, const uint8_t* __restrict__ V, const char* __restrict__ ws, void* __restrict__ Y, void* __restrict__ Z, TsArgs a, TsArgs b, int groups) {
+  if ((int)blockIdx.x < groups) tile_dealt_body<F, RT>(W, ws, Y, a, blockIdx.x, groups);
+  else tile_dealt_body<G, RT>(V, ws, Z, b, blockIdx.x - groups, gridDim.x - groups);
+}
+
 static inline size_t ts_chunk_bytes(int rt, bool off, int pc) {
   return (size_t)16 * rt * (256 * pc + 16) + (size_t)(8 * pc * 16 * rt + 2 * pc * 16) * 4 * (off ? 2 : 1);
 }
@@ -787,23 +800,47 @@ static int ts_launch(const TsCall& c, int ks, hipStream_t stream) {
   }
 }
 
+// what the kernel is told of a product, and the LDS that it takes
 template <class F, int RT>
-static int ts_dealt_launch(const TsCall& c, hipStream_t stream) {
-  if (c.M > 16 * RT || c.row_blocks != 1) return GGUF_NOT_TAKEN;
+static TsArgs ts_dealt_args(const TsCall& c, size_t& lds) {
   const int np = (c.K + 255) / 256, qk = F::KQ ? 256 : 32, bs = F::KQ ? F::PB : F::PB / 8;
   const int64_t pitch = c.w_pitch ? c.w_pitch : (int64_t)(c.K / qk) * bs;
   const bool aligned = F::PB % 16 == 0 && pitch % 16 == 0 && (uintptr_t)c.W % 16 == 0;
   const int ppr = (aligned ? F::PB / 16 : (F::PB + 29) / 16) | 1;   // (odd: banks)
-  size_t lds = (size_t)TS_NW * ts_dealt_place<F, RT>(ppr, (c.M + 3) / 4) + 16 + TsTable<F>::value;
+  lds = (size_t)TS_NW * ts_dealt_place<F, RT>(ppr, (c.M + 3) / 4) + 16 + TsTable<F>::value;
   if (lds < (size_t)TS_NW * RT * 1024) lds = (size_t)TS_NW * RT * 1024;
+  return {c.M, c.N, c.K, (int)q8_kp(c.K), (uint32_t)pitch, (uint32_t)q8_row_bytes(c.K), np, 3, ppr, 0, 0, 1, (uint32_t)((0x100000000ull + ppr - 1) / ppr), 0, 0, 0, 0, 0,
+          c.gemv_sums ? 2 : 1, c.dtype, c.ldy ? c.ldy : (int64_t)c.N, c.bias};
+}
+template <class F, int RT>
+static int ts_dealt_launch(const TsCall& c, hipStream_t stream) {
+  if (c.M > 16 * RT || c.row_blocks != 1) return GGUF_NOT_TAKEN;
+  size_t lds;
+  const TsArgs a = ts_dealt_args<F, RT>(c, lds);
   if (lds > 160 * 1024) return GGUF_NOT_TAKEN;
   auto kern = tile_dealt_kernel<F, RT>;
   static std::atomic<uint64_t> done{0};
   if (lds > 64 * 1024) allow_large_lds(kern, 160 * 1024, done);
-  const TsArgs a = {c.M, c.N, c.K, (int)q8_kp(c.K), (uint32_t)pitch, (uint32_t)q8_row_bytes(c.K), np, 3, ppr, 0, 0, 1, (uint32_t)((0x100000000ull + ppr - 1) / ppr), 0, 0, 0, 0, 0,
-                    c.gemv_sums ? 2 : 1, c.dtype, c.ldy ? c.ldy : (int64_t)c.N, c.bias};
   hipLaunchKernelGGL(kern, dim3((unsigned)((c.N + 15) / 16)), dim3(64 * TS_NW), lds, stream, (const uint8_t*)c.W, (const char*)c.ws, c.Y, a);
   return launch_status();
+}
+template <class F, class G, int RT>
+static int ts_dealt_pair_launch(const TsCall& c, const TsCall& d, hipStream_t stream) {
+  size_t lds, lds2;
+  const TsArgs a = ts_dealt_args<F, RT>(c, lds), b = ts_dealt_args<G, RT>(d, lds2);
+  if (lds < lds2) lds = lds2;
+  if (lds > 160 * 1024) return GGUF_NOT_TAKEN;
+  auto kern = tile_dealt_pair_kernel<F, G, RT>;
+  static std::atomic<uint64_t> done{0};
+  if (lds > 64 * 1024) allow_large_lds(kern, 160 * 1024, done);
+  const int groups = (c.N + 15) / 16;
+  hipLaunchKernelGGL(kern, dim3((unsigned)groups + (unsigned)((d.N + 15) / 16)), dim3(64 * TS_NW), lds, stream, (const uint8_t*)c.W, (const uint8_t*)d.W, (const char*)c.ws,
+                     c.Y, d.Y, a, b, groups);
+  return launch_status();
+}
+template <class F, class G>
+static int ts_dealt_pair(const TsCall& c, const TsCall& d, hipStream_t s) {
+  return c.M <= 16 ? ts_dealt_pair_launch<F, G, 1>(c, d, s) : ts_dealt_pair_launch<F, G, 2>(c, d, s);
 }
 
 template <class F, int RT>

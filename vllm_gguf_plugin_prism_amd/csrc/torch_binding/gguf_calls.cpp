@@ -284,6 +284,19 @@ PyObject* merged_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const gguf_stream_t stream = stream_of(dev);
     char* dst = (char*)y.mutable_data_ptr();
     const char* b = bias ? (const char*)bias->const_data_ptr() : nullptr;
+    // two matrices on the kernels of a few rows: x is quantized once, and they run side by side
+    const bool gemv = parts[0].path == PATH_MMVQ;
+    const auto pitch_of = [&](const Part& p) { return w->size(0) > 1 ? w->stride(0) : p.rb; };
+    if (parts.size() == 2 && m <= 32 && parts[0].path == parts[1].path && (gemv || parts[0].path == PATH_MMQ) &&
+        gguf_linear_two_takes((int)parts[0].type, parts[0].end - parts[0].start, pitch_of(parts[0]), (int)parts[1].type, parts[1].end - parts[1].start, pitch_of(parts[1]), k, m, gemv)) {
+      const Part &p = parts[0], &q = parts[1];
+      const int64_t rows = p.end - p.start;
+      const c10::DataPtr ws = scratch(m * gguf_q8_1_row_bytes(k));
+      rc = gguf_linear_two((const char*)w->const_data_ptr() + p.start * pitch_of(p), pitch_of(p), (int)p.type, rows, dst, b,
+                           (const char*)w->const_data_ptr() + q.start * pitch_of(q), pitch_of(q), (int)q.type, q.end - q.start, dst + rows * esz, b ? b + rows * esz : nullptr,
+                           x->const_data_ptr(), dtype_code(x->scalar_type()), ws.get(), width, k, m, gemv, stream);
+      parts.clear();
+    }
     for (const Part& p : parts) {
       const int64_t rows = p.end - p.start;
       const int64_t pitch = w->size(0) > 1 ? w->stride(0) : p.rb;
