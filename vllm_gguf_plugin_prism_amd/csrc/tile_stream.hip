@@ -109,25 +109,29 @@ static double ts_most_work(int type) {
 
 // Where the panels of a column group are dealt to the waves of a workgroup (tile_dealt_kernel) instead.  Against whatever ran before (the
 // streaming tiles, the kernel of the packed blocks, the staged 16-row tiles, the GEMV), over 7900 random products of 5 .. 32 rows, N 256 ..
-// 28672, K 512 .. 18944, both operators: where these lines take it 1.28 times as fast on average, over all 1.21 (Q2_K 1.30, Q3_K 1.27, Q4_1 1.22,
-// Q4_K, Q6_K, Q8_0, Q4_0 1.20, Q5_K, Q5_0 1.16, IQ4_XS 1.25, IQ2 and IQ3 1.16 to 1.19), 0.9 % short of always taking the faster; one in sixty is
-// slower by more than 3 %, the worst by 20 %.  us, before / dealt: [4096,4096] 12 rows Q4_K 11.0 / 8.4, Q6_K 12.5 / 10.0, [4096,14336] 12 rows Q6_K
-// 25.4 / 18.9, [2048,2048] Q4_K 8.5 / 6.7.
+// 28672, K 512 .. 18944, both operators, with one column group per workgroup: where these lines take it 1.28 times as fast on average, over all 1.21
+// (Q2_K 1.30, Q3_K 1.27, Q4_1 1.22, Q4_K, Q6_K, Q8_0, Q4_0 1.20, Q5_K, Q5_0 1.16, IQ4_XS 1.25, IQ2 and IQ3 1.16 to 1.19); one in sixty is slower by more
+// than 3 %, the worst by 20 %.  With several, 17 .. 32 rows and more than 4096 columns are 1.11 times as fast again (700 products; up to 1.5).  us, before
+// / dealt: [4096,4096] 12 rows Q4_K 11.0 / 8.4, Q6_K 12.5 / 10.0, [4096,14336] 12 rows Q6_K 25.4 / 18.9, [2048,2048] Q4_K 8.5 / 6.7.
 static bool ts_dealt_takes(int type, int64_t M, int64_t N, int64_t K) {
   if (M < 5 || M > 32 || N > 0x7FFFFFF0ll || K > 0x7FFFFFF0ll) return false;
   const int64_t groups = (N + 15) / 16, np = (K + 255) / 256;
   // (a long K on few columns is cut between workgroups by the kernel of the packed blocks: [832,15872] Q6_K 11 rows 13.9 / 17.0)
   if ((type == T_Q4_K || type == T_Q5_K || type == T_Q6_K) && groups <= 56 && K > 13000) return false;
-  // two tiles of rows leave room for one workgroup per CU: one round, or rows long enough to be worth a beginning
-  if (M > 16) return groups <= 256 || (K >= 4096 && groups <= 768);
+  if (type == T_Q2_K && M > 16) return groups <= 256 || (K >= 4096 && groups <= 768);
   const bool blocks32 = type == T_Q4_0 || type == T_Q4_1 || type == T_Q5_0 || type == T_Q5_1 || type == T_Q8_0 || type == T_IQ4_NL;
+  const bool halves = type == T_Q4_1 || type == T_Q5_1;
+  // Two tiles of rows: workgroups of several groups (ts_dealt_groups); past two groups rows must be long enough for the sum at their end.  us, the
+  // streaming tiles / dealt, 20 rows: [14336,1536] Q4_K 10.4 / 8.7, [28672,1536] 14.0 / 14.2, [18944,4096] 27.3 / 19.5, [65536,4096] 58.4 / 55.1;
+  // Q8_0 [19008,2304] 24.0 / 25.4; Q5_K, at most four groups, [25728,3328] 29.2 / 33.0
+  if (M > 16) return groups <= 512 || (K >= 1024 && K >= (halves ? 2 * groups - 512 : blocks32 || type == T_Q5_K ? 4 * groups - 2048 : groups + groups / 4));
   // Every group reads the activations again: past 1536 of them the waves with columns of their own are ahead ([28672,4096] Q4_K, 16 rows
   // 21.5 / 24.5) unless K is too long for their LDS; and two panels per row are work for two waves of eight.
   if (!blocks32) return (groups <= 1536 && groups <= 256 * np) || K >= 12000;
   // (these decode more per panel, or keep two values per block and row: the beginning weighs less there)
-  if (M >= 9) return groups <= 512 || K >= 4096;
+  if (M >= 9) return groups <= 512 || K >= 4096 || (halves && K >= 2 * groups - 512);
   // the GEMV, one launch, is ahead on short rows, with Q5_0 and Q8_0 on small matrices ([480,2336] Q8_0 5 rows 5.4 / 6.9)
-  if (type == T_Q4_1 || type == T_Q5_1) return K >= 2048 && (groups <= 512 || K >= 8192);
+  if (halves) return K >= 2048 && (groups <= 512 || K >= 4096);
   return K >= 2048 && (N * K > 3000000 || (type != T_Q5_0 && type != T_Q8_0));
 }
 

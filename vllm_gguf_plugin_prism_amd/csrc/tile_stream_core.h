@@ -552,13 +552,17 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
 // What bounds it is the weight stream, and beside it the activations' way to every workgroup (2.3 us of [4096,14336]'s 15) and the
 // vector instructions of a panel (Q6_K 350: 5 us).  Without the quantizer's launch, us, streaming tiles / this, 12 rows: Q6_K [4096,14336]
 // 22.1 / 15.1, [4096,4096] 9.6 / 7.1, [1024,4096] 8.5 / 5.9; Q4_K [4096,14336] 16.9 / 11.7, [11008,4096] 13.4 / 10.7, [2048,2048] 5.8 / 4.0; 24
-// rows Q6_K [4096,14336] 29.5 / 25.0, [4096,4096] 11.5 / 8.9.  Tried and slower: workgroups that stay and walk several column groups, the
-// next one's first panel under way over the sum (0.86 to 1.06 times the speed: the addresses cost more than the beginning).
+// rows Q6_K [4096,14336] 29.5 / 25.0, [4096,4096] 11.5 / 8.9.
+// CG: up to so many column groups of a workgroup (ts_dealt_groups), a panel of K after the other: the activations' operands and block scales stay
+// in registers over the groups (the scales as the halves that they are), a group's panel is asked for while the one before is multiplied, and
+// there is one beginning and one sum for all.  From two on the groups are walked by a loop that is not unrolled, which moves the partial tiles
+// around by one each time: unrolled the compiler keeps more than there are registers.  Tried and slower: whole column groups one after the other,
+// the activations fetched again for each (0.86 to 1.06 times the speed of a workgroup each).
 template <class F, int RT> __host__ __device__ constexpr int ts_dealt_place(int ppr, int xn) { return 256 * ppr + 1024 * RT + 1024 * xn; }
 // (two workgroups of one tile of rows share a CU where its registers suffice)
 template <class F, int RT> constexpr int ts_dealt_waves() { return RT == 1 && !F::HALVES && (F::KQ || F::OFF != 1) ? 4 : 2; }
-template <class F, int RT>
-__device__ __forceinline__ void tile_dealt_body(const uint8_t* __restrict__ W, const char* __restrict__ ws, void* __restrict__ Y, const TsArgs& a, int wg, int groups) {
+template <class F, int RT, int CG>
+__device__ __forceinline__ void tile_dealt_body(const uint8_t* __restrict__ W, const char* __restrict__ ws, void* __restrict__ Y, const TsArgs& a, int wg, int wgs) {
   constexpr int NW = TS_NW;
   constexpr bool SUMS = ts_sums<F>(), OFFSET = F::OFF == 1;
   constexpr int PPR_MIN = (F::PB + 15) / 16, PPR_MAX = (F::PB + 29) / 16;
@@ -566,8 +570,9 @@ __device__ __forceinline__ void tile_dealt_body(const uint8_t* __restrict__ W, c
   extern __shared__ __align__(16) char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
-  const int total8 = groups & ~7;                           // each of the 8 XCDs gets a contiguous run of workgroups
+  const int total8 = wgs & ~7;                              // each of the 8 XCDs gets a contiguous run of workgroups
   if (wg < total8) wg = (wg & 7) * (total8 >> 3) + (wg >> 3);
+  const int ng = CG > 2 ? a.passes : CG;                    // column groups, the last of the last workgroup perhaps behind the matrix
   const int xn = (a.M + 3) >> 2;                            // fetches of quants per panel, four rows each
   const int w_bytes = 256 * a.ppr, place = ts_dealt_place<F, RT>(a.ppr, xn);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
@@ -577,29 +582,20 @@ __device__ __forceinline__ void tile_dealt_body(const uint8_t* __restrict__ W, c
   const uint8_t* const wbase = W - wmis;
   const uint32_t row_bytes = (uint32_t)(F::KQ ? a.np * F::PB : (a.K >> 5) * (F::PB / 8));
   const uint32_t last16 = ((uint32_t)(a.N - 1) * a.w_pitch + wmis + row_bytes - 1) & ~15u;   // the last granule that holds bytes of W
-  uint32_t w_row[NI], pc16[NI];                             // where the piece's row begins; the piece
+  uint32_t w_at[NI];                                        // the piece behind its row's beginning
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int p = min(64 * i + lane, 16 * a.ppr - 1);
     const uint32_t r = __umulhi((uint32_t)p, a.ppr_inv);
-    w_row[i] = (uint32_t)min(16 * wg + (int)r, a.N - 1) * a.w_pitch + wmis;
-    pc16[i] = (uint32_t)min(p - (int)r * a.ppr, PPR_MAX - 1) * 16;   // (the piece that only spaces rows: the last again)
+    w_at[i] = (uint32_t)min(16 * ng * wg + (int)r, a.N - 1) * a.w_pitch + wmis +
+              (uint32_t)min(p - (int)r * a.ppr, PPR_MAX - 1) * 16;   // (the piece that only spaces rows: the last again)
   }
-  uint32_t x_at[4 * RT], s_at[RT];
-#pragma unroll
-  for (int i = 0; i < 4 * RT; ++i) {
-    const int row = 4 * i + g;
-    x_at[i] = (uint32_t)min(row, a.M - 1) * a.ws_row_bytes + 16 * (uint32_t)(c ^ (row & 15));
-  }
-  // (a lane: half of a row's eight scales, in the upper half of the lanes of its sums)
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-    s_at[rt] = (uint32_t)min(16 * rt + ((lane & 31) >> 1), a.M - 1) * a.ws_row_bytes + (uint32_t)a.Kp + 16 * (lane & 1) + (SUMS && lane >= 32 ? 4 * a.plane * (a.Kp >> 5) : 0);
-  const auto request = [&](int p) {
-    const uint32_t to = lds0 + mine, off = (uint32_t)(p * F::PB);
+  const uint32_t step = 16 * a.w_pitch;                     // (a group behind the last column reads the last granule again)
+  const auto request_w = [&](int p, int j) {
+    const uint32_t to = lds0 + mine, off = (uint32_t)(p * F::PB) + (uint32_t)j * step;
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const uint32_t v = min(((w_row[i] + off) & ~15u) + pc16[i], last16);
+      const uint32_t v = min((w_at[i] + off) & ~15u, last16);
       if (i < FULL) {
         ts_fetch(v, wbase, to + 1024 * i);
       } else {   // (lanes past the panel's last piece stay out: their bytes would land behind it)
@@ -607,13 +603,29 @@ __device__ __forceinline__ void tile_dealt_body(const uint8_t* __restrict__ W, c
         ts_fetch_some(v, wbase, to + 1024 * i, on >= 64 ? ~0ull : on <= 0 ? 0ull : (1ull << on) - 1);
       }
     }
+  };
+  const auto request_x = [&](int p) {
+    const uint32_t to = lds0 + mine + w_bytes;
+    int l = lane;                                           // (opaque: computed every time, not kept in registers over the groups)
+    if constexpr (CG > 1) asm volatile("" : "+v"(l));
+    const int c = l & 15, g = l >> 4;
+  uint32_t x_at[4 * RT], s_at[RT];
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) ts_fetch(s_at[rt] + 32 * (uint32_t)p, ws, to + w_bytes + 1024 * rt);
+    for (int i = 0; i < 4 * RT; ++i) {
+      const int row = 4 * i + g;
+      x_at[i] = (uint32_t)min(row, a.M - 1) * a.ws_row_bytes + 16 * (uint32_t)(c ^ (row & 15));
+    }
+    // (a lane: half of a row's eight scales, in the upper half of the lanes of its sums)
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+      s_at[rt] = (uint32_t)min(16 * rt + ((l & 31) >> 1), a.M - 1) * a.ws_row_bytes + (uint32_t)a.Kp + 16 * (l & 1) + (SUMS && l >= 32 ? 4 * a.plane * (a.Kp >> 5) : 0);
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) ts_fetch(s_at[rt] + 32 * (uint32_t)p, ws, to + 1024 * rt);
 #pragma unroll
     for (int i = 0; i < 4 * RT; ++i)
-      if (i < xn) ts_fetch(x_at[i] + 256 * (uint32_t)p, ws, to + w_bytes + 1024 * RT + 1024 * i);
+      if (i < xn) ts_fetch(x_at[i] + 256 * (uint32_t)p, ws, to + 1024 * RT + 1024 * i);
   };
-  if (wave < a.np) request(wave);
+  if (wave < a.np) { request_w(wave, 0); request_x(wave); }
   if constexpr (TsTable<F>::value) {
     F::tables(smem + table_off);
     __syncthreads();
@@ -621,23 +633,23 @@ __device__ __forceinline__ void tile_dealt_body(const uint8_t* __restrict__ W, c
 
   const uint32_t half0 = g < 2 ? ~0u : 0u;                  // lanes that hold the first 16 values of a block
   const int nkb = a.K >> 5;
-  f32x4 acc[RT];
+  f32x4 acc[CG][RT];
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) acc[rt] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+  for (int j = 0; j < CG; ++j)
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) acc[j][rt] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
   const char* const at = smem + mine;
   const char* const scales = at + w_bytes;
-  const uint32_t w_lane = (uint32_t)min(16 * wg + c, a.N - 1) * a.w_pitch + wmis;
+  const uint32_t w_lane = (uint32_t)min(16 * ng * wg + c, a.N - 1) * a.w_pitch + wmis;
   for (int p = wave; p < a.np; p += NW) {
     const int left = nkb - 8 * p;                           // blocks of the panel inside the row
     ts_wait<0>();
-    F w;
-    if constexpr (TsTable<F>::value) w.tab = smem + table_off;
-    w.read(at + c * (16 * a.ppr), F::PB % 16 == 0 && a.ppr == F::PB / 16 ? 0u : (w_lane + (uint32_t)(p * F::PB)) & 15, g);
     u32x4_s xa[RT][4];
     float so[RT][2];
     // of rows 4 g + r, blocks 0 .. 7: the block scales, or, with HALVES, (scale, sum) as the halves that they are (behind a row's last
     // block lie the quantizer's zeros)
-    float d8[RT][4][8];
+    float d8[RT][4][CG > 1 && !F::HALVES ? 1 : 8];
+    uint32_t d8h[RT][4][4];                                  // CG > 1: as the halves that they are
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
 #pragma unroll
@@ -653,6 +665,10 @@ __device__ __forceinline__ void tile_dealt_body(const uint8_t* __restrict__ W, c
           const f32x4 v = *(const f32x4*)(scales + 1024 * rt + 32 * (4 * g + r) + 16 * h);
           f32x4 z = v;
           if constexpr (F::HALVES) z = *(const f32x4*)(scales + 1024 * rt + 512 + 32 * (4 * g + r) + 16 * h);
+          if constexpr (CG > 1 && !F::HALVES) {
+            d8h[rt][r][2 * h] = __builtin_bit_cast(uint32_t, (ts_h2){(_Float16)v[0], (_Float16)v[1]});
+            d8h[rt][r][2 * h + 1] = __builtin_bit_cast(uint32_t, (ts_h2){(_Float16)v[2], (_Float16)v[3]});
+          } else
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             if constexpr (F::HALVES) d8[rt][r][4 * h + e] = __builtin_bit_cast(float, (ts_h2){(_Float16)v[e], (_Float16)z[e]});
@@ -660,47 +676,70 @@ __device__ __forceinline__ void tile_dealt_body(const uint8_t* __restrict__ W, c
           }
         }
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // the place may be filled again
-    if (p + NW < a.np) request(p + NW);
     const auto of = [&](int rt, int b, int half) {
       f32x4 o;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         if constexpr (F::HALVES) o[r] = (float)__builtin_bit_cast(ts_h2, d8[rt][r][b])[half];
+        else if constexpr (CG > 1) o[r] = (float)__builtin_bit_cast(ts_h2, d8h[rt][r][b >> 1])[b & 1];
         else o[r] = d8[rt][r][b];
       }
       return o;
     };
-    ts_multiply<F, RT>(w, xa, so, left, g, half0, [&](int rt, int b) { return of(rt, b, 0); }, [&](int rt, int b) { return of(rt, b, 1); }, acc);
+#pragma unroll 1
+    for (int j = 0; j < ng; ++j) {
+      if (j > 0) ts_wait<0>();
+      F w;                                                  // (read behind the activations: before them Q6_K spills, and loses a tenth)
+      if constexpr (TsTable<F>::value) w.tab = smem + table_off;
+      w.read(at + c * (16 * a.ppr), F::PB % 16 == 0 && a.ppr == F::PB / 16 ? 0u : (w_lane + (uint32_t)(p * F::PB) + (uint32_t)j * step) & 15, g);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");    // the place may be filled again
+      if (j + 1 < ng) request_w(p, j + 1);
+      else if (p + NW < a.np) { request_w(p + NW, 0); request_x(p + NW); }
+      ts_multiply<F, RT>(w, xa, so, left, g, half0, [&](int rt, int b) { return of(rt, b, 0); }, [&](int rt, int b) { return of(rt, b, 1); }, acc[0]);
+      if constexpr (CG > 1) {                               // (the next group's tile first: a tile by number would be in scratch)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+          const f32x4 done = acc[0][rt];
+#pragma unroll
+          for (int i = 0; i < CG; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[i][rt][r] = i + 1 == ng || i + 1 == CG ? done[r] : acc[i + 1 < CG ? i + 1 : i][rt][r];
+        }
+      }
+    }
   }
 
   // ---- the eight partial tiles, added in the order of the waves
   __syncthreads();
-  float* const red = (float*)smem;                          // [NW][RT][64] of four floats, over the panels
+  float* const red = (float*)smem;                          // [NW][CG][RT][64] of four floats, over the panels
+  constexpr int T = CG * RT;
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) *(f32x4*)(red + ((wave * RT + rt) * 64 + lane) * 4) = acc[rt];
+  for (int j = 0; j < CG; ++j)
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) *(f32x4*)(red + ((wave * T + j * RT + rt) * 64 + lane) * 4) = acc[j][rt];
   __syncthreads();
-  if (tid < 256 * RT) {
-    const int n = tid & 15, m = tid >> 4, l = 16 * ((m >> 2) & 3) + n, rt = m >> 4;   // result row m, feature n of the group
-    float v = red[(rt * 64 + l) * 4 + (m & 3)];
+  for (int i = tid; i < 256 * RT * ng; i += 64 * NW) {
+    const int n = i & 15, m = (i >> 4) % (16 * RT), j = i / (256 * RT), l = 16 * ((m >> 2) & 3) + n, t = j * RT + (m >> 4);   // result row m, feature n of group j
+    float v = red[(t * 64 + l) * 4 + (m & 3)];
 #pragma unroll
-    for (int z = 1; z < NW; ++z) v += red[((z * RT + rt) * 64 + l) * 4 + (m & 3)];
-    if (m < a.M && 16 * wg + n < a.N) ts_store(Y, (int64_t)m * a.ldy + 16 * wg + n, v, a.bias, 16 * wg + n, a.dtype);
+    for (int z = 1; z < NW; ++z) v += red[((z * T + t) * 64 + l) * 4 + (m & 3)];
+    const int col = 16 * (ng * wg + j) + n;
+    if (m < a.M && col < a.N) ts_store(Y, (int64_t)m * a.ldy + col, v, a.bias, col, a.dtype);
   }
 }
 
-template <class F, int RT>
+template <class F, int RT, int CG>
 __global__ __launch_bounds__(64 * TS_NW, (ts_dealt_waves<F, RT>())) void tile_dealt_kernel(const uint8_t* __restrict__ W, const char* __restrict__ ws, void* __restrict__ Y, TsArgs a) {
-  tile_dealt_body<F, RT>(W, ws, Y, a, blockIdx.x, gridDim.x);
+  tile_dealt_body<F, RT, CG>(W, ws, Y, a, blockIdx.x, gridDim.x);
 }
 
 // The same for two matrices with the same rows of X, those of a merged layer whose recipe gives one of its tensors more bits: the
 // workgroups of the second, often too few for the chip by themselves, run beside the first's, and a launch less.
-template <class F, class G, int RT>
+template <class F, class G, int RT, int CG>
 __global__ __launch_bounds__(64 * TS_NW, (ts_dealt_waves<F, RT>() < ts_dealt_waves<G, RT>() ? ts_dealt_waves<F, RT>() : ts_dealt_waves<G, RT>())) void tile_dealt_pair_kernel(
-    const uint8_t* __restrict__ W, const uint8_t* __restrict__ V, const char* __restrict__ ws, void* __restrict__ Y, void* __restrict__ Z, TsArgs a, TsArgs b, int groups) {
-  if ((int)blockIdx.x < groups) tile_dealt_body<F, RT>(W, ws, Y, a, blockIdx.x, groups);
-  else tile_dealt_body<G, RT>(V, ws, Z, b, blockIdx.x - groups, gridDim.x - groups);
+    const uint8_t* __restrict__ W, const uint8_t* __restrict__ V, const char* __restrict__ ws, void* __restrict__ Y, void* __restrict__ Z, TsArgs a, TsArgs b, int wgs) {
+  if ((int)blockIdx.x < wgs) tile_dealt_body<F, RT, CG>(W, ws, Y, a, blockIdx.x, wgs);
+  else tile_dealt_body<G, RT, CG>(V, ws, Z, b, blockIdx.x - wgs, gridDim.x - wgs);
 }
 
 static inline size_t ts_chunk_bytes(int rt, bool off, int pc) {
@@ -800,47 +839,80 @@ static int ts_launch(const TsCall& c, int ks, hipStream_t stream) {
   }
 }
 
+// How many column groups a workgroup takes.  Where one of them fills a CU (two tiles of rows, or formats that need the registers), as many as
+// let one round do, up to what the registers hold: [11008,4096] Q4_K 20 rows, one to four groups 16.1 / 16.8 / 12.2 / 13.8 us, [28672,4096]
+// 35.5 / 32.3 / 32.2 / 27.5, eight 25.9.  Where two share a CU, two groups only between one and a half rounds and two: [16384,4096] Q4_K 12 rows 14.3 /
+// 12.6, [12288,4096] Q6_K 17.4 / 18.9.  (Q2_K, two products per block, spills, Q5_K at eight.)
+template <class F, int RT> constexpr int ts_dealt_most() { return F::OFF == 2 ? 1 : ts_dealt_waves<F, RT>() == 4 ? 2 : RT == 2 && F::KQ && !std::is_same<F, TQ5_K>::value ? 8 : 4; }
+template <class F, int RT>
+static inline int ts_dealt_groups(int groups) {
+  constexpr int MOST = ts_dealt_most<F, RT>();
+  if (MOST == 2) return groups > 768 && groups <= 1024 ? 2 : 1;
+  const int rounds = (groups + 256 * MOST - 1) / (256 * MOST);
+  return MOST == 1 ? 1 : (groups + 256 * rounds - 1) / (256 * rounds);
+}
 // what the kernel is told of a product, and the LDS that it takes
 template <class F, int RT>
-static TsArgs ts_dealt_args(const TsCall& c, size_t& lds) {
+static TsArgs ts_dealt_args(const TsCall& c, int ng, size_t& lds) {
   const int np = (c.K + 255) / 256, qk = F::KQ ? 256 : 32, bs = F::KQ ? F::PB : F::PB / 8;
   const int64_t pitch = c.w_pitch ? c.w_pitch : (int64_t)(c.K / qk) * bs;
   const bool aligned = F::PB % 16 == 0 && pitch % 16 == 0 && (uintptr_t)c.W % 16 == 0;
   const int ppr = (aligned ? F::PB / 16 : (F::PB + 29) / 16) | 1;   // (odd: banks)
   lds = (size_t)TS_NW * ts_dealt_place<F, RT>(ppr, (c.M + 3) / 4) + 16 + TsTable<F>::value;
-  if (lds < (size_t)TS_NW * RT * 1024) lds = (size_t)TS_NW * RT * 1024;
-  return {c.M, c.N, c.K, (int)q8_kp(c.K), (uint32_t)pitch, (uint32_t)q8_row_bytes(c.K), np, 3, ppr, 0, 0, 1, (uint32_t)((0x100000000ull + ppr - 1) / ppr), 0, 0, 0, 0, 0,
+  const int tiles = RT * (ng > 4 ? 8 : ng > 2 ? 4 : ng);    // (the sum's places are laid out for the most that an instance takes)
+  if (lds < (size_t)TS_NW * tiles * 1024) lds = (size_t)TS_NW * tiles * 1024;
+  return {c.M, c.N, c.K, (int)q8_kp(c.K), (uint32_t)pitch, (uint32_t)q8_row_bytes(c.K), np, 3, ppr, 0, 0, ng, (uint32_t)((0x100000000ull + ppr - 1) / ppr), 0, 0, 0, 0, 0,
           c.gemv_sums ? 2 : 1, c.dtype, c.ldy ? c.ldy : (int64_t)c.N, c.bias};
+}
+template <class F, int RT, int CG>
+static int ts_dealt_launch_cg(const TsCall& c, int ng, hipStream_t stream) {
+  size_t lds;
+  const TsArgs a = ts_dealt_args<F, RT>(c, ng, lds);
+  if (lds > 160 * 1024) return GGUF_NOT_TAKEN;
+  auto kern = tile_dealt_kernel<F, RT, CG>;
+  static std::atomic<uint64_t> done{0};
+  if (lds > 64 * 1024) allow_large_lds(kern, 160 * 1024, done);
+  hipLaunchKernelGGL(kern, dim3((unsigned)((c.N + 16 * ng - 1) / (16 * ng))), dim3(64 * TS_NW), lds, stream, (const uint8_t*)c.W, (const char*)c.ws, c.Y, a);
+  return launch_status();
 }
 template <class F, int RT>
 static int ts_dealt_launch(const TsCall& c, hipStream_t stream) {
   if (c.M > 16 * RT || c.row_blocks != 1) return GGUF_NOT_TAKEN;
-  size_t lds;
-  const TsArgs a = ts_dealt_args<F, RT>(c, lds);
+  constexpr int MOST = ts_dealt_most<F, RT>();
+  const int ng = ts_dealt_groups<F, RT>((c.N + 15) / 16);
+  if (ng == 1) return ts_dealt_launch_cg<F, RT, 1>(c, 1, stream);
+  if constexpr (MOST >= 2) {
+    if (ng == 2) return ts_dealt_launch_cg<F, RT, 2>(c, 2, stream);
+  }
+  if constexpr (MOST >= 4) {
+    if (ng <= 4) return ts_dealt_launch_cg<F, RT, 4>(c, ng, stream);
+  }
+  if constexpr (MOST == 8) return ts_dealt_launch_cg<F, RT, 8>(c, ng, stream);
+  return GGUF_NOT_TAKEN;
+}
+template <class F, class G, int RT, int CG>
+static int ts_dealt_pair_launch(const TsCall& c, const TsCall& d, hipStream_t stream) {
+  size_t lds, lds2;
+  const TsArgs a = ts_dealt_args<F, RT>(c, CG, lds), b = ts_dealt_args<G, RT>(d, CG, lds2);
+  if (lds < lds2) lds = lds2;
   if (lds > 160 * 1024) return GGUF_NOT_TAKEN;
-  auto kern = tile_dealt_kernel<F, RT>;
+  auto kern = tile_dealt_pair_kernel<F, G, RT, CG>;
   static std::atomic<uint64_t> done{0};
   if (lds > 64 * 1024) allow_large_lds(kern, 160 * 1024, done);
-  hipLaunchKernelGGL(kern, dim3((unsigned)((c.N + 15) / 16)), dim3(64 * TS_NW), lds, stream, (const uint8_t*)c.W, (const char*)c.ws, c.Y, a);
+  const int wgs = (c.N + 16 * CG - 1) / (16 * CG);
+  hipLaunchKernelGGL(kern, dim3((unsigned)wgs + (unsigned)((d.N + 16 * CG - 1) / (16 * CG))), dim3(64 * TS_NW), lds, stream, (const uint8_t*)c.W, (const uint8_t*)d.W,
+                     (const char*)c.ws, c.Y, d.Y, a, b, wgs);
   return launch_status();
 }
 template <class F, class G, int RT>
-static int ts_dealt_pair_launch(const TsCall& c, const TsCall& d, hipStream_t stream) {
-  size_t lds, lds2;
-  const TsArgs a = ts_dealt_args<F, RT>(c, lds), b = ts_dealt_args<G, RT>(d, lds2);
-  if (lds < lds2) lds = lds2;
-  if (lds > 160 * 1024) return GGUF_NOT_TAKEN;
-  auto kern = tile_dealt_pair_kernel<F, G, RT>;
-  static std::atomic<uint64_t> done{0};
-  if (lds > 64 * 1024) allow_large_lds(kern, 160 * 1024, done);
-  const int groups = (c.N + 15) / 16;
-  hipLaunchKernelGGL(kern, dim3((unsigned)groups + (unsigned)((d.N + 15) / 16)), dim3(64 * TS_NW), lds, stream, (const uint8_t*)c.W, (const uint8_t*)d.W, (const char*)c.ws,
-                     c.Y, d.Y, a, b, groups);
-  return launch_status();
+static int ts_dealt_pair_rt(const TsCall& c, const TsCall& d, hipStream_t s) {
+  const int ng = ts_dealt_groups<F, RT>((c.N + 15) / 16 + (d.N + 15) / 16);
+  if (ng > 2) return GGUF_NOT_TAKEN;                        // (each by itself: as many groups as suit it)
+  return ng == 1 ? ts_dealt_pair_launch<F, G, RT, 1>(c, d, s) : ts_dealt_pair_launch<F, G, RT, 2>(c, d, s);
 }
 template <class F, class G>
 static int ts_dealt_pair(const TsCall& c, const TsCall& d, hipStream_t s) {
-  return c.M <= 16 ? ts_dealt_pair_launch<F, G, 1>(c, d, s) : ts_dealt_pair_launch<F, G, 2>(c, d, s);
+  return c.M <= 16 ? ts_dealt_pair_rt<F, G, 1>(c, d, s) : ts_dealt_pair_rt<F, G, 2>(c, d, s);
 }
 
 template <class F, int RT>
