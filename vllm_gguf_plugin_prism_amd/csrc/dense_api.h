@@ -15,8 +15,8 @@
  * gguf_moe_mmq_layer with the workspace it asks for, at addresses divisible by 16, runs on the wide tiles.
  *
  * gguf_linear_two: two products of the same x, up to 32 rows, as two calls of gguf_mmvq_linear (gemv) or gguf_mmq_linear would run them
- * (the same results bit for bit), x quantized once and, for most pairs of types that recipes mix, in one launch behind that: shards of a merged
- * layer, columns of one result of this row pitch.  The workspace, M * gguf_q8_1_row_bytes(K), begins on 16 bytes.
+ * (the same results bit for bit), and for pairs of types that recipes mix in one launch: up to four rows of the GEMV, from five on behind the
+ * quantizer's, which other pairs share too.  They are shards of a merged layer, columns of one result of this row pitch.  The workspace, M * gguf_q8_1_row_bytes(K), begins on 16 bytes.
  * gguf_linear_two_takes: 1 for a pair that it serves. */
 #pragma once
 #include <stdint.h>

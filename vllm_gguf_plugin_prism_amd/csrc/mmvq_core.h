@@ -397,7 +397,7 @@ static inline StreamGeom stream_geom(int N, int K, int rows_per_wg, int64_t w_pi
 // T(T(act(gate)) * up), the values a separate act-and-multiply kernel would have stored (fused_moe.py:44-51,80).
 template <class F, int MT, int NW, int D, typename T, bool TILE, bool FULL, int STAGED, bool GATED>
 __device__ __forceinline__ void mmvq_stream_body(const uint8_t* __restrict__ W, const T* __restrict__ X, T* __restrict__ Y,
-                                                 const T* __restrict__ bias, int64_t ldy, const StreamGeom& geom, int act_fn) {
+                                                 const T* __restrict__ bias, int64_t ldy, const StreamGeom& geom, int act_fn, int wg) {
   static_assert(!GATED || MT == 1, "the gated variant quantizes one row");
   extern __shared__ __align__(16) char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -415,7 +415,7 @@ __device__ __forceinline__ void mmvq_stream_body(const uint8_t* __restrict__ W, 
   constexpr bool HALF = STAGED == LANES_HALF, SPANS = STAGED != 0 && !HALF, DMA = STAGED == STAGED_DMA;
   constexpr int SPAN = SPANS ? SpanOf<F>::value : 0;
 
-  const int r_begin = blockIdx.x * rows_per_wg;   // (the host launches ceil(N / rows_per_wg) workgroups: r_begin < N)
+  const int r_begin = wg * rows_per_wg;     // (the host launches ceil(N / rows_per_wg) workgroups: r_begin < N)
   const int r_end = min(N, r_begin + rows_per_wg);
   const int nrows = r_end - r_begin;
   if (nrows > 0) GGUF_PHASE(5);                // kernel arguments have arrived
@@ -727,7 +727,7 @@ template <class F, int MT, int NW, int D, typename T, bool TILE = false, bool FU
 __global__ __launch_bounds__(64 * NW) void mmvq_stream_kernel(const uint8_t* __restrict__ W, const T* __restrict__ X,
                                                                T* __restrict__ Y, const T* __restrict__ bias, int64_t ldy,
                                                                StreamGeom geom) {
-  mmvq_stream_body<F, MT, NW, D, T, TILE, FULL, STAGED, false>(W, X, Y, bias, ldy, geom, ACT_NONE);
+  mmvq_stream_body<F, MT, NW, D, T, TILE, FULL, STAGED, false>(W, X, Y, bias, ldy, geom, ACT_NONE, blockIdx.x);
 }
 
 // The per-pair MoE operator on the same kernel (reference: csrc/gguf/moe_vec.cuh:3-53): blockIdx.y is the flat
@@ -747,7 +747,7 @@ __global__ __launch_bounds__(64 * NW) void mmvq_stream_moe_kernel(const uint8_t*
   const int e = moe.topk_ids[z];
   if (moe.num_experts > 0 && (e < 0 || e >= moe.num_experts)) return;
   mmvq_stream_body<F, 1, NW, D, T, false, true, STAGED, GATED>(W + (int64_t)e * moe.expert_bytes, X + (int64_t)(z / moe.top_k) * moe.x_pitch,
-                                                               Y + (int64_t)z * geom.N, nullptr, (int64_t)geom.N, geom, moe.act);
+                                                               Y + (int64_t)z * geom.N, nullptr, (int64_t)geom.N, geom, moe.act, blockIdx.x);
 }
 
 // Whether the rows of W are whole 16-byte pieces at 16-byte aligned addresses.  Q3_K and Q6_K, whose rows are that only

@@ -44,6 +44,9 @@ int ts_dense(int type, const void* W, const void* x, int dtype, void* workspace,
 struct TsShard { const void* W; void* Y; int type; int64_t N; LinearArgs la; };
 bool ts_two_takes(int type, int64_t N, int64_t w_pitch, int type2, int64_t N2, int64_t w_pitch2, int64_t K, int64_t M, bool gemv);
 int ts_two(const TsShard& a, const TsShard& b, const void* x, int dtype, void* workspace, int64_t M, int K, bool gemv, hipStream_t s);
+// the same for up to four rows on the streaming GEMV (mmvq_pair.hip): whether a pair is taken; the call, or GGUF_NOT_TAKEN
+bool mmvq_pair_takes(int type, int64_t N, int64_t w_pitch, int type2, int64_t N2, int64_t w_pitch2, int64_t K, int64_t M);
+int mmvq_pair(const TsShard& a, const TsShard& b, const void* x, int dtype, int K, int M, hipStream_t s);
 int ts_pair(int type, const TsCall& c, int type2, const TsCall& d, hipStream_t s);   // in one launch; GGUF_NOT_TAKEN for most types
 bool ts_layer_takes(int type13, int type2, int64_t H, int64_t I, int64_t N_out, int64_t tokens, int64_t top_k, int64_t num_experts);
 double ts_layer_gain(int type13, int type2, int64_t H, int64_t I, int64_t N_out, int64_t tokens, int64_t top_k, int64_t num_experts);

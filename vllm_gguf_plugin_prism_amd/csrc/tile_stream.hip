@@ -351,8 +351,13 @@ int ts_moe(const void* W, const void* ws, void* Y, int dtype, int type, int N, i
 
 }  // namespace gguf
 
+namespace gguf {
+int mmvq_any(int type, const void* W, const void* x, void* q8_workspace, void* Y, int xdtype, int64_t N, int64_t K, int64_t M, hipStream_t s, const LinearArgs& la);
+}  // namespace gguf
+
 extern "C" int gguf_linear_two_takes(int type, int64_t N, int64_t w_row_pitch_bytes, int type2, int64_t N2, int64_t w_row_pitch_bytes2, int64_t K, int64_t M, int gemv) {
   if (M < 1 || M > 32 || N <= 0 || N2 <= 0 || K <= 0) return 0;
+  if (M <= 4) return gemv && gguf::mmvq_pair_takes(type, N, w_row_pitch_bytes, type2, N2, w_row_pitch_bytes2, K, M);
   return gguf::ts_two_takes(type, N, w_row_pitch_bytes, type2, N2, w_row_pitch_bytes2, K, M, gemv != 0);
 }
 
@@ -367,9 +372,13 @@ extern "C" int gguf_linear_two(const void* W, int64_t w_row_pitch_bytes, int typ
   if (xdtype < 0 || xdtype > 2) return GGUF_ERR_DTYPE;
   if (!W || !W2 || !x || !q8_workspace || !Y || !Y2) return GGUF_ERR_NULL;
   if (((uintptr_t)W & 1) || ((uintptr_t)W2 & 1) || (w_row_pitch_bytes & 1) || (w_row_pitch_bytes2 & 1) || !on16(q8_workspace)) return GGUF_ERR_SHAPE;
-  if (!ts_two_takes(type, N, w_row_pitch_bytes, type2, N2, w_row_pitch_bytes2, K, M, gemv != 0)) return GGUF_ERR_TYPE;
+  if (!gguf_linear_two_takes(type, N, w_row_pitch_bytes, type2, N2, w_row_pitch_bytes2, K, M, gemv)) return GGUF_ERR_TYPE;
   TsShard a = {W, Y, type, N, LinearArgs()}, b = {W2, Y2, type2, N2, LinearArgs()};
   a.la.w_pitch = w_row_pitch_bytes; a.la.ldy = y_row_pitch; a.la.bias = bias;
   b.la.w_pitch = w_row_pitch_bytes2; b.la.ldy = y_row_pitch; b.la.bias = bias2;
-  return ts_two(a, b, x, xdtype, q8_workspace, M, (int)K, gemv != 0, (hipStream_t)stream);
+  if (M > 4) return ts_two(a, b, x, xdtype, q8_workspace, M, (int)K, gemv != 0, (hipStream_t)stream);
+  int rc = mmvq_pair(a, b, x, xdtype, (int)K, (int)M, (hipStream_t)stream);
+  if (rc != GGUF_NOT_TAKEN) return rc;
+  rc = mmvq_any(type, W, x, q8_workspace, Y, xdtype, N, K, M, (hipStream_t)stream, a.la);
+  return rc != GGUF_OK ? rc : mmvq_any(type2, W2, x, q8_workspace, Y2, xdtype, N2, K, M, (hipStream_t)stream, b.la);
 }

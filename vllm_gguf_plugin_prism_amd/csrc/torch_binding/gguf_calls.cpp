@@ -284,7 +284,7 @@ PyObject* merged_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const gguf_stream_t stream = stream_of(dev);
     char* dst = (char*)y.mutable_data_ptr();
     const char* b = bias ? (const char*)bias->const_data_ptr() : nullptr;
-    // two matrices on the kernels of a few rows: x is quantized once, and they run side by side
+    // two matrices on the GEMV or the kernels of a few rows: x is quantized once, and they run side by side
     const bool gemv = parts[0].path == PATH_MMVQ;
     const auto pitch_of = [&](const Part& p) { return w->size(0) > 1 ? w->stride(0) : p.rb; };
     if (parts.size() == 2 && m <= 32 && parts[0].path == parts[1].path && (gemv || parts[0].path == PATH_MMQ) &&
