@@ -556,7 +556,8 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
 // CG: up to so many column groups of a workgroup (ts_dealt_groups), a panel of K after the other: the activations' operands and block scales stay
 // in registers over the groups (the scales as the halves that they are), a group's panel is asked for while the one before is multiplied, and
 // there is one beginning and one sum for all.  From two on the groups are walked by a loop that is not unrolled, which moves the partial tiles
-// around by one each time: unrolled the compiler keeps more than there are registers.  Tried and slower: whole column groups one after the other,
+// around by one each time: unrolled the compiler keeps more than there are registers.  (A ring of two weight panels per wave: 0.8 to 1.03 times
+// the speed.)  Tried and slower: whole column groups one after the other,
 // the activations fetched again for each (0.86 to 1.06 times the speed of a workgroup each).
 template <class F, int RT> __host__ __device__ constexpr int ts_dealt_place(int ppr, int xn) { return 256 * ppr + 1024 * RT + 1024 * xn; }
 // (two workgroups of one tile of rows share a CU where its registers suffice)
@@ -841,13 +842,13 @@ static int ts_launch(const TsCall& c, int ks, hipStream_t stream) {
 
 // How many column groups a workgroup takes.  Where one of them fills a CU (two tiles of rows, or formats that need the registers), as many as
 // let one round do, up to what the registers hold: [11008,4096] Q4_K 20 rows, one to four groups 16.1 / 16.8 / 12.2 / 13.8 us, [28672,4096]
-// 35.5 / 32.3 / 32.2 / 27.5, eight 25.9.  Where two share a CU, two groups only between one and a half rounds and two: [16384,4096] Q4_K 12 rows 14.3 /
-// 12.6, [12288,4096] Q6_K 17.4 / 18.9.  (Q2_K, two products per block, spills, Q5_K at eight.)
+// 35.5 / 32.3 / 32.2 / 27.5, eight 25.9.  Where two share a CU, two groups between one and a half rounds and two, and of super-blocks
+// past two and three quarters: [16384,4096] Q4_K 12 rows 14.3 / 12.6, [28672,4096] Q6_K 29.4 / 28.8, but [10000,4096] 0.9 of the speed.  (Q2_K, two products per block, spills, Q5_K at eight.)
 template <class F, int RT> constexpr int ts_dealt_most() { return F::OFF == 2 ? 1 : ts_dealt_waves<F, RT>() == 4 ? 2 : RT == 2 && F::KQ && !std::is_same<F, TQ5_K>::value ? 8 : 4; }
 template <class F, int RT>
 static inline int ts_dealt_groups(int groups) {
   constexpr int MOST = ts_dealt_most<F, RT>();
-  if (MOST == 2) return groups > 768 && groups <= 1024 ? 2 : 1;
+  if (MOST == 2) return (groups > 768 && groups <= 1024) || (F::KQ && groups > 1408) ? 2 : 1;
   const int rounds = (groups + 256 * MOST - 1) / (256 * MOST);
   return MOST == 1 ? 1 : (groups + 256 * rounds - 1) / (256 * rounds);
 }
