@@ -748,18 +748,21 @@ static inline size_t ts_chunk_bytes(int rt, bool off, int pc) {
 }
 
 // From which row block on a product of an MoE layer is cut finer: the workgroups run in rounds of `slots`, and what is left for a last,
-// partly filled one takes about as long as a full one -- a beginning and an end worth about five panels, and its waves' panels one
-// behind the other -- on a chip that is mostly idle.  There a workgroup takes four column groups instead of eight and deals K to two
-// waves each, half the panels per wave.  (The number of blocks is an estimate: blocks past the last full round that it expects
-// are cut finer in any case.)  us per layer, before / now: 64 experts, top-8, Q4_0 [2048 -> 1024], 64 tokens 80.1 / 76.1; 8 experts, top-2, Q4_0
-// [3072 -> 3072], 42 tokens 93 / 63; 32 experts, top-4, Q5_K [3584 -> 1280], 19 tokens 98 / 83.  Of 100 random layers with streaming tiles one in a
-// hundred slower by more than 2 %.  (All blocks cut finer: 0.98 times the speed, the last full round as well 0.99.)
+// partly filled one takes about as long as a full one, a beginning and an end worth about five panels and its waves' panels one
+// behind the other, on a chip that is mostly idle.  There a workgroup takes four column groups instead of eight and deals K to two
+// waves each, half the panels per wave, where that is one round with a fifth to spare (the number of blocks is an estimate, and
+// one more than a round holds is a second one) and saves three panels at least.  (Blocks past the last full round that it
+// expects are cut finer in any case.)  us per layer, before / now: 64 experts, top-8, Q4_0 [2048 -> 1024], 64 tokens 80.1 / 76.1; 8 experts, top-2,
+// Q4_0 [1792 -> 3584], 43 tokens 58 / 52; 64 experts, top-6, Q4_K [2304 -> 1792], 10 tokens 88 / 82.  Over 200 random layers on streaming tiles
+// Q4_K 3.3 %, Q4_0, Q5_K 1.5 %, none slower by more than 2; without the room and the margin as much, but one in fourteen slower, by up to 8 %.  Q6_K
+// and Q8_0, whose weights are on their way at the rate that memory has with half the chip's waves, gain nothing (1.000, 1.003) and lose
+// up to 7 % where one block more than estimated is there: not cut.
 static inline int ts_tail(const TsCall& c, int np, int passes, int cols, int col_wgs, int slots) {
   const int cap = slots / col_wgs;                          // blocks per round
   if (np < 2 || cap == 0) return c.row_blocks;
   const int full = (int)(c.live_blocks / cap);
-  const double rest = c.live_blocks - (double)full * cap, rounds = ceil(rest * ((cols + 3) / 4) / slots);
-  const bool finer = rounds * ((np + 1) / 2 + 5.0) < passes * np + 5.0;
+  const double rest = c.live_blocks - (double)full * cap;
+  const bool finer = 1.2 * rest * ((cols + 3) / 4) <= slots && (np + 1) / 2 + 3 < passes * np;
   const int64_t from = (int64_t)(finer ? full : full + 1) * cap;
   return from < c.row_blocks ? (int)from : c.row_blocks;
 }
@@ -773,7 +776,7 @@ static int ts_launch_d(const TsCall& c, int ks, TsArgs a, size_t lds, hipStream_
   }
   const int cols = GATE ? c.gate.inner / 8 : (c.N + 15) / 16, per_wg = TS_NW / ks * a.passes;
   const int col_wgs = (cols + per_wg - 1) / per_wg;
-  a.coarse_blocks = SPLIT || RT != 1 || !c.moe.sorted_token_ids ? c.row_blocks : ts_tail(c, a.np, a.passes, cols, col_wgs, lds <= 80 * 1024 ? 512 : 256);
+  a.coarse_blocks = SPLIT || RT != 1 || F::PB > 200 || !c.moe.sorted_token_ids ? c.row_blocks : ts_tail(c, a.np, a.passes, cols, col_wgs, lds <= 80 * 1024 ? 512 : 256);
   const int64_t coarse = (int64_t)col_wgs * a.coarse_blocks, total = coarse + (int64_t)((cols + 3) / 4) * (c.row_blocks - a.coarse_blocks);
   if (total > 0x7FFFFFFFll) return GGUF_ERR_SHAPE;
   a.coarse = (int)coarse;
