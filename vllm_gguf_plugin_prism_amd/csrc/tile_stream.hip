@@ -126,7 +126,7 @@ static bool ts_dealt_takes(int type, int64_t M, int64_t N, int64_t K) {
   // Q8_0 [19008,2304] 24.0 / 25.4; Q5_K, at most four groups, [25728,3328] 29.2 / 33.0
   if (M > 16) return groups <= 512 || (K >= 1024 && K >= (halves ? 2 * groups - 512 : blocks32 || type == T_Q5_K ? 4 * groups - 2048 : groups + groups / 4));
   // Two panels per row are work for two waves of eight.  Past 1408 groups workgroups of two read the activations half as often: [28672,4096] 12 rows
-  // Q6_K 32.0 / 29.2, [33056,8192] 8 rows Q4_K 61.7 / 41.1, IQ2_XXS from 2050 groups on 1.4 to 1.6 times as fast; but Q4_K, whose decoding is the
+  // Q6_K 32.0 / 30.0, [33056,8192] 8 rows Q4_K 61.7 / 41.1, IQ2_XXS from 2050 groups on 1.4 to 1.6 times as fast; but Q4_K, whose decoding is the
   // least, up to two full rounds at nine rows and more ([25456,10496] 44.6 / 48.6, [28672,4096] 20.4 / 20.9), and Q2_K, one group always.
   const bool behind = type == T_Q2_K ? groups > 1536 : type == T_Q4_K && M >= 9 && groups > 1536 && groups <= 2048;
   if (!blocks32) return (!behind && groups <= 256 * np) || K >= 12000;

@@ -116,16 +116,18 @@ __device__ __forceinline__ void ts_multiply(F& w, const u32x4_s (&xa)[RT][4], co
     w.mins(g, m0, m1);
     if (!F::KQ && left < 8) { m0 = g < left ? m0 : 0.0f; m1 = 4 + g < left ? m1 : 0.0f; }
   }
-  // (the offsets of four blocks, then their products: the partial sums stay small, and so does what they round off)
+  // A sum of the panel's own, added to the row's at its end: the partial sums stay small, and so does what they round off.  So too with the
+  // offsets of four blocks, which cancel most of their products: they come between the second and the third (rel-L2 against 64 bits, Q4_K, 5 .. 32
+  // rows, activations of one sign / normal: 10.2e-7 / 1.50e-7 with the offsets in front, now 5.8e-7 / 1.33e-7;
+  // Q6_K 1.17e-7 with the sum carried on from panel to panel, now 0.95e-7).
   f32x4 part[RT];
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-    part[rt] = OFFSET ? __builtin_amdgcn_mfma_f32_16x16x4f32(so[rt][0], -m0, (f32x4){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0) : acc[rt];
+  for (int rt = 0; rt < RT; ++rt) part[rt] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int b = 0; b < 8; ++b) {
-    if (OFFSET && b == 4) {
+    if (OFFSET && (b & 3) == 2) {
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt) part[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(so[rt][1], -m1, part[rt], 0, 0, 0);
+      for (int rt = 0; rt < RT; ++rt) part[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(so[rt][b >> 2], b < 4 ? -m0 : -m1, part[rt], 0, 0, 0);
     }
     const uint2 q = w.codes(b, g);
     const long bv = (long)(((uint64_t)q.y << 32) | q.x);
@@ -171,7 +173,7 @@ __device__ __forceinline__ void ts_multiply(F& w, const u32x4_s (&xa)[RT][4], co
     }
   }
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) acc[rt] = OFFSET ? acc[rt] + part[rt] : part[rt];
+  for (int rt = 0; rt < RT; ++rt) acc[rt] += part[rt];
 }
 
 template <class F, int RT, bool GATE, bool SPLIT, int D>
@@ -845,15 +847,22 @@ static int ts_launch(const TsCall& c, int ks, hipStream_t stream) {
 
 // How many column groups a workgroup takes.  Where one of them fills a CU (two tiles of rows, or formats that need the registers), as many as
 // let one round do, up to what the registers hold: [11008,4096] Q4_K 20 rows, one to four groups 16.1 / 16.8 / 12.2 / 13.8 us, [28672,4096]
-// 35.5 / 32.3 / 32.2 / 27.5, eight 25.9.  Where two share a CU, two groups between one and a half rounds and two, and of super-blocks
-// past two and three quarters: [16384,4096] Q4_K 12 rows 14.3 / 12.6, [28672,4096] Q6_K 29.4 / 28.8, but [10000,4096] 0.9 of the speed.  (Q2_K, two products per block, spills, Q5_K at eight.)
-template <class F, int RT> constexpr int ts_dealt_most() { return F::OFF == 2 ? 1 : ts_dealt_waves<F, RT>() == 4 ? 2 : RT == 2 && F::KQ && !std::is_same<F, TQ5_K>::value ? 8 : 4; }
+// 35.5 / 32.3 / 32.2 / 27.5, eight 25.9.  Where two share a CU, two groups between one and a half rounds and two, and past two and three
+// quarters: [16384,4096] Q4_K 12 rows 14.3 / 12.6, but [10000,4096] 0.9 of the speed; of those formats whose two groups fit the registers (the
+// others spill: Q6_K 0.9, IQ2_S 0.95 of the speed).  (Q2_K, two products per block, spills, Q5_K at eight.)
+template <class F, class = void> struct TsOneGroup { static constexpr bool value = false; };   // F::ONE_GROUP: registers for one group at four waves per SIMD
+template <class F> struct TsOneGroup<F, std::void_t<decltype(F::ONE_GROUP)>> { static constexpr bool value = F::ONE_GROUP; };
+template <class F, int RT> constexpr int ts_dealt_most() {
+  if (F::OFF == 2) return 1;
+  if (ts_dealt_waves<F, RT>() == 4) return F::KQ && !TsOneGroup<F>::value ? 2 : 1;
+  return RT == 2 && F::KQ && !std::is_same<F, TQ5_K>::value ? 8 : 4;
+}
 template <class F, int RT>
 static inline int ts_dealt_groups(int groups) {
   constexpr int MOST = ts_dealt_most<F, RT>();
-  if (MOST == 2) return (groups > 768 && groups <= 1024) || (F::KQ && groups > 1408) ? 2 : 1;
+  if (MOST <= 2) return MOST == 2 && ((groups > 768 && groups <= 1024) || groups > 1408) ? 2 : 1;
   const int rounds = (groups + 256 * MOST - 1) / (256 * MOST);
-  return MOST == 1 ? 1 : (groups + 256 * rounds - 1) / (256 * rounds);
+  return (groups + 256 * rounds - 1) / (256 * rounds);
 }
 // what the kernel is told of a product, and the LDS that it takes
 template <class F, int RT>
@@ -910,9 +919,12 @@ static int ts_dealt_pair_launch(const TsCall& c, const TsCall& d, hipStream_t st
 }
 template <class F, class G, int RT>
 static int ts_dealt_pair_rt(const TsCall& c, const TsCall& d, hipStream_t s) {
-  const int ng = ts_dealt_groups<F, RT>((c.N + 15) / 16 + (d.N + 15) / 16);
-  if (ng > 2) return GGUF_NOT_TAKEN;                        // (each by itself: as many groups as suit it)
-  return ng == 1 ? ts_dealt_pair_launch<F, G, RT, 1>(c, d, s) : ts_dealt_pair_launch<F, G, RT, 2>(c, d, s);
+  if constexpr (RT == 2) {
+    const int ng = ts_dealt_groups<F, RT>((c.N + 15) / 16 + (d.N + 15) / 16);
+    if (ng > 2) return GGUF_NOT_TAKEN;                      // (each by itself: as many groups as suit it)
+    if (ng == 2) return ts_dealt_pair_launch<F, G, RT, 2>(c, d, s);
+  }
+  return ts_dealt_pair_launch<F, G, RT, 1>(c, d, s);
 }
 template <class F, class G>
 static int ts_dealt_pair(const TsCall& c, const TsCall& d, hipStream_t s) {

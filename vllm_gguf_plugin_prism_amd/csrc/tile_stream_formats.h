@@ -114,7 +114,7 @@ struct TQ5_K {
 // times the value, still exact in int8), and the scale is a quarter.
 struct TQ6_K {
   static constexpr int PB = 210, G = 16, OFF = 0;
-  static constexpr bool KQ = true, HALVES = false;
+  static constexpr bool KQ = true, HALVES = false, ONE_GROUP = true;
   uint2 ql[4], qh[2];
   uint4 sc;
   uint32_t d;
@@ -369,7 +369,7 @@ struct TIQ4_NL : T32<18> {
 // d (6-bit scale - 32) per 32 values: d, the scales' top bits, their nibbles, the codes as in IQ4_NL
 struct TIQ4_XS {
   static constexpr int PB = 136, G = 32, OFF = 0;
-  static constexpr bool KQ = true, HALVES = false;
+  static constexpr bool KQ = true, HALVES = false, ONE_GROUP = true;
   uint2 head, q[8];
   __device__ __forceinline__ void read(const char* p, uint32_t at, int g) {
     if ((at & 7) == 0) {

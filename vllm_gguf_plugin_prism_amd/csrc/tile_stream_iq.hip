@@ -69,6 +69,7 @@ struct TIQ2_XS : TIQ2<FmtIQ2_XS> {
   __device__ __forceinline__ uint2 codes(int b, int) const { return ts_signed(((const uint2*)tab)[at8[b] & 0xFFFF], tab + 512 * 8, at8[b] >> 16); }
 };
 struct TIQ2_S : TIQ2<FmtIQ2_S> {
+  static constexpr bool ONE_GROUP = true;
   __device__ __forceinline__ void read(const char* p, uint32_t at, int g) {
     d = lds_h(p, at);
 #pragma unroll
