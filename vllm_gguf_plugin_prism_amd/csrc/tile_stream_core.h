@@ -23,7 +23,7 @@
 //     panel; their partial tiles are added through LDS in the order of K (SPLIT).  Else a wave finishes its columns alone.
 // Measured (us per call with the quantizer's launch, before -> now; 5.15 TB/s is what a copy of 1 GiB reaches): [28672,8192]
 // Q4_K, 16 rows 45.7 -> 37.6 (3.5 TB/s with the quantizer's 3.5 us inside), 32 rows 73.7 -> 54.0; [6144,4096] Q8_0, 16 rows 18.8 -> 13.4;
-// [12288,1024] Q6_K, 16 rows 21.5 -> 11.7.  MoE layers: Q4_0, 64 experts, top-8, 64 tokens 112 -> 86; Q4_K with Q6_K, 128
+// [12288,1024] Q6_K, 16 rows 21.5 -> 11.7.  MoE layers: Q4_0, 64 experts, top-8, 64 tokens 112 -> 76; Q4_K with Q6_K, 128
 // experts, 300 tokens 262 -> 175.  What is left is the beginning of a workgroup (first chunk of activations, first
 // panels: 4 to 6 us) and the vector instructions around the multiplications.
 // Arithmetic as in the other integer kernels (mmq.cuh:2-104, vecdotq.cuh: exact int32 block sums, scales in fp32).
