@@ -86,6 +86,7 @@ template <int XR> __host__ __device__ __forceinline__ constexpr int ts_scale_at(
 // bytes of LDS that a format's tables take (F::TABLE, filled by F::tables, read through the member tab), 0 for most
 template <class F, class = void> struct TsTable { static constexpr int value = 0; };
 template <class F> struct TsTable<F, std::void_t<decltype(F::TABLE)>> { static constexpr int value = (F::TABLE + 15) / 16 * 16; };
+template <class F> constexpr bool ts_fine() { return F::PB <= 200; }   // an MoE layer's last round of workgroups may be cut finer (ts_tail)
 template <class F> constexpr bool ts_sums() { return F::OFF == 1 || F::HALVES; }   // the activations' block sums are wanted
 
 // A panel's products: acc += what the lane's column of it has with the rows of X.  xa: the lane's quants of the eight blocks; so: block
@@ -193,7 +194,7 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
   // ---- which rows, columns and panels
   // What the last round of workgroups has to do is cut finer (ts_tail): half as many column groups, two waves to each.
   const bool is_moe = RT == 1 && moe.sorted_token_ids != nullptr;   // (blocks of 16 slots only)
-  const bool fine = RT == 1 && !SPLIT && (int)blockIdx.x >= a.coarse;
+  const bool fine = RT == 1 && !SPLIT && ts_fine<F>() && (int)blockIdx.x >= a.coarse;
   int wg = fine ? blockIdx.x - a.coarse : blockIdx.x;
   const int rb = fine ? row_blocks - a.coarse_blocks : a.coarse_blocks;
   const int total8 = (fine ? total - a.coarse : a.coarse) & ~7;   // each of the 8 XCDs gets a contiguous run of workgroups
@@ -778,7 +779,7 @@ static int ts_launch_d(const TsCall& c, int ks, TsArgs a, size_t lds, hipStream_
   }
   const int cols = GATE ? c.gate.inner / 8 : (c.N + 15) / 16, per_wg = TS_NW / ks * a.passes;
   const int col_wgs = (cols + per_wg - 1) / per_wg;
-  a.coarse_blocks = SPLIT || RT != 1 || F::PB > 200 || !c.moe.sorted_token_ids ? c.row_blocks : ts_tail(c, a.np, a.passes, cols, col_wgs, lds <= 80 * 1024 ? 512 : 256);
+  a.coarse_blocks = SPLIT || RT != 1 || !ts_fine<F>() || !c.moe.sorted_token_ids ? c.row_blocks : ts_tail(c, a.np, a.passes, cols, col_wgs, lds <= 80 * 1024 ? 512 : 256);
   const int64_t coarse = (int64_t)col_wgs * a.coarse_blocks, total = coarse + (int64_t)((cols + 3) / 4) * (c.row_blocks - a.coarse_blocks);
   if (total > 0x7FFFFFFFll) return GGUF_ERR_SHAPE;
   a.coarse = (int)coarse;
