@@ -14,7 +14,7 @@
  * gguf_mmq_layer_unit: the same, with 2 added to 1 (past 32 rows) and 4 where the half-precision unit would run a call that these decline.  gguf_moe_mmq_layer_wide: whether
  * gguf_moe_mmq_layer with the workspace it asks for, at addresses divisible by 16, runs on the wide tiles.
  *
- * gguf_linear_two: two products of the same x, up to 32 rows, as two calls of gguf_mmvq_linear (gemv) or gguf_mmq_linear would run them
+ * gguf_linear_two: two products of the same x, up to 32 rows, as calls of gguf_mmvq_linear (gemv: bit 0 the first, bit 1 the second) or gguf_mmq_linear would run them
  * (the same results bit for bit), and for pairs of types that recipes mix in one launch: up to four rows of the GEMV, from five on behind the
  * quantizer's, which other pairs share too.  They are shards of a merged layer, columns of one result of this row pitch.  The workspace, M * gguf_q8_1_row_bytes(K), begins on 16 bytes.
  * gguf_linear_two_takes: 1 for a pair that it serves. */

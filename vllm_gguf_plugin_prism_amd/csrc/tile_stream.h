@@ -41,9 +41,9 @@ bool ts_stream_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch,
 bool ts_dense_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, bool gemv = false);   // gemv: in place of the GEMV
 int ts_dense(int type, const void* W, const void* x, int dtype, void* workspace, void* Y, int64_t M, int N, int K, bool gemv, const LinearArgs& la, hipStream_t s);
 // two products of the same rows of X, both with their panels dealt to the waves of a workgroup: the rows are quantized once
-struct TsShard { const void* W; void* Y; int type; int64_t N; LinearArgs la; };
-bool ts_two_takes(int type, int64_t N, int64_t w_pitch, int type2, int64_t N2, int64_t w_pitch2, int64_t K, int64_t M, bool gemv);
-int ts_two(const TsShard& a, const TsShard& b, const void* x, int dtype, void* workspace, int64_t M, int K, bool gemv, hipStream_t s);
+struct TsShard { const void* W; void* Y; int type; int64_t N; bool gemv; LinearArgs la; };
+bool ts_two_takes(int type, int64_t N, int64_t w_pitch, bool gemv, int type2, int64_t N2, int64_t w_pitch2, bool gemv2, int64_t K, int64_t M);
+int ts_two(const TsShard& a, const TsShard& b, const void* x, int dtype, void* workspace, int64_t M, int K, hipStream_t s);
 // the same for up to four rows on the streaming GEMV (mmvq_pair.hip): whether a pair is taken; the call, or GGUF_NOT_TAKEN
 bool mmvq_pair_takes(int type, int64_t N, int64_t w_pitch, int type2, int64_t N2, int64_t w_pitch2, int64_t K, int64_t M);
 int mmvq_pair(const TsShard& a, const TsShard& b, const void* x, int dtype, int K, int M, hipStream_t s);

@@ -291,17 +291,17 @@ static TsCall ts_dense_call(int type, const void* W, int dtype, int64_t M, int N
   return c;
 }
 
-bool ts_two_takes(int type, int64_t N, int64_t w_pitch, int type2, int64_t N2, int64_t w_pitch2, int64_t K, int64_t M, bool gemv) {
-  return ts_dense_takes(type, M, N, K, w_pitch, gemv) && ts_dense_takes(type2, M, N2, K, w_pitch2, gemv) && ts_dealt_takes(type, M, N, K) && ts_dealt_takes(type2, M, N2, K);
+bool ts_two_takes(int type, int64_t N, int64_t w_pitch, bool gemv, int type2, int64_t N2, int64_t w_pitch2, bool gemv2, int64_t K, int64_t M) {
+  return ts_dense_takes(type, M, N, K, w_pitch, gemv) && ts_dense_takes(type2, M, N2, K, w_pitch2, gemv2) && ts_dealt_takes(type, M, N, K) && ts_dealt_takes(type2, M, N2, K);
 }
 
-int ts_two(const TsShard& a, const TsShard& b, const void* x, int dtype, void* workspace, int64_t M, int K, bool gemv, hipStream_t s) {
+int ts_two(const TsShard& a, const TsShard& b, const void* x, int dtype, void* workspace, int64_t M, int K, hipStream_t s) {
   int rc = quantize_q8_1(x, dtype, workspace, M, K, s, 0, nullptr, true);
   if (rc != GGUF_OK) return rc;
   const TsShard* const shards[2] = {&a, &b};
   TsCall c[2];
   for (int i = 0; i < 2; ++i) {
-    c[i] = ts_dense_call(shards[i]->type, shards[i]->W, dtype, M, (int)shards[i]->N, K, gemv, shards[i]->la);
+    c[i] = ts_dense_call(shards[i]->type, shards[i]->W, dtype, M, (int)shards[i]->N, K, shards[i]->gemv, shards[i]->la);
     c[i].ws = workspace; c[i].Y = shards[i]->Y; c[i].M = (int)M;
     c[i].row_blocks = 1; c[i].live_blocks = 1;
   }
@@ -359,8 +359,8 @@ int mmvq_any(int type, const void* W, const void* x, void* q8_workspace, void* Y
 
 extern "C" int gguf_linear_two_takes(int type, int64_t N, int64_t w_row_pitch_bytes, int type2, int64_t N2, int64_t w_row_pitch_bytes2, int64_t K, int64_t M, int gemv) {
   if (M < 1 || M > 32 || N <= 0 || N2 <= 0 || K <= 0) return 0;
-  if (M <= 4) return gemv && gguf::mmvq_pair_takes(type, N, w_row_pitch_bytes, type2, N2, w_row_pitch_bytes2, K, M);
-  return gguf::ts_two_takes(type, N, w_row_pitch_bytes, type2, N2, w_row_pitch_bytes2, K, M, gemv != 0);
+  if (M <= 4) return gemv == 3 && gguf::mmvq_pair_takes(type, N, w_row_pitch_bytes, type2, N2, w_row_pitch_bytes2, K, M);
+  return gguf::ts_two_takes(type, N, w_row_pitch_bytes, gemv & 1, type2, N2, w_row_pitch_bytes2, gemv & 2, K, M);
 }
 
 extern "C" int gguf_linear_two(const void* W, int64_t w_row_pitch_bytes, int type, int64_t N, void* Y, const void* bias, const void* W2, int64_t w_row_pitch_bytes2, int type2,
@@ -375,10 +375,10 @@ extern "C" int gguf_linear_two(const void* W, int64_t w_row_pitch_bytes, int typ
   if (!W || !W2 || !x || !q8_workspace || !Y || !Y2) return GGUF_ERR_NULL;
   if (((uintptr_t)W & 1) || ((uintptr_t)W2 & 1) || (w_row_pitch_bytes & 1) || (w_row_pitch_bytes2 & 1) || !on16(q8_workspace)) return GGUF_ERR_SHAPE;
   if (!gguf_linear_two_takes(type, N, w_row_pitch_bytes, type2, N2, w_row_pitch_bytes2, K, M, gemv)) return GGUF_ERR_TYPE;
-  TsShard a = {W, Y, type, N, LinearArgs()}, b = {W2, Y2, type2, N2, LinearArgs()};
+  TsShard a = {W, Y, type, N, (gemv & 1) != 0, LinearArgs()}, b = {W2, Y2, type2, N2, (gemv & 2) != 0, LinearArgs()};
   a.la.w_pitch = w_row_pitch_bytes; a.la.ldy = y_row_pitch; a.la.bias = bias;
   b.la.w_pitch = w_row_pitch_bytes2; b.la.ldy = y_row_pitch; b.la.bias = bias2;
-  if (M > 4) return ts_two(a, b, x, xdtype, q8_workspace, M, (int)K, gemv != 0, (hipStream_t)stream);
+  if (M > 4) return ts_two(a, b, x, xdtype, q8_workspace, M, (int)K, (hipStream_t)stream);
   int rc = mmvq_pair(a, b, x, xdtype, (int)K, (int)M, (hipStream_t)stream);
   if (rc != GGUF_NOT_TAKEN) return rc;
   rc = mmvq_any(type, W, x, q8_workspace, Y, xdtype, N, K, M, (hipStream_t)stream, a.la);

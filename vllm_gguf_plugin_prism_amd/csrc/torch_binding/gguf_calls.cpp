@@ -285,9 +285,10 @@ PyObject* merged_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     char* dst = (char*)y.mutable_data_ptr();
     const char* b = bias ? (const char*)bias->const_data_ptr() : nullptr;
     // two matrices on the GEMV or the kernels of a few rows: x is quantized once, and they run side by side
-    const bool gemv = parts[0].path == PATH_MMVQ;
     const auto pitch_of = [&](const Part& p) { return w->size(0) > 1 ? w->stride(0) : p.rb; };
-    if (parts.size() == 2 && m <= 32 && parts[0].path == parts[1].path && (gemv || parts[0].path == PATH_MMQ) &&
+    const bool two = parts.size() == 2 && m <= 32 && parts[0].path != PATH_DENSE && parts[1].path != PATH_DENSE;
+    const int gemv = two ? (parts[0].path == PATH_MMVQ) | (parts[1].path == PATH_MMVQ) << 1 : 0;
+    if (two &&
         gguf_linear_two_takes((int)parts[0].type, parts[0].end - parts[0].start, pitch_of(parts[0]), (int)parts[1].type, parts[1].end - parts[1].start, pitch_of(parts[1]), k, m, gemv)) {
       const Part &p = parts[0], &q = parts[1];
       const int64_t rows = p.end - p.start;
