@@ -32,14 +32,19 @@ def test_dense_edges(qtype, m, n, k, pad):
 # a few pairs per expert and enough experts that a wave walks two (or four) column groups; inner sizes that end inside a
 # workgroup's features; the longest K of the gated product; a pair whose expert does not exist
 @pytest.mark.parametrize("qtype,tokens,e,hid,inner", [(o.Q4_0, 60, 40, 288, 1056), (o.Q8_0, 24, 6, 4096, 800), (o.Q4_K, 60, 40, 256, 1280),
-                                                      (o.Q5_K, 24, 6, 4096, 256), (o.Q6_K, 24, 6, 4096, 768)])
+                                                      (o.Q5_K, 24, 6, 4096, 256), (o.Q6_K, 24, 6, 4096, 768), (o.Q4_0, 60, 40, 736, 1056),
+                                                      (o.Q8_0, 90, 44, 544, 2080), (o.Q4_K, 60, 40, 2304, 1024), (o.Q6_K, 40, 36, 1280, 1280), (o.Q5_K, 12, 6, 768, 512)])
 def test_moe_layer_edges(qtype, tokens, e, hid, inner):
+    check_layer(qtype, tokens, e, hid, inner)
+
+
+def check_layer(qtype, tokens, e, hid, inner, routing=None):
     from vllm_gguf_plugin_prism_amd import ops
     rng = np.random.default_rng(hid + inner)
     top_k = 2
     w13 = np.stack([o.make_weights(rng, qtype, 2 * inner, hid) for _ in range(e)])
     w2 = np.stack([o.make_weights(rng, qtype, hid, inner) for _ in range(e)])
-    ids = np.stack([rng.permutation(e)[:top_k] for _ in range(tokens)]).astype(np.int32)
+    ids = np.stack([rng.permutation(e)[:top_k] for _ in range(tokens)]).astype(np.int32) if routing is None else routing.copy()
     ids[3, 1] = e + 2
     wts = rng.random((tokens, top_k)).astype(np.float32)
     x = rng.standard_normal((tokens, hid)).astype(np.float32)
@@ -69,9 +74,44 @@ def test_dense_where_it_is_taken(qtype, m, n, k):
     assert o.rel_l2(y.cpu().numpy(), o.mul_mat_a8(w, x, qtype, n, "mmq")) <= 1e-5
 
 
-# layers whose last round of workgroups is cut finer: behind a full round in both products, an odd number of panels dealt to two waves,
-# more blocks than expected, inner sizes that end inside a workgroup's features; all of a product in one round
-@pytest.mark.parametrize("qtype,tokens,e,hid,inner", [(o.Q4_0, 60, 40, 736, 1056), (o.Q8_0, 90, 44, 544, 2080), (o.Q4_K, 60, 40, 2304, 1024), (o.Q6_K, 40, 36, 1280, 1280),
-                                                      (o.Q5_K, 12, 6, 768, 512)])
+# Layers of which both products deal K of their last blocks to two waves each: behind full rounds and from the first block on, an even and an odd
+# number of panels, one of them in part, one panel per wave, inner sizes that end inside a workgroup's features.  Every expert is the same and
+# so is every token: so are the results, bit for bit, whichever block a pair is in.
+LAST_ROUND = [(o.Q4_0, 62, 4, 2016, 2048), (o.Q4_0, 42, 30, 1056, 1056), (o.Q4_K, 43, 6, 2304, 2048), (o.Q5_K, 34, 34, 2048, 512)]
+
+
+def many_blocks(tokens, e):
+    """Two experts per token so that as many blocks of 16 slots as possible hold pairs: one pair of every expert, then 16 more at a time."""
+    count, left = np.ones(e, np.int64), 2 * tokens - e
+    for i in range(left // 16 + 1):
+        count[i % e] += min(16, left - 16 * i)
+    return np.repeat(np.arange(e), count).reshape(tokens, 2).astype(np.int32)
+
+
+def last_blocks(qtype, tokens, e, hid, inner, ids):
+    """How many blocks with pairs have K dealt to two waves, in either product."""
+    from vllm_gguf_plugin_prism_amd import _lib
+    live = int(((np.bincount(ids[ids < e], minlength=e) + 15) // 16).sum())
+    start = [_lib.lib().gguf_moe_mmq_layer_finer(qtype, qtype, hid, inner, hid, 2, tokens, e, product) for product in (1, 2)]
+    return [live - at if at >= 0 else 0 for at in start]
+
+
+@pytest.mark.parametrize("qtype,tokens,e,hid,inner", LAST_ROUND)
+def test_moe_rows_do_not_depend_on_their_block(qtype, tokens, e, hid, inner):
+    from vllm_gguf_plugin_prism_amd import ops
+    rng = np.random.default_rng(hid)
+    ids = many_blocks(tokens, e)
+    assert min(last_blocks(qtype, tokens, e, hid, inner, ids)) > 0
+    w13, w2 = (torch.from_numpy(o.make_weights(rng, qtype, *shape)).cuda().repeat(e, 1, 1) for shape in ((2 * inner, hid), (hid, inner)))
+    x = torch.from_numpy(rng.standard_normal(hid).astype(np.float32)).cuda()[None]
+    x = (x * (4.0 / ops.ggml_mul_mat_a8(w13[0], x, qtype, 2 * inner).abs().max())).repeat(tokens, 1)
+    got = ops.moe_mmq_layer(x, w13, w2, torch.full((tokens, 2), 0.5, device="cuda"), torch.from_numpy(ids).cuda(), qtype, qtype, "silu")
+    assert bool(got.isfinite().all()) and torch.equal(got, got[:1].repeat(tokens, 1))
+
+
+@pytest.mark.parametrize("qtype,tokens,e,hid,inner", LAST_ROUND)
 def test_moe_layer_last_round(qtype, tokens, e, hid, inner):
-    test_moe_layer_edges(qtype, tokens, e, hid, inner)
+    ids = many_blocks(tokens, e)
+    ids[3, 1] = e + 2
+    assert min(last_blocks(qtype, tokens, e, hid, inner, ids)) > 0
+    check_layer(qtype, tokens, e, hid, inner, ids)

@@ -13,6 +13,8 @@
  * half-precision unit's, 0 another; up to 32 rows the one that stands behind tile_dealt_kernel, whose lines are its own.
  * gguf_mmq_layer_unit: the same, with 2 added to 1 (past 32 rows) and 4 where the half-precision unit would run a call that these decline.  gguf_moe_mmq_layer_wide: whether
  * gguf_moe_mmq_layer with the workspace it asks for, at addresses divisible by 16, runs on the wide tiles.
+ * gguf_moe_mmq_layer_finer: the block of 16 slots from which on the first or second product (product) of a layer on the streaming tiles deals K to
+ * two waves each; -1: none, or a layer that they do not take.
  *
  * gguf_linear_two: two products of the same x, up to 32 rows, as calls of gguf_mmvq_linear (gemv: bit 0 the first, bit 1 the second) or gguf_mmq_linear would run them
  * (the same results bit for bit), and for pairs of types that recipes mix in one launch: up to four rows of the GEMV, from five on behind the
@@ -28,6 +30,7 @@ int64_t gguf_dense_linear_workspace_bytes(int64_t N, int64_t K, int64_t M);
 int gguf_dense_linear(const void* W, int64_t w_row_pitch_bytes, const void* x, int xdtype, void* workspace, void* Y, int64_t y_row_pitch,
                       const void* bias, int type, int64_t N, int64_t K, int64_t M, int64_t workspace_bytes, void* stream);
 int64_t gguf_mmq_layer_workspace_bytes(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes);
+int gguf_moe_mmq_layer_finer(int type13, int type2, int64_t H, int64_t I, int64_t N_out, int64_t top_k, int64_t tokens, int64_t num_experts, int product);
 int gguf_moe_mmq_layer_wide(int type13, int type2, int64_t H, int64_t I, int64_t N_out, int64_t top_k, int64_t tokens, int64_t num_experts);
 int gguf_mmq_layer_unit(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes);
 int gguf_linear_two_takes(int type, int64_t N, int64_t w_row_pitch_bytes, int type2, int64_t N2, int64_t w_row_pitch_bytes2, int64_t K, int64_t M, int gemv);

@@ -33,6 +33,7 @@ struct TsCall {
   int row_blocks;              // tiles of 16 rt rows (dense) or blocks of slots
   double live_blocks;          // how many of them hold pairs, estimated (dense: all)
   Gate16 gate;                 // rows != null: the gated epilogue
+  int* finer_from;             // not null: nothing is launched, and this says from which row block on K is dealt to two waves each (ts_tail)
 };
 
 // tile_stream.hip: whether a call is taken -- a dense product of M rows, a layer with this many (token, expert) pairs, an

@@ -332,8 +332,7 @@ int ts_dense(int type, const void* W, const void* x, int dtype, void* workspace,
   return GGUF_OK;
 }
 
-int ts_moe(const void* W, const void* ws, void* Y, int dtype, int type, int N, int K, int num_sorted, const MoeArgs& moe, hipStream_t s,
-           const Gate16& gate) {
+static TsCall ts_moe_call(const void* W, const void* ws, void* Y, int dtype, int N, int K, int num_sorted, const MoeArgs& moe, const Gate16& gate) {
   TsCall c = {};
   c.W = W;
   c.ws = ws;
@@ -347,6 +346,12 @@ int ts_moe(const void* W, const void* ws, void* Y, int dtype, int type, int N, i
   c.row_blocks = num_sorted / 16;
   c.live_blocks = moe_blocks_estimate(num_sorted, moe.num_pairs, 16);
   c.gate = gate;
+  return c;
+}
+
+int ts_moe(const void* W, const void* ws, void* Y, int dtype, int type, int N, int K, int num_sorted, const MoeArgs& moe, hipStream_t s,
+           const Gate16& gate) {
+  const TsCall c = ts_moe_call(W, ws, Y, dtype, N, K, num_sorted, moe, gate);
   if (c.row_blocks == 0) return GGUF_OK;
   return taken(ts_any(type, c, s));
 }
@@ -356,6 +361,22 @@ int ts_moe(const void* W, const void* ws, void* Y, int dtype, int type, int N, i
 namespace gguf {
 int mmvq_any(int type, const void* W, const void* x, void* q8_workspace, void* Y, int xdtype, int64_t N, int64_t K, int64_t M, hipStream_t s, const LinearArgs& la);
 }  // namespace gguf
+
+extern "C" int gguf_moe_mmq_layer_finer(int type13, int type2, int64_t H, int64_t I, int64_t N_out, int64_t top_k, int64_t tokens, int64_t num_experts, int product) {
+  using namespace gguf;
+  if (H <= 0 || I <= 0 || N_out <= 0 || top_k <= 0 || tokens <= 0 || num_experts <= 0 || product < 1 || product > 2) return -1;
+  if (block_elems(type13) == 0 || block_elems(type2) == 0 || !ts_layer_takes(type13, type2, H, I, N_out, tokens, top_k, num_experts)) return -1;
+  const int64_t pairs = tokens * top_k, sorted = (pairs + num_experts * 15) / 16 * 16;
+  static const int32_t some[1] = {0};                       // (stands for the arrays that the call would have: nothing reads it)
+  int from = -1;
+  MoeArgs moe = {some, some, some, 0, product == 1 ? (int)top_k : 1, (int)pairs, 0};
+  const int type = product == 1 ? type13 : type2;
+  moe.expert_stride = (product == 1 ? 2 * I : N_out) * ((product == 1 ? H : I) / block_elems(type)) * block_bytes(type);
+  const Gate16 gate = product == 1 ? Gate16{(char*)some, 0, (int)I, 0, 0} : Gate16{};
+  TsCall c = ts_moe_call(nullptr, nullptr, nullptr, GGUF_DTYPE_F16, (int)(product == 1 ? 2 * I : N_out), (int)(product == 1 ? H : I), (int)sorted, moe, gate);
+  c.finer_from = &from;
+  return ts_any(type, c, nullptr) == GGUF_OK && from < c.row_blocks ? from : -1;
+}
 
 extern "C" int gguf_linear_two_takes(int type, int64_t N, int64_t w_row_pitch_bytes, int type2, int64_t N2, int64_t w_row_pitch_bytes2, int64_t K, int64_t M, int gemv) {
   if (M < 1 || M > 32 || N <= 0 || N2 <= 0 || K <= 0) return 0;

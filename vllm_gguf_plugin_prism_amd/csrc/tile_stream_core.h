@@ -86,15 +86,16 @@ template <int XR> __host__ __device__ __forceinline__ constexpr int ts_scale_at(
 // bytes of LDS that a format's tables take (F::TABLE, filled by F::tables, read through the member tab), 0 for most
 template <class F, class = void> struct TsTable { static constexpr int value = 0; };
 template <class F> struct TsTable<F, std::void_t<decltype(F::TABLE)>> { static constexpr int value = (F::TABLE + 15) / 16 * 16; };
-template <class F> constexpr bool ts_fine() { return F::PB <= 200; }   // an MoE layer's last round of workgroups may be cut finer (ts_tail)
+// formats of which an MoE layer's last round of workgroups may be cut finer (ts_tail; the other two that layers have, Q6_K and Q8_0, gain nothing)
+template <class F> constexpr bool ts_fine() { return std::is_same<F, TQ4_0>::value || std::is_same<F, TQ4_K>::value || std::is_same<F, TQ5_K>::value; }
 template <class F> constexpr bool ts_sums() { return F::OFF == 1 || F::HALVES; }   // the activations' block sums are wanted
 
-// A panel's products: acc += what the lane's column of it has with the rows of X.  xa: the lane's quants of the eight blocks; so: block
+// A panel's products: part = what the lane's column of it has with the rows of X.  xa: the lane's quants of the eight blocks; so: block
 // sums g and 4 + g of row c; left: blocks of the panel inside the row; half0: all bits in the lanes that hold the first 16
 // values of a block; d8_of, s8_of: block scales and sums of the lane's four result rows.
 template <class F, int RT, class D8, class S8>
 __device__ __forceinline__ void ts_multiply(F& w, const u32x4_s (&xa)[RT][4], const float (&so)[RT][2], int left, int g, uint32_t half0, D8 d8_of, S8 s8_of,
-                                            f32x4 (&acc)[RT]) {
+                                            f32x4 (&part)[RT]) {
   constexpr bool OFFSET = F::OFF == 1;
   const v4i seed = {kSeedBits, kSeedBits, kSeedBits, kSeedBits};
   float dw[8 * (32 / F::G)];
@@ -117,11 +118,10 @@ __device__ __forceinline__ void ts_multiply(F& w, const u32x4_s (&xa)[RT][4], co
     w.mins(g, m0, m1);
     if (!F::KQ && left < 8) { m0 = g < left ? m0 : 0.0f; m1 = 4 + g < left ? m1 : 0.0f; }
   }
-  // A sum of the panel's own, added to the row's at its end: the partial sums stay small, and so does what they round off.  So too with the
+  // A sum of the panel's own, added to the row's by the caller: the partial sums stay small, and so does what they round off.  So too with the
   // offsets of four blocks, which cancel most of their products: they come between the second and the third (rel-L2 against 64 bits, Q4_K, 5 .. 32
   // rows, activations of one sign / normal: 10.2e-7 / 1.50e-7 with the offsets in front, now 5.8e-7 / 1.33e-7;
   // Q6_K 1.17e-7 with the sum carried on from panel to panel, now 0.95e-7).
-  f32x4 part[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) part[rt] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -173,15 +173,14 @@ __device__ __forceinline__ void ts_multiply(F& w, const u32x4_s (&xa)[RT][4], co
       }
     }
   }
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) acc[rt] += part[rt];
 }
 
-template <class F, int RT, bool GATE, bool SPLIT, int D>
+template <class F, int RT, bool GATE, bool SPLIT, int D, bool MOE>
 __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_stream_kernel(const uint8_t* __restrict__ W, const char* __restrict__ ws,
                                                                                   void* __restrict__ Y, TsArgs a, MoeArgs moe, Gate16 gate,
                                                                                   int row_blocks, int total) {
-  static_assert(!GATE || (RT == 1 && !SPLIT), "a gated product takes its column groups whole, for 16 slots");
+  static_assert(!GATE || (MOE && !SPLIT), "a gated product is a layer's and takes its column groups whole");
+  static_assert(!MOE || RT == 1, "blocks of 16 slots");
   static_assert(D >= 2 && D <= 4, "one wait per number of panels requested behind the one at hand");
   constexpr int NW = TS_NW, XR = 16 * RT, XR_LOG2 = RT == 1 ? 4 : 5;
   constexpr bool SUMS = ts_sums<F>(), OFFSET = F::OFF == 1;
@@ -193,15 +192,15 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
 
   // ---- which rows, columns and panels
   // What the last round of workgroups has to do is cut finer (ts_tail): half as many column groups, two waves to each.
-  const bool is_moe = RT == 1 && moe.sorted_token_ids != nullptr;   // (blocks of 16 slots only)
-  const bool fine = RT == 1 && !SPLIT && ts_fine<F>() && (int)blockIdx.x >= a.coarse;
+  constexpr bool FINER = MOE && !SPLIT && ts_fine<F>();
+  const bool fine = FINER && (int)blockIdx.x >= a.coarse;
   int wg = fine ? blockIdx.x - a.coarse : blockIdx.x;
   const int rb = fine ? row_blocks - a.coarse_blocks : a.coarse_blocks;
   const int total8 = (fine ? total - a.coarse : a.coarse) & ~7;   // each of the 8 XCDs gets a contiguous run of workgroups
   if (wg < total8) wg = (wg & 7) * (total8 >> 3) + (wg >> 3);
   // (the blocks of one expert are neighbours: they share its weights)
   const int col_wg = rb == 1 ? wg : (int)__umulhi((uint32_t)wg, fine ? a.fine_inv : a.rb_inv), block = wg - col_wg * rb + (fine ? a.coarse_blocks : 0);
-  if (is_moe) {
+  if constexpr (MOE) {
     const int live = moe.num_tokens_post_padded[0], e = moe.expert_ids[block];
     if (block * XR >= live || e < 0 || e > 255) return;     // (experts above 255: the reference's guard, moe.cuh:33)
     W += (int64_t)e * moe.expert_stride;
@@ -341,7 +340,7 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
     }
   };
 
-  if (is_moe) {
+  if constexpr (MOE) {
     // The weights do not wait for the routing: the pairs behind a block's slots come as scalar loads, which have a counter
     // of their own, and are waited for behind the first requests of weights without waiting for the weights.
     int slot_ids[16];
@@ -372,15 +371,18 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
 
   const uint32_t half0 = g < 2 ? ~0u : 0u;                  // lanes that hold the first 16 values of a block
   const auto store = [&](int m, int n, float v) {           // result row m of this workgroup's tile, feature n (all lanes together)
-    const int row = is_moe ? __shfl(pair_at, m) : block * XR + m;
-    if (n < a.N && row < (is_moe ? moe.num_pairs : a.M)) ts_store(Y, (int64_t)row * a.ldy + n, v, a.bias, n, a.dtype);
+    const int row = MOE ? __shfl(pair_at, m) : block * XR + m;
+    if (n < a.N && row < (MOE ? moe.num_pairs : a.M)) ts_store(Y, (int64_t)row * a.ldy + n, v, a.bias, n, a.dtype);
   };
   const int chunks = (a.np + PC - 1) >> a.pc_log2;
   int t = 0, slot = 0;                                      // tasks done, ring slot of the next
-  f32x4 acc[RT], kept[4];                                   // kept (gated): the last four column groups' sums
+  // Where blocks may have K dealt to two waves, the others too add the even and the odd panels in two sums: a pair's result does not
+  // depend on the block that it is in.
+  f32x4 acc[RT], odd, kept[4];                              // kept (gated): the last four column groups' sums
   for (int pass = 0; pass < passes; ++pass) {
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) acc[rt] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+  odd = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
   const int pass_end = min(tasks, (pass + 1) * np_mine);
   int p = ks;
   for (int ch = 0; ch < chunks; ++ch) {
@@ -427,8 +429,13 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
       ++t;
       slot = slot + 1 == D ? 0 : slot + 1;
 
+      f32x4 part[RT];
       ts_multiply<F, RT>(w, xa, so, left, g, half0, [&](int rt, int b) { return *(const f32x4*)(xd + ts_scale_at<XR>(8 * pl) + ts_scale_at<XR>(b) + 16 * rt + 4 * g); },
-                         [&](int rt, int b) { return *(const f32x4*)(xd + ts_scale_at<XR>(8 * PC) + ts_scale_at<XR>(8 * pl) + ts_scale_at<XR>(b) + 16 * rt + 4 * g); }, acc);
+                         [&](int rt, int b) { return *(const f32x4*)(xd + ts_scale_at<XR>(8 * PC) + ts_scale_at<XR>(8 * pl) + ts_scale_at<XR>(b) + 16 * rt + 4 * g); }, part);
+      if (FINER && (p & 1)) odd += part[0];
+      else
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) acc[rt] += part[rt];
     }
     // ---- the next chunk of activations
     if constexpr (SPLIT) {
@@ -443,12 +450,13 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
       }
     }
   }
+  if constexpr (FINER) acc[0] += odd;                       // (a finer workgroup's waves have one of the two)
   if constexpr (GATE) {
 #pragma unroll
     for (int i = 0; i < 3; ++i) kept[i] = kept[i + 1];
     kept[3] = acc[0];
   } else if constexpr (!SPLIT) {
-    if (RT == 1 && fine) {                                  // the two waves' sums, over the activations
+    if (fine) {                                             // the two waves' sums, over the activations
       f32x4* const red = (f32x4*)smem;
       __syncthreads();
       if (ks) red[cs * 64 + lane] = acc[0];
@@ -699,7 +707,10 @@ __device__ __forceinline__ void tile_dealt_body(const uint8_t* __restrict__ W, c
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");    // the place may be filled again
       if (j + 1 < ng) request_w(p, j + 1);
       else if (p + NW < a.np) { request_w(p + NW, 0); request_x(p + NW); }
-      ts_multiply<F, RT>(w, xa, so, left, g, half0, [&](int rt, int b) { return of(rt, b, 0); }, [&](int rt, int b) { return of(rt, b, 1); }, acc[0]);
+      f32x4 part[RT];
+      ts_multiply<F, RT>(w, xa, so, left, g, half0, [&](int rt, int b) { return of(rt, b, 0); }, [&](int rt, int b) { return of(rt, b, 1); }, part);
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) acc[0][rt] += part[rt];
       if constexpr (CG > 1) {                               // (the next group's tile first: a tile by number would be in scratch)
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
@@ -770,16 +781,16 @@ static inline int ts_tail(const TsCall& c, int np, int passes, int cols, int col
   return from < c.row_blocks ? (int)from : c.row_blocks;
 }
 
-template <class F, int RT, bool GATE, bool SPLIT, int D>
+template <class F, int RT, bool GATE, bool SPLIT, int D, bool MOE>
 static int ts_launch_d(const TsCall& c, int ks, TsArgs a, size_t lds, hipStream_t stream) {
-  auto kern = tile_stream_kernel<F, RT, GATE, SPLIT, D>;
-  if (lds > 64 * 1024) {
-    static std::atomic<uint64_t> done{0};
-    allow_large_lds(kern, 160 * 1024, done);
-  }
+  auto kern = tile_stream_kernel<F, RT, GATE, SPLIT, D, MOE>;
   const int cols = GATE ? c.gate.inner / 8 : (c.N + 15) / 16, per_wg = TS_NW / ks * a.passes;
   const int col_wgs = (cols + per_wg - 1) / per_wg;
-  a.coarse_blocks = SPLIT || RT != 1 || !ts_fine<F>() || !c.moe.sorted_token_ids ? c.row_blocks : ts_tail(c, a.np, a.passes, cols, col_wgs, lds <= 80 * 1024 ? 512 : 256);
+  a.coarse_blocks = SPLIT || !MOE || !ts_fine<F>() ? c.row_blocks : ts_tail(c, a.np, a.passes, cols, col_wgs, lds <= 80 * 1024 ? 512 : 256);
+  if (c.finer_from) {
+    *c.finer_from = a.coarse_blocks;
+    return GGUF_OK;
+  }
   const int64_t coarse = (int64_t)col_wgs * a.coarse_blocks, total = coarse + (int64_t)((cols + 3) / 4) * (c.row_blocks - a.coarse_blocks);
   if (total > 0x7FFFFFFFll) return GGUF_ERR_SHAPE;
   a.coarse = (int)coarse;
@@ -787,6 +798,10 @@ static int ts_launch_d(const TsCall& c, int ks, TsArgs a, size_t lds, hipStream_
   a.fine_inv = (uint32_t)((0x100000000ull + c.row_blocks - a.coarse_blocks - 1) / (c.row_blocks > a.coarse_blocks ? c.row_blocks - a.coarse_blocks : 1));
   // the quotients by reciprocal are exact while dividend times divisor stays below 2^32
   if (total * c.row_blocks > 0xFFFFFFFFll || (int64_t)c.moe.num_pairs * (c.moe.top_k > 0 ? c.moe.top_k : 1) > 0xFFFFFFFFll) return GGUF_ERR_SHAPE;
+  if (lds > 64 * 1024) {
+    static std::atomic<uint64_t> done{0};
+    allow_large_lds(kern, 160 * 1024, done);
+  }
   hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(64 * TS_NW), lds, stream, (const uint8_t*)c.W, (const char*)c.ws, c.Y, a, c.moe, c.gate,
                      c.row_blocks, (int)total);
   return launch_status();
@@ -802,12 +817,12 @@ static inline int ts_passes(int np, double rounds) {
   return passes;
 }
 
-template <class F, int RT, bool GATE, bool SPLIT>
+template <class F, int RT, bool GATE, bool SPLIT, bool MOE>
 static int ts_launch(const TsCall& c, int ks, hipStream_t stream) {
   const int np = (c.K + 255) / 256, qk = F::KQ ? 256 : 32, bs = F::KQ ? F::PB : F::PB / 8;
   const int64_t pitch = c.w_pitch ? c.w_pitch : (int64_t)(c.K / qk) * bs;
   // pieces per row and panel: one more where a panel may begin inside one
-  const bool aligned = F::PB % 16 == 0 && pitch % 16 == 0 && (uintptr_t)c.W % 16 == 0 && (!c.moe.sorted_token_ids || c.moe.expert_stride % 16 == 0);
+  const bool aligned = F::PB % 16 == 0 && pitch % 16 == 0 && (uintptr_t)c.W % 16 == 0 && (!MOE || c.moe.expert_stride % 16 == 0);
   // (an odd number, so that the same field of 16 rows lies in different banks: [23376,1856] of Q4_0, 16 rows of X 23.2 -> 19.2 us)
   const int ppr = (aligned ? F::PB / 16 : (F::PB + 29) / 16) | 1, top_k = c.moe.top_k > 0 ? c.moe.top_k : 1;
   const auto bytes = [&](int pc, int nbuf, int d) { return nbuf * ts_chunk_bytes(RT, ts_sums<F>(), pc) + (size_t)TS_NW * d * 256 * ppr + 16 + TsTable<F>::value; };
@@ -840,9 +855,9 @@ static int ts_launch(const TsCall& c, int ks, hipStream_t stream) {
                     (uint32_t)((0x100000000ull + ppr - 1) / ppr), 0, (uint32_t)((0x100000000ull + top_k - 1) / top_k), 0, 0, 0,
                     c.gemv_sums ? 2 : 1, c.dtype, c.ldy ? c.ldy : (int64_t)c.N, c.bias};
   switch (d) {
-    case 4: return ts_launch_d<F, RT, GATE, SPLIT, 4>(c, ks, a, lds, stream);
-    case 3: return ts_launch_d<F, RT, GATE, SPLIT, 3>(c, ks, a, lds, stream);
-    default: return ts_launch_d<F, RT, GATE, SPLIT, 2>(c, ks, a, lds, stream);
+    case 4: return ts_launch_d<F, RT, GATE, SPLIT, 4, MOE>(c, ks, a, lds, stream);
+    case 3: return ts_launch_d<F, RT, GATE, SPLIT, 3, MOE>(c, ks, a, lds, stream);
+    default: return ts_launch_d<F, RT, GATE, SPLIT, 2, MOE>(c, ks, a, lds, stream);
   }
 }
 
@@ -932,19 +947,21 @@ static int ts_dealt_pair(const TsCall& c, const TsCall& d, hipStream_t s) {
   return c.M <= 16 ? ts_dealt_pair_rt<F, G, 1>(c, d, s) : ts_dealt_pair_rt<F, G, 2>(c, d, s);
 }
 
-template <class F, int RT>
+template <class F, int RT, bool MOE = false>
 static int ts_run_rt(const TsCall& c, hipStream_t stream) {
   const int np = (c.K + 255) / 256;
-  if (c.dealt) {
-    const int rc = ts_dealt_launch<F, RT>(c, stream);
-    if (rc != GGUF_NOT_TAKEN) return rc;
+  if constexpr (!MOE) {
+    if (c.dealt) {
+      const int rc = ts_dealt_launch<F, RT>(c, stream);
+      if (rc != GGUF_NOT_TAKEN) return rc;
+    }
   }
   const int ks = ts_ks(np, c.live_blocks * ((c.N + 15) / 16));
   if (ks == 1 && np <= 16) {
-    const int rc = ts_launch<F, RT, false, false>(c, 1, stream);
+    const int rc = ts_launch<F, RT, false, false, MOE>(c, 1, stream);
     if (rc != GGUF_NOT_TAKEN) return rc;
   }
-  return ts_launch<F, RT, false, true>(c, ks, stream);
+  return ts_launch<F, RT, false, true, MOE>(c, ks, stream);
 }
 
 template <class F>
@@ -957,7 +974,7 @@ template <class F>
 static int ts_run(const TsCall& c, hipStream_t stream) {
   if (!c.moe.sorted_token_ids) return ts_dense_run<F>(c, stream);
   if (c.rt != 1) return GGUF_NOT_TAKEN;
-  return c.gate.rows ? ts_launch<F, 1, true, false>(c, 1, stream) : ts_run_rt<F, 1>(c, stream);
+  return c.gate.rows ? ts_launch<F, 1, true, false, true>(c, 1, stream) : ts_run_rt<F, 1, true>(c, stream);
 }
 
 }  // namespace gguf
