@@ -90,12 +90,13 @@ template <class F> struct TsTable<F, std::void_t<decltype(F::TABLE)>> { static c
 template <class F> constexpr bool ts_fine() { return std::is_same<F, TQ4_0>::value || std::is_same<F, TQ4_K>::value || std::is_same<F, TQ5_K>::value; }
 template <class F> constexpr bool ts_sums() { return F::OFF == 1 || F::HALVES; }   // the activations' block sums are wanted
 
-// A panel's products: part = what the lane's column of it has with the rows of X.  xa: the lane's quants of the eight blocks; so: block
-// sums g and 4 + g of row c; left: blocks of the panel inside the row; half0: all bits in the lanes that hold the first 16
+// A panel's products: sum += (without ADD sum =) what the lane's column of it has with the rows of X.  (Handing the panel's sums to every caller
+// takes registers off the kernels that only add them, and 4 % off the speed of Q2_K, 1 % of Q4_K and Q5_K at two tiles of rows.)  xa: the
+// lane's quants of the eight blocks; so: block sums g and 4 + g of row c; left: blocks of the panel inside the row; half0: all bits in the lanes that hold the first 16
 // values of a block; d8_of, s8_of: block scales and sums of the lane's four result rows.
-template <class F, int RT, class D8, class S8>
+template <class F, int RT, bool ADD, class D8, class S8>
 __device__ __forceinline__ void ts_multiply(F& w, const u32x4_s (&xa)[RT][4], const float (&so)[RT][2], int left, int g, uint32_t half0, D8 d8_of, S8 s8_of,
-                                            f32x4 (&part)[RT]) {
+                                            f32x4 (&sum)[RT]) {
   constexpr bool OFFSET = F::OFF == 1;
   const v4i seed = {kSeedBits, kSeedBits, kSeedBits, kSeedBits};
   float dw[8 * (32 / F::G)];
@@ -118,10 +119,11 @@ __device__ __forceinline__ void ts_multiply(F& w, const u32x4_s (&xa)[RT][4], co
     w.mins(g, m0, m1);
     if (!F::KQ && left < 8) { m0 = g < left ? m0 : 0.0f; m1 = 4 + g < left ? m1 : 0.0f; }
   }
-  // A sum of the panel's own, added to the row's by the caller: the partial sums stay small, and so does what they round off.  So too with the
+  // A sum of the panel's own, added to the row's at its end: the partial sums stay small, and so does what they round off.  So too with the
   // offsets of four blocks, which cancel most of their products: they come between the second and the third (rel-L2 against 64 bits, Q4_K, 5 .. 32
   // rows, activations of one sign / normal: 10.2e-7 / 1.50e-7 with the offsets in front, now 5.8e-7 / 1.33e-7;
   // Q6_K 1.17e-7 with the sum carried on from panel to panel, now 0.95e-7).
+  f32x4 part[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) part[rt] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -173,6 +175,8 @@ __device__ __forceinline__ void ts_multiply(F& w, const u32x4_s (&xa)[RT][4], co
       }
     }
   }
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) sum[rt] = ADD ? sum[rt] + part[rt] : part[rt];
 }
 
 template <class F, int RT, bool GATE, bool SPLIT, int D, bool MOE>
@@ -429,13 +433,13 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
       ++t;
       slot = slot + 1 == D ? 0 : slot + 1;
 
-      f32x4 part[RT];
-      ts_multiply<F, RT>(w, xa, so, left, g, half0, [&](int rt, int b) { return *(const f32x4*)(xd + ts_scale_at<XR>(8 * pl) + ts_scale_at<XR>(b) + 16 * rt + 4 * g); },
-                         [&](int rt, int b) { return *(const f32x4*)(xd + ts_scale_at<XR>(8 * PC) + ts_scale_at<XR>(8 * pl) + ts_scale_at<XR>(b) + 16 * rt + 4 * g); }, part);
-      if (FINER && (p & 1)) odd += part[0];
-      else
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) acc[rt] += part[rt];
+      f32x4 part[RT];                                       // (FINER: of the panel alone)
+      ts_multiply<F, RT, !FINER>(w, xa, so, left, g, half0, [&](int rt, int b) { return *(const f32x4*)(xd + ts_scale_at<XR>(8 * pl) + ts_scale_at<XR>(b) + 16 * rt + 4 * g); },
+                         [&](int rt, int b) { return *(const f32x4*)(xd + ts_scale_at<XR>(8 * PC) + ts_scale_at<XR>(8 * pl) + ts_scale_at<XR>(b) + 16 * rt + 4 * g); }, FINER ? part : acc);
+      if constexpr (FINER) {
+        if (p & 1) odd += part[0];
+        else acc[0] += part[0];
+      }
     }
     // ---- the next chunk of activations
     if constexpr (SPLIT) {
@@ -707,10 +711,7 @@ __device__ __forceinline__ void tile_dealt_body(const uint8_t* __restrict__ W, c
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");    // the place may be filled again
       if (j + 1 < ng) request_w(p, j + 1);
       else if (p + NW < a.np) { request_w(p + NW, 0); request_x(p + NW); }
-      f32x4 part[RT];
-      ts_multiply<F, RT>(w, xa, so, left, g, half0, [&](int rt, int b) { return of(rt, b, 0); }, [&](int rt, int b) { return of(rt, b, 1); }, part);
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) acc[0][rt] += part[rt];
+      ts_multiply<F, RT, true>(w, xa, so, left, g, half0, [&](int rt, int b) { return of(rt, b, 0); }, [&](int rt, int b) { return of(rt, b, 1); }, acc[0]);
       if constexpr (CG > 1) {                               // (the next group's tile first: a tile by number would be in scratch)
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
