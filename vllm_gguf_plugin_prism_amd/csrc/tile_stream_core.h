@@ -563,7 +563,7 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
 // In LDS: the panel's bytes, block scales and sums of its sixteen rows of X (32 bytes each, 512 the plane), their quants, 256 bytes
 // a row.  An operand is 16 bytes of each of sixteen rows, all in the same banks: piece j of row r lies in place j ^ r, which the
 // fetch sees to (a lane asks for the piece that belongs where its bytes land).  Rows past X are fetched up to a multiple of four
-// only: what lies in LDS behind them stands in rows of the result that are not stored.
+// only: the rest of the place holds whatever it held, for rows of the result that are not stored.
 // What bounds it is the weight stream, and beside it the activations' way to every workgroup (2.3 us of [4096,14336]'s 15) and the
 // vector instructions of a panel (Q6_K 350: 5 us).  Without the quantizer's launch, us, streaming tiles / this, 12 rows: Q6_K [4096,14336]
 // 22.1 / 15.1, [4096,4096] 9.6 / 7.1, [1024,4096] 8.5 / 5.9; Q4_K [4096,14336] 16.9 / 11.7, [11008,4096] 13.4 / 10.7, [2048,2048] 5.8 / 4.0; 24
@@ -574,7 +574,15 @@ __global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_st
 // around by one each time: unrolled the compiler keeps more than there are registers.  (A ring of two weight panels per wave: 0.8 to 1.03 times
 // the speed.)  Tried and slower: whole column groups one after the other,
 // the activations fetched again for each (0.86 to 1.06 times the speed of a workgroup each).
-template <class F, int RT> __host__ __device__ constexpr int ts_dealt_place(int ppr, int xn) { return 256 * ppr + 1024 * RT + 1024 * xn; }
+template <int RT> __host__ __device__ constexpr int ts_dealt_place(int ppr) { return 256 * ppr + 1024 * RT + 4096 * RT; }
+// where, behind the panel's bytes, piece 4 i + g of the quants of row 16 rt + c begins
+template <int RT> __host__ __device__ constexpr int ts_dealt_quants(int rt, int i, int c, int g) { return 1024 * RT + 4096 * rt + 256 * c + 16 * ((4 * i + g) ^ c); }
+template <int RT> constexpr bool ts_dealt_reads_inside() {
+  for (int u = 0; u < 256 * RT; ++u)
+    if (ts_dealt_quants<RT>(u >> 8, u & 3, (u >> 2) & 15, (u >> 6) & 3) + 16 > ts_dealt_place<RT>(0)) return false;
+  return true;
+}
+static_assert(ts_dealt_reads_inside<1>() && ts_dealt_reads_inside<2>(), "a wave reads its own place only");
 // (two workgroups of one tile of rows share a CU where its registers suffice)
 template <class F, int RT> constexpr int ts_dealt_waves() { return RT == 1 && !F::HALVES && (F::KQ || F::OFF != 1) ? 4 : 2; }
 template <class F, int RT, int CG>
@@ -590,7 +598,7 @@ __device__ __forceinline__ void tile_dealt_body(const uint8_t* __restrict__ W, c
   if (wg < total8) wg = (wg & 7) * (total8 >> 3) + (wg >> 3);
   const int ng = CG > 2 ? a.passes : CG;                    // column groups, the last of the last workgroup perhaps behind the matrix
   const int xn = (a.M + 3) >> 2;                            // fetches of quants per panel, four rows each
-  const int w_bytes = 256 * a.ppr, place = ts_dealt_place<F, RT>(a.ppr, xn);
+  const int w_bytes = 256 * a.ppr, place = ts_dealt_place<RT>(a.ppr);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
   const int mine = wave * place, table_off = NW * place + 16;   // (a last field's cut may touch the word behind its row)
 
@@ -669,7 +677,7 @@ __device__ __forceinline__ void tile_dealt_body(const uint8_t* __restrict__ W, c
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) xa[rt][i] = *(const u32x4_s*)(scales + 1024 * RT + 4096 * rt + 256 * c + 16 * ((4 * i + g) ^ c));
+      for (int i = 0; i < 4; ++i) xa[rt][i] = *(const u32x4_s*)(scales + ts_dealt_quants<RT>(rt, i, c, g));
       if constexpr (OFFSET) {
         so[rt][0] = *(const float*)(scales + 1024 * rt + 512 + 32 * c + 4 * g);
         so[rt][1] = *(const float*)(scales + 1024 * rt + 512 + 32 * c + 16 + 4 * g);
@@ -888,7 +896,7 @@ static TsArgs ts_dealt_args(const TsCall& c, int ng, size_t& lds) {
   const int64_t pitch = c.w_pitch ? c.w_pitch : (int64_t)(c.K / qk) * bs;
   const bool aligned = F::PB % 16 == 0 && pitch % 16 == 0 && (uintptr_t)c.W % 16 == 0;
   const int ppr = (aligned ? F::PB / 16 : (F::PB + 29) / 16) | 1;   // (odd: banks)
-  lds = (size_t)TS_NW * ts_dealt_place<F, RT>(ppr, (c.M + 3) / 4) + 16 + TsTable<F>::value;
+  lds = (size_t)TS_NW * ts_dealt_place<RT>(ppr) + 16 + TsTable<F>::value;
   const int tiles = RT * (ng > 4 ? 8 : ng > 2 ? 4 : ng);    // (the sum's places are laid out for the most that an instance takes)
   if (lds < (size_t)TS_NW * tiles * 1024) lds = (size_t)TS_NW * tiles * 1024;
   return {c.M, c.N, c.K, (int)q8_kp(c.K), (uint32_t)pitch, (uint32_t)q8_row_bytes(c.K), np, 3, ppr, 0, 0, ng, (uint32_t)((0x100000000ull + ppr - 1) / ppr), 0, 0, 0, 0, 0,
