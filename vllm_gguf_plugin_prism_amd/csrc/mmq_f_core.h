@@ -30,7 +30,8 @@
 // each; a step takes 1.2 us, a super-block, which is four steps and its end, 5.9 (Q6_K 8.0).  So what is left out counts, not
 // what is hidden: with decoding in 30 instead of 50 vector instructions per wave and step (masks and the 1024s as one
 // instruction, high nibbles left where they are), LDS addresses whose constants lie in the instructions (40 additions fewer per
-// super-block) and the contraction in front of the other wave's decoding the same product takes 299 -> 287 us, Q6_K 170 -> 168.  The
+// super-block) and the contraction in front of the other wave's decoding the same product takes 299 -> 287 us; Q6_K ([18944,3584], 512 rows) 169 -> 165, once
+// the addresses of the store are formed behind the loop: held over it they put 7 registers of Q5_K and 11 to 14 of Q6_K into scratch (168).  The
 // contraction alone, matrix instructions and multiply-adds in registers, takes a SIMD 50 to 56 ns per 32 x 32 x 32 block at any
 // interleaving (one wave or two, bursts of one to four blocks, 16 x 16 x 32 tiles): the clock falls as they get denser.
 // Tried and slower: four waves per workgroup and two workgroups per CU (decoding twice), the two waves of a SIMD decoding at
@@ -466,6 +467,7 @@ __global__ __launch_bounds__(64 * MMQF_WM * MMQF_WN, 2) void mmqf_kernel(const u
 
   // ---- store: lane = one row of X, 16 features per tile in runs of four
   float* const mine = sb1 - sb0 < a.r.units ? partial + (int64_t)(2 * work.worker + segment) * (M_T * N_T) : nullptr;
+  const int ln = afresh(lane);                              // (the places formed from it: not in scratch from before the first tile on)
 #pragma unroll
   for (int i = 0; i < TN; ++i)
 #pragma unroll
@@ -474,9 +476,9 @@ __global__ __launch_bounds__(64 * MMQF_WM * MMQF_WN, 2) void mmqf_kernel(const u
       for (int q = 0; q < 4; ++q) {
         const tile_f4v v = {acc[i][k][4 * q], acc[i][k][4 * q + 1], acc[i][k][4 * q + 2], acc[i][k][4 * q + 3]};
         if (mine) {   // in the order of the registers: [wave][tile][run][lane] of four
-          *(tile_f4v*)(mine + (((wave * TN * TM + i * TM + k) * 4 + q) * 64 + lane) * 4) = v;
+          *(tile_f4v*)(mine + (((wave * TN * TM + i * TM + k) * 4 + q) * 64 + ln) * 4) = v;
         } else {
-          tile_store(v, m_base + 32 * (TM * wm + k) + lrow, n_base + 32 * (TN * wn + i) + 8 * q + 4 * lhalf, Y, bias, a.r);
+          tile_store(v, m_base + 32 * (TM * wm + k) + (ln & 31), n_base + 32 * (TN * wn + i) + 8 * q + 4 * (ln >> 5), Y, bias, a.r);
         }
       }
   }
