@@ -233,7 +233,7 @@ __global__ __launch_bounds__(64 * MMQF_WM * MMQF_WN, 2) void mmqf_kernel(const u
   constexpr int BUF = mmqf_buffer_bytes<F>(), PLANE_AT = 2 * BUF + 64 * M_T;
   constexpr int XI = M_T / 8 / NWV;                         // fetches of 8 rows of X per wave and step
   static_assert(4 * N_T == 64 * NWV && M_T == 256, "a thread per part of a row's step; a fetch per row of block scales");
-  extern __shared__ __align__(16) char smem[];
+  extern __shared__ __align__(128) char smem[];             // (rows of 128 bytes, whose pieces are told apart by xor with their addresses)
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN, lrow = lane & 31, lhalf = lane >> 5;
 
