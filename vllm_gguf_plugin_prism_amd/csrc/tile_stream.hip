@@ -362,6 +362,14 @@ namespace gguf {
 int mmvq_any(int type, const void* W, const void* x, void* q8_workspace, void* Y, int xdtype, int64_t N, int64_t K, int64_t M, hipStream_t s, const LinearArgs& la);
 }  // namespace gguf
 
+extern "C" int gguf_linear_dealt(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int gemv) {
+  using namespace gguf;
+  if (N <= 0 || K <= 0 || block_elems(type) == 0 || K % block_elems(type) || !ts_dense_takes(type, M, N, K, w_row_pitch_bytes, gemv != 0)) return 0;
+  LinearArgs la;
+  la.w_pitch = w_row_pitch_bytes;
+  return ts_dense_call(type, nullptr, GGUF_DTYPE_F16, M, (int)N, (int)K, gemv != 0, la).dealt;
+}
+
 extern "C" int gguf_moe_mmq_layer_finer(int type13, int type2, int64_t H, int64_t I, int64_t N_out, int64_t top_k, int64_t tokens, int64_t num_experts, int product) {
   using namespace gguf;
   if (H <= 0 || I <= 0 || N_out <= 0 || top_k <= 0 || tokens <= 0 || num_experts <= 0 || product < 1 || product > 2) return -1;

@@ -234,12 +234,18 @@ def _dense_result_fits(X: torch.Tensor, row: int, out: torch.Tensor | None, bias
 
 
 def _mmq_route(quant_type: int, row: int, col: int, vecs: int, w_pitch: int, workspace_bytes: int | None = None) -> int:
-    """The kernel that :func:`ggml_mul_mat_a8` runs on its own workspace or one of this size: 1 the streaming tile kernel,
-    4 the wide tiles, 2 the half-precision unit's whole-number GEMM, 0 another (up to 32 rows: the one behind tile_dealt_kernel)."""
+    """The kernel that :func:`ggml_mul_mat_a8` runs on its own workspace or one of this size where not :func:`_linear_dealt`: 1 the streaming
+    tile kernel, 4 the wide tiles, 2 the half-precision unit's whole-number GEMM, 0 another."""
     L = _lib.lib()
     if workspace_bytes is None:
         workspace_bytes = L.gguf_mmq_layer_workspace_bytes(int(quant_type), row, col, vecs, w_pitch)
     return L.gguf_mmq_layer_route(int(quant_type), row, col, vecs, w_pitch, workspace_bytes)
+
+
+def _linear_dealt(quant_type: int, row: int, col: int, vecs: int, w_pitch: int, gemv: bool = False) -> bool:
+    """Whether :func:`ggml_mul_mat_a8` (``gemv``: :func:`ggml_mul_mat_vec_a8`) runs tile_dealt_kernel, which comes before the
+    kernels of :func:`_mmq_route`."""
+    return bool(_lib.lib().gguf_linear_dealt(int(quant_type), row, col, vecs, w_pitch, int(gemv)))
 
 
 def _mmq_unit(quant_type: int, row: int, col: int, vecs: int, w_pitch: int) -> int:
