@@ -107,34 +107,63 @@ static double ts_most_work(int type) {
   return 0;
 }
 
-// Where the panels of a column group are dealt to the waves of a workgroup (tile_dealt_kernel) instead.  Against whatever ran before (the
-// streaming tiles, the kernel of the packed blocks, the staged 16-row tiles, the GEMV), over 7900 random products of 5 .. 32 rows, N 256 ..
-// 28672, K 512 .. 18944, both operators, with one column group per workgroup: where these lines take it 1.28 times as fast on average, over all 1.21
-// (Q2_K 1.30, Q3_K 1.27, Q4_1 1.22, Q4_K, Q6_K, Q8_0, Q4_0 1.20, Q5_K, Q5_0 1.16, IQ4_XS 1.25, IQ2 and IQ3 1.16 to 1.19); one in sixty is slower by more
-// than 3 %, the worst by 20 %.  With several, 17 .. 32 rows and more than 4096 columns are 1.11 times as fast again (700 products; up to 1.5).  us, before
+// Where the panels of a column group are dealt to the waves of a workgroup (tile_dealt_kernel) instead.  Against what runs otherwise (the
+// streaming tiles, the kernel of the packed blocks, the staged 16-row tiles, the GEMV), over 23000 random products of 5 .. 32 rows, N 256 ..
+// 57344, K 512 .. 18944, both operators: 1.21 times as fast over all; one in 180 is slower by more than 3 %, the worst by 15 %.  us, before
 // / dealt: [4096,4096] 12 rows Q4_K 11.0 / 8.4, Q6_K 12.5 / 10.0, [4096,14336] 12 rows Q6_K 25.4 / 18.9, [2048,2048] Q4_K 8.5 / 6.7.
-static bool ts_dealt_takes(int type, int64_t M, int64_t N, int64_t K) {
+// What it has against it are short rows, where the sum of eight partial tiles and the activations' way to every workgroup weigh, and the sizes that
+// suit the streaming tiles best: their workgroups fill more than 0.76 of a round with 779 .. 1024 column groups (a pair of waves each)
+// and with 1557 .. 2048 (`full`, `round`).
+static bool ts_dealt_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, bool gemv) {
   if (M < 5 || M > 32 || N > 0x7FFFFFF0ll || K > 0x7FFFFFF0ll) return false;
   const int64_t groups = (N + 15) / 16, np = (K + 255) / 256;
-  // (a long K on few columns is cut between workgroups by the kernel of the packed blocks: [832,15872] Q6_K 11 rows 13.9 / 17.0)
-  if ((type == T_Q4_K || type == T_Q5_K || type == T_Q6_K) && groups <= 56 && K > 13000) return false;
-  if (type == T_Q2_K && M > 16) return groups <= 256 || (K >= 4096 && groups <= 768);
   const bool blocks32 = type == T_Q4_0 || type == T_Q4_1 || type == T_Q5_0 || type == T_Q5_1 || type == T_Q8_0 || type == T_IQ4_NL;
-  const bool halves = type == T_Q4_1 || type == T_Q5_1;
+  const bool halves = type == T_Q4_1 || type == T_Q5_1, packed = type == T_Q4_K || type == T_Q5_K || type == T_Q6_K;
+  const bool grids = type == T_IQ2_XXS || type == T_IQ2_XS || type == T_IQ2_S || type == T_IQ3_XXS || type == T_IQ3_S;
+  const bool round = groups > 1556 && groups <= 2048, full = round || (groups > 778 && groups <= 1024);
+  // The tile operator's kernel of the packed blocks cuts a long K on few columns between workgroups ([832,15872] Q6_K 11 rows 13.9 / 17.0, [624,11520]
+  // Q5_K 31 rows 13.6 / 15.5, [416,17440] Q4_0 26 rows 19.3 / 22.5); the GEMV operator, which has none, is 1.4 to 1.7 times as fast dealt.
+  if (!gemv && packed && groups <= (M > 16 ? 64 : 56) && K > (M > 16 ? 11000 : 13000)) return false;
+  if (!gemv && type == T_Q4_0 && M > 16 && groups <= 56 && K > 13000) return false;
   // Two tiles of rows: workgroups of several groups (ts_dealt_groups); past two groups rows must be long enough for the sum at their end.  us, the
   // streaming tiles / dealt, 20 rows: [14336,1536] Q4_K 10.4 / 8.7, [28672,1536] 14.0 / 14.2, [18944,4096] 27.3 / 19.5, [65536,4096] 58.4 / 55.1;
-  // Q8_0 [19008,2304] 24.0 / 25.4; Q5_K, at most four groups, [25728,3328] 29.2 / 33.0
-  if (M > 16) return groups <= 512 || (K >= 1024 && K >= (halves ? 2 * groups - 512 : blocks32 || type == T_Q5_K ? 4 * groups - 2048 : groups + groups / 4));
-  // Two panels per row are work for two waves of eight.  Past 1408 groups workgroups of two read the activations half as often: [28672,4096] 12 rows
-  // Q6_K 32.0 / 30.0, [33056,8192] 8 rows Q4_K 61.7 / 41.1, IQ2_XXS from 2050 groups on 1.4 to 1.6 times as fast; but Q4_K, whose decoding is the
-  // least, up to two full rounds at nine rows and more ([25456,10496] 44.6 / 48.6, [28672,4096] 20.4 / 20.9), and Q2_K, one group always.
-  const bool behind = type == T_Q2_K ? groups > 1536 : type == T_Q4_K && M >= 9 && groups > 1536 && groups <= 2048;
-  if (!blocks32) return (!behind && groups <= 256 * np) || K >= 12000;
+  // full: [13800,1280] Q6_K 23 rows 12.8 / 14.6, [25772,2304] IQ4_XS 23.5 / 25.2, but [16384,2048] Q4_K 1.13 times as fast.
+  if (M > 16) {
+    if (type == T_Q2_K) return groups <= 256 || (K >= 4096 && groups <= 768);
+    if (groups <= 512) return true;
+    if (K < 1024) return false;
+    if (halves) return K >= (full ? 2 * groups : 2 * groups - 512);
+    // (blocks of 32 values and Q5_K: at most four groups; [17952,2560] Q8_0 29 rows 22.7 / 26.0, [23152,4352] 33.9 / 36.8, [27289,4864] 38.1 / 43.3)
+    if (type == T_Q8_0) return round ? K > 8192 : K >= 4 * groups - (groups <= 768 ? 2048 : 1800);
+    if (blocks32 || type == T_Q5_K) return round ? K >= 6144 : K >= 4 * groups - (full ? 1024 : 2048);
+    return K >= (full ? groups * 7 / 4 : groups * 5 / 4);
+  }
+  if (!blocks32) {
+    // Two panels per row are work for two waves of eight.
+    if (groups > 256 * np && K < 12000) return false;
+    // Past one round the formats that decode least lose most to it: [25456,10496] Q4_K 9 rows 44.6 / 48.6, [28656,3840] Q5_K 15 rows 23.3 / 25.8, both at 0.9 to
+    // 1.0 of the speed at any K; Q6_K and IQ4_XS up to 4096 ([28672,4096] Q6_K 12 rows 0.97), grids up to 2048, Q2_K, one group always, up to 12000.
+    // Before and behind it the dealt kernel reads the activations once per two groups, or has the CUs that the others leave: [24000,4096] Q4_K
+    // 1.05, [36000,4096] 1.18 times as fast, grids 1.3 to 1.6.
+    if (type == T_Q2_K) return groups <= 1536 || K >= 12000;
+    if (packed && type != T_Q6_K && round) return false;
+    if ((type == T_Q6_K || type == T_IQ4_XS) && round) return K > 4096;
+    // (Q4_K: [20224,1280] 15 rows 10.2 / 10.8; four fetches of activations a panel: [22224,11008] 16 rows 45.6 / 52.0, 14 rows 1.01)
+    if (type == T_Q4_K && groups > 1024) return K > 2048 && (M <= 14 || groups > 1536);
+    // (IQ2_S, the most lookups in the registers of one group: [14400,1280] 11 rows 11.4 / 13.8, [14304,1792] 13.6 / 14.8, [30720,2560] 25.5 / 29.5)
+    if (grids && groups > 512) return K > (type != T_IQ2_S ? (round ? 2048 : 1280) : round ? 3072 : full ? 2048 : 1536);
+    // (the GEMV, one launch: [1760,768] 6 rows 4.8 / 5.2, [3136,1280] 5.6 / 6.0)
+    return !(type == T_IQ4_XS && M <= 8 && groups <= 256 && K < 2048);
+  }
   // (these decode more per panel, or keep two values per block and row: the beginning weighs less there)
+  if (type == T_Q8_0 && full) return false;                 // [13712,12032] 14 rows 42.0 / 47.3, [26720,4096] 16 rows 28.1 / 31.0; 0.98 of the speed on average
+  if (type == T_Q4_0 && round && K < (M >= 9 ? 8192 : 4096)) return false;   // [27664,4832] 16 rows 34.7 / 37.4, [26592,2816] 5 rows 19.6 / 21.5
   if (M >= 9) return groups <= 512 || K >= 4096 || (halves && K >= 2 * groups - 512);
-  // the GEMV, one launch, is ahead on short rows, with Q5_0 and Q8_0 on small matrices ([480,2336] Q8_0 5 rows 5.4 / 6.9)
-  if (halves) return K >= 2048 && (groups <= 512 || K >= 4096);
-  return K >= 2048 && (N * K > 3000000 || (type != T_Q5_0 && type != T_Q8_0));
+  // the GEMV, one launch, is ahead on short rows, with Q5_0 and Q8_0 on small matrices ([480,2336] Q8_0 5 rows 5.4 / 6.9) and where rows that do not begin
+  // on 16 bytes are cut out of two reads each ([1072,2272] Q5_1 5 rows 6.0 / 7.3, [736,2752] Q4_0 6.0 / 6.6; up to 14 % with longer ones of few columns)
+  if (K < 2048 || (halves && groups > 512 && K < 4096)) return false;
+  if (M <= 6 && w_pitch % 16 != 0 && K < 4096 && N * K <= 6000000 && type != T_IQ4_NL) return false;
+  return N * K > 3000000 || (type != T_Q5_0 && type != T_Q8_0);
 }
 
 // Where tile_stream_kernel is the faster one of those that do not deal panels.
@@ -186,7 +215,7 @@ bool ts_stream_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch,
 
 // Dense products on either kernel.
 bool ts_dense_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, bool gemv) {
-  return ((gemv ? ts_gemv_type_ok(type) : ts_tile_type_ok(type)) && ts_dealt_takes(type, M, N, K) && ts_size_ok(N, w_pitch, M, K)) ||
+  return ((gemv ? ts_gemv_type_ok(type) : ts_tile_type_ok(type)) && ts_dealt_takes(type, M, N, K, w_pitch, gemv) && ts_size_ok(N, w_pitch, M, K)) ||
          ts_stream_takes(type, M, N, K, w_pitch, gemv);
 }
 
@@ -286,13 +315,14 @@ static TsCall ts_dense_call(int type, const void* W, int dtype, int64_t M, int N
   c.rt = M <= 16 ? 1 : 2;
   c.w_pitch = la.w_pitch; c.ldy = la.ldy; c.bias = la.bias;
   c.gemv = gemv;
-  c.dealt = ts_dealt_takes(type, M, N, K);
+  c.dealt = ts_dealt_takes(type, M, N, K, la.w_pitch ? la.w_pitch : (int64_t)K / block_elems(type) * block_bytes(type), gemv);
   c.gemv_sums = gemv && (type == T_Q4_K || type == T_Q5_K);   // (the others' offset is on the stored sums there too)
   return c;
 }
 
 bool ts_two_takes(int type, int64_t N, int64_t w_pitch, bool gemv, int type2, int64_t N2, int64_t w_pitch2, bool gemv2, int64_t K, int64_t M) {
-  return ts_dense_takes(type, M, N, K, w_pitch, gemv) && ts_dense_takes(type2, M, N2, K, w_pitch2, gemv2) && ts_dealt_takes(type, M, N, K) && ts_dealt_takes(type2, M, N2, K);
+  return ts_dense_takes(type, M, N, K, w_pitch, gemv) && ts_dense_takes(type2, M, N2, K, w_pitch2, gemv2) && ts_dealt_takes(type, M, N, K, w_pitch, gemv) &&
+         ts_dealt_takes(type2, M, N2, K, w_pitch2, gemv2);
 }
 
 int ts_two(const TsShard& a, const TsShard& b, const void* x, int dtype, void* workspace, int64_t M, int K, hipStream_t s) {
