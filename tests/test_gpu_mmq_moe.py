@@ -819,8 +819,9 @@ def test_mmq_nine_to_32_rows(qtype, dt):
 @pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("qtype", [o.Q4_K, o.Q5_K, o.Q6_K, o.Q4_0, o.Q8_0])
 def test_mmq_up_to_16_rows_from_packed_blocks(qtype, dt):
-    """Q4_K, Q5_K, Q6_K with at most 32 rows of X (and Q4_0, Q8_0 with nine to 16) build their MFMA operands straight from the packed blocks, K split over the waves
-    of a workgroup: one super-block of K, a stretch that fills LDS (K = 4096), K beyond it (split over workgroups as
+    """Q4_K, Q5_K, Q6_K with at most 32 rows of X (and Q4_0, Q8_0 with nine to 16), whose MFMA operands are built straight from the packed blocks, K split over the waves
+    of a workgroup (most of these sizes have their panels dealt to the waves by now; K split over workgroups: test_gpu_few_rows.py,
+    test_kernels_of_what_is_not_dealt): one super-block of K, a stretch that fills LDS (K = 4096), K beyond it (split over workgroups as
     well, and the same call without room for partial tiles), few columns (split down to a super-block per wave), the
     two-column-tile variant of wide outputs with a ragged last tile, a row slice of a wider weight tensor with bias
     into a column slice of a wider result, and a slice whose rows are not 16-byte aligned (Q4_K / Q5_K take the staged

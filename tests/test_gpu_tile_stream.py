@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 SHORT, DEEP = (o.Q4_0, o.Q8_0), (o.Q4_K, o.Q5_K, o.Q6_K)
 
 
-# one and two tiles of rows, full and with a row over; a last column group of one column; rows of X shorter than a panel,
+# (dealt to the waves of a workgroup, all but one) one and two tiles of rows, full and with a row over; a last column group of one column; rows of X shorter than a panel,
 # ending inside one, in one chunk, in two, in more than a chunk's double buffer; rows of W a pitch apart that moves them
 # through all positions inside 16 bytes
 @pytest.mark.parametrize("qtype,m,n,k,pad", [(q, *s) for q in SHORT for s in (
@@ -60,8 +60,9 @@ def check_layer(qtype, tokens, e, hid, inner, routing=None):
     assert o.rel_l2(got.cpu().numpy(), want) <= 1e-3
 
 
-# sizes that the cost rule sends here: more column groups than a round of workgroups holds and a last one in part, K in
-# chunks, one and two tiles of rows, fewer rows than half a tile
+# sizes that the cost rule sends here from the other kernels; all but the widest have their panels dealt to the waves of a workgroup (what is not:
+# test_gpu_few_rows.py, test_kernels_of_what_is_not_dealt): more column groups than a round of workgroups holds and a last one in part, one and
+# two tiles of rows, fewer rows than half a tile
 @pytest.mark.parametrize("qtype,m,n,k", [(q, *s) for q in DEEP for s in ((5, 5200, 4352), (24, 5205, 4096), (8, 12300, 2304), (16, 28688, 512))] + [
     (o.Q4_0, 12, 2560, 4096), (o.Q8_0, 24, 2048, 8192)])
 def test_dense_where_it_is_taken(qtype, m, n, k):
