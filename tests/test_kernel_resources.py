@@ -7,7 +7,9 @@ import pytest
 from vllm_gguf_plugin_prism_amd import _lib
 
 # Kernels whose registers are counted out: a value that goes to scratch is a trip through memory, per tile or per step.
-WHOLE_IN_REGISTERS = ("mmqf_kernel", "tile_stream_kernel", "tile_dealt_pair_kernel", "tile_wide_kernel", "mmvq_pair_kernel")
+# (IQ3_S with one tile of rows and two column groups: three registers, and faster than with one group by 3 %)
+EXCEPT = ("6TIQ3_SELi1ELi2E",)
+WHOLE_IN_REGISTERS = ("mmqf_kernel", "tile_stream_kernel", "tile_dealt_kernel", "tile_dealt_pair_kernel", "tile_wide_kernel", "mmvq_pair_kernel")
 
 
 def kernels(data: bytes):
@@ -47,4 +49,4 @@ def scratch():
 @pytest.mark.parametrize("kernel", WHOLE_IN_REGISTERS)
 def test_nothing_goes_to_scratch(kernel, scratch):
     of = {name: n for name, n in scratch.items() if f"{len(kernel)}{kernel}I" in name}   # (mangled: length, name, template arguments)
-    assert of and not {name: n for name, n in of.items() if n}
+    assert of and not {name: n for name, n in of.items() if n and not any(e in name for e in EXCEPT)}

@@ -633,7 +633,7 @@ __device__ __forceinline__ void tile_dealt_body(const uint8_t* __restrict__ W, c
     int l = lane;                                           // (opaque: computed every time, not kept in registers over the groups)
     if constexpr (CG > 1) asm volatile("" : "+v"(l));
     const int c = l & 15, g = l >> 4;
-  uint32_t x_at[4 * RT], s_at[RT];
+    uint32_t x_at[4 * RT], s_at[RT];
 #pragma unroll
     for (int i = 0; i < 4 * RT; ++i) {
       const int row = 4 * i + g;
@@ -874,7 +874,7 @@ static int ts_launch(const TsCall& c, int ks, hipStream_t stream) {
 // let one round do, up to what the registers hold: [11008,4096] Q4_K 20 rows, one to four groups 16.1 / 16.8 / 12.2 / 13.8 us, [28672,4096]
 // 35.5 / 32.3 / 32.2 / 27.5, eight 25.9.  Where two share a CU, two groups between one and a half rounds and two, and past two and three
 // quarters: [16384,4096] Q4_K 12 rows 14.3 / 12.6, but [10000,4096] 0.9 of the speed; of those formats whose two groups fit the registers (the
-// others spill: Q6_K 0.9, IQ2_S 0.95 of the speed).  (Q2_K, two products per block, spills, Q5_K at eight.)
+// others spill: Q6_K 0.9, IQ2_S 0.95 of the speed; IQ3_S spills three and gains 1.03 all the same).  (Q2_K, two products per block, spills, Q5_K at eight.)
 template <class F, class = void> struct TsOneGroup { static constexpr bool value = false; };   // F::ONE_GROUP: registers for one group at four waves per SIMD
 template <class F> struct TsOneGroup<F, std::void_t<decltype(F::ONE_GROUP)>> { static constexpr bool value = F::ONE_GROUP; };
 template <class F, int RT> constexpr int ts_dealt_most() {
