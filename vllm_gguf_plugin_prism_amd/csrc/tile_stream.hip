@@ -109,60 +109,62 @@ static double ts_most_work(int type) {
 
 // Where the panels of a column group are dealt to the waves of a workgroup (tile_dealt_kernel) instead.  Against what runs otherwise (the
 // streaming tiles, the kernel of the packed blocks, the staged 16-row tiles, the GEMV), over 23000 random products of 5 .. 32 rows, N 256 ..
-// 57344, K 512 .. 18944, both operators: 1.21 times as fast over all; one in 180 is slower by more than 3 %, the worst by 15 %.  us, before
+// 57344, K 512 .. 18944, both operators: 1.21 times as fast over all; one in 140 is slower by more than 3 %, the worst by 22 %.  us, before
 // / dealt: [4096,4096] 12 rows Q4_K 11.0 / 8.4, Q6_K 12.5 / 10.0, [4096,14336] 12 rows Q6_K 25.4 / 18.9, [2048,2048] Q4_K 8.5 / 6.7.
-// What it has against it are short rows, where the sum of eight partial tiles and the activations' way to every workgroup weigh, and the sizes that
-// suit the streaming tiles best: their workgroups fill more than 0.76 of a round with 779 .. 1024 column groups (a pair of waves each)
-// and with 1557 .. 2048 (`full`, `round`).
+// What it has against it are short rows, where the sum of eight partial tiles and the activations' way to every workgroup weigh, panels that the eight
+// waves cannot share evenly (K = 1280: five of them, 2304: one with two), and the sizes that suit the streaming tiles best: their workgroups fill
+// more than 0.76 of a round with 779 .. 1024 column groups (a pair of waves each) and with 1557 .. 2048 (`full`, `round`).
 static bool ts_dealt_takes(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, bool gemv) {
   if (M < 5 || M > 32 || N > 0x7FFFFFF0ll || K > 0x7FFFFFF0ll) return false;
   const int64_t groups = (N + 15) / 16, np = (K + 255) / 256;
   const bool blocks32 = type == T_Q4_0 || type == T_Q4_1 || type == T_Q5_0 || type == T_Q5_1 || type == T_Q8_0 || type == T_IQ4_NL;
   const bool halves = type == T_Q4_1 || type == T_Q5_1, packed = type == T_Q4_K || type == T_Q5_K || type == T_Q6_K;
   const bool grids = type == T_IQ2_XXS || type == T_IQ2_XS || type == T_IQ2_S || type == T_IQ3_XXS || type == T_IQ3_S;
-  const bool round = groups > 1556 && groups <= 2048, full = round || (groups > 778 && groups <= 1024);
-  // The tile operator's kernel of the packed blocks cuts a long K on few columns between workgroups ([832,15872] Q6_K 11 rows 13.9 / 17.0, [624,11520]
-  // Q5_K 31 rows 13.6 / 15.5, [416,17440] Q4_0 26 rows 19.3 / 22.5); the GEMV operator, which has none, is 1.4 to 1.7 times as fast dealt.
-  if (!gemv && packed && groups <= (M > 16 ? 64 : 56) && K > (M > 16 ? 11000 : 13000)) return false;
-  if (!gemv && type == T_Q4_0 && M > 16 && groups <= 56 && K > 13000) return false;
+  const bool round = groups > 1556 && groups <= 2048, full = round || (groups > 778 && groups <= 1024), even = (np & 7) == 0 || (np & 7) == 7;
+  // The tile operator's kernel of the packed blocks cuts a long K on few columns between workgroups ([832,15872] Q6_K 11 rows 13.9 / 17.0); the GEMV
+  // operator, which has none, is 1.4 to 1.7 times as fast dealt.  (Not from shorter rows on, where that is as fast on average, [528,12800] Q5_K 29
+  // rows 14.3 / 15.9 at worst: q, k and v of two formats share a launch only where each is dealt, [432,11008] Q6_K beside [256,11008] Q5_K 19 rows 39 / 17.)
+  if (!gemv && packed && groups <= 56 && K > 13000) return false;
   // Two tiles of rows: workgroups of several groups (ts_dealt_groups); past two groups rows must be long enough for the sum at their end.  us, the
   // streaming tiles / dealt, 20 rows: [14336,1536] Q4_K 10.4 / 8.7, [28672,1536] 14.0 / 14.2, [18944,4096] 27.3 / 19.5, [65536,4096] 58.4 / 55.1;
   // full: [13800,1280] Q6_K 23 rows 12.8 / 14.6, [25772,2304] IQ4_XS 23.5 / 25.2, but [16384,2048] Q4_K 1.13 times as fast.
   if (M > 16) {
     if (type == T_Q2_K) return groups <= 256 || (K >= 4096 && groups <= 768);
     if (groups <= 512) return true;
-    if (K < 1024) return false;
-    if (halves) return K >= (full ? 2 * groups : 2 * groups - 512);
-    // (blocks of 32 values and Q5_K: at most four groups; [17952,2560] Q8_0 29 rows 22.7 / 26.0, [23152,4352] 33.9 / 36.8, [27289,4864] 38.1 / 43.3)
-    if (type == T_Q8_0) return round ? K > 8192 : K >= 4 * groups - (groups <= 768 ? 2048 : 1800);
-    if (blocks32 || type == T_Q5_K) return round ? K >= 6144 : K >= 4 * groups - (full ? 1024 : 2048);
-    return K >= (full ? groups * 7 / 4 : groups * 5 / 4);
+    if (K < 1024 || (full && np <= 5)) return false;
+    if (halves) return K >= 2 * groups - 512;
+    // (blocks of 32 values and Q5_K: at most four groups; [17952,2560] Q8_0 29 rows 22.7 / 26.0, [14384,2304] 17.1 / 17.9, [27289,4864] 38.1 / 43.3)
+    if (type == T_Q8_0) return round ? K > 8192 : K >= 4 * groups - (groups <= 1024 ? 2048 : 1800) && !(full && np > 8 && np <= 12);
+    if (blocks32 || type == T_Q5_K) return round ? K >= (type == T_Q5_0 ? 4608 : 6144) : K >= 4 * groups - 2048;
+    return K >= groups * 5 / 4 && !(round && np == 9);
   }
   if (!blocks32) {
     // Two panels per row are work for two waves of eight.
     if (groups > 256 * np && K < 12000) return false;
-    // Past one round the formats that decode least lose most to it: [25456,10496] Q4_K 9 rows 44.6 / 48.6, [28656,3840] Q5_K 15 rows 23.3 / 25.8, both at 0.9 to
-    // 1.0 of the speed at any K; Q6_K and IQ4_XS up to 4096 ([28672,4096] Q6_K 12 rows 0.97), grids up to 2048, Q2_K, one group always, up to 12000.
+    // A round: the formats that decode least lose most, [25456,10496] Q4_K 9 rows 44.6 / 48.6, [28656,3840] Q5_K 15 rows 23.3 / 25.8, 0.9 to 1.0 of the speed; Q6_K
+    // and IQ4_XS up to 4096 ([26704,2304] Q6_K 16 rows 22.0 / 23.3, but, even, [26896,2048] 10 rows 22.7 / 20.7), grids up to 2048, Q2_K, one group always, up to 12000.
     // Before and behind it the dealt kernel reads the activations once per two groups, or has the CUs that the others leave: [24000,4096] Q4_K
     // 1.05, [36000,4096] 1.18 times as fast, grids 1.3 to 1.6.
     if (type == T_Q2_K) return groups <= 1536 || K >= 12000;
-    if (packed && type != T_Q6_K && round) return false;
-    if ((type == T_Q6_K || type == T_IQ4_XS) && round) return K > 4096;
-    // (Q4_K: [20224,1280] 15 rows 10.2 / 10.8; four fetches of activations a panel: [22224,11008] 16 rows 45.6 / 52.0, 14 rows 1.01)
-    if (type == T_Q4_K && groups > 1024) return K > 2048 && (M <= 14 || groups > 1536);
-    // (IQ2_S, the most lookups in the registers of one group: [14400,1280] 11 rows 11.4 / 13.8, [14304,1792] 13.6 / 14.8, [30720,2560] 25.5 / 29.5)
-    if (grids && groups > 512) return K > (type != T_IQ2_S ? (round ? 2048 : 1280) : round ? 3072 : full ? 2048 : 1536);
-    // (the GEMV, one launch: [1760,768] 6 rows 4.8 / 5.2, [3136,1280] 5.6 / 6.0)
-    return !(type == T_IQ4_XS && M <= 8 && groups <= 256 && K < 2048);
+    if (type == T_Q4_K && round) return K >= 12000;
+    if (type == T_Q5_K && round) return K > (M <= 8 ? 4096 : 8192);
+    if ((type == T_Q6_K || type == T_IQ4_XS) && round) return K > 4096 || even;
+    if (type == T_Q4_K && groups > 1024) return K > 1536;   // [20224,1280] 15 rows 10.2 / 10.8
+    // (IQ2_S, the most lookups in the registers of one group: [14400,1280] 11 rows 11.4 / 13.8, [14304,1792] 13.6 / 14.8, [30720,2560] 25.5 / 29.5;
+    // up to eight rows the others are the GEMV: [10640,768] IQ2_XS 6 rows 10.1 / 8.5)
+    if (type == T_IQ2_S && groups > 512 && M >= 9) return K > (round ? 3072 : full ? 2048 : 1536);
+    if (grids && groups > 512 && M >= 9) return K > (round ? 2048 : 768) || (round && even);   // [10064,768] IQ2_XXS 13 rows 8.1 / 8.7
+    // (IQ4_XS up to eight rows on the GEMV is one launch, [1760,768] 6 rows 4.8 / 5.2, but beside Q5_K 11 / 6)
+    return true;
   }
   // (these decode more per panel, or keep two values per block and row: the beginning weighs less there)
-  if (type == T_Q8_0 && full) return false;                 // [13712,12032] 14 rows 42.0 / 47.3, [26720,4096] 16 rows 28.1 / 31.0; 0.98 of the speed on average
-  if (type == T_Q4_0 && round && K < (M >= 9 ? 8192 : 4096)) return false;   // [27664,4832] 16 rows 34.7 / 37.4, [26592,2816] 5 rows 19.6 / 21.5
+  if ((type == T_Q8_0 || type == T_Q4_0) && round && M >= 9 && K < 8192) return false;   // [26720,4096] Q8_0 16 rows 28.1 / 31.0, [27664,4832] Q4_0 34.7 / 37.4
+  if (type == T_Q4_0 && round && M <= 6 && K < 4096) return false;   // [26592,2816] 5 rows 19.6 / 21.5, but [27156,2560] 8 rows 27.9 / 21.5
   if (M >= 9) return groups <= 512 || K >= 4096 || (halves && K >= 2 * groups - 512);
   // the GEMV, one launch, is ahead on short rows, with Q5_0 and Q8_0 on small matrices ([480,2336] Q8_0 5 rows 5.4 / 6.9) and where rows that do not begin
-  // on 16 bytes are cut out of two reads each ([1072,2272] Q5_1 5 rows 6.0 / 7.3, [736,2752] Q4_0 6.0 / 6.6; up to 14 % with longer ones of few columns)
+  // on 16 bytes are cut out of two reads each ([1072,2272] Q5_1 5 rows 6.0 / 7.3; up to 14 % with longer ones of few columns)
   if (K < 2048 || (halves && groups > 512 && K < 4096)) return false;
-  if (M <= 6 && w_pitch % 16 != 0 && K < 4096 && N * K <= 6000000 && type != T_IQ4_NL) return false;
+  if (M <= 6 && w_pitch % 16 != 0 && K < 2560 && N * K <= 6000000 && type != T_IQ4_NL) return false;
   return N * K > 3000000 || (type != T_Q5_0 && type != T_Q8_0);
 }
 
