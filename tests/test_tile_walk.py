@@ -1,0 +1,30 @@
+"""Which products the walking tile kernel (csrc/tile_walk_core.h) takes, and what the compiler gave it (no GPU needed)."""
+import pytest
+
+from test_kernel_resources import kernels
+from vllm_gguf_plugin_prism_amd import _lib, ops
+
+Q4_0, Q5_0, Q8_0, Q4_K, Q5_K, Q6_K = 2, 6, 8, 12, 13, 14
+
+
+# measured, us, the kernels that run otherwise / walked
+@pytest.mark.parametrize("qt,m,n,k,plan", [
+    (Q8_0, 77, 14336, 4096, (3, 4)), (Q4_K, 64, 4096, 4096, (1, 8)), (Q4_K, 128, 4096, 4096, (2, 8)), (Q8_0, 64, 4096, 4096, (1, 8)),   # 38.7 / 26.5, 16.1 / 10.8, 24.9 / 13.2, 19.4 / 12.6
+    (Q4_K, 1501, 25456, 512, (0, 0)), (Q4_K, 1319, 8368, 512, (0, 0)), (Q6_K, 64, 4096, 4096, (0, 0)),                                  # 91 / 137, 37 / 50, not a format of it
+    (Q4_K, 32, 4096, 4096, (0, 0)), (Q4_K, 2049, 4096, 4096, (0, 0))])                                                                  # at most 32 rows; not measured
+def test_the_faster_kernel_is_taken(qt, m, n, k, plan):
+    qk, size = ops.quant_sizes(qt)
+    assert ops._linear_walk(qt, n, k, m, k // qk * size) == plan
+
+
+# the records of 33 rows are those of 64: more than the quantized rows, which are the least that a workspace holds
+def test_a_workspace_without_room_is_not_taken():
+    L, m, n, k, pitch = _lib.lib(), 33, 4096, 4096, 4096 // 256 * 144
+    records = 64 * k // 256 * 288
+    assert records > m * L.gguf_q8_1_row_bytes(k) and L.gguf_mmq_layer_workspace_bytes(Q4_K, n, k, m, pitch) >= records
+    assert ops._linear_walk(Q4_K, n, k, m, pitch, records)[0] and ops._linear_walk(Q4_K, n, k, m, pitch, records - 1) == (0, 0)
+
+
+def test_nothing_goes_to_scratch():
+    of = {name: n for name, n in kernels(_lib.LIB_PATH.read_bytes()) if "16tile_walk_kernelI" in name}
+    assert of and not any(of.values())

@@ -9,10 +9,12 @@
  *
  * gguf_mmq_layer_workspace_bytes: the workspace with which gguf_mmq_linear on GGUF_MMQ_AUTO runs at full speed for weights
  * of this type, at a 16-byte boundary.  (gguf_mmq_workspace_bytes_engine does not know the type.)  gguf_mmq_layer_route: the
- * kernel that such a call with a workspace of this size runs where its panels are not dealt: 1 the streaming tile kernel, 4 the wide tiles, 2 the
+ * kernel that such a call with a workspace of this size runs where it is neither dealt nor walked: 1 the streaming tile kernel, 4 the wide tiles, 2 the
  * half-precision unit's, 0 another.  gguf_linear_dealt: 1 where they are, by tile_dealt_kernel, which comes before all of these (5 .. 32 rows;
  * gemv: of gguf_mmvq_linear), with rows in a workspace that begins on 16 bytes.
- * gguf_mmq_layer_unit: the same, with 2 added to 1 (past 32 rows) and 4 where the half-precision unit would run a call that these decline.  gguf_moe_mmq_layer_wide: whether
+ * gguf_linear_walk: where a call of more than 32 rows with a workspace of this size runs tile_walk_kernel, which comes before them too, 16 times the tiles of
+ * 32 rows that a workgroup has and its waves, else 0.
+ * gguf_mmq_layer_unit: the kernel of gguf_mmq_layer_route, with 2 added to 1 (past 32 rows) and 4 where the half-precision unit would run a call that these decline.  gguf_moe_mmq_layer_wide: whether
  * gguf_moe_mmq_layer with the workspace it asks for, at addresses divisible by 16, runs on the wide tiles.
  * gguf_moe_mmq_layer_finer: the block of 16 slots from which on the first or second product (product) of a layer on the streaming tiles deals K to
  * two waves each; -1: none, or a layer that they do not take.
@@ -37,6 +39,7 @@ int gguf_mmq_layer_unit(int type, int64_t N, int64_t K, int64_t M, int64_t w_row
 int gguf_linear_two_takes(int type, int64_t N, int64_t w_row_pitch_bytes, int type2, int64_t N2, int64_t w_row_pitch_bytes2, int64_t K, int64_t M, int gemv);
 int gguf_linear_two(const void* W, int64_t w_row_pitch_bytes, int type, int64_t N, void* Y, const void* bias, const void* W2, int64_t w_row_pitch_bytes2, int type2,
                     int64_t N2, void* Y2, const void* bias2, const void* x, int xdtype, void* q8_workspace, int64_t y_row_pitch, int64_t K, int64_t M, int gemv, void* stream);
+int gguf_linear_walk(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes);
 int gguf_linear_dealt(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int gemv);
 int gguf_mmq_layer_route(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes);
 #ifdef __cplusplus

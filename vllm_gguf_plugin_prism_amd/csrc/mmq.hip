@@ -28,6 +28,7 @@
 #include "dense_api.h"
 #include "mmq_f.h"
 #include "tile_stream.h"
+#include "tile_walk.h"
 #include "tile_wide.h"
 #include "mmq_formats.h"
 #include "q8_1_device.h"
@@ -894,7 +895,14 @@ extern "C" int64_t gguf_mmq_layer_workspace_bytes(int type, int64_t N, int64_t K
   const int64_t others = gguf::mmqf_takes(type, M, N, K, w_row_pitch_bytes, INT64_MAX, 0)
                              ? gguf::mmqf_rows_bytes(M, K) + gguf::mmqf_plan((int)M, (int)N, (int)K, INT64_MAX).partial_bytes()
                              : gguf_mmq_workspace_bytes_engine(M, N, K, GGUF_MMQ_INT8);
-  return gguf::wide_dense_room(type, M, N, K, w_row_pitch_bytes, others);
+  const int64_t room = gguf::wide_dense_room(type, M, N, K, w_row_pitch_bytes, others), walk = gguf::walk_may_take(type, M) ? gguf::walk_rows_bytes(M, K) : 0;
+  return room > walk ? room : walk;
+}
+
+extern "C" int gguf_linear_walk(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes) {
+  if (M <= 0 || N <= 0 || K <= 0 || M > 0x7FFFFFF0LL || N > 0x7FFFFFF0LL || K > 0x7FFFFFF0LL) return 0;
+  const gguf::WalkPlan p = gguf::walk_plan(type, M, N, K, w_row_pitch_bytes, workspace_bytes);
+  return 16 * p.rt + p.nw;
 }
 
 extern "C" int gguf_mmq_layer_route(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes) {
@@ -963,6 +971,10 @@ int gguf::mmq_linear_impl(const void* W, int64_t w_row_pitch_bytes, const void* 
   if (workspace_bytes < M * (q8_row_bytes(K) + (engine == GGUF_MMQ_HALF ? 2 * q8_half_pitch(K) : 0))) return GGUF_ERR_WORKSPACE;
   const int64_t partial_room = workspace_bytes - rows_bytes;
   const bool tiles_at_5 = M <= 16 && rows16_direct_pays(type, (int)M, N, K, true) && rows16_direct_takes(W, w_row_pitch_bytes, type, (int)M, (int)N, (int)K, partial_room > 0 ? partial_room : 0);
+  if (engine == GGUF_MMQ_AUTO && on16(q8_workspace)) {
+    const WalkPlan p = walk_plan(type, M, N, K, w_row_pitch_bytes, workspace_bytes);
+    if (p.rt) return walk_linear(type, W, x, xdtype, q8_workspace, Y, (int)M, (int)N, (int)K, p, la, s);
+  }
   // (it fetches the quantized rows in pieces of 16 bytes)
   if (engine != GGUF_MMQ_HALF && (M <= 32 || engine == GGUF_MMQ_AUTO) && on16(q8_workspace) && ts_dense_takes(type, M, N, K, w_row_pitch_bytes))
     return ts_dense(type, W, x, xdtype, q8_workspace, Y, M, (int)N, (int)K, false, la, s);

@@ -1,0 +1,341 @@
+// Products of some tens to some hundred rows of activations on 32 columns per workgroup, whose waves walk K on their own.
+//
+// What such a product loses is waiting: tiles of 128 rows leave most CUs with one wave per SIMD, a barrier per step of K lines the waves up behind the
+// slowest fetch (mmq_i_core.h: 2.2 us a step, tile_wide_core.h: a chunk of X lasts less than its successor takes to come), and K cut between
+// workgroups costs a launch and a way through memory for the parts.  Here
+//   * a workgroup is 32 weight rows by 32 R rows of X, and its NW waves deal K among them, a panel of 256 values each in turn; no barrier stands
+//     before the sum of their tiles, which is formed in LDS and stored;
+//   * the panel's packed bytes come straight to the wave's own place in LDS (global_load_lds), are taken into registers and give the place to the next
+//     panel; where LDS has room for two, the panel after the next is on its way;
+//   * X lies in memory in the order in which the matrix unit takes it (tile_walk.h), 1 KB per block of 32 values and 32 rows, a fetch whose lanes follow
+//     one another: eight of these are on their way to a ring in the wave's place.  The L2 hands out 30 TB/s of such pieces (registers or LDS, 130 bytes per ns
+//     and CU), so that nothing is shared between the waves of a workgroup;
+//   * one v_mfma_i32_32x32x32_i8 per block; the sum leaves the matrix unit as a float (the accumulator starts at the bits of 1.5 * 2^23, which stay in
+//     sixteen registers of their own: as constants the compiler moves them into every result, 1.3 times as long) and costs two multiply-adds per result:
+//     a lane holds one row of X, whose block scale is a register, and sixteen weight rows, whose block scales come from LDS once per block for all
+//     R tiles.  The mins of the super-block formats are a contraction over the eight blocks in half precision, exact.
+// Four waves and two workgroups per CU, or eight waves where the output has few columns; R = 1 .. 4, as the rows fill them (walk_us).
+// Measured, us per call with the quantizer, before / now: [4096,4096] 64 rows Q4_K 16.1 / 10.8, Q8_0 19.4 / 12.6, 128 rows Q4_K 24.9 / 13.2; Q8_0 [14336,4096] 77
+// rows 38.7 / 26.5 (its weights take 12.4 from memory).  Over 7100 random products of the five formats (33 .. 2048 rows) 1.20 times the speed.
+// What bounds it: at few rows the beginning and the end of a workgroup (7 us of [4096,4096]'s 8 beside the quantizer); at many the vector instructions and the
+// traffic through LDS, which do not overlap as they might: a block of 32 x 32 x 32 takes a SIMD 100 ns, where its matrix instruction and 32 multiply-adds take
+// 58, the fetches of X and of weights 13 each, the operand reads 9.
+// Tried and no faster: block scales from lane to lane (row_newbcast) instead of through LDS; each workgroup touching a share of X first, so that all find it in the L2.
+// Arithmetic as in the other integer kernels (mmq.cuh:2-104: exact int32 block sums, scales in fp32); rel-L2 against 64 bits over 40 random products per format, normal
+// activations, the kernels before / this: Q8_0 9.8e-8 / 7.7e-8, Q5_0 9.7 / 7.7, Q4_0 13.2 / 7.7, Q4_K 14.4 / 11.6, Q5_K 9.3 / 8.1; of one sign Q8_0 10.0 / 7.8, Q5_0 7.0 / 5.3,
+// Q4_0 46 / 31, Q4_K 117 / 85, Q5_K 5.8 / 4.7: with one and two tiles of rows a panel has a sum of its own.
+#pragma once
+#include "mmq_i_core.h"
+#include "q8_1_device.h"
+#include "tile_walk.h"
+#include "tile_walk_formats.h"
+#include <type_traits>
+#include <utility>
+
+namespace gguf {
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float walk_f4 __attribute__((ext_vector_type(4)));
+
+struct WalkArgs {
+  int M, N, np, nkb;           // rows of X, weight rows, panels and blocks per row (the last panel may have fewer than eight)
+  int row_tiles;               // tiles of 32 rows of X
+  int tiles, run;              // workgroups that have work, and of them an XCD's
+  int band, band_tiles, last_band;   // row blocks that are walked together, all their tiles, and the row blocks of the last ones
+  uint32_t band_inv, all_inv, last_inv;   // 2^32 / (band, band_tiles, last_band) rounded up
+  uint32_t w_pitch;
+  int dtype, quads;            // GGUF_DTYPE_* of Y; rows of Y take stores of four values
+  int64_t ldy;
+  const void* bias;
+};
+
+template <int N> __device__ __forceinline__ void walk_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+// wave-uniform 16-byte-per-lane fetch into LDS: lane l's bytes land at m0 + 16 l
+__device__ __forceinline__ void walk_fetch(uint32_t at, const void* base, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(at), "s"(base), "s"(lds) : "memory");
+}
+// the same for lanes 0 .. 31 (all lanes are active before and after)
+__device__ __forceinline__ void walk_fetch_half(uint32_t at, const void* base, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(at), "s"(base), "s"(lds), "s"(0xFFFFFFFFull) : "memory");
+}
+template <typename T>
+__device__ __forceinline__ void walk_store(const walk_f4& v, T* y, const T* bias, int n, int N, int quads) {
+  if (quads && n + 3 < N) {
+    struct alignas(4 * sizeof(T)) { T v[4]; } o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o.v[e] = finish<T>(v[e], bias, n + e);
+    *(decltype(o)*)(y + n) = o;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < N) y[n + e] = finish<T>(v[e], bias, n + e);
+  }
+}
+
+__device__ __forceinline__ void walk_pin(float (&v)[16]) {   // the sixteen values are computed at this point
+  asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
+  asm volatile("" : "+v"(v[8]), "+v"(v[9]), "+v"(v[10]), "+v"(v[11]), "+v"(v[12]), "+v"(v[13]), "+v"(v[14]), "+v"(v[15]));
+}
+
+// A wave's place in LDS: D panels | PD tiles of X | block scales and sums of a panel's rows of X | scales for the lanes that hold results
+constexpr int WALK_PD = 8;
+template <class F> constexpr int walk_ppr() { return ((F::CUT ? F::PB + 29 : F::PB) / 16) | 1; }   // 16-byte pieces of a panel row (odd: banks)
+template <class F> constexpr int64_t walk_row_bytes(int64_t K) { return F::KQ ? K / 256 * F::PB : K / 32 * (F::PB / 8); }
+template <class F> constexpr int walk_head() { return F::OFF ? 1024 : 512; }
+template <class F, int R, int D> constexpr int walk_place() { return 512 * walk_ppr<F>() * D + 1024 * WALK_PD + walk_head<F>() * R + (F::OFF == MINS ? 1152 : 1024); }
+template <class F, int R, int NW, int D> constexpr size_t walk_lds() {
+  return (size_t)NW * walk_place<F, R, D>() + 16 > (size_t)NW * R * 4096 ? (size_t)NW * walk_place<F, R, D>() + 16 : (size_t)NW * R * 4096;
+}
+template <class F, int R, int NW> constexpr int walk_slots() { return walk_lds<F, R, NW, 2>() <= NW * 20 * 1024 ? 2 : 1; }
+
+template <int U> struct WalkUnit { static constexpr int value = U; };
+template <class L, int... U> __device__ __forceinline__ void walk_units(const L& unit, std::integer_sequence<int, U...>) { (unit(WalkUnit<U>()), ...); }
+
+template <class F, int R, int NW, int D>
+__global__ __launch_bounds__(64 * NW, 2) void tile_walk_kernel(const uint8_t* __restrict__ W, const char* __restrict__ X, void* __restrict__ Y, WalkArgs a) {
+  constexpr int PPR = walk_ppr<F>(), SLOT = 512 * PPR, NI = (32 * PPR + 63) / 64, PD = WALK_PD, U = 8 * R;   // (the last fetch of a panel: lanes 0 .. 31)
+  constexpr int HEAD = walk_head<F>(), XR_AT = SLOT * D, HD_AT = XR_AT + 1024 * PD, SC_AT = HD_AT + HEAD * R, PLACE = walk_place<F, R, D>();
+  constexpr bool PART = R <= 2;                             // a panel's sum of its own, where the registers hold it
+  constexpr int DB = F::CUT && R >= 3 ? 1 : 2;              // block scales in registers, of this block and, where these suffice, of the next
+  constexpr int NL = NI + R;                                // fetches of a panel and of the heads of a panel's rows of X
+  static_assert(PD == 8 && U % PD == 0, "the ring's places are the same in every panel; the waits below count to eight");
+  static_assert(PPR % 2 == 1 && walk_lds<F, R, NW, D>() <= 160 * 1024, "the last fetch of a panel is half a fetch; LDS");
+  extern __shared__ __align__(16) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lrow = lane & 31, half = lane >> 5;
+  // ---- which rows and columns.  Each XCD has a run of tiles, as long as another's; the row blocks of a band follow one another, so that they find
+  // their weights in the L2, and a band is as tall as its rows of X fit there.
+  const int local = blockIdx.x >> 3, tile = (blockIdx.x & 7) * a.run + local;
+  if (local >= a.run || tile >= a.tiles) return;
+  const int bnd = a.band_tiles == 1 ? tile : (int)__umulhi((uint32_t)tile, a.all_inv), in = tile - bnd * a.band_tiles;
+  const bool last = (bnd + 1) * a.band_tiles >= a.tiles;    // (whose row blocks may be fewer)
+  const int rows = last ? a.last_band : a.band, col = rows == 1 ? in : (int)__umulhi((uint32_t)in, last ? a.last_inv : a.band_inv);
+  const int rb = bnd * a.band + in - col * rows, n0 = 32 * col;
+  char* const mine = smem + wave * PLACE;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem + wave * PLACE;
+
+  // ---- weights: piece number -> (row of the panel, 16-byte piece of it)
+  const uint32_t wmis = F::CUT ? (uint32_t)((uintptr_t)W & 15) : 0u;
+  const uint8_t* const wbase = W - wmis;
+  const uint32_t row_bytes = F::KQ ? (uint32_t)(a.np * F::PB) : (uint32_t)(a.nkb * (F::PB / 8));
+  const uint32_t last16 = ((uint32_t)(a.N - 1) * a.w_pitch + wmis + row_bytes - 1) & ~15u;   // the last granule that holds bytes of W
+  uint32_t w_at[NI], w_piece[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int q = min(64 * i + lane, 32 * PPR - 1), r = q / PPR;
+    w_at[i] = (uint32_t)min(n0 + r, a.N - 1) * a.w_pitch + wmis;
+    w_piece[i] = 16 * (uint32_t)(q - r * PPR);
+  }
+  const char* xt[R];
+#pragma unroll
+  for (int k = 0; k < R; ++k) xt[k] = X + (int64_t)min(rb * R + k, a.row_tiles - 1) * a.np * WALK_REC;
+  const auto request_w = [&](int p, int slot) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const uint32_t v = min(((w_at[i] + (uint32_t)(p * F::PB)) & ~15u) + w_piece[i], last16);
+      if (i < NI - 1) walk_fetch(v, wbase, lds0 + slot * SLOT + 1024 * i);
+      else walk_fetch_half(v, wbase, lds0 + slot * SLOT + 1024 * i);
+    }
+  };
+  const auto request_heads = [&](int p) {
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      const char* const base = xt[k] + (int64_t)p * WALK_REC + WALK_D_AT;
+      if (F::OFF) walk_fetch(16 * lane, base, lds0 + HD_AT + 1024 * k);
+      else walk_fetch_half(16 * lane, base, lds0 + HD_AT + 512 * k);
+    }
+  };
+  const auto request_x = [&](int p, int u) { walk_fetch(16 * lane, xt[u % R] + ((int64_t)p * WALK_REC + 1024 * (u / R)), lds0 + XR_AT + 1024 * (u % PD)); };
+
+  float acc[R][16];
+#pragma unroll
+  for (int k = 0; k < R; ++k)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[k][r] = 0.0f;
+  if (wave < a.np) {
+    request_w(wave, 0);
+    request_heads(wave);
+    if (D == 2 && wave + NW < a.np) request_w(wave + NW, 1);
+#pragma unroll
+    for (int u = 0; u < PD; ++u) request_x(wave, u);
+  }
+  v16i seed;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) seed[r] = kSeedBits;
+  asm volatile("" : "+v"(seed));                            // (opaque: as constants they are moved into every result's registers)
+  float* const scales = (float*)(mine + SC_AT);
+
+  const auto panel = [&](int p, int slot, auto any) {
+    constexpr bool MORE = decltype(any)::value;             // another panel follows
+    // This panel, asked for one (D = 2: two) panels ago, and its heads; behind them the tiles under way.
+    if (D == 2 && p == wave && MORE) walk_wait<PD + NI>();
+    else walk_wait<PD>();
+    F w;
+    const uint32_t at = F::CUT ? ((uint32_t)min(n0 + lrow, a.N - 1) * a.w_pitch + wmis + (uint32_t)(p * F::PB)) & 15 : 0u;
+    w.read(mine + slot * SLOT + lrow * (16 * PPR), at, half);
+    uint4 dh[R], sh[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      dh[k] = *(const uint4*)(mine + HD_AT + HEAD * k + 16 * lrow);
+      if (F::OFF) sh[k] = *(const uint4*)(mine + HD_AT + HEAD * k + 512 + 16 * lrow);
+    }
+    if (!F::KQ && a.nkb < 8 * (p + 1)) w.limit(a.nkb - 8 * p);
+    w.scale_to(scales, lrow, half);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // the panel's place may be filled again
+    const bool refill = D == 1 ? MORE : MORE && p + 2 * NW < a.np;
+    if constexpr (MORE) request_heads(p + NW);
+    if (refill) request_w(p + D * NW, slot);
+    // Unit u's tile has landed.  Asked for behind it: of the tiles under way with u = 0 the others, else two less (those that take the places of the last
+    // two units are asked for behind this), and, if it was asked for before this panel began, what was asked for then.
+    const auto ready = [&](auto at) {
+      constexpr int u = decltype(at)::value, behind = u == 0 ? PD - 1 : u == 1 ? PD - 2 : PD - 3;
+      if constexpr (!MORE) {
+        walk_wait<(U - 1 - u < behind ? U - 1 - u : behind)>();
+      } else if constexpr (u >= PD) {
+        walk_wait<behind>();
+      } else {
+        if (refill) walk_wait<behind + NL>();
+        else walk_wait<behind + R>();
+      }
+    };
+    float part[PART ? R : 1][16];
+    v4i xo[2];
+    v16i s[2];
+    walk_f4 dw[DB][4];
+    const auto load_x = [&](int u) { xo[u & 1] = *(const v4i*)(mine + XR_AT + 1024 * (u % PD) + 16 * lane); };
+    const auto load_dw = [&](int b) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) dw[b % DB][q] = *(const walk_f4*)(scales + 32 * b + 8 * q + 4 * half);
+    };
+    v4i wo = w.codes(0, half);
+    ready(WalkUnit<0>());
+    load_x(0);
+    ready(WalkUnit<1>());
+    load_x(1);
+    load_dw(0);
+    s[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wo, xo[0], seed, 0, 0, 0);
+    const auto unit = [&](auto at) {
+      constexpr int u = decltype(at)::value, b = u / R, k = u % R;
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (u + 2 < U) {
+        ready(WalkUnit<u + 2>());
+        load_x(u + 2);
+      }
+      if (DB == 2 && k == 0 && b + 1 < 8) load_dw(b + 1);
+      if (u + PD < U) request_x(p, u + PD);                 // (unit u's operand has been read: its matrix instruction has started)
+      else if (MORE) request_x(p + NW, u + PD - U);
+      if (u + 1 < U && (u + 1) % R == 0) wo = w.codes((u + 1) / R, half);
+      const uint32_t dp = b < 2 ? dh[k].x : b < 4 ? dh[k].y : b < 6 ? dh[k].z : dh[k].w;
+      float d8 = half_bits(b & 1 ? dp >> 16 : dp & 0xFFFF);
+      asm volatile("" : "+v"(d8));                          // (a float from here on: the compiler would have every multiply-add convert it, in a form that takes twice as long)
+      const float nd = -kSeed * d8;
+      float (&sum)[16] = PART ? part[PART ? k : 0] : acc[k];
+      float m8 = 0.0f;
+      if constexpr (F::OFF == EIGHTS) {
+        const uint32_t sp = b < 2 ? sh[k].x : b < 4 ? sh[k].y : b < 6 ? sh[k].z : sh[k].w;
+        m8 = -8.0f * half_bits(b & 1 ? sp >> 16 : sp & 0xFFFF);
+        asm volatile("" : "+v"(m8));
+      }
+      if (u + 1 < U) s[(u + 1) & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wo, xo[(u + 1) & 1], seed, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        float v = __builtin_fmaf(__builtin_bit_cast(float, (int)s[u & 1][r]), d8, nd);   // d8 times the block's sum, rounded once
+        if constexpr (F::OFF == EIGHTS) v += m8;
+        sum[r] = PART && b == 0 ? v * dw[b % DB][r >> 2][r & 3] : __builtin_fmaf(v, dw[b % DB][r >> 2][r & 3], sum[r]);
+      }
+      // The offsets, a contraction over eight (the upper half of the lanes holds values 8 .. 15, zeros), in the middle of the panel
+      if constexpr (F::OFF == MINS) if constexpr (b == 3) {
+        const uint4 none = make_uint4(0, 0, 0, 0), mv = half ? none : w.offsets(), sv = half ? none : sh[k];
+        f32x16 zero;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) zero[r] = 0.0f;
+        const f32x16 off = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, mv), __builtin_bit_cast(f16x8, sv), zero, 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const walk_f4 dm = *(const walk_f4*)(scales + 256 + 8 * q + 4 * half);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) sum[4 * q + e] = __builtin_fmaf(off[4 * q + e], dm[e], sum[4 * q + e]);
+        }
+      }
+      if constexpr (PART && b == 7)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[k][r] += sum[r];
+      walk_pin(PART && b == 7 ? acc[k] : sum);
+      if (DB == 1 && k == R - 1 && b + 1 < 8) load_dw(b + 1);
+    };
+    walk_units(unit, std::make_integer_sequence<int, U>());
+  };
+  if (wave < a.np) {
+    int p = wave, slot = 0;
+    for (; p + NW < a.np; p += NW) {
+      panel(p, slot, std::true_type());
+      if (D == 2) slot ^= 1;
+    }
+    panel(p, slot, std::false_type());
+  }
+
+  // ---- the waves' partial tiles, added in pairs
+  __syncthreads();
+  walk_f4* const red = (walk_f4*)smem;                      // [wave][tile][run of four and half][row ^ that]
+#pragma unroll
+  for (int k = 0; k < R; ++k)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) red[((wave * R + k) * 8 + 2 * q + half) * 32 + (lrow ^ (2 * q + half))] = (walk_f4){acc[k][4 * q], acc[k][4 * q + 1], acc[k][4 * q + 2], acc[k][4 * q + 3]};
+  __syncthreads();
+  for (int i = tid; i < R * 256; i += 64 * NW) {
+    const int q = i & 7, row = (i >> 3) & 31, k = i >> 8, m = 32 * (rb * R + k) + row;
+    walk_f4 v[NW];
+#pragma unroll
+    for (int z = 0; z < NW; ++z) v[z] = red[((z * R + k) * 8 + q) * 32 + (row ^ q)];
+#pragma unroll
+    for (int d = 1; d < NW; d *= 2)
+#pragma unroll
+      for (int z = 0; z < NW; z += 2 * d) v[z] += v[z + d];
+    if (m < a.M) {
+      if (a.dtype == GGUF_DTYPE_F16) walk_store<_Float16>(v[0], (_Float16*)Y + (int64_t)m * a.ldy, (const _Float16*)a.bias, n0 + 4 * q, a.N, a.quads);
+      else if (a.dtype == GGUF_DTYPE_BF16) walk_store<bf16_t>(v[0], (bf16_t*)Y + (int64_t)m * a.ldy, (const bf16_t*)a.bias, n0 + 4 * q, a.N, a.quads);
+      else walk_store<float>(v[0], (float*)Y + (int64_t)m * a.ldy, (const float*)a.bias, n0 + 4 * q, a.N, a.quads);
+    }
+  }
+}
+
+template <class F, int R, int NW>
+static int walk_launch(const WalkCall& c, hipStream_t stream) {
+  constexpr int D = walk_slots<F, R, NW>();
+  constexpr size_t lds = walk_lds<F, R, NW, D>();
+  const WalkBands bands = walk_bands(R, c.M, c.N, c.K);
+  if (!bands.ok) return GGUF_NOT_TAKEN;
+  auto kern = tile_walk_kernel<F, R, NW, D>;
+  static std::atomic<uint64_t> done{0};
+  allow_large_lds(kern, lds, done);
+  const int64_t pitch = c.la.w_pitch ? c.la.w_pitch : walk_row_bytes<F>(c.K), ldy = c.la.ldy ? c.la.ldy : (int64_t)c.N;
+  const int run = (bands.tiles + 7) / 8, elt = c.dtype == GGUF_DTYPE_F32 ? 4 : 2;
+  const auto inverse = [](int d) { return (uint32_t)((0x100000000ull + d - 1) / d); };
+  const WalkArgs a = {c.M, c.N, (c.K + 255) / 256, c.K / 32, (c.M + 31) / 32, bands.tiles, run, bands.band, bands.band_tiles, bands.last,
+                      inverse(bands.band), inverse(bands.band_tiles), inverse(bands.last), (uint32_t)pitch, c.dtype,
+                      ldy % 4 == 0 && (uintptr_t)c.Y % (4 * elt) == 0, ldy, c.la.bias};
+  hipLaunchKernelGGL(kern, dim3((unsigned)(8 * run)), dim3(64 * NW), lds, stream, (const uint8_t*)c.W, (const char*)c.x, c.Y, a);
+  return launch_status();
+}
+
+template <class F>
+static int walk_run(const WalkCall& c, hipStream_t s) {
+  switch (c.plan.rt * 16 + c.plan.nw) {
+    case 1 * 16 + 4: return walk_launch<F, 1, 4>(c, s);
+    case 1 * 16 + 8: return walk_launch<F, 1, 8>(c, s);
+    case 2 * 16 + 4: return walk_launch<F, 2, 4>(c, s);
+    case 2 * 16 + 8: return walk_launch<F, 2, 8>(c, s);
+    case 3 * 16 + 4: return walk_launch<F, 3, 4>(c, s);
+    case 4 * 16 + 4: return walk_launch<F, 4, 4>(c, s);
+  }
+  return GGUF_NOT_TAKEN;
+}
+// A: the panels that begin on whole 16-byte pieces
+template <class A, class F>
+static int walk_run_either(const WalkCall& c, hipStream_t s) {
+  const int64_t pitch = c.la.w_pitch ? c.la.w_pitch : walk_row_bytes<A>(c.K);
+  return (uintptr_t)c.W % 16 == 0 && pitch % 16 == 0 ? walk_run<A>(c, s) : walk_run<F>(c, s);
+}
+
+}  // namespace gguf

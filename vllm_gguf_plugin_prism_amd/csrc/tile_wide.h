@@ -34,6 +34,7 @@ int wide_layer(const void* X, int xdtype, void* workspace, const void* W13, int 
 // A dense product: the plan (rt 0: it runs otherwise), the workspace to ask for, and the call
 struct WidePlan { int rt, ksplit, passes; };
 WidePlan wide_dense_plan(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, int64_t workspace_bytes);
+double wide_dense_us(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, int64_t workspace_bytes);
 int64_t wide_dense_room(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, int64_t others_bytes);
 bool wide_dense_aligned(int type, const void* W);   // whether the weights begin where it can fetch them
 int wide_dense(int type, const void* W, const void* x, int dtype, void* workspace, void* Y, int M, int N, int K, const WidePlan& p, const LinearArgs& la, hipStream_t s);

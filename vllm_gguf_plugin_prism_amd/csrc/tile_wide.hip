@@ -211,6 +211,13 @@ WidePlan wide_dense_plan(int type, int64_t M, int64_t N, int64_t K, int64_t w_pi
   return p.rt && us < wide_margin(type, M) * wide_others_us(type, (int)M, (int)N, (int)K, workspace_bytes) ? p : WidePlan{0, 1, 1};
 }
 
+// How long a product that it takes is estimated to take here, else a time beyond any other's
+double wide_dense_us(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, int64_t workspace_bytes) {
+  double us = 1e30;
+  if (wide_dense_ok(type, M, N, K, w_pitch)) wide_best(type, (int)M, (int)N, (int)K, workspace_bytes, us);
+  return us;
+}
+
 // The workspace that takes the call, given the size that the others would want: theirs where that costs less than a tenth.
 int64_t wide_dense_room(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, int64_t others_bytes) {
   if (!wide_dense_ok(type, M, N, K, w_pitch)) return others_bytes;

@@ -173,7 +173,8 @@ def ggml_mul_mat_a8(W: torch.Tensor, X: torch.Tensor, quant_type: int, row: int,
 
     ``engine``: ``"int8"`` keeps the reference's integer arithmetic (exact int8 dot products per block on int8 MFMA,
     block scales in fp32).  ``"auto"`` keeps it, too, on the unit that is faster: K-quant, Q4_0, Q4_1 and Q5_1 products past
-    some tens of rows run as exact whole numbers on half-precision MFMA (csrc/tile_wide_core.h, csrc/mmq_f_core.h).  ``"half"`` is opt-in and
+    some tens of rows run as exact whole numbers on half-precision MFMA (csrc/tile_wide_core.h, csrc/mmq_f_core.h) where that is faster than
+    the integer unit (csrc/tile_walk_core.h, csrc/mmq_i_core.h).  ``"half"`` is opt-in and
     multiplies the dequantized, rounded operands on half-precision MFMA (about 2e-4 relative deviation from the integer
     result, half and bfloat16 results only).  ``out`` / ``bias`` / sliced ``W``: as for :func:`ggml_mul_mat_vec_a8`."""
     out, w_pitch, ldy = _shard_args(W, X, quant_type, row, out, bias)
@@ -234,7 +235,7 @@ def _dense_result_fits(X: torch.Tensor, row: int, out: torch.Tensor | None, bias
 
 
 def _mmq_route(quant_type: int, row: int, col: int, vecs: int, w_pitch: int, workspace_bytes: int | None = None) -> int:
-    """The kernel that :func:`ggml_mul_mat_a8` runs on its own workspace or one of this size where not :func:`_linear_dealt`: 1 the streaming
+    """The kernel that :func:`ggml_mul_mat_a8` runs on its own workspace or one of this size where neither :func:`_linear_dealt` nor :func:`_linear_walk`: 1 the streaming
     tile kernel, 4 the wide tiles, 2 the half-precision unit's whole-number GEMM, 0 another."""
     L = _lib.lib()
     if workspace_bytes is None:
@@ -246,6 +247,15 @@ def _linear_dealt(quant_type: int, row: int, col: int, vecs: int, w_pitch: int, 
     """Whether :func:`ggml_mul_mat_a8` (``gemv``: :func:`ggml_mul_mat_vec_a8`) runs tile_dealt_kernel, which comes before the
     kernels of :func:`_mmq_route`."""
     return bool(_lib.lib().gguf_linear_dealt(int(quant_type), row, col, vecs, w_pitch, int(gemv)))
+
+
+def _linear_walk(quant_type: int, row: int, col: int, vecs: int, w_pitch: int, workspace_bytes: int | None = None) -> tuple[int, int]:
+    """(Tiles of 32 rows, waves to a workgroup) with which :func:`ggml_mul_mat_a8` runs tile_walk_kernel, which comes before the kernels of
+    :func:`_mmq_route`, on its own workspace or one of this size; (0, 0): it does not."""
+    L = _lib.lib()
+    if workspace_bytes is None:
+        workspace_bytes = L.gguf_mmq_layer_workspace_bytes(int(quant_type), row, col, vecs, w_pitch)
+    return divmod(L.gguf_linear_walk(int(quant_type), row, col, vecs, w_pitch, workspace_bytes), 16)
 
 
 def _mmq_unit(quant_type: int, row: int, col: int, vecs: int, w_pitch: int) -> int:
