@@ -8,7 +8,9 @@ from oracle import gguf_oracle as o
 
 pytestmark = pytest.mark.gpu
 
-TYPES = (o.Q4_0, o.Q5_0, o.Q8_0, o.Q4_K, o.Q5_K)
+BLOCKS = (o.Q4_0, o.Q5_0, o.Q8_0, o.Q4_K, o.Q5_K)   # a scale per 32 values
+GROUPS = (o.Q6_K, o.Q3_K)                            # per 16
+TYPES = BLOCKS + GROUPS
 OLDER = (o.Q4_0, o.Q5_0, o.Q8_0)
 
 
@@ -43,10 +45,16 @@ def walked(qtype, m, n, k, plan=None):
 
 # each height of tiles with each number of waves that it has: waves without a panel, with one, two and three; last tiles of rows and columns in part; rows of
 # W a pitch apart that moves them through the positions inside 16 bytes
-@pytest.mark.parametrize("qtype", TYPES)
-@pytest.mark.parametrize("m,n,k,pad,plan", [(33, 323, 512, 0, (1, 4)), (67, 4148, 1280, 2, (1, 4)), (35, 308, 1280, 0, (1, 8)), (37, 332, 4352, 6, (1, 8)),
-                                            (33, 8734, 512, 0, (2, 4)), (135, 3307, 2304, 14, (2, 4)), (36, 4317, 1280, 2, (2, 8)), (142, 1635, 5376, 0, (2, 8)),
-                                            (65, 11337, 512, 6, (3, 4)), (332, 2814, 2304, 0, (3, 4)), (193, 5656, 1792, 10, (4, 4)), (591, 2387, 2304, 0, (4, 4))])
+@pytest.mark.parametrize("qtype,m,n,k,pad,plan", [(q, *s) for q in BLOCKS for s in (
+    (33, 323, 512, 0, (1, 4)), (67, 4148, 1280, 2, (1, 4)), (35, 308, 1280, 0, (1, 8)), (37, 332, 4352, 6, (1, 8)),
+    (33, 8734, 512, 0, (2, 4)), (135, 3307, 2304, 14, (2, 4)), (36, 4317, 1280, 2, (2, 8)), (142, 1635, 5376, 0, (2, 8)),
+    (65, 11337, 512, 6, (3, 4)), (332, 2814, 2304, 0, (3, 4)), (193, 5656, 1792, 10, (4, 4)), (591, 2387, 2304, 0, (4, 4)))] + [
+    (q, *s) for q in GROUPS for s in (
+    (35, 301, 512, 2, (1, 4)), (67, 4148, 1280, 4, (1, 4)), (33, 4267, 2560, 0, (1, 4)), (34, 305, 1280, 0, (1, 8)), (36, 325, 4352, 6, (1, 8)),
+    (35, 8218, 512, 8, (2, 4)), (33, 8279, 1280, 10, (2, 4)), (36, 4123, 1280, 12, (2, 8)), (71, 8418, 1280, 14, (3, 4)))] + [
+    (o.Q6_K, 135, 3307, 2304, 2, (2, 4)), (o.Q6_K, 142, 1635, 5376, 0, (2, 8)), (o.Q6_K, 202, 4585, 2304, 0, (3, 4)),
+    (o.Q3_K, 97, 4257, 2304, 2, (2, 4)), (o.Q3_K, 104, 2174, 4352, 0, (2, 8)), (o.Q3_K, 202, 4241, 2304, 0, (3, 4)),
+    (o.Q3_K, 98, 8309, 512, 0, (4, 4)), (o.Q3_K, 97, 8336, 1280, 6, (4, 4)), (o.Q3_K, 296, 4202, 2304, 14, (4, 4))])
 def test_edges(qtype, m, n, k, pad, plan):
     product(qtype, m, n, k, pad, rows=np.r_[:3, m - 35:m], check=walked(qtype, m, n, k, plan))
 
@@ -96,7 +104,9 @@ def test_rows_do_not_meet():
 
 # The kernels behind it at sizes where they still run: those whose estimate is shorter (few panels of many rows, few columns of long ones) ...
 @pytest.mark.parametrize("qtype,m,n,k,route", [(o.Q4_0, 686, 2071, 320, 0), (o.Q4_0, 1782, 386, 256, 4), (o.Q5_0, 925, 552, 256, 0), (o.Q8_0, 1164, 539, 256, 0),
-                                               (o.Q4_K, 717, 741, 256, 4), (o.Q4_K, 1007, 369, 9472, 2), (o.Q5_K, 1219, 569, 256, 4), (o.Q5_K, 822, 307, 14592, 2)])
+                                               (o.Q4_K, 717, 741, 256, 4), (o.Q4_K, 1007, 369, 9472, 2), (o.Q5_K, 1219, 569, 256, 4), (o.Q5_K, 822, 307, 14592, 2),
+                                               (o.Q6_K, 66, 14616, 512, 0), (o.Q6_K, 633, 805, 256, 4), (o.Q6_K, 716, 306, 13056, 2), (o.Q3_K, 34, 23956, 256, 4),
+                                               (o.Q3_K, 73, 16260, 256, 0)])
 def test_kernels_of_what_is_not_walked(qtype, m, n, k, route):
     from vllm_gguf_plugin_prism_amd import ops
 

@@ -72,7 +72,7 @@ int quantize_wide(const void* x, int xdtype, void* records, int64_t M, int64_t K
 
 // The records of tile_walk.h.  A workgroup has 32 rows of 64 values, eight threads to a row.
 template <typename T>
-__global__ __launch_bounds__(256) void quantize_walk_kernel(const T* __restrict__ x, char* __restrict__ records, int K, int np, int64_t M) {
+__global__ __launch_bounds__(256) void quantize_walk_kernel(const T* __restrict__ x, char* __restrict__ records, int K, int np, int64_t M, bool groups) {
   const int row = threadIdx.x >> 3, k = 64 * blockIdx.x + 8 * (threadIdx.x & 7), b = (k >> 5) & 7;
   const int64_t m = 32 * (int64_t)blockIdx.y + row;
   if (m >= M) return;                            // (all eight threads of the row: quads stay together)
@@ -80,17 +80,17 @@ __global__ __launch_bounds__(256) void quantize_walk_kernel(const T* __restrict_
   if (k < K) load8<T>(x + m * (int64_t)K + k, v);   // (behind K: zeros)
   const Q8Quad q = q8_1_quantize8(v);
   char* const rec = records + ((int64_t)blockIdx.y * np + (k >> 8)) * WALK_REC;
-  *(uint2*)(rec + 1024 * b + 16 * ((k & 16) * 2 + row) + (k & 8)) = q.q;
+  *(uint2*)(rec + 1024 * b + (groups ? 32 * (k & 16) + 8 * (4 * (k & 8) + row) : 16 * (2 * (k & 16) + row) + (k & 8))) = q.q;
   if ((threadIdx.x & 3) == 0) {
     *(_Float16*)(rec + WALK_D_AT + 16 * row + 2 * b) = (_Float16)q.d;
     *(_Float16*)(rec + WALK_S_AT + 16 * row + 2 * b) = (_Float16)q.s;
   }
 }
 
-int quantize_walk(const void* x, int xdtype, void* records, int64_t M, int64_t K, hipStream_t stream) {
+int quantize_walk(const void* x, int xdtype, void* records, int64_t M, int64_t K, bool groups, hipStream_t stream) {
   const int np = (int)((K + 255) / 256);
   GGUF_DISPATCH_DTYPE(xdtype, hipLaunchKernelGGL(quantize_walk_kernel<scalar_t>, dim3(4 * np, (unsigned)((M + 31) / 32)), dim3(256), 0, stream, (const scalar_t*)x,
-                                                 (char*)records, (int)K, np, M));
+                                                 (char*)records, (int)K, np, M, groups));
   return launch_status();
 }
 

@@ -6,12 +6,13 @@
 namespace gguf {
 
 // The quantized activations as the kernel takes them: a record per 32 rows and 256 values, [rows / 32][K / 256][WALK_REC], in the order in which a wave's
-// lanes take them: the quants of block b (32 values), 16 bytes of row r's upper or lower half h at 1024 b + 16 (32 h + r); eight block scales of row r,
+// lanes take them: the quants of block b (32 values), 16 bytes of row r's upper or lower half h at 1024 b + 16 (32 h + r), or, for weights with a scale
+// per 16 values (`groups`), 8 bytes of half h of its group g at 1024 b + 512 g + 8 (32 h + r); eight block scales of row r,
 // halves, at WALK_D_AT + 16 r, and as many block sums at WALK_S_AT + 16 r.  Zeros behind K; rows past the last one may be anything: they are read and
 // multiplied but not stored, and no result of another row sees them.
 constexpr int WALK_REC = 9216, WALK_D_AT = 8192, WALK_S_AT = 8704;
 static inline int64_t walk_rows_bytes(int64_t M, int64_t K) { return (M + 31) / 32 * ((K + 255) / 256) * WALK_REC; }
-int quantize_walk(const void* x, int xdtype, void* records, int64_t M, int64_t K, hipStream_t stream);   // q8_1.hip
+int quantize_walk(const void* x, int xdtype, void* records, int64_t M, int64_t K, bool groups, hipStream_t stream);   // q8_1.hip
 
 // Tiles of 32 rt rows, nw waves to a workgroup; rt 0: not taken
 struct WalkPlan { int rt, nw; };

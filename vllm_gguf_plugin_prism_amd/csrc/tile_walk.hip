@@ -13,6 +13,8 @@ int walk_q5_0(const WalkCall& c, hipStream_t s);
 int walk_q8_0(const WalkCall& c, hipStream_t s);
 int walk_q4_k(const WalkCall& c, hipStream_t s);
 int walk_q5_k(const WalkCall& c, hipStream_t s);
+int walk_q6_k(const WalkCall& c, hipStream_t s);
+int walk_q3_k(const WalkCall& c, hipStream_t s);
 
 static int walk_any(int type, const WalkCall& c, hipStream_t s) {
   switch (type) {
@@ -21,14 +23,17 @@ static int walk_any(int type, const WalkCall& c, hipStream_t s) {
     case T_Q8_0: return walk_q8_0(c, s);
     case T_Q4_K: return walk_q4_k(c, s);
     case T_Q5_K: return walk_q5_k(c, s);
+    case T_Q6_K: return walk_q6_k(c, s);
+    case T_Q3_K: return walk_q3_k(c, s);
   }
   return GGUF_NOT_TAKEN;
 }
 
 // About how long a product takes, us, quantizer included, with each of the plans: rounds of workgroups on the chip (two of four waves share a CU, one of
 // eight has it for itself) with the panels that a wave walks, which take longer beside other workgroups; the weights, the rows of X, the result.
-// Fitted to 7100 products of random sizes (33 .. 2048 rows, 512 .. 28672 columns, K 512 .. 18944), right to 8 %; the plan chosen by it takes 0.9 %
-// longer than the best.
+// Fitted to 12900 products of random sizes (33 .. 2048 rows, 512 .. 28672 columns, K 512 .. 18944), right to 8 %; the plan chosen by it takes 0.9 %
+// longer than the best.  (panel 0: no such plan.  Q6_K's tiles of 128 rows have no registers left for the sums of a panel, and without those the result is
+// less exact than the other kernels' (1.3e-7 of it against 0.9e-7).)
 struct WalkType { int type; double panel[6], weights[2]; };
 struct WalkShape { int rt, nw; double base, part, alone, x, y; };
 static const WalkType walk_types[] = {
@@ -37,6 +42,8 @@ static const WalkType walk_types[] = {
       {T_Q8_0, {2.15, 2.09, 2.97, 2.8, 3.28, 4.18}, {0.11, 0.175}},
       {T_Q4_K, {1.84, 1.68, 2.67, 2.48, 3.76, 4.95}, {0.0696, 0.117}},
       {T_Q5_K, {1.86, 1.74, 2.87, 2.64, 3.96, 5.14}, {0.0766, 0.132}},
+      {T_Q6_K, {3.18, 2.94, 4.77, 4.47, 6.50, 0.0}, {0.094, 0.172}},
+      {T_Q3_K, {2.27, 2.13, 3.14, 2.87, 4.02, 5.05}, {0.062, 0.125}},
 };
 static const WalkShape walk_shapes[] = {
       {1, 4, 5.07, 0.221, 0.612, 1.78, 1.5},
@@ -56,13 +63,14 @@ static double walk_us(const WalkType& t, int shape, int M, int N, int K) {
          1e-6 * (t.weights[p.nw == 8] * N * K + p.x * M * K + p.y * M * N);
 }
 
-// How long the kernels take that run otherwise, by their own estimates and what 7100 products took of those, by type (mmq_int_us is fitted to the
-// K-quants).  The streaming tiles, which small matrices run on, have none: they take 1.2 times as long (1.18 to 1.22 by type; of 1900 products six were slower
+// How long the kernels take that run otherwise, by their own estimates and what 12900 products took of those, by type (mmq_int_us is fitted to the
+// K-quants).  The streaming tiles, which small matrices run on, have none: they take 1.14 (Q6_K) to 1.25 times as long (of 2900 products six were slower
 // here by more than a tenth).
 static double walk_others_us(int type, int M, int N, int K, int64_t w_pitch, int64_t workspace_bytes) {
   if (ts_dense_takes(type, M, N, K, w_pitch)) return 1e30;
   const int64_t int8_rows = (M * q8_row_bytes(K) + 255) / 256 * 256;
-  const double few = M <= 64 ? 0.9 : 1.0, factor = type == T_Q4_0 ? 0.87 * few : type == T_Q5_0 ? 0.79 * few : type == T_Q8_0 ? 0.785 * few : 1.09;
+  const double few = M <= 64 ? 0.9 : 1.0, factor = type == T_Q4_0 ? 0.87 * few : type == T_Q5_0 ? 0.79 * few : type == T_Q8_0 ? 0.785 * few :
+                                                        type == T_Q6_K ? 1.02 : type == T_Q3_K ? 1.05 : 1.09;
   double us = factor * mmq_int_us(type, M, N, K, workspace_bytes > int8_rows ? workspace_bytes - int8_rows : 0);
   if (mmqf_takes(type, M, N, K, w_pitch, workspace_bytes, int8_rows)) us = std::min(us, mmqf_us(type, M, N, K, workspace_bytes - mmqf_rows_bytes(M, K)));
   return std::min(us, 1.06 * wide_dense_us(type, M, N, K, w_pitch, workspace_bytes));
@@ -74,8 +82,8 @@ bool walk_may_take(int type, int64_t M) {
   return false;
 }
 
-// Where it is the faster one by these estimates: over 7100 products of 33 to 2048 rows 1.20 times as fast as what ran before on average, a hundred of them more than 3 %
-// slower, none by more than 18 %.  us, before / now, quantizer included: [4096,4096] 64 rows Q4_K 16.1 / 10.8, Q8_0 19.4 / 12.6, 128 rows Q4_K 24.9 / 13.2;
+// Where it is the faster one by these estimates: over 12900 products of 33 to 2048 rows 1.20 times as fast as what ran before on average (Q6_K 1.12, Q3_K 1.26), 140 of them
+// more than 3 % slower, none by more than 18 %.  us, before / now, quantizer included: [4096,4096] 64 rows Q4_K 16.1 / 10.8, Q8_0 19.4 / 12.6, 128 rows Q4_K 24.9 / 13.2;
 // [14336,4096] Q8_0 77 rows 38.7 / 26.5; but short rows of many columns keep to the others: [25456,512] Q4_K 1501 rows 91 / 137.  (Past 2048 rows: not measured.)
 WalkPlan walk_plan(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, int64_t workspace_bytes) {
   if (!walk_may_take(type, M) || K % block_elems(type) != 0) return {0, 0};
@@ -88,7 +96,7 @@ WalkPlan walk_plan(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, i
   double least = 1e30;
   for (int i = 0; i < 6; ++i) {
     const WalkShape& p = walk_shapes[i];
-    if ((p.rt > 1 && M <= 32 * (p.rt - 1)) || !walk_bands(p.rt, M, N, K).ok) continue;
+    if (t->panel[i] == 0.0 || (p.rt > 1 && M <= 32 * (p.rt - 1)) || !walk_bands(p.rt, M, N, K).ok) continue;
     const double us = walk_us(*t, i, (int)M, (int)N, (int)K);
     if (us < least) { least = us; best = {p.rt, p.nw}; }
   }
@@ -96,7 +104,7 @@ WalkPlan walk_plan(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, i
 }
 
 int walk_linear(int type, const void* W, const void* x, int dtype, void* workspace, void* Y, int M, int N, int K, const WalkPlan& p, const LinearArgs& la, hipStream_t s) {
-  int rc = quantize_walk(x, dtype, workspace, M, K, s);
+  int rc = quantize_walk(x, dtype, workspace, M, K, type == T_Q6_K, s);
   if (rc != GGUF_OK) return rc;
   const WalkCall c = {W, workspace, Y, dtype, M, N, K, p, la};
   return taken(walk_any(type, c, s));

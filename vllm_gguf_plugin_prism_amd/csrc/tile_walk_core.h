@@ -13,17 +13,19 @@
 //   * one v_mfma_i32_32x32x32_i8 per block; the sum leaves the matrix unit as a float (the accumulator starts at the bits of 1.5 * 2^23, which stay in
 //     sixteen registers of their own: as constants the compiler moves them into every result, 1.3 times as long) and costs two multiply-adds per result:
 //     a lane holds one row of X, whose block scale is a register, and sixteen weight rows, whose block scales come from LDS once per block for all
-//     R tiles.  The mins of the super-block formats are a contraction over the eight blocks in half precision, exact.
+//     R tiles.  The mins of the super-block formats are a contraction over the eight blocks in half precision, exact.  Q6_K, with a scale per 16 values, takes two
+//     v_mfma_i32_32x32x16_i8 per block and twice the multiply-adds; Q3_K has its integer scales in the operand, which is still eight bits, and one scale per panel.
 // Four waves and two workgroups per CU, or eight waves where the output has few columns; R = 1 .. 4, as the rows fill them (walk_us).
 // Measured, us per call with the quantizer, before / now: [4096,4096] 64 rows Q4_K 16.1 / 10.8, Q8_0 19.4 / 12.6, 128 rows Q4_K 24.9 / 13.2; Q8_0 [14336,4096] 77
-// rows 38.7 / 26.5 (its weights take 12.4 from memory).  Over 7100 random products of the five formats (33 .. 2048 rows) 1.20 times the speed.
+// rows 38.7 / 26.5 (its weights take 12.4 from memory), Q6_K [4096,4096] 64 rows 20.4 / 13.6, Q3_K [14336,4096] 512 rows 128 / 98.  Over random products (33 .. 2048
+// rows) of the formats with a scale per 32 values 1.20 times the speed, of Q6_K 1.12, of Q3_K 1.26.
 // What bounds it: at few rows the beginning and the end of a workgroup (7 us of [4096,4096]'s 8 beside the quantizer); at many the vector instructions and the
 // traffic through LDS, which do not overlap as they might: a block of 32 x 32 x 32 takes a SIMD 100 ns, where its matrix instruction and 32 multiply-adds take
 // 58, the fetches of X and of weights 13 each, the operand reads 9.
 // Tried and no faster: block scales from lane to lane (row_newbcast) instead of through LDS; each workgroup touching a share of X first, so that all find it in the L2.
 // Arithmetic as in the other integer kernels (mmq.cuh:2-104: exact int32 block sums, scales in fp32); rel-L2 against 64 bits over 40 random products per format, normal
-// activations, the kernels before / this: Q8_0 9.8e-8 / 7.7e-8, Q5_0 9.7 / 7.7, Q4_0 13.2 / 7.7, Q4_K 14.4 / 11.6, Q5_K 9.3 / 8.1; of one sign Q8_0 10.0 / 7.8, Q5_0 7.0 / 5.3,
-// Q4_0 46 / 31, Q4_K 117 / 85, Q5_K 5.8 / 4.7: with one and two tiles of rows a panel has a sum of its own.
+// activations, the kernels before / this: Q8_0 9.8e-8 / 7.7e-8, Q5_0 9.7 / 7.7, Q4_0 13.2 / 7.7, Q4_K 14.4 / 11.6, Q5_K 9.3 / 8.1, Q6_K 9.9 / 8.8, Q3_K 8.1 / 7.5; of one sign Q8_0 10.0 / 7.8, Q5_0 7.0 / 5.3,
+// Q4_0 46 / 31, Q4_K 117 / 85, Q5_K 5.8 / 4.7, Q6_K 9.9 / 8.9, Q3_K 8.2 / 7.7: with one and two tiles of rows (Q6_K: and three, Q3_K always) a panel has a sum of its own.
 #pragma once
 #include "mmq_i_core.h"
 #include "q8_1_device.h"
@@ -50,13 +52,15 @@ struct WalkArgs {
 };
 
 template <int N> __device__ __forceinline__ void walk_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-// wave-uniform 16-byte-per-lane fetch into LDS: lane l's bytes land at m0 + 16 l
-__device__ __forceinline__ void walk_fetch(uint32_t at, const void* base, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(at), "s"(base), "s"(lds) : "memory");
+// wave-uniform 16-byte-per-lane fetch into LDS: lane l's bytes land at lds + AT + 16 l.  (The sum is formed here, by a scalar instruction: as an operand the
+// compiler may have formed it in a vector register, with the addresses that the lanes read from.)
+template <int AT> __device__ __forceinline__ void walk_fetch(uint32_t at, const void* base, uint32_t lds) {
+  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(at), "s"(base), "s"(lds), "n"(AT) : "memory", "scc");
 }
 // the same for lanes 0 .. 31 (all lanes are active before and after)
-__device__ __forceinline__ void walk_fetch_half(uint32_t at, const void* base, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(at), "s"(base), "s"(lds), "s"(0xFFFFFFFFull) : "memory");
+template <int AT> __device__ __forceinline__ void walk_fetch_half(uint32_t at, const void* base, uint32_t lds) {
+  asm volatile("s_add_u32 m0, %2, %4\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(at), "s"(base), "s"(lds), "s"(0xFFFFFFFFull), "n"(AT)
+               : "memory", "scc");
 }
 template <typename T>
 __device__ __forceinline__ void walk_store(const walk_f4& v, T* y, const T* bias, int n, int N, int quads) {
@@ -82,7 +86,8 @@ constexpr int WALK_PD = 8;
 template <class F> constexpr int walk_ppr() { return ((F::CUT ? F::PB + 29 : F::PB) / 16) | 1; }   // 16-byte pieces of a panel row (odd: banks)
 template <class F> constexpr int64_t walk_row_bytes(int64_t K) { return F::KQ ? K / 256 * F::PB : K / 32 * (F::PB / 8); }
 template <class F> constexpr int walk_head() { return F::OFF ? 1024 : 512; }
-template <class F, int R, int D> constexpr int walk_place() { return 512 * walk_ppr<F>() * D + 1024 * WALK_PD + walk_head<F>() * R + (F::OFF == MINS ? 1152 : 1024); }
+template <class F> constexpr int walk_scales() { return (F::WHOLE ? 128 : F::G == 16 ? 2048 : 1024) + (F::OFF == MINS ? 128 : 0); }
+template <class F, int R, int D> constexpr int walk_place() { return 512 * walk_ppr<F>() * D + 1024 * WALK_PD + walk_head<F>() * R + walk_scales<F>(); }
 template <class F, int R, int NW, int D> constexpr size_t walk_lds() {
   return (size_t)NW * walk_place<F, R, D>() + 16 > (size_t)NW * R * 4096 ? (size_t)NW * walk_place<F, R, D>() + 16 : (size_t)NW * R * 4096;
 }
@@ -93,12 +98,12 @@ template <class L, int... U> __device__ __forceinline__ void walk_units(const L&
 
 template <class F, int R, int NW, int D>
 __global__ __launch_bounds__(64 * NW, 2) void tile_walk_kernel(const uint8_t* __restrict__ W, const char* __restrict__ X, void* __restrict__ Y, WalkArgs a) {
-  constexpr int PPR = walk_ppr<F>(), SLOT = 512 * PPR, NI = (32 * PPR + 63) / 64, PD = WALK_PD, U = 8 * R;   // (the last fetch of a panel: lanes 0 .. 31)
+  constexpr int PPR = walk_ppr<F>(), SLOT = 512 * PPR, NI = (32 * PPR + 63) / 64, PD = WALK_PD, GS = 32 / F::G, U = 8 * R * GS;   // (the last fetch of a panel: lanes 0 .. 31)
   constexpr int HEAD = walk_head<F>(), XR_AT = SLOT * D, HD_AT = XR_AT + 1024 * PD, SC_AT = HD_AT + HEAD * R, PLACE = walk_place<F, R, D>();
-  constexpr bool PART = R <= 2;                             // a panel's sum of its own, where the registers hold it
+  constexpr bool PART = R <= (F::G == 16 ? 3 : 2) || F::WHOLE;                             // a panel's sum of its own, where the registers hold it
   constexpr int DB = F::CUT && R >= 3 ? 1 : 2;              // block scales in registers, of this block and, where these suffice, of the next
   constexpr int NL = NI + R;                                // fetches of a panel and of the heads of a panel's rows of X
-  static_assert(PD == 8 && U % PD == 0, "the ring's places are the same in every panel; the waits below count to eight");
+  static_assert(PD == 8 && 8 * R % PD == 0, "the ring's places are the same in every panel; the waits below count to eight");
   static_assert(PPR % 2 == 1 && walk_lds<F, R, NW, D>() <= 160 * 1024, "the last fetch of a panel is half a fetch; LDS");
   extern __shared__ __align__(16) char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -130,22 +135,26 @@ __global__ __launch_bounds__(64 * NW, 2) void tile_walk_kernel(const uint8_t* __
 #pragma unroll
   for (int k = 0; k < R; ++k) xt[k] = X + (int64_t)min(rb * R + k, a.row_tiles - 1) * a.np * WALK_REC;
   const auto request_w = [&](int p, int slot) {
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
+    const uint32_t to = lds0 + slot * SLOT;
+    walk_units([&](auto at) {
+      constexpr int i = decltype(at)::value;
       const uint32_t v = min(((w_at[i] + (uint32_t)(p * F::PB)) & ~15u) + w_piece[i], last16);
-      if (i < NI - 1) walk_fetch(v, wbase, lds0 + slot * SLOT + 1024 * i);
-      else walk_fetch_half(v, wbase, lds0 + slot * SLOT + 1024 * i);
-    }
+      if constexpr (i < NI - 1) walk_fetch<1024 * i>(v, wbase, to);
+      else walk_fetch_half<1024 * i>(v, wbase, to);
+    }, std::make_integer_sequence<int, NI>());
   };
   const auto request_heads = [&](int p) {
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
+    walk_units([&](auto at) {
+      constexpr int k = decltype(at)::value;
       const char* const base = xt[k] + (int64_t)p * WALK_REC + WALK_D_AT;
-      if (F::OFF) walk_fetch(16 * lane, base, lds0 + HD_AT + 1024 * k);
-      else walk_fetch_half(16 * lane, base, lds0 + HD_AT + 512 * k);
-    }
+      if constexpr (F::OFF) walk_fetch<HD_AT + 1024 * k>(16 * lane, base, lds0);
+      else walk_fetch_half<HD_AT + 512 * k>(16 * lane, base, lds0);
+    }, std::make_integer_sequence<int, R>());
   };
-  const auto request_x = [&](int p, int u) { walk_fetch(16 * lane, xt[u % R] + ((int64_t)p * WALK_REC + 1024 * (u / R)), lds0 + XR_AT + 1024 * (u % PD)); };
+  const auto request_x = [&](int p, auto at) {              // tile x of a panel
+    constexpr int x = decltype(at)::value;
+    walk_fetch<XR_AT + 1024 * (x % PD)>(16 * lane, xt[x % R] + ((int64_t)p * WALK_REC + 1024 * (x / R)), lds0);
+  };
 
   float acc[R][16];
 #pragma unroll
@@ -156,8 +165,7 @@ __global__ __launch_bounds__(64 * NW, 2) void tile_walk_kernel(const uint8_t* __
     request_w(wave, 0);
     request_heads(wave);
     if (D == 2 && wave + NW < a.np) request_w(wave + NW, 1);
-#pragma unroll
-    for (int u = 0; u < PD; ++u) request_x(wave, u);
+    walk_units([&](auto x) { request_x(wave, x); }, std::make_integer_sequence<int, PD>());
   }
   v16i seed;
 #pragma unroll
@@ -185,46 +193,58 @@ __global__ __launch_bounds__(64 * NW, 2) void tile_walk_kernel(const uint8_t* __
     const bool refill = D == 1 ? MORE : MORE && p + 2 * NW < a.np;
     if constexpr (MORE) request_heads(p + NW);
     if (refill) request_w(p + D * NW, slot);
-    // Unit u's tile has landed.  Asked for behind it: of the tiles under way with u = 0 the others, else two less (those that take the places of the last
-    // two units are asked for behind this), and, if it was asked for before this panel began, what was asked for then.
-    const auto ready = [&](auto at) {
-      constexpr int u = decltype(at)::value, behind = u == 0 ? PD - 1 : u == 1 ? PD - 2 : PD - 3;
-      if constexpr (!MORE) {
-        walk_wait<(U - 1 - u < behind ? U - 1 - u : behind)>();
-      } else if constexpr (u >= PD) {
-        walk_wait<behind>();
-      } else {
-        if (refill) walk_wait<behind + NL>();
-        else walk_wait<behind + R>();
-      }
+    // A unit is a block's group of values and a tile of rows, in the order (block, group, tile).  Tile x of the panel (block x / R, rows x % R) takes the place of tile
+    // x - PD as soon as the last unit of that has its operand.  Here unit u, which needs tile x, makes sure that it has landed, before unit `now` has asked for
+    // its tile: behind it were asked for all tiles up to that one's and, if it was asked for before this panel began, what was asked for then.
+    const auto ready = [&](auto at, auto before) {
+      constexpr int u = decltype(at)::value, now = decltype(before)::value, x = u / (R * GS) * R + u % R;
+      constexpr int asked = PD + now / (R * GS) * R + (now / R % GS == GS - 1 ? now % R : 0), behind = (MORE || asked < 8 * R ? asked : 8 * R) - 1 - x;
+      if constexpr (u / R % GS != 0) return;                // (its first group's unit has made sure)
+      else if constexpr (!MORE || x >= PD) walk_wait<behind>();
+      else if (refill) walk_wait<behind + NL>();
+      else walk_wait<behind + R>();
     };
     float part[PART ? R : 1][16];
-    v4i xo[2];
+    typedef typename std::conditional<GS == 2, long, v4i>::type Codes;
+    Codes xo[2], wo;
     v16i s[2];
     walk_f4 dw[DB][4];
-    const auto load_x = [&](int u) { xo[u & 1] = *(const v4i*)(mine + XR_AT + 1024 * (u % PD) + 16 * lane); };
-    const auto load_dw = [&](int b) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) dw[b % DB][q] = *(const walk_f4*)(scales + 32 * b + 8 * q + 4 * half);
+    const auto load_x = [&](int u) {
+      const int x = u / (R * GS) * R + u % R, g = u / R % GS;
+      xo[u & 1] = *(const Codes*)(mine + XR_AT + 1024 * (x % PD) + 512 * g + (GS == 2 ? 8 : 16) * lane);
     };
-    v4i wo = w.codes(0, half);
-    ready(WalkUnit<0>());
+    const auto load_dw = [&](int i) {                       // scale i of the panel's rows
+#pragma unroll
+      for (int q = 0; q < 4; ++q) dw[i % DB][q] = *(const walk_f4*)(scales + 32 * i + 8 * q + 4 * half);
+    };
+    const auto load_w = [&](int i) {
+      if constexpr (GS == 2) wo = w.codes(i >> 1, i & 1);
+      else wo = w.codes(i, half);
+    };
+    const auto mfma = [&](int u) {
+      if constexpr (GS == 2) s[u & 1] = __builtin_amdgcn_mfma_i32_32x32x16_i8(wo, xo[u & 1], seed, 0, 0, 0);
+      else s[u & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wo, xo[u & 1], seed, 0, 0, 0);
+    };
+    load_w(0);
+    ready(WalkUnit<0>(), WalkUnit<0>());
     load_x(0);
-    ready(WalkUnit<1>());
+    ready(WalkUnit<1>(), WalkUnit<0>());
     load_x(1);
-    load_dw(0);
-    s[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wo, xo[0], seed, 0, 0, 0);
+    if (!F::WHOLE) load_dw(0);
+    mfma(0);
     const auto unit = [&](auto at) {
-      constexpr int u = decltype(at)::value, b = u / R, k = u % R;
+      constexpr int u = decltype(at)::value, i = u / R, b = i / GS, k = u % R, x = b * R + k;   // i: the scale of the panel
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (u + 2 < U) {
-        ready(WalkUnit<u + 2>());
+        ready(WalkUnit<u + 2>(), at);
         load_x(u + 2);
       }
-      if (DB == 2 && k == 0 && b + 1 < 8) load_dw(b + 1);
-      if (u + PD < U) request_x(p, u + PD);                 // (unit u's operand has been read: its matrix instruction has started)
-      else if (MORE) request_x(p + NW, u + PD - U);
-      if (u + 1 < U && (u + 1) % R == 0) wo = w.codes((u + 1) / R, half);
+      if (!F::WHOLE && DB == 2 && k == 0 && u + R < U) load_dw(i + 1);
+      if constexpr (i % GS == GS - 1) {                               // (the unit's operand has been read: its matrix instruction has started)
+        if constexpr (x + PD < 8 * R) request_x(p, WalkUnit<x + PD>());
+        else if constexpr (MORE) request_x(p + NW, WalkUnit<x + PD - 8 * R>());
+      }
+      if (u + 1 < U && k == R - 1) load_w(i + 1);
       const uint32_t dp = b < 2 ? dh[k].x : b < 4 ? dh[k].y : b < 6 ? dh[k].z : dh[k].w;
       float d8 = half_bits(b & 1 ? dp >> 16 : dp & 0xFFFF);
       asm volatile("" : "+v"(d8));                          // (a float from here on: the compiler would have every multiply-add convert it, in a form that takes twice as long)
@@ -236,13 +256,14 @@ __global__ __launch_bounds__(64 * NW, 2) void tile_walk_kernel(const uint8_t* __
         m8 = -8.0f * half_bits(b & 1 ? sp >> 16 : sp & 0xFFFF);
         asm volatile("" : "+v"(m8));
       }
-      if (u + 1 < U) s[(u + 1) & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wo, xo[(u + 1) & 1], seed, 0, 0, 0);
+      if (u + 1 < U) mfma(u + 1);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         float v = __builtin_fmaf(__builtin_bit_cast(float, (int)s[u & 1][r]), d8, nd);   // d8 times the block's sum, rounded once
         if constexpr (F::OFF == EIGHTS) v += m8;
-        sum[r] = PART && b == 0 ? v * dw[b % DB][r >> 2][r & 3] : __builtin_fmaf(v, dw[b % DB][r >> 2][r & 3], sum[r]);
+        if constexpr (F::WHOLE) sum[r] = i == 0 ? v : sum[r] + v;
+        else sum[r] = PART && i == 0 ? v * dw[i % DB][r >> 2][r & 3] : __builtin_fmaf(v, dw[i % DB][r >> 2][r & 3], sum[r]);
       }
       // The offsets, a contraction over eight (the upper half of the lanes holds values 8 .. 15, zeros), in the middle of the panel
       if constexpr (F::OFF == MINS) if constexpr (b == 3) {
@@ -258,11 +279,13 @@ __global__ __launch_bounds__(64 * NW, 2) void tile_walk_kernel(const uint8_t* __
           for (int e = 0; e < 4; ++e) sum[4 * q + e] = __builtin_fmaf(off[4 * q + e], dm[e], sum[4 * q + e]);
         }
       }
-      if constexpr (PART && b == 7)
+      if constexpr (PART && u + R >= U) {
+        if (F::WHOLE && k == 0) load_dw(0);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[k][r] += sum[r];
-      walk_pin(PART && b == 7 ? acc[k] : sum);
-      if (DB == 1 && k == R - 1 && b + 1 < 8) load_dw(b + 1);
+        for (int r = 0; r < 16; ++r) acc[k][r] = F::WHOLE ? __builtin_fmaf(sum[r], dw[0][r >> 2][r & 3], acc[k][r]) : acc[k][r] + sum[r];
+      }
+      walk_pin(PART && u + R >= U ? acc[k] : sum);
+      if (!F::WHOLE && DB == 1 && k == R - 1 && u + 1 < U) load_dw(i + 1);
     };
     walk_units(unit, std::make_integer_sequence<int, U>());
   };
@@ -327,7 +350,8 @@ static int walk_run(const WalkCall& c, hipStream_t s) {
     case 2 * 16 + 4: return walk_launch<F, 2, 4>(c, s);
     case 2 * 16 + 8: return walk_launch<F, 2, 8>(c, s);
     case 3 * 16 + 4: return walk_launch<F, 3, 4>(c, s);
-    case 4 * 16 + 4: return walk_launch<F, 4, 4>(c, s);
+    case 4 * 16 + 4:
+      if constexpr (F::G == 32) return walk_launch<F, 4, 4>(c, s);   // (else there is no such plan)
   }
   return GGUF_NOT_TAKEN;
 }
