@@ -85,6 +85,7 @@ EXPORTS = tuple(_SIGNATURES)
 # entry points behind the layer calls only (csrc/dense_api.h), not part of the public header
 _LAYER_SIGNATURES = {
     "gguf_dense_linear_takes": (_c.c_int, [_c.c_int, _c.c_int, _c.c_int64, _c.c_int64, _c.c_int64]),
+    "gguf_dense_linear_walk": (_c.c_int, [_c.c_int, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64]),
     "gguf_dense_linear_workspace_bytes": (_c.c_int64, [_c.c_int64, _c.c_int64, _c.c_int64]),
     "gguf_mmq_layer_workspace_bytes": (_c.c_int64, [_c.c_int, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64]),
     "gguf_mmq_layer_unit": (_c.c_int, [_c.c_int, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64]),

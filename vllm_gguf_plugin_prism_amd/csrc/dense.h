@@ -12,6 +12,8 @@ struct DenseCall {
   LinearArgs la;
 };
 
+double dense_us(int M, int N, int K);   // about how long it takes
+
 int dense_iq4_xs(const DenseCall& c, const TilePlan& p, hipStream_t s);
 int dense_iq4_nl(const DenseCall& c, const TilePlan& p, hipStream_t s);
 int dense_iq2_xxs(const DenseCall& c, const TilePlan& p, hipStream_t s);

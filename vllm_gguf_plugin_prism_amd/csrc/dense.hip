@@ -1,6 +1,8 @@
 // Plans, dispatch and entry points of the codebook formats' GEMM (dense_core.h).
 #include "dense.h"
 #include "dense_api.h"
+#include "dense_walk.h"
+#include <algorithm>
 
 namespace gguf {
 
@@ -42,6 +44,12 @@ static TilePlan dense_plan(int M, int N, int K, double& least) {
   return best;
 }
 
+double dense_us(int M, int N, int K) {
+  double us;
+  (void)dense_plan(M, N, K, us);
+  return us;
+}
+
 static int dense_any(int type, const DenseCall& c, const TilePlan& p, hipStream_t s) {
   switch (type) {
     case T_IQ2_XXS: return dense_iq2_xxs(c, p, s);
@@ -77,7 +85,14 @@ extern "C" int gguf_dense_linear_takes(int type, int xdtype, int64_t N, int64_t 
 extern "C" int64_t gguf_dense_linear_workspace_bytes(int64_t N, int64_t K, int64_t M) {
   if (M <= 0 || N <= 0 || K <= 0 || M > 0x7FFFFFF0LL || N > 0x7FFFFFF0LL || K > 0x7FFFFFF0LL) return 0;
   double us;
-  return gguf::dense_plan((int)M, (int)N, (int)K, us).partial_bytes();
+  return std::max(gguf::dense_plan((int)M, (int)N, (int)K, us).partial_bytes(), gguf::dwalk_workspace_bytes(M, K));
+}
+
+extern "C" int gguf_dense_linear_walk(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes) {
+  using namespace gguf;
+  if (!gguf_dense_linear_takes(type, GGUF_DTYPE_F16, N, K, M)) return 0;
+  const WalkPlan p = dwalk_plan(type, M, N, K, w_row_pitch_bytes, workspace_bytes);
+  return 16 * p.rt + p.nw;
 }
 
 extern "C" int gguf_dense_linear(const void* W, int64_t w_row_pitch_bytes, const void* x, int xdtype, void* workspace, void* Y,
@@ -94,10 +109,16 @@ extern "C" int gguf_dense_linear(const void* W, int64_t w_row_pitch_bytes, const
   const TilePlan p = dense_plan((int)M, (int)N, (int)K, us);
   if (!W || !x || !Y || (p.shared && !workspace)) return GGUF_ERR_NULL;
   if (((uintptr_t)W & 1) || (w_row_pitch_bytes & 1) || ((uintptr_t)x & 15)) return GGUF_ERR_SHAPE;
+  LinearArgs la;
+  la.w_pitch = w_row_pitch_bytes;
+  la.ldy = y_row_pitch;
+  la.bias = bias;
+  // some tens of rows: waves that walk on their own, where the workspace has room for their rows
+  if (workspace && !((uintptr_t)workspace & 15)) {
+    const WalkPlan walk = dwalk_plan(type, M, N, K, w_row_pitch_bytes, workspace_bytes);
+    if (walk.rt) return dwalk_linear(type, W, x, xdtype, workspace, Y, (int)M, (int)N, (int)K, walk, la, (hipStream_t)stream);
+  }
   if (p.shared && (workspace_bytes < p.partial_bytes() || ((uintptr_t)workspace & 15))) return GGUF_ERR_WORKSPACE;
-  DenseCall c = {W, x, Y, xdtype, (int)M, (int)N, (int)K, (float*)workspace, LinearArgs()};
-  c.la.w_pitch = w_row_pitch_bytes;
-  c.la.ldy = y_row_pitch;
-  c.la.bias = bias;
+  const DenseCall c = {W, x, Y, xdtype, (int)M, (int)N, (int)K, (float*)workspace, la};
   return dense_any(type, c, p, (hipStream_t)stream);
 }

@@ -5,7 +5,9 @@
  * the weights rounded to X's dtype as gguf_dequantize rounds them and a 32-bit sum, the two steps of the reference's
  * fallback (quantization/linear.py:50-58) in one kernel.  Arguments as for gguf_mmq_linear; X and Y fp16 or bf16, X at a
  * 16-byte boundary, its rows dense.  gguf_dense_linear_takes: 1 for a call that it serves.  The workspace may be null
- * where gguf_dense_linear_workspace_bytes is 0; it needs no initialisation.
+ * where gguf_dense_linear_workspace_bytes is 0; it needs no initialisation; with less than that the call is slower, with less than its partial tiles take GGUF_ERR_WORKSPACE.
+ * gguf_dense_linear_walk: where a call with a workspace of this size, at a 16-byte boundary, runs dense_walk_kernel, 16 times the tiles of 32 rows that a workgroup has and its
+ * waves, else 0.
  *
  * gguf_mmq_layer_workspace_bytes: the workspace with which gguf_mmq_linear on GGUF_MMQ_AUTO runs at full speed for weights
  * of this type, at a 16-byte boundary.  (gguf_mmq_workspace_bytes_engine does not know the type.)  gguf_mmq_layer_route: the
@@ -30,6 +32,7 @@ extern "C" {
 #endif
 int gguf_dense_linear_takes(int type, int xdtype, int64_t N, int64_t K, int64_t M);
 int64_t gguf_dense_linear_workspace_bytes(int64_t N, int64_t K, int64_t M);
+int gguf_dense_linear_walk(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes);
 int gguf_dense_linear(const void* W, int64_t w_row_pitch_bytes, const void* x, int xdtype, void* workspace, void* Y, int64_t y_row_pitch,
                       const void* bias, int type, int64_t N, int64_t K, int64_t M, int64_t workspace_bytes, void* stream);
 int64_t gguf_mmq_layer_workspace_bytes(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes);

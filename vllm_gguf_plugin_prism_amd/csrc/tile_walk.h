@@ -30,8 +30,8 @@ struct WalkCall {
 // on their way, the row blocks of a band one after the other for each group of columns; the last band has `last`.  ok: the kernel's quotients by
 // reciprocal are exact (dividend times divisor stays below 2^32).
 struct WalkBands { int tiles, band, band_tiles, last; bool ok; };
-static inline WalkBands walk_bands(int rt, int64_t M, int64_t N, int64_t K) {
-  const int64_t cols = (N + 31) / 32, blocks = (M + 32 * rt - 1) / (32 * rt), fit = (3 << 20) / (rt * ((K + 255) / 256) * WALK_REC);
+static inline WalkBands walk_bands(int rt, int64_t M, int64_t N, int64_t K, int rec = WALK_REC) {
+  const int64_t cols = (N + 31) / 32, blocks = (M + 32 * rt - 1) / (32 * rt), fit = (3 << 20) / (rt * ((K + 255) / 256) * rec);
   const int64_t band = fit >= blocks ? blocks : fit > 1 ? fit : 1, tiles = cols * blocks;
   return {(int)tiles, (int)band, (int)(cols * band), (int)(blocks - (blocks - 1) / band * band), tiles <= 0x7FFFFFF && tiles * cols * band <= 0xFFFFFFFFll};
 }
