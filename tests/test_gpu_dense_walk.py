@@ -11,12 +11,14 @@ FORMATS = sorted(D.IMATRIX_QUANT_TYPES)
 TOLERANCE = {torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}   # two roundings to 16 bits (product, product plus bias), each half a unit in the last place of 11 or 8 bits
 
 
-EDGES = [(33, 4155, 512, 2, (1, 4)), (68, 4327, 1280, 0, (1, 4)), (69, 4313, 2304, 6, (1, 4)), (18, 1205, 1280, 0, (1, 8)), (27, 3001, 2560, 4, (1, 8)), (17, 3693, 4352, 0, (1, 8)),
+EDGES = [(33, 4155, 512, 2, (1, 4)), (68, 4327, 1280, 0, (1, 4)), (69, 4313, 2304, 6, (1, 4)), (35, 1144, 512, 0, (1, 8)), (71, 1215, 3072, 4, (1, 8)), (79, 1564, 5120, 0, (1, 8)),
          (65, 5539, 768, 0, (2, 4)), (99, 4120, 1280, 8, (2, 4)), (65, 5513, 2304, 0, (2, 4)), (553, 466, 768, 10, (2, 8)), (35, 4405, 2304, 0, (2, 8)), (68, 2981, 4352, 2, (2, 8)),
          (129, 6575, 768, 12, (3, 4)), (197, 4104, 1280, 0, (3, 4)), (135, 5986, 2304, 0, (3, 4)), (203, 4894, 768, 0, (4, 4)), (193, 5530, 1280, 14, (4, 4)), (203, 5506, 2304, 0, (4, 4)),
-         (614, 1380, 1536, 0, (4, 8)), (613, 915, 2304, 2, (4, 8)), (194, 2856, 5120, 0, (4, 8))]
-BEHIND = [(D.IQ3_XXS, 18, 230, 1280), (D.IQ3_XXS, 71, 210, 1536), (D.IQ3_XXS, 129, 210, 1280), (D.IQ3_XXS, 35, 8986, 512), (D.IQ4_XS, 66, 5487, 512), (D.IQ3_XXS, 129, 3343, 512),
-          (D.IQ4_XS, 17, 1, 256), (D.IQ1_S, 65, 300, 2816), (D.IQ2_S, 1025, 300, 512)]
+         (614, 1380, 1536, 0, (4, 8)), (613, 915, 2304, 2, (4, 8)), (194, 2856, 5120, 0, (4, 8)),
+         (5, 41, 1280, 0, (17, 8)), (16, 1182, 2304, 2, (17, 8)), (32, 3001, 1280, 6, (17, 8)), (5, 1801, 5120, 0, (17, 8)), (5, 8254, 512, 4, (17, 4)), (9, 11006, 1280, 0, (17, 4)),
+         (13, 24757, 2304, 0, (17, 4))]   # (17: one tile of rows, loaded as they lie)
+BEHIND = [(D.IQ3_XXS, 4, 230, 1280), (D.IQ3_XXS, 71, 210, 1536), (D.IQ3_XXS, 129, 210, 1280), (D.IQ3_XXS, 35, 8986, 512), (D.IQ4_XS, 66, 5487, 512), (D.IQ3_XXS, 129, 3343, 512),
+          (D.IQ2_S, 24, 4096, 18944), (D.IQ1_S, 65, 300, 2816), (D.IQ2_S, 1025, 300, 512)]
 
 
 def plan(qt, m, n, k, pitch, size=None):
@@ -57,7 +59,7 @@ def test_edges(qt, m, n, k, pad, want):
 
 
 # K in blocks of 32: the last panel has one block, three, seven
-@pytest.mark.parametrize("m,n,k,pad", [(70, 4100, 2080, 0), (45, 3333, 1120, 2), (130, 4444, 2528, 0), (37, 3333, 992, 6)])
+@pytest.mark.parametrize("m,n,k,pad", [(70, 4100, 2080, 0), (45, 3333, 1120, 2), (130, 4444, 2528, 0), (37, 3333, 992, 6), (20, 3333, 160, 0), (32, 1700, 992, 2), (7, 2001, 2080, 0)])
 def test_last_panels(m, n, k, pad):
     check(D.IQ4_NL, torch.float16, m, n, k, None, pad)
 
@@ -65,22 +67,24 @@ def test_last_panels(m, n, k, pad):
 # both types, weights that begin anywhere, results that are columns of a wider tensor
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("offset,pad,column,spare", [(0, 0, 0, 0), (2, 14, 3, 4), (16, 16, 4, 4), (6, 4, 1, 0)])
+@pytest.mark.parametrize("m", [34, 13])
 @pytest.mark.parametrize("qt", FORMATS)
-def test_forms(qt, offset, pad, column, spare, dt):
-    check(qt, dt, 34, 3301, 1280, None, pad, offset, column, spare)
+def test_forms(qt, m, offset, pad, column, spare, dt):
+    check(qt, dt, m, 3301, 1280, None, pad, offset, column, spare)
 
 
 # a value that is not a number stays in its row
-def test_rows_do_not_meet():
+@pytest.mark.parametrize("m", [34, 13])
+def test_rows_do_not_meet(m):
     from vllm_gguf_plugin_prism_amd import ops
-    m, n, k = 34, 3301, 1280
+    n, k = 3301, 1280
     w = torch.from_numpy(synth.make_weights(np.random.default_rng(1), D.IQ3_S, n, k)).cuda()
     assert plan(D.IQ3_S, m, n, k, w.shape[1])[0]
     x = torch.randn(m, k, dtype=torch.bfloat16, device="cuda")
     y = ops.dense_linear(w, x, D.IQ3_S, n)
-    x[33, 1000] = float("nan")
+    x[m - 1, 1000] = float("nan")
     z = ops.dense_linear(w, x, D.IQ3_S, n)
-    assert bool(z[33].isnan().all()) and torch.equal(z[:33], y[:33])
+    assert bool(z[m - 1].isnan().all()) and torch.equal(z[:m - 1], y[:m - 1])
 
 
 # the kernel behind it: products that it does not take, and a workspace with no room for the rows

@@ -91,8 +91,8 @@ extern "C" int64_t gguf_dense_linear_workspace_bytes(int64_t N, int64_t K, int64
 extern "C" int gguf_dense_linear_walk(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes) {
   using namespace gguf;
   if (!gguf_dense_linear_takes(type, GGUF_DTYPE_F16, N, K, M)) return 0;
-  const WalkPlan p = dwalk_plan(type, M, N, K, w_row_pitch_bytes, workspace_bytes);
-  return 16 * p.rt + p.nw;
+  const DwalkPlan p = dwalk_plan(type, M, N, K, w_row_pitch_bytes, workspace_bytes);
+  return 256 * p.direct + 16 * p.rt + p.nw;
 }
 
 extern "C" int gguf_dense_linear(const void* W, int64_t w_row_pitch_bytes, const void* x, int xdtype, void* workspace, void* Y,
@@ -113,12 +113,10 @@ extern "C" int gguf_dense_linear(const void* W, int64_t w_row_pitch_bytes, const
   la.w_pitch = w_row_pitch_bytes;
   la.ldy = y_row_pitch;
   la.bias = bias;
-  // some tens of rows: waves that walk on their own, where the workspace has room for their rows
-  if (workspace && !((uintptr_t)workspace & 15)) {
-    const WalkPlan walk = dwalk_plan(type, M, N, K, w_row_pitch_bytes, workspace_bytes);
-    if (walk.rt) return dwalk_linear(type, W, x, xdtype, workspace, Y, (int)M, (int)N, (int)K, walk, la, (hipStream_t)stream);
-  }
   if (p.shared && (workspace_bytes < p.partial_bytes() || ((uintptr_t)workspace & 15))) return GGUF_ERR_WORKSPACE;
+  // some or some tens of rows: waves that walk on their own, those that want records where the workspace has room for them
+  const DwalkPlan walk = dwalk_plan(type, M, N, K, w_row_pitch_bytes, workspace && !((uintptr_t)workspace & 15) ? workspace_bytes : 0);
+  if (walk.rt) return dwalk_linear(type, W, x, xdtype, workspace, Y, (int)M, (int)N, (int)K, walk, la, (hipStream_t)stream);
   const DenseCall c = {W, x, Y, xdtype, (int)M, (int)N, (int)K, (float*)workspace, la};
   return dense_any(type, c, p, (hipStream_t)stream);
 }

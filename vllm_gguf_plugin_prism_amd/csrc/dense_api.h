@@ -7,7 +7,7 @@
  * 16-byte boundary, its rows dense.  gguf_dense_linear_takes: 1 for a call that it serves.  The workspace may be null
  * where gguf_dense_linear_workspace_bytes is 0; it needs no initialisation; with less than that the call is slower, with less than its partial tiles take GGUF_ERR_WORKSPACE.
  * gguf_dense_linear_walk: where a call with a workspace of this size, at a 16-byte boundary, runs dense_walk_kernel, 16 times the tiles of 32 rows that a workgroup has and its
- * waves, else 0.
+ * waves, and 256 where it loads X as it lies, else 0.
  *
  * gguf_mmq_layer_workspace_bytes: the workspace with which gguf_mmq_linear on GGUF_MMQ_AUTO runs at full speed for weights
  * of this type, at a 16-byte boundary.  (gguf_mmq_workspace_bytes_engine does not know the type.)  gguf_mmq_layer_route: the

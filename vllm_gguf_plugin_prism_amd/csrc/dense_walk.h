@@ -11,18 +11,21 @@ namespace gguf {
 constexpr int DWALK_REC = 16384;
 static inline int64_t dwalk_rows_bytes(int64_t M, int64_t K) { return (M + 31) / 32 * ((K + 255) / 256) * DWALK_REC; }
 
+// Tiles of 32 rt rows, nw waves; direct: one tile of rows, loaded from X as it lies
+struct DwalkPlan { int rt, nw; bool direct; };
+
 struct DwalkCall {
   const void* W;
-  const void* x;               // records
+  const void* x;               // records; of a direct plan the rows as they lie
   void* Y;
   int dtype, M, N, K;
-  WalkPlan plan;
+  DwalkPlan plan;
   LinearArgs la;
 };
 
 // Whether a product runs here with a workspace of this size, and how (rt 0: not); the workspace that takes; the call
-WalkPlan dwalk_plan(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, int64_t workspace_bytes);
+DwalkPlan dwalk_plan(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, int64_t workspace_bytes);
 int64_t dwalk_workspace_bytes(int64_t M, int64_t K);
-int dwalk_linear(int type, const void* W, const void* x, int dtype, void* workspace, void* Y, int M, int N, int K, const WalkPlan& p, const LinearArgs& la, hipStream_t s);
+int dwalk_linear(int type, const void* W, const void* x, int dtype, void* workspace, void* Y, int M, int N, int K, const DwalkPlan& p, const LinearArgs& la, hipStream_t s);
 
 }  // namespace gguf

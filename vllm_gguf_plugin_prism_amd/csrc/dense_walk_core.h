@@ -7,13 +7,14 @@
 //   * A lane decodes sixteen values of one weight row, half of a block of 32, as dense_core.h does, rounded to X's type: two operands of v_mfma_f32_32x32x16.  The order of K
 //     inside a block is the lanes': values 16 h .. of the block belong to half h.
 //   * X is put into that order by a launch of its own (dwalk_rows_kernel: 2.3 us), so that an operand is 1 KB whose lanes follow one another, loaded straight to
-//     registers, three blocks ahead (four tiles of rows: one, where the registers hold no more).  (From X as it lies, without that launch: 17 rows of [5120,5120] 11.9 instead of
-//     13.3 us, but 64 rows 22.5 instead of 15.7: an instruction touches 32 lines.)
-// Measured, us, before / now: IQ4_XS [5120,5120] 17 rows 18.6 / 13.3, 128 rows 24.7 / 22, 256 rows 32.4 / 31.6; [4096,4096] 64 rows 19.2 / 11.6; [14336,4096] 64 rows 27.7 / 23; IQ2_XXS
+//     registers, three blocks ahead (four tiles of rows: one, where the registers hold no more).
+//   * DIRECT: one tile of rows, taken from X as it lies, without that launch: an instruction touches a line per row, which few enough rows allow (17 rows of [5120,5120] 11.0
+//     instead of 12.6 us; 32 rows of [28672,4096] 42 instead of 33, 64 of [5120,5120] 22.5 instead of 15.7).
+// Measured, us, before / now: IQ4_XS [14336,4096] 12 rows 27.6 / 17.5; [5120,5120] 17 rows 17.5 / 11.0, 128 rows 24.7 / 22, 256 rows 32.4 / 31.6; [4096,4096] 64 rows 19.2 / 11.6; [14336,4096] 64 rows 27.7 / 23; IQ2_XXS
 // [4096,5120] 100 rows 25.8 / 15.9.  What bounds it: the decoding (65 vector instructions a block, again for every tile of rows) and the matrix instructions, which overlap
 // little (tile_walk_core.h), and how the workgroups fill the chip.  Tried and no faster: seven blocks of X ahead.
 // The operands are the ones of dense_kernel, in another order of the fp32 sum: 60 random products, rel-L2 of the half results against 64 bits 2.074e-4 both, results that are
-// not the nearest half 0.08 % both.
+// not the nearest half 0.08 % both; of 5 .. 32 rows 0.082 before and 0.074 % now, with activations of one sign 0.064 and 0.060 %.
 #pragma once
 #include "dense_core.h"
 #include "dense_walk.h"
@@ -30,7 +31,7 @@ template <class F, int R, int NW> constexpr size_t dwalk_lds() {
   return table + (place > (size_t)NW * R * 4096 ? place : (size_t)NW * R * 4096);
 }
 
-template <class F, int R, int NW, typename T>
+template <class F, int R, int NW, bool DIRECT, typename T>
 __global__ __launch_bounds__(64 * NW, 2) void dense_walk_kernel(const uint8_t* __restrict__ W, const char* __restrict__ X, T* __restrict__ Y, WalkArgs a) {
   constexpr int UB = dwalk_unit<F>(), PPR = dwalk_ppr(UB), SLOT = 512 * PPR, NI = (32 * PPR + 63) / 64;   // (the last fetch of a panel: lanes 0 .. 31)
   typedef DenseType<T> D;
@@ -71,7 +72,8 @@ __global__ __launch_bounds__(64 * NW, 2) void dense_walk_kernel(const uint8_t* _
   };
   const char* xt[R];
 #pragma unroll
-  for (int k = 0; k < R; ++k) xt[k] = X + (int64_t)min(rb * R + k, a.row_tiles - 1) * a.np * DWALK_REC;
+  for (int k = 0; k < R; ++k) xt[k] = DIRECT ? X : X + (int64_t)min(rb * R + k, a.row_tiles - 1) * a.np * DWALK_REC;
+  const uint32_t x_lane = DIRECT ? (uint32_t)min(lrow, a.M - 1) * (uint32_t)(64 * a.nkb) + 32 * (uint32_t)half : 16 * (uint32_t)lane;
   typedef typename D::v8 v8;
   constexpr int XD = R >= 4 ? 2 : 4;                     // blocks of activations in registers
   v8 x[XD][R][2];
@@ -79,14 +81,14 @@ __global__ __launch_bounds__(64 * NW, 2) void dense_walk_kernel(const uint8_t* _
 #pragma unroll
     for (int k = 0; k < R; ++k)
 #pragma unroll
-      for (int t = 0; t < 2; ++t) o[k][t] = *(const v8*)(xt[k] + ((int64_t)p * DWALK_REC + 2048 * b + 1024 * t) + 16 * (uint32_t)lane);
+      for (int t = 0; t < 2; ++t) o[k][t] = *(const v8*)(xt[k] + ((int64_t)p * (DIRECT ? 512 : DWALK_REC) + (DIRECT ? 64 * b + 16 * t : 2048 * b + 1024 * t)) + x_lane);
   };
 
-  dense_f16v acc[R];
+  dense_f16v acc[R], high;                               // DIRECT: the values 8 .. 15 of a half summed on their own (dense_kernel's parts of K are short: so are these chains)
 #pragma unroll
   for (int k = 0; k < R; ++k)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[k][r] = 0.0f;
+    for (int r = 0; r < 16; ++r) acc[k][r] = high[r] = 0.0f;
   if (wave < a.np) {
     request_w(wave, 0);
 #pragma unroll
@@ -134,11 +136,14 @@ __global__ __launch_bounds__(64 * NW, 2) void dense_walk_kernel(const uint8_t* _
 #pragma unroll
       for (int k = 0; k < R; ++k) acc[k] = D::mfma(w0, x[b % XD][k][0], acc[k]);
 #pragma unroll
-      for (int k = 0; k < R; ++k) acc[k] = D::mfma(w1, x[b % XD][k][1], acc[k]);
+      for (int k = 0; k < R; ++k)
+        if (DIRECT) high = D::mfma(w1, x[b % XD][k][1], high);
+        else acc[k] = D::mfma(w1, x[b % XD][k][1], acc[k]);
     }
   }
 
   // ---- the waves' partial tiles, added in pairs
+  if (DIRECT) acc[0] += high;
   __syncthreads();
   walk_f4* const red = (walk_f4*)(smem + TABLE);            // [wave][tile][run of four and half][row ^ that]
 #pragma unroll
@@ -159,12 +164,12 @@ __global__ __launch_bounds__(64 * NW, 2) void dense_walk_kernel(const uint8_t* _
   }
 }
 
-template <class F, int R, int NW, typename T>
+template <class F, int R, int NW, bool DIRECT, typename T>
 static int dwalk_launch(const DwalkCall& c, hipStream_t stream) {
   constexpr size_t lds = dwalk_lds<F, R, NW>();
   const WalkBands tiles = walk_bands(R, c.M, c.N, c.K, DWALK_REC);
   if (!tiles.ok) return GGUF_NOT_TAKEN;
-  auto kern = dense_walk_kernel<F, R, NW, T>;
+  auto kern = dense_walk_kernel<F, R, NW, DIRECT, T>;
   static std::atomic<uint64_t> done{0};
   allow_large_lds(kern, lds, done);
   const int64_t pitch = c.la.w_pitch ? c.la.w_pitch : (int64_t)(c.K / F::QK) * F::BS, ldy = c.la.ldy ? c.la.ldy : (int64_t)c.N;
@@ -180,13 +185,13 @@ static int dwalk_launch(const DwalkCall& c, hipStream_t stream) {
 template <class F, typename T>
 static int dwalk_typed(const DwalkCall& c, hipStream_t s) {
   switch (c.plan.rt * 16 + c.plan.nw) {
-    case 1 * 16 + 4: return dwalk_launch<F, 1, 4, T>(c, s);
-    case 1 * 16 + 8: return dwalk_launch<F, 1, 8, T>(c, s);
-    case 2 * 16 + 4: return dwalk_launch<F, 2, 4, T>(c, s);
-    case 2 * 16 + 8: return dwalk_launch<F, 2, 8, T>(c, s);
-    case 3 * 16 + 4: return dwalk_launch<F, 3, 4, T>(c, s);
-    case 4 * 16 + 4: return dwalk_launch<F, 4, 4, T>(c, s);
-    case 4 * 16 + 8: return dwalk_launch<F, 4, 8, T>(c, s);
+    case 1 * 16 + 4: return c.plan.direct ? dwalk_launch<F, 1, 4, true, T>(c, s) : dwalk_launch<F, 1, 4, false, T>(c, s);
+    case 1 * 16 + 8: return c.plan.direct ? dwalk_launch<F, 1, 8, true, T>(c, s) : dwalk_launch<F, 1, 8, false, T>(c, s);
+    case 2 * 16 + 4: return dwalk_launch<F, 2, 4, false, T>(c, s);
+    case 2 * 16 + 8: return dwalk_launch<F, 2, 8, false, T>(c, s);
+    case 3 * 16 + 4: return dwalk_launch<F, 3, 4, false, T>(c, s);
+    case 4 * 16 + 4: return dwalk_launch<F, 4, 4, false, T>(c, s);
+    case 4 * 16 + 8: return dwalk_launch<F, 4, 8, false, T>(c, s);
   }
   return GGUF_NOT_TAKEN;
 }
