@@ -43,7 +43,6 @@ template <> struct DenseType<bf16_t> {
 };
 
 typedef float dense_f16v __attribute__((ext_vector_type(16)));
-typedef float dense_f2v __attribute__((ext_vector_type(2)));
 
 template <int J> struct DenseStep { static constexpr int value = J; };
 
@@ -97,17 +96,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2 * OCC) void dense_kernel(const uint
       else return F::fetch(w_row + (uint32_t)ib * F::BS, 0, h);
     };
     const auto stash = [&](const typename F::Raw& raw, int j, int buf) {   // step j of its unit
-      uint32_t v[4];
-      const float d = F::decode(raw, table, 2 * j + (w_p >> 1), h, v), dn = -128.0f * d;
-      uint32_t o[8];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t b = v[i] ^ 0x80808080u;              // (the bytes plus 128: their conversion is one instruction each)
-        const float f0 = __builtin_fmaf((float)(b & 255u), d, dn), f1 = __builtin_fmaf((float)((b >> 8) & 255u), d, dn);
-        const float f2 = __builtin_fmaf((float)((b >> 16) & 255u), d, dn), f3 = __builtin_fmaf((float)(b >> 24), d, dn);
-        o[2 * i] = __builtin_bit_cast(uint32_t, __builtin_convertvector((dense_f2v){f0, f1}, typename D::v2));
-        o[2 * i + 1] = __builtin_bit_cast(uint32_t, __builtin_convertvector((dense_f2v){f2, f3}, typename D::v2));
-      }
+      uint32_t v[4], s[2] = {0, 0}, o[8];
+      const float d = F::decode(raw, table, 2 * j + (w_p >> 1), h, v, s);
+      dense_operands<F, typename D::v2>(v, s, d, o);
       char* const row = smem + (buf * BUF + 128 * (M_T + w_n));
       *(uint4*)(row + 16 * ((2 * w_p) ^ w_swz)) = make_uint4(o[0], o[1], o[2], o[3]);
       *(uint4*)(row + 16 * ((2 * w_p + 1) ^ w_swz)) = make_uint4(o[4], o[5], o[6], o[7]);

@@ -11,7 +11,7 @@
 //   * DIRECT: one tile of rows, taken from X as it lies, without that launch: an instruction touches a line per row, which few enough rows allow (17 rows of [5120,5120] 11.0
 //     instead of 12.6 us; 32 rows of [28672,4096] 42 instead of 33, 64 of [5120,5120] 22.5 instead of 15.7).
 // Measured, us, before / now: IQ4_XS [14336,4096] 12 rows 27.6 / 17.5; [5120,5120] 17 rows 17.5 / 11.0, 128 rows 24.7 / 22, 256 rows 32.4 / 31.6; [4096,4096] 64 rows 19.2 / 11.6; [14336,4096] 64 rows 27.7 / 23; IQ2_XXS
-// [4096,5120] 100 rows 25.8 / 15.9.  What bounds it: the decoding (65 vector instructions a block, again for every tile of rows) and the matrix instructions, which overlap
+// [4096,5120] 100 rows 25.8 / 15.9.  What bounds it: the decoding (60 to 75 vector instructions a block, again for every tile of rows) and the matrix instructions, which overlap
 // little (tile_walk_core.h), and how the workgroups fill the chip.  Tried and no faster: seven blocks of X ahead.
 // The operands are the ones of dense_kernel, in another order of the fp32 sum: 60 random products, rel-L2 of the half results against 64 bits 2.074e-4 both, results that are
 // not the nearest half 0.08 % both; of 5 .. 32 rows 0.082 before and 0.074 % now, with activations of one sign 0.064 and 0.060 %.
@@ -121,17 +121,9 @@ __global__ __launch_bounds__(64 * NW, 2) void dense_walk_kernel(const uint8_t* _
       }
       const typename F::Raw now = raw;
       if (b < 7) raw = F::fetch(F::QK == 256 ? row : row + (b + 1) * F::BS, F::QK == 256 ? b + 1 : 0, half);
-      uint32_t v[4];
-      const float d = F::decode(now, table, b, half, v), dn = -128.0f * d;
-      uint32_t o[8];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t c = v[i] ^ 0x80808080u;              // (the bytes plus 128: their conversion is one instruction each)
-        const float f0 = __builtin_fmaf((float)(c & 255u), d, dn), f1 = __builtin_fmaf((float)((c >> 8) & 255u), d, dn);
-        const float f2 = __builtin_fmaf((float)((c >> 16) & 255u), d, dn), f3 = __builtin_fmaf((float)(c >> 24), d, dn);
-        o[2 * i] = __builtin_bit_cast(uint32_t, __builtin_convertvector((dense_f2v){f0, f1}, typename D::v2));
-        o[2 * i + 1] = __builtin_bit_cast(uint32_t, __builtin_convertvector((dense_f2v){f2, f3}, typename D::v2));
-      }
+      uint32_t v[4], s[2] = {0, 0}, o[8];
+      const float d = F::decode(now, table, b, half, v, s);
+      dense_operands<F, typename D::v2>(v, s, d, o);
       const v8 w0 = __builtin_bit_cast(v8, make_uint4(o[0], o[1], o[2], o[3])), w1 = __builtin_bit_cast(v8, make_uint4(o[4], o[5], o[6], o[7]));
 #pragma unroll
       for (int k = 0; k < R; ++k) acc[k] = D::mfma(w0, x[b % XD][k][0], acc[k]);
