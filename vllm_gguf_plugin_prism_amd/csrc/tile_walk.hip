@@ -33,17 +33,18 @@ static int walk_any(int type, const WalkCall& c, hipStream_t s) {
 // eight has it for itself) with the panels that a wave walks, which take longer beside other workgroups; the weights, the rows of X, the result.
 // Fitted to 12900 products of random sizes (33 .. 2048 rows, 512 .. 28672 columns, K 512 .. 18944), right to 8 %; the plan chosen by it takes 0.9 %
 // longer than the best.  (panel 0: no such plan.  Q6_K's tiles of 128 rows have no registers left for the sums of a panel, and without those the result is
-// less exact than the other kernels' (1.3e-7 of it against 0.9e-7).)
-struct WalkType { int type; double panel[6], weights[2]; };
+// less exact than the other kernels' (1.3e-7 of it against 0.9e-7).)  moved: formats in blocks of 32 whose rows begin anywhere, as K is no multiple of 256, take longer than that;
+// of 670 such products of 20M weights and more 71 were more than 3 % slower here than by what ran before ([10544,16960] Q8_0 346 rows 256 / 242 us), with these factors 24.
+struct WalkType { int type; double panel[6], weights[2], moved; };
 struct WalkShape { int rt, nw; double base, part, alone, x, y; };
 static const WalkType walk_types[] = {
-      {T_Q4_0, {2.38, 2.29, 3.57, 3.38, 4.78, 6.23}, {0.0582, 0.105}},
-      {T_Q5_0, {2.56, 2.51, 3.47, 3.34, 4.37, 5.39}, {0.0763, 0.142}},
-      {T_Q8_0, {2.15, 2.09, 2.97, 2.8, 3.28, 4.18}, {0.11, 0.175}},
-      {T_Q4_K, {1.84, 1.68, 2.67, 2.48, 3.76, 4.95}, {0.0696, 0.117}},
-      {T_Q5_K, {1.86, 1.74, 2.87, 2.64, 3.96, 5.14}, {0.0766, 0.132}},
-      {T_Q6_K, {3.18, 2.94, 4.77, 4.47, 6.50, 0.0}, {0.094, 0.172}},
-      {T_Q3_K, {2.27, 2.13, 3.14, 2.87, 4.02, 5.05}, {0.062, 0.125}},
+      {T_Q4_0, {2.38, 2.29, 3.57, 3.38, 4.78, 6.23}, {0.0582, 0.105}, 1.05},
+      {T_Q5_0, {2.56, 2.51, 3.47, 3.34, 4.37, 5.39}, {0.0763, 0.142}, 1.07},
+      {T_Q8_0, {2.15, 2.09, 2.97, 2.8, 3.28, 4.18}, {0.11, 0.175}, 1.09},
+      {T_Q4_K, {1.84, 1.68, 2.67, 2.48, 3.76, 4.95}, {0.0696, 0.117}, 1.0},
+      {T_Q5_K, {1.86, 1.74, 2.87, 2.64, 3.96, 5.14}, {0.0766, 0.132}, 1.0},
+      {T_Q6_K, {3.18, 2.94, 4.77, 4.47, 6.50, 0.0}, {0.094, 0.172}, 1.0},
+      {T_Q3_K, {2.27, 2.13, 3.14, 2.87, 4.02, 5.05}, {0.062, 0.125}, 1.0},
 };
 static const WalkShape walk_shapes[] = {
       {1, 4, 5.07, 0.221, 0.612, 1.78, 1.5},
@@ -59,8 +60,8 @@ static double walk_us(const WalkType& t, int shape, int M, int N, int K) {
   const double slots = p.nw == 8 || (t.type == T_Q8_0 && p.rt >= 3 && K % 256 != 0) ? 256.0 : 512.0;
   const int per = ((K + 255) / 256 + p.nw - 1) / p.nw;
   const double r = (double)((M + 32 * p.rt - 1) / (32 * p.rt)) * (double)((N + 31) / 32) / slots;
-  return p.base + (t.panel[shape] * per + p.part) * (p.alone + (1.0 - p.alone) * (r < 1.0 ? r : 1.0)) * 0.5 * (ceil(r) + (r > 1.0 ? r : 1.0)) +
-         1e-6 * (t.weights[p.nw == 8] * N * K + p.x * M * K + p.y * M * N);
+  return (K % 256 != 0 ? t.moved : 1.0) * (p.base + (t.panel[shape] * per + p.part) * (p.alone + (1.0 - p.alone) * (r < 1.0 ? r : 1.0)) * 0.5 * (ceil(r) + (r > 1.0 ? r : 1.0)) +
+         1e-6 * (t.weights[p.nw == 8] * N * K + p.x * M * K + p.y * M * N));
 }
 
 // How long the kernels take that run otherwise, by their own estimates and what 12900 products took of those, by type (mmq_int_us is fitted to the
