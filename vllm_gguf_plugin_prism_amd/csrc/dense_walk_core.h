@@ -10,7 +10,7 @@
 //     registers, three blocks ahead (four tiles of rows: one, where the registers hold no more).
 //   * DIRECT: one tile of rows, taken from X as it lies, without that launch: an instruction touches a line per row, which few enough rows allow (17 rows of [5120,5120] 11.0
 //     instead of 12.6 us; 32 rows of [28672,4096] 42 instead of 33, 64 of [5120,5120] 22.5 instead of 15.7).
-// Measured, us, before / now: IQ4_XS [14336,4096] 12 rows 27.6 / 17.5; [5120,5120] 17 rows 17.5 / 11.0, 128 rows 24.7 / 22, 256 rows 32.4 / 31.6; [4096,4096] 64 rows 19.2 / 11.6; [14336,4096] 64 rows 27.7 / 23; IQ2_XXS
+// Measured, us, before / now: IQ4_XS [14336,4096] 12 rows 27.6 / 17.5; [5120,5120] 17 rows 17.5 / 11.0, 128 rows 24.7 / 22, 256 rows 32.4 / 30.0 to 32.0 by machine; [4096,4096] 64 rows 19.2 / 11.6; [14336,4096] 64 rows 27.7 / 23; IQ2_XXS
 // [4096,5120] 100 rows 25.8 / 15.9.  What bounds it: the decoding (60 to 75 vector instructions a block, again for every tile of rows) and the matrix instructions, which overlap
 // little (tile_walk_core.h), and how the workgroups fill the chip.  Tried and no faster: seven blocks of X ahead.
 // The operands are the ones of dense_kernel, in another order of the fp32 sum: 60 random products, rel-L2 of the half results against 64 bits 2.074e-4 both, results that are
