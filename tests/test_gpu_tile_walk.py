@@ -102,6 +102,36 @@ def test_rows_do_not_meet():
     assert bool(z[40].isnan().all()) and torch.equal(z[:40], y[:40]) and torch.equal(z[41:], y[41:])
 
 
+# A block whose largest value is past 127 times a half's largest has an infinite scale (its sum of the inputs is finite here: the two large ones cancel): the result is an infinity of
+# the sum's sign, no number where the sum is 0.  The rows beside it have the bits that they have without it.
+@pytest.mark.parametrize("qtype,m,n,k,pad,plan", [(q, *s) for q in BLOCKS for s in ((35, 308, 1280, 0, (1, 8)), (135, 3307, 2304, 14, (2, 4)), (332, 2814, 2304, 0, (3, 4)), (591, 2387, 2304, 2, (4, 4)))] + [
+    (q, 35, 301, 512, 2, (1, 4)) for q in GROUPS] + [(o.Q6_K, 142, 1635, 5376, 0, (2, 8)), (o.Q6_K, 202, 4585, 2304, 0, (3, 4)), (o.Q3_K, 202, 4241, 2304, 0, (3, 4)), (o.Q3_K, 296, 4202, 2304, 14, (4, 4))])
+def test_infinite_block_scales(qtype, m, n, k, pad, plan):
+    from vllm_gguf_plugin_prism_amd import ops
+    rng = np.random.default_rng(n)
+    packed = o.make_weights(rng, qtype, n, k)
+    w = torch.zeros(n, packed.shape[1] + pad, dtype=torch.uint8, device="cuda")[:, :packed.shape[1]]
+    w.copy_(torch.from_numpy(packed))
+    assert ops._linear_walk(qtype, n, k, m, w.stride(0)) == plan
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    without = ops.ggml_mul_mat_a8(w, torch.from_numpy(x).cuda(), qtype, n).cpu()
+    places = {0: (0, 0, 17), 2: (k - 32, 3, 30), 5: (k // 64 * 32, 8, 9), 31: (256, 20, 1), m - 1: (k - 64, 31, 5)}   # row: block, places of the large values in it
+    for row, (at, i, j) in places.items():
+        x[row, at + i], x[row, at + j] = 3e9, -3e9
+    got = ops.ggml_mul_mat_a8(w, torch.from_numpy(x).cuda(), qtype, n).cpu()
+    rows = list(places)
+    q, d8, s8 = o.quantize_q8_1(x[rows])
+    wi, ws, _, group = o.unpack(packed, qtype)
+    values = (np.repeat(ws, group, axis=1).astype(np.float64) * wi).reshape(n, k)   # (whole numbers of at most 36 bits times a half: exact)
+    for r, (row, (at, _, _)) in enumerate(places.items()):
+        assert np.isinf(d8[r, at // 32]) and np.isfinite(s8[r, at // 32])
+        sums = values[:, at:at + 32] @ q[r, at:at + 32].astype(np.float64)
+        want = torch.from_numpy(np.where(sums == 0, np.nan, np.copysign(np.inf, sums)))
+        assert torch.equal(got[row].double().nan_to_num(0, 1, -1), want.nan_to_num(0, 1, -1)) and bool((got[row].isnan() == want.isnan()).all())
+    others = [r for r in range(m) if r not in places]
+    assert torch.equal(got[others], without[others])
+
+
 # The kernels behind it at sizes where they still run: those whose estimate is shorter (few panels of many rows, few columns of long ones) ...
 @pytest.mark.parametrize("qtype,m,n,k,route", [(o.Q4_0, 686, 2071, 320, 0), (o.Q4_0, 1782, 386, 256, 4), (o.Q5_0, 925, 552, 256, 0), (o.Q8_0, 1164, 539, 256, 0),
                                                (o.Q4_K, 717, 741, 256, 4), (o.Q4_K, 1007, 369, 9472, 2), (o.Q5_K, 1219, 569, 256, 4), (o.Q5_K, 822, 307, 14592, 2),

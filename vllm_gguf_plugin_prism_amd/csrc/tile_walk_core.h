@@ -101,13 +101,11 @@ __global__ __launch_bounds__(64 * NW, 2) void tile_walk_kernel(const uint8_t* __
   constexpr int PPR = walk_ppr<F>(), SLOT = 512 * PPR, NI = (32 * PPR + 63) / 64, PD = WALK_PD, GS = 32 / F::G, U = 8 * R * GS;   // (the last fetch of a panel: lanes 0 .. 31)
   constexpr int HEAD = walk_head<F>(), XR_AT = SLOT * D, HD_AT = XR_AT + 1024 * PD, SC_AT = HD_AT + HEAD * R, PLACE = walk_place<F, R, D>();
   constexpr bool PART = R <= (F::G == 16 ? 3 : 2) || F::WHOLE;                             // a panel's sum of its own, where the registers hold it
-  constexpr int DB = F::CUT && R >= 3 ? 1 : 2;              // block scales in registers, of this block and, where these suffice, of the next
   constexpr int NL = NI + R;                                // fetches of a panel and of the heads of a panel's rows of X
   static_assert(PD == 8 && 8 * R % PD == 0, "the ring's places are the same in every panel; the waits below count to eight");
   static_assert(PPR % 2 == 1 && walk_lds<F, R, NW, D>() <= 160 * 1024, "the last fetch of a panel is half a fetch; LDS");
   extern __shared__ __align__(16) char smem[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lrow = lane & 31, half = lane >> 5;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // ---- which rows and columns.  Each XCD has a run of tiles, as long as another's; the row blocks of a band follow one another, so that they find
   // their weights in the L2, and a band is as tall as its rows of X fit there.
   const int local = blockIdx.x >> 3, tile = (blockIdx.x & 7) * a.run + local;
@@ -124,21 +122,25 @@ __global__ __launch_bounds__(64 * NW, 2) void tile_walk_kernel(const uint8_t* __
   const uint8_t* const wbase = W - wmis;
   const uint32_t row_bytes = F::KQ ? (uint32_t)(a.np * F::PB) : (uint32_t)(a.nkb * (F::PB / 8));
   const uint32_t last16 = ((uint32_t)(a.N - 1) * a.w_pitch + wmis + row_bytes - 1) & ~15u;   // the last granule that holds bytes of W
-  uint32_t w_at[NI], w_piece[NI];
+  int lane = tid & 63, lrow = lane & 31, half = lane >> 5;
+  const auto w_from = [&](int i, int of) {                  // where row and piece of fetch i begin
+    const int q = min(64 * i + of, 32 * PPR - 1), r = q / PPR;
+    return make_uint2((uint32_t)min(n0 + r, a.N - 1) * a.w_pitch + wmis, 16 * (uint32_t)(q - r * PPR));
+  };
+  uint2 w_at[NI];
 #pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const int q = min(64 * i + lane, 32 * PPR - 1), r = q / PPR;
-    w_at[i] = (uint32_t)min(n0 + r, a.N - 1) * a.w_pitch + wmis;
-    w_piece[i] = 16 * (uint32_t)(q - r * PPR);
-  }
+  for (int i = 0; i < NI; ++i) w_at[i] = w_from(i, lane);
   const char* xt[R];
 #pragma unroll
   for (int k = 0; k < R; ++k) xt[k] = X + (int64_t)min(rb * R + k, a.row_tiles - 1) * a.np * WALK_REC;
-  const auto request_w = [&](int p, int slot) {
+  const auto request_w = [&](int p, int slot, auto safe) {
     const uint32_t to = lds0 + slot * SLOT;
+    int of = lane;
+    if (decltype(safe)::value) asm volatile("" : "+v"(of));   // (formed at each panel: the registers are short)
     walk_units([&](auto at) {
       constexpr int i = decltype(at)::value;
-      const uint32_t v = min(((w_at[i] + (uint32_t)(p * F::PB)) & ~15u) + w_piece[i], last16);
+      const uint2 from = decltype(safe)::value ? w_from(i, of) : w_at[i];
+      const uint32_t v = min(((from.x + (uint32_t)(p * F::PB)) & ~15u) + from.y, last16);
       if constexpr (i < NI - 1) walk_fetch<1024 * i>(v, wbase, to);
       else walk_fetch_half<1024 * i>(v, wbase, to);
     }, std::make_integer_sequence<int, NI>());
@@ -157,24 +159,17 @@ __global__ __launch_bounds__(64 * NW, 2) void tile_walk_kernel(const uint8_t* __
   };
 
   float acc[R][16];
+  v16i seed;
 #pragma unroll
   for (int k = 0; k < R; ++k)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[k][r] = 0.0f;
-  if (wave < a.np) {
-    request_w(wave, 0);
-    request_heads(wave);
-    if (D == 2 && wave + NW < a.np) request_w(wave + NW, 1);
-    walk_units([&](auto x) { request_x(wave, x); }, std::make_integer_sequence<int, PD>());
-  }
-  v16i seed;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) seed[r] = kSeedBits;
-  asm volatile("" : "+v"(seed));                            // (opaque: as constants they are moved into every result's registers)
   float* const scales = (float*)(mine + SC_AT);
 
-  const auto panel = [&](int p, int slot, auto any) {
-    constexpr bool MORE = decltype(any)::value;             // another panel follows
+  // (SAFE: as below, for activations whose block scale may be infinite)
+  const auto panel = [&](int p, int slot, auto any, auto safe) {
+    constexpr bool MORE = decltype(any)::value, SAFE = decltype(safe)::value;   // MORE: another panel follows
+    constexpr int DB = (F::CUT && R >= 3) || SAFE ? 1 : 2;  // block scales in registers, of this block and, where these suffice, of the next
     // This panel, asked for one (D = 2: two) panels ago, and its heads; behind them the tiles under way.
     if (D == 2 && p == wave && MORE) walk_wait<PD + NI>();
     else walk_wait<PD>();
@@ -192,7 +187,7 @@ __global__ __launch_bounds__(64 * NW, 2) void tile_walk_kernel(const uint8_t* __
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // the panel's place may be filled again
     const bool refill = D == 1 ? MORE : MORE && p + 2 * NW < a.np;
     if constexpr (MORE) request_heads(p + NW);
-    if (refill) request_w(p + D * NW, slot);
+    if (refill) request_w(p + D * NW, slot, safe);
     // A unit is a block's group of values and a tile of rows, in the order (block, group, tile).  Tile x of the panel (block x / R, rows x % R) takes the place of tile
     // x - PD as soon as the last unit of that has its operand.  Here unit u, which needs tile x, makes sure that it has landed, before unit `now` has asked for
     // its tile: behind it were asked for all tiles up to that one's and, if it was asked for before this panel began, what was asked for then.
@@ -250,6 +245,7 @@ __global__ __launch_bounds__(64 * NW, 2) void tile_walk_kernel(const uint8_t* __
       asm volatile("" : "+v"(d8));                          // (a float from here on: the compiler would have every multiply-add convert it, in a form that takes twice as long)
       const float nd = -kSeed * d8;
       float (&sum)[16] = PART ? part[PART ? k : 0] : acc[k];
+      const bool over = SAFE && GS == 2 && d8 == __builtin_inff();
       float m8 = 0.0f;
       if constexpr (F::OFF == EIGHTS) {
         const uint32_t sp = b < 2 ? sh[k].x : b < 4 ? sh[k].y : b < 6 ? sh[k].z : sh[k].w;
@@ -260,9 +256,22 @@ __global__ __launch_bounds__(64 * NW, 2) void tile_walk_kernel(const uint8_t* __
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        float v = __builtin_fmaf(__builtin_bit_cast(float, (int)s[u & 1][r]), d8, nd);   // d8 times the block's sum, rounded once
+        const float bits = __builtin_bit_cast(float, (int)s[u & 1][r]);
+        float v = SAFE ? (bits - kSeed) * d8 : __builtin_fmaf(bits, d8, nd);   // d8 times the block's sum, rounded once
+        if constexpr (SAFE && (F::OFF == EIGHTS || F::WHOLE)) asm("" : "+v"(v));   // (a product that is rounded: not half of a multiply-add)
         if constexpr (F::OFF == EIGHTS) v += m8;
-        if constexpr (F::WHOLE) sum[r] = i == 0 ? v : sum[r] + v;
+        if constexpr (SAFE && GS == 2) {                    // (the scale is taken times the sum of both groups, formed in the panel's)
+          static_assert(PART, "a panel has a sum of its own");
+          const float w8 = dw[i % DB][r >> 2][r & 3];
+          float group = (bits - kSeed) * w8;                // (rounded: the two are then equal and opposite where the exact ones are)
+          asm volatile("" : "+v"(group));
+          const float both = sum[r] + group, finite = i == 0 ? v * w8 : __builtin_fmaf(v, w8, sum[r]);
+          if constexpr (i % GS == 0) sum[r] = over ? group : finite;
+          else {
+            acc[k][r] = over ? __builtin_fmaf(both, d8, acc[k][r]) : acc[k][r];
+            sum[r] = over ? 0.0f : finite;
+          }
+        } else if constexpr (F::WHOLE) sum[r] = i == 0 ? v : sum[r] + v;
         else sum[r] = PART && i == 0 ? v * dw[i % DB][r >> 2][r & 3] : __builtin_fmaf(v, dw[i % DB][r >> 2][r & 3], sum[r]);
       }
       // The offsets, a contraction over eight (the upper half of the lanes holds values 8 .. 15, zeros), in the middle of the panel
@@ -289,13 +298,38 @@ __global__ __launch_bounds__(64 * NW, 2) void tile_walk_kernel(const uint8_t* __
     };
     walk_units(unit, std::make_integer_sequence<int, U>());
   };
-  if (wave < a.np) {
+  const auto walk = [&](auto safe) {
+    if (wave >= a.np) return;
+    request_w(wave, 0, safe);
+    request_heads(wave);
+    if (D == 2 && wave + NW < a.np) request_w(wave + NW, 1, safe);
+    walk_units([&](auto x) { request_x(wave, x); }, std::make_integer_sequence<int, PD>());
+#pragma unroll
+    for (int r = 0; r < 16; ++r) seed[r] = kSeedBits;
+    asm volatile("" : "+v"(seed));                          // (opaque: as constants they are moved into every result's registers)
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[k][r] = 0.0f;
     int p = wave, slot = 0;
     for (; p + NW < a.np; p += NW) {
-      panel(p, slot, std::true_type());
+      panel(p, slot, std::true_type(), safe);
       if (D == 2) slot ^= 1;
     }
-    panel(p, slot, std::false_type());
+    panel(p, slot, std::false_type(), safe);
+  };
+  walk(std::false_type());
+  // An activation past 8.3e6 has a block scale that a half does not hold: infinity, which the multiply-add takes from itself, so that none of the row's results is a number (one of
+  // them tells; rows past the last one may be anything).  Its product with the sum is an infinity, of a sum of 0 no number, as in the other kernels: a wave that finds such a
+  // row walks again with the seed taken off first.  The rows beside it get the same bits.  (The test is 0.1 us of 11.)
+  bool none = false;
+#pragma unroll
+  for (int k = 0; k < R; ++k) none |= __builtin_isnan(acc[k][0]) && 32 * (rb * R + k) + lrow < a.M;
+  if (__any(none)) {
+    asm volatile("" : "+v"(lane));                          // (what is formed from it is formed again: kept beside the first walk, it would go to scratch)
+    lrow = lane & 31;
+    half = lane >> 5;
+    walk(std::true_type());
   }
 
   // ---- the waves' partial tiles, added in pairs
@@ -306,7 +340,7 @@ __global__ __launch_bounds__(64 * NW, 2) void tile_walk_kernel(const uint8_t* __
 #pragma unroll
     for (int q = 0; q < 4; ++q) red[((wave * R + k) * 8 + 2 * q + half) * 32 + (lrow ^ (2 * q + half))] = (walk_f4){acc[k][4 * q], acc[k][4 * q + 1], acc[k][4 * q + 2], acc[k][4 * q + 3]};
   __syncthreads();
-  for (int i = tid; i < R * 256; i += 64 * NW) {
+  for (int i = 64 * wave + lane; i < R * 256; i += 64 * NW) {
     const int q = i & 7, row = (i >> 3) & 31, k = i >> 8, m = 32 * (rb * R + k) + row;
     walk_f4 v[NW];
 #pragma unroll
