@@ -219,8 +219,9 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // and types lists their ggml types.  Neighbouring shards of one type whose rows lie next to each other and which take
 // the same path are one matrix with more rows and so one call: q and k of a mixed recipe, [4096 + 1024, 4096] Q4_K,
 // 9.1 -> 5.6 us of kernel time.  The path is that of the shards, each by its own rows, as in the reference's policy, and past
-// 32 rows of X, where launches no longer count, a run keeps to the matrix unit that its largest shard takes by itself;
-// within that, how many workgroups share a sum over K depends on the rows of the whole matrix, so a result may differ from
+// 32 rows of X a run keeps to the matrix unit that its largest shard takes by itself, or both are on the walking tiles
+// (csrc/tile_walk_core.h), whatever stands behind those: 120 such q and k of 33 to 2037 rows took 1.43 times as long shard
+// by shard as they take as one matrix.  Within that, how K is shared depends on the rows of the whole matrix, so a result may differ from
 // the single shard's by the order of a 32-bit sum.  (dispatch.py, _shard_runs, does the same.)
 PyObject* merged_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 6) return PyErr_Format(PyExc_TypeError, "merged_linear takes 6 arguments"), nullptr;
@@ -232,10 +233,12 @@ PyObject* merged_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t m = x->size(0), k = x->size(1);
   const size_t esz = x->element_size();
   struct Part { int64_t start, end, type, rb, largest; Path path; };
-  const auto unit = [&](const Part& p, int64_t rows) {
-    if (m <= 32) return 0;
+  const auto same_unit = [&](const Part& p, int64_t rows, int64_t rows2) {
+    if (m <= 32) return true;
     const int64_t pitch = w->size(0) > 1 ? w->stride(0) : p.rb;
-    return gguf_mmq_layer_unit((int)p.type, rows, k, m, pitch, gguf_mmq_layer_workspace_bytes((int)p.type, rows, k, m, pitch));
+    const int64_t room = gguf_mmq_layer_workspace_bytes((int)p.type, rows, k, m, pitch), room2 = gguf_mmq_layer_workspace_bytes((int)p.type, rows2, k, m, pitch);
+    return gguf_mmq_layer_unit((int)p.type, rows, k, m, pitch, room) == gguf_mmq_layer_unit((int)p.type, rows2, k, m, pitch, room2) ||
+           (gguf_linear_walk((int)p.type, rows, k, m, pitch, room) && gguf_linear_walk((int)p.type, rows2, k, m, pitch, room2));
   };
   std::vector<Part> parts;
   int64_t width = 0;
@@ -257,7 +260,7 @@ PyObject* merged_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
       Part& last = parts.back();
       const int64_t largest = std::max(last.largest, rows);
       if (last.end == p.start && last.type == p.type && last.rb == p.rb && last.path == p.path &&
-          (p.path != PATH_MMQ || unit(p, largest) == unit(p, p.end - last.start))) {
+          (p.path != PATH_MMQ || same_unit(p, largest, p.end - last.start))) {
         last.end = p.end;
         last.largest = largest;
         continue;

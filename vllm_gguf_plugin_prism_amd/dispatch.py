@@ -195,12 +195,15 @@ def apply_linear(x, weight, weight_type: int, *, shard_ids=(), shard_offset_map=
 def _shard_runs(x, weight, shards):
     """Which shards ``(first row, row behind the last, bytes of a row, type)`` of a merged layer are one matrix: neighbours
     of one type and path whose rows touch, as ``(path, shards)``.  The path is that of every shard by its own rows, and
-    past the few rows of X that are bound by launches and weights (32) the run keeps to the matrix unit that its largest
-    shard takes by itself.  gguf_calls.cpp does the same."""
+    past 32 rows of X the run keeps to the matrix unit that its largest shard takes by itself, or both are on the walking
+    tiles.  gguf_calls.cpp does the same."""
     from . import ops
 
-    def unit(t, rows):
-        return x.dim() == 2 and int(x.shape[0]) > 32 and ops._mmq_unit(t, rows, x.shape[1], x.shape[0], weight.stride(0))
+    def same_unit(t, rows, rows2):
+        if x.dim() != 2 or x.shape[0] <= 32:
+            return True
+        sizes = [(t, n, x.shape[1], x.shape[0], weight.stride(0)) for n in (rows, rows2)]
+        return ops._mmq_unit(*sizes[0]) == ops._mmq_unit(*sizes[1]) or all(ops._linear_walk(*s)[0] for s in sizes)
 
     runs = []
     for shard in shards:
@@ -210,7 +213,7 @@ def _shard_runs(x, weight, shards):
             last = runs[-1][1]
             if last[-1][1:] == (start, row_bytes, t):
                 largest = max(b - a for a, b, _, _ in (*last, shard))
-                if path != "mmq" or unit(t, largest) == unit(t, end - last[0][0]):
+                if path != "mmq" or same_unit(t, largest, end - last[0][0]):
                     last.append(shard)
                     continue
         runs.append((path, [shard]))
