@@ -321,7 +321,7 @@ __global__ __launch_bounds__(64 * NW, 2) void tile_walk_kernel(const uint8_t* __
   walk(std::false_type());
   // An activation past 8.3e6 has a block scale that a half does not hold: infinity, which the multiply-add takes from itself, so that none of the row's results is a number (one of
   // them tells; rows past the last one may be anything).  Its product with the sum is an infinity, of a sum of 0 no number, as in the other kernels: a wave that finds such a
-  // row walks again with the seed taken off first.  The rows beside it get the same bits.  (The test is 0.1 us of 11.)
+  // row walks again with the seed taken off first.  The rows beside it get the same bits.  (The test is 0.1 us of 11, the second walk as long as the first and half as long again.)
   bool none = false;
 #pragma unroll
   for (int k = 0; k < R; ++k) none |= __builtin_isnan(acc[k][0]) && 32 * (rb * R + k) + lrow < a.M;
@@ -329,7 +329,15 @@ __global__ __launch_bounds__(64 * NW, 2) void tile_walk_kernel(const uint8_t* __
     asm volatile("" : "+v"(lane));                          // (what is formed from it is formed again: kept beside the first walk, it would go to scratch)
     lrow = lane & 31;
     half = lane >> 5;
-    walk(std::true_type());
+    bool infinite = false;                                  // (else it is an activation or a weight that is no number, and stays that)
+    for (int p = wave; p < a.np; p += NW)
+#pragma unroll
+      for (int k = 0; k < R; ++k) {
+        const uint4 d = *(const uint4*)(xt[k] + ((int64_t)p * WALK_REC + WALK_D_AT) + 16 * lrow);
+        const auto inf = [](uint32_t two) { return (two & 0xFFFFu) == 0x7C00u || two >> 16 == 0x7C00u; };
+        infinite |= (inf(d.x) | inf(d.y) | inf(d.z) | inf(d.w)) && 32 * (rb * R + k) + lrow < a.M;
+      }
+    if (__any(infinite)) walk(std::true_type());
   }
 
   // ---- the waves' partial tiles, added in pairs
