@@ -18,6 +18,13 @@ def test_the_faster_kernel_is_taken(qt, m, n, k, plan):
     assert ops._linear_walk(qt, n, k, m, k // qk * size) == plan
 
 
+# rows of Q8_0 a pitch apart that moves the panels inside 16 bytes, as in a padded merged tensor: LDS then has room for one workgroup of tall tiles (84 / 135 and, on these tiles,
+# 44 / 41; tiles of 96 rows 61)
+@pytest.mark.parametrize("m,n,k,pitch,plan", [(593, 13696, 2304, 2448, (4, 4)), (593, 13696, 2304, 2454, (0, 0)), (356, 2208, 7424, 7890, (2, 4))])
+def test_panels_that_begin_anywhere(m, n, k, pitch, plan):
+    assert ops._linear_walk(Q8_0, n, k, m, pitch) == plan
+
+
 # the records of 33 rows are those of 64: more than the quantized rows, which are the least that a workspace holds
 def test_a_workspace_without_room_is_not_taken():
     L, m, n, k, pitch = _lib.lib(), 33, 4096, 4096, 4096 // 256 * 144

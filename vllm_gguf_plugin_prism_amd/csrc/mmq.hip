@@ -972,7 +972,7 @@ int gguf::mmq_linear_impl(const void* W, int64_t w_row_pitch_bytes, const void* 
   const int64_t partial_room = workspace_bytes - rows_bytes;
   const bool tiles_at_5 = M <= 16 && rows16_direct_pays(type, (int)M, N, K, true) && rows16_direct_takes(W, w_row_pitch_bytes, type, (int)M, (int)N, (int)K, partial_room > 0 ? partial_room : 0);
   if (engine == GGUF_MMQ_AUTO && on16(q8_workspace)) {
-    const WalkPlan p = walk_plan(type, M, N, K, w_row_pitch_bytes, workspace_bytes);
+    const WalkPlan p = walk_plan(type, M, N, K, w_row_pitch_bytes, workspace_bytes, on16(W));
     if (p.rt) return walk_linear(type, W, x, xdtype, q8_workspace, Y, (int)M, (int)N, (int)K, p, la, s);
   }
   // (it fetches the quantized rows in pieces of 16 bytes)

@@ -38,7 +38,7 @@ static inline WalkBands walk_bands(int rt, int64_t M, int64_t N, int64_t K, int 
 
 // Whether a product runs here with a workspace of this size, and how; the workspace that takes; the call
 bool walk_may_take(int type, int64_t M);                    // (a workspace for a call that may be taken has room for its records)
-WalkPlan walk_plan(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, int64_t workspace_bytes);
+WalkPlan walk_plan(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, int64_t workspace_bytes, bool w_on16 = true);   // w_on16: W begins on 16 bytes
 int walk_linear(int type, const void* W, const void* x, int dtype, void* workspace, void* Y, int M, int N, int K, const WalkPlan& p, const LinearArgs& la, hipStream_t s);
 
 }  // namespace gguf

@@ -35,6 +35,9 @@ static int walk_any(int type, const WalkCall& c, hipStream_t s) {
 // longer than the best.  (panel 0: no such plan.  Q6_K's tiles of 128 rows have no registers left for the sums of a panel, and without those the result is
 // less exact than the other kernels' (1.3e-7 of it against 0.9e-7).)  moved: formats in blocks of 32 whose rows begin anywhere, as K is no multiple of 256, take longer than that;
 // of 670 such products of 20M weights and more 71 were more than 3 % slower here than by what ran before ([10544,16960] Q8_0 346 rows 256 / 242 us), with these factors 24.
+// cut: the panels begin anywhere inside 16 bytes, by the address and pitch of W (walk_run_either).  Q8_0 then has no tiles of 96 or 128 rows, for which LDS has room for one workgroup
+// per CU only ([13696,2304] 593 rows, padded, 135 us; by what runs otherwise 84), and where K is a multiple of 256, as in a padded merged tensor, takes that factor too (400 such products 1.22 times as fast as by what ran before, four of them more than 3 % slower, none by 8); the others are estimated well without it (Q4_0, Q5_0,
+// Q4_K, Q5_K: 415 products, five more than 3 % slower, none by 9; with it they would leave 1.1 to 1.2 times).
 struct WalkType { int type; double panel[6], weights[2], moved; };
 struct WalkShape { int rt, nw; double base, part, alone, x, y; };
 static const WalkType walk_types[] = {
@@ -54,13 +57,12 @@ static const WalkShape walk_shapes[] = {
       {3, 4, 5.46, 1.25, 0.641, 1.57, 0.642},
       {4, 4, 5.92, 1.07, 0.636, 1.39, 0.802},
 };
-static double walk_us(const WalkType& t, int shape, int M, int N, int K) {
+static double walk_us(const WalkType& t, int shape, int M, int N, int K, bool cut) {
   const WalkShape& p = walk_shapes[shape];
-  // (Q8_0 whose panels begin anywhere: LDS for one workgroup of tall tiles)
-  const double slots = p.nw == 8 || (t.type == T_Q8_0 && p.rt >= 3 && K % 256 != 0) ? 256.0 : 512.0;
+  const double slots = p.nw == 8 ? 256.0 : 512.0;
   const int per = ((K + 255) / 256 + p.nw - 1) / p.nw;
   const double r = (double)((M + 32 * p.rt - 1) / (32 * p.rt)) * (double)((N + 31) / 32) / slots;
-  return (K % 256 != 0 ? t.moved : 1.0) * (p.base + (t.panel[shape] * per + p.part) * (p.alone + (1.0 - p.alone) * (r < 1.0 ? r : 1.0)) * 0.5 * (ceil(r) + (r > 1.0 ? r : 1.0)) +
+  return (K % 256 != 0 || (t.type == T_Q8_0 && cut) ? t.moved : 1.0) * (p.base + (t.panel[shape] * per + p.part) * (p.alone + (1.0 - p.alone) * (r < 1.0 ? r : 1.0)) * 0.5 * (ceil(r) + (r > 1.0 ? r : 1.0)) +
          1e-6 * (t.weights[p.nw == 8] * N * K + p.x * M * K + p.y * M * N));
 }
 
@@ -86,19 +88,20 @@ bool walk_may_take(int type, int64_t M) {
 // Where it is the faster one by these estimates: over 12900 products of 33 to 2048 rows 1.20 times as fast as what ran before on average (Q6_K 1.12, Q3_K 1.26), 140 of them
 // more than 3 % slower, none by more than 18 %.  us, before / now, quantizer included: [4096,4096] 64 rows Q4_K 16.1 / 10.8, Q8_0 19.4 / 12.6, 128 rows Q4_K 24.9 / 13.2;
 // [14336,4096] Q8_0 77 rows 38.7 / 26.5; but short rows of many columns keep to the others: [25456,512] Q4_K 1501 rows 91 / 137.  (Past 2048 rows: not measured.)
-WalkPlan walk_plan(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, int64_t workspace_bytes) {
+WalkPlan walk_plan(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, int64_t workspace_bytes, bool w_on16) {
   if (!walk_may_take(type, M) || K % block_elems(type) != 0) return {0, 0};
   const int64_t pitch = w_pitch ? w_pitch : K / block_elems(type) * block_bytes(type);
   // (offsets inside the matrix are 32-bit)
   if (N * pitch > 0xFFFF0000ll || walk_rows_bytes(M, K) > workspace_bytes) return {0, 0};
   const WalkType* t = walk_types;
   while (t->type != type) ++t;
+  const bool cut = !w_on16 || pitch % 16 != 0;
   WalkPlan best = {0, 0};
   double least = 1e30;
   for (int i = 0; i < 6; ++i) {
     const WalkShape& p = walk_shapes[i];
-    if (t->panel[i] == 0.0 || (p.rt > 1 && M <= 32 * (p.rt - 1)) || !walk_bands(p.rt, M, N, K).ok) continue;
-    const double us = walk_us(*t, i, (int)M, (int)N, (int)K);
+    if (t->panel[i] == 0.0 || (type == T_Q8_0 && cut && p.rt > 2) || (p.rt > 1 && M <= 32 * (p.rt - 1)) || !walk_bands(p.rt, M, N, K).ok) continue;
+    const double us = walk_us(*t, i, (int)M, (int)N, (int)K, cut);
     if (us < least) { least = us; best = {p.rt, p.nw}; }
   }
   return best.rt && least < 0.94 * walk_others_us(type, (int)M, (int)N, (int)K, pitch, workspace_bytes) ? best : WalkPlan{0, 0};

@@ -391,9 +391,11 @@ static int walk_run(const WalkCall& c, hipStream_t s) {
     case 1 * 16 + 8: return walk_launch<F, 1, 8>(c, s);
     case 2 * 16 + 4: return walk_launch<F, 2, 4>(c, s);
     case 2 * 16 + 8: return walk_launch<F, 2, 8>(c, s);
-    case 3 * 16 + 4: return walk_launch<F, 3, 4>(c, s);
+    case 3 * 16 + 4:
+      if constexpr (F::TALL >= 3) return walk_launch<F, 3, 4>(c, s);   // (else there is no such plan)
+      break;
     case 4 * 16 + 4:
-      if constexpr (F::G == 32) return walk_launch<F, 4, 4>(c, s);   // (else there is no such plan)
+      if constexpr (F::TALL >= 4) return walk_launch<F, 4, 4>(c, s);
   }
   return GGUF_NOT_TAKEN;
 }

@@ -7,6 +7,7 @@
 //   read()   takes the lane's bytes into registers (so that the LDS slot can be filled again); scale_to() leaves the scales for the lanes that
 //            hold the results: [8][32] block scales ([16][32] with G = 16) and, of MINS, [32] -dmin
 //   G        values per weight scale: 32, or 16 (v_mfma_i32_32x32x16_i8 twice per block: the lane's codes of a group are k = 8 half .. 8 half + 7 of it)
+//   TALL     the most tiles of 32 rows that a workgroup has (walk_plan)
 //   WHOLE    the integer scales are in the codes, and the panel has one scale per row: [32] scales
 //   limit()  the panel has only so many blocks; what lies behind them need not be a number (formats of 32-value blocks)
 #pragma once
@@ -19,7 +20,7 @@ enum WalkOffset { NO_OFFSET, MINS, EIGHTS };
 template <bool C>
 struct KQ4_K : WQ4_KT<C> {
   static constexpr bool KQ = true, WHOLE = false;
-  static constexpr int OFF = MINS, G = 32;
+  static constexpr int OFF = MINS, G = 32, TALL = 4;
   using WQ4_KT<C>::h;
   using WQ4_KT<C>::q;
   __device__ __forceinline__ void scale_to(float* to, int row, int half) const {
@@ -63,7 +64,7 @@ struct KQ5_K : KQ4_K<C> {   // Q4_K with a fifth bit, bit b of qh[k] for block b
 template <bool C>
 struct KQ8_0 : W32<34, C> {
   static constexpr bool KQ = false, WHOLE = false;
-  static constexpr int OFF = NO_OFFSET, G = 32;
+  static constexpr int OFF = NO_OFFSET, G = 32, TALL = C ? 2 : 4;
   using W32<34, C>::q;
   __device__ __forceinline__ void read(const char* p, uint32_t at, int half) { this->read_blocks(p, at, 16 * half); }
   __device__ __forceinline__ v4i codes(int b, int) const { return (v4i){(int)q[b].x, (int)q[b].y, (int)q[b].z, (int)q[b].w}; }
@@ -73,7 +74,7 @@ struct KQ8_0 : W32<34, C> {
 template <bool C>
 struct KQ4_0 : W32<18, C> {
   static constexpr bool KQ = false, WHOLE = false;
-  static constexpr int OFF = EIGHTS, G = 32;
+  static constexpr int OFF = EIGHTS, G = 32, TALL = 4;
   using W32<18, C>::q;
   __device__ __forceinline__ void read(const char* p, uint32_t at, int) { this->read_blocks(p, at, 0); }
   __device__ __forceinline__ v4i codes(int b, int half) const {
@@ -89,7 +90,7 @@ template <bool C>
 struct KQ5_0 {
   static constexpr int PB = 176;
   static constexpr bool KQ = false, CUT = C, WHOLE = false;
-  static constexpr int OFF = NO_OFFSET, G = 32;
+  static constexpr int OFF = NO_OFFSET, G = 32, TALL = 4;
   uint4 q[8];
   uint32_t d[4], qh[4];
   __device__ __forceinline__ void limit(int left) {
@@ -126,7 +127,7 @@ struct KQ5_0 {
 // Block b = 4 n + t: low nibbles (t < 2) or high ones of ql[64 n + 32 (t % 2) ..], bits 2 t of qh[32 n ..]; a scale per 16 values.  The code less 32 lies in
 // the top six bits of the byte (four times the value), and the scale is a quarter.
 struct KQ6_K {
-  static constexpr int PB = 210, OFF = NO_OFFSET, G = 16;
+  static constexpr int PB = 210, OFF = NO_OFFSET, G = 16, TALL = 3;
   static constexpr bool KQ = true, CUT = true, WHOLE = false;
   uint2 l[4][2], hi[2][2];                                  // of the lane's eight values of a block's lower and upper half
   uint2 sc;                                                 // the scales of half the blocks
@@ -167,7 +168,7 @@ struct KQ6_K {
 // takes them from two registers.  Block b = 4 n + t: bits 2 t of qs[32 n ..], the third bit, of the other sign, bit b of hmask[k]; scale 2 b + half: four
 // bits of the first eight bytes, two of the last four.
 struct KQ3_K {
-  static constexpr int PB = 110, OFF = NO_OFFSET, G = 32;
+  static constexpr int PB = 110, OFF = NO_OFFSET, G = 32, TALL = 4;
   static constexpr bool KQ = true, CUT = true, WHOLE = true;
   uint4 q[2], hm;
   uint32_t sc[3], d;
