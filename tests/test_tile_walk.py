@@ -12,6 +12,7 @@ Q4_0, Q5_0, Q8_0, Q3_K, Q4_K, Q5_K, Q6_K, Q2_K = 2, 6, 8, 11, 12, 13, 14, 10
     (Q8_0, 77, 14336, 4096, (3, 4)), (Q4_K, 64, 4096, 4096, (1, 8)), (Q4_K, 128, 4096, 4096, (2, 8)), (Q8_0, 64, 4096, 4096, (1, 8)),   # 38.7 / 26.5, 16.1 / 10.8, 24.9 / 13.2, 19.4 / 12.6
     (Q4_K, 1501, 25456, 512, (0, 0)), (Q4_K, 1319, 8368, 512, (0, 0)), (Q2_K, 64, 4096, 4096, (0, 0)),                                  # 91 / 137, 37 / 50, not a format of it
     (Q6_K, 64, 4096, 4096, (1, 8)), (Q6_K, 512, 18944, 3584, (0, 0)), (Q3_K, 512, 14336, 4096, (4, 4)),                                 # 20.4 / 13.6, 184 / 187, 128 / 98
+    (Q6_K, 118, 4400, 3328, (0, 0)), (Q4_K, 143, 3504, 15872, (0, 0)),                                                                  # 25.1 / 30.8, 52.8 / 61.1
     (Q4_K, 32, 4096, 4096, (0, 0)), (Q4_K, 2049, 4096, 4096, (0, 0))])                                                                  # at most 32 rows; not measured
 def test_the_faster_kernel_is_taken(qt, m, n, k, plan):
     qk, size = ops.quant_sizes(qt)

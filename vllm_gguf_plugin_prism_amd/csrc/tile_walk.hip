@@ -62,13 +62,14 @@ static double walk_us(const WalkType& t, int shape, int M, int N, int K, bool cu
   const double slots = p.nw == 8 ? 256.0 : 512.0;
   const int per = ((K + 255) / 256 + p.nw - 1) / p.nw;
   const double r = (double)((M + 32 * p.rt - 1) / (32 * p.rt)) * (double)((N + 31) / 32) / slots;
-  return (K % 256 != 0 || (t.type == T_Q8_0 && cut) ? t.moved : 1.0) * (p.base + (t.panel[shape] * per + p.part) * (p.alone + (1.0 - p.alone) * (r < 1.0 ? r : 1.0)) * 0.5 * (ceil(r) + (r > 1.0 ? r : 1.0)) +
+  const double last = p.nw == 8 ? 0.6 : 0.5, rounds = last * ceil(r) + (1.0 - last) * (r > 1.0 ? r : 1.0);   // (what a round in part costs: alone on a CU, eight waves wait longer)
+  return (K % 256 != 0 || (t.type == T_Q8_0 && cut) ? t.moved : 1.0) * (p.base + (t.panel[shape] * per + p.part) * (p.alone + (1.0 - p.alone) * (r < 1.0 ? r : 1.0)) * rounds +
          1e-6 * (t.weights[p.nw == 8] * N * K + p.x * M * K + p.y * M * N));
 }
 
 // How long the kernels take that run otherwise, by their own estimates and what 12900 products took of those, by type (mmq_int_us is fitted to the
-// K-quants).  The streaming tiles, which small matrices run on, have none: they take 1.14 (Q6_K) to 1.25 times as long (of 2900 products six were slower
-// here by more than a tenth).
+// K-quants).  The streaming tiles, which small matrices run on, have none: they take 1.14 (Q6_K) to 1.25 times as long (of 2691 products 15 were slower here by
+// more than 3 %, eight of those among the 296 of K = 512, which are 1.16 times as fast).
 static double walk_others_us(int type, int M, int N, int K, int64_t w_pitch, int64_t workspace_bytes) {
   if (ts_dense_takes(type, M, N, K, w_pitch)) return 1e30;
   const int64_t int8_rows = (M * q8_row_bytes(K) + 255) / 256 * 256;
@@ -85,8 +86,9 @@ bool walk_may_take(int type, int64_t M) {
   return false;
 }
 
-// Where it is the faster one by these estimates: over 12900 products of 33 to 2048 rows 1.20 times as fast as what ran before on average (Q6_K 1.12, Q3_K 1.26), 140 of them
-// more than 3 % slower, none by more than 18 %.  us, before / now, quantizer included: [4096,4096] 64 rows Q4_K 16.1 / 10.8, Q8_0 19.4 / 12.6, 128 rows Q4_K 24.9 / 13.2;
+// Where it is the faster one by these estimates, by 8 %: over the 12900 products of the fit 1.19 times as fast as what ran before on average (Q6_K 1.12, Q3_K 1.26), 44 of them more
+// than 3 % slower (88 with 6 % and with half the last round counted for eight waves too).  Drawn after the fit, taken ones: 1500 of its ranges 1.23, 13 more than 3 % slower, the
+// worst 0.87; 300 of longer rows (to 57344) or more columns (to 152064) 1.17, eight, 0.89.  us, before / now, quantizer included: [4096,4096] 64 rows Q4_K 16.1 / 10.8, Q8_0 19.4 / 12.6, 128 rows Q4_K 24.9 / 13.2;
 // [14336,4096] Q8_0 77 rows 38.7 / 26.5; but short rows of many columns keep to the others: [25456,512] Q4_K 1501 rows 91 / 137.  (Past 2048 rows: not measured.)
 WalkPlan walk_plan(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, int64_t workspace_bytes, bool w_on16) {
   if (!walk_may_take(type, M) || K % block_elems(type) != 0) return {0, 0};
@@ -104,7 +106,7 @@ WalkPlan walk_plan(int type, int64_t M, int64_t N, int64_t K, int64_t w_pitch, i
     const double us = walk_us(*t, i, (int)M, (int)N, (int)K, cut);
     if (us < least) { least = us; best = {p.rt, p.nw}; }
   }
-  return best.rt && least < 0.94 * walk_others_us(type, (int)M, (int)N, (int)K, pitch, workspace_bytes) ? best : WalkPlan{0, 0};
+  return best.rt && least < 0.92 * walk_others_us(type, (int)M, (int)N, (int)K, pitch, workspace_bytes) ? best : WalkPlan{0, 0};
 }
 
 int walk_linear(int type, const void* W, const void* x, int dtype, void* workspace, void* Y, int M, int N, int K, const WalkPlan& p, const LinearArgs& la, hipStream_t s) {
