@@ -10,14 +10,16 @@ pytestmark = pytest.mark.gpu
 
 DENSE = (o.Q4_0, o.Q4_K, o.Q5_K, o.Q6_K, o.Q2_K, o.Q3_K, o.Q4_1, o.Q5_1)
 ONES = (o.Q4_1, o.Q5_1)
+WALKED = (o.Q4_0, o.Q4_K, o.Q5_K, o.Q6_K, o.Q3_K)   # (the walking tiles take most of their sizes)
 
 
 # one row over a tile of 32 and of 64; a last column tile of one, four, some columns; one panel, K in one part and in
 # several, a part that is longer than another; more tiles than a round of workgroups; rows of W a pitch apart that moves
 # them through the positions inside 16 bytes (whole 16 bytes where only those are taken)
-@pytest.mark.parametrize("qtype", DENSE)
-@pytest.mark.parametrize("m,n,k,pad", [(513, 1025, 256, 0), (577, 1300, 768, 2), (33, 4101, 4096, 0), (513, 2052, 512, 6), (577, 256, 8192, 0),
-                                       (40, 8196, 2048, 0), (97, 25604, 256, 0)])
+@pytest.mark.parametrize("qtype,m,n,k,pad", [(q, *s) for q in DENSE if q not in WALKED for s in (
+    (513, 1025, 256, 0), (577, 1300, 768, 2), (33, 4101, 4096, 0), (513, 2052, 512, 6), (577, 256, 8192, 0), (40, 8196, 2048, 0), (97, 25604, 256, 0))] + [
+    (q, *s) for q in WALKED for s in ((783, 1145, 256, 0), (38, 760, 15872, 2), (581, 106, 9216, 6), (33, 16527, 2304, 0), (97, 25604, 256, 0))] + [
+    (q, 513, 2052, 512, 6) for q in (o.Q4_0, o.Q4_K, o.Q6_K)])
 def test_dense_edges(qtype, m, n, k, pad):
     check_dense(qtype, m, n, k, 8 * pad if qtype in ONES else pad)
 
@@ -39,8 +41,8 @@ def test_two_passes():
 
 # the half-precision unit where it is still the fastest: a row and a column over a tile, tiles cut into runs; whole rounds and a
 # shared rest (the oracle on rows of several tiles)
-@pytest.mark.parametrize("qtype", (o.Q4_K, o.Q5_K, o.Q6_K))
-@pytest.mark.parametrize("m,n,k,pad", [(511, 2177, 8192, 2), (700, 2176, 5120, 0)])
+@pytest.mark.parametrize("qtype,m,n,k,pad", [(q, *s) for q in (o.Q4_K, o.Q5_K) for s in ((2051, 513, 8192, 2), (2100, 2176, 5120, 0))] + [
+    (o.Q6_K, 511, 2177, 8192, 2), (o.Q6_K, 700, 2176, 5120, 0)])
 def test_half_precision_unit_behind_them(qtype, m, n, k, pad):
     check_dense(qtype, m, n, k, pad, np.r_[:3, 250:260, m - 30:m], 2)
 
@@ -51,7 +53,7 @@ def check_dense(qtype, m, n, k, pad, rows=np.s_[:], unit=4):
     w = o.make_weights(rng, qtype, n, k)
     wd = torch.zeros(n, w.shape[1] + pad, dtype=torch.uint8, device="cuda")[:, :w.shape[1]]
     wd.copy_(torch.from_numpy(w))
-    assert ops._mmq_route(qtype, n, k, m, wd.stride(0)) == unit
+    assert ops._mmq_route(qtype, n, k, m, wd.stride(0)) == unit and ops._linear_walk(qtype, n, k, m, wd.stride(0)) == (0, 0)
     x = rng.standard_normal((m, k)).astype(np.float32) + 0.3
     bias = rng.standard_normal(n).astype(np.float32)
     y = ops.ggml_mul_mat_a8(wd, torch.from_numpy(x).cuda(), qtype, n, bias=torch.from_numpy(bias).cuda())
@@ -61,14 +63,14 @@ def check_dense(qtype, m, n, k, pad, rows=np.s_[:], unit=4):
 # 16-bit results in columns of a wider tensor (from an odd one on: single stores): K in parts with a ragged N, in one part, two
 # passes over the rows
 @pytest.mark.parametrize("dt", (torch.float16, torch.bfloat16))
-@pytest.mark.parametrize("qtype,m,n,k,column", [(q, *s) for q in (o.Q4_0, o.Q2_K, o.Q3_K, o.Q4_1, o.Q5_1)
-                                                for s in ((33, 4101, 4096, 3), (577, 1300, 768, 4))] + [(o.Q2_K, 2041, 2052, 3072, 1)])
+@pytest.mark.parametrize("qtype,m,n,k,column", [(q, *s) for q in (o.Q2_K, o.Q4_1, o.Q5_1) for s in ((33, 4101, 4096, 3), (577, 1300, 768, 4))] + [
+    (q, *s) for q in (o.Q4_0, o.Q3_K) for s in ((34, 1010, 12288, 3), (783, 1145, 256, 4))] + [(o.Q2_K, 2041, 2052, 3072, 1)])
 def test_16_bit_results(qtype, m, n, k, column, dt):
     from vllm_gguf_plugin_prism_amd import ops
     rng = np.random.default_rng(n + m)
     rows = np.r_[:33] if m < 2000 else np.r_[:3, 1020:1030, m - 30:m]
     w = o.make_weights(rng, qtype, n, k)
-    assert ops._mmq_route(qtype, n, k, m, w.shape[1]) == 4
+    assert ops._mmq_route(qtype, n, k, m, w.shape[1]) == 4 and ops._linear_walk(qtype, n, k, m, w.shape[1]) == (0, 0)
     x = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).to(dt)
     bias = torch.from_numpy(rng.standard_normal(n).astype(np.float32)).to(dt)
     wide = torch.full((m, column + n + 4), 7.0, dtype=dt, device="cuda")
@@ -80,11 +82,13 @@ def test_16_bit_results(qtype, m, n, k, column, dt):
 
 
 # the largest operands and sums, and scales that are subnormal halves (an offset that is rounded away would be all of it)
-@pytest.mark.parametrize("qtype", DENSE)
-def test_largest_sums_and_smallest_scales(qtype):
+# (the last sizes: the walking tiles)
+@pytest.mark.parametrize("qtype,m,n", [(q, 520, 384) for q in DENSE if q not in WALKED] + [(q, 33, 23472) for q in WALKED] + [(q, 520, 384) for q in WALKED])
+def test_largest_sums_and_smallest_scales(qtype, m, n):
     from vllm_gguf_plugin_prism_amd import ops
     rng = np.random.default_rng(qtype)
-    n, k, m = 384, 512, 520
+    k = 512
+    assert (ops._linear_walk(qtype, n, k, m, k // ops.quant_sizes(qtype)[0] * ops.quant_sizes(qtype)[1]) != (0, 0)) == (qtype in WALKED and m == 520)
     block, size = o.QUANT_SIZES[qtype]
     w = o.make_weights(rng, qtype, n, k).reshape(n, k // block, size)
     if qtype == o.Q6_K:
