@@ -435,7 +435,8 @@ def main() -> int:
                         _timed_ms(call, 20)   # (untimed: whichever engine came first paid 7 % for the clocks coming up)
                     ms = _timed_ms(call, 20, eager=args.profile)
                     tops = 2.0 * m * n * k / (ms * 1e-3) / 1e12
-                    on_half = engine == "half" or (engine == "auto" and ops._mmq_route(Q6_K, n, k, m, k // 256 * 210) in (2, 4))
+                    shape = (Q6_K, n, k, m, k // 256 * 210)
+                    on_half = engine == "half" or (engine == "auto" and not ops._linear_walk(*shape)[0] and ops._mmq_route(*shape) in (2, 4))
                     table[f"{n}x{k}@M{m}"] = {"ms": ms, "TOPS": tops, "unit": "half-precision MFMA" if on_half else "int8 MFMA",
                                               **({"frac_f16_peak": tops / F16_PEAK_TFLOPS} if on_half else
                                                  {"frac_int8_peak": tops / INT8_PEAK_TOPS, "frac_int8_legacy_k_peak": tops / INT8_LEGACY_PEAK_TOPS})}
