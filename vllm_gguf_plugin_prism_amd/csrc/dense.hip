@@ -74,8 +74,9 @@ extern "C" int gguf_dense_linear_takes(int type, int xdtype, int64_t N, int64_t 
   // (offsets inside X are 32-bit, the units of all tiles are counted in an int)
   if (2 * M * K > 0xFFFF0000LL || (M / 64 + 1) * (N / 128 + 1) * (K / 256 + 1) > 0x7FFFFFFFLL) return 0;
   // Where it is faster than a dense copy and a library product, which take about 28 us at least (host), else 12, 0.85 per
-  // million weights and the product at 1.3 PFLOP/s.  Measured, this / those, us: [5120,5120] 17 rows 19 / 35, 128 25 / 43,
-  // 256 33 / 61, 384 43 / 47, 600 61 / 56; [17408,5120] 128 48 / 84, 384 102 / 114, 600 172 / 150; [2048,2048] 256 17 / 27.
+  // million weights and the product at 1.3 PFLOP/s.  Measured, what a call runs (this or dense_walk_core.h) / those, us in a graph, without the
+  // host's time: IQ4_XS [5120,5120] 17 rows 13 / 34, 128 27 / 44, 256 34 / 62; [17408,5120] 128 rows IQ2_XXS 54 / 105, IQ4_XS 61 / 92, 384 118 / 129 and 126 / 115,
+  // 512 IQ2_XXS 138 / 146; IQ1_M [2048,2048] 256 13 / 22.
   double us;
   (void)dense_plan((int)M, (int)N, (int)K, us);
   const double weights = (double)N * K * 1e-6, two = 12.0 + 0.85 * weights + 2.0 * M * weights / 1300.0;

@@ -12,9 +12,9 @@
 // packed bytes fetched a step ahead into registers.  M_T = 256: waves of 64 x 64, one workgroup per CU; 128 and 64: waves
 // of 32 x 64 and 32 x 32 on half the registers, two workgroups per CU, one decoding while the other multiplies.
 //
-// Measured, us per call, this / a dense copy and a library product: IQ4_XS [5120,5120] 17 rows 19 / 35, 64 21 / 37, 256
-// 34 / 61; IQ2_XXS [17408,5120] 64 rows 38 / 79, 256 77 / 105, 512 126 / 139; IQ1_M [2048,2048] 128 rows 14 / 29.  What bounds
-// it at many rows is the fetching of a step, about 1 us behind its request: 16 rows of packed bytes per load instruction
+// Measured, us per call in a graph, this / a dense copy and a library product: IQ4_XS [5120,5120] 64 rows 22.5 / 36.5, [17408,5120] 128
+// 61 / 92, 384 126 / 115; IQ2_XXS [17408,5120] 64 rows 40 / 97, 128 54 / 105, 256 83 / 127, 512 138 / 146.  (Some rows to some hundred of
+// smaller matrices run dense_walk_core.h.)  What bounds it at many rows is the fetching of a step, about 1 us behind its request: 16 rows of packed bytes per load instruction
 // cost the memory pipeline as much as the rows of X do, and neither is asked for more than a step ahead ([5120,5120], 2048
 // rows: 168 us, without the packed bytes' fetch 124, without the decoding 114, matrix instructions and operand reads alone
 // 93).  At few rows it is the decoding and the partial tiles.

@@ -22,8 +22,9 @@
 // workgroup.  Two buffers, one barrier per step.  Whole rounds of tiles have a workgroup per tile; the super-blocks of the
 // tiles behind them are dealt in equal runs to all CUs (192 tiles on 256 CUs: 343 -> 288 us).
 //
-// Measured against the int8 engine, us per call with the quantizer: [4096,14336] Q4_K, 1531 rows 404 -> 288, 512 rows
-// 148 -> 107; [18944,3584] 512 rows 179 -> 139; Q6_K [4096,14336] 1531 rows 462 -> 389, [18944,3584] 512 rows 177 -> 176.
+// Measured against the int8 engine, us per call with the quantizer: [4096,14336] 2100 rows Q4_K 615 -> 410, Q5_K 630 -> 415, 3000 rows Q4_K 834 -> 560; Q6_K
+// [4096,14336] 1531 rows 485 -> 388, [18944,3584] 512 rows 199 -> 164, 1024 rows 369 -> 298.  (Up to 2048 rows Q4_K and Q5_K run tile_walk_core.h mostly: the figures of 1531
+// rows below are those of this kernel, by which it was built.)
 // What bounds it now is vector issue beside the matrix unit, at a clock that falls to about 2.0 GHz under this load: by
 // counters ([4096,14336] Q4_K, 1531 rows) the vector ALU issues in 64 % of the SIMD cycles and the matrix unit is busy in
 // 32 %, Q6_K 52 % and 45 %.  The matrix instructions, the multiply-adds and the operand reads of a step take about 0.45 us
@@ -33,7 +34,8 @@
 // super-block) and the contraction in front of the other wave's decoding the same product takes 299 -> 287 us; Q6_K ([18944,3584], 512 rows) 169 -> 165, once
 // the addresses of the store are formed behind the loop: held over it they put 7 registers of Q5_K and 11 to 14 of Q6_K into scratch (168).  The
 // contraction alone, matrix instructions and multiply-adds in registers, takes a SIMD 50 to 56 ns per 32 x 32 x 32 block at any
-// interleaving (one wave or two, bursts of one to four blocks, 16 x 16 x 32 tiles): the clock falls as they get denser.
+// interleaving (one wave or two, bursts of one to four blocks, 16 x 16 x 32 tiles): the clock falls as they get denser.  Q6_K's, four matrix instructions and 16
+// multiply-adds, takes 82 to 86 ns (16 x 16 x 32: 71): of [18944,3584], 512 rows, 85 to 89 of the 164 us (1036 blocks per SIMD).
 // Tried and slower: four waves per workgroup and two workgroups per CU (decoding twice), the two waves of a SIMD decoding at
 // different times, the fetches of X in front of the operand reads or spread over the step; the barrier in the middle of a step
 // and the next step's operands behind it, so that no step begins with waiting (same bits, 299 -> 316 us, Q6_K 170 -> 190).

@@ -18,7 +18,7 @@
 // Four waves and two workgroups per CU, or eight waves where the output has few columns; R = 1 .. 4, as the rows fill them (walk_us).
 // Measured, us per call with the quantizer, before / now: [4096,4096] 64 rows Q4_K 16.1 / 10.8, Q8_0 19.4 / 12.6, 128 rows Q4_K 24.9 / 13.2; Q8_0 [14336,4096] 77
 // rows 38.7 / 26.5 (its weights take 12.4 from memory), Q6_K [4096,4096] 64 rows 20.4 / 13.6, Q3_K [14336,4096] 512 rows 128 / 98.  Over random products (33 .. 2048
-// rows) of the formats with a scale per 32 values 1.20 times the speed, of Q6_K 1.12, of Q3_K 1.26.
+// rows) of the formats with a scale per 32 values 1.17 to 1.22 times the speed, of Q6_K 1.12, of Q3_K 1.26 (walk_plan).
 // What bounds it: at few rows the beginning and the end of a workgroup (7 us of [4096,4096]'s 8 beside the quantizer); at many the vector instructions and the
 // traffic through LDS, which do not overlap as they might: a block of 32 x 32 x 32 takes a SIMD 100 ns, where its matrix instruction and 32 multiply-adds take
 // 58, the fetches of X and of weights 13 each, the operand reads 9.
@@ -321,7 +321,7 @@ __global__ __launch_bounds__(64 * NW, 2) void tile_walk_kernel(const uint8_t* __
   walk(std::false_type());
   // An activation past 8.3e6 has a block scale that a half does not hold: infinity, which the multiply-add takes from itself, so that none of the row's results is a number (one of
   // them tells; rows past the last one may be anything).  Its product with the sum is an infinity, of a sum of 0 no number, as in the other kernels: a wave that finds such a
-  // row walks again with the seed taken off first.  The rows beside it get the same bits.  (The test is 0.1 us of 11, the second walk as long as the first and half as long again.)
+  // row walks again with the seed taken off first.  The rows beside it get the same bits.  (The test is 0.1 us of 11; a product with such a row takes 1.2 to 1.55 times as long.)
   bool none = false;
 #pragma unroll
   for (int k = 0; k < R; ++k) none |= __builtin_isnan(acc[k][0]) && 32 * (rb * R + k) + lrow < a.M;
