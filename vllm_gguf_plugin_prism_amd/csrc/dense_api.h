@@ -15,7 +15,7 @@
  * half-precision unit's, 0 another.  gguf_linear_dealt: 1 where they are, by tile_dealt_kernel, which comes before all of these (5 .. 32 rows;
  * gemv: of gguf_mmvq_linear), with rows in a workspace that begins on 16 bytes.
  * gguf_linear_walk: where a call of more than 32 rows with a workspace of this size runs tile_walk_kernel, which comes before them too, 16 times the tiles of
- * 32 rows that a workgroup has and its waves, else 0.
+ * 32 rows that a workgroup has and its waves, else 0 (of weights that begin on 16 bytes: others of Q8_0 may run otherwise).
  * gguf_mmq_layer_unit: the kernel of gguf_mmq_layer_route, with 2 added to 1 (past 32 rows) and 4 where the half-precision unit would run a call that these decline.  gguf_moe_mmq_layer_wide: whether
  * gguf_moe_mmq_layer with the workspace it asks for, at addresses divisible by 16, runs on the wide tiles.
  * gguf_moe_mmq_layer_finer: the block of 16 slots from which on the first or second product (product) of a layer on the streaming tiles deals K to
