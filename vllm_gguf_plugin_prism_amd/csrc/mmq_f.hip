@@ -9,7 +9,7 @@ namespace gguf {
 double mmqf_us(int type, int M, int N, int K, int64_t avail) {
   const TilePlan p = mmqf_plan(M, N, K, avail);
   const int nsb = K / 256, rounds = (p.whole + 255) / 256;
-  const double sb = type == T_Q4_K ? 5.85 : type == T_Q5_K ? 6.2 : 8.0;
+  const double sb = type == T_Q4_K ? 5.85 : type == T_Q5_K ? 6.2 : 7.2;
   double us = 6.5 + rounds * (nsb * sb + 8.6) + 1e-6 * M * (0.9 * K + 1.2 * N);
   if (p.shared > 0) us += p.per * sb + (type == T_Q6_K ? 3.8 : 2.2) + 0.036 * (p.workers + p.shared) + 0.23 * nsb / p.per;
   return us;

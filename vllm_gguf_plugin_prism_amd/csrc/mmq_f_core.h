@@ -9,13 +9,15 @@
 // covers 16 values: 41 to 90 ns per 32 x 32 x 32 block and SIMD at full rate, of which the matrix unit needs 14.  Here the
 // integer scale sc goes into the weight operand.  sc * q is a whole number of at most 11 bits (Q4_K 63 * 15, Q5_K
 // 63 * 31), which half precision holds exactly; so are the quants of X; and the block's sum stays below 2^24, so the fp32
-// accumulator of v_mfma_f32_32x32x16_f16 holds it exactly, too, and hands it over as a float.  One multiply-add per result
+// accumulator of v_mfma_f32_16x16x32_f16 holds it exactly, too, and hands it over as a float.  One multiply-add per result
 // and block is left (by d8, which is one register: a lane holds one row of X), and one per result and super-block for d:
-// 34 ns per 32 x 32 x 32 block.  Q6_K's products have 13 bits: two operands, q * (sc & ~15) and q * (sc & 15), 56 ns.
+// 34 ns per 32 x 32 x 32 block.  Q6_K's products have 12 bits and a sign: two operands, the product rounded to half precision and what that
+// leaves out, -1, 0 or 1 and hardly ever not 0: a matrix unit that multiplies zeros draws less, and the clock gives way less ([18944,3584] 512
+// rows 150 us with the operands q * (sc & ~15) and q * (sc & 15), 144 so).
 // The offset term is a contraction over the eight blocks of a super-block of exact halves (the mins are 6-bit whole
 // numbers, the stored sums are halves): one more matrix instruction per super-block.
 //
-// Work split: workgroup tiles of 256 rows of X by 128 weight rows, eight waves of 64 x 64 (four accumulators of 32 x 32,
+// Work split: workgroup tiles of 256 rows of X by 128 weight rows, eight waves of 64 x 64 (sixteen accumulators of 16 x 16,
 // each twice: the super-block's sum and the total).  K in steps of 64: the rows of X (whole numbers in half precision,
 // written by the quantizer) go straight to LDS (global_load_lds, 16-byte pieces, the piece number xored with the row's so
 // that the operand reads meet all banks), the packed weights of the next step through registers, decoded once per
@@ -23,19 +25,21 @@
 // tiles behind them are dealt in equal runs to all CUs (192 tiles on 256 CUs: 343 -> 288 us).
 //
 // Measured against the int8 engine, us per call with the quantizer: [4096,14336] 2100 rows Q4_K 615 -> 410, Q5_K 630 -> 415, 3000 rows Q4_K 834 -> 560; Q6_K
-// [4096,14336] 1531 rows 485 -> 388, [18944,3584] 512 rows 199 -> 164, 1024 rows 369 -> 298.  (Up to 2048 rows Q4_K and Q5_K run tile_walk_core.h mostly: the figures of 1531
+// [4096,14336] 1531 rows 485 -> 355, [18944,3584] 512 rows 199 -> 144, 1024 rows 369 -> 280.  (Up to 2048 rows Q4_K and Q5_K run tile_walk_core.h mostly: the figures of 1531
 // rows below are those of this kernel, by which it was built.)
 // What bounds it now is vector issue beside the matrix unit, at a clock that falls to about 2.0 GHz under this load: by
 // counters ([4096,14336] Q4_K, 1531 rows) the vector ALU issues in 64 % of the SIMD cycles and the matrix unit is busy in
 // 32 %, Q6_K 52 % and 45 %.  The matrix instructions, the multiply-adds and the operand reads of a step take about 0.45 us
-// each; a step takes 1.2 us, a super-block, which is four steps and its end, 5.9 (Q6_K 8.0).  So what is left out counts, not
+// each; a step takes 1.2 us, a super-block, which is four steps and its end, 5.9 (Q6_K 7.2).  So what is left out counts, not
 // what is hidden: with decoding in 30 instead of 50 vector instructions per wave and step (masks and the 1024s as one
 // instruction, high nibbles left where they are), LDS addresses whose constants lie in the instructions (40 additions fewer per
 // super-block) and the contraction in front of the other wave's decoding the same product takes 299 -> 287 us; Q6_K ([18944,3584], 512 rows) 169 -> 165, once
 // the addresses of the store are formed behind the loop: held over it they put 7 registers of Q5_K and 11 to 14 of Q6_K into scratch (168).  The
-// contraction alone, matrix instructions and multiply-adds in registers, takes a SIMD 50 to 56 ns per 32 x 32 x 32 block at any
-// interleaving (one wave or two, bursts of one to four blocks, 16 x 16 x 32 tiles): the clock falls as they get denser.  Q6_K's, four matrix instructions and 16
-// multiply-adds, takes 82 to 86 ns (16 x 16 x 32: 71): of [18944,3584], 512 rows, 85 to 89 of the 164 us (1036 blocks per SIMD).
+// contraction alone, matrix instructions and multiply-adds in registers, takes a SIMD 48 to 56 ns per 32 x 32 x 32 block of one operand at any
+// interleaving (one wave or two, bursts of one to four blocks): vector instructions hide behind matrix instructions only in part, and the clock falls as
+// both get denser.  Of two operands it takes 82 to 86 ns on tiles of 32 x 32 and 71 on tiles of 16 x 16, whose results need half the registers
+// on the way: Q6_K [18944,3584] 512 rows 156 -> 150 us, [4096,14336] 1531 rows 390 -> 374 (Q4_K and Q5_K 0.5 % slower).  A unit's matrix instructions are
+// issued two units ahead of its multiply-adds (one ahead: 155 us, three: no change).
 // Tried and slower: four waves per workgroup and two workgroups per CU (decoding twice), the two waves of a SIMD decoding at
 // different times, the fetches of X in front of the operand reads or spread over the step; the barrier in the middle of a step
 // and the next step's operands behind it, so that no step begins with waiting (same bits, 299 -> 316 us, Q6_K 170 -> 190).
@@ -47,7 +51,6 @@ namespace gguf {
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x2_m __attribute__((ext_vector_type(2)));
 
 // Whole numbers x below 1024 as the halves 1024 + x: the bits `mask` of both halves of v (`magic`, 0x64006400, in a vector register,
@@ -155,31 +158,28 @@ struct FQ6_K {
   static __device__ __forceinline__ float d(const Head& hd) { return (float)__builtin_bit_cast(_Float16, (uint16_t)hd.d); }
   static __device__ __forceinline__ float dmin(const Head&) { return 0.0f; }
   static __device__ __forceinline__ uint4 mins(const Head&) { return make_uint4(0, 0, 0, 0); }
-  // four 6-bit codes -> (code - 32) * (sc & ~15) and (code - 32) * (sc & 15), whole numbers of 10 bits (times 16) and 9 bits
-  static __device__ __forceinline__ void planes(uint32_t v, f16x2 sh, f16x2 sl, uint32_t& h0, uint32_t& h1, uint32_t& l0, uint32_t& l1) {
+  // four 6-bit codes -> (code - 32) * scale rounded to half precision, at most 12 bits, and what that leaves out, -1, 0 or 1
+  static __device__ __forceinline__ void planes(uint32_t v, f16x2 s, uint32_t& h0, uint32_t& h1, uint32_t& l0, uint32_t& l1) {
     const f16x2 k = twice((_Float16)1056.0f);
-    const f16x2 a = magic_bytes<0>(v) - k, b = magic_bytes<1>(v) - k;
-    h0 = bits2(a * sh);
-    h1 = bits2(b * sh);
-    l0 = bits2(a * sl);
-    l1 = bits2(b * sl);
+    const f16x2 a = magic_bytes<0>(v) - k, b = magic_bytes<1>(v) - k, ha = a * s, hb = b * s;
+    h0 = bits2(ha);
+    h1 = bits2(hb);
+    l0 = bits2(__builtin_elementwise_fma(a, s, -ha));
+    l1 = bits2(__builtin_elementwise_fma(b, s, -hb));
   }
   template <int J> static __device__ __forceinline__ void decode(const Raw& r, const Scales&, int p, uint4 (&lo)[2], uint4 (&hi)[2]) {
     // scales of the values of this part: group p / 2 of blocks 2 j and 2 j + 1
     const uint32_t w = r.s >> (8 * (p >> 1));
-    // scale & 15 and, its sign bit flipped and taken off again, scale & ~15
-    const uint32_t c0 = bits2(magic_twice<0>(w)), c1 = bits2(magic_twice<2>(w));
-    const f16x2 k = twice((_Float16)1024.0f), kh = twice((_Float16)1152.0f);
-    const f16x2 sl0 = __builtin_bit_cast(f16x2, c0 & 0x640F640Fu) - k, sh0 = __builtin_bit_cast(f16x2, (c0 ^ 0x00800080u) & 0x64F064F0u) - kh;
-    const f16x2 sl1 = __builtin_bit_cast(f16x2, c1 & 0x640F640Fu) - k, sh1 = __builtin_bit_cast(f16x2, (c1 ^ 0x00800080u) & 0x64F064F0u) - kh;
+    const f16x2 k = twice((_Float16)1152.0f);               // (the sign bit flipped: 1024 + 128 + scale)
+    const f16x2 s0 = __builtin_bit_cast(f16x2, bits2(magic_twice<0>(w)) ^ 0x00800080u) - k, s1 = __builtin_bit_cast(f16x2, bits2(magic_twice<2>(w)) ^ 0x00800080u) - k;
     uint32_t a[2][4], b[2][4];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const uint32_t q0 = i ? r.l0.y : r.l0.x, q1 = i ? r.l1.y : r.l1.x, t = i ? r.h.y : r.h.x;
       const uint32_t v0 = J & 1 ? ((q0 >> 4) & 0x0F0F0F0Fu) | (t & 0x30303030u) : (q0 & 0x0F0F0F0Fu) | ((t << 4) & 0x30303030u);
       const uint32_t v1 = J & 1 ? ((q1 >> 4) & 0x0F0F0F0Fu) | ((t >> 2) & 0x30303030u) : (q1 & 0x0F0F0F0Fu) | ((t << 2) & 0x30303030u);
-      planes(v0, sh0, sl0, a[0][2 * i], a[0][2 * i + 1], a[1][2 * i], a[1][2 * i + 1]);
-      planes(v1, sh1, sl1, b[0][2 * i], b[0][2 * i + 1], b[1][2 * i], b[1][2 * i + 1]);
+      planes(v0, s0, a[0][2 * i], a[0][2 * i + 1], a[1][2 * i], a[1][2 * i + 1]);
+      planes(v1, s1, b[0][2 * i], b[0][2 * i + 1], b[1][2 * i], b[1][2 * i + 1]);
     }
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -195,14 +195,11 @@ struct MmqfArgs {
   uint32_t x_pitch, rows;      // bytes between the rows of X; rows of the planes
 };
 
-// The sixteen values are computed at this point.
-__device__ __forceinline__ void pin16(float (&v)[16]) {
-  asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
-  asm volatile("" : "+v"(v[8]), "+v"(v[9]), "+v"(v[10]), "+v"(v[11]), "+v"(v[12]), "+v"(v[13]), "+v"(v[14]), "+v"(v[15]));
-}
+// The four values are computed at this point.
+__device__ __forceinline__ void pin4(float (&v)[4]) { asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3])); }
 
-// eight waves of TM x TN tiles of 32 x 32
-constexpr int MMQF_WM = 4, MMQF_WN = 2, MMQF_TM = 2, MMQF_TN = 2, MMQF_MT = 32 * MMQF_WM * MMQF_TM, MMQF_NT = 32 * MMQF_WN * MMQF_TN;
+// eight waves of TM x TN tiles of 16 x 16
+constexpr int MMQF_WM = 4, MMQF_WN = 2, MMQF_TM = 4, MMQF_TN = 4, MMQF_MT = 16 * MMQF_WM * MMQF_TM, MMQF_NT = 16 * MMQF_WN * MMQF_TN;
 
 template <class F>
 __host__ __device__ constexpr int mmqf_buffer_bytes() { return 128 * (MMQF_MT + F::PLANES * MMQF_NT); }
@@ -237,7 +234,7 @@ __global__ __launch_bounds__(64 * MMQF_WM * MMQF_WN, 2) void mmqf_kernel(const u
   static_assert(4 * N_T == 64 * NWV && M_T == 256, "a thread per part of a row's step; a fetch per row of block scales");
   extern __shared__ __align__(128) char smem[];             // (rows of 128 bytes, whose pieces are told apart by xor with their addresses)
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / WN, wn = wave % WN, lrow = lane & 31, lhalf = lane >> 5;
+  const int wm = wave / WN, wn = wave % WN, lrow = lane & 15, lgroup = lane >> 4;
 
   const TileWork work = tile_work(a.r);
   const int unit_end = work.end;
@@ -305,36 +302,28 @@ __global__ __launch_bounds__(64 * MMQF_WM * MMQF_WN, 2) void mmqf_kernel(const u
     }
   };
 
-  float acc[TN][TM][16], part_acc[TN][TM][16];
+  float acc[TN][TM][4], part_acc[TN][TM][4];
 #pragma unroll
   for (int i = 0; i < TN; ++i)
 #pragma unroll
     for (int k = 0; k < TM; ++k)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][k][r] = 0.0f;
-  f32x16 zero;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) zero[r] = 0.0f;
+      for (int r = 0; r < 4; ++r) acc[i][k][r] = 0.0f;
+  const tile_f4v zero = {0.0f, 0.0f, 0.0f, 0.0f};
 
-  // ---- one step of K: eight (block, tile pair) units, the matrix instructions of the next unit in front of the scaling
+  // ---- one step of K: 32 units, a block and a pair of tiles each
   const int swz = (lrow >> 1) & 7;                          // (tile bases are multiples of 16 rows)
-  // (the operands of block b, half h are 64 b + 32 h away, by xor: rows are 128 bytes)
-  const uint32_t op0 = 128 * lrow + 16 * (lhalf ^ swz), x_op = lds0 + 128 * 32 * TM * wm, w_op = lds0 + 128 * (M_T + 32 * TN * wn);
-  struct Operands { f16x8 x[TM][2], w[TN][F::PLANES][2]; };
-  const auto load_x = [&](uint32_t at, int b, int k, Operands& o) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) o.x[k][h] = lds_get<f16x8>((at ^ (64 * b + 32 * h)) + 4096 * k);
-  };
+  // (the operands of block b are 64 b away, by xor: rows are 128 bytes)
+  const uint32_t op0 = 128 * lrow + 16 * (lgroup ^ swz), x_op = lds0 + 128 * 16 * TM * wm, w_op = lds0 + 128 * (M_T + 16 * TN * wn);
+  struct Operands { f16x8 x[2][TM], w[TN][F::PLANES]; };
+  const auto load_x = [&](uint32_t at, int b, int k, Operands& o) { o.x[b][k] = lds_get<f16x8>((at ^ (64 * b)) + 2048 * k); };
   const auto load_w = [&](uint32_t at, int b, int i, Operands& o) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int pl = 0; pl < F::PLANES; ++pl) o.w[i][pl][h] = lds_get<f16x8>((at ^ (64 * b + 32 * h)) + (128 * N_T * pl + 4096 * i));
+    for (int pl = 0; pl < F::PLANES; ++pl) o.w[i][pl] = lds_get<f16x8>((at ^ (64 * b)) + (128 * N_T * pl + 2048 * i));
   };
-  // A unit is a block and a pair of tiles, U units per block.  The matrix instructions of unit u + 1 stand between the
-  // multiply-adds of unit u (each waits for the one before it), and an operand's successor is read as soon as the last
-  // instruction that takes it has started.
-  constexpr int U = TM * TN, P = 2 * F::PLANES;
+  // The matrix instructions of unit v + AHEAD stand between the multiply-adds of unit v (each waits for the one before it), and an operand's
+  // successor is read as soon as the last instruction that takes it has started.
+  constexpr int U = TM * TN, P = F::PLANES, AHEAD = 2;
   const auto load_first = [&](int buf, Operands& o) {
     const uint32_t xat = x_op + buf * BUF + afresh(op0), wat = w_op + buf * BUF + afresh(op0);
 #pragma unroll
@@ -344,77 +333,74 @@ __global__ __launch_bounds__(64 * MMQF_WM * MMQF_WN, 2) void mmqf_kernel(const u
   };
   const auto contract = [&](auto step, int buf, int pb, Operands& o) {
     constexpr int J = decltype(step)::value;
-    const uint32_t xd = lds0 + 2 * BUF + 32 * M_T * pb + 128 * TM * wm + 4 * (afresh(lane) & 31), xat = x_op + buf * BUF + afresh(op0), wat = w_op + buf * BUF + afresh(op0);
-    f32x16 s[2];
+    const uint32_t xd = lds0 + 2 * BUF + 32 * M_T * pb + 64 * TM * wm + 4 * (afresh(lane) & 15), xat = x_op + buf * BUF + afresh(op0), wat = w_op + buf * BUF + afresh(op0);
+    tile_f4v s[4];
     float d8[2][TM];
 #pragma unroll
     for (int k = 0; k < TM; ++k) {
-      d8[0][k] = lds_get<float>(xd + (8 * J * M_T + 128 * k));
-      d8[1][k] = lds_get<float>(xd + (8 * J * M_T + 4 * M_T + 128 * k));
+      d8[0][k] = lds_get<float>(xd + (8 * J * M_T + 64 * k));
+      d8[1][k] = lds_get<float>(xd + (8 * J * M_T + 4 * M_T + 64 * k));
     }
-    const auto mfma = [&](int u, int piece, f32x16& v) {
-      const int i = u / TM, k = u % TM, pl = piece >> 1, h = piece & 1;
-      v = __builtin_amdgcn_mfma_f32_32x32x16_f16(o.w[i][pl][h], o.x[k][h], piece == 0 ? zero : v, 0, 0, 0);
+    const auto mfma = [&](int v, int pl) {
+      const int b = v / U, i = v % U / TM, k = v % TM;
+      s[v & 3] = __builtin_amdgcn_mfma_f32_16x16x32_f16(o.w[i][pl], o.x[b][k], pl == 0 ? zero : s[v & 3], 0, 0, 0);
     };
 #pragma unroll
-    for (int piece = 0; piece < P; ++piece) mfma(0, piece, s[0]);
+    for (int v = 0; v < AHEAD; ++v)
+#pragma unroll
+      for (int pl = 0; pl < P; ++pl) mfma(v, pl);
 #pragma unroll
     for (int v = 0; v < 2 * U; ++v) {
-      const int b = v / U, u = v % U, i = u / TM, k = u % TM;
+      const int b = v / U, u = v % U, i = u / TM, k = u % TM, n = v + AHEAD;
 #pragma unroll
-      for (int piece = 0; piece < P; ++piece) {
-        if (v + 1 < 2 * U) mfma((v + 1) % U, piece, s[(v + 1) & 1]);
-        if (piece == P - 1 && v < U) {   // (unit v + 1 of the first block has its operands)
-          const int un = v + 1, in = un / TM, kn = un % TM;
-          if (un < U && kn == TM - 1 && in < TN) load_w(wat, 1, in, o);
-          if (un < U && in == TN - 1) load_x(xat, 1, kn, o);
+      for (int pl = 0; pl < P; ++pl) {
+        if (n < 2 * U) mfma(n, pl);
+        if (pl == P - 1 && n < U) {
+          if (n % TM == TM - 1) load_w(wat, 1, n / TM, o);
+          if (n / TM == TN - 2) load_x(xat, 1, n % TM, o);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int r = 16 / P * piece; r < 16 / P * (piece + 1); ++r)
-          part_acc[i][k][r] = J == 0 && b == 0 ? s[v & 1][r] * d8[b][k] : __builtin_fmaf(s[v & 1][r], d8[b][k], part_acc[i][k][r]);
+        for (int r = 4 / P * pl; r < 4 / P * (pl + 1); ++r)
+          part_acc[i][k][r] = J == 0 && b == 0 ? s[v & 3][r] * d8[b][k] : __builtin_fmaf(s[v & 3][r], d8[b][k], part_acc[i][k][r]);
         __builtin_amdgcn_sched_barrier(0);
       }
       // (here and not later: the compiler would keep the products and scale them all at the end of the super-block)
-      pin16(part_acc[i][k]);
+      pin4(part_acc[i][k]);
     }
   };
   // the end of a super-block
   const auto fold = [&]() {
-    const int ln = afresh(lane), row = ln & 31, half = ln >> 5;
-    const uint32_t at = lds0 + PLANE_AT + 16 * M_T + 4 * (32 * TN * wn + 4 * half);    // d of the lane's first result
+    const int ln = afresh(lane), row = ln & 15, group = ln >> 4;
+    const uint32_t at = lds0 + PLANE_AT + 16 * M_T + 4 * (16 * TN * wn + 4 * group);   // d of the lane's first result
     u32x4_m sv[TM];
     if constexpr (F::OFF)
 #pragma unroll
       for (int k = 0; k < TM; ++k) {
-        // (a contraction over eight: the upper half of the lanes holds values 8 .. 15, zeros beside mins, which are finite)
-        sv[k] = lds_get<u32x4_m>(lds0 + PLANE_AT + 16 * (32 * (TM * wm) + row) + 512 * k);
-        if (half) sv[k] = (u32x4_m){0, 0, 0, 0};
+        // (a contraction over eight: the other lanes hold values 8 .. 31, zeros beside mins, which are finite)
+        sv[k] = lds_get<u32x4_m>(lds0 + PLANE_AT + 16 * (16 * (TM * wm) + row) + 256 * k);
+        if (group) sv[k] = (u32x4_m){0, 0, 0, 0};
       }
 #pragma unroll
     for (int i = 0; i < TN; ++i) {
       __builtin_amdgcn_sched_barrier(0);
-      f32x16 off[F::OFF ? TM : 1];
-      tile_f4v d[4], dm[4];
+      tile_f4v off[F::OFF ? TM : 1], d, dm;
       if constexpr (F::OFF) {
-        const u32x4_m mv = lds_get<u32x4_m>(lds0 + PLANE_AT + 16 * M_T + 8 * N_T + 16 * (32 * TN * wn + row) + 512 * i);
+        const u32x4_m mv = lds_get<u32x4_m>(lds0 + PLANE_AT + 16 * M_T + 8 * N_T + 16 * (16 * TN * wn + row) + 256 * i);
 #pragma unroll
         for (int k = 0; k < TM; ++k)
-          off[k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, mv), __builtin_bit_cast(f16x8, sv[k]), zero, 0, 0, 0);
+          off[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, mv), __builtin_bit_cast(f16x8, sv[k]), zero, 0, 0, 0);
       }
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        d[q] = lds_get<tile_f4v>(at + (128 * i + 32 * q));
-        if (F::OFF) dm[q] = lds_get<tile_f4v>(at + (4 * N_T + 128 * i + 32 * q));
-      }
+      d = lds_get<tile_f4v>(at + 64 * i);
+      if (F::OFF) dm = lds_get<tile_f4v>(at + (4 * N_T + 64 * i));
 #pragma unroll
       for (int k = 0; k < TM; ++k) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          acc[i][k][r] = __builtin_fmaf(part_acc[i][k][r], d[r >> 2][r & 3], acc[i][k][r]);
-          if constexpr (F::OFF) acc[i][k][r] = __builtin_fmaf(off[k][r], dm[r >> 2][r & 3], acc[i][k][r]);
+        for (int r = 0; r < 4; ++r) {
+          acc[i][k][r] = __builtin_fmaf(part_acc[i][k][r], d[r], acc[i][k][r]);
+          if constexpr (F::OFF) acc[i][k][r] = __builtin_fmaf(off[k][r], dm[r], acc[i][k][r]);
         }
-        pin16(acc[i][k]);
+        pin4(acc[i][k]);
       }
     }
   };
@@ -467,22 +453,20 @@ __global__ __launch_bounds__(64 * MMQF_WM * MMQF_WN, 2) void mmqf_kernel(const u
     }
   }
 
-  // ---- store: lane = one row of X, 16 features per tile in runs of four
+  // ---- store: lane = one row of X, four features per tile
   float* const mine = sb1 - sb0 < a.r.units ? partial + (int64_t)(2 * work.worker + segment) * (M_T * N_T) : nullptr;
-  const int ln = afresh(lane);                              // (the places formed from it: not in scratch from before the first tile on)
+  const int ln = afresh(lane), group = ln >> 4;             // (the places formed from it: not in scratch from before the first tile on)
 #pragma unroll
   for (int i = 0; i < TN; ++i)
 #pragma unroll
-    for (int k = 0; k < TM; ++k)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const tile_f4v v = {acc[i][k][4 * q], acc[i][k][4 * q + 1], acc[i][k][4 * q + 2], acc[i][k][4 * q + 3]};
-        if (mine) {   // in the order of the registers: [wave][tile][run][lane] of four
-          *(tile_f4v*)(mine + (((wave * TN * TM + i * TM + k) * 4 + q) * 64 + ln) * 4) = v;
-        } else {
-          tile_store(v, m_base + 32 * (TM * wm + k) + (ln & 31), n_base + 32 * (TN * wn + i) + 8 * q + 4 * (ln >> 5), Y, bias, a.r);
-        }
+    for (int k = 0; k < TM; ++k) {
+      const tile_f4v v = {acc[i][k][0], acc[i][k][1], acc[i][k][2], acc[i][k][3]};
+      if (mine) {   // in the order that tile_reduce_kernel adds: [wave][tile of 32 x 32][run][lane] of four
+        *(tile_f4v*)(mine + (((wave * 4 + (i >> 1) * 2 + (k >> 1)) * 4 + 2 * (i & 1) + (group >> 1)) * 64 + 32 * (group & 1) + 16 * (k & 1) + (ln & 15)) * 4) = v;
+      } else {
+        tile_store(v, m_base + 16 * (TM * wm + k) + (ln & 15), n_base + 16 * (TN * wn + i) + 4 * group, Y, bias, a.r);
       }
+    }
   }
 }
 
@@ -499,7 +483,7 @@ static int mmqf_typed(const MmqfCall& c, hipStream_t stream) {
   hipLaunchKernelGGL(kern, dim3(p.whole + p.workers), dim3(64 * MMQF_WM * MMQF_WN), lds, stream, (const uint8_t*)c.W, (const char*)c.x.x,
                      (const char*)c.x.d, (const char*)c.x.s, (T*)c.Y, c.partial, (const T*)c.la.bias, a);
   if (p.shared > 0)
-    hipLaunchKernelGGL((tile_reduce_kernel<MMQF_WM, MMQF_WN, MMQF_TM, MMQF_TN, T>), dim3(p.shared, MMQF_WM * MMQF_WN * MMQF_TM * MMQF_TN), dim3(256),
+    hipLaunchKernelGGL((tile_reduce_kernel<MMQF_WM, MMQF_WN, MMQF_TM / 2, MMQF_TN / 2, T>), dim3(p.shared, MMQF_WM * MMQF_WN * MMQF_TM * MMQF_TN / 4), dim3(256),
                        0, stream, c.partial, (T*)c.Y, (const T*)c.la.bias, a.r);
   return launch_status();
 }
