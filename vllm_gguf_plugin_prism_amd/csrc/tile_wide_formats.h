@@ -142,10 +142,9 @@ struct WQ6_K {
   }
   __device__ __forceinline__ void operand(int b, int, f16x8 (&o)[2][2]) const {
     const int n = b >> 2, t = b & 3;
-    // 1024 + the scale's byte, twice; its upper half as 128 more than it is
+    // 1024 + 128 + the scale, twice
     const uint32_t c = __builtin_bit_cast(uint32_t, __builtin_amdgcn_perm(0x64646464u, word(sc, b >> 1), b & 1 ? 0x04020402u : 0x04000400u));
-    const f16x2 sl = __builtin_bit_cast(f16x2, c & 0x640F640Fu) - both(1024.0f);
-    const f16x2 sh = __builtin_bit_cast(f16x2, (c ^ 0x00800080u) & 0x64F064F0u) - both(1152.0f);
+    const f16x2 s = __builtin_bit_cast(f16x2, c ^ 0x00800080u) - both(1152.0f);
     const auto codes = [&](int i) {
       const uint32_t a = word(l[2 * n + (t & 1)], i), u = word(hi[n], i);
       return ((t < 2 ? a : a >> 4) & 0x0F0F0F0Fu) | ((t == 0 ? u << 4 : t == 1 ? u << 2 : t == 2 ? u : u >> 2) & 0x30303030u);
@@ -154,8 +153,11 @@ struct WQ6_K {
     for (int i = 0; i < 2; ++i) {
       const uint32_t x = codes(2 * i), y = codes(2 * i + 1);
       const f16x2 k = both(1056.0f), x0 = wide_bytes<0>(x) - k, x1 = wide_bytes<1>(x) - k, y0 = wide_bytes<0>(y) - k, y1 = wide_bytes<1>(y) - k;
-      o[0][i] = wide_operand(x0 * sh, x1 * sh, y0 * sh, y1 * sh);
-      o[1][i] = wide_operand(x0 * sl, x1 * sl, y0 * sl, y1 * sl);
+      // the products rounded to half precision, and what that leaves out: -1, 0 or 1
+      const f16x2 px = x0 * s, qx = x1 * s, py = y0 * s, qy = y1 * s;
+      o[0][i] = wide_operand(px, qx, py, qy);
+      o[1][i] = wide_operand(__builtin_elementwise_fma(x0, s, -px), __builtin_elementwise_fma(x1, s, -qx), __builtin_elementwise_fma(y0, s, -py),
+                             __builtin_elementwise_fma(y1, s, -qy));
     }
   }
 };
