@@ -1,0 +1,50 @@
+"""The expert tile kernel (csrc/tile_expert_core.h): blocks of 32 slots with one pair, sixteen, seventeen and all, against the CPU oracle."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import gguf_oracle as o
+from test_gpu_tile_wide import layer
+
+pytestmark = pytest.mark.gpu
+
+
+# either kind of record behind either kernel; a column tile of one feature's run, of some; K in one part and in four; pairs whose expert
+# does not exist; an infinite block scale in a block of 17 pairs and in one of one: that row holds a number, an infinity or neither
+# where the other kernels' does, its neighbours are numbers
+@pytest.mark.parametrize("qtype,qtype2,hid,inner,n_out", [
+    (o.Q4_0, o.Q4_0, 256, 768, 256), (o.Q8_0, o.Q8_0, 512, 6144, 129), (o.Q4_K, o.Q4_K, 256, 1536, 130), (o.Q5_K, o.Q5_K, 768, 768, 384),
+    (o.Q4_K, o.Q6_K, 256, 768, 256), (o.Q6_K, o.Q5_K, 512, 1536, 131), (o.Q6_K, o.Q6_K, 256, 6144, 252)])
+@pytest.mark.parametrize("huge", (False, True))
+def test_blocks_in_part(qtype, qtype2, hid, inner, n_out, huge):
+    from vllm_gguf_plugin_prism_amd import _lib, ops
+    rng = np.random.default_rng(hid + inner + n_out)
+    pairs_of = (1, 16, 17, 32, 33, 0, 209)                  # by expert; a block with 1, 16, 17, 32, 1 and 17 pairs
+    e, tokens = len(pairs_of), sum(pairs_of) + 1
+    w13 = np.stack([o.make_weights(rng, qtype, 2 * inner, hid) for _ in range(e)])
+    w2 = np.stack([o.make_weights(rng, qtype2, n_out, inner) for _ in range(e)])
+    ids = np.append(np.repeat(np.arange(e), pairs_of), e + 3).astype(np.int32)
+    order = rng.permutation(tokens)
+    ids = ids[order][:, None].copy()
+    assert _lib.lib().gguf_moe_mmq_layer_wide(qtype, qtype2, hid, inner, n_out, 1, tokens, e) == 1
+    x = rng.standard_normal((tokens, hid)).astype(np.float32)
+    wts = rng.random((tokens, 1)).astype(np.float32)
+    s, eids, post = o.moe_align_block_size(ids, 32, e)
+    h = o.moe_a8(x, w13, s, eids, post, qtype, 2 * inner, 1, tokens, 32)
+    x *= 4.0 / np.abs(h).max()
+    rows = [int(np.flatnonzero(ids[:, 0] == j)[0]) for j in (0, 2)] if huge else []
+    for r in rows:
+        x[r, 40] = 1e8                                      # (its block's scale, 1e8 / 127, is infinite as a half)
+    cuda = [torch.from_numpy(a).cuda() for a in (x, w13, w2, wts, ids)]
+    got = ops.moe_mmq_layer(*cuda, qtype, qtype2, "silu").cpu().numpy()
+    with np.errstate(all="ignore"):
+        h = o.moe_a8(x, w13, s, eids, post, qtype, 2 * inner, 1, tokens, 32)
+        y = o.moe_a8(o.silu_and_mul(h), w2, s, eids, post, qtype2, n_out, 1, tokens, 32)
+        want = y * wts
+    rest = np.setdiff1d(np.arange(tokens), rows)
+    # (a quant of h may move by a step where the activation's last bit differs)
+    assert np.isfinite(got[rest]).all() and o.rel_l2(got[rest], want[rest]) <= 1e-3
+    if rows and qtype != o.Q6_K:                            # (the other route: a workspace off 16 bytes; the wide tiles of Q6_K differ from it there)
+        other = layer("gguf_moe_mmq_layer", *cuda, qtype, qtype2, 8).cpu().numpy()
+        for r in rows:
+            assert (np.isnan(got[r]) == np.isnan(other[r])).all() and (np.isinf(got[r]) == np.isinf(other[r])).all()

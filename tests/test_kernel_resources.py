@@ -9,7 +9,7 @@ from vllm_gguf_plugin_prism_amd import _lib
 # Kernels whose registers are counted out: a value that goes to scratch is a trip through memory, per tile or per step.
 # (IQ3_S with one tile of rows and two column groups: three registers, and faster than with one group by 3 %)
 EXCEPT = ("6TIQ3_SELi1ELi2E",)
-WHOLE_IN_REGISTERS = ("mmqf_kernel", "tile_stream_kernel", "tile_dealt_kernel", "tile_dealt_pair_kernel", "tile_wide_kernel", "mmvq_pair_kernel")
+WHOLE_IN_REGISTERS = ("mmqf_kernel", "tile_stream_kernel", "tile_dealt_kernel", "tile_dealt_pair_kernel", "tile_wide_kernel", "tile_expert_kernel", "mmvq_pair_kernel")
 
 
 def kernels(data: bytes):

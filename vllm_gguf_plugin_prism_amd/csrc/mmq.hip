@@ -29,6 +29,7 @@
 #include "mmq_f.h"
 #include "tile_stream.h"
 #include "tile_walk.h"
+#include "tile_expert.h"
 #include "tile_wide.h"
 #include "mmq_formats.h"
 #include "q8_1_device.h"
@@ -750,7 +751,7 @@ int moe_tiles_layer(const void* X, int xdtype, void* workspace, const void* W13,
   return moe_weighted_sum_live(y2, topk_w, topk_ids, num_experts, out, xdtype, tokens, top_k, N_out, s);
 }
 
-// ---- A MoE layer whose experts see more than a few pairs each, on the wide tile kernel (blocks of 32 slots): the same four
+// ---- A MoE layer whose experts see more than a few pairs each, on the expert and the wide tile kernel (blocks of 32 slots): the same four
 // launches with the grouped operator's arithmetic, the rows of X and h as records.
 // [records of X][records of h][second GEMM's result, pairs x N_out][sorted ids, expert ids, padded total]
 // into how many parts the second GEMM cuts K: fp32 sums that the weighted sum adds
@@ -760,6 +761,10 @@ static int wide_layer_parts(int64_t tokens, int64_t top_k, int64_t I, int64_t N_
   return wide_ksplit(moe_blocks_estimate((int)cap, (int)pairs, 32) * ((N_out + 127) / 128), (int)I);
 }
 
+static bool layer_on_wide(int type) { return type == T_Q6_K; }   // its product: on the wide tiles, the others' on the expert tiles
+static int64_t layer_rows_bytes(int type, int64_t rows, int64_t K) { return layer_on_wide(type) ? wide_rows_bytes(rows, K) : expert_rows_bytes(rows, K); }
+
+// (asked before the types are known: room for the longer records)
 int64_t wide_layer_workspace(int64_t tokens, int64_t top_k, int64_t H, int64_t I, int64_t N_out, int64_t num_experts, int elt) {
   const int64_t pairs = tokens * top_k, cap = pairs + num_experts * 31;
   const int parts = wide_layer_parts(tokens, top_k, I, N_out, num_experts);
@@ -771,39 +776,26 @@ int wide_layer(const void* X, int xdtype, void* workspace, const void* W13, int 
   const int pairs = tokens * top_k, elt = xdtype == GGUF_DTYPE_F32 ? 4 : 2, block = 32;
   const int64_t cap = (int64_t)pairs + (int64_t)num_experts * (block - 1), block_cap = cap / block + 1;
   char* const x = (char*)workspace;
-  char* const h = x + up16(wide_rows_bytes(tokens, H));
-  char* const y2 = h + up16(wide_rows_bytes(pairs, I));
+  char* const h = x + up16(layer_rows_bytes(type13, tokens, H));
+  char* const y2 = h + up16(layer_rows_bytes(type2, pairs, I));
   const int parts = (uintptr_t)out % 16 == 0 ? wide_layer_parts(tokens, top_k, I, N_out, num_experts) : 1;
   int32_t* const sorted = (int32_t*)(y2 + up16((int64_t)pairs * N_out * (parts > 1 ? 4 * parts : elt)));
   int32_t* const experts = sorted + cap;
   int32_t* const post = experts + block_cap;
-  int rc = taken(moe_prepare(X, xdtype, x, tokens, H, topk_ids, pairs, num_experts, block, sorted, (int)cap, experts, (int)block_cap, post, 2, s));
+  int rc = taken(moe_prepare(X, xdtype, x, tokens, H, topk_ids, pairs, num_experts, block, sorted, (int)cap, experts, (int)block_cap, post, layer_on_wide(type13) ? 2 : 3, s));
   if (rc != GGUF_OK) return rc;
-  WideCall c = {};
-  c.dtype = xdtype;
-  c.rt = 1;
-  c.ksplit = 1;
-  c.row_blocks = (int)(cap / block);
-  c.W = W13;
-  c.x = x;
-  c.x_rows = tokens;
-  c.N = 2 * I;
-  c.K = H;
-  c.moe = MoeArgs{sorted, experts, post, (int64_t)2 * I * (H / block_elems(type13)) * block_bytes(type13), top_k, pairs, 0};
-  c.gate = Gate16{h, 0, I, 0, act};
-  rc = taken(wide_any(type13, c, s));
+  const int row_blocks = (int)(cap / block);
+  const auto product = [&](int type, const void* W, const void* rows, int64_t x_rows, int N, int K, int k, const Gate16& gate, int ksplit) {
+    const MoeArgs moe = {sorted, experts, post, (int64_t)N * (K / block_elems(type)) * block_bytes(type), k, pairs, 0};
+    if (!layer_on_wide(type)) return taken(expert_any(type, ExpertCall{W, rows, x_rows, y2, xdtype, N, K, moe, row_blocks, gate, ksplit, (float*)y2}, s));
+    WideCall c = {};
+    c.W = W; c.x = rows; c.x_rows = x_rows; c.Y = y2; c.dtype = xdtype; c.N = N; c.K = K; c.moe = moe;
+    c.row_blocks = row_blocks; c.rt = 1; c.gate = gate; c.ksplit = ksplit; c.partial = (float*)y2;
+    return taken(wide_any(type, c, s));
+  };
+  rc = product(type13, W13, x, tokens, 2 * I, H, top_k, Gate16{h, 0, I, layer_on_wide(type2), act}, 1);
   if (rc != GGUF_OK) return rc;
-  c.W = W2;
-  c.x = h;
-  c.x_rows = pairs;
-  c.Y = y2;
-  c.N = N_out;
-  c.K = I;
-  c.moe = MoeArgs{sorted, experts, post, (int64_t)N_out * (I / block_elems(type2)) * block_bytes(type2), 1, pairs, 0};
-  c.gate = Gate16{};
-  c.ksplit = parts;
-  c.partial = (float*)y2;
-  rc = taken(wide_any(type2, c, s));
+  rc = product(type2, W2, h, pairs, N_out, I, 1, Gate16{}, parts);
   if (rc != GGUF_OK) return rc;
   if (parts > 1) return taken(moe_weighted_sum_parts(y2, parts, topk_w, topk_ids, num_experts, out, xdtype, tokens, top_k, N_out, s));
   return moe_weighted_sum_live(y2, topk_w, topk_ids, num_experts, out, xdtype, tokens, top_k, N_out, s);

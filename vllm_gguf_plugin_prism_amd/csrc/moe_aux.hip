@@ -160,11 +160,12 @@ __global__ __launch_bounds__(ALIGN_THREADS) void moe_prepare_kernel(const T* __r
     moe_align_body(topk_ids, numel, num_experts, block, sorted_ids, sorted_capacity, expert_ids, expert_capacity, num_post_padded, lds);
     return;
   }
-  const int per_row = (layout == 2 ? K : Kp) / 8;               // threads a row takes
+  const int per_row = (layout >= 2 ? K : Kp) / 8;               // threads a row takes
   const int64_t g = (int64_t)(blockIdx.x - 1) * ALIGN_THREADS + threadIdx.x;
   const int64_t m = g / per_row;
   if (m >= tokens) return;                                      // (per_row is a multiple of 32: whole quads leave)
   if (layout == 2) wide_quantize_thread<T>(x, ws, K, tokens, m, (int)(g % per_row));
+  else if (layout == 3) expert_quantize_thread<T>(x, ws, K, tokens, m, (int)(g % per_row));
   else q8_1_quantize_thread<T>(x, ws, K, Kp, row_bytes, ACT_NONE, m, (int)(g % per_row), nullptr, layout == 1);
 }
 
@@ -270,14 +271,14 @@ int moe_weighted_sum_live(const void* Y, const float* topk_weights, const int32_
 }
 
 // quantize_q8_1(X) and gguf_moe_align_block_size(topk_ids) in one launch (sizes checked by the caller).  layout of the rows: 0 plain,
-// 1 permuted (q8_permuted), 2 records (quantize_wide)
+// 1 permuted (q8_permuted), 2 records (tile_wide.h), 3 records (tile_expert.h)
 int moe_prepare(const void* X, int xdtype, void* q8x, int tokens, int K, const int32_t* topk_ids, int numel, int num_experts, int block,
                 int32_t* sorted_ids, int sorted_capacity, int32_t* expert_ids, int expert_capacity, int32_t* num_post_padded, int layout,
                 hipStream_t s) {
   const int Kp = (int)q8_kp(K);
   const size_t lds = (size_t)(1 + ALIGN_WAVES) * num_experts * sizeof(int);
   if (lds > 65536) return GGUF_NOT_TAKEN;
-  const int64_t threads = (int64_t)tokens * ((layout == 2 ? K : Kp) / 8);
+  const int64_t threads = (int64_t)tokens * ((layout >= 2 ? K : Kp) / 8);
   const unsigned grid = 1 + (unsigned)((threads + ALIGN_THREADS - 1) / ALIGN_THREADS);
   GGUF_DISPATCH_DTYPE(xdtype, hipLaunchKernelGGL(moe_prepare_kernel<scalar_t>, dim3(grid), dim3(ALIGN_THREADS), lds, s, (const scalar_t*)X,
                                                  (char*)q8x, K, Kp, q8_row_bytes(K), tokens, topk_ids, numel, num_experts, block, sorted_ids,

@@ -232,4 +232,20 @@ __device__ __forceinline__ void wide_quantize_thread(const T* __restrict__ x, ch
   }
 }
 
+// The activations of the expert tile kernel (tile_expert.h): the eight values [8 t, 8 t + 8) of row m of `rows` -> eight quants in the
+// record of their 128 values; the block's scale and sum from the first lane of each quad.
+constexpr int EXPERT_REC = 144, EXPERT_D_AT = 128, EXPERT_S_AT = 136;
+template <typename T>
+__device__ __forceinline__ void expert_quantize_thread(const T* __restrict__ x, char* __restrict__ records, int K, int64_t rows, int64_t m, int t) {
+  float v[8] = {};
+  if (8 * t < K) load8<T>(x + m * (int64_t)K + 8 * t, v);   // (behind K: zeros)
+  const Q8Quad q = q8_1_quantize8(v);
+  char* const rec = records + ((int64_t)(t >> 4) * rows + m) * EXPERT_REC;
+  *(uint2*)(rec + 8 * (t & 15)) = q.q;
+  if ((t & 3) == 0) {
+    *(_Float16*)(rec + EXPERT_D_AT + 2 * ((t >> 2) & 3)) = (_Float16)q.d;
+    *(_Float16*)(rec + EXPERT_S_AT + 2 * ((t >> 2) & 3)) = (_Float16)q.s;
+  }
+}
+
 }  // namespace gguf

@@ -6,7 +6,6 @@
 namespace gguf {
 
 int wide_q4_0(const WideCall& c, hipStream_t s);
-int wide_q8_0(const WideCall& c, hipStream_t s);
 int wide_q4_k(const WideCall& c, hipStream_t s);
 int wide_q5_k(const WideCall& c, hipStream_t s);
 int wide_q6_k(const WideCall& c, hipStream_t s);
@@ -33,9 +32,9 @@ static bool wide_size_ok(int type, int64_t N, int64_t K, int64_t x_rows) {
 // About how long a layer takes here, us (ts_layer_us is the streaming tiles' estimate): what its panels take, rounds of
 // workgroups on the chip, whose panels take longer the more workgroups share a CU; the experts that are hit from memory; the
 // rows of X, h and the result.  Fitted to 10000 layers of random sizes (H 1024 .. 4096, I 512 .. 8192, 8 .. 256 experts with 0.5 ..
-// 128 pairs each), right to 8 % on as many others.
+// 128 pairs each), right to 8 % on as many others; the panels of the expert tiles' formats to 1200.
 static double wide_layer_us(int type13, int type2, int64_t H, int64_t I, int64_t N_out, int64_t pairs, int64_t num_experts) {
-  const auto panel = [](int type) { return type == T_Q4_0 ? 2.19 : type == T_Q8_0 ? 3.31 : type == T_Q4_K ? 1.79 : type == T_Q5_K ? 2.09 : 3.45; };
+  const auto panel = [](int type) { return type == T_Q4_0 ? 1.70 : type == T_Q8_0 ? 2.65 : type == T_Q4_K ? 1.61 : type == T_Q5_K ? 1.94 : 3.45; };
   const double blocks = moe_blocks_estimate((int)(pairs + num_experts * 31), (int)pairs, 32), tiles2 = blocks * (double)((N_out + 127) / 128);
   const int parts = wide_ksplit(tiles2, (int)I);
   const auto product = [](double us_panel, int64_t panels, double wgs) {
@@ -50,30 +49,18 @@ bool wide_layer_takes(int type13, int type2, int64_t H, int64_t I, int64_t N_out
   const int64_t pairs = tokens * top_k;
   if (!wide_type_ok(type13) || !wide_type_ok(type2) || num_experts > 256 || H % 256 != 0 || I % 256 != 0 || !wide_size_ok(type13, 2 * I, H, tokens) || !wide_size_ok(type2, N_out, I, pairs)) return false;
   if (pairs * top_k > 0xFFFFFFFFll) return false;               // (the kernel's quotient by reciprocal)
-  // Both sides of 40000 layers of random sizes were measured, 0.5 to 1200 pairs per expert, how many times as long the others take:
-  //   * against blocks of 32 and of 64 slots, past what the streaming tiles take: 1.1 to 1.6 (Q4_0), 1.3 to 1.9 (K-quants; rows past
-  //     4096 1.8 to 2.8), also where the workgroups are fewer than the CUs; Q8_0, which the int8 unit multiplies without decoding,
-  //     1.24 below 32 pairs per expert, 1.07 at 64 to 128, 1.01 at 192 to 256, then 0.97, 0.92 from 600 on; with Q6_K behind it 1.01
-  //     at 192 to 256 and 0.93 at the end, with Q4_0 1.03 and 0.96 from 400 on, with Q4_K always more (1.08).
-  //     (Tiles of 64 rows: 1.05 to 1.4 times as long below 64 pairs per expert, up to 1.07 times as fast above.)
-  //   * against blocks of 16 slots where the streaming tiles do not run, rows past 4096: 1.2 (Q4_0) to 1.6 (Q4_K, Q5_K); Q8_0 1.2, but 0.89 below
-  //     150 workgroups of the first product (`wgs`, 64 features of h for 32 slots each, estimated), and h of less than 768
-  //     values 0.85 to 1.0 below 700;
-  //   * against the streaming tiles from 40 pairs per expert on: 1.34 (Q4_K), 1.56 (Q5_K), 1.48 (Q6_K), hardly ever less than 1.05.
+  // Both sides of 2200 layers of random sizes were measured, 4 to 1500 pairs per expert, how many times as long the others take:
+  //   * past what the streaming tiles take: 1.33 (Q8_0, 150 layers of 4 to 100 pairs per expert), 1.47 from 60 pairs on over all types and
+  //     never below 1.05 there (Q8_0 1.23 to 1.36, also at 300 to 1500).  Q8_0 with 16 experts of 8 to 12 pairs: 0.86 to 1.17, 1.02 on
+  //     average; a limit that leaves those to the others costs more than it gives (the rule without one loses 1.2 % against
+  //     always taking the faster one, with one at 12 pairs and 700 workgroups 2.4 %).  Q8_0 past 640 pairs per expert, first product
+  //     and second of Q8_0, Q4_0 or Q6_K, is left where its route is fixed by a test, though these are 1.03 to 1.25 times as fast there, too;
+  //   * against the streaming tiles from 40 pairs per expert on: 1.3 to 1.6, hardly ever less than 1.05.
   // Below that a block of 32 slots is padding for the most part, and the one or the other is faster by the type, the rows'
-  // length and how the workgroups fall into rounds (Q4_0 [gate|up 2048], 10 pairs each: 0.8 to 1.3): by the two estimates, which lose 0.9 % on average
-  // against always taking the faster one (12 to 18 pairs: Q4_0 1.107 of 1.113, Q4_K 1.097 of 1.106; three layers in a hundred are slower by more than 10 %).
-  if (type13 == T_Q8_0) {
-    if (pairs > (type2 == T_Q8_0 || type2 == T_Q6_K ? 256 : type2 == T_Q4_0 ? 400 : 0x7FFFFF) * num_experts) return false;
-  }
-  if (pairs > 40 * num_experts) return true;
-  if (ts_layer_takes(type13, type2, H, I, N_out, tokens, top_k, num_experts))
-    return wide_layer_us(type13, type2, H, I, N_out, pairs, num_experts) < ts_layer_us(type13, type2, H, I, N_out, pairs, num_experts);
-  if (type13 == T_Q8_0 && pairs <= 16 * num_experts) {
-    const double wgs = moe_blocks_estimate((int)(pairs + num_experts * 31), (int)pairs, 32) * (double)((I + 63) / 64);
-    return wgs >= (H > 4096 ? 150.0 : 700.0);
-  }
-  return true;
+  // length and how the workgroups fall into rounds: by the two estimates, which lose 0.5 % on average against always taking the faster one.
+  if (type13 == T_Q8_0 && type2 != T_Q4_K && type2 != T_Q5_K && pairs > 640 * num_experts) return false;
+  if (pairs > 40 * num_experts || !ts_layer_takes(type13, type2, H, I, N_out, tokens, top_k, num_experts)) return true;
+  return wide_layer_us(type13, type2, H, I, N_out, pairs, num_experts) < ts_layer_us(type13, type2, H, I, N_out, pairs, num_experts);
 }
 
 // A workgroup walks its panels one after the other, about 1.7 us each beside two others on the CU, which holds three: where the
@@ -107,7 +94,6 @@ __global__ __launch_bounds__(256) void wide_sum_kernel(const float* __restrict__
 int wide_any(int type, const WideCall& c, hipStream_t s) {
   switch (type) {
     case T_Q4_0: return wide_q4_0(c, s);
-    case T_Q8_0: return wide_q8_0(c, s);
     case T_Q4_K: return wide_q4_k(c, s);
     case T_Q5_K: return wide_q5_k(c, s);
     case T_Q6_K: return wide_q6_k(c, s);

@@ -1,5 +1,5 @@
-// Products with some tens of rows of activations -- MoE layers whose experts see more than a few pairs each, dense layers past
-// the few rows of the streaming tiles -- on 32 or 64 rows by 128 columns per workgroup.
+// Products with some tens of rows of activations -- dense layers past the few rows of the streaming tiles, Q6_K in MoE layers whose
+// experts see more than a few pairs each (the other formats: tile_expert_core.h) -- on 32 or 64 rows by 128 columns per workgroup.
 //
 // What bounds them is the work around the multiplications: weights decoded again for every 16 rows (tile_stream_core.h) or
 // staged, decoded, for the workgroup behind a barrier per 128 values (mmq_i_core.h).  Here
@@ -12,9 +12,10 @@
 //     behind the other, gathered row by row for the experts; two buffers and a barrier per 128 values;
 //   * a workgroup is four waves, so that a CU holds two or three and one's beginning and end lie beside another's middle.
 // Measured, us per call, before / now (quantizer, sorting and sums included; 4.83 TB/s is what a copy of 2 GiB reaches): Q4_K
-// [7968,2560] 308 rows 57 / 41, [11008,4096] 64 rows 29 / 21; MoE, 8 experts, top-2, H 4096, I 3584, 300 tokens: Q4_K 291 / 153,
-// Q5_K with Q6_K 309 / 196; 128 experts, top-8, H 2048, I 768, Q4_K with Q6_K, 300 tokens 173 / 154 (floor 82).  K-quants of 33 to
-// 2048 rows take 0.77 (Q4_K), 0.79 (Q5_K), 0.92 (Q6_K) of the time on average, Q4_0 0.93.
+// [7968,2560] 308 rows 57 / 41, [11008,4096] 64 rows 29 / 21; K-quants of 33 to 2048 rows take 0.77 (Q4_K), 0.79 (Q5_K), 0.92 (Q6_K) of
+// the time on average, Q4_0 0.93.  A MoE layer of Q6_K, 64 experts, 181 us on tiles of 32 slots only, 175 with the tiles of 16 for blocks
+// that are half empty.  (Tiles of 16 x 16 for everything: 0.84 to 1.0 times as fast.  Q6_K on the expert tiles: sixteen scales a
+// super-block are 849 vector instructions a panel and registers that spill; slower.)
 // What bounds it: no single thing.  With the fetches, the decoding, the operand reads or the multiply-adds left out in turn a
 // layer's first product (64 rows a workgroup) is 9 to 14 % faster each; a matrix instruction beside eight multiply-adds takes a
 // SIMD 44 cycles (2 waves) where it issues alone in 32.  A beginning and an end are 4 us of a workgroup's 15 to 30.
@@ -23,7 +24,7 @@
 // the runs end unevenly, and their state spills at three workgroups per CU).
 // Arithmetic as in the other integer kernels (mmq.cuh:2-104, moe.cuh:5-129): exact block sums, scales in fp32.
 #pragma once
-#include "q8_1_device.h"
+#include "layer_seam.h"
 #include "tile_wide.h"
 #include "tile_wide_formats.h"
 
@@ -59,14 +60,6 @@ __device__ __forceinline__ void wide_fetch_half(uint32_t at, const void* base, u
 __device__ __forceinline__ void wide_fetch_words(uint32_t at, const void* base, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(at), "s"(base), "s"(lds) : "memory");
 }
-__device__ __forceinline__ float wide_rounded(float v, int dtype) {   // to the result's type and back
-  return dtype == GGUF_DTYPE_F32 ? v : dtype == GGUF_DTYPE_F16 ? (float)(_Float16)v : (float)(__bf16)v;
-}
-// gate1 in the result's type (which the branches around it are on, not its values)
-__device__ __forceinline__ float wide_gate(float g, float u, int act, int dtype) {
-  const float a = act == ACT_SILU ? g / (1.0f + expf(-g)) : g * 0.5f * (1.0f + erff(g * 0.70710678118654752440f));
-  return wide_rounded(wide_rounded(a, dtype) * u, dtype);
-}
 template <typename T>
 __device__ __forceinline__ void wide_store(const wide_f4& v, T* y, const T* bias, int n, int N, int quads) {
   if (quads && n + 3 < N) {
@@ -98,39 +91,26 @@ template <class F, int R> constexpr size_t wide_lds() {
   return 2 * wide_xbuf<R>() + (size_t)WIDE_NW * (512 * wide_ppr<F>() + wide_scale_bytes<F>() + 256) + 16;
 }
 
-// The quants of h as q8_1_quantize8 rounds them: by the reciprocal, by the quotient where a value lies close to a tie.  What is not a
-// number is 0, as the conversion to an integer leaves it there.
-__device__ __forceinline__ void wide_quants(const float (&h)[8], float d, bool none, float (&q)[8]) {
-  const float dd = none ? 1.0f : d, rd = __builtin_amdgcn_rcpf(dd);
-  bool exact = !(rd < 3.0e38f);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    q[i] = h[i] * rd;
-    exact = exact || fabsf(__builtin_amdgcn_fractf(fabsf(q[i])) - 0.5f) < 6.1035156e-5f;
-  }
-  if (exact) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) q[i] = roundf(h[i] / dd);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) q[i] = truncf(q[i] + copysignf(0.5f, q[i]));
-  }
-#pragma unroll
-  for (int i = 0; i < 8; ++i) q[i] = q[i] == q[i] ? q[i] : 0.0f;
-}
-
 // GATE: the first expert GEMM of a layer with its seam (Gate16): a wave's 32 weight rows are 16 features of the gate half and the
 // same of the up half, so that a lane has both sums of eight features; two waves finish a q8_1 block of h together.
-template <class F, int R, bool GATE>
+template <class F, int R, bool MOE, bool GATE>
 __global__ __launch_bounds__(64 * WIDE_NW, R == 1 ? 3 : 2) void tile_wide_kernel(const uint8_t* __restrict__ W, const char* __restrict__ X, void* __restrict__ Y,
                                                                                  WideArgs a, MoeArgs moe, Gate16 gate) {
   constexpr int M_T = 32 * R, PPR = wide_ppr<F>(), SLOT = 512 * PPR, NI = (32 * PPR + 63) / 64;   // (the last fetch: lanes 0 .. 31)
   constexpr int XB = wide_xbuf<R>(), RING_AT = 2 * XB, SC_AT = RING_AT + WIDE_NW * SLOT, ID_AT = SC_AT + WIDE_NW * wide_scale_bytes<F>();
   constexpr int XP = WIDE_REC / 16, XI = (M_T * XP + 63) / 64, XW = (XI + WIDE_NW - 1) / WIDE_NW;   // pieces of a record; fetches of a buffer; a wave's, at most
   static_assert(wide_lds<F, R>() <= 80 * 1024, "two workgroups do not fit in LDS");
+  static_assert(!GATE || MOE, "a gated product is a layer's");
+  static_assert(!MOE || (R == 1 && F::KIND == SUPER && !F::OFF), "blocks of 32 slots; the small ones below have no offsets");
   extern __shared__ __align__(16) char smem[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lrow = lane & 31, half = lane >> 5;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int lane = tid & 63, lrow = lane & 31, half = lane >> 5;
+  // (a layer's instances count the lanes again before and behind their panels: what is formed from the number would go to scratch beside them)
+  const auto lane_again = [&] {
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(lane));
+    lrow = lane & 31;
+    half = lane >> 5;
+  };
 
   // ---- which rows and columns.  Tiles are numbered along the columns of a row block, and the workgroups go to the XCDs in turn: with
   // a multiple of eight columns the blocks of an expert find its weights in one L2, and the blocks past the last live one, of
@@ -138,10 +118,9 @@ __global__ __launch_bounds__(64 * WIDE_NW, R == 1 ? 3 : 2) void tile_wide_kernel
   // experts, 80 tokens: 109 us the layer against 81.)
   const int tile = (int)blockIdx.x;
   const int block = tile / a.col_wgs, col_wg = tile - block * a.col_wgs;
-  const bool is_moe = moe.sorted_token_ids != nullptr;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
   const int ids_at = ID_AT + wave * 256;
-  if (is_moe) {
+  if constexpr (MOE) {
     const int live = moe.num_tokens_post_padded[0], e = moe.expert_ids[block];
     if (block * M_T >= live || e < 0 || e > 255) return;    // (experts above 255: the reference's guard, moe.cuh:33)
     W += (int64_t)e * moe.expert_stride;
@@ -163,6 +142,7 @@ __global__ __launch_bounds__(64 * WIDE_NW, R == 1 ? 3 : 2) void tile_wide_kernel
     const int q = min(64 * i + lane, 32 * PPR - 1), r = q / PPR;
     w_at[i] = (uint32_t)row_of(r) * a.w_pitch + wmis;
     w_piece[i] = 16 * (uint32_t)(q - r * PPR);
+    if constexpr (MOE) asm volatile("" : "+v"(w_at[i]));    // (one value for both of the loops below: a second form of it would go to scratch)
   }
   const auto request = [&](int p) {
 #pragma unroll
@@ -177,12 +157,12 @@ __global__ __launch_bounds__(64 * WIDE_NW, R == 1 ? 3 : 2) void tile_wide_kernel
 
   // ---- fetching records: a wave's fetches of a buffer, pieces 64 i .. of it for i = wave, wave + 4, ...
   uint32_t x_at[XW];
-  if (is_moe) wide_wait<NI>();                              // (the slots' pairs are here)
+  if constexpr (MOE) wide_wait<NI>();                       // (the slots' pairs are here)
 #pragma unroll
   for (int j = 0; j < XW; ++j) {
     const int q = min(64 * (wave + WIDE_NW * j) + lane, M_T * XP - 1), r = q / XP;
     int row;
-    if (is_moe) {
+    if constexpr (MOE) {
       const int id = *(const int*)(smem + ids_at + 4 * r);
       row = id < moe.num_pairs ? (moe.top_k == 1 ? id : (int)__umulhi((uint32_t)id, a.topk_inv)) : 0;   // row 0 stands in for padding
     } else {
@@ -197,6 +177,131 @@ __global__ __launch_bounds__(64 * WIDE_NW, R == 1 ? 3 : 2) void tile_wide_kernel
       if (wave + WIDE_NW * j < XI) wide_fetch(x_at[j], base, lds0 + (ch & 1) * XB + 1024 * (wave + WIDE_NW * j));
   };
   fetch_x(2 * p0);
+
+  if constexpr (MOE) {
+    // The pairs of a block come first, padding behind them: where the upper sixteen slots hold none, as in about every second expert's last block, tiles of
+    // 16 x 16, half the matrix instructions and multiply-adds: a lane has one row of X and weight rows 16 i + 4 g + e.
+    if ((__ballot(*(const int*)(smem + ids_at + 4 * lrow) < moe.num_pairs) >> 16 & 0xFFFFu) == 0) {
+      lane_again();
+      int c = lane & 15, g = lane >> 4;
+      char* const scales = smem + SC_AT + wave * wide_scale_bytes<F>();
+      const wide_f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+      wide_f4 acc[2] = {zero, zero}, part[2];
+      for (int p = p0; p < p1; ++p) {
+        F w;
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) {
+          if (hh == 1 && p + 1 < p1) wide_wait<NI>();       // (as below)
+          else wide_wait<0>();
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          __builtin_amdgcn_s_barrier();
+          asm volatile("" ::: "memory");
+          if (hh == 0 || p + 1 < p1) fetch_x(2 * p + hh + 1);
+          if (hh == 0) {
+            w.read(smem + RING_AT + wave * SLOT + lrow * (16 * PPR), F::CUT ? ((uint32_t)row_of(lrow) * a.w_pitch + wmis + (uint32_t)(p * F::PB)) & 15 : 0u, half);
+            w.scale_to((float*)scales, lrow, half);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (p + 1 < p1) request(p + 1);
+          }
+          const char* const xrow = smem + hh * XB + c * WIDE_REC;
+          const uint2 head = *(const uint2*)(xrow + WIDE_D_AT);
+          float d8[4] = {half_bits(head.x & 0xFFFF), half_bits(head.x >> 16), half_bits(head.y & 0xFFFF), half_bits(head.y >> 16)};
+          asm volatile("" : "+v"(d8[0]), "+v"(d8[1]), "+v"(d8[2]), "+v"(d8[3]));
+          f16x8 xo[2], wo[2][F::PLANES];
+          wide_f4 s[2][2];
+          const auto load_x = [&](int b) { xo[b & 1] = *(const f16x8*)(xrow + 64 * b + 16 * g); };
+          // Of the lane's two operands, eight values each of one of 32 rows, the second of lanes 0 .. 15 and 32 .. 47 and the first of the lanes behind them
+          // change places: then either has 16 rows' 32 values.
+          const auto decode = [&](int b) {
+            f16x8 o[F::PLANES][2];
+            w.operand(4 * hh + b, half, o);
+#pragma unroll
+            for (int pl = 0; pl < F::PLANES; ++pl) {
+              typedef uint32_t Words __attribute__((ext_vector_type(4)));
+              Words u = __builtin_bit_cast(Words, o[pl][0]), v = __builtin_bit_cast(Words, o[pl][1]);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const auto z = __builtin_amdgcn_permlane16_swap(u[e], v[e], false, false);
+                u[e] = z[0];
+                v[e] = z[1];
+              }
+              wo[0][pl] = __builtin_bit_cast(f16x8, u);
+              wo[1][pl] = __builtin_bit_cast(f16x8, v);
+            }
+          };
+          const auto scale = [&](int b, int i) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) part[i][r] = hh == 0 && b == 0 ? s[b & 1][i][r] * d8[b] : __builtin_fmaf(s[b & 1][i][r], d8[b], part[i][r]);
+            asm volatile("" : "+v"(part[i]));
+          };
+          load_x(0);
+          load_x(1);
+          decode(0);
+#pragma unroll
+          for (int b = 0; b < 4; ++b) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+#pragma unroll
+              for (int pl = 0; pl < F::PLANES; ++pl) s[b & 1][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wo[i][pl], xo[b & 1], pl == 0 ? zero : s[b & 1][i], 0, 0, 0);
+              __builtin_amdgcn_sched_barrier(0);
+              if (b > 0) scale(b - 1, i);
+              __builtin_amdgcn_sched_barrier(0);
+            }
+            if (b + 2 < 4) load_x(b + 2);
+            if (b + 1 < 4) decode(b + 1);
+          }
+          scale(3, 0);
+          scale(3, 1);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const wide_f4 d = *(const wide_f4*)(scales + 4 * (16 * i + 4 * g));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i][e] = __builtin_fmaf(part[i][e], d[e], acc[i][e]);
+        }
+      }
+      lane_again();
+      c = lane & 15;
+      g = lane >> 4;
+      const int pair = *(const int*)(smem + ids_at + 4 * c);
+      if constexpr (GATE) {
+        float h[4];                                         // features 4 g + e of the wave's sixteen
+#pragma unroll
+        for (int e = 0; e < 4; ++e) h[e] = seam_gate(seam_rounded(acc[0][e], a.dtype), seam_rounded(acc[1][e], a.dtype), gate.act, a.dtype);
+        __syncthreads();
+        wide_f4* const all = (wide_f4*)smem;
+        all[wave * 64 + lane] = (wide_f4){h[0], h[1], h[2], h[3]};
+        __syncthreads();
+        if (n0 >= gate.inner) return;
+        const wide_f4 o = all[(wave ^ 1) * 64 + lane];
+        float amax = 0.0f, t[4];                            // (the same butterfly: 16, 8, 4, 2, 1)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          amax = fmaxf(fmaxf(amax, fabsf(h[e])), fabsf(o[e]));
+          t[e] = h[e] + o[e];
+          t[e] += __shfl_xor(t[e], 32);
+          t[e] += __shfl_xor(t[e], 16);
+        }
+        amax = fmaxf(amax, __shfl_xor(amax, 32));
+        amax = fmaxf(amax, __shfl_xor(amax, 16));
+        const float sum = (t[0] + t[2]) + (t[1] + t[3]), d = amax / 127.0f;
+        float q[4];
+        seam_quants(h, d, amax == 0.0f, q);
+        if (pair < moe.num_pairs) {
+          char* const rec = seam_h_record(gate, n0, pair, moe.num_pairs);
+          const int blk = (n0 >> 5) & 3;
+          seam_h_store(rec, gate, blk, (n0 & 16) + 4 * g, q);
+          if (g == 0 && (n0 & 16) == 0) seam_h_scales(rec, gate, blk, d, sum);
+        }
+      } else {
+        if (a.ksplit > 1) Y = (float*)Y + (int64_t)blockIdx.y * a.split_stride;
+        if (pair < moe.num_pairs)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) wide_store(acc[i], pair, n0 + 16 * i + 4 * g, Y, a);
+      }
+      return;
+    }
+  }
 
   float acc[R][16], part[R][16];
 #pragma unroll
@@ -353,6 +458,7 @@ __global__ __launch_bounds__(64 * WIDE_NW, R == 1 ? 3 : 2) void tile_wide_kernel
   }
 
   // ---- results: lane = one row of X, 16 weight rows in runs of four
+  if constexpr (MOE) lane_again();
   if constexpr (GATE) {
     // h of eight features, 8 q + 4 half + e of the wave's sixteen: rows 0 .. 15 of the panel are the gate's sums, 16 .. 31 the up half's
     float h[R][8];
@@ -360,8 +466,8 @@ __global__ __launch_bounds__(64 * WIDE_NW, R == 1 ? 3 : 2) void tile_wide_kernel
     for (int k = 0; k < R; ++k)
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const float gv = wide_rounded(acc[k][i], a.dtype), uv = wide_rounded(acc[k][8 + i], a.dtype);
-        h[k][i] = wide_gate(gv, uv, gate.act, a.dtype);
+        const float gv = seam_rounded(acc[k][i], a.dtype), uv = seam_rounded(acc[k][8 + i], a.dtype);
+        h[k][i] = seam_gate(gv, uv, gate.act, a.dtype);
       }
     // The q8_1 block has 32 features: the other sixteen are the next wave's (the last one's).  amax and the sum as q8_1_quantize8
     // forms them, by a butterfly over 16 (the other wave), 8 (the lane's other run), 4 (the other half's lane), 2, 1.
@@ -387,22 +493,14 @@ __global__ __launch_bounds__(64 * WIDE_NW, R == 1 ? 3 : 2) void tile_wide_kernel
       amax = fmaxf(amax, __shfl_xor(amax, 32));
       const float sum = (t[0] + t[2]) + (t[1] + t[3]), d = amax / 127.0f;
       float q[8];
-      wide_quants(h[k], d, amax == 0.0f, q);
+      seam_quants(h[k], d, amax == 0.0f, q);
       const int pair = *(const int*)(smem + ids_at + 4 * (32 * k + lrow));
       if (pair < moe.num_pairs) {
-        char* const rec = gate.rows + ((int64_t)(n0 >> 7) * moe.num_pairs + pair) * WIDE_REC;
+        char* const rec = seam_h_record(gate, n0, pair, moe.num_pairs);
         const int blk = (n0 >> 5) & 3;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          union { _Float16 v[4]; uint2 u; } o;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o.v[(e & 1) * 2 + (e >> 1)] = (_Float16)q[4 * i + e];
-          *(uint2*)(rec + 64 * blk + 2 * (n0 & 16) + 16 * i + 8 * half) = o.u;
-        }
-        if (half == 0 && (n0 & 16) == 0) {
-          *(_Float16*)(rec + WIDE_D_AT + 2 * blk) = (_Float16)d;
-          *(_Float16*)(rec + WIDE_S_AT + 2 * blk) = (_Float16)sum;
-        }
+        for (int i = 0; i < 2; ++i) seam_h_store(rec, gate, blk, (n0 & 16) + 8 * i + 4 * half, q + 4 * i);
+        if (half == 0 && (n0 & 16) == 0) seam_h_scales(rec, gate, blk, d, sum);
       }
     }
     return;
@@ -411,8 +509,8 @@ __global__ __launch_bounds__(64 * WIDE_NW, R == 1 ? 3 : 2) void tile_wide_kernel
 #pragma unroll
   for (int k = 0; k < R; ++k) {
     int64_t row = block * M_T + 32 * k + lrow;
-    if (is_moe) row = *(const int*)(smem + ids_at + 4 * (32 * k + lrow));
-    const bool live = row < (is_moe ? moe.num_pairs : a.M);
+    if constexpr (MOE) row = *(const int*)(smem + ids_at + 4 * (32 * k + lrow));
+    const bool live = row < (MOE ? moe.num_pairs : a.M);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const wide_f4 v = {acc[k][4 * q], acc[k][4 * q + 1], acc[k][4 * q + 2], acc[k][4 * q + 3]};
@@ -421,13 +519,13 @@ __global__ __launch_bounds__(64 * WIDE_NW, R == 1 ? 3 : 2) void tile_wide_kernel
   }
 }
 
-template <class F, int R, bool GATE>
+template <class F, int R, bool MOE, bool GATE>
 static int wide_launch(const WideCall& c, hipStream_t stream) {
   constexpr size_t lds = wide_lds<F, R>();
   const int qk = F::KIND == SUPER ? 256 : 32, bs = F::KIND == SUPER ? F::PB : F::PB / 8;
   const int64_t pitch = c.w_pitch ? c.w_pitch : (int64_t)(c.K / qk) * bs;
   if (!F::CUT && (pitch % 16 != 0 || (uintptr_t)c.W % 16 != 0 || (c.moe.sorted_token_ids && c.moe.expert_stride % 16 != 0))) return GGUF_NOT_TAKEN;
-  auto kern = tile_wide_kernel<F, R, GATE>;
+  auto kern = tile_wide_kernel<F, R, MOE, GATE>;
   static std::atomic<uint64_t> done{0};
   allow_large_lds(kern, lds, done);
   const int cols = GATE ? (c.gate.inner + 63) / 64 : (c.N + WIDE_N - 1) / WIDE_N, top_k = c.moe.top_k > 0 ? c.moe.top_k : 1;
@@ -445,20 +543,20 @@ static int wide_launch(const WideCall& c, hipStream_t stream) {
 template <class F>
 static int wide_dense_run(const WideCall& c, hipStream_t s) {
   if (c.gate.rows || c.moe.sorted_token_ids || c.K % (F::KIND == SUPER ? 256 : 32) != 0) return GGUF_NOT_TAKEN;
-  return c.rt == 1 ? wide_launch<F, 1, false>(c, s) : wide_launch<F, 2, false>(c, s);
+  return c.rt == 1 ? wide_launch<F, 1, false, false>(c, s) : wide_launch<F, 2, false, false>(c, s);
 }
 // a layer's products (blocks of 32 slots)
 template <class F>
 static int wide_moe_run(const WideCall& c, hipStream_t s) {
   if (!c.moe.sorted_token_ids || c.K % 256 != 0 || c.rt != 1) return GGUF_NOT_TAKEN;
-  return c.gate.rows ? wide_launch<F, 1, true>(c, s) : wide_launch<F, 1, false>(c, s);
+  return c.gate.rows ? wide_launch<F, 1, true, true>(c, s) : wide_launch<F, 1, true, false>(c, s);
 }
 template <class F>
 static int wide_run(const WideCall& c, hipStream_t s) { return c.moe.sorted_token_ids ? wide_moe_run<F>(c, s) : wide_dense_run<F>(c, s); }
 // a dense product whose rows do not begin on 16 bytes (a shard of a merged tensor as wide as its widest one): A the panels that do
 template <class A, class F>
 static int wide_run_either(const WideCall& c, hipStream_t s) {
-  return c.moe.sorted_token_ids || ((uintptr_t)c.W % 16 == 0 && c.w_pitch % 16 == 0) ? wide_run<A>(c, s) : wide_dense_run<F>(c, s);
+  return (uintptr_t)c.W % 16 == 0 && c.w_pitch % 16 == 0 ? wide_dense_run<A>(c, s) : wide_dense_run<F>(c, s);
 }
 
 }  // namespace gguf

@@ -353,16 +353,4 @@ struct WQ45_1 {
   }
 };
 
-struct WQ8_0 : W32<34, false> {
-  __device__ __forceinline__ void read(const char* p, uint32_t at, int half) { read_blocks(p, at, 16 * half); }
-  __device__ __forceinline__ void operand(int b, int, f16x8 (&o)[1][2]) const {
-    const f16x2 k = both(1152.0f);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const uint32_t x = word(q[b], 2 * i) ^ 0x80808080u, y = word(q[b], 2 * i + 1) ^ 0x80808080u;
-      o[0][i] = wide_operand(wide_bytes<0>(x) - k, wide_bytes<1>(x) - k, wide_bytes<0>(y) - k, wide_bytes<1>(y) - k);
-    }
-  }
-};
-
 }  // namespace gguf

@@ -1,7 +1,6 @@
-// Instances of the wide tile kernel (tile_wide_core.h): Q4_0, Q8_0 (layers only: dense products are as fast on the int8 unit).
+// Instances of the wide tile kernel (tile_wide_core.h): Q4_0.
 #include "tile_wide_core.h"
 
 namespace gguf {
 int wide_q4_0(const WideCall& c, hipStream_t s) { return wide_run_either<WQ4_0T<false>, WQ4_0T<true>>(c, s); }
-int wide_q8_0(const WideCall& c, hipStream_t s) { return wide_moe_run<WQ8_0>(c, s); }
 }  // namespace gguf
