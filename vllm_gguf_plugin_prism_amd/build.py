@@ -27,6 +27,8 @@ FLAGS = [
     # packed fp32 VALU forms are kept out of the generated code on purpose
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
+    # a kernel's leading scalar arguments lie in registers when a wave begins (csrc/mmvq_core.h, GGUF_GEOM)
+    "-mllvm", "-amdgpu-kernarg-preload-count=16",
 ]
 
 

@@ -32,7 +32,8 @@ template <class F, int R, int NW> constexpr size_t dwalk_lds() {
 }
 
 template <class F, int R, int NW, bool DIRECT, typename T>
-__global__ __launch_bounds__(64 * NW, 2) void dense_walk_kernel(const uint8_t* __restrict__ W, const char* __restrict__ X, T* __restrict__ Y, WalkArgs a) {
+__global__ __launch_bounds__(64 * NW, 2) void dense_walk_kernel(const uint8_t* __restrict__ W, const char* __restrict__ X, GGUF_WALK_HEAD, T* __restrict__ Y, WalkEnd end) {
+  const WalkArgs a = GGUF_WALK_ARGS;
   constexpr int UB = dwalk_unit<F>(), PPR = dwalk_ppr(UB), SLOT = 512 * PPR, NI = (32 * PPR + 63) / 64;   // (the last fetch of a panel: lanes 0 .. 31)
   typedef DenseType<T> D;
   extern __shared__ __align__(16) char smem[];
@@ -166,11 +167,9 @@ static int dwalk_launch(const DwalkCall& c, hipStream_t stream) {
   allow_large_lds(kern, lds, done);
   const int64_t pitch = c.la.w_pitch ? c.la.w_pitch : (int64_t)(c.K / F::QK) * F::BS, ldy = c.la.ldy ? c.la.ldy : (int64_t)c.N;
   const int run = (tiles.tiles + 7) / 8;
-  const auto inverse = [](int d) { return (uint32_t)((0x100000000ull + d - 1) / d); };
-  const WalkArgs a = {c.M, c.N, (c.K + 255) / 256, c.K / 32, (c.M + 31) / 32, tiles.tiles, run, tiles.band, tiles.band_tiles, tiles.last,
-                      inverse(tiles.band), inverse(tiles.band_tiles), inverse(tiles.last), (uint32_t)pitch, c.dtype,
-                      ldy % 4 == 0 && (uintptr_t)c.Y % (4 * sizeof(T)) == 0, ldy, c.la.bias};
-  hipLaunchKernelGGL(kern, dim3((unsigned)(8 * run)), dim3(64 * NW), lds, stream, (const uint8_t*)c.W, (const char*)c.x, (T*)c.Y, a);
+  const WalkEnd end = {c.dtype, ldy % 4 == 0 && (uintptr_t)c.Y % (4 * sizeof(T)) == 0, ldy, c.la.bias};
+  hipLaunchKernelGGL(kern, dim3((unsigned)(8 * run)), dim3(64 * NW), lds, stream, (const uint8_t*)c.W, (const char*)c.x,
+                     GGUF_WALK_HEAD_ARGS(tiles, c.N, (uint32_t)pitch, c.K, c.M), (T*)c.Y, end);
   return launch_status();
 }
 

@@ -14,11 +14,11 @@ namespace gguf {
 
 // Workgroups before `wgs` have rows of W, the others rows of V.
 template <class F, int DF, int SF, class G, int DG, int SG, int MT, int NW, typename T>
-__global__ __launch_bounds__(64 * NW) void mmvq_pair_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ V, const T* __restrict__ X, T* __restrict__ Y,
-                                                            T* __restrict__ Z, const T* __restrict__ bias, const T* __restrict__ bias2, int64_t ldy, int wgs, StreamGeom geom,
-                                                            StreamGeom geom2) {
-  if ((int)blockIdx.x < wgs) mmvq_stream_body<F, MT, NW, DF, T, false, MT <= 2, SF, false>(W, X, Y, bias, ldy, geom, ACT_NONE, blockIdx.x);
-  else mmvq_stream_body<G, MT, NW, DG, T, false, MT <= 2, SG, false>(V, X, Z, bias2, ldy, geom2, ACT_NONE, blockIdx.x - wgs);
+__global__ __launch_bounds__(64 * NW) void mmvq_pair_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ V, const T* __restrict__ X, int wgs, GGUF_GEOM,
+                                                            uint32_t pitch2, int n2, int rows2, T* __restrict__ Y, T* __restrict__ Z, const T* __restrict__ bias,
+                                                            const T* __restrict__ bias2, int64_t ldy) {
+  if ((int)blockIdx.x < wgs) mmvq_stream_body<F, MT, NW, DF, T, false, MT <= 2, SF, false>(W, X, Y, bias, ldy, GGUF_GEOM_OF, ACT_NONE, blockIdx.x);
+  else mmvq_stream_body<G, MT, NW, DG, T, false, MT <= 2, SG, false>(V, X, Z, bias2, ldy, StreamGeom{pitch2, n2, g_k, rows2, g_packed, g_g8_inv}, ACT_NONE, blockIdx.x - wgs);
 }
 
 template <class F, int MT, int NW, int D, int STAGED>
@@ -45,9 +45,9 @@ static int pair_launch(const PairCall& c) {
   static std::atomic<uint64_t> done{0};
   if (lds > 64 * 1024) allow_large_lds(kern, 160 * 1024, done);
   const int wgs = ((int)c.a.N + c.r1 - 1) / c.r1, wgs2 = ((int)c.b.N + c.r2 - 1) / c.r2;
-  hipLaunchKernelGGL(kern, dim3(wgs + wgs2), dim3(64 * NW), lds, c.stream, (const uint8_t*)c.a.W, (const uint8_t*)c.b.W, (const T*)c.x, (T*)c.a.Y, (T*)c.b.Y,
-                     (const T*)c.a.la.bias, (const T*)c.b.la.bias, c.a.la.ldy, wgs, stream_geom((int)c.a.N, c.K, c.r1, c.a.la.w_pitch, c.M, NW),
-                     stream_geom((int)c.b.N, c.K, c.r2, c.b.la.w_pitch, c.M, NW));
+  const StreamGeom g1 = stream_geom((int)c.a.N, c.K, c.r1, c.a.la.w_pitch, c.M, NW), g2 = stream_geom((int)c.b.N, c.K, c.r2, c.b.la.w_pitch, c.M, NW);
+  hipLaunchKernelGGL(kern, dim3(wgs + wgs2), dim3(64 * NW), lds, c.stream, (const uint8_t*)c.a.W, (const uint8_t*)c.b.W, (const T*)c.x, wgs, GGUF_GEOM_ARGS(g1),
+                     g2.w_pitch, g2.N, g2.rows_per_wg, (T*)c.a.Y, (T*)c.b.Y, (const T*)c.a.la.bias, (const T*)c.b.la.bias, c.a.la.ldy);
   return launch_status();
 }
 

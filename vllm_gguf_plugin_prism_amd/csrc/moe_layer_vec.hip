@@ -38,27 +38,28 @@ int moe_sorted_layer(const void* X, int xdtype, void* workspace, const void* W13
                      const float* topk_w, void* out, int H, int I, int N_out, int top_k, int tokens, int act, int num_experts, int block,
                      hipStream_t s);
 
+// What the end of the first kernel needs.  (What its beginning does comes as scalars, in front: GGUF_GEOM.  R: features per band, a multiple of 32; I: inner
+// features; the experts' matrices follow one another, 2 I rows each.)
 struct MoeUpArgs {
-  const int32_t* topk_ids;
-  int64_t expert_bytes;    // between the matrices of two experts
   char* ws;                // q8_1 rows of h, one per pair
   int64_t ws_row_bytes;
-  int top_k, num_experts, act;
-  int I, R, kp_i;          // inner features; features per band (a multiple of 32); q8_kp(I)
+  int act, kp_i;           // (q8_kp(I))
 };
 
 template <class F, int NW, typename T, bool HALF>
-__global__ __launch_bounds__(64 * NW) void moe_up_act_kernel(const uint8_t* __restrict__ W, const T* __restrict__ X, MoeUpArgs moe, StreamGeom geom) {
+__global__ __launch_bounds__(64 * NW) void moe_up_act_kernel(const uint8_t* __restrict__ W, const T* __restrict__ X, const int32_t* __restrict__ topk_ids, uint32_t w_pitch, int K,
+                                                            uint32_t packed, uint32_t topk_inv, int num_experts, int I, int R, MoeUpArgs moe) {
   extern __shared__ __align__(16) char smem[];
   constexpr int NT = 64 * NW, D = 2;
+  const StreamGeom geom = {w_pitch, 2 * I, K, 2 * R, packed, 0};
   const int z = blockIdx.y;
-  const int e = moe.topk_ids[z];
-  if (moe.num_experts > 0 && (e < 0 || e >= moe.num_experts)) return;   // names no weights: its row is never read
+  const int e = topk_ids[z];
+  X += (int64_t)(topk_inv ? __umulhi((uint32_t)z, topk_inv) : (uint32_t)z) * K;
+  if (num_experts > 0 && (e < 0 || e >= num_experts)) return;   // names no weights: its row is never read
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int K = geom.K, nb = K >> 5, g8 = K >> 3, S = geom.S(), slots = geom.slots();
-  const int I = moe.I, R = moe.R, vrows = 2 * R;      // virtual rows of the band: R of the gate half, then R of the up half
-  X += (int64_t)(z / moe.top_k) * K;
-  W += (int64_t)e * moe.expert_bytes;
+  const int nb = K >> 5, g8 = K >> 3, S = geom.S(), slots = geom.slots();
+  const int vrows = 2 * R;                             // virtual rows of the band: R of the gate half, then R of the up half
+  W += (int64_t)e * (2 * I) * w_pitch;
   int8_t* lq = (int8_t*)smem;                          // [K]
   float* ldv = (float*)(smem + (size_t)K);             // [nb]
   float* lav = ldv + nb;                               // [nb]
@@ -84,7 +85,7 @@ __global__ __launch_bounds__(64 * NW) void moe_up_act_kernel(const uint8_t* __re
   const auto load_row = [&](int i) {
     const int v = min((on ? slot : 0) + slots * i, vrows - 1);
     const int row = v < R ? g0 + min(v, ng - 1) : I + g0 + min(v - R, ng - 1);
-    return F::load(W + (int64_t)row * geom.w_pitch, 0, u, tab);
+    return F::load(W + (int64_t)row * w_pitch, 0, u, tab);
   };
   // ---- the token's row -> q8_1 in LDS (four lanes per 32-value block), its first requests ahead of the weights'
   const auto quantize_group = [&](const raw8<T>& raw, int q) {
@@ -164,23 +165,22 @@ __global__ __launch_bounds__(64 * NW) void moe_up_act_kernel(const uint8_t* __re
   }
 }
 
+// The rest of the second kernel's arguments.  (side: the rows of the band that one pair's waves walk side by side, << 24, and 65536 / top_k + 1: n / top_k for n < 4096 as
+// (n * that) >> 16; ws: q8_1 rows of the pairs; the experts' matrices follow one another, N rows each.)
 struct MoeSumArgs {
-  const int32_t* topk_ids;
   const float* topk_w;
-  int64_t expert_bytes;    // between the matrices of two experts
-  const char* ws;          // q8_1 rows of the pairs
   int64_t ws_row_bytes;
-  int top_k, num_experts, slots, kp;   // slots: rows of the band that one pair's waves walk side by side; kp = q8_kp(K)
-  uint32_t tk_inv;         // 65536 / top_k + 1: n / top_k for n < 4096 as (n * tk_inv) >> 16
+  int kp;                  // q8_kp(K)
 };
 
 template <class F, int NW, typename T, bool HALF>
-__global__ __launch_bounds__(64 * NW) void moe_down_sum_kernel(const uint8_t* __restrict__ W, T* __restrict__ out, MoeSumArgs moe, StreamGeom geom) {
+__global__ __launch_bounds__(64 * NW) void moe_down_sum_kernel(const uint8_t* __restrict__ W, const char* __restrict__ ws, const int32_t* __restrict__ topk_ids, uint32_t w_pitch, int N, int K,
+                                                              int rows_per_wg, uint32_t packed, int top_k, int num_experts, uint32_t side, T* __restrict__ out, MoeSumArgs moe) {
   extern __shared__ __align__(16) char smem[];
   constexpr int NT = 64 * NW, D = 2;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int token = blockIdx.y, top_k = moe.top_k;
-  const int N = geom.N, K = geom.K, rows_per_wg = geom.rows_per_wg;
+  const StreamGeom geom = {w_pitch, N, K, rows_per_wg, packed, 0};
+  const int token = blockIdx.y;
   const int nb = K >> 5, S = geom.S();
   char* tab = smem;
   float* part = (float*)(tab + ((F::TABLE_BYTES + 15) & ~15));   // [top_k][rows_per_wg][G]
@@ -191,15 +191,15 @@ __global__ __launch_bounds__(64 * NW) void moe_down_sum_kernel(const uint8_t* __
   // this (half-)wave: which pair, which of the pair's side-by-side rows, which stretch of the row
   const int wh = HALF ? 2 * wave + (lane >> 5) : wave;
   const int rs = geom.slot_of(wh), step = wh - rs * S;
-  const int slots = moe.slots;
+  const int slots = (int)(side >> 24);
   const bool on = rs < slots * top_k;
-  const int slot = on ? (int)(((uint32_t)rs * moe.tk_inv) >> 16) : 0;   // rs / top_k
+  const int slot = on ? (int)(((uint32_t)rs * (side & 0xFFFFFFu)) >> 16) : 0;   // rs / top_k
   const int pair = on ? rs - slot * top_k : 0;                          // rs % top_k
   const int u_raw = HALF ? step * 32 + (lane & 31) : step * 64 + lane;
   const int u = min(u_raw, nb - 1);
   const int z = token * top_k + pair;
-  int e = moe.topk_ids[z];
-  const bool known = moe.num_experts <= 0 || (e >= 0 && e < moe.num_experts);   // a pair that names no expert adds nothing
+  int e = topk_ids[z];
+  const bool known = num_experts <= 0 || (e >= 0 && e < num_experts);   // a pair that names no expert adds nothing
   if (!known) e = 0;
   const bool lane_on = on && known && u_raw < nb;
 
@@ -207,14 +207,14 @@ __global__ __launch_bounds__(64 * NW) void moe_down_sum_kernel(const uint8_t* __
     F::init_tables(tab);
     __syncthreads();
   }
-  const uint8_t* wbase = W + (int64_t)e * moe.expert_bytes + (int64_t)r_begin * geom.w_pitch;
-  const auto load_row = [&](int i) { return F::load(wbase + (int64_t)min(slot + slots * i, nrows - 1) * geom.w_pitch, 0, u, tab); };
+  const uint8_t* wbase = W + ((int64_t)e * N + r_begin) * w_pitch;
+  const auto load_row = [&](int i) { return F::load(wbase + (int64_t)min(slot + slots * i, nrows - 1) * w_pitch, 0, u, tab); };
   typename F::Regs pre[D];
 #pragma unroll
   for (int d = 0; d < D; ++d) pre[d] = load_row(d);
   // the pair's quantized activations, this lane's unit of them, straight from the workspace (a row the first kernel
   // left unwritten -- an unknown expert -- is not read)
-  const char* xrow = moe.ws + (int64_t)(known ? z : token * top_k) * moe.ws_row_bytes;
+  const char* xrow = ws + (int64_t)(known ? z : token * top_k) * moe.ws_row_bytes;
   Act x;
   x.q = (const int8_t*)xrow;
   x.d = (const float*)(xrow + moe.kp);
@@ -243,8 +243,8 @@ __global__ __launch_bounds__(64 * NW) void moe_down_sum_kernel(const uint8_t* __
     for (int p = 0; p < top_k; ++p) {
       float y = 0.0f;
       for (int st = 0; st < G; ++st) y += part[((size_t)p * rows_per_wg + i) * G + st];
-      const int ep = moe.topk_ids[token * top_k + p];
-      if (moe.num_experts > 0 && (ep < 0 || ep >= moe.num_experts)) continue;
+      const int ep = topk_ids[token * top_k + p];
+      if (num_experts > 0 && (ep < 0 || ep >= num_experts)) continue;
       const T scaled = from_f32<T>(to_f32<T>(from_f32<T>(y)) * moe.topk_w[token * top_k + p]);
       total += to_f32<T>(scaled);
     }
@@ -349,14 +349,16 @@ static int moe_up_typed(const void* W, const void* X, const int32_t* ids, void* 
   const MoeUpPlan p = moe_up_plan<F>(H, I, pairs);
   if (!p.ok) return GGUF_ERR_SHAPE;
   const int64_t pitch = (int64_t)(H / F::QK) * F::BS;
-  const MoeUpArgs moe = {ids, (int64_t)2 * I * pitch, (char*)ws, q8_row_bytes(I), top_k, num_experts, act, I, p.R, (int)q8_kp(I)};
+  const MoeUpArgs moe = {(char*)ws, q8_row_bytes(I), act, (int)q8_kp(I)};
+  const uint32_t topk_inv = top_k > 1 ? (uint32_t)((0x100000000ull + top_k - 1) / top_k) : 0u;   // z / top_k as the upper half of z times that (z * top_k < 2^32: 65535 pairs at most)
   const StreamGeom geom = stream_geom(2 * I, H, 2 * p.R, pitch, 1, NW, p.rows.half);
   const auto go = [&](auto kern) {
     if (p.lds > 64 * 1024) {
       static std::atomic<uint64_t> done{0};
       allow_large_lds(kern, 160 * 1024, done);
     }
-    hipLaunchKernelGGL(kern, dim3(p.bands, pairs), dim3(64 * NW), p.lds, stream, (const uint8_t*)W, (const T*)X, moe, geom);
+    hipLaunchKernelGGL(kern, dim3(p.bands, pairs), dim3(64 * NW), p.lds, stream, (const uint8_t*)W, (const T*)X, ids, geom.w_pitch, H, geom.packed, topk_inv, num_experts, I,
+                       p.R, moe);
   };
   if (p.rows.half) go(moe_up_act_kernel<F, NW, T, true>);
   else go(moe_up_act_kernel<F, NW, T, false>);
@@ -370,15 +372,15 @@ static int moe_sum_typed(const void* W, const void* ws, const int32_t* ids, cons
   const MoeSumPlan p = moe_sum_plan<F>(N, K, top_k, tokens);
   if (!p.ok) return GGUF_ERR_SHAPE;
   const int64_t pitch = (int64_t)(K / F::QK) * F::BS;
-  const MoeSumArgs moe = {ids, wts, (int64_t)N * pitch, (const char*)ws, q8_row_bytes(K), top_k, num_experts, p.slots, (int)q8_kp(K),
-                          65536u / (uint32_t)top_k + 1u};
+  const MoeSumArgs moe = {wts, q8_row_bytes(K), (int)q8_kp(K)};
   const StreamGeom geom = stream_geom(N, K, p.rows_per_wg, pitch, 1, NW, p.rows.half);
   const auto go = [&](auto kern) {
     if (p.lds > 64 * 1024) {
       static std::atomic<uint64_t> done{0};
       allow_large_lds(kern, 160 * 1024, done);
     }
-    hipLaunchKernelGGL(kern, dim3(p.grid, tokens), dim3(64 * NW), p.lds, stream, (const uint8_t*)W, (T*)out, moe, geom);
+    hipLaunchKernelGGL(kern, dim3(p.grid, tokens), dim3(64 * NW), p.lds, stream, (const uint8_t*)W, (const char*)ws, ids, geom.w_pitch, N, K, p.rows_per_wg, geom.packed,
+                       top_k, num_experts, (uint32_t)p.slots << 24 | (65536u / (uint32_t)top_k + 1u), (T*)out, moe);
   };
   if (p.rows.half) go(moe_down_sum_kernel<F, NW, T, true>);
   else go(moe_down_sum_kernel<F, NW, T, false>);

@@ -51,6 +51,19 @@ struct TsArgs {
   const void* bias;
 };
 
+// What the first requests are formed from comes as scalars in front as well (GGUF_GEOM, mmvq_core.h): the kernels take those fields from there.
+#define GGUF_TS_HEAD uint32_t h_pitch, uint32_t h_ws_row, int h_m, int h_n, int h_k, uint32_t h_small, uint32_t h_ppr_inv
+#define GGUF_TS_HEAD_ARGS(a)                                                                                                                                             \
+  (a).w_pitch, (a).ws_row_bytes, (a).M, (a).N, (a).K,                                                                                                                     \
+      (uint32_t)(a).ppr | (uint32_t)(a).ks_log2 << 8 | (uint32_t)(a).pc_log2 << 10 | (uint32_t)(a).nbuf << 13 | (uint32_t)(a).plane << 15 | (uint32_t)(a).passes << 17, (a).ppr_inv
+__device__ __forceinline__ TsArgs ts_args(GGUF_TS_HEAD, TsArgs a) {
+  a.w_pitch = h_pitch; a.ws_row_bytes = h_ws_row; a.M = h_m; a.N = h_n; a.K = h_k; a.ppr_inv = h_ppr_inv;
+  a.Kp = (int)q8_kp(h_k); a.np = (h_k + 255) >> 8;
+  a.ppr = h_small & 255; a.ks_log2 = h_small >> 8 & 3; a.pc_log2 = h_small >> 10 & 7; a.nbuf = h_small >> 13 & 3; a.plane = h_small >> 15 & 3; a.passes = h_small >> 17;
+  return a;
+}
+#define GGUF_TS_ARGS(rest) ts_args(h_pitch, h_ws_row, h_m, h_n, h_k, h_small, h_ppr_inv, rest)
+
 typedef uint32_t u32x4_s __attribute__((ext_vector_type(4)));
 typedef _Float16 ts_h2 __attribute__((ext_vector_type(2)));
 
@@ -180,9 +193,10 @@ __device__ __forceinline__ void ts_multiply(F& w, const u32x4_s (&xa)[RT][4], co
 }
 
 template <class F, int RT, bool GATE, bool SPLIT, int D, bool MOE>
-__global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_stream_kernel(const uint8_t* __restrict__ W, const char* __restrict__ ws,
-                                                                                  void* __restrict__ Y, TsArgs a, MoeArgs moe, Gate16 gate,
-                                                                                  int row_blocks, int total) {
+__global__ __launch_bounds__(64 * TS_NW, RT == 1 && !SPLIT ? 4 : 2) void tile_stream_kernel(const uint8_t* __restrict__ W, const char* __restrict__ ws, GGUF_TS_HEAD,
+                                                                                  int row_blocks, int total, void* __restrict__ Y, TsArgs rest, MoeArgs moe,
+                                                                                  Gate16 gate) {
+  const TsArgs a = GGUF_TS_ARGS(rest);
   static_assert(!GATE || (MOE && !SPLIT), "a gated product is a layer's and takes its column groups whole");
   static_assert(!MOE || RT == 1, "blocks of 16 slots");
   static_assert(D >= 2 && D <= 4, "one wait per number of panels requested behind the one at hand");
@@ -758,16 +772,18 @@ __device__ __forceinline__ void tile_dealt_body(const uint8_t* __restrict__ W, c
 }
 
 template <class F, int RT, int CG>
-__global__ __launch_bounds__(64 * TS_NW, (ts_dealt_waves<F, RT>())) void tile_dealt_kernel(const uint8_t* __restrict__ W, const char* __restrict__ ws, void* __restrict__ Y, TsArgs a) {
-  tile_dealt_body<F, RT, CG>(W, ws, Y, a, blockIdx.x, gridDim.x);
+__global__ __launch_bounds__(64 * TS_NW, (ts_dealt_waves<F, RT>())) void tile_dealt_kernel(const uint8_t* __restrict__ W, const char* __restrict__ ws, GGUF_TS_HEAD, int wgs, void* __restrict__ Y,
+                                                                                                 TsArgs rest) {
+  // (of many groups the scalars would go to scratch: from memory they are loaded where they are wanted)
+  tile_dealt_body<F, RT, CG>(W, ws, Y, CG > 2 ? rest : GGUF_TS_ARGS(rest), blockIdx.x, wgs);
 }
 
 // The same for two matrices with the same rows of X, those of a merged layer whose recipe gives one of its tensors more bits: the
 // workgroups of the second, often too few for the chip by themselves, run beside the first's, and a launch less.
 template <class F, class G, int RT, int CG>
 __global__ __launch_bounds__(64 * TS_NW, (ts_dealt_waves<F, RT>() < ts_dealt_waves<G, RT>() ? ts_dealt_waves<F, RT>() : ts_dealt_waves<G, RT>())) void tile_dealt_pair_kernel(
-    const uint8_t* __restrict__ W, const uint8_t* __restrict__ V, const char* __restrict__ ws, void* __restrict__ Y, void* __restrict__ Z, TsArgs a, TsArgs b, int wgs) {
-  if ((int)blockIdx.x < wgs) tile_dealt_body<F, RT, CG>(W, ws, Y, a, blockIdx.x, wgs);
+    const uint8_t* __restrict__ W, const char* __restrict__ ws, GGUF_TS_HEAD, int wgs, const uint8_t* __restrict__ V, void* __restrict__ Y, void* __restrict__ Z, TsArgs rest, TsArgs b) {
+  if ((int)blockIdx.x < wgs) tile_dealt_body<F, RT, CG>(W, ws, Y, GGUF_TS_ARGS(rest), blockIdx.x, wgs);
   else tile_dealt_body<G, RT, CG>(V, ws, Z, b, blockIdx.x - wgs, gridDim.x - wgs);
 }
 
@@ -816,8 +832,8 @@ static int ts_launch_d(const TsCall& c, int ks, TsArgs a, size_t lds, hipStream_
     static std::atomic<uint64_t> done{0};
     allow_large_lds(kern, 160 * 1024, done);
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(64 * TS_NW), lds, stream, (const uint8_t*)c.W, (const char*)c.ws, c.Y, a, c.moe, c.gate,
-                     c.row_blocks, (int)total);
+  hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(64 * TS_NW), lds, stream, (const uint8_t*)c.W, (const char*)c.ws, GGUF_TS_HEAD_ARGS(a),
+                     c.row_blocks, (int)total, c.Y, a, c.moe, c.gate);
   return launch_status();
 }
 
@@ -915,7 +931,8 @@ static int ts_dealt_launch_cg(const TsCall& c, int ng, hipStream_t stream) {
   auto kern = tile_dealt_kernel<F, RT, CG>;
   static std::atomic<uint64_t> done{0};
   if (lds > 64 * 1024) allow_large_lds(kern, 160 * 1024, done);
-  hipLaunchKernelGGL(kern, dim3((unsigned)((c.N + 16 * ng - 1) / (16 * ng))), dim3(64 * TS_NW), lds, stream, (const uint8_t*)c.W, (const char*)c.ws, c.Y, a);
+  const int wgs = (c.N + 16 * ng - 1) / (16 * ng);
+  hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(64 * TS_NW), lds, stream, (const uint8_t*)c.W, (const char*)c.ws, GGUF_TS_HEAD_ARGS(a), wgs, c.Y, a);
   return launch_status();
 }
 template <class F, int RT>
@@ -943,8 +960,8 @@ static int ts_dealt_pair_launch(const TsCall& c, const TsCall& d, hipStream_t st
   static std::atomic<uint64_t> done{0};
   if (lds > 64 * 1024) allow_large_lds(kern, 160 * 1024, done);
   const int wgs = (c.N + 16 * CG - 1) / (16 * CG);
-  hipLaunchKernelGGL(kern, dim3((unsigned)wgs + (unsigned)((d.N + 16 * CG - 1) / (16 * CG))), dim3(64 * TS_NW), lds, stream, (const uint8_t*)c.W, (const uint8_t*)d.W,
-                     (const char*)c.ws, c.Y, d.Y, a, b, wgs);
+  hipLaunchKernelGGL(kern, dim3((unsigned)wgs + (unsigned)((d.N + 16 * CG - 1) / (16 * CG))), dim3(64 * TS_NW), lds, stream, (const uint8_t*)c.W, (const char*)c.ws,
+                     GGUF_TS_HEAD_ARGS(a), wgs, (const uint8_t*)d.W, c.Y, d.Y, a, b);
   return launch_status();
 }
 template <class F, class G, int RT>

@@ -51,6 +51,17 @@ struct WalkArgs {
   const void* bias;
 };
 
+// What the first requests are formed from comes as scalars in front (GGUF_GEOM, mmvq_core.h), the rest behind.
+struct WalkEnd { int dtype, quads; int64_t ldy; const void* bias; };
+#define GGUF_WALK_HEAD int h_tiles, uint32_t h_bands, int h_n, uint32_t h_pitch, int h_nkb, int h_m, uint32_t h_band_inv, uint32_t h_all_inv, uint32_t h_last_inv
+#define GGUF_WALK_ARGS                                                                                                                                                     \
+  WalkArgs{h_m, h_n, (h_nkb + 7) >> 3, h_nkb, (h_m + 31) >> 5, h_tiles, (h_tiles + 7) >> 3, (int)(h_bands & 0xFFFF), (int)(h_bands & 0xFFFF) * ((h_n + 31) >> 5),            \
+           (int)(h_bands >> 16), h_band_inv, h_all_inv, h_last_inv, h_pitch, end.dtype, end.quads, end.ldy, end.bias}
+// (a band's rows of X fit in 3 MB: less than 2^16 row blocks)
+static inline uint32_t walk_inverse(int d) { return (uint32_t)((0x100000000ull + d - 1) / d); }
+#define GGUF_WALK_HEAD_ARGS(b, n, pitch, k, m) \
+  (b).tiles, (uint32_t)(b).band | (uint32_t)(b).last << 16, n, pitch, (k) / 32, m, walk_inverse((b).band), walk_inverse((b).band_tiles), walk_inverse((b).last)
+
 template <int N> __device__ __forceinline__ void walk_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 // wave-uniform 16-byte-per-lane fetch into LDS: lane l's bytes land at lds + AT + 16 l.  (The sum is formed here, by a scalar instruction: as an operand the
 // compiler may have formed it in a vector register, with the addresses that the lanes read from.)
@@ -97,7 +108,8 @@ template <int U> struct WalkUnit { static constexpr int value = U; };
 template <class L, int... U> __device__ __forceinline__ void walk_units(const L& unit, std::integer_sequence<int, U...>) { (unit(WalkUnit<U>()), ...); }
 
 template <class F, int R, int NW, int D>
-__global__ __launch_bounds__(64 * NW, 2) void tile_walk_kernel(const uint8_t* __restrict__ W, const char* __restrict__ X, void* __restrict__ Y, WalkArgs a) {
+__global__ __launch_bounds__(64 * NW, 2) void tile_walk_kernel(const uint8_t* __restrict__ W, const char* __restrict__ X, GGUF_WALK_HEAD, void* __restrict__ Y, WalkEnd end) {
+  const WalkArgs a = GGUF_WALK_ARGS;
   constexpr int PPR = walk_ppr<F>(), SLOT = 512 * PPR, NI = (32 * PPR + 63) / 64, PD = WALK_PD, GS = 32 / F::G, U = 8 * R * GS;   // (the last fetch of a panel: lanes 0 .. 31)
   constexpr int HEAD = walk_head<F>(), XR_AT = SLOT * D, HD_AT = XR_AT + 1024 * PD, SC_AT = HD_AT + HEAD * R, PLACE = walk_place<F, R, D>();
   constexpr bool PART = R <= (F::G == 16 ? 3 : 2) || F::WHOLE;                             // a panel's sum of its own, where the registers hold it
@@ -376,11 +388,9 @@ static int walk_launch(const WalkCall& c, hipStream_t stream) {
   allow_large_lds(kern, lds, done);
   const int64_t pitch = c.la.w_pitch ? c.la.w_pitch : walk_row_bytes<F>(c.K), ldy = c.la.ldy ? c.la.ldy : (int64_t)c.N;
   const int run = (bands.tiles + 7) / 8, elt = c.dtype == GGUF_DTYPE_F32 ? 4 : 2;
-  const auto inverse = [](int d) { return (uint32_t)((0x100000000ull + d - 1) / d); };
-  const WalkArgs a = {c.M, c.N, (c.K + 255) / 256, c.K / 32, (c.M + 31) / 32, bands.tiles, run, bands.band, bands.band_tiles, bands.last,
-                      inverse(bands.band), inverse(bands.band_tiles), inverse(bands.last), (uint32_t)pitch, c.dtype,
-                      ldy % 4 == 0 && (uintptr_t)c.Y % (4 * elt) == 0, ldy, c.la.bias};
-  hipLaunchKernelGGL(kern, dim3((unsigned)(8 * run)), dim3(64 * NW), lds, stream, (const uint8_t*)c.W, (const char*)c.x, c.Y, a);
+  const WalkEnd end = {c.dtype, ldy % 4 == 0 && (uintptr_t)c.Y % (4 * elt) == 0, ldy, c.la.bias};
+  hipLaunchKernelGGL(kern, dim3((unsigned)(8 * run)), dim3(64 * NW), lds, stream, (const uint8_t*)c.W, (const char*)c.x,
+                     GGUF_WALK_HEAD_ARGS(bands, c.N, (uint32_t)pitch, c.K, c.M), c.Y, end);
   return launch_status();
 }
 
