@@ -89,6 +89,8 @@ _LAYER_SIGNATURES = {
     "gguf_dense_linear_workspace_bytes": (_c.c_int64, [_c.c_int64, _c.c_int64, _c.c_int64]),
     "gguf_mmq_layer_workspace_bytes": (_c.c_int64, [_c.c_int, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64]),
     "gguf_mmq_layer_unit": (_c.c_int, [_c.c_int, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64]),
+    "gguf_mmvq_linear_whole": (_c.c_int, [_c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_int, _c.c_void_p, _c.c_int64, _c.c_void_p, _c.c_int, _c.c_int64, _c.c_int64,
+                                          _c.c_int64, _c.c_void_p, _c.c_void_p]),
     "gguf_moe_mmq_layer_wide": (_c.c_int, [_c.c_int, _c.c_int, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64]),
     "gguf_moe_mmq_layer_finer": (_c.c_int, [_c.c_int, _c.c_int, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int]),
     "gguf_linear_walk": (_c.c_int, [_c.c_int, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64]),

@@ -21,6 +21,9 @@
  * gguf_moe_mmq_layer_finer: the block of 16 slots from which on the first or second product (product) of a layer on the streaming tiles deals K to
  * two waves each; -1: none, or a layer that they do not take.
  *
+ * gguf_mmvq_linear_whole: a call of gguf_mmvq_linear that needs no workspace, up to four rows which the GEMV quantizes by itself; taken = 0, and nothing is launched, for
+ * another (more rows; rows too long for its LDS).
+ *
  * gguf_linear_two: two products of the same x, up to 32 rows, as calls of gguf_mmvq_linear (gemv: bit 0 the first, bit 1 the second) or gguf_mmq_linear would run them
  * (the same results bit for bit), and for pairs of types that recipes mix in one launch: up to four rows of the GEMV, from five on behind the
  * quantizer's, which other pairs share too.  They are shards of a merged layer, columns of one result of this row pitch.  The workspace, M * gguf_q8_1_row_bytes(K), begins on 16 bytes.
@@ -39,6 +42,8 @@ int64_t gguf_mmq_layer_workspace_bytes(int type, int64_t N, int64_t K, int64_t M
 int gguf_moe_mmq_layer_finer(int type13, int type2, int64_t H, int64_t I, int64_t N_out, int64_t top_k, int64_t tokens, int64_t num_experts, int product);
 int gguf_moe_mmq_layer_wide(int type13, int type2, int64_t H, int64_t I, int64_t N_out, int64_t top_k, int64_t tokens, int64_t num_experts);
 int gguf_mmq_layer_unit(int type, int64_t N, int64_t K, int64_t M, int64_t w_row_pitch_bytes, int64_t workspace_bytes);
+int gguf_mmvq_linear_whole(const void* W, int64_t w_row_pitch_bytes, const void* x, int xdtype, void* Y, int64_t y_row_pitch, const void* bias, int type, int64_t N, int64_t K,
+                           int64_t M, void* stream, int* taken);
 int gguf_linear_two_takes(int type, int64_t N, int64_t w_row_pitch_bytes, int type2, int64_t N2, int64_t w_row_pitch_bytes2, int64_t K, int64_t M, int gemv);
 int gguf_linear_two(const void* W, int64_t w_row_pitch_bytes, int type, int64_t N, void* Y, const void* bias, const void* W2, int64_t w_row_pitch_bytes2, int type2,
                     int64_t N2, void* Y2, const void* bias2, const void* x, int xdtype, void* q8_workspace, int64_t y_row_pitch, int64_t K, int64_t M, int gemv, void* stream);

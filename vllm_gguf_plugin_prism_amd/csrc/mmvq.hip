@@ -1,6 +1,7 @@
 // C entry points of the decode-path GEMV and of the per-pair MoE GEMV.  The kernels live in mmvq_core.h and are
 // instantiated per group of formats in the mmvq_<group>.hip files; this file validates and routes by ggml type.
 #include "gguf_common.h"
+#include "dense_api.h"
 #include "tile_stream.h"
 
 namespace gguf {
@@ -45,7 +46,7 @@ int mmvq_any(int type, const void* W, const void* x, void* q8_workspace, void* Y
   // and both sides' times: ts_dense_takes).  The operator's workspace, the quantized rows, is what they want.
   const int64_t pitch = la.w_pitch ? la.w_pitch : K / block_elems(type) * block_bytes(type);
   if (!la.tile_sums && on16(q8_workspace) && ts_dense_takes(type, M, N, K, pitch, true))
-    return ts_dense(type, W, x, xdtype, q8_workspace, Y, M, (int)N, (int)K, true, la, s);
+    return !q8_workspace ? GGUF_NOT_TAKEN : ts_dense(type, W, x, xdtype, q8_workspace, Y, M, (int)N, (int)K, true, la, s);
   switch (type) {
     case T_Q4_0: return mmvq_group_std_a(type, W, x, q8_workspace, Y, xdtype, N, K, M, s, la);
     case T_Q4_1: return mmvq_group_std_a(type, W, x, q8_workspace, Y, xdtype, N, K, M, s, la);
@@ -71,10 +72,9 @@ int mmvq_any(int type, const void* W, const void* x, void* q8_workspace, void* Y
 }
 }  // namespace gguf
 
-extern "C" int gguf_mmvq_linear(const void* W, int64_t w_row_pitch_bytes, const void* x, int xdtype, void* q8_workspace, void* Y,
-                                int64_t y_row_pitch, const void* bias, int type, int64_t N, int64_t K, int64_t M,
-                                gguf_stream_t stream) {
-  using namespace gguf;
+namespace gguf {
+static int mmvq_linear(const void* W, int64_t w_row_pitch_bytes, const void* x, int xdtype, void* q8_workspace, bool whole, void* Y, int64_t y_row_pitch, const void* bias,
+                       int type, int64_t N, int64_t K, int64_t M, hipStream_t stream) {
   const int qk = block_elems(type);
   if (qk == 0) return GGUF_ERR_TYPE;
   if (N < 0 || M < 0 || K <= 0 || K % qk != 0 || N > 0x7FFFFFF0LL || K > 0x7FFFFFF0LL) return GGUF_ERR_SHAPE;
@@ -85,10 +85,25 @@ extern "C" int gguf_mmvq_linear(const void* W, int64_t w_row_pitch_bytes, const 
   la.bias = bias;
   if (xdtype < 0 || xdtype > 2) return GGUF_ERR_DTYPE;
   if (N == 0 || M == 0) return GGUF_OK;
-  if (!W || !x || !q8_workspace || !Y) return GGUF_ERR_NULL;
+  if (!W || !x || (!q8_workspace && !whole) || !Y) return GGUF_ERR_NULL;
   // packed blocks sit at even addresses (every block size is even): the GEMV's block loads rely on it
   if (((uintptr_t)W & 1) || (w_row_pitch_bytes & 1)) return GGUF_ERR_SHAPE;
-  return mmvq_any(type, W, x, q8_workspace, Y, xdtype, N, K, M, (hipStream_t)stream, la);
+  return mmvq_any(type, W, x, q8_workspace, Y, xdtype, N, K, M, stream, la);
+}
+}  // namespace gguf
+
+extern "C" int gguf_mmvq_linear(const void* W, int64_t w_row_pitch_bytes, const void* x, int xdtype, void* q8_workspace, void* Y,
+                                int64_t y_row_pitch, const void* bias, int type, int64_t N, int64_t K, int64_t M,
+                                gguf_stream_t stream) {
+  return gguf::mmvq_linear(W, w_row_pitch_bytes, x, xdtype, q8_workspace, false, Y, y_row_pitch, bias, type, N, K, M, (hipStream_t)stream);
+}
+
+extern "C" int gguf_mmvq_linear_whole(const void* W, int64_t w_row_pitch_bytes, const void* x, int xdtype, void* Y, int64_t y_row_pitch, const void* bias, int type, int64_t N,
+                                      int64_t K, int64_t M, void* stream, int* taken) {
+  using namespace gguf;
+  const int rc = M > 4 ? GGUF_NOT_TAKEN : mmvq_linear(W, w_row_pitch_bytes, x, xdtype, nullptr, true, Y, y_row_pitch, bias, type, N, K, M, (hipStream_t)stream);
+  *taken = rc != GGUF_NOT_TAKEN;
+  return *taken ? rc : GGUF_OK;
 }
 
 extern "C" int gguf_mmvq(const void* W, const void* x, int xdtype, void* q8_workspace, void* Y, int type, int64_t N,

@@ -1017,6 +1017,7 @@ static int mmvq_typed(const void* W, const void* x, void* ws, void* Y, int xdtyp
     }
     if (ok) return launch_status();
   }
+  if (!ws) return GGUF_NOT_TAKEN;                  // (gguf_mmvq_linear_whole; nothing has been launched)
   const int rc = quantize_q8_1(x, xdtype, ws, M, K, stream);
   if (rc != GGUF_OK) return rc;
   const int64_t rb = q8_row_bytes(K);

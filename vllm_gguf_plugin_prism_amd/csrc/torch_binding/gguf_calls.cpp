@@ -130,6 +130,12 @@ int run_shard(const Shard& s, const at::Tensor& x, int xcode, gguf_stream_t stre
     const c10::DataPtr ws = scratch(bytes);
     return gguf_dense_linear(s.w, s.pitch, x.const_data_ptr(), xcode, ws.get(), s.y, s.ldy, s.bias, s.type, s.rows, k, m, bytes, stream);
   }
+  // (scratch that no kernel of the call uses: host time of a call of [3072,1024] Q8_0, one row, with / without 4.11 / 3.82 us)
+  if (s.path == PATH_MMVQ) {
+    int taken;
+    const int rc = gguf_mmvq_linear_whole(s.w, s.pitch, x.const_data_ptr(), xcode, s.y, s.ldy, s.bias, s.type, s.rows, k, m, stream, &taken);
+    if (taken) return rc;
+  }
   const int64_t bytes = s.path == PATH_MMQ ? gguf_mmq_layer_workspace_bytes(s.type, s.rows, k, m, s.pitch) : m * gguf_q8_1_row_bytes(k);
   const c10::DataPtr ws = scratch(bytes);
   if (s.path == PATH_MMVQ)
