@@ -28,3 +28,18 @@ def test_bits_of_the_call_with_a_workspace(qtype, m, n, k, taken, dt):
         assert torch.equal(y[:, :n], ops.ggml_mul_mat_vec_a8(w, x, qtype, n, bias=bias))
     else:
         assert bool((y == 7.0).all())
+
+
+# rows handed out to half-waves, whose addresses move on by a turn's rows: a last band that is a row short, two turns and twelve, the kernel of eight waves;
+# tables of 256 to 2048 entries placed by 1024 threads and by 512
+@pytest.mark.parametrize("qtype", (o.IQ2_XXS, o.IQ2_S, o.IQ3_S, o.IQ1_S, o.IQ1_M, o.Q4_0, o.Q8_0))
+@pytest.mark.parametrize("n,k", [(2831, 5120), (2555, 3072), (17401, 1024), (100, 512)])
+def test_half_waves_and_tables(qtype, n, k):
+    from vllm_gguf_plugin_prism_amd import ops
+    rng = np.random.default_rng(n)
+    w = o.make_weights(rng, qtype, n, k)
+    x = rng.standard_normal((1, k)).astype(np.float32)
+    rows = np.r_[:12, n // 2:n // 2 + 24, n - 24:n]
+    y = ops.ggml_mul_mat_vec_a8(torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda(), qtype, n).cpu().numpy()
+    # (fp32 sums of K / 32 block products in another order: 1e-5 of their norm, the tolerance of the GEMV's other tests)
+    assert np.isfinite(y).all() and o.rel_l2(y[:, rows], o.mul_mat_a8(w[rows], x, qtype, len(rows), "mmvq")) <= 1e-5

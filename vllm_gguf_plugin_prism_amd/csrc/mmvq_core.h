@@ -401,6 +401,32 @@ static inline StreamGeom stream_geom(int N, int K, int rows_per_wg, int64_t w_pi
   return g;
 }
 
+// The codes of a format's table in registers, a thread's share (formats without a table: nothing)
+template <class F, int NT, bool TABLE = (F::TABLE_BYTES > 0)> struct TableCodes {
+  struct Codes {};
+  static __device__ __forceinline__ void fetch(Codes&, int) {}
+  static __device__ __forceinline__ void place(const Codes&, char*, int) {}
+};
+template <class F, int NT> struct TableCodes<F, NT, true> {
+  static constexpr int N = (F::CODES + NT - 1) / NT;
+  struct Codes { uint32_t c[N]; };
+  static __device__ __forceinline__ void fetch(Codes& k, int tid) {
+    typedef const __attribute__((address_space(1))) uint16_t* Global;
+    Global codes = (Global)F::codes();
+    asm volatile("" : "+s"(codes));               // (not known to be constant, and the memory clobbered behind: the loads stay here)
+#pragma unroll
+    for (int i = 0; i < N; ++i) k.c[i] = codes[min(tid + NT * i, F::CODES - 1)];
+    asm volatile("" ::: "memory");
+  }
+  static __device__ __forceinline__ void place(const Codes& k, char* tab, int tid) {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (tid + NT * i < F::CODES) F::grid_entry(tab, tid + NT * i, k.c[i]);
+    static_assert(F::SIGNS <= NT, "a sign mask per thread");
+    if (tid < F::SIGNS) F::sign_entry(tab, tid);
+  }
+};
+
 // GATED (one activation row only): the row of X is [gate | up], K values each, and what is quantized is
 // T(T(act(gate)) * up), the values a separate act-and-multiply kernel would have stored (fused_moe.py:44-51,80).
 template <class F, int MT, int NW, int D, typename T, bool TILE, bool FULL, int STAGED, bool GATED>
@@ -415,11 +441,12 @@ __device__ __forceinline__ void mmvq_stream_body(const uint8_t* __restrict__ W, 
   const int nb = K >> 5;                       // 32-weight units per row
   const int S = geom.S();                      // waves per row
   const int slots = geom.slots();              // rows in flight side by side (>= 1, checked by the host)
-  int8_t* lq = (int8_t*)smem;                  // [MT][K]
-  float* ldv = (float*)(smem + (size_t)MT * K);  // [MT][nb]
+  static_assert(F::TABLE_BYTES % 16 == 0, "what lies behind the table");
+  char* tab = smem;                            // (in front: an entry's address is its number's alone, the table's an immediate)
+  int8_t* lq = (int8_t*)smem + F::TABLE_BYTES; // [MT][K]
+  float* ldv = (float*)(smem + F::TABLE_BYTES + (size_t)MT * K);  // [MT][nb]
   float* lav = ldv + MT * nb;                  // [MT][nb]
-  char* tab = (char*)(lav + (F::AUX != AUX_NONE ? MT * nb : 0));
-  float* part = (float*)(tab + F::TABLE_BYTES);  // [rows_per_wg][S][4 (HALF: 2) groups of 16 lanes][MT]
+  float* part = lav + (F::AUX != AUX_NONE ? MT * nb : 0);  // [rows_per_wg][S][4 (HALF: 2) groups of 16 lanes][MT]
   constexpr bool HALF = STAGED == LANES_HALF, SPANS = STAGED != 0 && !HALF, DMA = STAGED == STAGED_DMA;
   constexpr int SPAN = SPANS ? SpanOf<F>::value : 0;
 
@@ -440,10 +467,12 @@ __device__ __forceinline__ void mmvq_stream_body(const uint8_t* __restrict__ W, 
   const bool lane_on = wave_on && u_raw < nb;
   const int u = min(u_raw, nb - 1);
 
-  if (F::TABLE_BYTES > 0) {
-    F::init_tables(tab);
-    __syncthreads();
-  }
+  // The codes of the format's table are asked for first of all, and its entries are placed once the first weights are on their way: filling it before they were
+  // asked for cost the time of a trip to memory (one row: IQ2_XXS [17408,5120] 9.52 / 9.10 us, IQ3_XXS [5120,5120] 6.5 / 5.9, IQ3_S [4096,4096]
+  // 5.5 / 4.8, IQ1_S [14336,4096] 7.4 / 6.75).
+  constexpr int NT = 64 * NW;
+  typename TableCodes<F, NT>::Codes codes;
+  TableCodes<F, NT>::fetch(codes, tid);
 
   // Loads are issued unconditionally (row index clamped into the band) so that every iteration issues the
   // same number of loads and the hardware load counter can be waited on exactly, slot by slot.
@@ -453,7 +482,21 @@ __device__ __forceinline__ void mmvq_stream_body(const uint8_t* __restrict__ W, 
   const int span_bytes = STAGED == STAGED_ALIGNED || DMA ? SPAN : SPANS ? max(16, min(SPAN, (K / F::QK) * F::BS - (wave_on ? step : 0) * SPAN)) : 0;
   typedef SpanRegs<SPANS ? SPAN : 16, ANY> Span;
   [[maybe_unused]] uint32_t mis[D];   // ANY: where in its first 16-byte piece the stretch of each row in flight starts
+  // HALF: the row is a lane's, and a product of 64 bits for it on every turn is a tenth of the loop (two multiplications at a quarter of the rate, five
+  // more instructions; IQ2_XXS [17408,5120] 9.66 / 9.52 us): the address moves on by one turn's rows while there is another, and stays where there is none.
+  const int below = wave_on ? nrows - slot : 0;   // (rows from this slot on)
+  [[maybe_unused]] const uint8_t* at = wbase + (uint64_t)(uint32_t)min(slot, nrows - 1) * (uint32_t)rowbytes;
+  [[maybe_unused]] int next = slots;
   auto load_row = [&](int i, [[maybe_unused]] uint32_t& m16) {
+    if constexpr (HALF) {                         // (called once for each i, in order)
+      const auto r = F::load(at, 0, u, tab);
+      const uint64_t turn = (uint64_t)(uint32_t)slots * (uint32_t)rowbytes;
+      uint32_t lo = next < below ? (uint32_t)turn : 0u, hi = next < below ? (uint32_t)(turn >> 32) : 0u;
+      asm volatile("" : "+v"(lo), "+v"(hi));      // (opaque: the compiler would branch around the load of a row that is the same again, and wait for the one before)
+      at += (uint64_t)hi << 32 | lo;
+      next += slots;
+      return r;
+    } else {
     const int row = min(slot + slots * i, nrows - 1);
     if constexpr (SPANS) {   // (the host takes this variant only for rows it can fetch as whole 16-byte pieces)
       Span r;
@@ -469,6 +512,7 @@ __device__ __forceinline__ void mmvq_stream_body(const uint8_t* __restrict__ W, 
       return r;
     } else {
       return F::load(wbase + (int64_t)row * rowbytes, 0, u, tab);
+    }
     }
   };
   // this wave's staging area for one span (DMA: a ring of D), behind the partial sums
@@ -496,7 +540,6 @@ __device__ __forceinline__ void mmvq_stream_body(const uint8_t* __restrict__ W, 
   // then the weights of the first D rows, then quantize the activations into LDS (four lanes per 32-value
   // block) while the weights fly.  The activation loads go first so that waiting for them does not also
   // wait for the weight loads behind them.  Groups past the end are clamped and their stores predicated.
-  constexpr int NT = 64 * NW;
   const int g8 = K >> 3;
   // FULL: all MT rows of the tile exist (m_act == MT), known at compile time.  Otherwise rows m_act .. MT-1 are
   // computed on whatever the LDS holds and never stored.
@@ -551,6 +594,7 @@ __device__ __forceinline__ void mmvq_stream_body(const uint8_t* __restrict__ W, 
       first_rows(on_tag);
       __builtin_amdgcn_sched_barrier(0);
       GGUF_PHASE(7);
+      TableCodes<F, NT>::place(codes, tab, tid);
       return;
     }
     raw8<T> xraw[QG > 0 ? QG : 1], xup[GATED && QG > 0 ? QG : 1];
@@ -592,6 +636,7 @@ __device__ __forceinline__ void mmvq_stream_body(const uint8_t* __restrict__ W, 
         if constexpr (GATED) xup[g].hold();
       }
     }
+    TableCodes<F, NT>::place(codes, tab, tid);   // (here, where the compiler knows how many loads are younger)
 #pragma unroll
     for (int g = 0; g < QG; ++g) quantize_group(xraw[g], xup[GATED ? g : 0], tid + g * NT);
   };
@@ -619,7 +664,6 @@ __device__ __forceinline__ void mmvq_stream_body(const uint8_t* __restrict__ W, 
   __syncthreads();
   GGUF_PHASE(2);                               // every wave's share is in LDS
   // (the two quotients below are the kernel's only divisions; here they run while the first weights are still on their way)
-  const int my_rows = wave_on && nrows > slot ? (nrows - slot + slots - 1) / slots : 0;  // rows slot, slot+slots, ...
   const int max_rows = (nrows + slots - 1) / slots;  // trip count of the row loop, same for every wave
 
   // this lane's column of every activation vector, held in registers for the whole row loop
@@ -664,7 +708,7 @@ __device__ __forceinline__ void mmvq_stream_body(const uint8_t* __restrict__ W, 
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         dma_row(i + D, r);
       }
-      finish_row(cur, i, i < my_rows);
+      finish_row(cur, i, slots * i < below);
       r = r + 1 == D ? 0 : r + 1;
     }
   }
@@ -673,7 +717,7 @@ __device__ __forceinline__ void mmvq_stream_body(const uint8_t* __restrict__ W, 
 #pragma unroll
     for (int d = 0; d < D; ++d) {
       const int i = i0 + d;
-      const bool row_ok = i < my_rows;
+      const bool row_ok = slots * i < below;
       float acc[MT];
       typename F::Regs cur;
       if constexpr (SPANS) {

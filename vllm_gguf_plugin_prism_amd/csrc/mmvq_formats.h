@@ -279,32 +279,56 @@ struct FmtIQ4_XS {
   }
 };
 
+// The tables of the grid formats in LDS.  A format has CODES entries, each from a code of 16 bits (codes()), and SIGNS sign masks of eight bytes: grid_entry(table, t, code) and
+// sign_entry place one.  init_tables does it in one go; the streaming GEMV asks for the codes before anything else and places the entries while its
+// first weights are on their way (mmvq_core.h).
+__device__ __forceinline__ uint2 sign_mask(int t, int count) {  // 128: 7 bits + parity bit; 256: plain byte
+  const uint32_t sg = count == 128 ? (uint32_t)t | ((__builtin_popcount(t) & 1) << 7) : (uint32_t)t;
+  uint32_t m[2] = {0, 0};
+#pragma unroll
+  for (int j = 0; j < 8; ++j) m[j >> 2] |= ((sg >> j) & 1 ? 0xFFu : 0u) << (8 * (j & 3));
+  return make_uint2(m[0], m[1]);
+}
+__device__ __forceinline__ uint2 grid2_of(uint32_t code) {  // 8 magnitudes {8,25,43}
+  uint32_t w[2] = {0, 0};
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const uint32_t c = (code >> (2 * j)) & 3;
+    w[j >> 2] |= (8 + 17 * c + (c >> 1)) << (8 * (j & 3));
+  }
+  return make_uint2(w[0], w[1]);
+}
+__device__ __forceinline__ uint32_t grid3_of(uint32_t code, bool xxs) {  // 4 magnitudes
+  uint32_t w = 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t c = (code >> (3 * j)) & 7;
+    w |= (4 + 8 * c + (xxs ? 2 * ((c + 1) >> 3) : 0)) << (8 * j);
+  }
+  return w;
+}
+__device__ __forceinline__ uint32_t grid1_of(uint32_t code) {  // eight values {0,1,2}, value j in nibble j
+  uint32_t w = 0;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) w |= ((code >> (2 * j)) & 3) << (4 * j);
+  return w;
+}
+template <class F>
+__device__ __forceinline__ void fill_tables(char* tab) {
+  for (int t = threadIdx.x; t < F::CODES; t += blockDim.x) F::grid_entry(tab, t, F::codes()[t]);
+  for (int t = threadIdx.x; t < F::SIGNS; t += blockDim.x) F::sign_entry(tab, t);
+}
+
 // ------------------------------------------------------------------ IQ2_XXS (vecdotq.cuh:1531-1552)
 // LDS tables: the 256-entry grid expanded to 8 magnitudes per entry, and the 128 sign patterns as byte masks.
 struct FmtIQ2_XXS {
   static constexpr int QK = 256, BS = 66, AUX = AUX_NONE, TABLE_BYTES = 256 * 8 + 128 * 8;
   struct Regs { uint16_t d; uint2 g; };
-  static __device__ __forceinline__ void init_tables(char* tab) {
-    uint2* grid = (uint2*)tab;
-    uint2* sgn = grid + 256;
-    for (int t = threadIdx.x; t < 256; t += blockDim.x) {
-      const uint32_t code = k_iq2xxs_grid_codes[t];
-      uint32_t w[2] = {0, 0};
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const uint32_t c = (code >> (2 * j)) & 3;
-        w[j >> 2] |= (8 + 17 * c + (c >> 1)) << (8 * (j & 3));
-      }
-      grid[t] = make_uint2(w[0], w[1]);
-      if (t < 128) {
-        const uint32_t sg = t | ((__builtin_popcount(t) & 1) << 7);
-        uint32_t m[2] = {0, 0};
-#pragma unroll
-        for (int j = 0; j < 8; ++j) m[j >> 2] |= ((sg >> j) & 1 ? 0xFFu : 0u) << (8 * (j & 3));
-        sgn[t] = make_uint2(m[0], m[1]);
-      }
-    }
-  }
+  static constexpr int CODES = 256, SIGNS = 128;
+  static __device__ __forceinline__ const uint16_t* codes() { return k_iq2xxs_grid_codes; }
+  static __device__ __forceinline__ void grid_entry(char* tab, int t, uint32_t code) { ((uint2*)tab)[t] = grid2_of(code); }
+  static __device__ __forceinline__ void sign_entry(char* tab, int t) { ((uint2*)(tab + CODES * 8))[t] = sign_mask(t, SIGNS); }
+  static __device__ __forceinline__ void init_tables(char* tab) { fill_tables<FmtIQ2_XXS>(tab); }
   static __device__ __forceinline__ Regs load(const uint8_t* row, int u0, int u, const char*) {
     const int uu = u0 + u, sb = uu >> 3, ib = uu & 7;
     const uint8_t* b = row + (int64_t)sb * BS;
@@ -341,50 +365,6 @@ struct FmtIQ2_XXS {
 // ================================================================== the other thirteen formats
 // bits 0..3 of b -> bit 0 of bytes 0..3 (the four partial products never share a bit, so nothing carries)
 __device__ __forceinline__ uint32_t spread4(uint32_t b) { return ((b & 0xFu) * 0x00204081u) & 0x01010101u; }
-
-// LDS table fillers shared by the grid formats
-__device__ __forceinline__ void fill_sign_masks(uint2* sgn, int count) {  // 128: 7 bits + parity bit; 256: plain byte
-  for (int t = threadIdx.x; t < count; t += blockDim.x) {
-    const uint32_t sg = count == 128 ? (uint32_t)t | ((__builtin_popcount(t) & 1) << 7) : (uint32_t)t;
-    uint32_t m[2] = {0, 0};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) m[j >> 2] |= ((sg >> j) & 1 ? 0xFFu : 0u) << (8 * (j & 3));
-    sgn[t] = make_uint2(m[0], m[1]);
-  }
-}
-__device__ __forceinline__ void fill_grid2(uint2* grid, const uint16_t* codes, int count) {  // 8 magnitudes {8,25,43}
-  for (int t = threadIdx.x; t < count; t += blockDim.x) {
-    const uint32_t code = codes[t];
-    uint32_t w[2] = {0, 0};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const uint32_t c = (code >> (2 * j)) & 3;
-      w[j >> 2] |= (8 + 17 * c + (c >> 1)) << (8 * (j & 3));
-    }
-    grid[t] = make_uint2(w[0], w[1]);
-  }
-}
-__device__ __forceinline__ void fill_grid3(uint32_t* grid, const uint16_t* codes, int count, bool xxs) {  // 4 magnitudes
-  for (int t = threadIdx.x; t < count; t += blockDim.x) {
-    const uint32_t code = codes[t];
-    uint32_t w = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t c = (code >> (3 * j)) & 7;
-      w |= (4 + 8 * c + (xxs ? 2 * ((c + 1) >> 3) : 0)) << (8 * j);
-    }
-    grid[t] = w;
-  }
-}
-__device__ __forceinline__ void fill_grid1(uint32_t* grid) {  // eight values {0,1,2}, value j in nibble j
-  for (int t = threadIdx.x; t < 2048; t += blockDim.x) {
-    const uint32_t code = k_iq1s_grid_gpu_codes[t];
-    uint32_t w = 0;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) w |= ((code >> (2 * j)) & 3) << (4 * j);
-    grid[t] = w;
-  }
-}
 
 // activations of a unit that is one whole q8_1 block: 32 quants, the block scale and one extra per-block value
 struct ActBlock32 { int2 a[4]; float d, s; const char* tab; };
@@ -665,10 +645,11 @@ struct FmtQ5_K {
 struct FmtIQ2_XS {
   static constexpr int QK = 256, BS = 74, AUX = AUX_NONE, TABLE_BYTES = 512 * 8 + 128 * 8;
   struct Regs { uint2 q; uint16_t d; uint8_t sc; };
-  static __device__ __forceinline__ void init_tables(char* tab) {
-    fill_grid2((uint2*)tab, k_iq2xs_grid_codes, 512);
-    fill_sign_masks((uint2*)tab + 512, 128);
-  }
+  static constexpr int CODES = 512, SIGNS = 128;
+  static __device__ __forceinline__ const uint16_t* codes() { return k_iq2xs_grid_codes; }
+  static __device__ __forceinline__ void grid_entry(char* tab, int t, uint32_t code) { ((uint2*)tab)[t] = grid2_of(code); }
+  static __device__ __forceinline__ void sign_entry(char* tab, int t) { ((uint2*)(tab + CODES * 8))[t] = sign_mask(t, SIGNS); }
+  static __device__ __forceinline__ void init_tables(char* tab) { fill_tables<FmtIQ2_XS>(tab); }
   static __device__ __forceinline__ Regs load(const uint8_t* row, int u0, int u, const char*) {
     const int uu = u0 + u, sb = uu >> 3, ib = uu & 7;
     const uint8_t* b = row + (int64_t)sb * BS;
@@ -696,10 +677,11 @@ struct FmtIQ2_XS {
 struct FmtIQ2_S {
   static constexpr int QK = 256, BS = 82, AUX = AUX_NONE, TABLE_BYTES = 1024 * 8 + 256 * 8;
   struct Regs { uint32_t q, sg; uint16_t d; uint8_t qh, sc; };
-  static __device__ __forceinline__ void init_tables(char* tab) {
-    fill_grid2((uint2*)tab, k_iq2s_grid_codes, 1024);
-    fill_sign_masks((uint2*)tab + 1024, 256);
-  }
+  static constexpr int CODES = 1024, SIGNS = 256;
+  static __device__ __forceinline__ const uint16_t* codes() { return k_iq2s_grid_codes; }
+  static __device__ __forceinline__ void grid_entry(char* tab, int t, uint32_t code) { ((uint2*)tab)[t] = grid2_of(code); }
+  static __device__ __forceinline__ void sign_entry(char* tab, int t) { ((uint2*)(tab + CODES * 8))[t] = sign_mask(t, SIGNS); }
+  static __device__ __forceinline__ void init_tables(char* tab) { fill_tables<FmtIQ2_S>(tab); }
   static __device__ __forceinline__ Regs load(const uint8_t* row, int u0, int u, const char*) {
     const int uu = u0 + u, sb = uu >> 3, ib = uu & 7;
     const uint8_t* b = row + (int64_t)sb * BS;
@@ -729,10 +711,11 @@ struct FmtIQ2_S {
 struct FmtIQ3_XXS {
   static constexpr int QK = 256, BS = 98, AUX = AUX_NONE, TABLE_BYTES = 256 * 4 + 128 * 8;
   struct Regs { uint2 q; uint32_t aux; uint16_t d; };
-  static __device__ __forceinline__ void init_tables(char* tab) {
-    fill_grid3((uint32_t*)tab, k_iq3xxs_grid_codes, 256, true);
-    fill_sign_masks((uint2*)(tab + 256 * 4), 128);
-  }
+  static constexpr int CODES = 256, SIGNS = 128;
+  static __device__ __forceinline__ const uint16_t* codes() { return k_iq3xxs_grid_codes; }
+  static __device__ __forceinline__ void grid_entry(char* tab, int t, uint32_t code) { ((uint32_t*)tab)[t] = grid3_of(code, true); }
+  static __device__ __forceinline__ void sign_entry(char* tab, int t) { ((uint2*)(tab + CODES * 4))[t] = sign_mask(t, SIGNS); }
+  static __device__ __forceinline__ void init_tables(char* tab) { fill_tables<FmtIQ3_XXS>(tab); }
   static __device__ __forceinline__ Regs load(const uint8_t* row, int u0, int u, const char*) {
     const int uu = u0 + u, sb = uu >> 3, ib = uu & 7;
     const uint8_t* b = row + (int64_t)sb * BS;
@@ -759,10 +742,11 @@ struct FmtIQ3_XXS {
 struct FmtIQ3_S {
   static constexpr int QK = 256, BS = 110, AUX = AUX_NONE, TABLE_BYTES = 512 * 4 + 256 * 8;
   struct Regs { uint2 q; uint32_t sg; uint16_t d; uint8_t qh, sc; };
-  static __device__ __forceinline__ void init_tables(char* tab) {
-    fill_grid3((uint32_t*)tab, k_iq3xs_grid_codes, 512, false);
-    fill_sign_masks((uint2*)(tab + 512 * 4), 256);
-  }
+  static constexpr int CODES = 512, SIGNS = 256;
+  static __device__ __forceinline__ const uint16_t* codes() { return k_iq3xs_grid_codes; }
+  static __device__ __forceinline__ void grid_entry(char* tab, int t, uint32_t code) { ((uint32_t*)tab)[t] = grid3_of(code, false); }
+  static __device__ __forceinline__ void sign_entry(char* tab, int t) { ((uint2*)(tab + CODES * 4))[t] = sign_mask(t, SIGNS); }
+  static __device__ __forceinline__ void init_tables(char* tab) { fill_tables<FmtIQ3_S>(tab); }
   static __device__ __forceinline__ Regs load(const uint8_t* row, int u0, int u, const char*) {
     const int uu = u0 + u, sb = uu >> 3, ib = uu & 7;
     const uint8_t* b = row + (int64_t)sb * BS;
@@ -794,7 +778,11 @@ struct FmtIQ3_S {
 struct FmtIQ1_S {
   static constexpr int QK = 256, BS = 50, AUX = AUX_S8, TABLE_BYTES = 2048 * 4;
   struct Regs { uint32_t q; uint16_t d, qh; };
-  static __device__ __forceinline__ void init_tables(char* tab) { fill_grid1((uint32_t*)tab); }
+  static constexpr int CODES = 2048, SIGNS = 0;
+  static __device__ __forceinline__ const uint16_t* codes() { return k_iq1s_grid_gpu_codes; }
+  static __device__ __forceinline__ void grid_entry(char* tab, int t, uint32_t code) { ((uint32_t*)tab)[t] = grid1_of(code); }
+  static __device__ __forceinline__ void sign_entry(char* tab, int t) {  }
+  static __device__ __forceinline__ void init_tables(char* tab) { fill_tables<FmtIQ1_S>(tab); }
   static __device__ __forceinline__ Regs load(const uint8_t* row, int u0, int u, const char*) {
     const int uu = u0 + u, sb = uu >> 3, ib = uu & 7;
     const uint8_t* b = row + (int64_t)sb * BS;
@@ -823,7 +811,11 @@ struct FmtIQ1_S {
 struct FmtIQ1_M {
   static constexpr int QK = 256, BS = 56, AUX = AUX_NONE, TABLE_BYTES = 2048 * 4;
   struct Regs { uint32_t q; uint2 sc; uint16_t qh; };
-  static __device__ __forceinline__ void init_tables(char* tab) { fill_grid1((uint32_t*)tab); }
+  static constexpr int CODES = 2048, SIGNS = 0;
+  static __device__ __forceinline__ const uint16_t* codes() { return k_iq1s_grid_gpu_codes; }
+  static __device__ __forceinline__ void grid_entry(char* tab, int t, uint32_t code) { ((uint32_t*)tab)[t] = grid1_of(code); }
+  static __device__ __forceinline__ void sign_entry(char* tab, int t) {  }
+  static __device__ __forceinline__ void init_tables(char* tab) { fill_tables<FmtIQ1_M>(tab); }
   static __device__ __forceinline__ Regs load(const uint8_t* row, int u0, int u, const char*) {
     const int uu = u0 + u, sb = uu >> 3, ib = uu & 7;
     const uint8_t* b = row + (int64_t)sb * BS;
