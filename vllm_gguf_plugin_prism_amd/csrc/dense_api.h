@@ -17,7 +17,7 @@
  * gguf_linear_walk: where a call of more than 32 rows with a workspace of this size runs tile_walk_kernel, which comes before them too, 16 times the tiles of
  * 32 rows that a workgroup has and its waves, else 0 (of weights that begin on 16 bytes: others of Q8_0 may run otherwise).
  * gguf_mmq_layer_unit: the kernel of gguf_mmq_layer_route, with 2 added to 1 (past 32 rows) and 4 where the half-precision unit would run a call that these decline.  gguf_moe_mmq_layer_wide: whether
- * gguf_moe_mmq_layer with the workspace it asks for, at addresses divisible by 16, runs on the wide tiles.
+ * gguf_moe_mmq_layer with the workspace it asks for, at addresses divisible by 16, runs on the expert and the wide tiles.
  * gguf_moe_mmq_layer_finer: the block of 16 slots from which on the first or second product (product) of a layer on the streaming tiles deals K to
  * two waves each; -1: none, or a layer that they do not take.
  *
