@@ -482,13 +482,14 @@ __device__ __forceinline__ void mmvq_stream_body(const uint8_t* __restrict__ W, 
   const int span_bytes = STAGED == STAGED_ALIGNED || DMA ? SPAN : SPANS ? max(16, min(SPAN, (K / F::QK) * F::BS - (wave_on ? step : 0) * SPAN)) : 0;
   typedef SpanRegs<SPANS ? SPAN : 16, ANY> Span;
   [[maybe_unused]] uint32_t mis[D];   // ANY: where in its first 16-byte piece the stretch of each row in flight starts
-  // HALF: the row is a lane's, and a product of 64 bits for it on every turn is a tenth of the loop (two multiplications at a quarter of the rate, five
-  // more instructions; IQ2_XXS [17408,5120] 9.66 / 9.52 us): the address moves on by one turn's rows while there is another, and stays where there is none.
+  // HALF: the row is a lane's, and a product of 64 bits for it on every turn is a tenth of a codebook format's loop (two multiplications at a quarter of the rate, five
+  // more instructions; IQ2_XXS [17408,5120] 9.66 / 9.52 us): there the address moves on by one turn's rows while there is another, and stays where there is none.
+  // (The other formats wait for memory and not for this: no change.)
   const int below = wave_on ? nrows - slot : 0;   // (rows from this slot on)
   [[maybe_unused]] const uint8_t* at = wbase + (uint64_t)(uint32_t)min(slot, nrows - 1) * (uint32_t)rowbytes;
   [[maybe_unused]] int next = slots;
   auto load_row = [&](int i, [[maybe_unused]] uint32_t& m16) {
-    if constexpr (HALF) {                         // (called once for each i, in order)
+    if constexpr (HALF && F::TABLE_BYTES > 0) {                         // (called once for each i, in order)
       const auto r = F::load(at, 0, u, tab);
       const uint64_t turn = (uint64_t)(uint32_t)slots * (uint32_t)rowbytes;
       uint32_t lo = next < below ? (uint32_t)turn : 0u, hi = next < below ? (uint32_t)(turn >> 32) : 0u;
@@ -664,6 +665,7 @@ __device__ __forceinline__ void mmvq_stream_body(const uint8_t* __restrict__ W, 
   __syncthreads();
   GGUF_PHASE(2);                               // every wave's share is in LDS
   // (the two quotients below are the kernel's only divisions; here they run while the first weights are still on their way)
+  const int my_rows = wave_on && nrows > slot ? (nrows - slot + slots - 1) / slots : 0;  // rows slot, slot+slots, ...
   const int max_rows = (nrows + slots - 1) / slots;  // trip count of the row loop, same for every wave
 
   // this lane's column of every activation vector, held in registers for the whole row loop
@@ -708,7 +710,7 @@ __device__ __forceinline__ void mmvq_stream_body(const uint8_t* __restrict__ W, 
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         dma_row(i + D, r);
       }
-      finish_row(cur, i, slots * i < below);
+      finish_row(cur, i, i < my_rows);
       r = r + 1 == D ? 0 : r + 1;
     }
   }
@@ -717,7 +719,7 @@ __device__ __forceinline__ void mmvq_stream_body(const uint8_t* __restrict__ W, 
 #pragma unroll
     for (int d = 0; d < D; ++d) {
       const int i = i0 + d;
-      const bool row_ok = slots * i < below;
+      const bool row_ok = i < my_rows;
       float acc[MT];
       typename F::Regs cur;
       if constexpr (SPANS) {
