@@ -50,3 +50,10 @@ def scratch():
 def test_nothing_goes_to_scratch(kernel, scratch):
     of = {name: n for name, n in scratch.items() if f"{len(kernel)}{kernel}I" in name}   # (mangled: length, name, template arguments)
     assert of and not {name: n for name, n in of.items() if n and not any(e in name for e in EXCEPT)}
+
+
+# the tile of the matrix instruction, a property of the format (measured: csrc/mmq_f_core.h)
+@pytest.mark.parametrize("fmt,tile", [("5FQ4_K", 32), ("5FQ5_K", 32), ("5FQ6_K", 16)])
+def test_tile_of_the_prefill_gemm(fmt, tile, scratch):
+    of = [name for name in scratch if "11mmqf_kernelI" in name and fmt in name]
+    assert of and all(f"Li{tile}E" in name for name in of)

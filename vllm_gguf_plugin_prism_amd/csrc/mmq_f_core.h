@@ -9,16 +9,16 @@
 // covers 16 values: 41 to 90 ns per 32 x 32 x 32 block and SIMD at full rate, of which the matrix unit needs 14.  Here the
 // integer scale sc goes into the weight operand.  sc * q is a whole number of at most 11 bits (Q4_K 63 * 15, Q5_K
 // 63 * 31), which half precision holds exactly; so are the quants of X; and the block's sum stays below 2^24, so the fp32
-// accumulator of v_mfma_f32_16x16x32_f16 holds it exactly, too, and hands it over as a float.  One multiply-add per result
+// accumulator of v_mfma_f32_32x32x16_f16 (Q6_K 16x16x32) holds it exactly, too, and hands it over as a float.  One multiply-add per result
 // and block is left (by d8, which is one register: a lane holds one row of X), and one per result and super-block for d:
-// 34 ns per 32 x 32 x 32 block.  Q6_K's products have 12 bits and a sign: two operands, the product rounded to half precision and what that
+// 34 ns per 32 x 32 x 32 block by that count at the full clock, 48 to 56 as measured (below).  Q6_K's products have 12 bits and a sign: two operands, the product rounded to half precision and what that
 // leaves out, -1, 0 or 1 and hardly ever not 0: a matrix unit that multiplies zeros draws less, and the clock gives way less ([18944,3584] 512
 // rows 150 us with the operands q * (sc & ~15) and q * (sc & 15), 144 so).
 // The offset term is a contraction over the eight blocks of a super-block of exact halves (the mins are 6-bit whole
 // numbers, the stored sums are halves): one more matrix instruction per super-block.
 //
-// Work split: workgroup tiles of 256 rows of X by 128 weight rows, eight waves of 64 x 64 (sixteen accumulators of 16 x 16,
-// each twice: the super-block's sum and the total).  K in steps of 64: the rows of X (whole numbers in half precision,
+// Work split: workgroup tiles of 256 rows of X by 128 weight rows, eight waves of 64 x 64 (four accumulators of 32 x 32, Q6_K sixteen of
+// 16 x 16, each twice: the super-block's sum and the total).  K in steps of 64: the rows of X (whole numbers in half precision,
 // written by the quantizer) go straight to LDS (global_load_lds, 16-byte pieces, the piece number xored with the row's so
 // that the operand reads meet all banks), the packed weights of the next step through registers, decoded once per
 // workgroup.  Two buffers, one barrier per step.  Whole rounds of tiles have a workgroup per tile; the super-blocks of the
@@ -38,8 +38,10 @@
 // contraction alone, matrix instructions and multiply-adds in registers, takes a SIMD 48 to 56 ns per 32 x 32 x 32 block of one operand at any
 // interleaving (one wave or two, bursts of one to four blocks): vector instructions hide behind matrix instructions only in part, and the clock falls as
 // both get denser.  Of two operands it takes 82 to 86 ns on tiles of 32 x 32 and 71 on tiles of 16 x 16, whose results need half the registers
-// on the way: Q6_K [18944,3584] 512 rows 156 -> 150 us, [4096,14336] 1531 rows 390 -> 374 (Q4_K and Q5_K 0.5 % slower).  A unit's matrix instructions are
-// issued two units ahead of its multiply-adds (one ahead: 155 us, three: no change).
+// on the way: Q6_K [18944,3584] 512 rows 156 -> 150 us, [4096,14336] 1531 rows 390 -> 374.  There a unit's matrix instructions are
+// issued two units ahead of its multiply-adds (one ahead: 155 us, three: no change).  One operand is faster on tiles of 32 x 32: [4096,14336] Q4_K 2100 / 3000 rows 405 / 550 us,
+// on tiles of 16 x 16 418 / 578, Q5_K 430 / 576 and 446 / 588; 80 random products of 1000 to 4096 rows 1.012 times as fast on average, 1.05 the most,
+// [4096,4096] 2500 rows 0.98.
 // Tried and slower: four waves per workgroup and two workgroups per CU (decoding twice), the two waves of a SIMD decoding at
 // different times, the fetches of X in front of the operand reads or spread over the step; the barrier in the middle of a step
 // and the next step's operands behind it, so that no step begins with waiting (same bits, 299 -> 316 us, Q6_K 170 -> 190).
@@ -51,6 +53,7 @@ namespace gguf {
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x2_m __attribute__((ext_vector_type(2)));
 
 // Whole numbers x below 1024 as the halves 1024 + x: the bits `mask` of both halves of v (`magic`, 0x64006400, in a vector register,
@@ -76,7 +79,7 @@ __device__ __forceinline__ f16x2 twice(_Float16 v) { return (f16x2){v, v}; }
 //   Head     what it takes from the super-block's header, loaded once per super-block; Scales: the same, unpacked
 //   PLANES   operands per weight;  OFF: the format has mins
 struct FQ4_K {
-  static constexpr int BS = 144, PLANES = 1;
+  static constexpr int BS = 144, PLANES = 1, TILE = 32;
   static constexpr bool OFF = true;
   struct Head { uint4 h; };
   struct Scales { uint32_t s[2]; };
@@ -144,7 +147,7 @@ struct FQ5_K : FQ4_K {   // Q4_K with a fifth bit, bit b of qh[k] for block b
 };
 
 struct FQ6_K {
-  static constexpr int BS = 210, PLANES = 2;
+  static constexpr int BS = 210, PLANES = 2, TILE = 16;
   static constexpr bool OFF = false;
   struct Head { uint32_t d; };
   struct Scales {};
@@ -195,11 +198,15 @@ struct MmqfArgs {
   uint32_t x_pitch, rows;      // bytes between the rows of X; rows of the planes
 };
 
-// The four values are computed at this point.
-__device__ __forceinline__ void pin4(float (&v)[4]) { asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3])); }
+// The values are computed at this point.
+__device__ __forceinline__ void pin(float (&v)[4]) { asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3])); }
+__device__ __forceinline__ void pin(float (&v)[16]) {
+  asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
+  asm volatile("" : "+v"(v[8]), "+v"(v[9]), "+v"(v[10]), "+v"(v[11]), "+v"(v[12]), "+v"(v[13]), "+v"(v[14]), "+v"(v[15]));
+}
 
-// eight waves of TM x TN tiles of 16 x 16
-constexpr int MMQF_WM = 4, MMQF_WN = 2, MMQF_TM = 4, MMQF_TN = 4, MMQF_MT = 16 * MMQF_WM * MMQF_TM, MMQF_NT = 16 * MMQF_WN * MMQF_TN;
+// eight waves of 64 x 64
+constexpr int MMQF_WM = 4, MMQF_WN = 2, MMQF_MT = 64 * MMQF_WM, MMQF_NT = 64 * MMQF_WN;
 
 template <class F>
 __host__ __device__ constexpr int mmqf_buffer_bytes() { return 128 * (MMQF_MT + F::PLANES * MMQF_NT); }
@@ -223,18 +230,32 @@ __device__ __forceinline__ u32x4_m as_vector(const uint4& v) { return (u32x4_m){
 
 template <int J> struct StepIndex { static constexpr int value = J; };
 
-template <class F, typename T>
+// Tiles of S x S, the format's choice: a block of 32 values is one instruction of 16 x 16 x 32 or two of 32 x 32 x 16.
+template <int S> struct MmqfTile;
+template <> struct MmqfTile<16> {
+  typedef tile_f4v Sums;
+  static constexpr int PIECES = 1, AHEAD = 2, SETS = 2;   // instructions a block; units asked for ahead; blocks of X in registers
+  static __device__ __forceinline__ Sums mfma(f16x8 w, f16x8 x, Sums s) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(w, x, s, 0, 0, 0); }
+};
+template <> struct MmqfTile<32> {
+  typedef f32x16 Sums;
+  static constexpr int PIECES = 2, AHEAD = 1, SETS = 1;
+  static __device__ __forceinline__ Sums mfma(f16x8 w, f16x8 x, Sums s) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(w, x, s, 0, 0, 0); }
+};
+
+template <class F, typename T, int S>
 __global__ __launch_bounds__(64 * MMQF_WM * MMQF_WN, 2) void mmqf_kernel(const uint8_t* __restrict__ W, const char* __restrict__ X,
                                                                const char* __restrict__ XD, const char* __restrict__ XS,
                                                                T* __restrict__ Y, float* __restrict__ partial,
                                                                const T* __restrict__ bias, MmqfArgs a) {
-  constexpr int WN = MMQF_WN, TM = MMQF_TM, TN = MMQF_TN, NWV = MMQF_WM * WN, M_T = MMQF_MT, N_T = MMQF_NT;
+  typedef MmqfTile<S> Tile;
+  constexpr int WN = MMQF_WN, TM = 64 / S, TN = 64 / S, R = S * S / 64, NWV = MMQF_WM * WN, M_T = MMQF_MT, N_T = MMQF_NT;   // R: results of a tile in a lane
   constexpr int BUF = mmqf_buffer_bytes<F>(), PLANE_AT = 2 * BUF + 64 * M_T;
   constexpr int XI = M_T / 8 / NWV;                         // fetches of 8 rows of X per wave and step
   static_assert(4 * N_T == 64 * NWV && M_T == 256, "a thread per part of a row's step; a fetch per row of block scales");
   extern __shared__ __align__(128) char smem[];             // (rows of 128 bytes, whose pieces are told apart by xor with their addresses)
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / WN, wn = wave % WN, lrow = lane & 15, lgroup = lane >> 4;
+  const int wm = wave / WN, wn = wave % WN, lrow = lane & (S - 1), lgroup = lane / S;
 
   const TileWork work = tile_work(a.r);
   const int unit_end = work.end;
@@ -302,28 +323,35 @@ __global__ __launch_bounds__(64 * MMQF_WM * MMQF_WN, 2) void mmqf_kernel(const u
     }
   };
 
-  float acc[TN][TM][4], part_acc[TN][TM][4];
+  float acc[TN][TM][R], part_acc[TN][TM][R];
 #pragma unroll
   for (int i = 0; i < TN; ++i)
 #pragma unroll
     for (int k = 0; k < TM; ++k)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc[i][k][r] = 0.0f;
-  const tile_f4v zero = {0.0f, 0.0f, 0.0f, 0.0f};
+      for (int r = 0; r < R; ++r) acc[i][k][r] = 0.0f;
+  typename Tile::Sums zero;
+#pragma unroll
+  for (int r = 0; r < R; ++r) zero[r] = 0.0f;
 
-  // ---- one step of K: 32 units, a block and a pair of tiles each
+  // ---- one step of K: 2 U units, a block and a pair of tiles each
   const int swz = (lrow >> 1) & 7;                          // (tile bases are multiples of 16 rows)
-  // (the operands of block b are 64 b away, by xor: rows are 128 bytes)
-  const uint32_t op0 = 128 * lrow + 16 * (lgroup ^ swz), x_op = lds0 + 128 * 16 * TM * wm, w_op = lds0 + 128 * (M_T + 16 * TN * wn);
-  struct Operands { f16x8 x[2][TM], w[TN][F::PLANES]; };
-  const auto load_x = [&](uint32_t at, int b, int k, Operands& o) { o.x[b][k] = lds_get<f16x8>((at ^ (64 * b)) + 2048 * k); };
+  // (the operands of block b, piece h are 64 b + 32 h away, by xor: rows are 128 bytes)
+  const uint32_t op0 = 128 * lrow + 16 * (lgroup ^ swz), x_op = lds0 + 128 * 64 * wm, w_op = lds0 + 128 * (M_T + 64 * wn);
+  constexpr int U = TM * TN, H = Tile::PIECES, P = H * F::PLANES, AHEAD = Tile::AHEAD, SETS = Tile::SETS;
+  struct Operands { f16x8 x[SETS][TM][H], w[TN][F::PLANES][H]; };
+  const auto load_x = [&](uint32_t at, int b, int k, Operands& o) {
+#pragma unroll
+    for (int h = 0; h < H; ++h) o.x[b % SETS][k][h] = lds_get<f16x8>((at ^ (64 * b + 32 * h)) + 128 * S * k);
+  };
   const auto load_w = [&](uint32_t at, int b, int i, Operands& o) {
 #pragma unroll
-    for (int pl = 0; pl < F::PLANES; ++pl) o.w[i][pl] = lds_get<f16x8>((at ^ (64 * b)) + (128 * N_T * pl + 2048 * i));
+    for (int h = 0; h < H; ++h)
+#pragma unroll
+      for (int pl = 0; pl < F::PLANES; ++pl) o.w[i][pl][h] = lds_get<f16x8>((at ^ (64 * b + 32 * h)) + (128 * N_T * pl + 128 * S * i));
   };
   // The matrix instructions of unit v + AHEAD stand between the multiply-adds of unit v (each waits for the one before it), and an operand's
   // successor is read as soon as the last instruction that takes it has started.
-  constexpr int U = TM * TN, P = F::PLANES, AHEAD = 2;
   const auto load_first = [&](int buf, Operands& o) {
     const uint32_t xat = x_op + buf * BUF + afresh(op0), wat = w_op + buf * BUF + afresh(op0);
 #pragma unroll
@@ -333,74 +361,77 @@ __global__ __launch_bounds__(64 * MMQF_WM * MMQF_WN, 2) void mmqf_kernel(const u
   };
   const auto contract = [&](auto step, int buf, int pb, Operands& o) {
     constexpr int J = decltype(step)::value;
-    const uint32_t xd = lds0 + 2 * BUF + 32 * M_T * pb + 64 * TM * wm + 4 * (afresh(lane) & 15), xat = x_op + buf * BUF + afresh(op0), wat = w_op + buf * BUF + afresh(op0);
-    tile_f4v s[4];
+    const uint32_t xd = lds0 + 2 * BUF + 32 * M_T * pb + 256 * wm + 4 * (afresh(lane) & (S - 1)), xat = x_op + buf * BUF + afresh(op0), wat = w_op + buf * BUF + afresh(op0);
+    typename Tile::Sums s[2 * AHEAD];
     float d8[2][TM];
 #pragma unroll
     for (int k = 0; k < TM; ++k) {
-      d8[0][k] = lds_get<float>(xd + (8 * J * M_T + 64 * k));
-      d8[1][k] = lds_get<float>(xd + (8 * J * M_T + 4 * M_T + 64 * k));
+      d8[0][k] = lds_get<float>(xd + (8 * J * M_T + 4 * S * k));
+      d8[1][k] = lds_get<float>(xd + (8 * J * M_T + 4 * M_T + 4 * S * k));
     }
-    const auto mfma = [&](int v, int pl) {
-      const int b = v / U, i = v % U / TM, k = v % TM;
-      s[v & 3] = __builtin_amdgcn_mfma_f32_16x16x32_f16(o.w[i][pl], o.x[b][k], pl == 0 ? zero : s[v & 3], 0, 0, 0);
+    const auto mfma = [&](int v, int piece) {
+      const int b = v / U, i = v % U / TM, k = v % TM, to = v % (2 * AHEAD);
+      s[to] = Tile::mfma(o.w[i][piece / H][piece % H], o.x[b % SETS][k][piece % H], piece == 0 ? zero : s[to]);
     };
 #pragma unroll
     for (int v = 0; v < AHEAD; ++v)
 #pragma unroll
-      for (int pl = 0; pl < P; ++pl) mfma(v, pl);
+      for (int piece = 0; piece < P; ++piece) mfma(v, piece);
 #pragma unroll
     for (int v = 0; v < 2 * U; ++v) {
-      const int b = v / U, u = v % U, i = u / TM, k = u % TM, n = v + AHEAD;
+      const int b = v / U, u = v % U, i = u / TM, k = u % TM, n = v + AHEAD, from = v % (2 * AHEAD);
 #pragma unroll
-      for (int pl = 0; pl < P; ++pl) {
-        if (n < 2 * U) mfma(n, pl);
-        if (pl == P - 1 && n < U) {
+      for (int piece = 0; piece < P; ++piece) {
+        if (n < 2 * U) mfma(n, piece);
+        if (piece == P - 1 && n < U) {
           if (n % TM == TM - 1) load_w(wat, 1, n / TM, o);
-          if (n / TM == TN - 2) load_x(xat, 1, n % TM, o);
+          if (n / TM == TN - SETS) load_x(xat, 1, n % TM, o);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int r = 4 / P * pl; r < 4 / P * (pl + 1); ++r)
-          part_acc[i][k][r] = J == 0 && b == 0 ? s[v & 3][r] * d8[b][k] : __builtin_fmaf(s[v & 3][r], d8[b][k], part_acc[i][k][r]);
+        for (int r = R / P * piece; r < R / P * (piece + 1); ++r)
+          part_acc[i][k][r] = J == 0 && b == 0 ? s[from][r] * d8[b][k] : __builtin_fmaf(s[from][r], d8[b][k], part_acc[i][k][r]);
         __builtin_amdgcn_sched_barrier(0);
       }
       // (here and not later: the compiler would keep the products and scale them all at the end of the super-block)
-      pin4(part_acc[i][k]);
+      pin(part_acc[i][k]);
     }
   };
   // the end of a super-block
   const auto fold = [&]() {
-    const int ln = afresh(lane), row = ln & 15, group = ln >> 4;
-    const uint32_t at = lds0 + PLANE_AT + 16 * M_T + 4 * (16 * TN * wn + 4 * group);   // d of the lane's first result
+    const int ln = afresh(lane), row = ln & (S - 1), group = ln / S;
+    const uint32_t at = lds0 + PLANE_AT + 16 * M_T + 4 * (64 * wn + 4 * group);        // d of the lane's first result
     u32x4_m sv[TM];
     if constexpr (F::OFF)
 #pragma unroll
       for (int k = 0; k < TM; ++k) {
-        // (a contraction over eight: the other lanes hold values 8 .. 31, zeros beside mins, which are finite)
-        sv[k] = lds_get<u32x4_m>(lds0 + PLANE_AT + 16 * (16 * (TM * wm) + row) + 256 * k);
+        // (a contraction over eight: the other lanes hold the values behind them, zeros beside mins, which are finite)
+        sv[k] = lds_get<u32x4_m>(lds0 + PLANE_AT + 16 * (64 * wm + row) + 16 * S * k);
         if (group) sv[k] = (u32x4_m){0, 0, 0, 0};
       }
 #pragma unroll
     for (int i = 0; i < TN; ++i) {
       __builtin_amdgcn_sched_barrier(0);
-      tile_f4v off[F::OFF ? TM : 1], d, dm;
+      typename Tile::Sums off[F::OFF ? TM : 1];
+      tile_f4v d[R / 4], dm[R / 4];
       if constexpr (F::OFF) {
-        const u32x4_m mv = lds_get<u32x4_m>(lds0 + PLANE_AT + 16 * M_T + 8 * N_T + 16 * (16 * TN * wn + row) + 256 * i);
+        const u32x4_m mv = lds_get<u32x4_m>(lds0 + PLANE_AT + 16 * M_T + 8 * N_T + 16 * (64 * wn + row) + 16 * S * i);
 #pragma unroll
-        for (int k = 0; k < TM; ++k)
-          off[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, mv), __builtin_bit_cast(f16x8, sv[k]), zero, 0, 0, 0);
+        for (int k = 0; k < TM; ++k) off[k] = Tile::mfma(__builtin_bit_cast(f16x8, mv), __builtin_bit_cast(f16x8, sv[k]), zero);
       }
-      d = lds_get<tile_f4v>(at + 64 * i);
-      if (F::OFF) dm = lds_get<tile_f4v>(at + (4 * N_T + 64 * i));
+#pragma unroll
+      for (int q = 0; q < R / 4; ++q) {
+        d[q] = lds_get<tile_f4v>(at + (4 * S * i + 32 * q));
+        if (F::OFF) dm[q] = lds_get<tile_f4v>(at + (4 * N_T + 4 * S * i + 32 * q));
+      }
 #pragma unroll
       for (int k = 0; k < TM; ++k) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          acc[i][k][r] = __builtin_fmaf(part_acc[i][k][r], d[r], acc[i][k][r]);
-          if constexpr (F::OFF) acc[i][k][r] = __builtin_fmaf(off[k][r], dm[r], acc[i][k][r]);
+        for (int r = 0; r < R; ++r) {
+          acc[i][k][r] = __builtin_fmaf(part_acc[i][k][r], d[r >> 2][r & 3], acc[i][k][r]);
+          if constexpr (F::OFF) acc[i][k][r] = __builtin_fmaf(off[k][r], dm[r >> 2][r & 3], acc[i][k][r]);
         }
-        pin4(acc[i][k]);
+        pin(acc[i][k]);
       }
     }
   };
@@ -453,20 +484,23 @@ __global__ __launch_bounds__(64 * MMQF_WM * MMQF_WN, 2) void mmqf_kernel(const u
     }
   }
 
-  // ---- store: lane = one row of X, four features per tile
+  // ---- store: lane = one row of X, R features per tile in runs of four
   float* const mine = sb1 - sb0 < a.r.units ? partial + (int64_t)(2 * work.worker + segment) * (M_T * N_T) : nullptr;
-  const int ln = afresh(lane), group = ln >> 4;             // (the places formed from it: not in scratch from before the first tile on)
+  const int ln = afresh(lane), group = ln / S;              // (the places formed from it: not in scratch from before the first tile on)
 #pragma unroll
   for (int i = 0; i < TN; ++i)
 #pragma unroll
-    for (int k = 0; k < TM; ++k) {
-      const tile_f4v v = {acc[i][k][0], acc[i][k][1], acc[i][k][2], acc[i][k][3]};
-      if (mine) {   // in the order that tile_reduce_kernel adds: [wave][tile of 32 x 32][run][lane] of four
-        *(tile_f4v*)(mine + (((wave * 4 + (i >> 1) * 2 + (k >> 1)) * 4 + 2 * (i & 1) + (group >> 1)) * 64 + 32 * (group & 1) + 16 * (k & 1) + (ln & 15)) * 4) = v;
-      } else {
-        tile_store(v, m_base + 16 * (TM * wm + k) + (ln & 15), n_base + 16 * (TN * wn + i) + 4 * group, Y, bias, a.r);
+    for (int k = 0; k < TM; ++k)
+#pragma unroll
+      for (int q = 0; q < R / 4; ++q) {
+        const tile_f4v v = {acc[i][k][4 * q], acc[i][k][4 * q + 1], acc[i][k][4 * q + 2], acc[i][k][4 * q + 3]};
+        if (mine) {   // in the order that tile_reduce_kernel adds: [wave][tile of 32 x 32][run][lane] of four
+          const int of32 = wave * 4 + S * i / 32 * 2 + S * k / 32, run = S == 32 ? q : 2 * (i & 1) + (group >> 1), at = S == 32 ? ln : 32 * (group & 1) + 16 * (k & 1) + (ln & 15);
+          *(tile_f4v*)(mine + ((of32 * 4 + run) * 64 + at) * 4) = v;
+        } else {
+          tile_store(v, m_base + 64 * wm + S * k + (ln & (S - 1)), n_base + 64 * wn + S * i + 8 * q + 4 * group, Y, bias, a.r);
+        }
       }
-    }
   }
 }
 
@@ -475,7 +509,7 @@ static int mmqf_typed(const MmqfCall& c, hipStream_t stream) {
   const TilePlan p = mmqf_plan(c.M, c.N, c.K, c.partial_bytes);
   constexpr size_t lds = mmqf_lds<F>();
   static_assert(lds <= 160 * 1024, "tile does not fit in LDS");
-  auto kern = mmqf_kernel<F, T>;
+  auto kern = mmqf_kernel<F, T, F::TILE>;
   static std::atomic<uint64_t> done{0};
   allow_large_lds(kern, lds, done);
   const MmqfArgs a = {tile_runs<T>(p, c.M, c.N, c.K / 256, c.Y, c.la.ldy ? c.la.ldy : (int64_t)c.N),
@@ -483,7 +517,7 @@ static int mmqf_typed(const MmqfCall& c, hipStream_t stream) {
   hipLaunchKernelGGL(kern, dim3(p.whole + p.workers), dim3(64 * MMQF_WM * MMQF_WN), lds, stream, (const uint8_t*)c.W, (const char*)c.x.x,
                      (const char*)c.x.d, (const char*)c.x.s, (T*)c.Y, c.partial, (const T*)c.la.bias, a);
   if (p.shared > 0)
-    hipLaunchKernelGGL((tile_reduce_kernel<MMQF_WM, MMQF_WN, MMQF_TM / 2, MMQF_TN / 2, T>), dim3(p.shared, MMQF_WM * MMQF_WN * MMQF_TM * MMQF_TN / 4), dim3(256),
+    hipLaunchKernelGGL((tile_reduce_kernel<MMQF_WM, MMQF_WN, 2, 2, T>), dim3(p.shared, MMQF_WM * MMQF_WN * 4), dim3(256),
                        0, stream, c.partial, (T*)c.Y, (const T*)c.la.bias, a.r);
   return launch_status();
 }
