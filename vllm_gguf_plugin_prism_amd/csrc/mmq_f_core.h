@@ -40,7 +40,7 @@
 // both get denser.  Of two operands it takes 82 to 86 ns on tiles of 32 x 32 and 71 on tiles of 16 x 16, whose results need half the registers
 // on the way: Q6_K [18944,3584] 512 rows 156 -> 150 us, [4096,14336] 1531 rows 390 -> 374.  There a unit's matrix instructions are
 // issued two units ahead of its multiply-adds (one ahead: 155 us, three: no change).  One operand is faster on tiles of 32 x 32: [4096,14336] Q4_K 2100 / 3000 rows 405 / 550 us,
-// on tiles of 16 x 16 418 / 578, Q5_K 430 / 576 and 446 / 588; 80 random products of 1000 to 4096 rows 1.012 times as fast on average, 1.05 the most,
+// on tiles of 16 x 16 418 / 578, Q5_K 430 / 576 and 446 / 588; 80 random products of 1000 to 4096 rows 1.012 times as fast on average, 0.97 to 1.06,
 // [4096,4096] 2500 rows 0.98.
 // Tried and slower: four waves per workgroup and two workgroups per CU (decoding twice), the two waves of a SIMD decoding at
 // different times, the fetches of X in front of the operand reads or spread over the step; the barrier in the middle of a step
