@@ -51,8 +51,10 @@ bool wide_layer_takes(int type13, int type2, int64_t H, int64_t I, int64_t N_out
   if (pairs * top_k > 0xFFFFFFFFll) return false;               // (the kernel's quotient by reciprocal)
   // Both sides of 2200 layers of random sizes were measured, 4 to 1500 pairs per expert, how many times as long the others take:
   //   * past what the streaming tiles take: 1.33 (Q8_0, 150 layers of 4 to 100 pairs per expert), 1.47 from 60 pairs on over all types and
-  //     never below 1.05 there (Q8_0 1.23 to 1.36, also at 300 to 1500).  Q8_0 past 640 pairs per expert, first product
-  //     and second of Q8_0, Q4_0 or Q6_K, is left where its route is fixed by a test, though these are 1.03 to 1.25 times as fast there, too;
+  //     never below 1.05 there (Q8_0 1.23 to 1.36, also at 300 to 2500, 1.15 at least).  A second product of Q6_K behind Q8_0, on the wide tiles here and on blocks of 64 slots
+  //     there, is up to 1.15 times as long here once it is long and its rows are many (277 layers of 200 to 2500 pairs per expert).  All of those that are more than
+  //     1 % slower but one have 2 pairs I N_out > 240e9, below which these tiles are 1.15 times as fast on average (the one, H 3072, I 5888: 0.91 to 0.98); the line there loses 0.5 % against always taking
+  //     the faster one, one at 640 pairs per expert 4.8 %;
   //   * Q8_0 past what they take (I below 768) with up to 16 pairs per expert, where the others have blocks of 16 slots and a panel there costs less while
   //     the workgroups are few, first of all the second product's (307 layers, H 256 .. 4096, I 256 or 512, 8 to 128 experts): from 180 blocks times (panels of a row of X + 1)
   //     on 1.17 (0.94 .. 1.65), below that 0.96 (0.89 .. 1.12); with the lighter panels of Q4_K, Q5_K from 60 on.  The line loses 0.5 % on average against
@@ -60,7 +62,7 @@ bool wide_layer_takes(int type13, int type2, int64_t H, int64_t I, int64_t N_out
   //   * against the streaming tiles from 40 pairs per expert on: 1.3 to 1.6, hardly ever less than 1.05.
   // Below that a block of 32 slots is padding for the most part, and the one or the other is faster by the type, the rows'
   // length and how the workgroups fall into rounds: by the two estimates, which lose 0.5 % on average against always taking the faster one.
-  if (type13 == T_Q8_0 && type2 != T_Q4_K && type2 != T_Q5_K && pairs > 640 * num_experts) return false;
+  if (type13 == T_Q8_0 && type2 == T_Q6_K && pairs > 256 * num_experts && 2.0 * (double)pairs * (double)I * (double)N_out > 240e9) return false;
   if (pairs > 40 * num_experts) return true;
   if (!ts_layer_takes(type13, type2, H, I, N_out, tokens, top_k, num_experts)) {
     if (type13 != T_Q8_0 || H > 4096 || I >= 768 || pairs > 16 * num_experts) return true;
