@@ -48,3 +48,38 @@ def test_blocks_in_part(qtype, qtype2, hid, inner, n_out, huge):
         other = layer("gguf_moe_mmq_layer", *cuda, qtype, qtype2, 8).cpu().numpy()
         for r in rows:
             assert (np.isnan(got[r]) == np.isnan(other[r])).all() and (np.isinf(got[r]) == np.isinf(other[r])).all()
+
+
+# rows that hold an activation that is no number, some in every block: they are not walked again, as a row whose block scale is infinite is (that is 1.7 times the
+# layer's time); the rows beside them keep their bits
+@pytest.mark.parametrize("qtype", (o.Q4_K, o.Q4_0))
+def test_rows_without_numbers_take_one_walk(qtype):
+    from vllm_gguf_plugin_prism_amd import _lib
+    rng = np.random.default_rng(qtype)
+    tokens, e, hid, inner = 600, 8, 2048, 1024
+    assert _lib.lib().gguf_moe_mmq_layer_wide(qtype, qtype, hid, inner, hid, 1, tokens, e) == 1
+    w13 = np.stack([o.make_weights(rng, qtype, 2 * inner, hid) for _ in range(e)])
+    w2 = np.stack([o.make_weights(rng, qtype, hid, inner) for _ in range(e)])
+    ids, wts = rng.permutation(np.arange(tokens) % e).astype(np.int32)[:, None].copy(), rng.random((tokens, 1)).astype(np.float32)
+    x = torch.from_numpy(0.01 * rng.standard_normal((tokens, hid)).astype(np.float32)).cuda()
+    rest = [torch.from_numpy(a).cuda() for a in (w13, w2, wts, ids)]
+    none = torch.zeros(tokens, dtype=torch.bool, device="cuda")
+    none[::6] = True
+    with_none = x.clone()
+    with_none[none, 1000] = float("nan")
+    want, us = layer("gguf_moe_mmq_layer", x, *rest, qtype, qtype), {}
+    got = layer("gguf_moe_mmq_layer", with_none, *rest, qtype, qtype)
+    assert torch.equal(got[~none], want[~none]) and bool(got[none].isnan().any(1).all()) and bool(want.isfinite().all())
+    L, out = _lib.lib(), torch.empty_like(x)
+    nbytes = L.gguf_moe_mmq_layer_workspace_bytes(qtype, qtype, tokens, 1, hid, inner, hid, e, 0)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    for rows in (x, with_none) * 10:
+        begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        begin.record()
+        for _ in range(10):
+            assert L.gguf_moe_mmq_layer(rows.data_ptr(), 0, rest[0].data_ptr(), qtype, rest[1].data_ptr(), qtype, rest[3].data_ptr(), rest[2].data_ptr(), ws.data_ptr(), nbytes,
+                                        out.data_ptr(), hid, inner, hid, 1, tokens, 1, e, torch.cuda.current_stream().cuda_stream) == 0
+        end.record()
+        end.synchronize()
+        us[rows is x] = min(us.get(rows is x, 1e9), begin.elapsed_time(end) * 100.0)
+    assert us[False] < 1.25 * us[True], us

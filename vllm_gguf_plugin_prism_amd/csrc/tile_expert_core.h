@@ -299,20 +299,40 @@ __global__ __launch_bounds__(64 * EXPERT_NW, 3) void tile_expert_kernel(const ui
     constexpr bool SMALL = decltype(small)::value;
     walk(std::false_type(), small);
     // An activation past 8.3e6 has a block scale that a half does not hold: infinity, which the multiply-add takes from itself, so that none of the row's results is
-    // a number (one of them tells).  Its product with the sum is an infinity, of a sum of 0 no number: where a row has none, all four waves walk again with the seed taken
-    // off first.  The rows beside it get the same bits.
+    // a number (one of them tells).  Its product with the sum is an infinity, of a sum of 0 no number: where a row has none, the waves look through the records that they
+    // fetch, and if a block scale is infinite, all four walk again with the seed taken off first (else it is an activation or a weight that is no number, and
+    // stays that).  The rows beside it get the same bits.
     {
       const bool none = __any(__builtin_isnan(acc[0]) && *(const int*)(smem + ids_at + 4 * (SMALL ? c : lrow)) < moe.num_pairs);
       if (lane == 0) *(int*)(smem + FLAG_AT + 4 * wave) = none;
       __syncthreads();
-      const int4 flags = *(const int4*)(smem + FLAG_AT);
-      if (flags.x | flags.y | flags.z | flags.w) {
+      const auto flagged = [&] {
+        const int4 flags = *(const int4*)(smem + FLAG_AT);
+        return (flags.x | flags.y | flags.z | flags.w) != 0;
+      };
+      if (flagged()) {
         int l = tid & 63;
         asm volatile("" : "+v"(l));                           // (what is formed from it is formed again: kept beside the first walk, it would go to scratch)
+        bool infinite = false;                                // (from the addresses of the fetches: nothing more is held over the walk)
+        for (int ch = 2 * p0; ch < 2 * p1; ++ch)
+#pragma unroll
+          for (int j = 0; j < XW; ++j) {
+            const int q = 64 * (wave + EXPERT_NW * j) + l;
+            if (q >= EXPERT_M * XP || q % XP != EXPERT_D_AT / 16) continue;   // (the piece of a record that begins with its scales)
+            const uint2 d = *(const uint2*)(X + (uint64_t)(uint32_t)ch * a.x_plane + x_at[j]);
+            const auto inf = [](uint32_t two) { return (two & 0xFFFFu) == 0x7C00u || two >> 16 == 0x7C00u; };
+            infinite |= inf(d.x) | inf(d.y);
+          }
+        infinite = __any(infinite);
+        __syncthreads();                                      // (the first flags have been read)
+        if (l == 0) *(int*)(smem + FLAG_AT + 4 * wave) = infinite;
+        __syncthreads();
         lrow = l & 31; half = l >> 5; c = l & 15; g = l >> 4;
-        request(p0, std::true_type());
-        fetch_x(2 * p0);
-        walk(std::true_type(), small);
+        if (flagged()) {
+          request(p0, std::true_type());
+          fetch_x(2 * p0);
+          walk(std::true_type(), small);
+        }
       }
     }
 
