@@ -83,3 +83,26 @@ def test_rows_without_numbers_take_one_walk(qtype):
         end.synchronize()
         us[rows is x] = min(us.get(rows is x, 1e9), begin.elapsed_time(end) * 100.0)
     assert us[False] < 1.25 * us[True], us
+
+
+# two experts with the same weights, the rows of one, three to sixteen of a block, among those of the other, which fill theirs: the same bits, tiles of 16 x 16 or of
+# 32 x 32 (activations of one sign too, whose offsets are as large as the products)
+@pytest.mark.parametrize("qtype,qtype2", [(o.Q4_0, o.Q4_0), (o.Q8_0, o.Q8_0), (o.Q4_K, o.Q4_K), (o.Q5_K, o.Q5_K), (o.Q6_K, o.Q6_K)])
+@pytest.mark.parametrize("few", (3, 16))
+@pytest.mark.parametrize("one_sign", (False, True))
+def test_a_pair_has_the_bits_it_has_in_a_full_block(qtype, qtype2, few, one_sign):
+    from vllm_gguf_plugin_prism_amd import _lib
+    rng = np.random.default_rng(qtype + few)
+    e, hid, inner, full = 3, 768, 1024, 32
+    counts = (few, full, 150)
+    tokens = sum(counts)
+    assert _lib.lib().gguf_moe_mmq_layer_wide(qtype, qtype2, hid, inner, hid, 1, tokens, e) == 1
+    w13 = np.stack([o.make_weights(rng, qtype, 2 * inner, hid)] * 2 + [o.make_weights(rng, qtype, 2 * inner, hid)])
+    w2 = np.stack([o.make_weights(rng, qtype2, hid, inner)] * 2 + [o.make_weights(rng, qtype2, hid, inner)])
+    x = 0.05 * rng.standard_normal((tokens, hid)).astype(np.float32)
+    x = 0.02 * np.abs(x) if one_sign else x                 # (so that sums of h fit in a half)
+    x[few:2 * few] = x[:few]
+    ids = np.repeat(np.arange(e), counts).astype(np.int32)[:, None].copy()
+    cuda = [torch.from_numpy(a).cuda() for a in (x, w13, w2, np.ones((tokens, 1), np.float32), ids)]
+    got = layer("gguf_moe_mmq_layer", *cuda, qtype, qtype2)
+    assert bool(got.isfinite().all()) and torch.equal(got[:few], got[few:2 * few])
