@@ -464,7 +464,7 @@ def main() -> int:
             "per_shape": tables["int8"],
             "default_engine": {"value": auto512, "unit": "TOPS", "per_shape": tables["auto"],
                                "note": "engine='auto', what gguf_mmq and the dispatch run: the same exact whole-number products, per shape "
-                                       "on int8 MFMA or, where its cost estimate is lower, on v_mfma_f32_32x32x16_f16"},
+                                       "on int8 MFMA or, where its cost estimate is lower, on v_mfma_f32_16x16x32_f16"},
             "half_engine": {"value": half512, "unit": "TOPS", "frac_of_f16_mfma_peak": half512 / F16_PEAK_TFLOPS,
                             "per_shape": tables["half"],
                             "note": "engine='half', opt-in: dequantized operands on v_mfma_f32_32x32x16_f16; not the "

@@ -28,8 +28,8 @@
 // [4096,14336] 1531 rows 485 -> 355, [18944,3584] 512 rows 199 -> 144, 1024 rows 369 -> 280.  (Up to 2048 rows Q4_K and Q5_K run tile_walk_core.h mostly: the figures of 1531
 // rows below are those of this kernel, by which it was built.)
 // What bounds it now is vector issue beside the matrix unit, at a clock that falls to about 2.0 GHz under this load: by
-// counters ([4096,14336] Q4_K, 1531 rows) the vector ALU issues in 64 % of the SIMD cycles and the matrix unit is busy in
-// 32 %, Q6_K 52 % and 45 %.  The matrix instructions, the multiply-adds and the operand reads of a step take about 0.45 us
+// counters ([4096,14336] Q4_K, 1531 rows) the vector ALU issues in 61 % of the SIMD cycles and the matrix unit is busy in
+// 35 %, Q6_K ([18944,3584], 512 rows) 46 % and 38 %.  The matrix instructions, the multiply-adds and the operand reads of a step take about 0.45 us
 // each; a step takes 1.2 us, a super-block, which is four steps and its end, 5.9 (Q6_K 7.2).  So what is left out counts, not
 // what is hidden: with decoding in 30 instead of 50 vector instructions per wave and step (masks and the 1024s as one
 // instruction, high nibbles left where they are), LDS addresses whose constants lie in the instructions (40 additions fewer per

@@ -41,9 +41,9 @@ static inline double moe_blocks_estimate(int num_sorted, int num_pairs, int bloc
 // row of a second activation workspace, which the second expert GEMM reads as it is (no [pairs][2 inner] tensor, no
 // quantize launch).
 struct Gate16 {
-  char* rows;             // q8_1 rows of h, one per pair
+  char* rows;             // q8_1 rows of h, one per pair (expert and wide tiles: records, layer_seam.h)
   int64_t row_bytes;
-  int inner, kp, act;     // features of each half; q8_kp(inner); ACT_SILU / ACT_GELU
+  int inner, kp, act;     // features of each half; q8_kp(inner) (expert and wide tiles: 1 where the records are the wide tiles', else 0); ACT_SILU / ACT_GELU
 };
 
 // --------------------------------------------------------------------------------------------

@@ -468,7 +468,7 @@ __device__ __forceinline__ void mmvq_stream_body(const uint8_t* __restrict__ W, 
   const int u = min(u_raw, nb - 1);
 
   // The codes of the format's table are asked for first of all, and its entries are placed once the first weights are on their way: filling it before they were
-  // asked for cost the time of a trip to memory (one row: IQ2_XXS [17408,5120] 9.52 / 9.10 us, IQ3_XXS [5120,5120] 6.5 / 5.9, IQ3_S [4096,4096]
+  // asked for cost the time of a trip to memory (one row: IQ2_XXS [17408,5120] 9.5 / 9.0 to 9.1 us, IQ3_XXS [5120,5120] 6.5 / 5.9, IQ3_S [4096,4096]
   // 5.5 / 4.8, IQ1_S [14336,4096] 7.4 / 6.75).
   constexpr int NT = 64 * NW;
   typename TableCodes<F, NT>::Codes codes;
@@ -483,7 +483,7 @@ __device__ __forceinline__ void mmvq_stream_body(const uint8_t* __restrict__ W, 
   typedef SpanRegs<SPANS ? SPAN : 16, ANY> Span;
   [[maybe_unused]] uint32_t mis[D];   // ANY: where in its first 16-byte piece the stretch of each row in flight starts
   // HALF: the row is a lane's, and a product of 64 bits for it on every turn is a tenth of a codebook format's loop (two multiplications at a quarter of the rate, five
-  // more instructions; IQ2_XXS [17408,5120] 9.66 / 9.52 us): there the address moves on by one turn's rows while there is another, and stays where there is none.
+  // more instructions; IQ2_XXS [17408,5120] 1.015 times as long): there the address moves on by one turn's rows while there is another, and stays where there is none.
   // (The other formats wait for memory and not for this: no change.)
   const int below = wave_on ? nrows - slot : 0;   // (rows from this slot on)
   [[maybe_unused]] const uint8_t* at = wbase + (uint64_t)(uint32_t)min(slot, nrows - 1) * (uint32_t)rowbytes;
@@ -719,7 +719,7 @@ __device__ __forceinline__ void mmvq_stream_body(const uint8_t* __restrict__ W, 
 #pragma unroll
     for (int d = 0; d < D; ++d) {
       const int i = i0 + d;
-      const bool row_ok = HALF && F::TABLE_BYTES > 0 ? slots * i < below : i < my_rows;   // (the same; by the first IQ2_XXS [17408,5120] takes 9.35 us for 9.8, by the second Q8_0 [5120,5120] 7.0 for 7.3)
+      const bool row_ok = HALF && F::TABLE_BYTES > 0 ? slots * i < below : i < my_rows;   // (the same; with the second IQ2_XXS [17408,5120] takes 1.05 times as long, with the first Q8_0 [5120,5120] 1.04 times)
       float acc[MT];
       typename F::Regs cur;
       if constexpr (SPANS) {

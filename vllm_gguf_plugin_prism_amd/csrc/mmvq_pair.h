@@ -12,7 +12,8 @@
 
 namespace gguf {
 
-// Workgroups before `wgs` have rows of W, the others rows of V.
+// Workgroups before `wgs` have rows of W, the others rows of V.  (Of the arguments the first 14 words are in registers, to pitch2: n2 and rows2 are loaded, and the
+// workgroups of V wait for them before their first requests.)
 template <class F, int DF, int SF, class G, int DG, int SG, int MT, int NW, typename T>
 __global__ __launch_bounds__(64 * NW) void mmvq_pair_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ V, const T* __restrict__ X, int wgs, GGUF_GEOM,
                                                             uint32_t pitch2, int n2, int rows2, T* __restrict__ Y, T* __restrict__ Z, const T* __restrict__ bias,

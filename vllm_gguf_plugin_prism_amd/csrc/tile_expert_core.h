@@ -13,7 +13,8 @@
 //     and half the multiply-adds, the same bits (a pair's result does not depend on how many share its block).
 // Measured, us per layer, half-precision tiles / these: Q4_K 128 experts 300 tokens 137 / 121, Q5_K 178 / 156, Q4_0 64 experts 200 tokens 115 / 98, Q8_0 122 /
 // 109, Q4_0 128 experts 120 tokens 119 / 99, Q4_K 8 experts 95 / 82; Q4_K with Q6_K, 128 experts, top-8,
-// H 2048, I 768, 300 tokens 156 / 142 (floor 82); 200 layers of random sizes, 65 to 1500 tokens: 1.09 on average, the worst 0.965.
+// H 2048, I 768, 300 tokens 153 to 162 / 142 to 150 (floor 82); 300 layers of random sizes, 65 to 1500 tokens, by the rule of wide_layer_takes (tile_wide.hip): 1.106 on
+// average, the slowest 0.994.
 // Error against 64 bits over K 512 .. 8192 (rms, second product; normal / one-sign activations; half-precision tiles, then these, in 1e-8): Q4_0
 // 13.6 / 8.0, 8.2 / 5.0; Q8_0 11.2 / 12.1, 7.9 / 8.1; Q4_K 9.9 / 18.4, 8.5 / 10.4; Q5_K 9.8 / 18.1, 8.8 / 10.6.
 // Tried and slower: two sets of weight scales in registers, the next block's under way (120 to 133 us, 156 to 237: they spill).

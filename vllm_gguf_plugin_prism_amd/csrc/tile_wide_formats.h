@@ -119,7 +119,7 @@ struct WQ5_KT : WQ4_KT<C> {   // Q4_K with a fifth bit, bit b of qh[k] for block
 };
 
 // Block b = 4 n + t: low nibbles (t < 2) or high ones of ql[64 n + 32 (t % 2) ..], bits 2 t of qh[32 n ..]; a scale per 16
-// values, so one for a lane and block.  (code - 32) * scale has 13 bits: two operands, on scale & ~15 and scale & 15.
+// values, so one for a lane and block.  (code - 32) * scale has 12 bits and a sign: two operands, the product rounded to half precision and what that leaves out.
 struct WQ6_K {
   static constexpr int PB = 210, PLANES = 2, KIND = SUPER;
   static constexpr bool CUT = true, OFF = false, MIN16 = false;
